@@ -135,27 +135,32 @@ def stream_ptr(dev):
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
-_workspaces: dict = {}
-_retired: list = []
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp): the ordinary calls with their checks, allocation, scratch and
+    launch in one native call.  Its functions return None where the Python path has to take the call."""
+    global _host
+    if _host is None:
+        lib()                                # the shared library first: a missing build is reported there
+        try:
+            from bitstack_amd import _host as native
+        except ImportError as e:
+            raise RuntimeError(f"bitstack_amd/_host.so is missing or does not load ({e}): build it with `make -C {_CSRC}` "
+                               "(or __graft_entry__.build()); there is no fallback path") from e
+        _host = native
+    return _host
 
 
 def workspace(dev, nbytes: int):
-    """Per-(device, stream) scratch tensor, grown on demand.  Kernels on one
-    stream are ordered, so reusing it across calls on that stream is safe.
+    """Scratch tensor of the device's current stream, grown on demand: one per (device, stream), shared with the
+    native host path.  Kernels on one stream are ordered, so reusing it across calls on that stream is safe.
 
     A buffer that is outgrown is kept alive for the life of the process, never
     handed back to the allocator: a HIP graph captured while it was current has
     its address baked in, and its replays must keep writing into memory nobody
     else owns.  (A graph captured before a growth still uses the old buffer; it
     stays correct, it just does not share scratch with later eager calls.)"""
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
-    with _lock:
-        buf = _workspaces.get(key)
-        if buf is None or buf.numel() < nbytes:
-            if buf is not None:
-                _retired.append(buf)
-            # grow geometrically so that a sequence of slowly growing requests retires few buffers
-            size = max(nbytes, 1 << 20, 0 if buf is None else 2 * buf.numel())
-            buf = torch.empty(size, dtype=torch.uint8, device=dev)
-            _workspaces[key] = buf
-    return buf
+    index = torch.cuda.current_device() if dev.index is None else dev.index
+    return host().workspace(index, nbytes)

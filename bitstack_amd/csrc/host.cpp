@@ -1,0 +1,364 @@
+// The host path of the Python layer in native code: a CPython module (bitstack_amd/_host.so) over the C ABI.
+//
+// A decode call is two kernels of 3 to 20 us, and one BitStackLinear.forward spent 25 us on the host in Python (slicing
+// the stacked buffers, a dozen property reads per tensor, the workspace table, three context managers, a ctypes call of
+// 14 arguments): every call below about 25 us of GPU time ran at the speed of the interpreter.  Here the same checks,
+// the output's allocation, the workspace and the launch are one call of METH_FASTCALL.  Whatever is not the ordinary case -
+// tensors on the CPU or on two devices, another dtype, non-contiguous tensors, no tokens, no blocks - is answered with None
+// and takes the Python path, which converts, or raises its documented errors.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <map>
+#include <mutex>
+#include <utility>
+#include <vector>
+
+#include "../../include/bitstack_hip.h"
+
+namespace {
+
+// ---- scratch -----------------------------------------------------------------------------------
+// One scratch tensor per (device, stream), grown geometrically.  Kernels on one stream are ordered, so reusing it across
+// calls on that stream is safe.  A buffer that is outgrown is never handed back to the allocator: a HIP graph
+// captured while it was current has its address baked in, and its replays must keep writing into memory nobody else
+// owns.  (A graph captured before a growth still uses the old buffer; it stays correct, it just does not share scratch
+// with later eager calls.)  The table lives until the process ends: tensors must not outlive the HIP runtime's tear-down.
+struct Scratch {
+    std::mutex lock;
+    std::map<std::pair<int, hipStream_t>, at::Tensor> current;
+    std::vector<at::Tensor> retired;
+};
+Scratch &scratch() {
+    static Scratch *s = new Scratch;
+    return *s;
+}
+
+at::Tensor workspace_for(int device, hipStream_t stream, int64_t bytes) {
+    Scratch &s = scratch();
+    std::lock_guard<std::mutex> guard(s.lock);
+    at::Tensor &t = s.current[{device, stream}];
+    if (!t.defined() || t.numel() < bytes) {
+        int64_t size = bytes > (1 << 20) ? bytes : (1 << 20);
+        if (t.defined()) {
+            // grow geometrically so that a sequence of slowly growing requests retires few buffers
+            if (2 * t.numel() > size) size = 2 * t.numel();
+            s.retired.push_back(t);
+        }
+        t = at::empty({size}, at::TensorOptions().dtype(at::kByte).device(at::kCUDA, (c10::DeviceIndex)device));
+    }
+    return t;
+}
+
+// ---- arguments -----------------------------------------------------------------------------------
+const at::Tensor *tensor_arg(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+bool plain(const at::Tensor &t, at::ScalarType type, c10::Device dev) {
+    return t.scalar_type() == type && t.device() == dev && t.is_contiguous();
+}
+
+PyObject *raise_status(int status, const char *what) {
+    PyErr_Format(PyExc_RuntimeError, "%s failed with status %d: %s", what, status, bs_error_string(status));
+    return nullptr;
+}
+
+// The first `blocks` of the stacked buffers of one matrix, if they are what the C ABI takes as they lie.
+struct Matrix {
+    const at::Tensor *q, *u, *vt;
+    int64_t I, M, N, K;
+};
+bool matrix_args(PyObject *const *a, int64_t blocks, c10::Device dev, Matrix &m) {
+    m.q = tensor_arg(a[0]);
+    m.u = tensor_arg(a[1]);
+    m.vt = tensor_arg(a[2]);
+    if (!m.q || !m.u || !m.vt) return false;
+    if (!plain(*m.q, at::kByte, dev) || !plain(*m.u, at::kHalf, dev) || !plain(*m.vt, at::kHalf, dev)) return false;
+    if (m.q->dim() != 2 || m.u->dim() != 3 || m.vt->dim() != 3) return false;
+    m.I = blocks;
+    m.M = m.u->size(1);
+    m.K = m.u->size(2);
+    m.N = m.vt->size(2);
+    if (blocks < 1 || blocks > m.u->size(0) || blocks > m.vt->size(0) || blocks > m.q->size(0)) return false;
+    if (m.vt->size(1) != m.K || m.q->size(1) != (m.M * m.N + 7) / 8) return false;
+    return m.M > 0 && m.N > 0 && m.M * m.N < ((int64_t)1 << 40) && m.M < INT32_MAX && m.N < INT32_MAX;
+}
+
+bool int_arg(PyObject *o, int64_t &v) {
+    v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) return false;
+    return true;
+}
+
+at::Tensor new_half(at::IntArrayRef sizes, c10::Device dev) {
+    return at::Tensor(at::detail::empty_cuda(sizes, at::kHalf, dev, std::nullopt));
+}
+
+// The output shape: x's with the last dimension replaced.
+c10::SmallVector<int64_t, 6> output_sizes(const at::Tensor &x, int64_t last) {
+    c10::SmallVector<int64_t, 6> s(x.sizes().begin(), x.sizes().end());
+    s.back() = last;
+    return s;
+}
+
+// A guard only where the tensors' device is not the current one (asking costs less than setting it).
+struct DeviceScope {
+    c10::hip::OptionalHIPGuard guard;
+    explicit DeviceScope(c10::Device dev) {
+        if (c10::hip::current_device() != dev.index()) guard.set_index(dev.index());
+    }
+};
+
+// ---- entry points --------------------------------------------------------------------------------
+// forward(qweight, u, vt, blocks, x, bias or None) -> y, or None where the Python path has to take the call
+PyObject *host_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "forward takes 6 arguments");
+    try {
+        const at::Tensor *x = tensor_arg(a[4]);
+        const at::Tensor *bias = a[5] == Py_None ? nullptr : tensor_arg(a[5]);
+        int64_t blocks;
+        if (!int_arg(a[3], blocks)) return nullptr;
+        Matrix m;
+        if (!x || (a[5] != Py_None && !bias) || !x->is_cuda() || x->dim() < 1) Py_RETURN_NONE;
+        const c10::Device dev = x->device();
+        if (!plain(*x, at::kHalf, dev) || !matrix_args(a, blocks, dev, m)) Py_RETURN_NONE;
+        if (x->size(-1) != m.N || x->numel() == 0 || x->numel() / m.N >= INT32_MAX) Py_RETURN_NONE;
+        if (bias && (!plain(*bias, at::kHalf, dev) || bias->numel() != m.M)) Py_RETURN_NONE;
+        const int T = (int)(x->numel() / m.N);
+        const int64_t need = bs_workspace_bytes((int)m.I, (int)m.M, (int)m.N, (int)m.K, T);
+        if (need < 0) return raise_status((int)need, "bs_workspace_bytes");
+        DeviceScope scope(dev);
+        const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+        const at::Tensor ws = workspace_for(dev.index(), stream, need);
+        const at::Tensor y = new_half(output_sizes(*x, m.M), dev);
+        const int st = bs_forward((const uint8_t *)m.q->const_data_ptr(), m.u->const_data_ptr(), m.vt->const_data_ptr(),
+                                  x->const_data_ptr(), bias ? bias->const_data_ptr() : nullptr, y.mutable_data_ptr(), (int)m.I,
+                                  (int)m.M, (int)m.N, (int)m.K, T, ws.mutable_data_ptr(), ws.numel(), stream);
+        if (st != BS_OK) return raise_status(st, "bs_forward");
+        return THPVariable_Wrap(y);
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// rebuild(qweight, u, vt, blocks) -> w [M, N], or None
+PyObject *host_rebuild(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 4) return PyErr_Format(PyExc_TypeError, "rebuild takes 4 arguments");
+    try {
+        int64_t blocks;
+        if (!int_arg(a[3], blocks)) return nullptr;
+        const at::Tensor *u = tensor_arg(a[1]);
+        Matrix m;
+        if (!u || !u->is_cuda() || !matrix_args(a, blocks, u->device(), m)) Py_RETURN_NONE;
+        const c10::Device dev = u->device();
+        DeviceScope scope(dev);
+        const at::Tensor w = new_half({m.M, m.N}, dev);
+        const int st = bs_reconstruct_w((const uint8_t *)m.q->const_data_ptr(), m.u->const_data_ptr(), m.vt->const_data_ptr(),
+                                        w.mutable_data_ptr(), (int)m.I, (int)m.M, (int)m.N, (int)m.K,
+                                        c10::hip::getCurrentHIPStream(dev.index()).stream());
+        if (st != BS_OK) return raise_status(st, "bs_reconstruct_w");
+        return THPVariable_Wrap(w);
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// linear(x, w, bias or None) -> x @ w^T (+ bias), or None
+PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 3) return PyErr_Format(PyExc_TypeError, "linear takes 3 arguments");
+    try {
+        const at::Tensor *x = tensor_arg(a[0]), *w = tensor_arg(a[1]);
+        const at::Tensor *bias = a[2] == Py_None ? nullptr : tensor_arg(a[2]);
+        if (!x || !w || (a[2] != Py_None && !bias) || !x->is_cuda() || x->dim() < 1 || w->dim() != 2) Py_RETURN_NONE;
+        const c10::Device dev = x->device();
+        if (!plain(*x, at::kHalf, dev) || !plain(*w, at::kHalf, dev)) Py_RETURN_NONE;
+        const int64_t M = w->size(0), N = w->size(1);
+        if (M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX || x->size(-1) != N || x->numel() == 0 || x->numel() / N >= INT32_MAX) Py_RETURN_NONE;
+        if (bias && (!plain(*bias, at::kHalf, dev) || bias->numel() != M)) Py_RETURN_NONE;
+        DeviceScope scope(dev);
+        const at::Tensor y = new_half(output_sizes(*x, M), dev);
+        const int st = bs_linear_f16(x->const_data_ptr(), w->const_data_ptr(), bias ? bias->const_data_ptr() : nullptr,
+                                     y.mutable_data_ptr(), (int)(x->numel() / N), (int)M, (int)N,
+                                     c10::hip::getCurrentHIPStream(dev.index()).stream());
+        if (st != BS_OK) return raise_status(st, "bs_linear_f16");
+        return THPVariable_Wrap(y);
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// workspace(device index, nbytes) -> the scratch tensor of the device's current stream
+PyObject *host_workspace(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 2) return PyErr_Format(PyExc_TypeError, "workspace takes 2 arguments");
+    try {
+        int64_t dev, bytes;
+        if (!int_arg(a[0], dev) || !int_arg(a[1], bytes)) return nullptr;
+        return THPVariable_Wrap(workspace_for((int)dev, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(), bytes));
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// ---- a decode step's launches as one call -----------------------------------------------------------
+// The launches between the embedding and the last norm never change between steps: their arguments are laid
+// out once (make_steps) and issued in one call (run_steps) - nine kernels per layer at the cost of the launches alone.
+// The tensors behind the pointers are kept alive by the caller, who also lays the list out again when one is replaced.
+struct Step {
+    enum Kind { GROUP, ATTENTION, NORM } kind;
+    // GROUP
+    std::vector<bs_matrix> mats;
+    int N, K, T, epilogue, rms;
+    float eps;
+    const void *x, *residual;
+    void *y;
+    // ATTENTION
+    const void *qkv, *cos, *sin;
+    void *kcache, *vcache, *out;
+    const int64_t *pos;
+    int B, heads, kv_heads, head_dim, max_len;
+    // NORM: y[T, N] = RMSNorm of x with this weight vector
+    const void *weight;
+};
+struct Steps {
+    std::vector<Step> list;
+    int64_t need = 0;
+};
+const char *const STEPS = "bitstack_amd.steps";
+void free_steps(PyObject *cap) { delete (Steps *)PyCapsule_GetPointer(cap, STEPS); }
+
+// make_steps([("group", address of bs_matrix[n], n, N, K, x, T, eps or None, epilogue, residual or 0, y) |
+//             ("attention", qkv, kcache, vcache, cos, sin, pos, out, B, heads, kv_heads, head_dim, max_len) |
+//             ("norm", x, weight, y, T, H, eps), ...]) -> handle; every tensor as its address
+PyObject *host_make_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 1 || !PyList_Check(a[0])) return PyErr_Format(PyExc_TypeError, "make_steps takes a list");
+    Steps *steps = new Steps;
+    for (Py_ssize_t j = 0; j < PyList_GET_SIZE(a[0]); j++) {
+        PyObject *t = PyList_GET_ITEM(a[0], j);
+        Step s = {};
+        const char *kind = PyTuple_Check(t) && PyTuple_GET_SIZE(t) > 0 ? PyUnicode_AsUTF8(PyTuple_GET_ITEM(t, 0)) : nullptr;
+        bool ok = kind != nullptr;
+        unsigned long long p[7] = {0, 0, 0, 0, 0, 0, 0};
+        if (ok && kind[0] == 'g') {
+            PyObject *eps;
+            int count;
+            s.kind = Step::GROUP;
+            ok = PyArg_ParseTuple(t, "sKiiiKiOiKK", &kind, &p[0], &count, &s.N, &s.K, &p[1], &s.T, &eps, &s.epilogue, &p[2], &p[3]) &&
+                 count >= 1 && count <= BS_MAX_GROUP;
+            if (ok) {
+                const bs_matrix *m = (const bs_matrix *)(uintptr_t)p[0];
+                s.mats.assign(m, m + count);
+                s.rms = eps != Py_None;
+                s.eps = s.rms ? (float)PyFloat_AsDouble(eps) : 0.f;
+                s.x = (const void *)(uintptr_t)p[1];
+                s.residual = (const void *)(uintptr_t)p[2];
+                s.y = (void *)(uintptr_t)p[3];
+                const int64_t need = bs_forward_group_workspace_bytes(s.mats.data(), count, s.N, s.K, s.T);
+                if (need < 0) {
+                    delete steps;
+                    return raise_status((int)need, "bs_forward_group_workspace_bytes");
+                }
+                if (need > steps->need) steps->need = need;
+            }
+        } else if (ok && kind[0] == 'n') {
+            s.kind = Step::NORM;
+            ok = PyArg_ParseTuple(t, "sKKKiif", &kind, &p[0], &p[1], &p[2], &s.T, &s.N, &s.eps);
+            s.x = (const void *)(uintptr_t)p[0];
+            s.weight = (const void *)(uintptr_t)p[1];
+            s.y = (void *)(uintptr_t)p[2];
+        } else if (ok) {
+            s.kind = Step::ATTENTION;
+            ok = PyArg_ParseTuple(t, "sKKKKKKKiiiii", &kind, &p[0], &p[1], &p[2], &p[3], &p[4], &p[5], &p[6], &s.B, &s.heads, &s.kv_heads,
+                                  &s.head_dim, &s.max_len);
+            s.qkv = (const void *)(uintptr_t)p[0];
+            s.kcache = (void *)(uintptr_t)p[1];
+            s.vcache = (void *)(uintptr_t)p[2];
+            s.cos = (const void *)(uintptr_t)p[3];
+            s.sin = (const void *)(uintptr_t)p[4];
+            s.pos = (const int64_t *)(uintptr_t)p[5];
+            s.out = (void *)(uintptr_t)p[6];
+        }
+        if (!ok || PyErr_Occurred()) {
+            delete steps;
+            if (!PyErr_Occurred()) PyErr_Format(PyExc_ValueError, "make_steps: item %zd is not a launch", j);
+            return nullptr;
+        }
+        steps->list.push_back(std::move(s));
+    }
+    return PyCapsule_New(steps, STEPS, free_steps);
+}
+
+// run_steps(handle, device index): every launch, in order, on the device's current stream
+PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 2) return PyErr_Format(PyExc_TypeError, "run_steps takes 2 arguments");
+    try {
+        Steps *steps = (Steps *)PyCapsule_GetPointer(a[0], STEPS);
+        int64_t index;
+        if (!steps || !int_arg(a[1], index)) return nullptr;
+        const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)index);
+        DeviceScope scope(dev);
+        const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+        at::Tensor ws = workspace_for(dev.index(), stream, steps->need);
+        for (const Step &s : steps->list) {
+            int st;
+            if (s.kind == Step::GROUP) {
+                const int count = (int)s.mats.size();
+                for (int turn = 0;; turn++) {
+                    st = s.rms ? bs_forward_group_rms(s.mats.data(), count, s.N, s.K, s.x, s.T, s.eps, s.epilogue, s.residual, s.y,
+                                                      ws.mutable_data_ptr(), ws.numel(), stream)
+                               : bs_forward_group(s.mats.data(), count, s.N, s.K, s.x, s.T, s.epilogue, s.residual, s.y,
+                                                  ws.mutable_data_ptr(), ws.numel(), stream);
+                    if (st != BS_ERR_WORKSPACE || turn > 0) break;
+                    // another kernel has been chosen since (bs_set_decode_kernel): its scratch may be larger
+                    const int64_t need = bs_forward_group_workspace_bytes(s.mats.data(), count, s.N, s.K, s.T);
+                    ws = workspace_for(dev.index(), stream, need);
+                }
+                if (st != BS_OK) return raise_status(st, "bs_forward_group");
+            } else if (s.kind == Step::NORM) {
+                st = bs_rmsnorm_f16(s.x, s.weight, s.y, s.T, s.N, s.eps, stream);
+                if (st != BS_OK) return raise_status(st, "bs_rmsnorm_f16");
+            } else {
+                st = bs_attention_decode_f16(s.qkv, s.kcache, s.vcache, s.cos, s.sin, s.pos, s.out, s.B, s.heads, s.kv_heads, s.head_dim,
+                                             s.max_len, stream);
+                if (st != BS_OK) return raise_status(st, "bs_attention_decode_f16");
+            }
+        }
+        Py_RETURN_NONE;
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// argmax(x [B, V], out int64 [B]) -> True, or None
+PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 2) return PyErr_Format(PyExc_TypeError, "argmax takes 2 arguments");
+    try {
+        const at::Tensor *x = tensor_arg(a[0]), *out = tensor_arg(a[1]);
+        if (!x || !out || !x->is_cuda() || x->dim() != 2) Py_RETURN_NONE;
+        const c10::Device dev = x->device();
+        if (!plain(*x, at::kHalf, dev) || !plain(*out, at::kLong, dev) || out->numel() != x->size(0) || x->numel() == 0 ||
+            x->size(0) >= INT32_MAX || x->size(1) >= INT32_MAX)
+            Py_RETURN_NONE;
+        DeviceScope scope(dev);
+        const int st = bs_argmax_f16(x->const_data_ptr(), (int64_t *)out->mutable_data_ptr(), (int)x->size(0), (int)x->size(1),
+                                     c10::hip::getCurrentHIPStream(dev.index()).stream());
+        if (st != BS_OK) return raise_status(st, "bs_argmax_f16");
+        Py_RETURN_TRUE;
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+#define HOST_METHOD(name) {#name, (PyCFunction)(void (*)(void))host_##name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(linear), HOST_METHOD(workspace),
+                         HOST_METHOD(argmax), HOST_METHOD(make_steps), HOST_METHOD(run_steps), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native host path over libbitstack_hip.so.", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }

@@ -28,6 +28,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from bitstack_amd import _lib
 from bitstack_amd.utils.pack_utils import pack_sign, unpack_sign, unpack_sign_hip
 from bitstack_amd.utils.inference_utils import (
     bitstack_forward_hip,
@@ -117,9 +118,10 @@ class BitStackLinear(nn.Module):
         return qlinear
 
     # ---------------------------------------------------------------- forward
-    @torch.no_grad()
     def forward(self, x):
         level = self.fused_level
+        if level == 5:
+            return self.forward_l5(x)
         if level == 0:
             return self.forward_l0(x)
         if level == 1:
@@ -130,8 +132,6 @@ class BitStackLinear(nn.Module):
             return self.forward_l3(x)
         if level == 4:
             return self.forward_l4(x)
-        if level == 5:
-            return self.forward_l5(x)
         raise ValueError(f"Invalid fused_level: {self.fused_level}")
 
     def _stacked(self):
@@ -166,20 +166,34 @@ class BitStackLinear(nn.Module):
         sign = unpack_sign_hip(q.reshape(-1), torch.Size([self.w_bit, self.out_features, self.in_features]))
         return F.linear(x, reconstruct_w_hip(sign, u, vt), bias=self.bias)
 
+    def _rebuilt(self):
+        """The weight from the first w_bit stacked blocks: one native call where they lie as stack_blocks() left them."""
+        d = self.__dict__
+        if d.get("u") is not None and not self.no_avd:
+            w = _lib.host().rebuild(d.get("qweight"), d["u"], d.get("vt"), self.w_bit)
+            if w is not None:
+                return w
+        q, u, vt = self._stacked()
+        return unpack_and_reconstruct_w_hip(q, u, vt)
+
     @torch.no_grad()
     def forward_l3(self, x):
-        q, u, vt = self._stacked()
-        return F.linear(x, unpack_and_reconstruct_w_hip(q, u, vt), bias=self.bias)
+        return F.linear(x, self._rebuilt(), bias=self.bias)
 
     @torch.no_grad()
     def forward_l4(self, x):
-        q, u, vt = self._stacked()
-        return linear_f16_hip(x, unpack_and_reconstruct_w_hip(q, u, vt), self.bias)
+        return linear_f16_hip(x, self._rebuilt(), self.bias)
 
-    @torch.no_grad()
     def forward_l5(self, x):
-        q, u, vt = self._stacked()
-        return bitstack_forward_hip(q, u, vt, x, self.bias)
+        # (the native call records nothing for autograd; only the ordinary layout is taken there, None = not this one)
+        d = self.__dict__
+        if d.get("u") is not None and not self.no_avd:
+            y = _lib.host().forward(d.get("qweight"), d["u"], d.get("vt"), self.w_bit, x, self.bias)
+            if y is not None:
+                return y
+        with torch.no_grad():
+            q, u, vt = self._stacked()
+            return bitstack_forward_hip(q, u, vt, x, self.bias)
 
     # ------------------------------------------------------------ bookkeeping
     def memory_per_bit(self):

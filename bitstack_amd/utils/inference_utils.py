@@ -40,6 +40,9 @@ def reconstruct_w_hip(sign, u, vt):
 def unpack_and_reconstruct_w_hip(packed_sign, u, vt):
     """(sign * u @ vt).sum(0) straight from packed signs [I, M*N/8]
     (unpack_and_reconstruct_w_triton and _v2, inference_utils.py:371-387, :465-488)."""
+    w = _lib.host().rebuild(packed_sign, u, vt, u.shape[0])
+    if w is not None:
+        return w
     dev = _lib.require_gpu(packed_sign, u, vt)
     I, M, N, K = _dims(u, vt)
     if packed_sign.dtype != torch.uint8 or packed_sign.numel() != I * ((M * N + 7) // 8):
@@ -58,6 +61,9 @@ def bitstack_forward_hip(packed_sign, u, vt, x, bias=None):
     """y = x @ (sum_i sign_i * u_i @ vt_i)^T (+ bias) from packed signs; x is
     [..., N] fp16 (reconstruct_and_forward_triton, inference_utils.py:252-284,
     generalised to packed input, any leading shape and an optional bias)."""
+    y = _lib.host().forward(packed_sign, u, vt, u.shape[0], x, bias)
+    if y is not None:
+        return y
     dev = _lib.require_gpu(packed_sign, u, vt, x, bias)
     I, M, N, K = _dims(u, vt)
     if x.shape[-1] != N:
@@ -200,6 +206,8 @@ def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, ou
 
 def argmax_hip(x, out=None):
     """Index of the largest value of every row of x [B, V] (fp16), int64 [B]."""
+    if out is not None and _lib.host().argmax(x, out):
+        return out
     dev = _lib.require_gpu(x, out)
     if x.dim() != 2 or x.dtype != torch.float16 or not x.is_contiguous():
         raise ValueError("x must be a contiguous fp16 [B, V] tensor")
@@ -214,6 +222,9 @@ def argmax_hip(x, out=None):
 
 def linear_f16_hip(x, w, bias=None):
     """F.linear on the library's own MFMA kernel (fp16 in, fp32 accumulate)."""
+    y = _lib.host().linear(x, w, bias)
+    if y is not None:
+        return y
     dev = _lib.require_gpu(x, w, bias)
     M, N = w.shape
     x2, w = _f16c(x).view(-1, N), _f16c(w)

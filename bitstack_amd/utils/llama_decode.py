@@ -14,16 +14,17 @@ a HIP graph and replayed.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
 
+from bitstack_amd import _lib
 from bitstack_amd._lib import EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU
 from bitstack_amd.modules.BitStackLinear import BitStackLinear
-from bitstack_amd.utils.inference_utils import (MatrixGroup, argmax_hip, attention_decode_hip,
-                                                bitstack_forward_group_hip, rmsnorm_hip)
+from bitstack_amd.utils.inference_utils import MatrixGroup, argmax_hip, rmsnorm_hip
 
 PROJ = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj",
         "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj")
@@ -171,6 +172,7 @@ class SyntheticLlamaDecoder:
         self.span = torch.arange(max_len, device=self.dev)
         self.logits = None
         self._groups = None
+        self._steps = None                                                 # (addresses it was made for, launch list)
 
     @classmethod
     def from_checkpoint(cls, path, max_len, device, compression_config=None, niter=None, max_memory_MB=None, batch=1):
@@ -349,6 +351,7 @@ class SyntheticLlamaDecoder:
         launch itself, so the fused step has no RMSNorm kernel inside a layer."""
         s, B = self.s, self.batch
         self._groups = []
+        self._steps = None
 
         def folded(mods, weight):
             mats = []
@@ -373,23 +376,47 @@ class SyntheticLlamaDecoder:
         self._xa = torch.empty(B, s.hidden, **f16)
         self._xb = torch.empty(B, s.hidden, **f16)
 
-    @torch.no_grad()
-    def step_fused(self):
-        """Same step on the library's grouped forwards and decode-step kernels."""
+    def _launches(self):
+        """The launches of step_fused() between the embedding and the last norm as one native list (host.cpp), laid
+        out once: their arguments only change when the groups are rebuilt or a cache or table is replaced."""
         if self._groups is None:
             self._build_groups()
-        s = self.s
-        xa, xb = self._xa, self._xb
-        torch.index_select(self.embed, 0, self.token, out=xa)
-        for L in range(s.layers):
-            grp = self._groups[L]
-            bitstack_forward_group_hip(grp["qkv"], xa, EPI_NONE, out=self._qkv, rms_eps=s.rms_eps)
-            attention_decode_hip(self._qkv, self.kcache[L], self.vcache[L], self.cos, self.sin, self.pos,
-                                 s.heads, s.kv_heads, out=self._ctx)
-            bitstack_forward_group_hip(grp["o"], self._ctx, EPI_RESIDUAL, residual=xa, out=xb)
-            bitstack_forward_group_hip(grp["gate_up"], xb, EPI_SWIGLU, out=self._act, rms_eps=s.rms_eps)
-            bitstack_forward_group_hip(grp["down"], self._act, EPI_RESIDUAL, residual=xb, out=xa)
-        rmsnorm_hip(xa, self.final_norm, s.rms_eps, out=self._hn)
+        held = (self.kcache, self.vcache, self.cos, self.sin, self.pos)
+        key = tuple(t.data_ptr() for t in held)
+        if self._steps is not None and self._steps[0] == key:
+            return self._steps[1]
+        s, B = self.s, self.batch
+        d = s.head_dim
+        for t, shape, dtype in ((self.kcache, (s.layers, B, s.kv_heads, self.max_len, d), torch.float16),
+                                (self.vcache, (s.layers, B, s.kv_heads, self.max_len, d), torch.float16),
+                                (self.cos, (self.max_len, d // 2), torch.float16), (self.sin, (self.max_len, d // 2), torch.float16),
+                                (self.pos, (1,), torch.int64)):
+            if tuple(t.shape) != shape or t.dtype != dtype or not t.is_contiguous() or not t.is_cuda:
+                raise ValueError(f"the decode step needs a contiguous {dtype} tensor {shape} on the GPU, got {t.dtype} {tuple(t.shape)}")
+        xa, xb, qkv, ctx, act = (t.data_ptr() for t in (self._xa, self._xb, self._qkv, self._ctx, self._act))
+
+        def group(g, x, y, epilogue, eps=None, residual=0):
+            return ("group", ctypes.addressof(g.arr), g.n, g.N, g.K, x, B, eps, epilogue, residual, y)
+
+        items = []
+        for L, grp in enumerate(self._groups):
+            items.append(group(grp["qkv"], xa, qkv, EPI_NONE, eps=s.rms_eps))
+            items.append(("attention", qkv, self.kcache[L].data_ptr(), self.vcache[L].data_ptr(), self.cos.data_ptr(), self.sin.data_ptr(),
+                          self.pos.data_ptr(), ctx, B, s.heads, s.kv_heads, d, self.max_len))
+            items.append(group(grp["o"], ctx, xb, EPI_RESIDUAL, residual=xa))
+            items.append(group(grp["gate_up"], xb, act, EPI_SWIGLU, eps=s.rms_eps))
+            items.append(group(grp["down"], act, xa, EPI_RESIDUAL, residual=xb))
+        items.append(("norm", xa, self.final_norm.data_ptr(), self._hn.data_ptr(), B, s.hidden, s.rms_eps))
+        self._steps = (key, _lib.host().make_steps(items))
+        return self._steps[1]
+
+    @torch.no_grad()
+    def step_fused(self):
+        """Same step on the library's grouped forwards and decode-step kernels: q/k/v with the RMSNorm in front, attention,
+        o + residual, gate/up with the RMSNorm in front and the SiLU product, down + residual per layer."""
+        launches = self._launches()
+        torch.index_select(self.embed, 0, self.token, out=self._xa)
+        _lib.host().run_steps(launches, self._xa.device.index)
         self.logits = F.linear(self._hn, self.lm_head)
         argmax_hip(self.logits, out=self.token)
         self.pos.add_(1)

@@ -1,0 +1,65 @@
+"""The native host path (csrc/host.cpp) and the Python path behind it give the same results, and each call
+that is not the ordinary case is left to the Python path."""
+import pytest
+import torch
+
+from bitstack_amd import BitStackLinear, _lib
+from bitstack_amd.utils import inference_utils as IU
+from bitstack_amd.utils.synthetic import synthetic_layer
+
+
+def layer(I, M, N, T, dev, bias=True):
+    q, u, vt, x = synthetic_layer(M, N, I, T, seed=I + T, device=dev)
+    mod = BitStackLinear(0, N, M, 16, False, False, dev, fused_level=5)
+    mod.w_bit, mod.qweight, mod.u, mod.vt = I, q, u, vt
+    if bias:
+        mod.bias = (torch.randn(M, generator=torch.Generator().manual_seed(3)) * 0.1).half().to(dev)
+    return mod, x
+
+
+def test_unusual_arguments_are_left_to_python():
+    mod, x = layer(2, 16, 64, 3, "cpu")
+    H = _lib.host()
+    assert H.forward(mod.qweight, mod.u, mod.vt, 2, x, mod.bias) is None          # CPU tensors
+    assert H.rebuild(mod.qweight, mod.u, mod.vt, 2) is None
+    assert H.linear(x, x, None) is None
+    assert H.forward(None, None, None, 2, x, None) is None
+    with pytest.raises(RuntimeError, match="HIP device"):
+        mod(x)
+    with pytest.raises(TypeError):
+        H.forward(mod.qweight)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,T", [(1, 16, 512, 2), (3, 200, 1024, 5), (2, 100, 72, 3), (3, 256, 512, 130)])
+def test_native_and_python_paths_agree(I, M, N, T):
+    mod, x = layer(I, M, N, T, torch.device("cuda"))
+    H = _lib.host()
+    x3 = x.view(1, T, N).requires_grad_()
+    y = mod(x3)
+    assert y.shape == (1, T, M) and not y.requires_grad
+    assert H.forward(mod.qweight, mod.u, mod.vt, I, x, mod.bias) is not None
+    # the same call through a layout that only the Python path takes (columns of a wider tensor)
+    wide = torch.zeros(T, N + 8, dtype=torch.float16, device=x.device)
+    wide[:, :N] = x
+    assert H.forward(mod.qweight, mod.u, mod.vt, I, wide[:, :N], mod.bias) is None
+    assert torch.equal(y[0], IU.bitstack_forward_hip(mod.qweight, mod.u, mod.vt, wide[:, :N], mod.bias))
+    # fewer blocks than are stacked
+    mod.set_bit(1)
+    assert torch.equal(mod(x), IU.bitstack_forward_hip(mod.qweight[:1], mod.u[:1], mod.vt[:1], x, mod.bias))
+    mod.set_bit(I)
+    w = IU.unpack_and_reconstruct_w_hip(mod.qweight, mod.u, mod.vt)
+    assert torch.equal(w, mod._rebuilt())
+    assert torch.equal(IU.linear_f16_hip(x, w), IU.linear_f16_hip(wide[:, :N], w))
+
+
+@pytest.mark.gpu
+def test_scratch_is_one_tensor_per_stream_and_outgrown_ones_stay():
+    dev = torch.device("cuda")
+    a = _lib.workspace(dev, 1 << 20)
+    assert _lib.workspace(dev, 1000).data_ptr() == a.data_ptr()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        b = _lib.workspace(dev, 1000)
+        assert b.data_ptr() != a.data_ptr()
+    big = _lib.workspace(dev, 2 * a.numel() + 1)
+    assert big.numel() > 2 * a.numel() and big.data_ptr() != a.data_ptr()

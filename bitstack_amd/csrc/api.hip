@@ -1,6 +1,7 @@
 // C ABI glue: argument validation, path selection, status strings.
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 
 extern "C" int bs_version(void) { return BS_VERSION_NUMBER; }
@@ -63,8 +64,9 @@ static int64_t workspace_need(int I, int M, int N, int K, int T, bool library_ok
     if (T == 0) return 0;
     int64_t gemv = bs_gemv_workspace_bytes(I, M, N, K, T);
     if (gemv > 0) return round_up(gemv, 256);
-    // the rebuilt weight, then the library GEMM's own scratch where that is the kernel
-    return round_up((int64_t)M * N * 2, 256) + (library_ok && dense_wants_library(M, N) ? BS_DENSE_LIBRARY_WORKSPACE : 0);
+    // the rebuilt weight, then the library GEMM's own scratch where that is the kernel, or the product's partial sums
+    const bool library = library_ok && dense_wants_library(M, N);
+    return round_up((int64_t)M * N * 2, 256) + round_up(std::max(library ? BS_DENSE_LIBRARY_WORKSPACE : 0, bs_linear_parts_bytes(T, M, N)), 256);
 }
 
 extern "C" int64_t bs_workspace_bytes(int I, int M, int N, int K, int T) { return workspace_need(I, M, N, K, T, true); }
@@ -122,7 +124,8 @@ static int forward_impl(const uint8_t *packed, const void *u, const void *vt, co
                                       (char *)workspace + round_up((int64_t)M * N * 2, 256), s);
         if (st != BS_ERR_SHAPE) return st;      // enqueued, or failed for good; BS_ERR_SHAPE: declined before anything was enqueued
     }
-    return bs_launch_linear_f16((const half_t *)x, w, (const half_t *)bias, (half_t *)y, T, M, N, s);
+    return bs_launch_linear_parts((const half_t *)x, w, (const half_t *)bias, (half_t *)y, T, M, N,
+                                  (float *)((char *)workspace + round_up((int64_t)M * N * 2, 256)), s);
 }
 
 extern "C" int bs_forward(const uint8_t *packed, const void *u, const void *vt, const void *x,

@@ -61,6 +61,13 @@ int bs_launch_reconstruct_packed(const uint8_t *packed, const half_t *u, const h
                                  half_t *w, int I, int M, int N, int K, hipStream_t s);
 int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, half_t *y,
                          int T, int M, int N, hipStream_t s);
+// the large tiles with N % 64 == 0 (gemm_pipe.hip), bt x bf tokens x features per workgroup; splits > 1: the contracted
+// range in that many parts, part[splits][T][M] floats of scratch
+int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int bt, int bf,
+                          int splits, float *part, hipStream_t s);
+// the product behind a rebuilt weight (16-byte aligned x and w): tile and parts by shape, bs_linear_parts_bytes of scratch
+int64_t bs_linear_parts_bytes(int T, int M, int N);
+int bs_launch_linear_parts(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, float *part, hipStream_t s);
 // the same product through hipBLASLt (dense_lt.hip); BS_ERR_SHAPE = not available for this call
 constexpr int64_t BS_DENSE_LIBRARY_WORKSPACE = 64 << 20;
 int bs_launch_linear_library(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N,

@@ -5,19 +5,16 @@
 // row (A = tokens) or one column (B = features), i.e. one 16-byte read per
 // fragment.
 //
-// More than 128 tokens: linear_f16_kernel, WT x WF waves of AT x AF MFMA tiles each,
-// k-steps of GK columns through two LDS buffers; rows are padded by 8 halves so that
-// the lanes served per LDS cycle hit disjoint banks.  Four shapes are instantiated:
-// 256 x 256 (8 waves of 128 x 64; GK = 64 with two register sets of pieces in flight when N % 64 == 0 - a row's 128
-// bytes of a k-step are one cache line, fetched once; GK = 32 took every line from L2 twice, the halves a step apart and
-// the L1 too small to keep them - else GK = 32 with three sets) and 128 x 256 (8 waves of 64 x 64) for
-// grids that cover the chip, 128 x 128 and 64 x 64 (4 waves, two workgroups per CU,
-// the latter with GK = 128: half as many barriers) for the smaller ones; the launcher
-// takes the largest tile whose grid still has about 160 workgroups.
+// Above 128 tokens and with N a multiple of 64, tiles of 128 x 128 and more are gemm_pipe.hip's; this file holds the
+// others and the choice.  linear_f16_kernel: WT x WF waves of AT x AF MFMA tiles each, k-steps of GK columns through two
+// LDS buffers; rows are padded by 8 halves so that the lanes served per LDS cycle hit disjoint banks.  Four shapes:
+// 256 x 256 (8 waves of 128 x 64, GK = 32, three register sets of pieces in flight), 128 x 256 (8 waves of 64 x 64) and
+// 128 x 128 (4 waves) for N % 64 != 0, and 64 x 64 (4 waves, two workgroups per CU, GK = 128: half as many barriers) for
+// problems too small to fill the chip with anything larger.
 // The loop is software-pipelined at three levels, all through registers:
 //   - global requests run NS k-steps ahead through NS register sets (four where the registers allow it: the
 //     kernel waits for requests more than for anything else, and a fourth set is worth 3 to 13 %; five and six were
-//     no better; two for the 256 x 256 tile in k-steps of 64), all of them unconditional buffer loads: descriptor,
+//     no better), all of them unconditional buffer loads: descriptor,
 //     32-bit lane offset, scalar k offset;
 //   - the LDS writes of step s + 1 and the requests of step s + NS are cut into one
 //     portion per MFMA group instead of one burst per step;
@@ -184,7 +181,6 @@ __global__ __launch_bounds__(64 * WT * WF) void linear_f16_kernel(
     // the next one, so it can be written all along the step.
     using PF = std::integral_constant<int, NK>;
     using PS = std::integral_constant<int, NK - 1>;
-    using S2 = std::integral_constant<int, 2>;
     auto one_step = [&](auto cur, auto nxt, auto bufc, int step) {
         constexpr int buf = decltype(bufc)::value;
         static_for<NK / 2>([&](auto hc) {
@@ -328,48 +324,115 @@ __global__ __launch_bounds__(256) void linear_generic_kernel(
     }
 }
 
-// NS: register sets of pieces in flight.  TAILS: also instantiate the kernel for a contracted range that ends in a partial
-// k-step (false: the caller only comes with N % GK == 0).
-template <int WT, int WF, int AT, int AF, int GK, int NS = 3, bool TAILS = true>
+// NS: register sets of pieces in flight.  WHOLE: also instantiate the kernel for a contracted range without a partial last
+// k-step (false: the caller only comes with N % GK != 0).
+template <int WT, int WF, int AT, int AF, int GK, int NS = 3, bool WHOLE = true>
 int launch_tiled(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N,
                  hipStream_t s) {
     constexpr int BT = WT * AT * 32, BF = WF * AF * 32;
     constexpr size_t lds = (size_t)2 * (BT + BF) * lds_stride(GK) * sizeof(half_t);
     static bs_lds_grant granted[2][BS_MAX_DEVICES];
-    int st = bs_allow_lds((const void *)linear_f16_kernel<WT, WF, AT, AF, GK, false, NS>, lds, granted[0]);
-    if constexpr (TAILS) {
-        if (st == BS_OK) st = bs_allow_lds((const void *)linear_f16_kernel<WT, WF, AT, AF, GK, true, NS>, lds, granted[1]);
+    const dim3 grid((unsigned)bs_cdiv(M, BF), (unsigned)bs_cdiv(T, BT));
+    if (N % GK != 0) {
+        const int st = bs_allow_lds((const void *)linear_f16_kernel<WT, WF, AT, AF, GK, true, NS>, lds, granted[1]);
+        if (st != BS_OK) return st;
+        linear_f16_kernel<WT, WF, AT, AF, GK, true, NS><<<grid, 64 * WT * WF, lds, s>>>(x, w, bias, y, T, M, N);
+        return BS_OK;
     }
-    if (st != BS_OK) return st;
-    dim3 grid((unsigned)bs_cdiv(M, BF), (unsigned)bs_cdiv(T, BT));
-    if (N % GK == 0) {
+    if constexpr (WHOLE) {
+        const int st = bs_allow_lds((const void *)linear_f16_kernel<WT, WF, AT, AF, GK, false, NS>, lds, granted[0]);
+        if (st != BS_OK) return st;
         linear_f16_kernel<WT, WF, AT, AF, GK, false, NS><<<grid, 64 * WT * WF, lds, s>>>(x, w, bias, y, T, M, N);
-    } else {
-        if constexpr (TAILS)
-            linear_f16_kernel<WT, WF, AT, AF, GK, true, NS><<<grid, 64 * WT * WF, lds, s>>>(x, w, bias, y, T, M, N);
-        else
-            return BS_ERR_SHAPE;
+        return BS_OK;
     }
-    return BS_OK;
+    return BS_ERR_SHAPE;
 }
 
 }  // namespace
 
-// Which kernel a dense forward of these dimensions runs: tokens x features per workgroup
-// (0 x 0 for the one-wave-per-output kernel), and whether the contracted range ends in a
-// partial k-step.
+// Which kernel bs_linear_f16 runs for these dimensions: tokens x features per workgroup (0 x 0 for the
+// one-wave-per-output kernel), and whether the contracted range ends in a partial k-step.
 struct LinearTile { int bt, bf, gk; };
 static LinearTile linear_tile(int T, int M, int N, bool aligned) {
     if (!(N % 8 == 0 && aligned) || N >= (1 << 23)) return {0, 0, 0};     // (a tile's rows stay within 32-bit byte offsets)
     if (T <= 32 && N % 16 == 0) return {32, 32, 0};                       // linear_skinny_kernel
     if (T <= 128) return M >= 8192 ? LinearTile{128, 64, 64} : LinearTile{128, 32, 128};
     // The largest tile whose grid still covers most of the 256 CUs: 256 x 256 and
-    // 128 x 256 (8 waves) move the fewest bytes per flop; 128 x 128 and 64 x 64
-    // (4 waves, two workgroups per CU) keep a small problem spread over the chip.
+    // 128 x 256 move the fewest bytes per flop; 128 x 128 and 64 x 64
+    // keep a small problem spread over the chip.
     const auto wgs = [&](int bt, int bf) { return bs_cdiv(T, bt) * bs_cdiv(M, bf); };
     return wgs(256, 256) >= 160 ? LinearTile{256, 256, N % 64 == 0 ? 64 : 32} :
            wgs(128, 256) >= 160 ? LinearTile{128, 256, 64} :
            wgs(128, 128) >= 160 ? LinearTile{128, 128, 64} : LinearTile{64, 64, 128};
+}
+
+// The tile behind a rebuilt weight, where scratch for partial sums can be had too.  splits > 1: the contracted range is
+// cut into that many parts, whose sums a second kernel adds up: a few tokens on a large weight are a handful of large
+// tiles, which leave most of the chip idle, or many small ones, which move the most bytes per flop (509 tokens on
+// 4096 x 14336: 114 us with 64 x 64 tiles, 68 with 32 tiles of 256 x 256 in 8 parts each).
+struct LinearChoice { int bt, bf, splits; };      // bt == 0: as bs_linear_f16
+
+// Time in us that a tile of gemm_pipe.hip (64 x 64: linear_f16_kernel) is expected to take: rounds of workgroups over the
+// chip x k-steps of 64 columns x the time of one, which is shorter while part of the chip is idle (power), plus the sums.
+// The constants are a fit to 900 timings of 57 (tokens, M, N) from 20 x 4096 x 14336 to 16384 x 28672 x 8192; over those
+// the choice made with them is within 1 % of the best one on average, within 4 % on each.
+static double linear_cost(int bt, int bf, int splits, int T, int M, int N) {
+    const int a = bt > bf ? bt : bf, b = bt > bf ? bf : bt;
+    const double step = a == 256 ? (b == 256 ? 1.50 : b == 192 ? 1.14 : 0.95) : a == 192 ? 0.80 : b == 128 ? 0.96 : a == 128 ? 0.735 : 0.47;
+    const int64_t all = bs_cdiv(N, 64), steps = bs_cdiv(all, splits), parts = bs_cdiv(all, steps);
+    const int64_t wg = bs_cdiv(T, bt) * bs_cdiv(M, bf) * parts;
+    const int64_t slots = a <= 128 ? 512 : 256;   // (two workgroups of the small tiles share a CU)
+    const int64_t rounds = bs_cdiv(wg, slots);
+    const double idle = 1.0 - (double)wg / (double)(rounds * slots);
+    double us = rounds * steps * step * (slots == 512 && wg <= 256 ? 0.78 : 1.0) * (1.0 - 0.35 * idle / rounds) + 2.0;
+    if (parts > 1) us += 4.7 + 8e-6 * parts * T * M / 6.0;
+    return us;
+}
+
+static LinearChoice linear_choice(int T, int M, int N) {
+    if (N % 64 != 0 || N >= (1 << 23)) return {0, 0, 1};
+    // Partial sums only behind a weight that is beyond the static scratch by itself (a call that fits the static scratch
+    // is never refused, or run differently, for their sake; smaller weights gain little), never more of them than weight,
+    // and where a row of y can be written 16 bytes at a time.
+    const int64_t weight = (int64_t)M * N * 2;
+    const bool may_split = weight > (int64_t)BS_STATIC_SCRATCH_BYTES && M % 8 == 0;
+    if (T <= 128 && !may_split) return {0, 0, 1};
+    static const int tiles[][2] = {{256, 256}, {192, 256}, {256, 192}, {256, 128}, {128, 256}, {192, 128}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};
+    static const int cuts[] = {2, 3, 4, 6, 8, 12};
+    LinearChoice one = {0, 0, 1}, cut = {0, 0, 1};
+    double one_us = 1e30, cut_us = 1e30;
+    for (const auto &t : tiles) {
+        if (T > 128) {
+            const double us = linear_cost(t[0], t[1], 1, T, M, N);
+            if (us < one_us) one_us = us, one = {t[0], t[1], 1};
+        }
+        if (!may_split || t[1] == 64) continue;
+        for (int c : cuts) {
+            if ((int64_t)c * T * M * 4 > weight) break;
+            const double us = linear_cost(t[0], t[1], c, T, M, N);
+            if (us < cut_us) cut_us = us, cut = {t[0], t[1], c};
+        }
+    }
+    if (cut_us < 0.93 * one_us) return cut;       // (the estimate has to be clear: a second kernel and its traffic are certain)
+    return one.bf == 64 ? LinearChoice{0, 0, 1} : one;
+}
+// (asked for the scratch, then for the launch: the last answer of the thread is kept)
+static LinearChoice linear_choice_kept(int T, int M, int N) {
+    static thread_local int kT = 0, kM = 0, kN = 0;
+    static thread_local LinearChoice kept = {0, 0, 1};
+    if (T != kT || M != kM || N != kN) kept = linear_choice(T, M, N), kT = T, kM = M, kN = N;
+    return kept;
+}
+
+int64_t bs_linear_parts_bytes(int T, int M, int N) {
+    const LinearChoice c = linear_choice_kept(T, M, N);
+    return c.splits > 1 ? (int64_t)c.splits * T * M * 4 : 0;
+}
+
+int bs_launch_linear_parts(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, float *part, hipStream_t s) {
+    const LinearChoice c = linear_choice_kept(T, M, N);
+    if (c.bt == 0) return bs_launch_linear_f16(x, w, bias, y, T, M, N, s);
+    return bs_launch_linear_pipe(x, w, bias, y, T, M, N, c.bt, c.bf, c.splits, part, s);
 }
 
 int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, half_t *y,
@@ -382,18 +445,18 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
         linear_generic_kernel<<<(int)blocks, 256, 0, s>>>(x, w, bias, y, T, M, N);
     } else if (tile.gk == 0) {
         linear_skinny_kernel<1, 8, 8><<<(int)bs_cdiv(M, 32), 512, 0, s>>>(x, w, bias, y, T, M, N);
+    } else if (tile.bf >= 128 && N % 64 == 0) {
+        return bs_launch_linear_pipe(x, w, bias, y, T, M, N, tile.bt, tile.bf, 1, nullptr, s);
     } else if (tile.bt == 128 && tile.bf == 64) {
         st = launch_tiled<2, 2, 2, 1, 64>(x, w, bias, y, T, M, N, s);
     } else if (tile.bt == 128 && tile.bf == 32) {
         st = launch_tiled<4, 1, 1, 1, 128>(x, w, bias, y, T, M, N, s);
-    } else if (tile.bt == 256 && tile.gk == 64) {
-        st = launch_tiled<2, 4, 4, 2, 64, 2, false>(x, w, bias, y, T, M, N, s);
     } else if (tile.bt == 256) {
         st = launch_tiled<2, 4, 4, 2, 32>(x, w, bias, y, T, M, N, s);
     } else if (tile.bf == 256) {
-        st = launch_tiled<2, 4, 2, 2, 64, 4>(x, w, bias, y, T, M, N, s);
+        st = launch_tiled<2, 4, 2, 2, 64, 4, false>(x, w, bias, y, T, M, N, s);
     } else if (tile.bf == 128) {
-        st = launch_tiled<2, 2, 2, 2, 64, 4>(x, w, bias, y, T, M, N, s);
+        st = launch_tiled<2, 2, 2, 2, 64, 4, false>(x, w, bias, y, T, M, N, s);
     } else {
         st = launch_tiled<2, 2, 1, 1, 128, 4>(x, w, bias, y, T, M, N, s);
     }

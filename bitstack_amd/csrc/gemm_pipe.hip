@@ -1,0 +1,390 @@
+// The dense product's large tiles on gfx950: y[T, M] = x[T, N] @ w[M, N]^T (+ bias), fp16 in, fp32 accumulation, N % 64 == 0.
+//
+// A workgroup of 8 waves owns 64 AP rows of one operand ("P") x 128 AQ rows of the other ("Q") - tokens x features, or
+// (SWAP) features x tokens - and walks N in k-steps of 64 columns (one 128-byte line of every row).  Three things
+// distinguish it from linear_f16_kernel:
+//   - requests write LDS directly (16 bytes per lane): no registers hold pieces on their way and there are no LDS write
+//     instructions;
+//   - the two waves of every SIMD work in turns.  Waves 0-3 own the upper half of the P rows, waves 4-7 the lower
+//     half; a k-step of a wave is a MEMORY phase (all its fragments from LDS into registers) and a MATRIX phase (all its
+//     MFMAs), with a barrier behind each, and the lower half runs one phase behind: while one wave of a SIMD
+//     multiplies, the other one fetches;
+//   - v_mfma_f32_16x16x32_f16 instead of 32x32x16: the same rate per cycle, but under load this part is limited by
+//     power, and the smaller form (half the accumulator traffic per product) runs at a higher clock - 1.92 against
+//     1.71 GHz in a loop of MFMAs alone, 1.63 against 1.51 GHz in this kernel.
+// Measured with random data: 8192 x 8192 x 8192 767 us = 1.43 PFLOP/s (linear_f16_kernel's 256 x 256 tile 883 to 911 us,
+// torch's library 711), 16384 x 28672 x 8192 5.38 ms = 1.43 PFLOP/s (6.9 ms; 5.05), 2048 x 14336 x 4096 187 us (222; 179).
+// What bounds it: 2560 cycles per k-step of a 256 x 256 tile against 2048 of matrix time (the hand-over of the matrix pipe
+// at the two barriers and the issue of the requests), at the clock the power allows.  Measured and not kept: the last MFMAs
+// of a phase behind its barrier (841 against 811 us on 8192^3), requests in the MEMORY phases only (916), a single barrier
+// per k-step with both waves multiplying at once (846), four waves of 128 x 128 with three fragment sets (870).
+//
+// Phases are numbered on the wall: the upper half runs MEMORY(s) in phase 2 s and MATRIX(s) in phase 2 s + 1, the lower half
+// one later.  Stage s & 1 holds step s.  The upper P rows of a stage are read in phase 2 s only, the lower ones in
+// phase 2 s + 1 only, the Q rows in both; so the requests for step s + 2 go out
+//     upper P rows   by the upper waves in phase 2 s + 1 (their MATRIX(s))
+//     lower P rows   by the lower waves in phase 2 s + 2 (their MATRIX(s))
+//     Q rows         half by the lower waves in phase 2 s + 2, half by the upper waves in phase 2 s + 2 (their MEMORY(s + 1))
+// and are read from phase 2 s + 4 (2 s + 5) on: about two phases cover a request.  A wave waits for ITS requests of a
+// step (a counted wait: later ones stay in flight) in front of the barrier that opens the phase in which somebody reads them.
+//
+// LDS rows are 128 bytes without padding (a request writes 64 lanes x 16 bytes contiguously); the eight 16-byte pieces of a
+// row are XOR-ed with three bits of the row number, chosen so that the 16 lanes LDS serves together in a 16-byte read
+// (0-3, 12-15, 20-27 and so on) hit all 64 banks; the lane that requests a piece picks its column accordingly.
+// A features fragment takes rows 8 (i / 4) + i % 4 of its 32 features (+ 4 for the other fragment of the pair) as its
+// row i: a lane then ends with EIGHT consecutive features of one token, one 16-byte store.
+#include "common.h"
+
+#include <type_traits>
+#include <utility>
+
+namespace {
+
+template <class F, int... Is>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+constexpr int PK = 64;                        // columns per k-step
+typedef __attribute__((address_space(3))) void *lds_ptr;
+
+// wait until at most `n` of this wave's requests are in flight (the LDS counter is not waited for)
+template <int n>
+__device__ __forceinline__ void wait_requests() {
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// wait until this wave's LDS reads have arrived
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (0 << 8)); }
+
+__device__ __forceinline__ void phase_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// SPLIT: the contracted range is cut into parts of `steps_per_split` k-steps; part p of every tile goes to part[p][T][M] in
+// fp32, linear_split_sum_kernel adds them up.
+// wide: M % 8 == 0 and y (part) 16-byte aligned: whole 16-byte stores.  Otherwise the outputs of y pass through LDS, so that a
+// store instruction still writes whole runs of a row.
+template <int AP, int AQ, bool SWAP, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
+    const half_t *__restrict__ x, const half_t *__restrict__ w, const half_t *__restrict__ bias,
+    half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide) {
+    constexpr int BP = 64 * AP, BQ = 128 * AQ;
+    constexpr int BT = SWAP ? BQ : BP, BF = SWAP ? BP : BQ;
+    constexpr int QJ = 2 * AQ;                // Q requests per wave and k-step (8 rows each); AP of P
+    constexpr int P = 2 * AP, Q = 2 * AQ;     // 16-row fragments of a wave
+    // one array per operand and stage: the compiler then knows that a request for one stage does not touch the other
+    __shared__ __attribute__((aligned(1024))) half_t sp0[BP * PK], sp1[BP * PK], sq0[BQ * PK], sq1[BQ * PK];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wp = wave >> 2, wq = wave & 3;
+    const int lm = lane & 15, g = lane >> 4;
+
+    // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2: every XCD gets a contiguous run of (split,
+    // tile) slots, tiles ordered so that those in flight on it at a time form a compact block (TGROUP token tiles x
+    // consecutive feature tiles: 12 tile rows and columns in L2 for 32 tiles instead of 33; 16384 x 28672 x 8192 6.9 -> 6.1 ms
+    // from this alone).
+    int t0, m0, sp = 0;
+    {
+        const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, base = nb >> 3, rem = nb & 7;
+        int v = xcd * base + min(xcd, rem) + loc;
+        constexpr int TGROUP = 4;
+        const int tt = (T + BT - 1) / BT, ft = (M + BF - 1) / BF;
+        if (SPLIT) {
+            sp = v / (tt * ft);
+            v -= sp * (tt * ft);
+        }
+        const int grp = v / (TGROUP * ft), r = v - grp * TGROUP * ft, gs = min(TGROUP, tt - grp * TGROUP);
+        m0 = (r / gs) * BF;
+        t0 = (grp * TGROUP + r % gs) * BT;
+    }
+    const int all_steps = N / PK;
+    const int s_begin = SPLIT ? sp * steps_per_split : 0;
+    const int steps = SPLIT ? min(steps_per_split, all_steps - s_begin) : all_steps;
+
+    const half_t *xo = x + (int64_t)t0 * N + (int64_t)s_begin * PK, *wo = w + (int64_t)m0 * N + (int64_t)s_begin * PK;
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(SWAP ? wo : xo), 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(SWAP ? xo : wo), 0, -1, 0x00020000);
+    // three bits of the row number that its pieces are XOR-ed with: for whole runs of 16 rows (tokens), and for the rows a
+    // features fragment takes
+    auto swizzle = [](bool features, int r) { return features ? ((r >> 1) & 1) | (((r >> 3) & 3) << 1) : (r >> 1) & 7; };
+    // request j of this wave: 8 rows x 128 bytes; rows beyond T or M repeat the last one (their outputs are never stored)
+    const int prow = (wp * 4 + wq) * AP * 8, qrow = wave * QJ * 8;
+    const int p_last = SWAP ? M - 1 - m0 : T - 1 - t0, q_last = SWAP ? T - 1 - t0 : M - 1 - m0;
+    uint32_t voff_p[AP], voff_q[QJ];
+#pragma unroll
+    for (int j = 0; j < AP; j++) {
+        const int r = prow + 8 * j + (lane >> 3);
+        voff_p[j] = (uint32_t)min(r, p_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(SWAP, r));
+    }
+#pragma unroll
+    for (int j = 0; j < QJ; j++) {
+        const int r = qrow + 8 * j + (lane >> 3);
+        voff_q[j] = (uint32_t)min(r, q_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(!SWAP, r));
+    }
+    auto request_p = [&](auto stage, int step_, int j) {
+        half_t *dst = (decltype(stage)::value ? sp1 : sp0) + (prow + 8 * j) * PK;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], min(step_, steps - 1) * (PK * 2), 0, 0);
+    };
+    auto request_q = [&](auto stage, int step_, int j) {
+        half_t *dst = (decltype(stage)::value ? sq1 : sq0) + (qrow + 8 * j) * PK;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], min(step_, steps - 1) * (PK * 2), 0, 0);
+    };
+
+    float4_t acc[P][Q];
+#pragma unroll
+    for (int i = 0; i < P; i++)
+#pragma unroll
+        for (int j = 0; j < Q; j++) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+
+    // fragment kk (32 columns) of fragment row lm: piece 4 kk + g of row `frow` of the token or feature fragments
+    const int fr = 8 * (lm >> 2) + (lm & 3);                                  // this lane's row of a features fragment, + 4 (f & 1) + 32 (f / 2)
+    const int frow_p = SWAP ? fr : lm, frow_q = SWAP ? lm : fr;
+    const int swz_p = swizzle(SWAP, frow_p), swz_q = swizzle(!SWAP, frow_q);
+    auto frag_row = [](bool features, int i) { return features ? 32 * (i >> 1) + 4 * (i & 1) : 16 * i; };
+    half8_t fp[2][P], fq[2][Q];
+    auto load_frags = [&](auto stage) {
+        const half_t *ps = (decltype(stage)::value ? sp1 : sp0) + (wp * AP * 32 + frow_p) * PK;
+        const half_t *qs = (decltype(stage)::value ? sq1 : sq0) + (wq * AQ * 32 + frow_q) * PK;
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            const int pp = 8 * ((4 * kk + g) ^ swz_p), pq = 8 * ((4 * kk + g) ^ swz_q);
+#pragma unroll
+            for (int j = 0; j < Q; j++) fq[kk][j] = *reinterpret_cast<const half8_t *>(qs + frag_row(!SWAP, j) * PK + pq);
+#pragma unroll
+            for (int i = 0; i < P; i++) fp[kk][i] = *reinterpret_cast<const half8_t *>(ps + frag_row(SWAP, i) * PK + pp);
+        }
+    };
+    // quarter q of a k-step: columns 32 (q / 2) .. + 31, half of the P fragments (features are the first MFMA operand)
+    auto mfmas = [&](int q) {
+#pragma unroll
+        for (int i = (q & 1) * AP; i < (q & 1) * AP + AP; i++)
+#pragma unroll
+            for (int j = 0; j < Q; j++)
+                acc[i][j] = SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_f16(fp[q >> 1][i], fq[q >> 1][j], acc[i][j], 0, 0, 0)
+                                 : __builtin_amdgcn_mfma_f32_16x16x32_f16(fq[q >> 1][j], fp[q >> 1][i], acc[i][j], 0, 0, 0);
+    };
+    using Z = std::integral_constant<int, 0>;
+    using O = std::integral_constant<int, 1>;
+
+    // ---- fill: step 0 by everybody, then what the first phases would have requested for step 1 ----------
+#pragma unroll
+    for (int j = 0; j < QJ; j++) request_q(Z{}, 0, j);
+#pragma unroll
+    for (int j = 0; j < AP; j++) request_p(Z{}, 0, j);
+    if (wp == 0) {
+#pragma unroll
+        for (int j = 0; j < AP; j++) request_p(O{}, 1, j);
+        wait_requests<AP>();
+        phase_barrier();
+        auto step = [&](auto stage, int s) {
+            using Other = std::integral_constant<int, 1 - decltype(stage)::value>;
+            // MEMORY(s): the reads first, they are what the phase waits for
+            load_frags(stage);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < QJ; j++) request_q(Other{}, s + 1, j);
+            wait_lds();
+            phase_barrier();
+            // MATRIX(s)
+            __builtin_amdgcn_s_setprio(1);
+            static_for<4>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if constexpr (q < AP) request_p(stage, s + 2, q);
+                mfmas(q);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            __builtin_amdgcn_s_setprio(0);
+            wait_requests<AP>();               // the Q rows and upper P rows of step s + 1
+            phase_barrier();
+        };
+        int s = 0;
+        for (; s + 1 < steps; s += 2) {        // (no exit between the two: a path around the second one would make the
+            step(Z{}, s);                      // compiler wait for the wrong requests at the top of the loop)
+            step(O{}, s + 1);
+        }
+        if (s < steps) step(Z{}, s);
+        phase_barrier();
+    } else {
+#pragma unroll
+        for (int j = 0; j < QJ; j++) request_q(O{}, 1, j);
+#pragma unroll
+        for (int j = 0; j < AP; j++) request_p(O{}, 1, j);
+        wait_requests<AP + QJ>();
+        phase_barrier();
+        phase_barrier();
+        auto step = [&](auto stage, int s) {
+            // MEMORY(s)
+            load_frags(stage);
+            wait_lds();
+            wait_requests<AP>();               // the Q rows of step s + 1
+            phase_barrier();
+            // MATRIX(s)
+            __builtin_amdgcn_s_setprio(1);
+            static_for<4>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                // Q rows first: they are read one phase earlier
+                static_for<AP + QJ>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    if constexpr (j * 4 / (AP + QJ) == q) {
+                        if constexpr (j < QJ) request_q(stage, s + 2, j);
+                        else request_p(stage, s + 2, j - QJ);
+                    }
+                });
+                mfmas(q);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            __builtin_amdgcn_s_setprio(0);
+            wait_requests<AP + QJ>();          // the lower P rows of step s + 1
+            phase_barrier();
+        };
+        int s = 0;
+        for (; s + 1 < steps; s += 2) {
+            step(Z{}, s);
+            step(O{}, s + 1);
+        }
+        if (s < steps) step(Z{}, s);
+    }
+    wait_requests<0>();                        // (the repeated last step's)
+
+    // D[feature row, token]: the lane holds token lm of token fragment a, and of the pair of feature fragments (2 p, 2 p + 1)
+    // the eight features 32 p + 8 g .. + 7
+    constexpr int TA = SWAP ? Q : P, FP = SWAP ? AP : AQ;
+    const int tw = t0 + (SWAP ? wq * AQ : wp * AP) * 32, mw = m0 + (SWAP ? wp * AP : wq * AQ) * 32;
+    auto value = [&](int a, int p, int e) { return SWAP ? acc[2 * p + (e >> 2)][a][e & 3] : acc[a][2 * p + (e >> 2)][e & 3]; };
+    if (SPLIT || wide) {
+#pragma unroll
+        for (int p = 0; p < FP; p++) {
+            const int m = mw + 32 * p + 8 * g;
+            float bv[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) bv[e] = !SPLIT && bias && m + e < M ? (float)bias[m + e] : 0.f;
+#pragma unroll
+            for (int a = 0; a < TA; a++) {
+                const int t = tw + 16 * a + lm;
+                if (t >= T || m >= M) continue;
+                if (SPLIT) {
+                    float *o = part + ((int64_t)sp * T + t) * M + m;
+                    if (wide) {
+                        *reinterpret_cast<float4_t *>(o) = (float4_t){value(a, p, 0), value(a, p, 1), value(a, p, 2), value(a, p, 3)};
+                        *reinterpret_cast<float4_t *>(o + 4) = (float4_t){value(a, p, 4), value(a, p, 5), value(a, p, 6), value(a, p, 7)};
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            if (m + e < M) o[e] = value(a, p, e);
+                    }
+                } else {
+                    half8_t v;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = (half_t)(value(a, p, e) + bv[e]);
+                    *reinterpret_cast<half8_t *>(y + (int64_t)t * M + m) = v;
+                }
+            }
+        }
+    } else {
+        // 16 tokens x 32 features at a time through 1 KB of LDS per wave; 32 lanes then write 64 bytes of a row
+        phase_barrier();                       // (everybody's requests have landed)
+        half_t *buf = sq0 + wave * 512;
+        const int f = lane & 31, th = lane >> 5;
+#pragma unroll
+        for (int p = 0; p < FP; p++) {
+            const int m = mw + 32 * p + f;
+            const float bv = bias && m < M ? (float)bias[m] : 0.f;
+#pragma unroll
+            for (int a = 0; a < TA; a++) {
+                float4_t lo = {value(a, p, 0), value(a, p, 1), value(a, p, 2), value(a, p, 3)}, hi = {value(a, p, 4), value(a, p, 5), value(a, p, 6), value(a, p, 7)};
+                half8_t v;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[e] = (half_t)(lo[e] + __shfl(bv, 8 * g + e, 64));
+                    v[e + 4] = (half_t)(hi[e] + __shfl(bv, 8 * g + e + 4, 64));
+                }
+                *reinterpret_cast<half8_t *>(buf + lm * 32 + 8 * g) = v;
+                asm volatile("" ::: "memory");   // (the LDS operations of a wave execute in order)
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    const int t = tw + 16 * a + 2 * r + th;
+                    const half_t o = buf[(2 * r + th) * 32 + f];
+                    if (t < T && m < M) y[(int64_t)t * M + m] = o;
+                }
+                asm volatile("" ::: "memory");
+            }
+        }
+    }
+}
+
+// y = fp16(sum over the parts in order + bias): eight outputs per thread (WIDE: M % 8 == 0, 16-byte aligned y), or one
+template <bool WIDE>
+__global__ __launch_bounds__(256) void linear_split_sum_kernel(const float *__restrict__ part, const half_t *__restrict__ bias,
+                                                               half_t *__restrict__ y, int splits, int64_t total, int M) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * (WIDE ? 8 : 1);
+    if (i >= total) return;
+    const int m = (int)(i % M);
+    if (WIDE) {
+        float4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+        for (int s = 0; s < splits; s++) {
+            const float *p = part + s * total + i;
+            a += *reinterpret_cast<const float4_t *>(p);
+            b += *reinterpret_cast<const float4_t *>(p + 4);
+        }
+        half8_t v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e] = (half_t)(a[e] + (bias ? (float)bias[m + e] : 0.f));
+            v[e + 4] = (half_t)(b[e] + (bias ? (float)bias[m + e + 4] : 0.f));
+        }
+        *reinterpret_cast<half8_t *>(y + i) = v;
+    } else {
+        float a = 0.f;
+        for (int s = 0; s < splits; s++) a += part[s * total + i];
+        y[i] = (half_t)(a + (bias ? (float)bias[m] : 0.f));
+    }
+}
+
+template <int AP, int AQ, bool SWAP>
+int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int splits, float *part, hipStream_t s) {
+    constexpr int BT = SWAP ? 128 * AQ : 64 * AP, BF = SWAP ? 64 * AP : 128 * AQ;
+    const unsigned tiles = (unsigned)(bs_cdiv(T, BT) * bs_cdiv(M, BF));
+    const int steps = (int)bs_cdiv(N / PK, splits);
+    splits = (int)bs_cdiv(N / PK, steps);     // every part holds at least one k-step
+    const int wide = M % 8 == 0 && bs_aligned(y, 16) && bs_aligned(part, 16);
+    if (splits == 1) {
+        linear_pipe_kernel<AP, AQ, SWAP, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+    } else {
+        linear_pipe_kernel<AP, AQ, SWAP, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        BS_LAUNCH_CHECK();
+        const int64_t total = (int64_t)T * M;
+        if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, splits, total, M);
+        else linear_split_sum_kernel<false><<<(unsigned)bs_cdiv(total, 256), 256, 0, s>>>(part, bias, y, splits, total, M);
+    }
+    BS_LAUNCH_CHECK();
+    return BS_OK;
+}
+
+}  // namespace
+
+// bt x bf: tokens x features per workgroup.  splits > 1: part holds splits * T * M floats.
+int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int bt, int bf,
+                          int splits, float *part, hipStream_t s) {
+    if (N % PK != 0 || splits < 1 || (splits > 1 && !part)) return BS_ERR_SHAPE;
+    switch (bt * 1000 + bf) {
+        case 256256: return launch_pipe<4, 2, false>(x, w, bias, y, T, M, N, splits, part, s);
+        case 192256: return launch_pipe<3, 2, false>(x, w, bias, y, T, M, N, splits, part, s);
+        case 256192: return launch_pipe<3, 2, true>(x, w, bias, y, T, M, N, splits, part, s);
+        case 256128: return launch_pipe<4, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
+        case 128256: return launch_pipe<4, 1, true>(x, w, bias, y, T, M, N, splits, part, s);
+        case 192128: return launch_pipe<3, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
+        case 128192: return launch_pipe<3, 1, true>(x, w, bias, y, T, M, N, splits, part, s);
+        case 128128: return launch_pipe<2, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
+        case 64128: return launch_pipe<1, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
+        default: return BS_ERR_SHAPE;
+    }
+}

@@ -95,7 +95,8 @@ int64_t bs_workspace_bytes(int I, int M, int N, int K, int T);
  * (bitstack/utils/inference_utils.py:171-284).
  *
  * T <= 4 runs the packed-sign GEMV (signs contracted on MFMA against
- * vt_i o x, scaled by u_i, all blocks in one pass; N % 512 == 0); 5 <= T <= 48
+ * vt_i o x, scaled by u_i, all blocks in one pass; N % 128 == 0 and at most N / 3
+ * columns missing from the last chunk of 512); 5 <= T <= 48
  * the strip kernel (16 x 16 patches of the weight rebuilt in registers and
  * multiplied by x at once, the weight never stored; N % 128 == 0; when it does
  * not take the shape, T <= 8 is two GEMV passes); 49 <= T <= 96 the same
@@ -149,7 +150,7 @@ int bs_forward_static(const uint8_t *packed, const void *u, const void *vt, cons
  * many partial sums per row and block bs_forward would use for these
  * dimensions; *waves == 0 means the decode kernel does not run them (the
  * strip kernel or the dense path does: more than 4 tokens with N % 128 == 0,
- * more than 8 tokens, N not a multiple of 512).  No counterpart in the reference
+ * more than 8 tokens, an N as bs_forward does not give it).  No counterpart in the reference
  * (Triton picks its configuration by autotuning,
  * bitstack/utils/inference_utils.py:8-39).
  */
@@ -186,7 +187,7 @@ int bs_forward_path(int I, int M, int N, int K, int T);
  * Test and benchmark hook: 0 = choose the decode kernel of one- and two-token
  * passes by shape (the default), BS_DECODE_F16 = always the fp16 kernel,
  * BS_DECODE_MX = the block-scaled kernel wherever it takes the shape
- * (N % 512 == 0, at most two tokens).  The setting belongs to the CALLING
+ * (one or two tokens).  The setting belongs to the CALLING
  * THREAD (every thread starts at 0): bs_workspace_bytes, bs_decode_plan and
  * bs_forward called from one thread always agree, whatever other threads set.
  * No counterpart in the reference.
@@ -263,7 +264,7 @@ int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_features, in
  *   BS_EPI_SWIGLU    n == 2, M_0 == M_1: y[T, M_0] = silu(first) * second
  *                    computed from the fp16-rounded results, as
  *                    `act_fn(gate_proj(h)) * up_proj(h)` in the MLP
- * Only shapes the decode kernel takes (every matrix: N % 512 == 0,
+ * Only shapes the decode kernel takes (every matrix: N as bs_forward gives it at T <= 4,
  * M * N < 2^31, alignment as bs_forward); anything else returns BS_ERR_SHAPE
  * and the caller issues bs_forward per matrix.  Workspace as bs_forward, size
  * from bs_forward_group_workspace_bytes (negative = status).

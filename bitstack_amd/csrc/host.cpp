@@ -169,6 +169,54 @@ PyObject *host_rebuild(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
 }
 
+// unpack(qweight [blocks, bytes], blocks, M, N) -> int8 signs [blocks, M, N], or None
+PyObject *host_unpack(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 4) return PyErr_Format(PyExc_TypeError, "unpack takes 4 arguments");
+    try {
+        const at::Tensor *q = tensor_arg(a[0]);
+        int64_t blocks, M, N;
+        if (!int_arg(a[1], blocks) || !int_arg(a[2], M) || !int_arg(a[3], N)) return nullptr;
+        if (!q || !q->is_cuda() || !plain(*q, at::kByte, q->device()) || q->dim() != 2) Py_RETURN_NONE;
+        if (blocks < 1 || blocks > q->size(0) || M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX || M * N % 8 != 0 || q->size(1) != M * N / 8)
+            Py_RETURN_NONE;                      // (blocks of whole bytes follow each other without padding)
+        const c10::Device dev = q->device();
+        DeviceScope scope(dev);
+        const at::Tensor s = at::Tensor(at::detail::empty_cuda({blocks, M, N}, at::kChar, dev, std::nullopt));
+        const int st = bs_unpack_sign((const uint8_t *)q->const_data_ptr(), (int8_t *)s.mutable_data_ptr(), blocks * M * N,
+                                      c10::hip::getCurrentHIPStream(dev.index()).stream());
+        if (st != BS_OK) return raise_status(st, "bs_unpack_sign");
+        return THPVariable_Wrap(s);
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
+// rebuild_from_sign(signs [I, M, N] int8, u, vt, I) -> w [M, N], or None (u and vt may hold more blocks)
+PyObject *host_rebuild_from_sign(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 4) return PyErr_Format(PyExc_TypeError, "rebuild_from_sign takes 4 arguments");
+    try {
+        const at::Tensor *s = tensor_arg(a[0]), *u = tensor_arg(a[1]), *vt = tensor_arg(a[2]);
+        int64_t I;
+        if (!int_arg(a[3], I)) return nullptr;
+        if (!s || !u || !vt || !u->is_cuda() || s->dim() != 3 || u->dim() != 3 || vt->dim() != 3) Py_RETURN_NONE;
+        const c10::Device dev = u->device();
+        if (!plain(*s, at::kChar, dev) || !plain(*u, at::kHalf, dev) || !plain(*vt, at::kHalf, dev)) Py_RETURN_NONE;
+        const int64_t M = u->size(1), K = u->size(2), N = vt->size(2);
+        if (I < 1 || s->size(0) != I || u->size(0) < I || vt->size(0) < I || vt->size(1) != K || s->size(1) != M || s->size(2) != N ||
+            M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX)
+            Py_RETURN_NONE;
+        DeviceScope scope(dev);
+        const at::Tensor w = new_half({M, N}, dev);
+        const int st = bs_reconstruct_w_from_sign((const int8_t *)s->const_data_ptr(), u->const_data_ptr(), vt->const_data_ptr(),
+                                                  w.mutable_data_ptr(), (int)I, (int)M, (int)N, (int)K,
+                                                  c10::hip::getCurrentHIPStream(dev.index()).stream());
+        if (st != BS_OK) return raise_status(st, "bs_reconstruct_w_from_sign");
+        return THPVariable_Wrap(w);
+    } catch (const std::exception &e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+}
+
 // linear(x, w, bias or None) -> x @ w^T (+ bias), or None
 PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 3) return PyErr_Format(PyExc_TypeError, "linear takes 3 arguments");
@@ -355,7 +403,7 @@ PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 #define HOST_METHOD(name) {#name, (PyCFunction)(void (*)(void))host_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(linear), HOST_METHOD(workspace),
+PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(unpack), HOST_METHOD(rebuild_from_sign), HOST_METHOD(linear), HOST_METHOD(workspace),
                          HOST_METHOD(argmax), HOST_METHOD(make_steps), HOST_METHOD(run_steps), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native host path over libbitstack_hip.so.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

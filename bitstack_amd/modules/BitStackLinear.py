@@ -152,10 +152,17 @@ class BitStackLinear(nn.Module):
             w += compose_weight(q, getattr(self, f"u_{i}"), getattr(self, f"vt_{i}"), self.no_avd, w.shape)
         return F.linear(x, w, bias=self.bias)
 
+    def _signs(self, q):
+        """int8 signs [w_bit, out, in] of the first w_bit stacked blocks."""
+        sign = _lib.host().unpack(q, self.w_bit, self.out_features, self.in_features)
+        if sign is not None:
+            return sign
+        return unpack_sign_hip(q.reshape(-1), torch.Size([self.w_bit, self.out_features, self.in_features]))
+
     @torch.no_grad()
     def forward_l1(self, x):
         q, u, vt = self._stacked()
-        sign = unpack_sign_hip(q.reshape(-1), torch.Size([self.w_bit, self.out_features, self.in_features]))
+        sign = self._signs(q)
         w = torch.matmul(u, vt)
         w = (w.mul_(sign)).sum(dim=0).contiguous()
         return F.linear(x, w, bias=self.bias)
@@ -163,8 +170,9 @@ class BitStackLinear(nn.Module):
     @torch.no_grad()
     def forward_l2(self, x):
         q, u, vt = self._stacked()
-        sign = unpack_sign_hip(q.reshape(-1), torch.Size([self.w_bit, self.out_features, self.in_features]))
-        return F.linear(x, reconstruct_w_hip(sign, u, vt), bias=self.bias)
+        sign = self._signs(q)
+        w = _lib.host().rebuild_from_sign(sign, u, vt, self.w_bit)
+        return F.linear(x, reconstruct_w_hip(sign, u, vt) if w is None else w, bias=self.bias)
 
     def _rebuilt(self):
         """The weight from the first w_bit stacked blocks: one native call where they lie as stack_blocks() left them."""

@@ -58,6 +58,8 @@ SIGNATURES.update({
     "bs_argmax_f16": (_I, [_P, _P, _I, _I, _P]),
     "bs_rmsnorm_f16": (_I, [_P, _P, _P, _I, _I, ctypes.c_float, _P]),
     "bs_attention_decode_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "bs_attention_decode_workspace_bytes": (_L, [_I, _I, _I, _I, _I]),
+    "bs_attention_decode_ws_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P]),
 })
 EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU = 0, 1, 2
 

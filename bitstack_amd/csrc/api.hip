@@ -251,20 +251,37 @@ extern "C" int bs_rmsnorm_f16(const void *x, const void *weight, void *y, int T,
     return bs_launch_rmsnorm((const half_t *)x, (const half_t *)weight, (half_t *)y, T, H, eps, (hipStream_t)stream);
 }
 
-extern "C" int bs_attention_decode_f16(const void *qkv, void *kcache, void *vcache, const void *cos, const void *sin,
-                                       const int64_t *pos, void *out, int B, int heads, int kv_heads, int head_dim,
-                                       int max_len, void *stream) {
-    if (B < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || head_dim != 128 || max_len < 1 ||
-        max_len > 8192)
-        return BS_ERR_SHAPE;
+static int attention_shape(int B, int heads, int kv_heads, int head_dim, int max_len) {
+    return B < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || head_dim != 128 || max_len < 1 || max_len > 8192 ? BS_ERR_SHAPE
+                                                                                                                          : BS_OK;
+}
+
+extern "C" int64_t bs_attention_decode_workspace_bytes(int B, int heads, int kv_heads, int head_dim, int max_len) {
+    const int st = attention_shape(B, heads, kv_heads, head_dim, max_len);
+    return st != BS_OK ? st : bs_attention_parts_bytes(B, heads, kv_heads, max_len);
+}
+
+extern "C" int bs_attention_decode_ws_f16(const void *qkv, void *kcache, void *vcache, const void *cos, const void *sin,
+                                          const int64_t *pos, void *out, int B, int heads, int kv_heads, int head_dim,
+                                          int max_len, void *workspace, int64_t workspace_bytes, void *stream) {
+    const int st = attention_shape(B, heads, kv_heads, head_dim, max_len);
+    if (st != BS_OK) return st;
     if (B == 0) return BS_OK;
     if (!qkv || !kcache || !vcache || !cos || !sin || !pos || !out) return BS_ERR_NULL;
     if (!bs_aligned(qkv, 16) || !bs_aligned(kcache, 16) || !bs_aligned(vcache, 16) || !bs_aligned(cos, 16) ||
         !bs_aligned(sin, 16) || !bs_aligned(pos, 8) || !bs_aligned(out, 16))
         return BS_ERR_ALIGN;
+    const bool room = workspace && bs_aligned(workspace, 16) &&
+                      workspace_bytes >= bs_attention_parts_bytes(B, heads, kv_heads, max_len);
     return bs_launch_attention_decode((const half_t *)qkv, (half_t *)kcache, (half_t *)vcache, (const half_t *)cos,
                                       (const half_t *)sin, pos, (half_t *)out, B, heads, kv_heads, head_dim, max_len,
-                                      (hipStream_t)stream);
+                                      room ? (float *)workspace : nullptr, (hipStream_t)stream);
+}
+
+extern "C" int bs_attention_decode_f16(const void *qkv, void *kcache, void *vcache, const void *cos, const void *sin,
+                                       const int64_t *pos, void *out, int B, int heads, int kv_heads, int head_dim,
+                                       int max_len, void *stream) {
+    return bs_attention_decode_ws_f16(qkv, kcache, vcache, cos, sin, pos, out, B, heads, kv_heads, head_dim, max_len, nullptr, 0, stream);
 }
 
 extern "C" int bs_argmax_f16(const void *x, int64_t *out, int B, int V, void *stream) {

@@ -106,4 +106,5 @@ int bs_launch_argmax(const half_t *x, int64_t *out, int B, int V, hipStream_t s)
 int bs_launch_rmsnorm(const half_t *x, const half_t *weight, half_t *y, int T, int H, float eps, hipStream_t s);
 int bs_launch_attention_decode(const half_t *qkv, half_t *kcache, half_t *vcache, const half_t *cos, const half_t *sin,
                                const int64_t *pos, half_t *out, int B, int heads, int kv_heads, int head_dim,
-                               int max_len, hipStream_t s);
+                               int max_len, float *part, hipStream_t s);
+int64_t bs_attention_parts_bytes(int B, int heads, int kv_heads, int max_len);   // scratch for `part` (0: none is used)

@@ -53,284 +53,231 @@ __global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *__re
     }
 }
 
-// One workgroup per (query head, sequence).  1024 threads = 64 groups of 16 lanes;
-// a group walks every 64th cached position, a lane owns 8 of the 128 dimensions
-// (one 16-byte load per cached row and lane, a row is one contiguous 256 bytes).
-// One pass: k and v of four positions are fetched together and folded into a
-// running (max, sum, weighted v) per group; the 64 groups are merged through LDS.
-constexpr int ATT_THREADS = 1024, ATT_GROUPS = ATT_THREADS / 16, ATT_D = 128, ATT_MAX_LEN = 8192;
+// One position of attention: a workgroup serves HP query heads of one KV head and sequence, its waves walk the cache in
+// tiles of 16 positions (tile = wave, wave + WAVES, ...) with a running (max, sum, weighted v) per wave, merged through LDS.
+//
+// Both products run on the matrix cores, the heads as columns (HP of 16 used):
+//   scores  S[position, head] = K q     16x16x32, K rows as loaded (a lane: position l % 16, dimensions 32 c + 8 (l / 16) ..)
+//   output  O[dim, head] += V^T P       16x16x32, four positions twice: P is split into two fp16 terms, p = hi + lo to 2^-22,
+//                                       and the eight k slots of a lane hold {hi, lo} against {v, v}, so the weights keep the
+//                                       precision they had as fp32 numbers
+// A lane of the scores holds positions 4 (l / 16) + i of head l % 16, which is what the second product wants of P; V needs no
+// transposition either: a lane loads dimensions 8 r .. 8 r + 7 (r = l % 16) of its four positions, and product number j takes
+// half j of each, so that its row r is dimension 8 r + j.  K of the next tile is requested behind the scores, V behind the
+// output product.
+//
+// What bounds it: the fetches, and below about a thousand positions the chain position -> first tile -> merge.  Folding
+// position by position on the VALU (32 instructions per position and head) took 46 us
+// on 8 sequences x 64 heads (8 KV heads) at position 2100 where this takes 22.5 (69 MB: 3.1 TB/s), 18.7 / 8.8 on 16 x 32 at 300,
+// 8.2 / 6.9 on 1 x 32 at 384.
+constexpr int ATT_D = 128, ATT_MAX_LEN = 8192, ATT_TILE = 16, ATT_SPLIT_LEN = 1025, ATT_WHOLE = 512, ATT_MAX_SPLITS = 16, ATT_PART = ATT_D + 4;
 
-__global__ __launch_bounds__(ATT_THREADS) void attention_decode_kernel(
+template <int HP, int WAVES, bool SPLIT>
+__global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
     const half_t *__restrict__ qkv, half_t *__restrict__ kcache, half_t *__restrict__ vcache,
     const half_t *__restrict__ cosv, const half_t *__restrict__ sinv, const int64_t *__restrict__ pos_ptr,
-    half_t *__restrict__ out, int heads, int kv_heads, int max_len) {
-    __shared__ float qs[ATT_D];                  // rotated query, pre-scaled
+    half_t *__restrict__ out, float *__restrict__ part, int B, int heads, int kv_heads, int max_len) {
+    constexpr int THREADS = WAVES * 64;
+    __shared__ __attribute__((aligned(16))) half_t qrot[HP][ATT_D];            // rotated queries
     __shared__ __attribute__((aligned(16))) half_t knew[ATT_D], vnew[ATT_D];   // this position's rotated k and v
-    __shared__ float gm[ATT_GROUPS], gl[ATT_GROUPS];             // per group: running max, sum of exp
-    __shared__ float accs[ATT_GROUPS][ATT_D];
-    const int tid = threadIdx.x, lane16 = tid & 15, grp = tid >> 4;
-    const int head = blockIdx.x, b = blockIdx.y;
-    const int rep = heads / kv_heads, hk = head / rep;
+    __shared__ float wm[HP][WAVES], wl[HP][WAVES];                             // per wave: running max, sum of exp
+    __shared__ __attribute__((aligned(16))) float wacc[HP][WAVES][ATT_D];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    // The workgroups of one KV head read the same rows: on one XCD (workgroups are dealt to the eight in turn) they share them
+    // in its L2.
+    const int rep = heads / kv_heads, share = rep / HP, pairs = B * kv_heads;
+    const int id = blockIdx.x;
+    const bool dealt = pairs % 8 == 0;
+    const int pair = dealt ? (id & 7) + 8 * (id / (8 * share)) : id / share, sub = dealt ? (id >> 3) % share : id % share;
+    const int b = pair / kv_heads, hk = pair % kv_heads, head0 = hk * rep + sub * HP;
     const int row = (heads + 2 * kv_heads) * ATT_D;
-    const half_t *q = qkv + (int64_t)b * row + head * ATT_D;
+    const half_t *qh = qkv + (int64_t)b * row + (int64_t)head0 * ATT_D;        // the HP query heads, contiguous
     const half_t *kn = qkv + (int64_t)b * row + (heads + hk) * ATT_D;
     const half_t *vn = qkv + (int64_t)b * row + (heads + kv_heads + hk) * ATT_D;
-    half_t *orow = out + ((int64_t)b * heads + head) * ATT_D;
-    // what does not depend on the position is fetched before the position is known
-    float qa = 0.f, qb = 0.f, ka = 0.f, kb = 0.f;
-    half_t vv = (half_t)0;
-    if (tid < ATT_D / 2) {
-        qa = (float)q[tid]; qb = (float)q[tid + ATT_D / 2];
-        ka = (float)kn[tid]; kb = (float)kn[tid + ATT_D / 2];
-    } else if (tid < ATT_D / 2 + ATT_D) {
-        vv = vn[tid - ATT_D / 2];
+    half_t *orow = out + ((int64_t)b * heads + head0) * ATT_D;
+    // Work items of the set-up: HP * 64 query pairs, 64 key pairs (dimension i and i + 64 rotate together), 128 values.  What
+    // does not depend on the position is fetched before the position is known.
+    constexpr int QP = HP * 64, ITEMS = QP + 64 + ATT_D;
+    static_assert(ITEMS <= THREADS, "one set-up item per thread");
+    float fa = 0.f, fb = 0.f;
+    if (tid < QP) {
+        const int h = tid >> 6, i = tid & 63;
+        fa = (float)qh[h * ATT_D + i]; fb = (float)qh[h * ATT_D + i + 64];
+    } else if (tid < QP + 64) {
+        fa = (float)kn[tid - QP]; fb = (float)kn[tid - QP + 64];
+    } else if (tid < ITEMS) {
+        fa = (float)vn[tid - QP - 64];
     }
     const int64_t pos64 = *pos_ptr;
     if (pos64 < 0 || pos64 >= max_len) {         // nothing sensible to do: defined output, no access outside the cache
-        if (tid < ATT_D) orow[tid] = (half_t)0;
+        if (!SPLIT)
+            for (int it = tid; it < HP * ATT_D; it += THREADS) orow[it] = (half_t)0;
         return;
     }
-    const int pos = (int)pos64;
+    // With the positions split, workgroup y of gridDim.y takes every gridDim.y-th round of tiles; up to ATT_WHOLE positions
+    // the first takes them all and writes the result itself (two rounds are shorter than the way through the second launch).
+    const bool split = SPLIT && pos64 > ATT_WHOLE;
+    if (SPLIT && !split && blockIdx.y > 0) return;
+    const int pos = (int)pos64, tiles = (pos + ATT_TILE - 1) / ATT_TILE;
     half_t *kc = kcache + ((int64_t)b * kv_heads + hk) * max_len * ATT_D;
     half_t *vc = vcache + ((int64_t)b * kv_heads + hk) * max_len * ATT_D;
 
-    if (tid < ATT_D / 2) {
-        const float c = (float)cosv[(int64_t)pos * (ATT_D / 2) + tid], s = (float)sinv[(int64_t)pos * (ATT_D / 2) + tid];
-        const float scale = 0.08838834764831845f;       // 1 / sqrt(128)
-        qs[tid] = (float)(half_t)(qa * c - qb * s) * scale;
-        qs[tid + ATT_D / 2] = (float)(half_t)(qb * c + qa * s) * scale;
-        knew[tid] = (half_t)(ka * c - kb * s);
-        knew[tid + ATT_D / 2] = (half_t)(kb * c + ka * s);
-    } else if (tid < ATT_D / 2 + ATT_D) {
-        vnew[tid - ATT_D / 2] = vv;
+    half8_t k8[4], v8[4];
+    auto fetch_k = [&](int t) {                  // rows past the last are the last again; their scores are masked
+        const half_t *p = kc + (int64_t)min(t * ATT_TILE + r16, pos - 1) * ATT_D + 8 * g;
+#pragma unroll
+        for (int c = 0; c < 4; c++) k8[c] = *reinterpret_cast<const half8_t *>(p + 32 * c);
+    };
+    auto fetch_v = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            v8[i] = *reinterpret_cast<const half8_t *>(vc + (int64_t)min(t * ATT_TILE + 4 * g + i, pos - 1) * ATT_D + 8 * r16);
+    };
+    const int step = split ? WAVES * (int)gridDim.y : WAVES;
+    int t = SPLIT ? wave + WAVES * (int)blockIdx.y : wave;
+    const bool own = t == tiles % step;          // the wave whose turn is next takes this step's own position
+    if (t < tiles) { fetch_k(t); fetch_v(t); }
+
+    if (tid < QP + 64) {
+        const int i = tid & 63;
+        const float c = (float)cosv[(int64_t)pos * (ATT_D / 2) + i], sn = (float)sinv[(int64_t)pos * (ATT_D / 2) + i];
+        const half_t lo = (half_t)(fa * c - fb * sn), hi = (half_t)(fb * c + fa * sn);
+        half_t *to = tid < QP ? qrot[tid >> 6] : knew;
+        to[i] = lo; to[i + 64] = hi;
+    } else if (tid < ITEMS) {
+        vnew[tid - QP - 64] = (half_t)fa;
     }
     __syncthreads();
-    if (head % rep == 0 && tid < ATT_D) {        // one head of the group appends to the cache
+    if (sub == 0 && blockIdx.y == 0 && tid < ATT_D) {               // one workgroup of the KV head appends this position to the cache
         kc[(int64_t)pos * ATT_D + tid] = knew[tid];
         vc[(int64_t)pos * ATT_D + tid] = vnew[tid];
     }
 
-    float qreg[8];
+    half8_t q8[4];
 #pragma unroll
-    for (int e = 0; e < 8; e++) qreg[e] = qs[8 * lane16 + e];
-    float m = -INFINITY, l = 0.f;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    auto score_of = [&](const half8_t k8) {
-        float d = 0.f;
+    for (int c = 0; c < 4; c++)
+        q8[c] = r16 < HP ? *reinterpret_cast<const half8_t *>(&qrot[r16 < HP ? r16 : 0][32 * c + 8 * g]) : (half8_t)(half_t)0;
+    const float scale2 = 0.08838834764831845f * 1.4426950408889634f;    // 1 / sqrt(128) * log2(e): the softmax runs in base 2
+    float m = -INFINITY, l = 0.f;                // of head l % 16; the sum over this lane's positions only
+    float4_t acc[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) d += qreg[e] * (float)k8[e];
+    for (int j = 0; j < 8; j++) acc[j] = (float4_t)0.f;
+    auto scores = [&]() {
+        float4_t s = (float4_t)0.f;
 #pragma unroll
-        for (int o = 8; o >= 1; o >>= 1) d += __shfl_xor(d, o, 64);
-        return d;                                 // the same value in all 16 lanes of the group
+        for (int c = 0; c < 4; c++) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[c], q8[c], s, 0, 0, 0);
+        return s;
     };
-    auto fold = [&](float sc, const half8_t v8) {
-        const float mn = fmaxf(m, sc);
-        const float r = __expf(m - mn), w = __expf(sc - mn);      // exp(-inf) = 0 on the first position
-        l = l * r + w;
+    auto fold = [&](const float4_t s, int valid) {                      // the tile's first `valid` positions (at least one)
+        float p[4], mx = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = acc[e] * r + w * (float)v8[e];
+        for (int i = 0; i < 4; i++) {
+            p[i] = 4 * g + i < valid ? s[i] * scale2 : -INFINITY;
+            mx = fmaxf(mx, p[i]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float mn = fmaxf(m, mx), r = __builtin_amdgcn_exp2f(m - mn);      // exp2(-inf) = 0 on the first tile
         m = mn;
-    };
-    for (int p0 = grp; p0 < pos; p0 += 4 * ATT_GROUPS) {
-        half8_t k8[4], v8[4];
+        half8_t p8;
+        float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int p = min(p0 + ATT_GROUPS * j, pos - 1);
-            k8[j] = *reinterpret_cast<const half8_t *>(kc + (int64_t)p * ATT_D + 8 * lane16);
-            v8[j] = *reinterpret_cast<const half8_t *>(vc + (int64_t)p * ATT_D + 8 * lane16);
+        for (int i = 0; i < 4; i++) {
+            p[i] = __builtin_amdgcn_exp2f(p[i] - mn);
+            sum += p[i];
+            p8[i] = (half_t)p[i];
+            p8[i + 4] = (half_t)(p[i] - (float)p8[i]);
+        }
+        l = l * r + sum;
+        if (__any(r != 1.f)) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc[j] *= r;
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float sc = score_of(k8[j]);
-            if (p0 + ATT_GROUPS * j < pos) fold(sc, v8[j]);
-        }
-    }
-    if (grp == 0)      // this step's own k and v, from LDS
-        fold(score_of(*reinterpret_cast<const half8_t *>(knew + 8 * lane16)),
-             *reinterpret_cast<const half8_t *>(vnew + 8 * lane16));
-    if (lane16 == 0) { gm[grp] = m; gl[grp] = l; }
-#pragma unroll
-    for (int e = 0; e < 8; e++) accs[grp][8 * lane16 + e] = acc[e];
-    __syncthreads();
-    if (tid < ATT_D) {
-        float mx = gm[0];
-#pragma unroll
-        for (int gq = 1; gq < ATT_GROUPS; gq++) mx = fmaxf(mx, gm[gq]);
-        float o = 0.f, den = 0.f;
-#pragma unroll
-        for (int gq = 0; gq < ATT_GROUPS; gq++) {
-            const float r = gl[gq] > 0.f ? __expf(gm[gq] - mx) : 0.f;     // groups that saw no position
-            o += r * accs[gq][tid];
-            den += r * gl[gq];
-        }
-        orow[tid] = (half_t)(o / den);
-    }
-}
-
-// Grouped-query variant for long caches: one workgroup serves REP query heads that share a
-// KV head, so a cached row is fetched once for REP heads (the fetches, not the arithmetic,
-// are what a long cache costs).  1024 threads = 64 groups of 16 lanes; a group walks every
-// 64th position, a lane owns 8 of the 128 dimensions.  The rotated queries stay in registers as fp16 pairs and the scores
-// are v_dot2_f32_f16 sums (fp16 products, fp32 accumulation) reduced over the 16 lanes with
-// DPP adds; the softmax runs in base 2 (log2(e) folded into the score scale).  Per head a
-// running (max, sum, weighted v); groups are merged by shuffles inside a wave, waves through LDS.
-constexpr int GQA_THREADS = 1024, GQA_WAVES = GQA_THREADS / 64;
-
-// sum over the 16 lanes of a DPP row (every lane ends with the total)
-__device__ __forceinline__ float row_sum16(float v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true));  // row_half_mirror
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, true));  // row_mirror
-    return v;
-}
-
-template <int REP>
-__global__ __launch_bounds__(GQA_THREADS) void attention_decode_gqa_kernel(
-    const half_t *__restrict__ qkv, half_t *__restrict__ kcache, half_t *__restrict__ vcache,
-    const half_t *__restrict__ cosv, const half_t *__restrict__ sinv, const int64_t *__restrict__ pos_ptr,
-    half_t *__restrict__ out, int heads, int kv_heads, int max_len) {
-    __shared__ __attribute__((aligned(16))) half_t qrot[REP][ATT_D];           // rotated queries
-    __shared__ __attribute__((aligned(16))) half_t knew[ATT_D], vnew[ATT_D];   // this position's rotated k and v
-    __shared__ float wm[REP][GQA_WAVES], wl[REP][GQA_WAVES];
-    __shared__ float wacc[REP][GQA_WAVES][ATT_D];
-    const int tid = threadIdx.x, lane16 = tid & 15, grp = tid >> 4, wave = tid >> 6;
-    const int head0 = blockIdx.x * REP, b = blockIdx.y;          // this workgroup's first query head
-    const int rep = heads / kv_heads, hk = head0 / rep;          // REP divides rep: all REP heads share KV head hk
-    const int row = (heads + 2 * kv_heads) * ATT_D;
-    const half_t *qb_ = qkv + (int64_t)b * row + (int64_t)head0 * ATT_D;        // the REP query heads, contiguous
-    const half_t *kn = qkv + (int64_t)b * row + (heads + hk) * ATT_D;
-    const half_t *vn = qkv + (int64_t)b * row + (heads + kv_heads + hk) * ATT_D;
-    // Work items of the set-up: REP * 64 query pairs, 64 key pairs (dimension i and i + 64 rotate
-    // together), 128 values; at most two per thread.  What does not depend on the position is
-    // fetched before the position is known.
-    constexpr int QP = REP * 64, ITEMS = QP + 64 + ATT_D;
-    static_assert(ITEMS <= 2 * GQA_THREADS, "two set-up items per thread");
-    float fa[2] = {0.f, 0.f}, fb[2] = {0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int it = tid + k * GQA_THREADS;
-        if (it < QP) {
-            const int h = it >> 6, i = it & 63;
-            fa[k] = (float)qb_[h * ATT_D + i]; fb[k] = (float)qb_[h * ATT_D + i + 64];
-        } else if (it < QP + 64) {
-            fa[k] = (float)kn[it - QP]; fb[k] = (float)kn[it - QP + 64];
-        } else if (it < ITEMS) {
-            fa[k] = (float)vn[it - QP - 64];
-        }
-    }
-    const int64_t pos64 = *pos_ptr;
-    if (pos64 < 0 || pos64 >= max_len) {         // nothing sensible to do: defined output, no access outside the cache
-        for (int it = tid; it < REP * ATT_D; it += GQA_THREADS)
-            out[((int64_t)b * heads + head0) * ATT_D + it] = (half_t)0;
-        return;
-    }
-    const int pos = (int)pos64;
-    half_t *kc = kcache + ((int64_t)b * kv_heads + hk) * max_len * ATT_D;
-    half_t *vc = vcache + ((int64_t)b * kv_heads + hk) * max_len * ATT_D;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int it = tid + k * GQA_THREADS;
-        if (it < QP + 64) {
-            const int i = it & 63;
-            const float c = (float)cosv[(int64_t)pos * (ATT_D / 2) + i], sn = (float)sinv[(int64_t)pos * (ATT_D / 2) + i];
-            const half_t lo = (half_t)(fa[k] * c - fb[k] * sn), hi = (half_t)(fb[k] * c + fa[k] * sn);
-            if (it < QP) { qrot[it >> 6][i] = lo; qrot[it >> 6][i + 64] = hi; }
-            else { knew[i] = lo; knew[i + 64] = hi; }
-        } else if (it < ITEMS) {
-            vnew[it - QP - 64] = (half_t)fa[k];
-        }
-    }
-    __syncthreads();
-    if (head0 % rep == 0 && tid < ATT_D) {       // one workgroup of the KV head appends this position to the cache
-        kc[(int64_t)pos * ATT_D + tid] = knew[tid];
-        vc[(int64_t)pos * ATT_D + tid] = vnew[tid];
-    }
-
-    half2_t qreg[REP][4];                        // this lane's 8 dimensions of every query
-#pragma unroll
-    for (int h = 0; h < REP; h++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) qreg[h][e] = *reinterpret_cast<const half2_t *>(&qrot[h][8 * lane16 + 2 * e]);
-    const float scale2 = 0.08838834764831845f * 1.4426950408889634f;    // 1 / sqrt(128) * log2(e)
-    float m[REP], l[REP], acc[REP][8];
-#pragma unroll
-    for (int h = 0; h < REP; h++) {
-        m[h] = -INFINITY;
-        l[h] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[h][e] = 0.f;
-    }
-    auto fold = [&](const half8_t k8, const half8_t v8) {
-        float vf[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) vf[e] = (float)v8[e];
-#pragma unroll
-        for (int h = 0; h < REP; h++) {
-            float d = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                d = __builtin_amdgcn_fdot2(qreg[h][e], (half2_t){k8[2 * e], k8[2 * e + 1]}, d, false);
-            const float sc = row_sum16(d) * scale2;                  // the same value in all 16 lanes of the group
-            const float mn = fmaxf(m[h], sc);
-            const float r = __builtin_amdgcn_exp2f(m[h] - mn), w = __builtin_amdgcn_exp2f(sc - mn);   // exp2(-inf) = 0 on the first position
-            l[h] = l[h] * r + w;
-#pragma unroll
-            for (int e = 0; e < 8; e++) acc[h][e] = acc[h][e] * r + w * vf[e];
-            m[h] = mn;
+        for (int j = 0; j < 8; j++) {
+            const half8_t v = {v8[0][j], v8[1][j], v8[2][j], v8[3][j], v8[0][j], v8[1][j], v8[2][j], v8[3][j]};
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p8, acc[j], 0, 0, 0);
         }
     };
-    constexpr int GROUPS = GQA_THREADS / 16;
-    for (int p0 = grp; p0 < pos; p0 += 4 * GROUPS) {
-        half8_t k8[4], v8[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int p = min(p0 + GROUPS * j, pos - 1);
-            k8[j] = *reinterpret_cast<const half8_t *>(kc + (int64_t)p * ATT_D + 8 * lane16);
-            v8[j] = *reinterpret_cast<const half8_t *>(vc + (int64_t)p * ATT_D + 8 * lane16);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (p0 + GROUPS * j < pos) fold(k8[j], v8[j]);
+    while (t < tiles) {
+        const float4_t s = scores();
+        const int next = t + step;
+        if (next < tiles) fetch_k(next);
+        fold(s, pos - t * ATT_TILE);
+        if (next < tiles) fetch_v(next);
+        t = next;
     }
-    if (grp == 0)      // this step's own k and v, from LDS
-        fold(*reinterpret_cast<const half8_t *>(knew + 8 * lane16), *reinterpret_cast<const half8_t *>(vnew + 8 * lane16));
-
-    // the four groups of a wave (lanes 16 and 32 apart), then the waves through LDS
+    if (own) {                                   // this step's own k and v, from LDS: a tile with one position
 #pragma unroll
-    for (int h = 0; h < REP; h++) {
-#pragma unroll
-        for (int o = 16; o <= 32; o <<= 1) {
-            const float m2 = __shfl_xor(m[h], o, 64), l2 = __shfl_xor(l[h], o, 64);
-            const float mn = fmaxf(m[h], m2);
-            const float r1 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[h] - mn);
-            const float r2 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m2 - mn);
-            l[h] = l[h] * r1 + l2 * r2;
-#pragma unroll
-            for (int e = 0; e < 8; e++) acc[h][e] = acc[h][e] * r1 + __shfl_xor(acc[h][e], o, 64) * r2;
-            m[h] = mn;
+        for (int c = 0; c < 4; c++) {
+            k8[c] = *reinterpret_cast<const half8_t *>(&knew[32 * c + 8 * g]);
+            v8[c] = *reinterpret_cast<const half8_t *>(&vnew[8 * r16]);
         }
-        if ((tid & 63) == 0) { wm[h][wave] = m[h]; wl[h][wave] = l[h]; }
-        if ((tid & 63) < 16) {
+        fold(scores(), 1);
+    }
+
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (r16 < HP) {
+        if (g == 0) { wm[r16][wave] = m; wl[r16][wave] = l; }
 #pragma unroll
-            for (int e = 0; e < 8; e++) wacc[h][wave][8 * lane16 + e] = acc[h][e];
+        for (int i = 0; i < 4; i++) {            // row 4 g + i of product j is dimension 8 (4 g + i) + j
+            float *to = &wacc[r16][wave][8 * (4 * g + i)];
+            *reinterpret_cast<float4_t *>(to) = (float4_t){acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+            *reinterpret_cast<float4_t *>(to + 4) = (float4_t){acc[4][i], acc[5][i], acc[6][i], acc[7][i]};
         }
     }
     __syncthreads();
-    for (int it = tid; it < REP * ATT_D; it += GQA_THREADS) {
+    for (int it = tid; it < HP * ATT_D; it += THREADS) {
         const int h = it >> 7, dim = it & (ATT_D - 1);
         float mx = wm[h][0];
 #pragma unroll
-        for (int w = 1; w < GQA_WAVES; w++) mx = fmaxf(mx, wm[h][w]);
+        for (int w = 1; w < WAVES; w++) mx = fmaxf(mx, wm[h][w]);
         float o = 0.f, den = 0.f;
 #pragma unroll
-        for (int w = 0; w < GQA_WAVES; w++) {
-            const float r = wl[h][w] > 0.f ? __builtin_amdgcn_exp2f(wm[h][w] - mx) : 0.f;     // waves that saw no position
+        for (int w = 0; w < WAVES; w++) {
+            const float r = wl[h][w] != 0.f ? __builtin_amdgcn_exp2f(wm[h][w] - mx) : 0.f;    // 0: a wave that saw no position
             o += r * wacc[h][w][dim];
             den += r * wl[h][w];
         }
-        out[((int64_t)b * heads + head0 + h) * ATT_D + dim] = (half_t)(o / den);
+        if (split) {                             // part[head][split][max, sum, pad, pad, weighted v]
+            float *to = part + (((int64_t)b * heads + head0 + h) * gridDim.y + blockIdx.y) * ATT_PART;
+            to[4 + dim] = o;
+            if (dim == 0) { to[0] = mx; to[1] = den; }
+        } else {
+            orow[it] = (half_t)(o / den);
+        }
     }
+}
+
+// The splits of one head put together: every load is requested at once, one memory round trip.
+template <int MAXS>
+__global__ __launch_bounds__(ATT_D) void attention_merge_kernel(const float *__restrict__ part, const int64_t *__restrict__ pos_ptr,
+                                                                half_t *__restrict__ out, int splits, int max_len) {
+    const int dim = threadIdx.x;
+    const float *p = part + (int64_t)blockIdx.x * splits * ATT_PART;
+    const int64_t pos = *pos_ptr;
+    float m[MAXS], l[MAXS], v[MAXS];
+#pragma unroll
+    for (int i = 0; i < MAXS; i++) {
+        const float *q = p + (int64_t)(i < splits ? i : 0) * ATT_PART;
+        m[i] = q[0]; l[i] = i < splits ? q[1] : 0.f; v[i] = q[4 + dim];
+    }
+    if (pos >= 0 && pos <= ATT_WHOLE) return;    // written by the first launch
+    if (pos < 0 || pos >= max_len) {             // nothing was summed
+        out[(int64_t)blockIdx.x * ATT_D + dim] = (half_t)0;
+        return;
+    }
+    float mx = m[0], o = 0.f, den = 0.f;
+#pragma unroll
+    for (int i = 1; i < MAXS; i++) mx = fmaxf(mx, m[i]);
+#pragma unroll
+    for (int i = 0; i < MAXS; i++) {
+        const float r = l[i] != 0.f ? __builtin_amdgcn_exp2f(m[i] - mx) : 0.f;
+        o += l[i] != 0.f ? r * v[i] : 0.f;
+        den += r * l[i];
+    }
+    out[(int64_t)blockIdx.x * ATT_D + dim] = (half_t)(o / den);
 }
 
 // Greedy token: index of the largest of V fp16 values per row (the lowest index among
@@ -387,26 +334,56 @@ int bs_launch_rmsnorm(const half_t *x, const half_t *weight, half_t *y, int T, i
     return BS_OK;
 }
 
+template <int HP, int WAVES, bool SPLIT>
+static void launch_attention(const half_t *qkv, half_t *kcache, half_t *vcache, const half_t *cos, const half_t *sin,
+                             const int64_t *pos, half_t *out, float *part, int splits, int B, int heads, int kv_heads, int max_len,
+                             hipStream_t s) {
+    attention_decode_kernel<HP, WAVES, SPLIT><<<dim3((int64_t)B * heads / HP, splits), WAVES * 64, 0, s>>>(
+        qkv, kcache, vcache, cos, sin, pos, out, part, B, heads, kv_heads, max_len);
+}
+
+// Parts that the positions are cut into (1: not cut).  One KV head's rows go through one CU at about 60 GB/s, so few heads over
+// a long cache leave the chip idle; the parts cost a second, summing launch.  32 heads, 8 KV heads, one sequence, not cut / cut:
+// 29 / 10 us at position 3000, 17 / 10 at 1500 (two sequences), 6.9 / 8.1 at 384, and only the length of the cache is known here.
+static int attention_splits(int B, int heads, int kv_heads, int max_len) {
+    const int rep = heads / kv_heads, hp = rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1;
+    const int64_t groups = (int64_t)B * heads / hp;
+    if (max_len < ATT_SPLIT_LEN || groups > 128 || groups < 1) return 1;
+    const int64_t fill = 256 / groups, longest = bs_cdiv(max_len, 256);       // 256 positions: one tile for each of 16 waves
+    const int64_t splits = fill < longest ? fill : longest;
+    return splits > ATT_MAX_SPLITS ? ATT_MAX_SPLITS : (int)splits;
+}
+
+int64_t bs_attention_parts_bytes(int B, int heads, int kv_heads, int max_len) {
+    const int splits = attention_splits(B, heads, kv_heads, max_len);
+    return splits > 1 ? (int64_t)B * heads * splits * ATT_PART * 4 : 0;
+}
+
 int bs_launch_attention_decode(const half_t *qkv, half_t *kcache, half_t *vcache, const half_t *cos, const half_t *sin,
                                const int64_t *pos, half_t *out, int B, int heads, int kv_heads, int head_dim,
-                               int max_len, hipStream_t s) {
+                               int max_len, float *part, hipStream_t s) {
     if (head_dim != ATT_D || max_len > ATT_MAX_LEN) return BS_ERR_SHAPE;
-    // Long caches and more (head, sequence) pairs than CUs: four (or two) query heads of a KV
-    // head per workgroup, a quarter (half) of the cache fetches.  A workgroup of the grouped
-    // kernel takes longer than one of the per-head kernel (3000 positions: 55 us against 25),
-    // so it only pays once the per-head kernel would need more than one round of workgroups
-    // (8 sequences x 64 heads at 2100 positions: 45 us against 79).
     const int rep = heads / kv_heads;
-    const bool grouped = max_len >= 1024 && (int64_t)B * heads > 256;
-    if (grouped && rep % 4 == 0)
-        attention_decode_gqa_kernel<4><<<dim3(heads / 4, B), GQA_THREADS, 0, s>>>(qkv, kcache, vcache, cos, sin, pos, out,
-                                                                                 heads, kv_heads, max_len);
-    else if (grouped && rep % 2 == 0)
-        attention_decode_gqa_kernel<2><<<dim3(heads / 2, B), GQA_THREADS, 0, s>>>(qkv, kcache, vcache, cos, sin, pos, out,
-                                                                                 heads, kv_heads, max_len);
-    else
-        attention_decode_kernel<<<dim3(heads, B), ATT_THREADS, 0, s>>>(qkv, kcache, vcache, cos, sin, pos, out, heads,
-                                                                      kv_heads, max_len);
+    const int64_t all = (int64_t)B * heads;
+    const int splits = part ? attention_splits(B, heads, kv_heads, max_len) : 1;
+    if (splits > 1) {
+        auto *launch = rep % 4 == 0 ? launch_attention<4, 16, true> : rep % 2 == 0 ? launch_attention<2, 16, true> : launch_attention<1, 16, true>;
+        launch(qkv, kcache, vcache, cos, sin, pos, out, part, splits, B, heads, kv_heads, max_len, s);
+        BS_LAUNCH_CHECK();
+        auto *merge = splits <= 4 ? attention_merge_kernel<4> : splits <= 8 ? attention_merge_kernel<8> : attention_merge_kernel<ATT_MAX_SPLITS>;
+        merge<<<(int)all, ATT_D, 0, s>>>(part, pos, out, splits, max_len);
+        BS_LAUNCH_CHECK();
+        return BS_OK;
+    }
+    // As few heads of a KV head per workgroup as still give at most one workgroup of 16 waves per CU: a CU's time is that of
+    // one KV head's rows however many heads share them, and fewer heads merge faster.  Past that, workgroups of 8 waves, two
+    // on a CU.
+    const int hp = rep % 4 == 0 && all > 512 ? 4 : rep % 2 == 0 && all > 256 ? 2 : 1;
+    const bool wide = all / hp <= 256;
+    auto *launch = hp == 4 ? (wide ? launch_attention<4, 16, false> : launch_attention<4, 8, false>)
+                 : hp == 2 ? (wide ? launch_attention<2, 16, false> : launch_attention<2, 8, false>)
+                           : (wide ? launch_attention<1, 16, false> : launch_attention<1, 8, false>);
+    launch(qkv, kcache, vcache, cos, sin, pos, out, nullptr, 1, B, heads, kv_heads, max_len, s);
     BS_LAUNCH_CHECK();
     return BS_OK;
 }

@@ -330,6 +330,8 @@ PyObject *host_make_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
             s.sin = (const void *)(uintptr_t)p[4];
             s.pos = (const int64_t *)(uintptr_t)p[5];
             s.out = (void *)(uintptr_t)p[6];
+            const int64_t need = ok ? bs_attention_decode_workspace_bytes(s.B, s.heads, s.kv_heads, s.head_dim, s.max_len) : 0;
+            if (need > steps->need) steps->need = need;      // (a shape that is not taken is reported by the call)
         }
         if (!ok || PyErr_Occurred()) {
             delete steps;
@@ -371,8 +373,8 @@ PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
                 st = bs_rmsnorm_f16(s.x, s.weight, s.y, s.T, s.N, s.eps, stream);
                 if (st != BS_OK) return raise_status(st, "bs_rmsnorm_f16");
             } else {
-                st = bs_attention_decode_f16(s.qkv, s.kcache, s.vcache, s.cos, s.sin, s.pos, s.out, s.B, s.heads, s.kv_heads, s.head_dim,
-                                             s.max_len, stream);
+                st = bs_attention_decode_ws_f16(s.qkv, s.kcache, s.vcache, s.cos, s.sin, s.pos, s.out, s.B, s.heads, s.kv_heads, s.head_dim,
+                                                s.max_len, ws.mutable_data_ptr(), ws.numel(), stream);
                 if (st != BS_OK) return raise_status(st, "bs_attention_decode_f16");
             }
         }

@@ -198,9 +198,12 @@ def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, ou
         raise ValueError("cos / sin must be contiguous [max_len, head_dim / 2]")
     y = out if out is not None else torch.empty((B, heads * d), dtype=torch.float16, device=dev)
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().bs_attention_decode_f16(_lib.ptr(qkv), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(_f16c(cos)),
-                                                      _lib.ptr(_f16c(sin)), _lib.ptr(pos), _lib.ptr(y), B, heads, kv_heads,
-                                                      d, max_len, _lib.stream_ptr(dev)), "bs_attention_decode_f16")
+        need = _lib.lib().bs_attention_decode_workspace_bytes(B, heads, kv_heads, d, max_len)
+        ws = _lib.workspace(dev, need) if need > 0 else None
+        _lib.check(_lib.lib().bs_attention_decode_ws_f16(_lib.ptr(qkv), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(_f16c(cos)),
+                                                         _lib.ptr(_f16c(sin)), _lib.ptr(pos), _lib.ptr(y), B, heads, kv_heads, d, max_len,
+                                                         _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(dev)),
+                   "bs_attention_decode_ws_f16")
     return y
 
 

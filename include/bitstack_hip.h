@@ -326,6 +326,16 @@ int bs_attention_decode_f16(const void *qkv, void *kcache, void *vcache, const v
                             int max_len, void *stream);
 
 /*
+ * The same with scratch.  Few heads over a long cache leave most of the chip idle; with bs_attention_decode_workspace_bytes
+ * (0: none is used; negative: an error status) of 16-byte aligned device scratch, which calls on one stream may share, the
+ * positions are cut into parts and summed by a second launch.  Without it, or with less, the call is bs_attention_decode_f16.
+ */
+int64_t bs_attention_decode_workspace_bytes(int B, int heads, int kv_heads, int head_dim, int max_len);
+int bs_attention_decode_ws_f16(const void *qkv, void *kcache, void *vcache, const void *cos, const void *sin,
+                               const int64_t *pos, void *out, int B, int heads, int kv_heads, int head_dim,
+                               int max_len, void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * out[b] = index of the largest of x[b, 0..V) (fp16; the lowest index among
  * equal values): the greedy token of a decode step from the logits.  Rows must
  * start 16-byte aligned (V % 8 == 0 when B > 1).  No counterpart in the

@@ -1,0 +1,65 @@
+"""Decode attention at the edges of its tiles: 16 positions a tile, 8 or 16 waves taking tiles in turn, 1, 2 or 4 heads a
+workgroup, workgroups of a KV head dealt to one XCD or not."""
+import numpy as np
+import pytest
+import torch
+
+from bitstack_amd.utils import inference_utils as IU
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,heads,kv", [(1, 32, 8), (2, 6, 2), (9, 32, 8), (9, 32, 32), (17, 32, 16), (17, 32, 8), (33, 32, 8)])
+def test_attention_at_tile_edges(B, heads, kv):
+    d, max_len = 128, 272
+    g = torch.Generator().manual_seed(B * 100 + heads + kv)
+    k = torch.randn(B, kv, max_len, d, generator=g).half()
+    v = torch.randn(B, kv, max_len, d, generator=g).half()
+    qkv = torch.randn(B, (heads + 2 * kv) * d, generator=g).half()
+    cos, sin = torch.ones(max_len, d // 2).half().cuda(), torch.zeros(max_len, d // 2).half().cuda()   # the rotation is exact
+    q = qkv[:, :heads * d].double().view(B, kv, heads // kv, d)
+    kn, vn = qkv[:, heads * d:(heads + kv) * d].view(B, kv, d), qkv[:, (heads + kv) * d:].view(B, kv, d)
+    kd, vd = k.cuda(), v.cuda()
+    for at in (0, 1, 15, 16, 17, 127, 128, 129, 255, 256, 257, max_len - 1):
+        print(f"attention B={B} heads={heads} kv={kv} at={at}", flush=True)
+        kc, vc = kd.clone(), vd.clone()
+        kc[:, :, at + 1:] = float("nan")        # what lies behind the position is not read
+        vc[:, :, at:] = float("nan")
+        got = IU.attention_decode_hip(qkv.cuda(), kc, vc, cos, sin, torch.tensor([at], device="cuda"), heads, kv)
+        ks, vs = k[:, :, :at + 1].double().clone(), v[:, :, :at + 1].double().clone()
+        ks[:, :, at], vs[:, :, at] = kn.double(), vn.double()
+        p = torch.softmax(torch.matmul(q, ks.transpose(2, 3)) / d ** 0.5, -1)
+        ref = torch.matmul(p, vs).reshape(B, heads * d).numpy()
+        assert torch.equal(kc[:, :, at].cpu(), kn) and torch.equal(vc[:, :, at].cpu(), vn)
+        assert torch.equal(kc[:, :, :at].cpu(), k[:, :, :at]) and torch.equal(vc[:, :, :at].cpu(), v[:, :, :at])
+        # one rounding to fp16; scores of size up to 5 in fp32 sums of 128 terms move the weights by at most 2^-14 of themselves
+        bound = np.abs(ref) * 2.0 ** -11 + np.abs(vs.numpy()).max() * 2.0 ** -14 + 2.0 ** -25
+        assert (np.abs(got.double().cpu().numpy() - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("B,heads,kv,max_len", [(1, 32, 8, 4096), (1, 32, 8, 1025), (1, 6, 2, 4100), (3, 8, 4, 2050), (2, 16, 16, 1100), (16, 32, 8, 1030)])
+def test_attention_over_split_positions(B, heads, kv, max_len):
+    """Few heads over a long cache: the positions in parts (up to 16 of them, most without a position early on)."""
+    d = 128
+    g = torch.Generator(device="cuda").manual_seed(B + heads + max_len)
+    k = torch.randn(B, kv, max_len, d, generator=g, device="cuda").half()
+    v = torch.randn(B, kv, max_len, d, generator=g, device="cuda").half()
+    qkv = torch.randn(B, (heads + 2 * kv) * d, generator=g, device="cuda").half()
+    cos, sin = torch.ones(max_len, d // 2).half().cuda(), torch.zeros(max_len, d // 2).half().cuda()
+    q = qkv[:, :heads * d].double().view(B, kv, heads // kv, d)
+    kn, vn = qkv[:, heads * d:(heads + kv) * d].view(B, kv, d), qkv[:, (heads + kv) * d:].view(B, kv, d)
+    for at in (0, 16, 511, 512, 513, 768, 769, 1000, max_len - 1):
+        print(f"split attention B={B} heads={heads} kv={kv} max_len={max_len} at={at}", flush=True)
+        kc, vc = k.clone(), v.clone()
+        kc[:, :, at:] = float("nan")
+        vc[:, :, at:] = float("nan")
+        got = IU.attention_decode_hip(qkv, kc, vc, cos, sin, torch.tensor([at], device="cuda"), heads, kv).double()
+        ks, vs = k[:, :, :at + 1].double(), v[:, :, :at + 1].double()
+        ks[:, :, at], vs[:, :, at] = kn.double(), vn.double()
+        p = torch.softmax((q.unsqueeze(3) * ks.unsqueeze(2)).sum(-1) / d ** 0.5, -1)
+        ref = (p.unsqueeze(-1) * vs.unsqueeze(2)).sum(3).reshape(B, heads * d)
+        assert torch.equal(kc[:, :, at], kn) and torch.equal(vc[:, :, at], vn)
+        bound = ref.abs() * 2.0 ** -11 + vs.abs().max() * 2.0 ** -14 + 2.0 ** -25      # as above
+        assert bool(((got - ref).abs() <= bound).all())
+    for at in (-1, max_len):                     # outside of the cache: zeros
+        assert not IU.attention_decode_hip(qkv, kc, vc, cos, sin, torch.tensor([at], device="cuda"), heads, kv).any()

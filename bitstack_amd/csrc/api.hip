@@ -251,6 +251,39 @@ extern "C" int bs_rmsnorm_f16(const void *x, const void *weight, void *y, int T,
     return bs_launch_rmsnorm((const half_t *)x, (const half_t *)weight, (half_t *)y, T, H, eps, (hipStream_t)stream);
 }
 
+extern "C" int bs_add_rmsnorm_f16(const void *x, const void *add, void *sum, const void *weight, void *y, int T, int H, float eps,
+                                  void *stream) {
+    if (T < 0 || H <= 0 || H % 8 != 0 || H > 16384) return BS_ERR_SHAPE;
+    if (T == 0) return BS_OK;
+    if (!x || !add || !sum || !weight || !y) return BS_ERR_NULL;
+    if (!bs_aligned(x, 16) || !bs_aligned(add, 16) || !bs_aligned(sum, 16) || !bs_aligned(weight, 16) || !bs_aligned(y, 16))
+        return BS_ERR_ALIGN;
+    return bs_launch_add_rmsnorm((const half_t *)x, (const half_t *)add, (half_t *)sum, (const half_t *)weight, (half_t *)y, T, H, eps,
+                                 (hipStream_t)stream);
+}
+
+extern "C" int bs_rope_store_f16(void *q, const void *k, const void *v, const void *cos, const void *sin, void *kcache, void *vcache,
+                                 int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream) {
+    if (B < 0 || n < 0 || n > max_len || heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 2 != 0 ||
+        (int64_t)B * n > INT32_MAX || ((int64_t)heads + 3 * (int64_t)kv_heads) * head_dim > INT32_MAX)
+        return BS_ERR_SHAPE;
+    if (B == 0 || n == 0) return BS_OK;
+    if (!q || !k || !v || !cos || !sin || !kcache || !vcache) return BS_ERR_NULL;
+    if (!bs_aligned(q, 16) || !bs_aligned(k, 16) || !bs_aligned(v, 16) || !bs_aligned(cos, 16) || !bs_aligned(sin, 16) ||
+        !bs_aligned(kcache, 16) || !bs_aligned(vcache, 16))
+        return BS_ERR_ALIGN;
+    return bs_launch_rope_store((half_t *)q, (const half_t *)k, (const half_t *)v, (const half_t *)cos, (const half_t *)sin,
+                                (half_t *)kcache, (half_t *)vcache, B, n, heads, kv_heads, head_dim, max_len, (hipStream_t)stream);
+}
+
+extern "C" int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream) {
+    if (count < 0 || count > ((int64_t)1 << 40)) return BS_ERR_SHAPE;
+    if (count == 0) return BS_OK;
+    if (!gate || !up || !y) return BS_ERR_NULL;
+    if (!bs_aligned(gate, 16) || !bs_aligned(up, 16) || !bs_aligned(y, 16)) return BS_ERR_ALIGN;
+    return bs_launch_silu_mul((const half_t *)gate, (const half_t *)up, (half_t *)y, count, (hipStream_t)stream);
+}
+
 static int attention_shape(int B, int heads, int kv_heads, int head_dim, int max_len) {
     return B < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || head_dim != 128 || max_len < 1 || max_len > 8192 ? BS_ERR_SHAPE
                                                                                                                           : BS_OK;

@@ -104,6 +104,12 @@ int bs_prefill_mode();
 // decode-step kernels around the linears (decode_step.hip)
 int bs_launch_argmax(const half_t *x, int64_t *out, int B, int V, hipStream_t s);
 int bs_launch_rmsnorm(const half_t *x, const half_t *weight, half_t *y, int T, int H, float eps, hipStream_t s);
+int bs_launch_add_rmsnorm(const half_t *x, const half_t *add, half_t *sum, const half_t *weight, half_t *y, int T, int H, float eps,
+                          hipStream_t s);
+// the same places when a whole prompt goes through a layer (prefill_step.hip)
+int bs_launch_rope_store(half_t *q, const half_t *k, const half_t *v, const half_t *cos, const half_t *sin, half_t *kcache,
+                         half_t *vcache, int B, int n, int heads, int kv_heads, int d, int max_len, hipStream_t s);
+int bs_launch_silu_mul(const half_t *gate, const half_t *up, half_t *y, int64_t count, hipStream_t s);
 int bs_launch_attention_decode(const half_t *qkv, half_t *kcache, half_t *vcache, const half_t *cos, const half_t *sin,
                                const int64_t *pos, half_t *out, int B, int heads, int kv_heads, int head_dim,
                                int max_len, float *part, hipStream_t s);

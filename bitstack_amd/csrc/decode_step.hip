@@ -12,10 +12,12 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// One workgroup per row; the row stays in registers between the two passes.
+// One workgroup per row; the row stays in registers between the two passes.  ADD: the row is fp16(x + add), which is written
+// too (sum may be x or add: a thread reads what it overwrites).
 constexpr int RMS_THREADS = 256, RMS_MAX_CHUNKS = 8;   // 256 * 8 * 8 halves = 16384 columns
 
-__global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *__restrict__ x,
+template <bool ADD>
+__global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *x, const half_t *add, half_t *sum,
                                                               const half_t *__restrict__ weight,
                                                               half_t *__restrict__ y, int H, float eps) {
     __shared__ float wsum[RMS_THREADS / 64];
@@ -29,6 +31,10 @@ __global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *__re
         const int col = (c * RMS_THREADS + tid) * 8;
         if (col < H) {
             v[c] = *reinterpret_cast<const half8_t *>(xr + col);
+            if (ADD) {
+                v[c] += *reinterpret_cast<const half8_t *>(add + (int64_t)blockIdx.x * H + col);
+                *reinterpret_cast<half8_t *>(sum + (int64_t)blockIdx.x * H + col) = v[c];
+            }
 #pragma unroll
             for (int e = 0; e < 8; e++) ss += (float)v[c][e] * (float)v[c][e];
         }
@@ -329,7 +335,15 @@ int bs_launch_argmax(const half_t *x, int64_t *out, int B, int V, hipStream_t s)
 
 int bs_launch_rmsnorm(const half_t *x, const half_t *weight, half_t *y, int T, int H, float eps, hipStream_t s) {
     if (H > RMS_THREADS * RMS_MAX_CHUNKS * 8) return BS_ERR_SHAPE;
-    rmsnorm_kernel<<<T, RMS_THREADS, 0, s>>>(x, weight, y, H, eps);
+    rmsnorm_kernel<false><<<T, RMS_THREADS, 0, s>>>(x, nullptr, nullptr, weight, y, H, eps);
+    BS_LAUNCH_CHECK();
+    return BS_OK;
+}
+
+int bs_launch_add_rmsnorm(const half_t *x, const half_t *add, half_t *sum, const half_t *weight, half_t *y, int T, int H, float eps,
+                          hipStream_t s) {
+    if (H > RMS_THREADS * RMS_MAX_CHUNKS * 8) return BS_ERR_SHAPE;
+    rmsnorm_kernel<true><<<T, RMS_THREADS, 0, s>>>(x, add, sum, weight, y, H, eps);
     BS_LAUNCH_CHECK();
     return BS_OK;
 }

@@ -179,6 +179,52 @@ def rmsnorm_hip(x, weight, eps, out=None):
     return y.view(x.shape)
 
 
+def add_rmsnorm_hip(x, add, weight, eps):
+    """(x + add, its RMSNorm): the sum takes the place of `add` (fp16, contiguous) and is returned."""
+    dev = _lib.require_gpu(x, add, weight)
+    H = x.shape[-1]
+    if x.dtype != torch.float16:             # a residual that is kept wider stays so
+        x = x + add
+        return x, rmsnorm_hip(x, weight, eps)
+    if add.dtype != torch.float16 or not add.is_contiguous() or add.shape != x.shape:
+        raise ValueError("add must be a contiguous fp16 tensor of x's shape")
+    x2, weight = _f16c(x).view(-1, H), _f16c(weight)
+    y = torch.empty_like(x2)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().bs_add_rmsnorm_f16(_lib.ptr(x2), _lib.ptr(add), _lib.ptr(add), _lib.ptr(weight), _lib.ptr(y), x2.shape[0], H,
+                                                 float(eps), _lib.stream_ptr(dev)), "bs_add_rmsnorm_f16")
+    return add, y.view(x.shape)
+
+
+def rope_store_hip(q, k, v, cos, sin, kcache, vcache, n):
+    """Positions 0 .. n - 1 of B sequences: RoPE on q [B * n, heads * d] in place, rotated k and v [B * n, kv * d] into the
+    caches [B, kv, max_len, d]."""
+    dev = _lib.require_gpu(q, k, v, cos, sin, kcache, vcache)
+    B, kv, max_len, d = kcache.shape
+    for t, shape in ((q, (B * n, q.shape[-1])), (k, (B * n, kv * d)), (v, (B * n, kv * d)), (cos, (max_len, d // 2)), (sin, (max_len, d // 2)),
+                     (kcache, kcache.shape), (vcache, kcache.shape)):
+        if t.dtype != torch.float16 or not t.is_contiguous() or tuple(t.shape) != tuple(shape):
+            raise ValueError(f"expected a contiguous fp16 tensor {tuple(shape)}, got {t.dtype} {tuple(t.shape)}")
+    if n > max_len or q.shape[1] % d:
+        raise ValueError("q must hold whole heads, n at most max_len positions")
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().bs_rope_store_f16(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(cos), _lib.ptr(sin), _lib.ptr(kcache),
+                                                _lib.ptr(vcache), B, n, q.shape[1] // d, kv, d, max_len, _lib.stream_ptr(dev)),
+                   "bs_rope_store_f16")
+
+
+def silu_mul_hip(gate, up):
+    """silu(gate) * up in gate's place (contiguous fp16 tensors of one shape)."""
+    dev = _lib.require_gpu(gate, up)
+    for t in (gate, up):
+        if t.dtype != torch.float16 or not t.is_contiguous() or t.shape != gate.shape:
+            raise ValueError("gate and up must be contiguous fp16 tensors of one shape")
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().bs_silu_mul_f16(_lib.ptr(gate), _lib.ptr(up), _lib.ptr(gate), gate.numel(), _lib.stream_ptr(dev)),
+                   "bs_silu_mul_f16")
+    return gate
+
+
 def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, out=None):
     """One decode position for B sequences: RoPE on q and k of qkv [B, (heads + 2 kv) * d],
     append k, v at *pos to the caches [B, kv, max_len, d], attention over 0..*pos;

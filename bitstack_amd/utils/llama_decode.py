@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from bitstack_amd import _lib
 from bitstack_amd._lib import EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU
 from bitstack_amd.modules.BitStackLinear import BitStackLinear
-from bitstack_amd.utils.inference_utils import MatrixGroup, argmax_hip, rmsnorm_hip
+from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
 
 PROJ = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj",
         "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj")
@@ -443,33 +443,50 @@ class SyntheticLlamaDecoder:
             if hidden is None or tuple(hidden.shape) != (B * n, s.hidden):
                 raise ValueError("resuming needs the kept input of that layer")
             x = hidden
-        cos, sin = self.cos[:n].view(1, 1, n, d // 2), self.sin[:n].view(1, 1, n, d // 2)
+        # sequences per attention call: a short prompt does not fill the chip by itself, and 1 GiB bounds the scores of an
+        # attention that would keep them
+        together = max(1, min(B, (1 << 30) // (4 * s.heads * n * n)))
+        # caches or tables of another layout or type, if a caller has put such in place, take the torch operations
+        plain = all(t.dtype == torch.float16 and t.is_contiguous() for t in (self.kcache, self.vcache, self.cos, self.sin))
+        hn = None
         for L in range(first_layer, s.layers):
             if keep is not None:
                 keep.append(x)
             lin = self.lin[L]
-            hn = rmsnorm_hip(x, self.norm_w[L, 0], s.rms_eps)
-            q = lin["self_attn.q_proj"](hn).view(B, n, s.heads, d).transpose(1, 2)
-            k = lin["self_attn.k_proj"](hn).view(B, n, s.kv_heads, d).transpose(1, 2)
-            v = lin["self_attn.v_proj"](hn).view(B, n, s.kv_heads, d).transpose(1, 2)
-            q, k = self._rope(q, cos, sin), self._rope(k, cos, sin)
-            self.kcache[L][:, :, :n].copy_(k)
-            self.vcache[L][:, :, :n].copy_(v)
-            ctx = torch.empty(B, n, s.hidden, dtype=torch.float16, device=self.dev)
-            for b in range(B):                                            # one sequence at a time bounds the scratch
-                o = F.scaled_dot_product_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], is_causal=True, enable_gqa=True)
-                ctx[b].copy_(o[0].transpose(0, 1).reshape(n, s.hidden))
-            x = x + lin["self_attn.o_proj"](ctx.view(B * n, s.hidden))
-            hn = rmsnorm_hip(x, self.norm_w[L, 1], s.rms_eps)
-            act = F.silu(lin["mlp.gate_proj"](hn))
-            act.mul_(lin["mlp.up_proj"](hn))
-            x = x + lin["mlp.down_proj"](act)
+            if hn is None:
+                hn = rmsnorm_hip(x, self.norm_w[L, 0], s.rms_eps)
+            q, k, v = (lin[p](hn) for p in PROJ[:3])
+            kc, vc = self.kcache[L], self.vcache[L]
+            if plain:
+                rope_store_hip(q, k, v, self.cos, self.sin, kc, vc, n)
+                q = q.view(B, n, s.heads, d).transpose(1, 2)
+            else:
+                cos, sin = self.cos[:n].view(1, 1, n, d // 2), self.sin[:n].view(1, 1, n, d // 2)
+                q = self._rope(q.view(B, n, s.heads, d).transpose(1, 2), cos, sin)
+                kc[:, :, :n].copy_(self._rope(k.view(B, n, s.kv_heads, d).transpose(1, 2), cos, sin))
+                vc[:, :, :n].copy_(v.view(B, n, s.kv_heads, d).transpose(1, 2))
+            k, v = kc[:, :, :n].to(q.dtype), vc[:, :, :n].to(q.dtype)
+            ctx = [F.scaled_dot_product_attention(q[b:b + together], k[b:b + together], v[b:b + together], is_causal=True, enable_gqa=True)
+                   .transpose(1, 2).reshape(-1, s.hidden) for b in range(0, B, together)]
+            ctx = ctx[0] if len(ctx) == 1 else torch.cat(ctx)
+            x, hn = add_rmsnorm_hip(x, lin["self_attn.o_proj"](ctx), self.norm_w[L, 1], s.rms_eps)
+            act = silu_mul_hip(lin["mlp.gate_proj"](hn), lin["mlp.up_proj"](hn))
+            down = lin["mlp.down_proj"](act)
+            if L + 1 < s.layers:
+                x, hn = add_rmsnorm_hip(x, down, self.norm_w[L + 1, 0], s.rms_eps)
+            elif all_logits:
+                x, hn = add_rmsnorm_hip(x, down, self.final_norm, s.rms_eps)
+            else:                                                         # the last position of each sequence
+                x, down = (t.view(B, n, s.hidden)[:, -1].contiguous() for t in (x, down))
+                x, hn = add_rmsnorm_hip(x, down, self.final_norm, s.rms_eps)
+        if hn is None:                                                    # no layer ran: first_layer is the layer count
+            x = x if all_logits else x.view(B, n, s.hidden)[:, -1].contiguous()
+            hn = rmsnorm_hip(x, self.final_norm, s.rms_eps)
         if all_logits:
-            full = F.linear(rmsnorm_hip(x, self.final_norm, s.rms_eps), self.lm_head).view(B, n, -1)
+            full = F.linear(hn, self.lm_head).view(B, n, -1)
             self.logits = full[:, -1].contiguous()
         else:
-            last = x.view(B, n, s.hidden)[:, -1].contiguous()
-            self.logits = F.linear(rmsnorm_hip(last, self.final_norm, s.rms_eps), self.lm_head)
+            self.logits = F.linear(hn, self.lm_head)
         self.token.copy_(self.logits.argmax(-1))
         self.pos.fill_(n)
         return full if all_logits else None

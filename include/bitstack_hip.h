@@ -310,6 +310,20 @@ int bs_forward_group_rms(const bs_matrix *mats, int n, int N, int K, const void 
  */
 int bs_rmsnorm_f16(const void *x, const void *weight, void *y, int T, int H, float eps, void *stream);
 
+/* sum[T, H] = fp16(x + add), y = RMSNorm of sum as above: a residual sum and the norm behind it.  sum may be x or add. */
+int bs_add_rmsnorm_f16(const void *x, const void *add, void *sum, const void *weight, void *y, int T, int H, float eps, void *stream);
+
+/*
+ * A whole prompt of B sequences, positions 0 .. n - 1: rotate q [B * n, heads * head_dim] in place and k into kcache
+ * (rotate-half RoPE, cos/sin [n or more, head_dim / 2]), copy v into vcache ([B, kv_heads, max_len, head_dim]; n <= max_len,
+ * head_dim even).  Computed in fp32, rounded once, as the decode step does.
+ */
+int bs_rope_store_f16(void *q, const void *k, const void *v, const void *cos, const void *sin, void *kcache, void *vcache,
+                      int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream);
+
+/* y[count] = fp16(silu(gate) * up); y may be gate or up. */
+int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream);
+
 /*
  * One decode position of grouped-query attention for B sequences that are all
  * at position *pos (device int64): rotate q and k of `qkv`

@@ -1,0 +1,56 @@
+"""The kernels between the linears of a prompt pass, against float64 (one rounding to fp16) or the plain kernel."""
+import pytest
+import torch
+
+from bitstack_amd.utils import inference_utils as IU
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,n,heads,kv,d,max_len", [(1, 1, 2, 1, 128, 1), (2, 5, 32, 8, 128, 9), (3, 7, 4, 4, 64, 7), (1, 3, 5, 1, 16, 4),
+                                                    (2, 3, 3, 3, 6, 5), (2, 33, 6, 2, 256, 40), (1, 2, 2, 2, 24, 2)])
+def test_rope_store(B, n, heads, kv, d, max_len):
+    g = torch.Generator(device="cuda").manual_seed(d + n)
+    q, k, v = (torch.randn(B * n, h * d, generator=g, device="cuda").half() for h in (heads, kv, kv))
+    ang = torch.rand(max_len, d // 2, generator=g, device="cuda") * 6.28
+    cos, sin = ang.cos().half(), ang.sin().half()
+    kc, vc = (torch.full((B, kv, max_len, d), 7.0, device="cuda").half() for _ in range(2))
+    rot = q.clone()
+    IU.rope_store_hip(rot, k, v, cos, sin, kc, vc, n)
+
+    def want(x, h):
+        x = x.double().view(B, n, h, d)
+        c, s = (t[:n].double().view(1, n, 1, d // 2) for t in (cos, sin))
+        a, b = x[..., :d // 2], x[..., d // 2:]
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+
+    # one rounding to fp16, and sums of two products of size up to 2^3 in fp32
+    def check(got, ref):
+        assert bool(((got.double() - ref).abs() <= ref.abs() * 2.0 ** -11 + 2.0 ** -20).all())
+    check(rot.view(B, n, heads, d), want(q, heads))
+    check(kc[:, :, :n].transpose(1, 2), want(k, kv))
+    assert torch.equal(vc[:, :, :n].transpose(1, 2), v.view(B, n, kv, d))
+    assert bool((kc[:, :, n:] == 7).all()) and bool((vc[:, :, n:] == 7).all())
+
+
+@pytest.mark.parametrize("count", [1, 7, 8, 9, 2047, 2048, 2049, 5 * 14336])
+def test_silu_mul(count):
+    g = torch.Generator(device="cuda").manual_seed(count)
+    a, b = (torch.randn(count, generator=g, device="cuda").half() * 4 for _ in range(2))
+    ref = a.double() * torch.sigmoid(a.double()) * b.double()
+    up = b.clone()
+    y = IU.silu_mul_hip(a, up)
+    assert y.data_ptr() == a.data_ptr() and torch.equal(up, b)
+    # one rounding (subnormal below 2^-14), and 2^-20 for exp, quotient and product in fp32
+    assert bool(((y.double() - ref).abs() <= ref.abs() * (2.0 ** -11 + 2.0 ** -20) + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("T,H", [(1, 8), (3, 2048), (2, 2056), (5, 4096), (2, 16384)])
+def test_add_rmsnorm(T, H):
+    g = torch.Generator(device="cuda").manual_seed(H)
+    x, add = (torch.randn(T, H, generator=g, device="cuda").half() for _ in range(2))
+    w = torch.rand(H, generator=g, device="cuda").half()
+    x0, want = x.clone(), x + add
+    s, y = IU.add_rmsnorm_hip(x, add, w, 1e-5)
+    assert torch.equal(s, want) and torch.equal(x, x0) and s.data_ptr() == add.data_ptr()
+    assert torch.equal(y, IU.rmsnorm_hip(want, w, 1e-5))

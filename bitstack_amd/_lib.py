@@ -59,6 +59,7 @@ SIGNATURES.update({
     "bs_rmsnorm_f16": (_I, [_P, _P, _P, _I, _I, ctypes.c_float, _P]),
     "bs_add_rmsnorm_f16": (_I, [_P, _P, _P, _P, _P, _I, _I, ctypes.c_float, _P]),
     "bs_rope_store_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
+    "bs_attention_prefill_f16": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
     "bs_silu_mul_f16": (_I, [_P, _P, _P, _L, _P]),
     "bs_attention_decode_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "bs_attention_decode_workspace_bytes": (_L, [_I, _I, _I, _I, _I]),

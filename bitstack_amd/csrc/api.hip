@@ -276,6 +276,18 @@ extern "C" int bs_rope_store_f16(void *q, const void *k, const void *v, const vo
                                 (half_t *)kcache, (half_t *)vcache, B, n, heads, kv_heads, head_dim, max_len, (hipStream_t)stream);
 }
 
+extern "C" int bs_attention_prefill_f16(const void *q, const void *kcache, const void *vcache, void *out, int B, int n, int heads,
+                                        int kv_heads, int head_dim, int max_len, void *stream) {
+    if (B < 0 || n < 0 || n > max_len || n > 32 * 65535 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || head_dim != 128 ||
+        (int64_t)B * heads > INT32_MAX)
+        return BS_ERR_SHAPE;
+    if (B == 0 || n == 0) return BS_OK;
+    if (!q || !kcache || !vcache || !out) return BS_ERR_NULL;
+    if (!bs_aligned(q, 16) || !bs_aligned(kcache, 16) || !bs_aligned(vcache, 16) || !bs_aligned(out, 16)) return BS_ERR_ALIGN;
+    return bs_launch_attention_prefill((const half_t *)q, (const half_t *)kcache, (const half_t *)vcache, (half_t *)out, B, n, heads,
+                                       kv_heads, max_len, (hipStream_t)stream);
+}
+
 extern "C" int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream) {
     if (count < 0 || count > ((int64_t)1 << 40)) return BS_ERR_SHAPE;
     if (count == 0) return BS_OK;

@@ -213,6 +213,23 @@ def rope_store_hip(q, k, v, cos, sin, kcache, vcache, n):
                    "bs_rope_store_f16")
 
 
+def attention_prefill_hip(q, kcache, vcache, n):
+    """Causal attention of positions 0 .. n - 1: q [B * n, heads * 128] rotated, k and v in the caches [B, kv, max_len, 128];
+    returns [B * n, heads * 128]."""
+    dev = _lib.require_gpu(q, kcache, vcache)
+    B, kv, max_len, d = kcache.shape
+    for t in (q, kcache, vcache):
+        if t.dtype != torch.float16 or not t.is_contiguous():
+            raise ValueError("q and the caches must be contiguous fp16 tensors")
+    if vcache.shape != kcache.shape or q.dim() != 2 or q.shape[0] != B * n or q.shape[1] % d or n > max_len:
+        raise ValueError("q must hold whole heads of B * n positions, n at most max_len")
+    y = torch.empty_like(q)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().bs_attention_prefill_f16(_lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(y), B, n, q.shape[1] // d,
+                                                       kv, d, max_len, _lib.stream_ptr(dev)), "bs_attention_prefill_f16")
+    return y
+
+
 def silu_mul_hip(gate, up):
     """silu(gate) * up in gate's place (contiguous fp16 tensors of one shape)."""
     dev = _lib.require_gpu(gate, up)

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from bitstack_amd import _lib
 from bitstack_amd._lib import EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU
 from bitstack_amd.modules.BitStackLinear import BitStackLinear
-from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
+from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, attention_prefill_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
 
 PROJ = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj",
         "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj")
@@ -421,6 +421,21 @@ class SyntheticLlamaDecoder:
         argmax_hip(self.logits, out=self.token)
         self.pos.add_(1)
 
+    def _attend(self, q, k, v, kc, vc, n, stored):
+        """prefill()'s attention on torch operations, for heads of other sizes or caches of another layout or type: `stored`
+        means that q is rotated and k, v are in the cache."""
+        s, B, d = self.s, self.batch, self.s.head_dim
+        q = q.view(B, n, s.heads, d).transpose(1, 2)
+        if not stored:
+            cos, sin = self.cos[:n].view(1, 1, n, d // 2), self.sin[:n].view(1, 1, n, d // 2)
+            q = self._rope(q, cos, sin)
+            kc[:, :, :n].copy_(self._rope(k.view(B, n, s.kv_heads, d).transpose(1, 2), cos, sin))
+            vc[:, :, :n].copy_(v.view(B, n, s.kv_heads, d).transpose(1, 2))
+        k, v = kc[:, :, :n].to(q.dtype), vc[:, :, :n].to(q.dtype)
+        # one sequence at a time bounds the scratch
+        return torch.cat([F.scaled_dot_product_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], is_causal=True, enable_gqa=True)
+                          .transpose(1, 2).reshape(n, s.hidden) for b in range(B)])
+
     @torch.no_grad()
     def prefill(self, prompt: torch.Tensor, all_logits=False, first_layer=0, hidden=None, keep=None):
         """The whole prompt [batch, len] in one pass: every linear sees batch * len tokens (the
@@ -443,9 +458,6 @@ class SyntheticLlamaDecoder:
             if hidden is None or tuple(hidden.shape) != (B * n, s.hidden):
                 raise ValueError("resuming needs the kept input of that layer")
             x = hidden
-        # sequences per attention call: a short prompt does not fill the chip by itself, and 1 GiB bounds the scores of an
-        # attention that would keep them
-        together = max(1, min(B, (1 << 30) // (4 * s.heads * n * n)))
         # caches or tables of another layout or type, if a caller has put such in place, take the torch operations
         plain = all(t.dtype == torch.float16 and t.is_contiguous() for t in (self.kcache, self.vcache, self.cos, self.sin))
         hn = None
@@ -459,16 +471,10 @@ class SyntheticLlamaDecoder:
             kc, vc = self.kcache[L], self.vcache[L]
             if plain:
                 rope_store_hip(q, k, v, self.cos, self.sin, kc, vc, n)
-                q = q.view(B, n, s.heads, d).transpose(1, 2)
+            if plain and d == 128:
+                ctx = attention_prefill_hip(q, kc, vc, n)
             else:
-                cos, sin = self.cos[:n].view(1, 1, n, d // 2), self.sin[:n].view(1, 1, n, d // 2)
-                q = self._rope(q.view(B, n, s.heads, d).transpose(1, 2), cos, sin)
-                kc[:, :, :n].copy_(self._rope(k.view(B, n, s.kv_heads, d).transpose(1, 2), cos, sin))
-                vc[:, :, :n].copy_(v.view(B, n, s.kv_heads, d).transpose(1, 2))
-            k, v = kc[:, :, :n].to(q.dtype), vc[:, :, :n].to(q.dtype)
-            ctx = [F.scaled_dot_product_attention(q[b:b + together], k[b:b + together], v[b:b + together], is_causal=True, enable_gqa=True)
-                   .transpose(1, 2).reshape(-1, s.hidden) for b in range(0, B, together)]
-            ctx = ctx[0] if len(ctx) == 1 else torch.cat(ctx)
+                ctx = self._attend(q, k, v, kc, vc, n, plain)
             x, hn = add_rmsnorm_hip(x, lin["self_attn.o_proj"](ctx), self.norm_w[L, 1], s.rms_eps)
             act = silu_mul_hip(lin["mlp.gate_proj"](hn), lin["mlp.up_proj"](hn))
             down = lin["mlp.down_proj"](act)

@@ -321,6 +321,14 @@ int bs_add_rmsnorm_f16(const void *x, const void *add, void *sum, const void *we
 int bs_rope_store_f16(void *q, const void *k, const void *v, const void *cos, const void *sin, void *kcache, void *vcache,
                       int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream);
 
+/*
+ * Causal attention of a whole prompt: out[B * n, heads * head_dim] = softmax(q k^T / sqrt(head_dim)) v, query j over positions
+ * 0 .. j, q [B * n, heads * head_dim] already rotated, k and v from the caches [B, kv_heads, max_len, head_dim] (n <= max_len).
+ * head_dim == 128.  Scores, sums and the softmax in fp32, its weights in fp16 for the product with v.
+ */
+int bs_attention_prefill_f16(const void *q, const void *kcache, const void *vcache, void *out, int B, int n, int heads, int kv_heads,
+                             int head_dim, int max_len, void *stream);
+
 /* y[count] = fp16(silu(gate) * up); y may be gate or up. */
 int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream);
 

@@ -54,3 +54,26 @@ def test_add_rmsnorm(T, H):
     s, y = IU.add_rmsnorm_hip(x, add, w, 1e-5)
     assert torch.equal(s, want) and torch.equal(x, x0) and s.data_ptr() == add.data_ptr()
     assert torch.equal(y, IU.rmsnorm_hip(want, w, 1e-5))
+
+
+@pytest.mark.parametrize("B,n,heads,kv,max_len", [(1, 1, 4, 1, 1), (2, 15, 8, 2, 20), (1, 16, 6, 3, 16), (3, 17, 5, 5, 40), (1, 31, 32, 8, 31),
+                                                  (2, 32, 8, 8, 33), (1, 33, 12, 4, 64), (2, 64, 4, 2, 64), (1, 65, 4, 4, 70), (1, 517, 8, 2, 600)])
+def test_attention_prefill(B, n, heads, kv, max_len):
+    print(f"prompt attention B={B} n={n} heads={heads} kv={kv}", flush=True)
+    d, rep = 128, heads // kv
+    g = torch.Generator(device="cuda").manual_seed(n + heads)
+    q = torch.randn(B * n, heads * d, generator=g, device="cuda").half()
+    kc, vc = (torch.randn(B, kv, max_len, d, generator=g, device="cuda").half() for _ in range(2))
+    kc[:, :, n:], vc[:, :, n:] = float("nan"), float("nan")          # not read
+    got = IU.attention_prefill_hip(q, kc, vc, n).double().view(B, n, kv, rep, d)
+    qd = q.double().view(B, n, kv, rep, d).permute(0, 2, 3, 1, 4)
+    kd, vd = (c[:, :, :n].double().unsqueeze(2).expand(B, kv, rep, n, d).contiguous() for c in (kc, vc))
+    s = torch.matmul(qd, kd.transpose(-1, -2).contiguous()) / d ** 0.5
+    s = s.masked_fill(torch.ones(n, n, device="cuda").triu(1).bool(), float("-inf"))
+    ref = torch.matmul(torch.softmax(s, -1), vd).permute(0, 3, 1, 2, 4)
+    # one rounding of the result, and one of every softmax weight (2^-11 of itself at most, weights sum to one; those below
+    # 2^-14 of the largest lose up to 2^-25 of it each)
+    bound = ref.abs() * 2.0 ** -11 + vd.abs().max() * (2.0 ** -11 + n * 2.0 ** -25)
+    assert bool(((got - ref).abs() <= bound).all())
+    # and not far from the error of one rounding over the whole
+    assert float((got - ref).norm() / ref.norm()) < 6e-4

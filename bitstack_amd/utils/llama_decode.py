@@ -394,6 +394,8 @@ class SyntheticLlamaDecoder:
             if tuple(t.shape) != shape or t.dtype != dtype or not t.is_contiguous() or not t.is_cuda:
                 raise ValueError(f"the decode step needs a contiguous {dtype} tensor {shape} on the GPU, got {t.dtype} {tuple(t.shape)}")
         xa, xb, qkv, ctx, act = (t.data_ptr() for t in (self._xa, self._xb, self._qkv, self._ctx, self._act))
+        kcache, vcache, cos, sin, pos = key
+        layer = 2 * B * s.kv_heads * self.max_len * d                      # bytes of a layer's cache
 
         def group(g, x, y, epilogue, eps=None, residual=0):
             return ("group", ctypes.addressof(g.arr), g.n, g.N, g.K, x, B, eps, epilogue, residual, y)
@@ -401,8 +403,7 @@ class SyntheticLlamaDecoder:
         items = []
         for L, grp in enumerate(self._groups):
             items.append(group(grp["qkv"], xa, qkv, EPI_NONE, eps=s.rms_eps))
-            items.append(("attention", qkv, self.kcache[L].data_ptr(), self.vcache[L].data_ptr(), self.cos.data_ptr(), self.sin.data_ptr(),
-                          self.pos.data_ptr(), ctx, B, s.heads, s.kv_heads, d, self.max_len))
+            items.append(("attention", qkv, kcache + L * layer, vcache + L * layer, cos, sin, pos, ctx, B, s.heads, s.kv_heads, d, self.max_len))
             items.append(group(grp["o"], ctx, xb, EPI_RESIDUAL, residual=xa))
             items.append(group(grp["gate_up"], xb, act, EPI_SWIGLU, eps=s.rms_eps))
             items.append(group(grp["down"], act, xa, EPI_RESIDUAL, residual=xb))

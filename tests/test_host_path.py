@@ -63,3 +63,13 @@ def test_scratch_is_one_tensor_per_stream_and_outgrown_ones_stay():
         assert b.data_ptr() != a.data_ptr()
     big = _lib.workspace(dev, 2 * a.numel() + 1)
     assert big.numel() > 2 * a.numel() and big.data_ptr() != a.data_ptr()
+
+
+def test_the_host_module_has_no_thread_local_storage():
+    """A module with a TLS segment that is never touched slows every thread-local access of the process (glibc before 2.39)."""
+    import struct
+    _lib.host()
+    data = open(_lib.host().__file__, "rb").read()
+    offset, size, count = struct.unpack_from("<Q", data, 32)[0], *struct.unpack_from("<HH", data, 54)
+    kinds = [struct.unpack_from("<I", data, offset + k * size)[0] for k in range(count)]
+    assert 1 in kinds and 7 not in kinds      # PT_LOAD, PT_TLS

@@ -58,9 +58,11 @@ SIGNATURES.update({
     "bs_argmax_f16": (_I, [_P, _P, _I, _I, _P]),
     "bs_rmsnorm_f16": (_I, [_P, _P, _P, _I, _I, ctypes.c_float, _P]),
     "bs_add_rmsnorm_f16": (_I, [_P, _P, _P, _P, _P, _I, _I, ctypes.c_float, _P]),
-    "bs_rope_store_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
-    "bs_attention_prefill_f16": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
-    "bs_silu_mul_f16": (_I, [_P, _P, _P, _L, _P]),
+    "bs_rope_store_f16": (_I, [_P, _I, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
+    "bs_forward_cat_workspace_bytes": (_L, [_P, _I, _I, _I, _I]),
+    "bs_forward_cat": (_I, [_P, _I, _I, _I, _P, _I, _P, _P, _L, _P]),
+    "bs_attention_prefill_f16": (_I, [_P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
+    "bs_silu_mul_f16": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "bs_attention_decode_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "bs_attention_decode_workspace_bytes": (_L, [_I, _I, _I, _I, _I]),
     "bs_attention_decode_ws_f16": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P]),

@@ -262,10 +262,11 @@ extern "C" int bs_add_rmsnorm_f16(const void *x, const void *add, void *sum, con
                                  (hipStream_t)stream);
 }
 
-extern "C" int bs_rope_store_f16(void *q, const void *k, const void *v, const void *cos, const void *sin, void *kcache, void *vcache,
-                                 int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream) {
+extern "C" int bs_rope_store_f16(void *q, int ldq, const void *k, const void *v, int ldkv, const void *cos, const void *sin,
+                                 void *kcache, void *vcache, int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream) {
     if (B < 0 || n < 0 || n > max_len || heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 2 != 0 ||
-        (int64_t)B * n > INT32_MAX || ((int64_t)heads + 3 * (int64_t)kv_heads) * head_dim > INT32_MAX)
+        (int64_t)B * n > INT32_MAX || ((int64_t)heads + 3 * (int64_t)kv_heads) * head_dim > INT32_MAX ||
+        ldq < (int64_t)heads * head_dim || ldkv < (int64_t)kv_heads * head_dim)
         return BS_ERR_SHAPE;
     if (B == 0 || n == 0) return BS_OK;
     if (!q || !k || !v || !cos || !sin || !kcache || !vcache) return BS_ERR_NULL;
@@ -273,27 +274,82 @@ extern "C" int bs_rope_store_f16(void *q, const void *k, const void *v, const vo
         !bs_aligned(kcache, 16) || !bs_aligned(vcache, 16))
         return BS_ERR_ALIGN;
     return bs_launch_rope_store((half_t *)q, (const half_t *)k, (const half_t *)v, (const half_t *)cos, (const half_t *)sin,
-                                (half_t *)kcache, (half_t *)vcache, B, n, heads, kv_heads, head_dim, max_len, (hipStream_t)stream);
+                                (half_t *)kcache, (half_t *)vcache, ldq, ldkv, B, n, heads, kv_heads, head_dim, max_len,
+                                (hipStream_t)stream);
 }
 
-extern "C" int bs_attention_prefill_f16(const void *q, const void *kcache, const void *vcache, void *out, int B, int n, int heads,
+extern "C" int bs_attention_prefill_f16(const void *q, int ldq, const void *kcache, const void *vcache, void *out, int B, int n, int heads,
                                         int kv_heads, int head_dim, int max_len, void *stream) {
     if (B < 0 || n < 0 || n > max_len || n > 32 * 65535 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || head_dim != 128 ||
-        (int64_t)B * heads > INT32_MAX)
+        (int64_t)B * heads > INT32_MAX || ldq < (int64_t)heads * head_dim || ldq % 8 != 0)
         return BS_ERR_SHAPE;
     if (B == 0 || n == 0) return BS_OK;
     if (!q || !kcache || !vcache || !out) return BS_ERR_NULL;
     if (!bs_aligned(q, 16) || !bs_aligned(kcache, 16) || !bs_aligned(vcache, 16) || !bs_aligned(out, 16)) return BS_ERR_ALIGN;
-    return bs_launch_attention_prefill((const half_t *)q, (const half_t *)kcache, (const half_t *)vcache, (half_t *)out, B, n, heads,
+    return bs_launch_attention_prefill((const half_t *)q, (const half_t *)kcache, (const half_t *)vcache, (half_t *)out, ldq, B, n, heads,
                                        kv_heads, max_len, (hipStream_t)stream);
 }
 
-extern "C" int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream) {
-    if (count < 0 || count > ((int64_t)1 << 40)) return BS_ERR_SHAPE;
-    if (count == 0) return BS_OK;
+extern "C" int bs_silu_mul_f16(const void *gate, const void *up, void *y, int T, int width, int ld, void *stream) {
+    if (T < 0 || width <= 0 || width > INT32_MAX - 4096 || ld < width) return BS_ERR_SHAPE;
+    if (T == 0) return BS_OK;
     if (!gate || !up || !y) return BS_ERR_NULL;
     if (!bs_aligned(gate, 16) || !bs_aligned(up, 16) || !bs_aligned(y, 16)) return BS_ERR_ALIGN;
-    return bs_launch_silu_mul((const half_t *)gate, (const half_t *)up, (half_t *)y, count, (hipStream_t)stream);
+    if (T > 1 && (width % 8 != 0 || ld % 8 != 0)) return BS_ERR_ALIGN;
+    return bs_launch_silu_mul((const half_t *)gate, (const half_t *)up, (half_t *)y, T, width, ld, (hipStream_t)stream);
+}
+
+// Several matrices on the same x as one product: rebuilt below each other, so that a narrow one (k, v) does not leave most of
+// the chip idle by itself.  us one by one / as one: 4096 + 1024 + 1024 rows of 4096 columns, 4 blocks: 84 / 61 at 130 tokens,
+// 103 / 72 at 700, 133 / 98 at 1400, 282 / 267 at 6000; 2 x 8192 rows of 3072 (96 MiB): 85 / 70, 111 / 101, 165 / 161, 501 / 491.
+// The limit is where the rebuilt weights no longer stay in the cache between the two launches: 2 x 10752 rows of 3072 (126 MiB)
+// 106 / 84 at 130 tokens but 359 / 363 at 3000, 2 x 12288 of 4096 (192 MiB) 198 / 223 at 700, 2 x 14336 of 4096 230 / 248.
+// With narrow matrices it pays further up: 8192 + 1024 + 1024 rows of 8192 (160 MiB) 207 / 163 at 700, 815 / 820 at 6000.
+constexpr int64_t CAT_WEIGHT = 96ll << 20, CAT_WEIGHT_FEW = 128ll << 20, CAT_WEIGHT_NARROW = 160ll << 20;   // bytes
+constexpr int CAT_FEW = 2048, CAT_NARROW_TOKENS = 4500;
+static int64_t cat_rows(const bs_matrix *mats, int n, int N, int K, int T) {
+    if (!mats || n < 2 || n > BS_MAX_GROUP) return 0;
+    int64_t rows = 0;
+    for (int j = 0; j < n; j++) {
+        if (mats[j].bias || mats[j].I < 1 || forward_dims(mats[j].I, mats[j].M, N, K, T) != BS_OK ||
+            bs_forward_path(mats[j].I, mats[j].M, N, K, T) != BS_PATH_REBUILD || dense_wants_library(mats[j].M, N))
+            return 0;
+        rows += mats[j].M;
+    }
+    int64_t narrowest = rows;
+    for (int j = 0; j < n; j++)
+        if (mats[j].M < narrowest) narrowest = mats[j].M;
+    const int64_t limit = 8 * narrowest <= rows && T <= CAT_NARROW_TOKENS ? CAT_WEIGHT_NARROW : T <= CAT_FEW ? CAT_WEIGHT_FEW : CAT_WEIGHT;
+    return N % 8 == 0 && rows * N * 2 <= limit ? rows : 0;
+}
+
+extern "C" int64_t bs_forward_cat_workspace_bytes(const bs_matrix *mats, int n, int N, int K, int T) {
+    if (T <= 0 || N <= 0) return 0;
+    const int64_t rows = cat_rows(mats, n, N, K, T);
+    return rows ? round_up(rows * N * 2, 256) + round_up(bs_linear_parts_bytes(T, (int)rows, N), 256) : 0;
+}
+
+extern "C" int bs_forward_cat(const bs_matrix *mats, int n, int N, int K, const void *x, int T, void *y, void *workspace,
+                              int64_t workspace_bytes, void *stream) {
+    const int64_t need = bs_forward_cat_workspace_bytes(mats, n, N, K, T);
+    if (need == 0) return BS_ERR_SHAPE;
+    if (!x || !y) return BS_ERR_NULL;
+    for (int j = 0; j < n; j++) {
+        if (!mats[j].packed || !mats[j].u || !mats[j].vt) return BS_ERR_NULL;
+        if (!bs_aligned(mats[j].packed, 16) || !bs_aligned(mats[j].vt, 16) || !bs_aligned(mats[j].u, 8)) return BS_ERR_ALIGN;
+    }
+    if (!bs_aligned(x, 16) || !bs_aligned(y, 2)) return BS_ERR_ALIGN;
+    if (!workspace || workspace_bytes < need || !bs_aligned(workspace, 256)) return BS_ERR_WORKSPACE;
+    half_t *w = (half_t *)workspace;
+    int64_t rows = 0;
+    for (int j = 0; j < n; j++) {
+        const int st = bs_launch_reconstruct_packed((const uint8_t *)mats[j].packed, (const half_t *)mats[j].u, (const half_t *)mats[j].vt,
+                                                    w + rows * N, mats[j].I, mats[j].M, N, K, (hipStream_t)stream);
+        if (st != BS_OK) return st;
+        rows += mats[j].M;
+    }
+    return bs_launch_linear_parts((const half_t *)x, w, nullptr, (half_t *)y, T, (int)rows, N,
+                                  (float *)((char *)workspace + round_up(rows * N * 2, 256)), (hipStream_t)stream);
 }
 
 static int attention_shape(int B, int heads, int kv_heads, int head_dim, int max_len) {

@@ -108,10 +108,10 @@ int bs_launch_add_rmsnorm(const half_t *x, const half_t *add, half_t *sum, const
                           hipStream_t s);
 // the same places when a whole prompt goes through a layer (prefill_step.hip)
 int bs_launch_rope_store(half_t *q, const half_t *k, const half_t *v, const half_t *cos, const half_t *sin, half_t *kcache,
-                         half_t *vcache, int B, int n, int heads, int kv_heads, int d, int max_len, hipStream_t s);
-int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int B, int n, int heads,
+                         half_t *vcache, int ldq, int ldkv, int B, int n, int heads, int kv_heads, int d, int max_len, hipStream_t s);
+int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int ldq, int B, int n, int heads,
                                 int kv_heads, int max_len, hipStream_t s);
-int bs_launch_silu_mul(const half_t *gate, const half_t *up, half_t *y, int64_t count, hipStream_t s);
+int bs_launch_silu_mul(const half_t *gate, const half_t *up, half_t *y, int T, int width, int ld, hipStream_t s);
 int bs_launch_attention_decode(const half_t *qkv, half_t *kcache, half_t *vcache, const half_t *cos, const half_t *sin,
                                const int64_t *pos, half_t *out, int B, int heads, int kv_heads, int head_dim,
                                int max_len, float *part, hipStream_t s);

@@ -15,14 +15,14 @@ template <int V>
 __global__ __launch_bounds__(THREADS) void rope_store_kernel(half_t *__restrict__ q, const half_t *__restrict__ k,
                                                              const half_t *__restrict__ v, const half_t *__restrict__ cosv,
                                                              const half_t *__restrict__ sinv, half_t *__restrict__ kcache,
-                                                             half_t *__restrict__ vcache, int n, int heads, int kv_heads, int d,
-                                                             int max_len) {
+                                                             half_t *__restrict__ vcache, int ldq, int ldkv, int n, int heads,
+                                                             int kv_heads, int d, int max_len) {
     typedef half_t vec_t __attribute__((ext_vector_type(V)));
     const int token = blockIdx.x, b = token / n, pos = token % n, d2 = d / 2;
     const int per = d2 / V, qi = heads * per, ki = kv_heads * per;               // items of q and of k; v has 2 * ki
-    q += (int64_t)token * heads * d;
-    k += (int64_t)token * kv_heads * d;
-    v += (int64_t)token * kv_heads * d;
+    q += (int64_t)token * ldq;
+    k += (int64_t)token * ldkv;
+    v += (int64_t)token * ldkv;
     cosv += (int64_t)pos * d2;
     sinv += (int64_t)pos * d2;
     const int64_t head_stride = (int64_t)max_len * d, at = (int64_t)b * kv_heads * head_stride + (int64_t)pos * d;
@@ -49,10 +49,14 @@ __global__ __launch_bounds__(THREADS) void rope_store_kernel(half_t *__restrict_
     }
 }
 
-// y = silu(gate) * up; eight values per thread.  y may be gate or up: a thread reads what it overwrites.  1400 x 14336: 36 us as
+// y[T, width] = silu(gate) * up, rows of gate and up ld apart; eight values per thread.  y may be gate or up (ld == width): a
+// thread reads what it overwrites.  1400 x 14336: 36 us as
 // two operations, 18.9 now (120 MB: 6.4 TB/s).
-__global__ __launch_bounds__(THREADS) void silu_mul_kernel(const half_t *gate, const half_t *up, half_t *y, int64_t count) {
-    const int64_t i = ((int64_t)blockIdx.x * THREADS + threadIdx.x) * 8;
+__global__ __launch_bounds__(THREADS) void silu_mul_kernel(const half_t *gate, const half_t *up, half_t *y, int width, int ld) {
+    const int i = (blockIdx.x * THREADS + threadIdx.x) * 8, count = width;
+    gate += (int64_t)blockIdx.y * ld;
+    up += (int64_t)blockIdx.y * ld;
+    y += (int64_t)blockIdx.y * width;
     auto one = [](float a, float b) { return (half_t)(a / (1.f + __expf(-a)) * b); };
     if (i + 8 <= count) {
         const half8_t a = *reinterpret_cast<const half8_t *>(gate + i), b = *reinterpret_cast<const half8_t *>(up + i);
@@ -61,7 +65,7 @@ __global__ __launch_bounds__(THREADS) void silu_mul_kernel(const half_t *gate, c
         for (int e = 0; e < 8; e++) o[e] = one((float)a[e], (float)b[e]);
         *reinterpret_cast<half8_t *>(y + i) = o;
     } else {
-        for (int64_t j = i; j < count; j++) y[j] = one((float)gate[j], (float)up[j]);
+        for (int j = i; j < count; j++) y[j] = one((float)gate[j], (float)up[j]);
     }
 }
 
@@ -80,7 +84,7 @@ constexpr int AP_D = 128, AP_Q = 32, AP_WAVES = 4;
 
 __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kcache,
                                                                              const half_t *__restrict__ vcache, half_t *__restrict__ out,
-                                                                             int n, int heads, int kv_heads, int max_len) {
+                                                                             int ldq, int n, int heads, int kv_heads, int max_len) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
     const int quads = (heads + AP_WAVES - 1) / AP_WAVES, b = blockIdx.x / quads, head = (blockIdx.x % quads) * AP_WAVES + wave;
     if (head >= heads) return;
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
     fetch_k(0);
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-        const half_t *p = q + ((int64_t)b * n + min(q0 + 16 * t + r16, n - 1)) * row + head * AP_D + 8 * g;
+        const half_t *p = q + ((int64_t)b * n + min(q0 + 16 * t + r16, n - 1)) * ldq + head * AP_D + 8 * g;
 #pragma unroll
         for (int c = 0; c < 4; c++) q8[t][c] = *reinterpret_cast<const half8_t *>(p + 32 * c);
     }
@@ -185,25 +189,28 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
 
 }  // namespace
 
-int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int B, int n, int heads,
+int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int ldq, int B, int n, int heads,
                                 int kv_heads, int max_len, hipStream_t s) {
     const dim3 grid((unsigned)(B * bs_cdiv(heads, AP_WAVES)), (unsigned)bs_cdiv(n, AP_Q));
-    attention_prefill_kernel<<<grid, AP_WAVES * 64, 0, s>>>(q, kcache, vcache, out, n, heads, kv_heads, max_len);
+    attention_prefill_kernel<<<grid, AP_WAVES * 64, 0, s>>>(q, kcache, vcache, out, ldq, n, heads, kv_heads, max_len);
     BS_LAUNCH_CHECK();
     return BS_OK;
 }
 
 int bs_launch_rope_store(half_t *q, const half_t *k, const half_t *v, const half_t *cos, const half_t *sin, half_t *kcache,
-                         half_t *vcache, int B, int n, int heads, int kv_heads, int d, int max_len, hipStream_t s) {
+                         half_t *vcache, int ldq, int ldkv, int B, int n, int heads, int kv_heads, int d, int max_len, hipStream_t s) {
     // 16-byte pieces where every row and half row starts on 16 bytes (the pointers do)
-    auto *kernel = d % 16 == 0 ? rope_store_kernel<8> : rope_store_kernel<1>;
-    kernel<<<B * n, THREADS, 0, s>>>(q, k, v, cos, sin, kcache, vcache, n, heads, kv_heads, d, max_len);
+    auto *kernel = d % 16 == 0 && ldq % 8 == 0 && ldkv % 8 == 0 ? rope_store_kernel<8> : rope_store_kernel<1>;
+    kernel<<<B * n, THREADS, 0, s>>>(q, k, v, cos, sin, kcache, vcache, ldq, ldkv, n, heads, kv_heads, d, max_len);
     BS_LAUNCH_CHECK();
     return BS_OK;
 }
 
-int bs_launch_silu_mul(const half_t *gate, const half_t *up, half_t *y, int64_t count, hipStream_t s) {
-    silu_mul_kernel<<<bs_cdiv(count, THREADS * 8), THREADS, 0, s>>>(gate, up, y, count);
+int bs_launch_silu_mul(const half_t *gate, const half_t *up, half_t *y, int T, int width, int ld, hipStream_t s) {
+    for (int t = 0; t < T; t += 65535) {         // (the grid's second dimension)
+        const dim3 grid((unsigned)bs_cdiv(width, THREADS * 8), (unsigned)(T - t < 65535 ? T - t : 65535));
+        silu_mul_kernel<<<grid, THREADS, 0, s>>>(gate + (int64_t)t * ld, up + (int64_t)t * ld, y + (int64_t)t * width, width, ld);
+    }
     BS_LAUNCH_CHECK();
     return BS_OK;
 }

@@ -196,50 +196,98 @@ def add_rmsnorm_hip(x, add, weight, eps):
     return add, y.view(x.shape)
 
 
+def _rows(t, shape):
+    """Row stride of a fp16 matrix whose rows are contiguous (a column slice of a wider one, for instance)."""
+    if t.dtype != torch.float16 or tuple(t.shape) != tuple(shape) or t.stride(1) != 1 or t.stride(0) < t.shape[1]:
+        raise ValueError(f"expected a fp16 matrix {tuple(shape)} with contiguous rows, got {t.dtype} {tuple(t.shape)} {t.stride()}")
+    return t.stride(0)
+
+
 def rope_store_hip(q, k, v, cos, sin, kcache, vcache, n):
     """Positions 0 .. n - 1 of B sequences: RoPE on q [B * n, heads * d] in place, rotated k and v [B * n, kv * d] into the
-    caches [B, kv, max_len, d]."""
+    caches [B, kv, max_len, d].  q, k and v may be column slices of one wider matrix."""
     dev = _lib.require_gpu(q, k, v, cos, sin, kcache, vcache)
     B, kv, max_len, d = kcache.shape
-    for t, shape in ((q, (B * n, q.shape[-1])), (k, (B * n, kv * d)), (v, (B * n, kv * d)), (cos, (max_len, d // 2)), (sin, (max_len, d // 2)),
-                     (kcache, kcache.shape), (vcache, kcache.shape)):
+    for t, shape in ((cos, (max_len, d // 2)), (sin, (max_len, d // 2)), (kcache, kcache.shape), (vcache, kcache.shape)):
         if t.dtype != torch.float16 or not t.is_contiguous() or tuple(t.shape) != tuple(shape):
             raise ValueError(f"expected a contiguous fp16 tensor {tuple(shape)}, got {t.dtype} {tuple(t.shape)}")
     if n > max_len or q.shape[1] % d:
         raise ValueError("q must hold whole heads, n at most max_len positions")
+    ldq, ldk, ldv = _rows(q, (B * n, q.shape[1])), _rows(k, (B * n, kv * d)), _rows(v, (B * n, kv * d))
+    if ldk != ldv:
+        raise ValueError("k and v must have the same row stride")
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().bs_rope_store_f16(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(cos), _lib.ptr(sin), _lib.ptr(kcache),
-                                                _lib.ptr(vcache), B, n, q.shape[1] // d, kv, d, max_len, _lib.stream_ptr(dev)),
-                   "bs_rope_store_f16")
+        _lib.check(_lib.lib().bs_rope_store_f16(_lib.ptr(q), ldq, _lib.ptr(k), _lib.ptr(v), ldk, _lib.ptr(cos), _lib.ptr(sin),
+                                                _lib.ptr(kcache), _lib.ptr(vcache), B, n, q.shape[1] // d, kv, d, max_len,
+                                                _lib.stream_ptr(dev)), "bs_rope_store_f16")
 
 
 def attention_prefill_hip(q, kcache, vcache, n):
-    """Causal attention of positions 0 .. n - 1: q [B * n, heads * 128] rotated, k and v in the caches [B, kv, max_len, 128];
-    returns [B * n, heads * 128]."""
+    """Causal attention of positions 0 .. n - 1: q [B * n, heads * 128] rotated (rows may be strided), k and v in the caches
+    [B, kv, max_len, 128]; returns [B * n, heads * 128]."""
     dev = _lib.require_gpu(q, kcache, vcache)
     B, kv, max_len, d = kcache.shape
-    for t in (q, kcache, vcache):
+    for t in (kcache, vcache):
         if t.dtype != torch.float16 or not t.is_contiguous():
-            raise ValueError("q and the caches must be contiguous fp16 tensors")
-    if vcache.shape != kcache.shape or q.dim() != 2 or q.shape[0] != B * n or q.shape[1] % d or n > max_len:
+            raise ValueError("the caches must be contiguous fp16 tensors")
+    if vcache.shape != kcache.shape or q.dim() != 2 or q.shape[1] % d or n > max_len:
         raise ValueError("q must hold whole heads of B * n positions, n at most max_len")
-    y = torch.empty_like(q)
+    ldq = _rows(q, (B * n, q.shape[1]))
+    y = torch.empty(q.shape, dtype=torch.float16, device=dev)
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().bs_attention_prefill_f16(_lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(y), B, n, q.shape[1] // d,
-                                                       kv, d, max_len, _lib.stream_ptr(dev)), "bs_attention_prefill_f16")
+        _lib.check(_lib.lib().bs_attention_prefill_f16(_lib.ptr(q), ldq, _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(y), B, n,
+                                                       q.shape[1] // d, kv, d, max_len, _lib.stream_ptr(dev)), "bs_attention_prefill_f16")
     return y
 
 
 def silu_mul_hip(gate, up):
-    """silu(gate) * up in gate's place (contiguous fp16 tensors of one shape)."""
+    """silu(gate) * up of two fp16 matrices: in gate's place if both are contiguous, else (column slices) a new matrix."""
     dev = _lib.require_gpu(gate, up)
-    for t in (gate, up):
-        if t.dtype != torch.float16 or not t.is_contiguous() or t.shape != gate.shape:
-            raise ValueError("gate and up must be contiguous fp16 tensors of one shape")
+    if up.shape != gate.shape or up.dtype != torch.float16 or gate.dtype != torch.float16:
+        raise ValueError("gate and up must be fp16 tensors of one shape")
+    if gate.is_contiguous() and up.is_contiguous():
+        y, T, width = gate, 1, gate.numel()
+        if width >= 1 << 31:                 # (the kernel counts a row in 32 bits)
+            T, width = gate.numel() // gate.shape[-1], gate.shape[-1]
+        ld = width
+    else:
+        T, width = gate.shape
+        y, ld = torch.empty(T, width, dtype=torch.float16, device=dev), _rows(gate, gate.shape)
+        if _rows(up, gate.shape) != ld:
+            raise ValueError("gate and up must have the same row stride")
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().bs_silu_mul_f16(_lib.ptr(gate), _lib.ptr(up), _lib.ptr(gate), gate.numel(), _lib.stream_ptr(dev)),
+        _lib.check(_lib.lib().bs_silu_mul_f16(_lib.ptr(gate), _lib.ptr(up), _lib.ptr(y), T, width, ld, _lib.stream_ptr(dev)),
                    "bs_silu_mul_f16")
-    return gate
+    return y
+
+
+def forward_cat_hip(modules, x):
+    """[T, M0 + M1 + ..]: what the modules (BitStackLinear, level 5) give for x [T, N], side by side from one product, or None
+    where that is not how they are computed (few tokens, a bias, another level, blocks not stacked)."""
+    from bitstack_amd.modules.BitStackLinear import BitStackLinear
+    for m in modules:
+        if type(m) is not BitStackLinear or m._forward_hooks or m._forward_pre_hooks:     # (a call of the module would do more)
+            return None
+        if m.fused_level != 5 or m.no_avd or m.bias is not None or getattr(m, "u", None) is None:
+            return None
+    if x.dtype != torch.float16 or x.dim() != 2 or not x.is_contiguous():
+        return None
+    stacked = [m._stacked() for m in modules]
+    if any(not t.is_contiguous() or t.device != x.device for s in stacked for t in s) or \
+            any(s[1].dtype != torch.float16 or s[2].dtype != torch.float16 or s[2].shape[1:] != (stacked[0][2].shape[1], x.shape[1]) for s in stacked):
+        return None
+    group = MatrixGroup([s + (None,) for s in stacked])
+    T = x.shape[0]
+    L = _lib.lib()
+    need = L.bs_forward_cat_workspace_bytes(group.arr, group.n, group.N, group.K, T)
+    if need <= 0:
+        return None
+    y = torch.empty((T, sum(group.M)), dtype=torch.float16, device=x.device)
+    with torch.cuda.device(x.device):
+        ws = _lib.workspace(x.device, need)
+        _lib.check(L.bs_forward_cat(group.arr, group.n, group.N, group.K, _lib.ptr(x), T, _lib.ptr(y), _lib.ptr(ws), ws.numel(),
+                                    _lib.stream_ptr(x.device)), "bs_forward_cat")
+    return y
 
 
 def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, out=None):

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from bitstack_amd import _lib
 from bitstack_amd._lib import EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU
 from bitstack_amd.modules.BitStackLinear import BitStackLinear
-from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, attention_prefill_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
+from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, attention_prefill_hip, forward_cat_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
 
 PROJ = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj",
         "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj")
@@ -468,7 +468,9 @@ class SyntheticLlamaDecoder:
             lin = self.lin[L]
             if hn is None:
                 hn = rmsnorm_hip(x, self.norm_w[L, 0], s.rms_eps)
-            q, k, v = (lin[p](hn) for p in PROJ[:3])
+            wide = s.heads * d, s.kv_heads * d
+            qkv = forward_cat_hip([lin[p] for p in PROJ[:3]], hn) if plain and d == 128 else None
+            q, k, v = qkv.split((wide[0], wide[1], wide[1]), 1) if qkv is not None else (lin[p](hn) for p in PROJ[:3])
             kc, vc = self.kcache[L], self.vcache[L]
             if plain:
                 rope_store_hip(q, k, v, self.cos, self.sin, kc, vc, n)
@@ -477,7 +479,8 @@ class SyntheticLlamaDecoder:
             else:
                 ctx = self._attend(q, k, v, kc, vc, n, plain)
             x, hn = add_rmsnorm_hip(x, lin["self_attn.o_proj"](ctx), self.norm_w[L, 1], s.rms_eps)
-            act = silu_mul_hip(lin["mlp.gate_proj"](hn), lin["mlp.up_proj"](hn))
+            both = forward_cat_hip([lin["mlp.gate_proj"], lin["mlp.up_proj"]], hn) if s.intermediate % 8 == 0 else None
+            act = silu_mul_hip(*(both.chunk(2, 1) if both is not None else (lin["mlp.gate_proj"](hn), lin["mlp.up_proj"](hn))))
             down = lin["mlp.down_proj"](act)
             if L + 1 < s.layers:
                 x, hn = add_rmsnorm_hip(x, down, self.norm_w[L + 1, 0], s.rms_eps)

@@ -314,23 +314,32 @@ int bs_rmsnorm_f16(const void *x, const void *weight, void *y, int T, int H, flo
 int bs_add_rmsnorm_f16(const void *x, const void *add, void *sum, const void *weight, void *y, int T, int H, float eps, void *stream);
 
 /*
- * A whole prompt of B sequences, positions 0 .. n - 1: rotate q [B * n, heads * head_dim] in place and k into kcache
+ * y[T, M0 + M1 + ..] = x of 2 to 4 matrices without bias, side by side, for the token counts whose weight is rebuilt
+ * (bs_forward_path 0): one product behind the rebuilds, the results of bs_forward.  bs_forward_cat_workspace_bytes is 0 where
+ * the call is not taken (another path, a bias, more than 96 to 160 MiB of rebuilt weight).
+ */
+int64_t bs_forward_cat_workspace_bytes(const bs_matrix *mats, int n, int N, int K, int T);
+int bs_forward_cat(const bs_matrix *mats, int n, int N, int K, const void *x, int T, void *y, void *workspace,
+                   int64_t workspace_bytes, void *stream);
+
+/*
+ * A whole prompt of B sequences, positions 0 .. n - 1: rotate q [B * n, heads * head_dim] in place (rows of q ldq, of k and v ldkv halves apart) and k into kcache
  * (rotate-half RoPE, cos/sin [n or more, head_dim / 2]), copy v into vcache ([B, kv_heads, max_len, head_dim]; n <= max_len,
  * head_dim even).  Computed in fp32, rounded once, as the decode step does.
  */
-int bs_rope_store_f16(void *q, const void *k, const void *v, const void *cos, const void *sin, void *kcache, void *vcache,
-                      int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream);
+int bs_rope_store_f16(void *q, int ldq, const void *k, const void *v, int ldkv, const void *cos, const void *sin,
+                      void *kcache, void *vcache, int B, int n, int heads, int kv_heads, int head_dim, int max_len, void *stream);
 
 /*
  * Causal attention of a whole prompt: out[B * n, heads * head_dim] = softmax(q k^T / sqrt(head_dim)) v, query j over positions
- * 0 .. j, q [B * n, heads * head_dim] already rotated, k and v from the caches [B, kv_heads, max_len, head_dim] (n <= max_len).
+ * 0 .. j, q [B * n, heads * head_dim] already rotated (rows ldq halves apart, ldq % 8 == 0), k and v from the caches [B, kv_heads, max_len, head_dim] (n <= max_len).
  * head_dim == 128.  Scores, sums and the softmax in fp32, its weights in fp16 for the product with v.
  */
-int bs_attention_prefill_f16(const void *q, const void *kcache, const void *vcache, void *out, int B, int n, int heads, int kv_heads,
+int bs_attention_prefill_f16(const void *q, int ldq, const void *kcache, const void *vcache, void *out, int B, int n, int heads, int kv_heads,
                              int head_dim, int max_len, void *stream);
 
-/* y[count] = fp16(silu(gate) * up); y may be gate or up. */
-int bs_silu_mul_f16(const void *gate, const void *up, void *y, int64_t count, void *stream);
+/* y[T, width] = fp16(silu(gate) * up), rows of gate and up ld apart (T > 1: width and ld % 8 == 0); y may be gate or up if ld == width. */
+int bs_silu_mul_f16(const void *gate, const void *up, void *y, int T, int width, int ld, void *stream);
 
 /*
  * One decode position of grouped-query attention for B sequences that are all

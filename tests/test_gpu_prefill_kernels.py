@@ -2,7 +2,9 @@
 import pytest
 import torch
 
+from bitstack_amd import BitStackLinear
 from bitstack_amd.utils import inference_utils as IU
+from bitstack_amd.utils.synthetic import synthetic_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +79,42 @@ def test_attention_prefill(B, n, heads, kv, max_len):
     assert bool(((got - ref).abs() <= bound).all())
     # and not far from the error of one rounding over the whole
     assert float((got - ref).norm() / ref.norm()) < 6e-4
+
+
+@pytest.mark.parametrize("T,N,shapes", [(129, 256, [(2, 64), (1, 40)]), (200, 1024, [(3, 512), (2, 128), (1, 128)]), (300, 136, [(2, 72), (2, 72)]),
+                                        (257, 4096, [(2, 4096), (3, 1024), (1, 1024)]), (140, 4096, [(1, 8184), (2, 8184)])])
+def test_forward_cat_is_the_matrices_side_by_side(T, N, shapes):
+    mods, x = [], None
+    for j, (I, M) in enumerate(shapes):
+        q, u, vt, xj = synthetic_layer(M, N, I, T, seed=j, device="cuda")
+        x = xj if x is None else x
+        mod = BitStackLinear(0, N, M, 16, False, False, "cuda", fused_level=5)
+        mod.w_bit, mod.qweight, mod.u, mod.vt = I, q, u, vt
+        mods.append(mod)
+    x = x.view(T, N).contiguous()
+    y = IU.forward_cat_hip(mods, x)
+    assert y is not None and y.shape == (T, sum(M for _, M in shapes))
+    want = torch.cat([m(x) for m in mods], 1).double()
+    # the same weights and fp32 sums, in another order at most: a last bit of fp16 here and there
+    assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -10 + want.abs().max() * 2.0 ** -13).all())
+    if N % 128 == 0:                                                     # (other column counts are rebuilt for any token count)
+        assert IU.forward_cat_hip(mods, x[:8].contiguous()) is None
+    mods[0].bias = torch.zeros(shapes[0][1], device="cuda").half()
+    assert IU.forward_cat_hip(mods, x) is None
+
+
+def test_column_slices_as_operands():
+    B, n, heads, kv, d, width = 2, 33, 4, 2, 128, 72
+    g = torch.Generator(device="cuda").manual_seed(5)
+    qkv = torch.randn(B * n, (heads + 2 * kv) * d, generator=g, device="cuda").half()
+    cos, sin = (torch.rand(40, d // 2, generator=g, device="cuda").half() for _ in range(2))
+    caches = [torch.zeros(B, kv, 40, d, device="cuda").half() for _ in range(4)]
+    q, k, v = qkv.split((heads * d, kv * d, kv * d), 1)
+    qc, kc, vc = (t.contiguous() for t in (q, k, v))
+    IU.rope_store_hip(qc, kc, vc, cos, sin, caches[0], caches[1], n)
+    IU.rope_store_hip(q, k, v, cos, sin, caches[2], caches[3], n)
+    assert torch.equal(q, qc) and torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+    assert torch.equal(IU.attention_prefill_hip(q, caches[2], caches[3], n), IU.attention_prefill_hip(qc, caches[0], caches[1], n))
+    both = torch.randn(5, 2 * width, generator=g, device="cuda").half()
+    a, b = both.chunk(2, 1)
+    assert torch.equal(IU.silu_mul_hip(a, b), IU.silu_mul_hip(a.contiguous(), b.contiguous()))

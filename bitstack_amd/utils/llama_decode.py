@@ -172,7 +172,7 @@ class SyntheticLlamaDecoder:
         self.span = torch.arange(max_len, device=self.dev)
         self.logits = None
         self._groups = None
-        self._steps = None                                                 # (addresses it was made for, launch list)
+        self._steps = None                                                 # (what it was made for, (launch list, last norm in it), its tensors)
 
     @classmethod
     def from_checkpoint(cls, path, max_len, device, compression_config=None, niter=None, max_memory_MB=None, batch=1):
@@ -377,47 +377,60 @@ class SyntheticLlamaDecoder:
         self._xb = torch.empty(B, s.hidden, **f16)
 
     def _launches(self):
-        """The launches of step_fused() between the embedding and the last norm as one native list (host.cpp), laid
-        out once: their arguments only change when the groups are rebuilt or a cache or table is replaced."""
+        """(the launches of step_fused() between the embedding and the last norm as one native list (host.cpp), whether that norm
+        is in it).  Laid out once and again whenever one of the tensors whose addresses it holds has become another one, by address,
+        shape, strides or type; it keeps those tensors alive."""
         if self._groups is None:
             self._build_groups()
-        held = (self.kcache, self.vcache, self.cos, self.sin, self.pos)
-        key = tuple(t.data_ptr() for t in held)
+        held = (self.kcache, self.vcache, self.cos, self.sin, self.pos, self.final_norm)
+        eps = self.s.rms_eps
+        key = (eps, *((t.data_ptr(), t.shape, t.stride(), t.dtype, t.device) for t in held))
         if self._steps is not None and self._steps[0] == key:
             return self._steps[1]
-        s, B = self.s, self.batch
-        d = s.head_dim
-        for t, shape, dtype in ((self.kcache, (s.layers, B, s.kv_heads, self.max_len, d), torch.float16),
-                                (self.vcache, (s.layers, B, s.kv_heads, self.max_len, d), torch.float16),
-                                (self.cos, (self.max_len, d // 2), torch.float16), (self.sin, (self.max_len, d // 2), torch.float16),
-                                (self.pos, (1,), torch.int64)):
-            if tuple(t.shape) != shape or t.dtype != dtype or not t.is_contiguous() or not t.is_cuda:
-                raise ValueError(f"the decode step needs a contiguous {dtype} tensor {shape} on the GPU, got {t.dtype} {tuple(t.shape)}")
+        s, B, dev = self.s, self.batch, self._xa.device
+        d, max_len = s.head_dim, self.kcache.shape[-2]
+
+        def need(t, ok, what):
+            if not ok or t.device != dev:
+                raise ValueError(f"the decode step needs {what} on {dev}, got {t.dtype} {tuple(t.shape)} {t.stride()} on {t.device}")
+
+        for t in (self.kcache, self.vcache):
+            need(t, t.dim() == 5 and t.shape[0] >= s.layers and tuple(t.shape[1:]) == (B, s.kv_heads, max_len, d)
+                 and t.dtype == torch.float16 and t[0].is_contiguous(), f"fp16 caches [layers, {B}, {s.kv_heads}, {max_len}, {d}], a layer contiguous,")
+        for t in (self.cos, self.sin):
+            need(t, tuple(t.shape) == (max_len, d // 2) and t.dtype == torch.float16 and t.is_contiguous(), f"a contiguous fp16 table {(max_len, d // 2)}")
+        need(self.pos, self.pos.numel() == 1 and self.pos.dtype == torch.int64, "one int64 position")
         xa, xb, qkv, ctx, act = (t.data_ptr() for t in (self._xa, self._xb, self._qkv, self._ctx, self._act))
-        kcache, vcache, cos, sin, pos = key
-        layer = 2 * B * s.kv_heads * self.max_len * d                      # bytes of a layer's cache
+        kcache, vcache, cos, sin, pos, norm = (t.data_ptr() for t in held)
+        klayer, vlayer = 2 * self.kcache.stride(0), 2 * self.vcache.stride(0)     # bytes from a layer's cache to the next
 
         def group(g, x, y, epilogue, eps=None, residual=0):
             return ("group", ctypes.addressof(g.arr), g.n, g.N, g.K, x, B, eps, epilogue, residual, y)
 
         items = []
         for L, grp in enumerate(self._groups):
-            items.append(group(grp["qkv"], xa, qkv, EPI_NONE, eps=s.rms_eps))
-            items.append(("attention", qkv, kcache + L * layer, vcache + L * layer, cos, sin, pos, ctx, B, s.heads, s.kv_heads, d, self.max_len))
+            items.append(group(grp["qkv"], xa, qkv, EPI_NONE, eps=eps))
+            items.append(("attention", qkv, kcache + L * klayer, vcache + L * vlayer, cos, sin, pos, ctx, B, s.heads, s.kv_heads, d, max_len))
             items.append(group(grp["o"], ctx, xb, EPI_RESIDUAL, residual=xa))
-            items.append(group(grp["gate_up"], xb, act, EPI_SWIGLU, eps=s.rms_eps))
+            items.append(group(grp["gate_up"], xb, act, EPI_SWIGLU, eps=eps))
             items.append(group(grp["down"], act, xa, EPI_RESIDUAL, residual=xb))
-        items.append(("norm", xa, self.final_norm.data_ptr(), self._hn.data_ptr(), B, s.hidden, s.rms_eps))
-        self._steps = (key, _lib.host().make_steps(items))
+        # a norm weight of another type or layout is converted or refused by rmsnorm_hip() in each step
+        w = self.final_norm
+        inside = tuple(w.shape) == (s.hidden,) and w.dtype == torch.float16 and w.is_contiguous() and w.device == dev
+        if inside:
+            items.append(("norm", xa, norm, self._hn.data_ptr(), B, s.hidden, eps))
+        self._steps = (key, (_lib.host().make_steps(items), inside), held)
         return self._steps[1]
 
     @torch.no_grad()
     def step_fused(self):
         """Same step on the library's grouped forwards and decode-step kernels: q/k/v with the RMSNorm in front, attention,
         o + residual, gate/up with the RMSNorm in front and the SiLU product, down + residual per layer."""
-        launches = self._launches()
+        launches, normed = self._launches()
         torch.index_select(self.embed, 0, self.token, out=self._xa)
         _lib.host().run_steps(launches, self._xa.device.index)
+        if not normed:
+            rmsnorm_hip(self._xa, self.final_norm, self.s.rms_eps, out=self._hn)
         self.logits = F.linear(self._hn, self.lm_head)
         argmax_hip(self.logits, out=self.token)
         self.pos.add_(1)

@@ -261,12 +261,19 @@ def silu_mul_hip(gate, up):
     return y
 
 
+def plainly_called(module):
+    """Whether a call of `module` is BitStackLinear's own forward and nothing else: no hook, of the module or of all modules, and no
+    forward of the instance.  Only then does nobody else see its input or hold its output."""
+    from bitstack_amd.modules.BitStackLinear import BitStackLinear
+    return (type(module) is BitStackLinear and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks and not torch.nn.modules.module._has_any_global_hook())
+
+
 def forward_cat_hip(modules, x):
     """[T, M0 + M1 + ..]: what the modules (BitStackLinear, level 5) give for x [T, N], side by side from one product, or None
     where that is not how they are computed (few tokens, a bias, another level, blocks not stacked)."""
-    from bitstack_amd.modules.BitStackLinear import BitStackLinear
     for m in modules:
-        if type(m) is not BitStackLinear or m._forward_hooks or m._forward_pre_hooks:     # (a call of the module would do more)
+        if not plainly_called(m):                # (a call of the module would do more)
             return None
         if m.fused_level != 5 or m.no_avd or m.bias is not None or getattr(m, "u", None) is None:
             return None

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from bitstack_amd import _lib
 from bitstack_amd._lib import EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU
 from bitstack_amd.modules.BitStackLinear import BitStackLinear
-from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, attention_prefill_hip, forward_cat_hip, rmsnorm_hip, rope_store_hip, silu_mul_hip
+from bitstack_amd.utils.inference_utils import MatrixGroup, add_rmsnorm_hip, argmax_hip, attention_prefill_hip, forward_cat_hip, plainly_called, rmsnorm_hip, rope_store_hip, silu_mul_hip
 
 PROJ = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj",
         "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj")
@@ -450,6 +450,26 @@ class SyntheticLlamaDecoder:
         return torch.cat([F.scaled_dot_product_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], is_causal=True, enable_gqa=True)
                           .transpose(1, 2).reshape(n, s.hidden) for b in range(B)])
 
+    @staticmethod
+    def _output(module, x):
+        """What the module gives for x, as a tensor that may be written over: a copy where somebody else may hold it."""
+        y = module(x)
+        return y if plainly_called(module) else y.clone(memory_format=torch.contiguous_format)
+
+    def _sum_norm(self, x, add, weight):
+        """(x + add, its RMSNorm); the sum takes the place of `add`."""
+        if add.dtype == torch.float16 and add.shape == x.shape:
+            return add_rmsnorm_hip(x, add, weight, self.s.rms_eps)
+        x = x + add
+        return x, rmsnorm_hip(x, weight, self.s.rms_eps)
+
+    @staticmethod
+    def _silu_mul(gate, up):
+        """silu(gate) * up, in gate's place."""
+        if gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape:
+            return silu_mul_hip(gate, up)
+        return F.silu(gate).mul_(up)
+
     @torch.no_grad()
     def prefill(self, prompt: torch.Tensor, all_logits=False, first_layer=0, hidden=None, keep=None):
         """The whole prompt [batch, len] in one pass: every linear sees batch * len tokens (the
@@ -481,27 +501,28 @@ class SyntheticLlamaDecoder:
             lin = self.lin[L]
             if hn is None:
                 hn = rmsnorm_hip(x, self.norm_w[L, 0], s.rms_eps)
-            wide = s.heads * d, s.kv_heads * d
+            wide = s.heads * d, s.kv_heads * d, s.kv_heads * d
             qkv = forward_cat_hip([lin[p] for p in PROJ[:3]], hn) if plain and d == 128 else None
-            q, k, v = qkv.split((wide[0], wide[1], wide[1]), 1) if qkv is not None else (lin[p](hn) for p in PROJ[:3])
+            q, k, v = qkv.split(wide, 1) if qkv is not None else (self._output(lin[p], hn) for p in PROJ[:3])
+            stored = plain and all(t.dtype == torch.float16 and t.shape == (B * n, w) for t, w in zip((q, k, v), wide))
             kc, vc = self.kcache[L], self.vcache[L]
-            if plain:
+            if stored:
                 rope_store_hip(q, k, v, self.cos, self.sin, kc, vc, n)
-            if plain and d == 128:
+            if stored and d == 128:
                 ctx = attention_prefill_hip(q, kc, vc, n)
             else:
-                ctx = self._attend(q, k, v, kc, vc, n, plain)
-            x, hn = add_rmsnorm_hip(x, lin["self_attn.o_proj"](ctx), self.norm_w[L, 1], s.rms_eps)
+                ctx = self._attend(q, k, v, kc, vc, n, stored)
+            x, hn = self._sum_norm(x, self._output(lin["self_attn.o_proj"], ctx), self.norm_w[L, 1])
             both = forward_cat_hip([lin["mlp.gate_proj"], lin["mlp.up_proj"]], hn) if s.intermediate % 8 == 0 else None
-            act = silu_mul_hip(*(both.chunk(2, 1) if both is not None else (lin["mlp.gate_proj"](hn), lin["mlp.up_proj"](hn))))
-            down = lin["mlp.down_proj"](act)
+            act = self._silu_mul(*(both.chunk(2, 1) if both is not None else (self._output(lin[p], hn) for p in PROJ[4:6])))
+            down = self._output(lin["mlp.down_proj"], act)
             if L + 1 < s.layers:
-                x, hn = add_rmsnorm_hip(x, down, self.norm_w[L + 1, 0], s.rms_eps)
+                x, hn = self._sum_norm(x, down, self.norm_w[L + 1, 0])
             elif all_logits:
-                x, hn = add_rmsnorm_hip(x, down, self.final_norm, s.rms_eps)
+                x, hn = self._sum_norm(x, down, self.final_norm)
             else:                                                         # the last position of each sequence
                 x, down = (t.view(B, n, s.hidden)[:, -1].contiguous() for t in (x, down))
-                x, hn = add_rmsnorm_hip(x, down, self.final_norm, s.rms_eps)
+                x, hn = self._sum_norm(x, down, self.final_norm)
         if hn is None:                                                    # no layer ran: first_layer is the layer count
             x = x if all_logits else x.view(B, n, s.hidden)[:, -1].contiguous()
             hn = rmsnorm_hip(x, self.final_norm, s.rms_eps)

@@ -437,18 +437,23 @@ class SyntheticLlamaDecoder:
 
     def _attend(self, q, k, v, kc, vc, n, stored):
         """prefill()'s attention on torch operations, for heads of other sizes or caches of another layout or type: `stored`
-        means that q is rotated and k, v are in the cache."""
+        means that q is rotated and k, v are in the cache.  Otherwise k and v are attended to as they are computed, whatever the
+        cache keeps of them."""
         s, B, d = self.s, self.batch, self.s.head_dim
         q = q.view(B, n, s.heads, d).transpose(1, 2)
-        if not stored:
+        if stored:
+            k, v = kc[:, :, :n], vc[:, :, :n]
+        else:
             cos, sin = self.cos[:n].view(1, 1, n, d // 2), self.sin[:n].view(1, 1, n, d // 2)
-            q = self._rope(q, cos, sin)
-            kc[:, :, :n].copy_(self._rope(k.view(B, n, s.kv_heads, d).transpose(1, 2), cos, sin))
-            vc[:, :, :n].copy_(v.view(B, n, s.kv_heads, d).transpose(1, 2))
-        k, v = kc[:, :, :n].to(q.dtype), vc[:, :, :n].to(q.dtype)
-        # one sequence at a time bounds the scratch
-        return torch.cat([F.scaled_dot_product_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], is_causal=True, enable_gqa=True)
-                          .transpose(1, 2).reshape(n, s.hidden) for b in range(B)])
+            k, v = (t.view(B, n, s.kv_heads, d).transpose(1, 2) for t in (k, v))
+            q, k = self._rope(q, cos, sin), self._rope(k, cos, sin)
+            kc[:, :, :n].copy_(k)
+            vc[:, :, :n].copy_(v)
+        ctx = torch.empty(B, n, s.hidden, dtype=torch.float16, device=self.dev)
+        for b in range(B):                                                # one sequence at a time bounds the scratch
+            o = F.scaled_dot_product_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], is_causal=True, enable_gqa=True)
+            ctx[b].copy_(o[0].transpose(0, 1).reshape(n, s.hidden))
+        return ctx.view(B * n, s.hidden)
 
     @staticmethod
     def _output(module, x):

@@ -135,10 +135,7 @@ __device__ inline void produce_finish(half_t *zt, int pg, int p, int r, half8_t 
     });
 }
 
-// WHOLE: N % 512 == 0.  The test of a partial last chunk costs the 3- and 4-token forms 1 % (14336 x 4096, 4 blocks, 36.7 against
-// 37.1 us), so shapes without one run a kernel without it.  Such shapes ran the rebuild and a dense product before: 11008
-// columns by 4096 rows, 8 blocks, one token: 60.9 us, now 18.1.
-template <int T, int WAVES, int R, bool WHOLE>
+template <int T, int WAVES, int R>
 __global__ __launch_bounds__(64 * WAVES, (T == 1 ? (WAVES == 16 ? 1 : WAVES == 4 && R == 4 ? 3 : 4) : (T == 2 ? (WAVES == 8 && R == 2 ? 4 : 2) : 1))) void gemv_kernel(
     const GemvGroup grp, const half_t *__restrict__ x, int N, int K, int n_chunks) {
     constexpr int RW = WAVES * R * 16;          // rows per workgroup
@@ -216,19 +213,14 @@ __global__ __launch_bounds__(64 * WAVES, (T == 1 ? (WAVES == 16 ? 1 : WAVES == 4
     };
     clear_acc();
 
-    // N is a multiple of 128, not always of 512: of a partial last chunk the lane groups g with 128 g beyond it are dead.
-    // Their vt counts as zero, so their Z is (whatever sign bytes they hold count for nothing), and their requests of vt and x
-    // repeat group 0's addresses: columns that are multiplied anyway, so a non-finite x there spoils no output it does not own.
     half8_t pv[COMBOS][2];        // vt pieces in flight for the next unit
     half8_t px[COMBOS][T][2];     // x pieces in flight for the next unit
-    bool p_live[COMBOS];          // their columns lie below N (wave-uniform)
     auto produce_issue = [&](int c) {
         if (WAVES > 8 && wave >= 8) return;
 #pragma unroll
         for (int k = 0; k < COMBOS; k++) {
             const int combo = wave + k * WAVES, pg = combo & 3, jb = combo >> 2;
-            p_live[k] = WHOLE || c * CH + 128 * pg < N;
-            const int col = c * CH + (p_live[k] ? 128 * pg : 0) + 8 * jb;            // wave-uniform
+            const int col = c * CH + 128 * pg + 8 * jb;            // wave-uniform
             const uint8_t *vs = reinterpret_cast<const uint8_t *>(vbase + col) + voff;
             pv[k][0] = *reinterpret_cast<const half8_t *>(vs);
             pv[k][1] = *reinterpret_cast<const half8_t *>(vs + 32);
@@ -247,7 +239,7 @@ __global__ __launch_bounds__(64 * WAVES, (T == 1 ? (WAVES == 16 ? 1 : WAVES == 4
         for (int k = 0; k < COMBOS; k++) {
             const int combo = wave + k * WAVES, pg = combo & 3, jb = combo >> 2;
             half8_t v0 = pv[k][0], v1 = pv[k][1];
-            if (!r_live || !p_live[k]) { v0 = (half8_t){0, 0, 0, 0, 0, 0, 0, 0}; v1 = v0; }
+            if (!r_live) { v0 = (half8_t){0, 0, 0, 0, 0, 0, 0, 0}; v1 = v0; }
 #pragma unroll
             for (int t = 0; t < T; t++) {
                 half_t *zt = zbuf + z_index(t, 0, 0, 0);
@@ -302,14 +294,8 @@ __global__ __launch_bounds__(64 * WAVES, (T == 1 ? (WAVES == 16 ? 1 : WAVES == 4
     };
 
     auto load_signs = [&](uint4_t (&w)[R], int c) {
-        if constexpr (WHOLE) {
 #pragma unroll
-            for (int jr = 0; jr < R; jr++) w[jr] = *reinterpret_cast<const uint4_t *>(qbase + c * (CH >> 3) + qoff[jr]);
-        } else {      // dead groups read the next row's bytes, behind the block's last row zeros (the range check of the descriptor)
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(qbase), 0, (int)(M * row_bytes), 0x00020000);
-#pragma unroll
-            for (int jr = 0; jr < R; jr++) w[jr] = __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, qoff[jr], c * (CH >> 3), 0));
-        }
+        for (int jr = 0; jr < R; jr++) w[jr] = *reinterpret_cast<const uint4_t *>(qbase + c * (CH >> 3) + qoff[jr]);
     };
 
     // D[r, m]: the lane holds ranks 4g..4g+3 of row (tile jr, lm).  Subtract the
@@ -598,7 +584,7 @@ int mx_rows_per_tile(const int *I, const int *M, int n, int N, int K, int T) {
 Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
     Plan p;
     p.n = n;
-    p.n_chunks = (int)bs_cdiv(N, CH);
+    p.n_chunks = N / CH;
     p.mx = 0;
     const int mx_r = mx_rows_per_tile(I, M, n, N, K, T);
     if (mx_r > 0) {
@@ -665,9 +651,8 @@ Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
     // One token, long stacks: one workgroup of 16 waves per CU.  Two 8-wave workgroups on a CU do
     // not share it evenly (the older one is served first and finishes a third earlier, the
     // younger one then runs on a half-empty CU); sixteen waves that meet at one barrier do.
-    // (128 registers a lane leave no room for the test of a partial last chunk.)
     const int *choice = cand[pick];
-    if (T == 1 && N % CH == 0) {
+    if (T == 1) {
         bool tall = true;
         int64_t units = 0;
         for (int j = 0; j < n; j++) {
@@ -749,19 +734,15 @@ struct GroupArgs {          // host-side view of one call
     int I[GEMV_MAX_GROUP], M[GEMV_MAX_GROUP];
 };
 
-template <int T, int WAVES, int R, bool WHOLE>
-int launch_whole(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K, hipStream_t s) {
-    const size_t lds = (size_t)2 * T * 16384 + (size_t)2 * WAVES * T * 64;
-    static bs_lds_grant granted[BS_MAX_DEVICES];      // per instantiation
-    const int st = bs_allow_lds((const void *)gemv_kernel<T, WAVES, R, WHOLE>, lds, granted);
-    if (st != BS_OK) return st;
-    gemv_kernel<T, WAVES, R, WHOLE><<<p.grid, 64 * WAVES, lds, s>>>(grp, x, N, K, p.n_chunks);
-    BS_LAUNCH_CHECK();
-    return BS_OK;
-}
 template <int T, int WAVES, int R>
 int launch_one(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K, hipStream_t s) {
-    return N % CH == 0 ? launch_whole<T, WAVES, R, true>(p, grp, x, N, K, s) : launch_whole<T, WAVES, R, false>(p, grp, x, N, K, s);
+    const size_t lds = (size_t)2 * T * 16384 + (size_t)2 * WAVES * T * 64;
+    static bs_lds_grant granted[BS_MAX_DEVICES];      // per instantiation
+    const int st = bs_allow_lds((const void *)gemv_kernel<T, WAVES, R>, lds, granted);
+    if (st != BS_OK) return st;
+    gemv_kernel<T, WAVES, R><<<p.grid, 64 * WAVES, lds, s>>>(grp, x, N, K, p.n_chunks);
+    BS_LAUNCH_CHECK();
+    return BS_OK;
 }
 
 // Only the (WAVES, R) pairs make_plan can choose for T tokens exist; any other pair is refused
@@ -771,7 +752,7 @@ template <int T>
 int launch_T(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K, hipStream_t s) {
     const int w = p.waves, r = p.R;
     if constexpr (T == 1) {
-        if (w == 16 && r == 4 && N % CH == 0) return launch_whole<1, 16, 4, true>(p, grp, x, N, K, s);
+        if (w == 16 && r == 4) return launch_one<1, 16, 4>(p, grp, x, N, K, s);
         if (w == 8 && r == 4) return launch_one<1, 8, 4>(p, grp, x, N, K, s);
     } else if constexpr (T == 2) {
         if (w == 8 && r == 2) return launch_one<2, 8, 2>(p, grp, x, N, K, s);
@@ -788,9 +769,8 @@ int launch_T(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K,
 }
 
 bool gemv_shape_ok(int I, int M, int N, int T) {
-    // Per-block byte offsets are kept in 32 bits inside the kernel.  A partial last chunk is worked through in full: taken
-    // where that adds at most a third (11008 columns: 2 %; 640 columns, a chunk and a quarter, are rebuilt).
-    return I >= 1 && I <= RED_MAXBLOCKS && T >= 1 && T <= 8 && N % 128 == 0 && M >= 1 && 3 * ((CH - N % CH) % CH) <= N &&
+    // per-block byte offsets are kept in 32 bits inside the kernel
+    return I >= 1 && I <= RED_MAXBLOCKS && T >= 1 && T <= 8 && N % CH == 0 && M >= 1 &&
            (int64_t)M * N < ((int64_t)1 << 31);
 }
 
@@ -817,7 +797,13 @@ int group_path(const int *I, const int *M, int n, int N, int K, int T) {
     if (n < 1 || n > GEMV_MAX_GROUP) return -1;
     if (T >= STRIP_MIN_T && T <= STRIP_MAX_T && strip_group_ok(I, M, n, N, K, T)) return 1;
     if (gemv_group_ok(I, M, n, N, T)) return 0;
-    return -1;
+    // One to four tokens on column counts that are multiples of 128 but not of 512: the strip kernel rounds the weight to fp16 once
+    // and multiplies with fp32 sums, as the rebuild and the dense product do that such shapes took before it, and no less exactly
+    // (error against float64 within 0.05 % of theirs: 11 shapes, three decomposed weights, 1, 2 and 4 tokens).  The factor-through kernels
+    // would round vt * x: 7 % further from float64 with 2 blocks of 11008 columns (2.94e-4 against 2.75e-4), 11 % on the block-scaled
+    // one.  us rebuild / strip, 4096 x 11008 with one token: 1 block 52 / 14, 4 blocks 72 / 28, 8 blocks 91 / 47; 2048 x 5504, 3
+    // blocks 32 / 12; 8192 x 3200, 4 blocks 40 / 21 (the block-scaled kernel, with that loss: 18 and 24 at 4 and 8 blocks of 4096 x 11008).
+    return N % CH != 0 && T < STRIP_MIN_T && strip_group_ok(I, M, n, N, K, T) ? 1 : -1;
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group

@@ -62,10 +62,10 @@ constexpr int MX_OPERAND = 64 * 16 + 64 * 8;        // bytes of one (half, q, te
 constexpr int MX_SCALES = 8 * 3 * MX_OPERAND;       // the scale words of a Z buffer follow its 24 operands
 constexpr int MX_ZBUF = MX_SCALES + 8 * 64 * 4;     // bytes per Z buffer
 
-// raw buffer descriptor from a pointer: no stride, `bytes` to the end of what may be read (-1: no limit short of 4 GiB, where
-// every offset used is checked by construction: rows clamped to M, columns to the unit)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t mx_rsrc(const void *p, int bytes = -1) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
+// raw buffer descriptor from a pointer: no stride, no range limit short of 4 GiB (every offset used with it is checked
+// by construction: rows clamped to M, columns to the unit)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mx_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, -1, 0x00020000);
 }
 
 __device__ __forceinline__ uint32_t mx_and_or(uint32_t w, uint32_t mask, uint32_t base) { return (w & mask) | base; }
@@ -209,10 +209,8 @@ __global__ __launch_bounds__(64 * MX_WAVES, 1) void gemv_mx_kernel(
     const int ph = wave >> 2, pj = wave & 3;
     uint32_t *stage = reinterpret_cast<uint32_t *>(lds + 2 * MX_ZBUF + wave * MX_STAGE);
 
-    // A unit whose second half lies beyond N reads the first half's addresses again there; x counts as zero for those
-    // columns, so they add nothing.  N is a multiple of 128: a half may end after one, two or three lane groups; x
-    // counts as zero in the columns beyond (a lane's eight columns are all below N or all beyond), and the sign words there
-    // - the next row's, or zeros behind the end of the block - count for nothing.
+    // a unit whose second half lies beyond N (N a multiple of 512 only) reads the first half's
+    // addresses again there; x counts as zero for those columns, so they add nothing
     auto half_cols = [&](int c, int h) { return (T == 1 && c * UC + 512 * h < N) ? 512 * h : 0; };
 
     // ---- the unit being loaded: (block li, row tile, 1024-column chunk lc) ------------------------
@@ -225,8 +223,7 @@ __global__ __launch_bounds__(64 * MX_WAVES, 1) void gemv_mx_kernel(
     __amdgpu_buffer_rsrc_t lv;  // vt of the block: rank 0, from the first column of half ph of the unit
     __amdgpu_buffer_rsrc_t lx;  // x (of token ph when T = 2) from the same column
     int l_h1;                   // byte offset of the unit's second half of a row (0 when it lies beyond N)
-    bool l_xlive;               // the columns this lane produces lie within N (per lane)
-    int l_col;                  // their byte offset in the half (the half's first columns where they do not)
+    bool l_xlive;               // the producer half of this wave lies within N
     auto set_unit = [&](int rowid, int c, bool new_row) {
         const int i = rowid / row_tiles;
         if (new_row) {
@@ -237,12 +234,11 @@ __global__ __launch_bounds__(64 * MX_WAVES, 1) void gemv_mx_kernel(
                 qoff[jr] = row * (uint32_t)row_bytes + 16u * g;
             }
         }
-        lq = mx_rsrc(packed + (int64_t)i * M * row_bytes + c * (UC >> 3), (int)(M * (uint32_t)row_bytes - (uint32_t)(c * (UC >> 3))));
+        lq = mx_rsrc(packed + (int64_t)i * M * row_bytes + c * (UC >> 3));
         l_h1 = half_cols(c, 1) >> 3;
         lv = mx_rsrc(vt + (int64_t)i * K * N + c * UC + half_cols(c, ph));
         lx = mx_rsrc(x + (T == 2 ? (int64_t)ph * N : 0) + c * UC + half_cols(c, ph));
-        l_xlive = (T == 2 || c * UC + 512 * ph < N) && c * UC + half_cols(c, ph) + 8 * lane < N;
-        l_col = l_xlive ? 16 * lane : 0;
+        l_xlive = T == 2 || c * UC + 512 * ph < N;
     };
 
     float4_t acc[R][T];
@@ -261,11 +257,11 @@ __global__ __launch_bounds__(64 * MX_WAVES, 1) void gemv_mx_kernel(
         // (ranks beyond K repeat rank K - 1 and are zeroed when the operands are formed: no branch around a load)
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            pv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(lv, l_col, min(4 * pj + k, K - 1) * N * 2, 0));
-        px = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(lx, l_col, 0, 0));
+            pv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(lv, 16 * lane, min(4 * pj + k, K - 1) * N * 2, 0));
+        px = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(lx, 16 * lane, 0, 0));
     };
     auto produce_write = [&](int buf) {
-        if (!l_xlive) px = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};        // (of vt it holds the half's first columns: an infinity there is in every output anyway)
+        if (!l_xlive) px = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
         mx_produce_finish(zl + buf * MX_ZBUF, stage, pv, px, ph, pj, lane);
     };
 
@@ -491,9 +487,9 @@ int launch_mx(int grid, const GemvGroup &grp, const half_t *x, int N, int K, int
 
 }  // namespace
 
-// Shapes the block-scaled kernel runs: one or two tokens.
+// Shapes the block-scaled kernel runs: whole 512-column halves, one or two tokens.
 bool bs_gemv_mx_takes(int N, int K, int R, int T) {
-    if (N % 128 != 0 || K < 1 || K > 16 || T < 1 || T > 2) return false;
+    if (N % 512 != 0 || K < 1 || K > 16 || T < 1 || T > 2) return false;
     return R == 1 || R == 2 || R == 4;
 }
 

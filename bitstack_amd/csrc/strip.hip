@@ -614,7 +614,7 @@ static int wide_choice(int I, int M, int N, int K, int T) {
     return walked ? 1 : panel ? 2 : 0;
 }
 
-// Which of this family's kernels a forward of these dimensions runs: 0 none, 1 strip_forward_kernel (5..48 tokens),
+// Which of this family's kernels a forward of these dimensions runs: 0 none, 1 strip_forward_kernel (up to 48 tokens),
 // 2 strip_wide_kernel (the walked strips), 3 the panel kernel.
 int bs_strip_kernel_choice(int I, int M, int N, int K, int T) {
     if (bs_strip_partials(I, M, N, K, T) == 0) return 0;

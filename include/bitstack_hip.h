@@ -95,11 +95,11 @@ int64_t bs_workspace_bytes(int I, int M, int N, int K, int T);
  * (bitstack/utils/inference_utils.py:171-284).
  *
  * T <= 4 runs the packed-sign GEMV (signs contracted on MFMA against
- * vt_i o x, scaled by u_i, all blocks in one pass; N % 128 == 0 and at most N / 3
- * columns missing from the last chunk of 512); 5 <= T <= 48
+ * vt_i o x, scaled by u_i, all blocks in one pass; N % 512 == 0); 5 <= T <= 48
  * the strip kernel (16 x 16 patches of the weight rebuilt in registers and
  * multiplied by x at once, the weight never stored; N % 128 == 0; when it does
- * not take the shape, T <= 8 is two GEMV passes); 49 <= T <= 96 the same
+ * not take the shape, T <= 8 is two GEMV passes), which also takes T <= 4 where
+ * N is a multiple of 128 but not of 512; 49 <= T <= 96 the same
  * patches with the strips walked by workgroups of 128 rows, where that beats
  * the next paths (N % 128 == 0, vt of all blocks of a strip within 40 KB of
  * LDS, workgroups that fill the chip or at most 6 blocks); otherwise, up to
@@ -150,7 +150,7 @@ int bs_forward_static(const uint8_t *packed, const void *u, const void *vt, cons
  * many partial sums per row and block bs_forward would use for these
  * dimensions; *waves == 0 means the decode kernel does not run them (the
  * strip kernel or the dense path does: more than 4 tokens with N % 128 == 0,
- * more than 8 tokens, an N as bs_forward does not give it).  No counterpart in the reference
+ * more than 8 tokens, N not a multiple of 512).  No counterpart in the reference
  * (Triton picks its configuration by autotuning,
  * bitstack/utils/inference_utils.py:8-39).
  */
@@ -178,7 +178,7 @@ int bs_decode_kernel(int I, int M, int N, int K, int T);
 #define BS_PATH_REBUILD    0   /* weight rebuilt into the workspace, then the dense product */
 #define BS_PATH_DECODE_F16 1   /* gemv_kernel: packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass */
 #define BS_PATH_DECODE_MX  2   /* gemv_mx_kernel: the same on the block-scaled fp4 x fp6 MFMA, 1..2 tokens */
-#define BS_PATH_STRIP      3   /* strip_forward_kernel: 5..48 tokens, patches rebuilt in registers */
+#define BS_PATH_STRIP      3   /* strip_forward_kernel: up to 48 tokens, patches rebuilt in registers */
 #define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups */
 #define BS_PATH_PANEL      5   /* panel_forward_kernel: up to 128 tokens, W tiles decoded into LDS */
 int bs_forward_path(int I, int M, int N, int K, int T);
@@ -187,7 +187,7 @@ int bs_forward_path(int I, int M, int N, int K, int T);
  * Test and benchmark hook: 0 = choose the decode kernel of one- and two-token
  * passes by shape (the default), BS_DECODE_F16 = always the fp16 kernel,
  * BS_DECODE_MX = the block-scaled kernel wherever it takes the shape
- * (one or two tokens).  The setting belongs to the CALLING
+ * (N % 512 == 0, at most two tokens).  The setting belongs to the CALLING
  * THREAD (every thread starts at 0): bs_workspace_bytes, bs_decode_plan and
  * bs_forward called from one thread always agree, whatever other threads set.
  * No counterpart in the reference.
@@ -252,7 +252,7 @@ int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_features, in
 
 /*
  * ---- decode step: several matrices per launch, fused epilogues -----------
- * One decode forward (T <= 48 tokens; more than 8 need N % 128 == 0) of up to 4 compressed matrices that read
+ * One decode forward (T <= 48 tokens; N % 128 == 0) of up to 4 compressed matrices that read
  * the same x, in one kernel pair: what q_proj/k_proj/v_proj (or gate_proj/
  * up_proj) of a decoder layer do with three (two) BitStackLinear.forward calls,
  * bitstack/modules/BitStackLinear.py:88-157, each as in bs_forward.  All share
@@ -264,8 +264,8 @@ int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_features, in
  *   BS_EPI_SWIGLU    n == 2, M_0 == M_1: y[T, M_0] = silu(first) * second
  *                    computed from the fp16-rounded results, as
  *                    `act_fn(gate_proj(h)) * up_proj(h)` in the MLP
- * Only shapes the decode kernel takes (every matrix: N as bs_forward gives it at T <= 4,
- * M * N < 2^31, alignment as bs_forward); anything else returns BS_ERR_SHAPE
+ * Only shapes the decode or the strip kernel takes (every matrix as bs_forward
+ * gives it at this T, M * N < 2^31 on the decode kernel, alignment as bs_forward); anything else returns BS_ERR_SHAPE
  * and the caller issues bs_forward per matrix.  Workspace as bs_forward, size
  * from bs_forward_group_workspace_bytes (negative = status).
  */

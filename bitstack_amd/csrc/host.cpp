@@ -14,9 +14,11 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <map>
+#include <memory>
 #include <mutex>
 #include <utility>
 #include <vector>
@@ -116,10 +118,12 @@ struct DeviceScope {
 };
 
 // ---- entry points --------------------------------------------------------------------------------
+// Each one's C++ exceptions become the Python errors torch itself raises for them (HANDLE_TH_ERRORS): an allocation that fails is
+// torch.OutOfMemoryError, for callers that back off on it.
 // forward(qweight, u, vt, blocks, x, bias or None) -> y, or None where the Python path has to take the call
 PyObject *host_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 6) return PyErr_Format(PyExc_TypeError, "forward takes 6 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *x = tensor_arg(a[4]);
         const at::Tensor *bias = a[5] == Py_None ? nullptr : tensor_arg(a[5]);
         int64_t blocks;
@@ -142,15 +146,13 @@ PyObject *host_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                   (int)m.M, (int)m.N, (int)m.K, T, ws.mutable_data_ptr(), ws.numel(), stream);
         if (st != BS_OK) return raise_status(st, "bs_forward");
         return THPVariable_Wrap(y);
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // rebuild(qweight, u, vt, blocks) -> w [M, N], or None
 PyObject *host_rebuild(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 4) return PyErr_Format(PyExc_TypeError, "rebuild takes 4 arguments");
-    try {
+    HANDLE_TH_ERRORS
         int64_t blocks;
         if (!int_arg(a[3], blocks)) return nullptr;
         const at::Tensor *u = tensor_arg(a[1]);
@@ -164,15 +166,13 @@ PyObject *host_rebuild(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                         c10::hip::getCurrentHIPStream(dev.index()).stream());
         if (st != BS_OK) return raise_status(st, "bs_reconstruct_w");
         return THPVariable_Wrap(w);
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // unpack(qweight [blocks, bytes], blocks, M, N) -> int8 signs [blocks, M, N], or None
 PyObject *host_unpack(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 4) return PyErr_Format(PyExc_TypeError, "unpack takes 4 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *q = tensor_arg(a[0]);
         int64_t blocks, M, N;
         if (!int_arg(a[1], blocks) || !int_arg(a[2], M) || !int_arg(a[3], N)) return nullptr;
@@ -186,15 +186,13 @@ PyObject *host_unpack(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                       c10::hip::getCurrentHIPStream(dev.index()).stream());
         if (st != BS_OK) return raise_status(st, "bs_unpack_sign");
         return THPVariable_Wrap(s);
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // rebuild_from_sign(signs [I, M, N] int8, u, vt, I) -> w [M, N], or None (u and vt may hold more blocks)
 PyObject *host_rebuild_from_sign(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 4) return PyErr_Format(PyExc_TypeError, "rebuild_from_sign takes 4 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *s = tensor_arg(a[0]), *u = tensor_arg(a[1]), *vt = tensor_arg(a[2]);
         int64_t I;
         if (!int_arg(a[3], I)) return nullptr;
@@ -212,15 +210,13 @@ PyObject *host_rebuild_from_sign(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                                   c10::hip::getCurrentHIPStream(dev.index()).stream());
         if (st != BS_OK) return raise_status(st, "bs_reconstruct_w_from_sign");
         return THPVariable_Wrap(w);
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // linear(x, w, bias or None) -> x @ w^T (+ bias), or None
 PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 3) return PyErr_Format(PyExc_TypeError, "linear takes 3 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *x = tensor_arg(a[0]), *w = tensor_arg(a[1]);
         const at::Tensor *bias = a[2] == Py_None ? nullptr : tensor_arg(a[2]);
         if (!x || !w || (a[2] != Py_None && !bias) || !x->is_cuda() || x->dim() < 1 || w->dim() != 2) Py_RETURN_NONE;
@@ -236,21 +232,17 @@ PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                      c10::hip::getCurrentHIPStream(dev.index()).stream());
         if (st != BS_OK) return raise_status(st, "bs_linear_f16");
         return THPVariable_Wrap(y);
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // workspace(device index, nbytes) -> the scratch tensor of the device's current stream
 PyObject *host_workspace(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 2) return PyErr_Format(PyExc_TypeError, "workspace takes 2 arguments");
-    try {
+    HANDLE_TH_ERRORS
         int64_t dev, bytes;
         if (!int_arg(a[0], dev) || !int_arg(a[1], bytes)) return nullptr;
         return THPVariable_Wrap(workspace_for((int)dev, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(), bytes));
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- a decode step's launches as one call -----------------------------------------------------------
@@ -285,7 +277,8 @@ void free_steps(PyObject *cap) { delete (Steps *)PyCapsule_GetPointer(cap, STEPS
 //             ("norm", x, weight, y, T, H, eps), ...]) -> handle; every tensor as its address
 PyObject *host_make_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 1 || !PyList_Check(a[0])) return PyErr_Format(PyExc_TypeError, "make_steps takes a list");
-    Steps *steps = new Steps;
+    HANDLE_TH_ERRORS
+    std::unique_ptr<Steps> steps(new Steps);
     for (Py_ssize_t j = 0; j < PyList_GET_SIZE(a[0]); j++) {
         PyObject *t = PyList_GET_ITEM(a[0], j);
         Step s = {};
@@ -307,10 +300,7 @@ PyObject *host_make_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
                 s.residual = (const void *)(uintptr_t)p[2];
                 s.y = (void *)(uintptr_t)p[3];
                 const int64_t need = bs_forward_group_workspace_bytes(s.mats.data(), count, s.N, s.K, s.T);
-                if (need < 0) {
-                    delete steps;
-                    return raise_status((int)need, "bs_forward_group_workspace_bytes");
-                }
+                if (need < 0) return raise_status((int)need, "bs_forward_group_workspace_bytes");
                 if (need > steps->need) steps->need = need;
             }
         } else if (ok && kind[0] == 'n') {
@@ -334,19 +324,21 @@ PyObject *host_make_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
             if (need > steps->need) steps->need = need;      // (a shape that is not taken is reported by the call)
         }
         if (!ok || PyErr_Occurred()) {
-            delete steps;
             if (!PyErr_Occurred()) PyErr_Format(PyExc_ValueError, "make_steps: item %zd is not a launch", j);
             return nullptr;
         }
         steps->list.push_back(std::move(s));
     }
-    return PyCapsule_New(steps, STEPS, free_steps);
+    PyObject *handle = PyCapsule_New(steps.get(), STEPS, free_steps);
+    if (handle) steps.release();                 // (the capsule's from here)
+    return handle;
+    END_HANDLE_TH_ERRORS
 }
 
 // run_steps(handle, device index): every launch, in order, on the device's current stream
 PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 2) return PyErr_Format(PyExc_TypeError, "run_steps takes 2 arguments");
-    try {
+    HANDLE_TH_ERRORS
         Steps *steps = (Steps *)PyCapsule_GetPointer(a[0], STEPS);
         int64_t index;
         if (!steps || !int_arg(a[1], index)) return nullptr;
@@ -379,15 +371,13 @@ PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
             }
         }
         Py_RETURN_NONE;
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // argmax(x [B, V], out int64 [B]) -> True, or None
 PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 2) return PyErr_Format(PyExc_TypeError, "argmax takes 2 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *x = tensor_arg(a[0]), *out = tensor_arg(a[1]);
         if (!x || !out || !x->is_cuda() || x->dim() != 2) Py_RETURN_NONE;
         const c10::Device dev = x->device();
@@ -399,9 +389,7 @@ PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                      c10::hip::getCurrentHIPStream(dev.index()).stream());
         if (st != BS_OK) return raise_status(st, "bs_argmax_f16");
         Py_RETURN_TRUE;
-    } catch (const std::exception &e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 #define HOST_METHOD(name) {#name, (PyCFunction)(void (*)(void))host_##name, METH_FASTCALL, nullptr}

@@ -73,3 +73,32 @@ def test_the_host_module_has_no_thread_local_storage():
     offset, size, count = struct.unpack_from("<Q", data, 32)[0], *struct.unpack_from("<HH", data, 54)
     kinds = [struct.unpack_from("<I", data, offset + k * size)[0] for k in range(count)]
     assert 1 in kinds and 7 not in kinds      # PT_LOAD, PT_TLS
+
+
+@pytest.fixture
+def little_memory():
+    """One GiB of GPU memory beyond what is reserved."""
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 30)) / total)
+    yield
+    torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.gpu
+def test_an_allocation_that_fails_is_torchs_out_of_memory_error(little_memory):
+    dev = torch.device("cuda")
+    H = _lib.host()
+    x, w = torch.zeros(1 << 16, 128, device=dev).half(), torch.zeros(1 << 15, 128, device=dev).half()
+    before = _lib.workspace(dev, 1)
+    with pytest.raises(torch.OutOfMemoryError):
+        H.linear(x, w, None)                                                      # 4 GiB of output
+    for _ in range(3):
+        with pytest.raises(torch.OutOfMemoryError):
+            _lib.workspace(dev, 4 << 30)
+    assert _lib.workspace(dev, 1).data_ptr() == before.data_ptr()                 # ... and the scratch is what it was
+    q, u, vt = torch.zeros(1, (1 << 15) * 16, dtype=torch.uint8, device=dev), torch.zeros(1, 1 << 15, 16, device=dev).half(), torch.zeros(1, 16, 128, device=dev).half()
+    with pytest.raises(torch.OutOfMemoryError):
+        H.forward(q, u, vt, 1, x, None)
+    with pytest.raises(torch.OutOfMemoryError):
+        H.unpack(torch.zeros(4, (1 << 29) // 8, dtype=torch.uint8, device=dev), 4, 1 << 20, 512)

@@ -43,19 +43,24 @@ Scratch &scratch() {
     return *s;
 }
 
+// The lock covers the table only: an allocation may wait for the device or for the interpreter, and may call back into Python
+// (out-of-memory observers, recorded stacks), which may come here again.
 at::Tensor workspace_for(int device, hipStream_t stream, int64_t bytes) {
     Scratch &s = scratch();
+    int64_t size = bytes > (1 << 20) ? bytes : (1 << 20);
+    {
+        std::lock_guard<std::mutex> guard(s.lock);
+        const at::Tensor &t = s.current[{device, stream}];
+        if (t.defined() && t.numel() >= bytes) return t;
+        // grow geometrically so that a sequence of slowly growing requests retires few buffers
+        if (t.defined() && 2 * t.numel() > size) size = 2 * t.numel();
+    }
+    at::Tensor fresh = at::empty({size}, at::TensorOptions().dtype(at::kByte).device(at::kCUDA, (c10::DeviceIndex)device));
     std::lock_guard<std::mutex> guard(s.lock);
     at::Tensor &t = s.current[{device, stream}];
-    if (!t.defined() || t.numel() < bytes) {
-        int64_t size = bytes > (1 << 20) ? bytes : (1 << 20);
-        if (t.defined()) {
-            // grow geometrically so that a sequence of slowly growing requests retires few buffers
-            if (2 * t.numel() > size) size = 2 * t.numel();
-            s.retired.push_back(t);
-        }
-        t = at::empty({size}, at::TensorOptions().dtype(at::kByte).device(at::kCUDA, (c10::DeviceIndex)device));
-    }
+    if (t.defined() && t.numel() >= bytes) return t;         // (another thread was quicker on this stream: `fresh` goes back unused)
+    if (t.defined()) s.retired.push_back(t);
+    t = fresh;
     return t;
 }
 

@@ -102,3 +102,38 @@ def test_an_allocation_that_fails_is_torchs_out_of_memory_error(little_memory):
         H.forward(q, u, vt, 1, x, None)
     with pytest.raises(torch.OutOfMemoryError):
         H.unpack(torch.zeros(4, (1 << 29) // 8, dtype=torch.uint8, device=dev), 4, 1 << 20, 512)
+
+
+@pytest.mark.gpu
+def test_scratch_can_be_asked_for_while_it_is_being_allocated(little_memory):
+    """An out-of-memory observer runs inside the allocation: what it calls may want scratch too."""
+    dev = torch.device("cuda")
+    have = _lib.workspace(dev, 1)
+    got = []
+    torch._C._cuda_attach_out_of_memory_observer(lambda *args: got.append(_lib.workspace(dev, 1).data_ptr()) if not got else None)
+    with pytest.raises(torch.OutOfMemoryError):
+        _lib.workspace(dev, 4 << 30)
+    assert got == [have.data_ptr()]
+
+
+@pytest.mark.gpu
+def test_threads_grow_the_scratch_of_one_stream_together():
+    import threading
+    dev = torch.device("cuda")
+    with torch.cuda.stream(torch.cuda.Stream()):
+        stream = torch.cuda.current_stream()
+        sizes, tensors = [], []
+        def grow(k):
+            with torch.cuda.stream(stream):
+                for j in range(1, 40):
+                    n = (1 << 20) + 4096 * j * (k + 1)
+                    t = _lib.workspace(dev, n)
+                    sizes.append(t.numel() >= n)
+                    tensors.append(t)
+        threads = [threading.Thread(target=grow, args=(k,)) for k in range(6)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert all(sizes) and len(sizes) == 6 * 39
+        assert len({t.data_ptr() for t in tensors}) <= 8 and _lib.workspace(dev, 1).data_ptr() == max(tensors, key=lambda t: t.numel()).data_ptr()

@@ -33,9 +33,15 @@ namespace {
 // captured while it was current has its address baked in, and its replays must keep writing into memory nobody else
 // owns.  (A graph captured before a growth still uses the old buffer; it stays correct, it just does not share scratch
 // with later eager calls.)  The table lives until the process ends: tensors must not outlive the HIP runtime's tear-down.
+// Threads that share a stream share its scratch, and other Python threads run during a call: what a call keeps there between two
+// of its kernels is safe because its launches are issued under `launching`.
+struct Space {
+    at::Tensor buffer;
+    std::mutex launching;
+};
 struct Scratch {
-    std::mutex lock;
-    std::map<std::pair<int, hipStream_t>, at::Tensor> current;
+    std::mutex lock;                             // of the table only
+    std::map<std::pair<int, hipStream_t>, Space> current;
     std::vector<at::Tensor> retired;
 };
 Scratch &scratch() {
@@ -43,25 +49,33 @@ Scratch &scratch() {
     return *s;
 }
 
-// The lock covers the table only: an allocation may wait for the device or for the interpreter, and may call back into Python
+struct Workspace {
+    at::Tensor buffer;
+    std::mutex *launching;
+    void *data() const { return buffer.mutable_data_ptr(); }
+};
+// No lock is held through the allocation: it may wait for the device or for the interpreter, and may call back into Python
 // (out-of-memory observers, recorded stacks), which may come here again.
-at::Tensor workspace_for(int device, hipStream_t stream, int64_t bytes) {
+Workspace workspace_for(int device, hipStream_t stream, int64_t bytes) {
     Scratch &s = scratch();
     int64_t size = bytes > (1 << 20) ? bytes : (1 << 20);
     {
         std::lock_guard<std::mutex> guard(s.lock);
-        const at::Tensor &t = s.current[{device, stream}];
-        if (t.defined() && t.numel() >= bytes) return t;
+        Space &space = s.current[{device, stream}];
+        const at::Tensor &t = space.buffer;
+        if (t.defined() && t.numel() >= bytes) return {t, &space.launching};
         // grow geometrically so that a sequence of slowly growing requests retires few buffers
         if (t.defined() && 2 * t.numel() > size) size = 2 * t.numel();
     }
     at::Tensor fresh = at::empty({size}, at::TensorOptions().dtype(at::kByte).device(at::kCUDA, (c10::DeviceIndex)device));
     std::lock_guard<std::mutex> guard(s.lock);
-    at::Tensor &t = s.current[{device, stream}];
-    if (t.defined() && t.numel() >= bytes) return t;         // (another thread was quicker on this stream: `fresh` goes back unused)
-    if (t.defined()) s.retired.push_back(t);
-    t = fresh;
-    return t;
+    Space &space = s.current[{device, stream}];
+    at::Tensor &t = space.buffer;
+    if (!t.defined() || t.numel() < bytes) {     // (else another thread was quicker on this stream: `fresh` goes back unused)
+        if (t.defined()) s.retired.push_back(t);
+        t = fresh;
+    }
+    return {t, &space.launching};
 }
 
 // ---- arguments -----------------------------------------------------------------------------------
@@ -78,22 +92,24 @@ PyObject *raise_status(int status, const char *what) {
 
 // The first `blocks` of the stacked buffers of one matrix, if they are what the C ABI takes as they lie.
 struct Matrix {
-    const at::Tensor *q, *u, *vt;
+    const uint8_t *q;
+    const void *u, *vt;
     int64_t I, M, N, K;
 };
 bool matrix_args(PyObject *const *a, int64_t blocks, c10::Device dev, Matrix &m) {
-    m.q = tensor_arg(a[0]);
-    m.u = tensor_arg(a[1]);
-    m.vt = tensor_arg(a[2]);
-    if (!m.q || !m.u || !m.vt) return false;
-    if (!plain(*m.q, at::kByte, dev) || !plain(*m.u, at::kHalf, dev) || !plain(*m.vt, at::kHalf, dev)) return false;
-    if (m.q->dim() != 2 || m.u->dim() != 3 || m.vt->dim() != 3) return false;
+    const at::Tensor *q = tensor_arg(a[0]), *u = tensor_arg(a[1]), *vt = tensor_arg(a[2]);
+    if (!q || !u || !vt) return false;
+    if (!plain(*q, at::kByte, dev) || !plain(*u, at::kHalf, dev) || !plain(*vt, at::kHalf, dev)) return false;
+    if (q->dim() != 2 || u->dim() != 3 || vt->dim() != 3) return false;
     m.I = blocks;
-    m.M = m.u->size(1);
-    m.K = m.u->size(2);
-    m.N = m.vt->size(2);
-    if (blocks < 1 || blocks > m.u->size(0) || blocks > m.vt->size(0) || blocks > m.q->size(0)) return false;
-    if (m.vt->size(1) != m.K || m.q->size(1) != (m.M * m.N + 7) / 8) return false;
+    m.M = u->size(1);
+    m.K = u->size(2);
+    m.N = vt->size(2);
+    if (blocks < 1 || blocks > u->size(0) || blocks > vt->size(0) || blocks > q->size(0)) return false;
+    if (vt->size(1) != m.K || q->size(1) != (m.M * m.N + 7) / 8) return false;
+    m.q = (const uint8_t *)q->const_data_ptr();
+    m.u = u->const_data_ptr();
+    m.vt = vt->const_data_ptr();
     return m.M > 0 && m.N > 0 && m.M * m.N < ((int64_t)1 << 40) && m.M < INT32_MAX && m.N < INT32_MAX;
 }
 
@@ -112,6 +128,20 @@ c10::SmallVector<int64_t, 6> output_sizes(const at::Tensor &x, int64_t last) {
     c10::SmallVector<int64_t, 6> s(x.sizes().begin(), x.sizes().end());
     s.back() = last;
     return s;
+}
+
+// Other Python threads run while a call allocates and launches: with the launch queue full, a launch waits for the device.
+// Pointers and sizes are read from the arguments before, and the caller holds the tensors.
+struct OtherThreadsRun {
+    PyThreadState *state = PyEval_SaveThread();
+    OtherThreadsRun() = default;
+    OtherThreadsRun(const OtherThreadsRun &) = delete;
+    ~OtherThreadsRun() { PyEval_RestoreThread(state); }
+};
+template <class F>
+auto while_others_run(F &&f) {
+    OtherThreadsRun scope;
+    return f();
 }
 
 // A guard only where the tensors' device is not the current one (asking costs less than setting it).
@@ -142,13 +172,18 @@ PyObject *host_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const int T = (int)(x->numel() / m.N);
         const int64_t need = bs_workspace_bytes((int)m.I, (int)m.M, (int)m.N, (int)m.K, T);
         if (need < 0) return raise_status((int)need, "bs_workspace_bytes");
-        DeviceScope scope(dev);
-        const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-        const at::Tensor ws = workspace_for(dev.index(), stream, need);
-        const at::Tensor y = new_half(output_sizes(*x, m.M), dev);
-        const int st = bs_forward((const uint8_t *)m.q->const_data_ptr(), m.u->const_data_ptr(), m.vt->const_data_ptr(),
-                                  x->const_data_ptr(), bias ? bias->const_data_ptr() : nullptr, y.mutable_data_ptr(), (int)m.I,
-                                  (int)m.M, (int)m.N, (int)m.K, T, ws.mutable_data_ptr(), ws.numel(), stream);
+        const void *xp = x->const_data_ptr(), *bp = bias ? bias->const_data_ptr() : nullptr;
+        const auto sizes = output_sizes(*x, m.M);
+        at::Tensor y;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+            const Workspace ws = workspace_for(dev.index(), stream, need);
+            y = new_half(sizes, dev);
+            std::lock_guard<std::mutex> launching(*ws.launching);
+            return bs_forward(m.q, m.u, m.vt, xp, bp, y.mutable_data_ptr(), (int)m.I, (int)m.M, (int)m.N, (int)m.K, T,
+                              ws.data(), ws.buffer.numel(), stream);
+        });
         if (st != BS_OK) return raise_status(st, "bs_forward");
         return THPVariable_Wrap(y);
     END_HANDLE_TH_ERRORS
@@ -164,11 +199,13 @@ PyObject *host_rebuild(PyObject *, PyObject *const *a, Py_ssize_t n) {
         Matrix m;
         if (!u || !u->is_cuda() || !matrix_args(a, blocks, u->device(), m)) Py_RETURN_NONE;
         const c10::Device dev = u->device();
-        DeviceScope scope(dev);
-        const at::Tensor w = new_half({m.M, m.N}, dev);
-        const int st = bs_reconstruct_w((const uint8_t *)m.q->const_data_ptr(), m.u->const_data_ptr(), m.vt->const_data_ptr(),
-                                        w.mutable_data_ptr(), (int)m.I, (int)m.M, (int)m.N, (int)m.K,
-                                        c10::hip::getCurrentHIPStream(dev.index()).stream());
+        at::Tensor w;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            w = new_half({m.M, m.N}, dev);
+            return bs_reconstruct_w(m.q, m.u, m.vt, w.mutable_data_ptr(), (int)m.I, (int)m.M, (int)m.N, (int)m.K,
+                                    c10::hip::getCurrentHIPStream(dev.index()).stream());
+        });
         if (st != BS_OK) return raise_status(st, "bs_reconstruct_w");
         return THPVariable_Wrap(w);
     END_HANDLE_TH_ERRORS
@@ -185,10 +222,13 @@ PyObject *host_unpack(PyObject *, PyObject *const *a, Py_ssize_t n) {
         if (blocks < 1 || blocks > q->size(0) || M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX || M * N % 8 != 0 || q->size(1) != M * N / 8)
             Py_RETURN_NONE;                      // (blocks of whole bytes follow each other without padding)
         const c10::Device dev = q->device();
-        DeviceScope scope(dev);
-        const at::Tensor s = at::Tensor(at::detail::empty_cuda({blocks, M, N}, at::kChar, dev, std::nullopt));
-        const int st = bs_unpack_sign((const uint8_t *)q->const_data_ptr(), (int8_t *)s.mutable_data_ptr(), blocks * M * N,
-                                      c10::hip::getCurrentHIPStream(dev.index()).stream());
+        const uint8_t *from = (const uint8_t *)q->const_data_ptr();
+        at::Tensor s;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            s = at::Tensor(at::detail::empty_cuda({blocks, M, N}, at::kChar, dev, std::nullopt));
+            return bs_unpack_sign(from, (int8_t *)s.mutable_data_ptr(), blocks * M * N, c10::hip::getCurrentHIPStream(dev.index()).stream());
+        });
         if (st != BS_OK) return raise_status(st, "bs_unpack_sign");
         return THPVariable_Wrap(s);
     END_HANDLE_TH_ERRORS
@@ -208,11 +248,15 @@ PyObject *host_rebuild_from_sign(PyObject *, PyObject *const *a, Py_ssize_t n) {
         if (I < 1 || s->size(0) != I || u->size(0) < I || vt->size(0) < I || vt->size(1) != K || s->size(1) != M || s->size(2) != N ||
             M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX)
             Py_RETURN_NONE;
-        DeviceScope scope(dev);
-        const at::Tensor w = new_half({M, N}, dev);
-        const int st = bs_reconstruct_w_from_sign((const int8_t *)s->const_data_ptr(), u->const_data_ptr(), vt->const_data_ptr(),
-                                                  w.mutable_data_ptr(), (int)I, (int)M, (int)N, (int)K,
-                                                  c10::hip::getCurrentHIPStream(dev.index()).stream());
+        const int8_t *sp = (const int8_t *)s->const_data_ptr();
+        const void *up = u->const_data_ptr(), *vp = vt->const_data_ptr();
+        at::Tensor w;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            w = new_half({M, N}, dev);
+            return bs_reconstruct_w_from_sign(sp, up, vp, w.mutable_data_ptr(), (int)I, (int)M, (int)N, (int)K,
+                                              c10::hip::getCurrentHIPStream(dev.index()).stream());
+        });
         if (st != BS_OK) return raise_status(st, "bs_reconstruct_w_from_sign");
         return THPVariable_Wrap(w);
     END_HANDLE_TH_ERRORS
@@ -230,11 +274,15 @@ PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const int64_t M = w->size(0), N = w->size(1);
         if (M < 1 || N < 1 || M >= INT32_MAX || N >= INT32_MAX || x->size(-1) != N || x->numel() == 0 || x->numel() / N >= INT32_MAX) Py_RETURN_NONE;
         if (bias && (!plain(*bias, at::kHalf, dev) || bias->numel() != M)) Py_RETURN_NONE;
-        DeviceScope scope(dev);
-        const at::Tensor y = new_half(output_sizes(*x, M), dev);
-        const int st = bs_linear_f16(x->const_data_ptr(), w->const_data_ptr(), bias ? bias->const_data_ptr() : nullptr,
-                                     y.mutable_data_ptr(), (int)(x->numel() / N), (int)M, (int)N,
-                                     c10::hip::getCurrentHIPStream(dev.index()).stream());
+        const void *xp = x->const_data_ptr(), *wp = w->const_data_ptr(), *bp = bias ? bias->const_data_ptr() : nullptr;
+        const int T = (int)(x->numel() / N);
+        const auto sizes = output_sizes(*x, M);
+        at::Tensor y;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            y = new_half(sizes, dev);
+            return bs_linear_f16(xp, wp, bp, y.mutable_data_ptr(), T, (int)M, (int)N, c10::hip::getCurrentHIPStream(dev.index()).stream());
+        });
         if (st != BS_OK) return raise_status(st, "bs_linear_f16");
         return THPVariable_Wrap(y);
     END_HANDLE_TH_ERRORS
@@ -246,7 +294,9 @@ PyObject *host_workspace(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
         int64_t dev, bytes;
         if (!int_arg(a[0], dev) || !int_arg(a[1], bytes)) return nullptr;
-        return THPVariable_Wrap(workspace_for((int)dev, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(), bytes));
+        return THPVariable_Wrap(while_others_run([&] {
+            return workspace_for((int)dev, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(), bytes).buffer;
+        }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -348,33 +398,42 @@ PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
         int64_t index;
         if (!steps || !int_arg(a[1], index)) return nullptr;
         const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)index);
-        DeviceScope scope(dev);
-        const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-        at::Tensor ws = workspace_for(dev.index(), stream, steps->need);
-        for (const Step &s : steps->list) {
-            int st;
-            if (s.kind == Step::GROUP) {
-                const int count = (int)s.mats.size();
-                for (int turn = 0;; turn++) {
-                    st = s.rms ? bs_forward_group_rms(s.mats.data(), count, s.N, s.K, s.x, s.T, s.eps, s.epilogue, s.residual, s.y,
-                                                      ws.mutable_data_ptr(), ws.numel(), stream)
-                               : bs_forward_group(s.mats.data(), count, s.N, s.K, s.x, s.T, s.epilogue, s.residual, s.y,
-                                                  ws.mutable_data_ptr(), ws.numel(), stream);
-                    if (st != BS_ERR_WORKSPACE || turn > 0) break;
-                    // another kernel has been chosen since (bs_set_decode_kernel): its scratch may be larger
-                    const int64_t need = bs_forward_group_workspace_bytes(s.mats.data(), count, s.N, s.K, s.T);
-                    ws = workspace_for(dev.index(), stream, need);
+        const char *what = nullptr;
+        const int st = while_others_run([&] {
+            int st = BS_OK;
+            DeviceScope scope(dev);
+            const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+            Workspace ws = workspace_for(dev.index(), stream, steps->need);
+            // one launch pair at a time: nothing is kept in the scratch from one to the next
+            auto issue = [&](const Step &s) {
+                std::lock_guard<std::mutex> launching(*ws.launching);
+                if (s.kind == Step::GROUP) {
+                    what = "bs_forward_group";
+                    return s.rms ? bs_forward_group_rms(s.mats.data(), (int)s.mats.size(), s.N, s.K, s.x, s.T, s.eps, s.epilogue, s.residual,
+                                                        s.y, ws.data(), ws.buffer.numel(), stream)
+                                 : bs_forward_group(s.mats.data(), (int)s.mats.size(), s.N, s.K, s.x, s.T, s.epilogue, s.residual, s.y,
+                                                    ws.data(), ws.buffer.numel(), stream);
                 }
-                if (st != BS_OK) return raise_status(st, "bs_forward_group");
-            } else if (s.kind == Step::NORM) {
-                st = bs_rmsnorm_f16(s.x, s.weight, s.y, s.T, s.N, s.eps, stream);
-                if (st != BS_OK) return raise_status(st, "bs_rmsnorm_f16");
-            } else {
-                st = bs_attention_decode_ws_f16(s.qkv, s.kcache, s.vcache, s.cos, s.sin, s.pos, s.out, s.B, s.heads, s.kv_heads, s.head_dim,
-                                                s.max_len, ws.mutable_data_ptr(), ws.numel(), stream);
-                if (st != BS_OK) return raise_status(st, "bs_attention_decode_f16");
+                if (s.kind == Step::NORM) {
+                    what = "bs_rmsnorm_f16";
+                    return bs_rmsnorm_f16(s.x, s.weight, s.y, s.T, s.N, s.eps, stream);
+                }
+                what = "bs_attention_decode_f16";
+                return bs_attention_decode_ws_f16(s.qkv, s.kcache, s.vcache, s.cos, s.sin, s.pos, s.out, s.B, s.heads, s.kv_heads, s.head_dim,
+                                                  s.max_len, ws.data(), ws.buffer.numel(), stream);
+            };
+            for (const Step &s : steps->list) {
+                st = issue(s);
+                if (st == BS_ERR_WORKSPACE && s.kind == Step::GROUP) {
+                    // another kernel has been chosen since (bs_set_decode_kernel): its scratch may be larger
+                    ws = workspace_for(dev.index(), stream, bs_forward_group_workspace_bytes(s.mats.data(), (int)s.mats.size(), s.N, s.K, s.T));
+                    st = issue(s);
+                }
+                if (st != BS_OK) break;
             }
-        }
+            return st;
+        });
+        if (st != BS_OK) return raise_status(st, what);
         Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
 }
@@ -389,9 +448,13 @@ PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
         if (!plain(*x, at::kHalf, dev) || !plain(*out, at::kLong, dev) || out->numel() != x->size(0) || x->numel() == 0 ||
             x->size(0) >= INT32_MAX || x->size(1) >= INT32_MAX)
             Py_RETURN_NONE;
-        DeviceScope scope(dev);
-        const int st = bs_argmax_f16(x->const_data_ptr(), (int64_t *)out->mutable_data_ptr(), (int)x->size(0), (int)x->size(1),
-                                     c10::hip::getCurrentHIPStream(dev.index()).stream());
+        const void *xp = x->const_data_ptr();
+        int64_t *op = (int64_t *)out->mutable_data_ptr();
+        const int B = (int)x->size(0), V = (int)x->size(1);
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            return bs_argmax_f16(xp, op, B, V, c10::hip::getCurrentHIPStream(dev.index()).stream());
+        });
         if (st != BS_OK) return raise_status(st, "bs_argmax_f16");
         Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS

@@ -172,7 +172,7 @@ class SyntheticLlamaDecoder:
         self.span = torch.arange(max_len, device=self.dev)
         self.logits = None
         self._groups = None
-        self._steps = None                                                 # (what it was made for, (launch list, last norm in it), its tensors)
+        self._steps = None                                                 # (what it was made for, (launch list, last norm in it, its tensors))
 
     @classmethod
     def from_checkpoint(cls, path, max_len, device, compression_config=None, niter=None, max_memory_MB=None, batch=1):
@@ -378,8 +378,8 @@ class SyntheticLlamaDecoder:
 
     def _launches(self):
         """(the launches of step_fused() between the embedding and the last norm as one native list (host.cpp), whether that norm
-        is in it).  Laid out once and again whenever one of the tensors whose addresses it holds has become another one, by address,
-        shape, strides or type; it keeps those tensors alive."""
+        is in it, every tensor whose address it holds).  Laid out once and again whenever one of the tensors has become another one,
+        by address, shape, strides or type.  Whoever runs the list holds the tensors meanwhile: other threads run too."""
         if self._groups is None:
             self._build_groups()
         held = (self.kcache, self.vcache, self.cos, self.sin, self.pos, self.final_norm)
@@ -419,19 +419,21 @@ class SyntheticLlamaDecoder:
         inside = tuple(w.shape) == (s.hidden,) and w.dtype == torch.float16 and w.is_contiguous() and w.device == dev
         if inside:
             items.append(("norm", xa, norm, self._hn.data_ptr(), B, s.hidden, eps))
-        self._steps = (key, (_lib.host().make_steps(items), inside), held)
+        kept = (held, self._groups, self._xa, self._xb, self._qkv, self._ctx, self._act, self._hn)
+        self._steps = (key, (_lib.host().make_steps(items), inside, kept))
         return self._steps[1]
 
     @torch.no_grad()
     def step_fused(self):
         """Same step on the library's grouped forwards and decode-step kernels: q/k/v with the RMSNorm in front, attention,
         o + residual, gate/up with the RMSNorm in front and the SiLU product, down + residual per layer."""
-        launches, normed = self._launches()
-        torch.index_select(self.embed, 0, self.token, out=self._xa)
-        _lib.host().run_steps(launches, self._xa.device.index)
+        launches, normed, kept = self._launches()
+        xa, hn = self._xa, self._hn
+        torch.index_select(self.embed, 0, self.token, out=xa)
+        _lib.host().run_steps(launches, xa.device.index)
         if not normed:
-            rmsnorm_hip(self._xa, self.final_norm, self.s.rms_eps, out=self._hn)
-        self.logits = F.linear(self._hn, self.lm_head)
+            rmsnorm_hip(xa, self.final_norm, self.s.rms_eps, out=hn)
+        self.logits = F.linear(hn, self.lm_head)
         argmax_hip(self.logits, out=self.token)
         self.pos.add_(1)
 

@@ -137,3 +137,72 @@ def test_threads_grow_the_scratch_of_one_stream_together():
             t.join()
         assert all(sizes) and len(sizes) == 6 * 39
         assert len({t.data_ptr() for t in tensors}) <= 8 and _lib.workspace(dev, 1).data_ptr() == max(tensors, key=lambda t: t.numel()).data_ptr()
+
+
+def _calls(dev):
+    """name -> a call of each entry point that launches."""
+    mod, x = layer(2, 512, 1024, 2, dev)
+    H = _lib.host()
+    w = mod._rebuilt()
+    sign = H.unpack(mod.qweight, 2, 512, 1024)
+    out = torch.zeros(2, dtype=torch.long, device=dev)
+    y = torch.empty(2, 1024, dtype=torch.float16, device=dev)
+    weight = torch.ones(1024, dtype=torch.float16, device=dev)
+    steps = H.make_steps([("norm", x.data_ptr(), weight.data_ptr(), y.data_ptr(), 2, 1024, 1e-5)])
+    return {"forward": lambda: H.forward(mod.qweight, mod.u, mod.vt, 2, x, mod.bias), "rebuild": lambda: H.rebuild(mod.qweight, mod.u, mod.vt, 2),
+            "unpack": lambda: H.unpack(mod.qweight, 2, 512, 1024), "rebuild_from_sign": lambda: H.rebuild_from_sign(sign, mod.u, mod.vt, 2),
+            "linear": lambda: H.linear(x, w, None), "argmax": lambda: H.argmax(x, out), "workspace": lambda: H.workspace(dev.index, 1),
+            "run_steps": lambda: (H.run_steps(steps, dev.index), y, weight)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["forward", "rebuild", "unpack", "rebuild_from_sign", "linear", "argmax", "workspace", "run_steps"])
+def test_other_threads_run_during_a_call(name):
+    import sys
+    import threading
+    import time
+    call = _calls(torch.device("cuda", torch.cuda.current_device()))[name]
+    call()
+    torch.cuda.synchronize()
+    ran = []
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=lambda: (time.sleep(0.05), ran.append(1)))
+    thread.start()
+    try:
+        sys.setswitchinterval(1000.0)            # from here a thread that computes keeps the interpreter until it lets go of it
+        end = time.perf_counter() + 0.15
+        while time.perf_counter() < end:
+            pass
+        assert not ran                           # (waiting for the interpreter since its sleep ended)
+        for _ in range(20000):
+            call()
+            if ran:
+                break
+        seen = bool(ran)                         # (a synchronisation lets go of it too)
+    finally:
+        sys.setswitchinterval(interval)
+    thread.join()
+    assert seen
+
+
+@pytest.mark.gpu
+def test_threads_that_share_a_stream_do_not_mix_their_scratch():
+    import threading
+    dev = torch.device("cuda")
+    work = [layer(I, M, N, T, dev) for I, M, N, T in ((3, 2048, 4096, 1), (2, 1024, 2048, 4), (2, 500, 640, 20), (3, 256, 512, 130))]
+    want = [mod(x) for mod, x in work]
+    wrong, total = [], []
+
+    def hammer(k):
+        mod, x = work[k]
+        for _ in range(300):
+            y = mod(x)
+            total.append(1)
+            if not torch.equal(y, want[k]):
+                wrong.append(k)
+    threads = [threading.Thread(target=hammer, args=(k,)) for k in range(len(work))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong and len(total) == 1200

@@ -172,3 +172,20 @@ def workspace(dev, nbytes: int):
     stays correct, it just does not share scratch with later eager calls.)"""
     index = torch.cuda.current_device() if dev.index is None else dev.index
     return host().workspace(index, nbytes)
+
+
+class scratch:
+    """`with scratch(dev, nbytes) as ws:` the scratch of workspace() for one C-ABI call that keeps something there between its
+    kernels: threads that share a stream share its scratch, and the interpreter lock is not held during such a call, so
+    the stream's other calls wait until the block is left."""
+
+    def __init__(self, dev, nbytes: int):
+        self.index = torch.cuda.current_device() if dev.index is None else dev.index
+        self.nbytes = int(nbytes)
+
+    def __enter__(self):
+        ws, self.key = host().hold(self.index, self.nbytes)
+        return ws
+
+    def __exit__(self, *error):
+        host().let_go(self.key)

@@ -300,6 +300,32 @@ PyObject *host_workspace(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// hold(device index, nbytes) -> (scratch tensor, key): as workspace(), with the stream's launches kept to this thread until let_go(key)
+PyObject *host_hold(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 2) return PyErr_Format(PyExc_TypeError, "hold takes 2 arguments");
+    HANDLE_TH_ERRORS
+        int64_t dev, bytes;
+        if (!int_arg(a[0], dev) || !int_arg(a[1], bytes)) return nullptr;
+        const Workspace ws = while_others_run([&] {
+            const Workspace w = workspace_for((int)dev, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(), bytes);
+            w.launching->lock();
+            return w;
+        });
+        PyObject *t = THPVariable_Wrap(ws.buffer), *key = PyLong_FromVoidPtr(ws.launching), *pair = t && key ? PyTuple_Pack(2, t, key) : nullptr;
+        Py_XDECREF(t);
+        Py_XDECREF(key);
+        if (!pair) ws.launching->unlock();
+        return pair;
+    END_HANDLE_TH_ERRORS
+}
+PyObject *host_let_go(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 1) return PyErr_Format(PyExc_TypeError, "let_go takes 1 argument");
+    std::mutex *m = (std::mutex *)PyLong_AsVoidPtr(a[0]);
+    if (!m) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "let_go takes what hold gave");
+    m->unlock();
+    Py_RETURN_NONE;
+}
+
 // ---- a decode step's launches as one call -----------------------------------------------------------
 // The launches between the embedding and the last norm never change between steps: their arguments are laid
 // out once (make_steps) and issued in one call (run_steps) - nine kernels per layer at the cost of the launches alone.
@@ -462,7 +488,7 @@ PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
 
 #define HOST_METHOD(name) {#name, (PyCFunction)(void (*)(void))host_##name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(unpack), HOST_METHOD(rebuild_from_sign), HOST_METHOD(linear), HOST_METHOD(workspace),
-                         HOST_METHOD(argmax), HOST_METHOD(make_steps), HOST_METHOD(run_steps), {nullptr, nullptr, 0, nullptr}};
+                         HOST_METHOD(hold), HOST_METHOD(let_go), HOST_METHOD(argmax), HOST_METHOD(make_steps), HOST_METHOD(run_steps), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native host path over libbitstack_hip.so.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -79,8 +79,7 @@ def bitstack_forward_hip(packed_sign, u, vt, x, bias=None):
     need = L.bs_workspace_bytes(I, M, N, K, T)
     if need < 0:
         _lib.check(int(need), "bs_workspace_bytes")
-    ws = _lib.workspace(dev, int(need))
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _lib.scratch(dev, need) as ws:
         _lib.check(L.bs_forward(_lib.ptr(packed_sign), _lib.ptr(u), _lib.ptr(vt), _lib.ptr(x2),
                                 _lib.ptr(bias), _lib.ptr(y), I, M, N, K, T, _lib.ptr(ws),
                                 ws.numel(), _lib.stream_ptr(dev)), "bs_forward")
@@ -154,8 +153,7 @@ def bitstack_forward_group_hip(group: MatrixGroup, x, epilogue=_lib.EPI_NONE, re
     y = out if out is not None else torch.empty((T, width), dtype=torch.float16, device=dev)
     if y.dtype != torch.float16 or not y.is_contiguous() or y.numel() != T * width:
         raise ValueError("out must be a contiguous fp16 [T, width] tensor")
-    ws = _lib.workspace(dev, need)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _lib.scratch(dev, need) as ws:
         if rms_eps is None:
             _lib.check(_lib.lib().bs_forward_group(group.arr, group.n, group.N, group.K, _lib.ptr(x2), T, epilogue,
                                                    _lib.ptr(residual), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
@@ -290,8 +288,7 @@ def forward_cat_hip(modules, x):
     if need <= 0:
         return None
     y = torch.empty((T, sum(group.M)), dtype=torch.float16, device=x.device)
-    with torch.cuda.device(x.device):
-        ws = _lib.workspace(x.device, need)
+    with torch.cuda.device(x.device), _lib.scratch(x.device, need) as ws:
         _lib.check(L.bs_forward_cat(group.arr, group.n, group.N, group.K, _lib.ptr(x), T, _lib.ptr(y), _lib.ptr(ws), ws.numel(),
                                     _lib.stream_ptr(x.device)), "bs_forward_cat")
     return y
@@ -315,12 +312,11 @@ def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, ou
     if cos.shape != (max_len, d // 2) or sin.shape != (max_len, d // 2) or not cos.is_contiguous() or not sin.is_contiguous():
         raise ValueError("cos / sin must be contiguous [max_len, head_dim / 2]")
     y = out if out is not None else torch.empty((B, heads * d), dtype=torch.float16, device=dev)
-    with torch.cuda.device(dev):
-        need = _lib.lib().bs_attention_decode_workspace_bytes(B, heads, kv_heads, d, max_len)
-        ws = _lib.workspace(dev, need) if need > 0 else None
+    need = max(0, int(_lib.lib().bs_attention_decode_workspace_bytes(B, heads, kv_heads, d, max_len)))     # (an error is the call's to report)
+    with torch.cuda.device(dev), _lib.scratch(dev, need) as ws:
         _lib.check(_lib.lib().bs_attention_decode_ws_f16(_lib.ptr(qkv), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(_f16c(cos)),
                                                          _lib.ptr(_f16c(sin)), _lib.ptr(pos), _lib.ptr(y), B, heads, kv_heads, d, max_len,
-                                                         _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(dev)),
+                                                         _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev)),
                    "bs_attention_decode_ws_f16")
     return y
 

@@ -189,20 +189,46 @@ def test_other_threads_run_during_a_call(name):
 def test_threads_that_share_a_stream_do_not_mix_their_scratch():
     import threading
     dev = torch.device("cuda")
-    work = [layer(I, M, N, T, dev) for I, M, N, T in ((3, 2048, 4096, 1), (2, 1024, 2048, 4), (2, 500, 640, 20), (3, 256, 512, 130))]
-    want = [mod(x) for mod, x in work]
+    calls = []
+    for I, M, N, T in ((3, 2048, 4096, 1), (2, 1024, 2048, 4), (2, 500, 640, 20), (3, 256, 512, 130)):
+        mod, x = layer(I, M, N, T, dev)
+        wide = torch.zeros(T, N + 8, dtype=torch.float16, device=dev)
+        wide[:, :N] = x
+        calls += [lambda mod=mod, x=x: mod(x), lambda mod=mod, x=wide[:, :N]: mod(x)]          # native, Python path
+    mods = [layer(2, M, 1024, 200, dev, bias=False) for M in (512, 128)]
+    calls.append(lambda: IU.forward_cat_hip([m for m, _ in mods], mods[0][1]))
+    group = IU.MatrixGroup.from_modules([m for m, _ in mods])
+    few = mods[0][1][:3].contiguous()
+    calls.append(lambda: IU.bitstack_forward_group_hip(group, few))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    qkv, cache = torch.randn(1, 48 * 128, generator=g, device=dev).half(), torch.randn(2, 1, 8, 2048, 128, generator=g, device=dev).half()
+    cos, pos = torch.rand(2048, 64, generator=g, device=dev).half(), torch.full((1,), 2000, device=dev)
+    calls.append(lambda: IU.attention_decode_hip(qkv, cache[0], cache[1], cos, cos, pos, 32, 8))
+    want = [call() for call in calls]
     wrong, total = [], []
 
     def hammer(k):
-        mod, x = work[k]
-        for _ in range(300):
-            y = mod(x)
+        for _ in range(100):
+            y = calls[k]()
             total.append(1)
             if not torch.equal(y, want[k]):
                 wrong.append(k)
-    threads = [threading.Thread(target=hammer, args=(k,)) for k in range(len(work))]
+    threads = [threading.Thread(target=hammer, args=(k,)) for k in range(len(calls))]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
-    assert not wrong and len(total) == 1200
+    assert not wrong and len(total) == 100 * len(calls)
+
+
+@pytest.mark.gpu
+def test_the_streams_launches_are_let_go_when_a_call_fails():
+    dev = torch.device("cuda")
+    with pytest.raises(RuntimeError):
+        with _lib.scratch(dev, 16) as ws:
+            assert ws.numel() >= 16
+            _lib.check(_lib.lib().bs_forward(None, None, None, None, None, None, 1, 16, 512, 16, 1, _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev)), "bs_forward")
+    mod, x = layer(1, 16, 512, 1, dev)
+    assert mod(x).shape == (1, 16)
+    with pytest.raises((ValueError, OverflowError, TypeError)):
+        _lib.host().let_go(0)

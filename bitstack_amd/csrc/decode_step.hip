@@ -66,7 +66,8 @@ __global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *x, c
 //   scores  S[position, head] = K q     16x16x32, K rows as loaded (a lane: position l % 16, dimensions 32 c + 8 (l / 16) ..)
 //   output  O[dim, head] += V^T P       16x16x32, four positions twice: P is split into two fp16 terms, p = hi + lo to 2^-22,
 //                                       and the eight k slots of a lane hold {hi, lo} against {v, v}, so the weights keep the
-//                                       precision they had as fp32 numbers
+//                                       precision they had as fp32 numbers; where an infinite v makes NaN of that, the wave
+//                                       goes over its positions again with fp32 weights (the check: 0.1 us)
 // A lane of the scores holds positions 4 (l / 16) + i of head l % 16, which is what the second product wants of P; V needs no
 // transposition either: a lane loads dimensions 8 r .. 8 r + 7 (r = l % 16) of its four positions, and product number j takes
 // half j of each, so that its row r is dimension 8 r + j.  K of the next tile is requested behind the scores, V behind the
@@ -140,7 +141,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
             v8[i] = *reinterpret_cast<const half8_t *>(vc + (int64_t)min(t * ATT_TILE + 4 * g + i, pos - 1) * ATT_D + 8 * r16);
     };
     const int step = split ? WAVES * (int)gridDim.y : WAVES;
-    int t = SPLIT ? wave + WAVES * (int)blockIdx.y : wave;
+    const int first = SPLIT ? wave + WAVES * (int)blockIdx.y : wave;
+    int t = first;
     const bool own = t == tiles % step;          // the wave whose turn is next takes this step's own position
     if (t < tiles) { fetch_k(t); fetch_v(t); }
 
@@ -213,19 +215,55 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
         if (next < tiles) fetch_v(next);
         t = next;
     }
-    if (own) {                                   // this step's own k and v, from LDS: a tile with one position
+    auto take_own = [&]() {                      // this step's own k and v, from LDS: a tile with one position
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             k8[c] = *reinterpret_cast<const half8_t *>(&knew[32 * c + 8 * g]);
             v8[c] = *reinterpret_cast<const half8_t *>(&vnew[8 * r16]);
         }
+    };
+    if (own) {
+        take_own();
         fold(scores(), 1);
     }
 
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if (r16 < HP) {
-        if (g == 0) { wm[r16][wave] = m; wl[r16][wave] = l; }
+    if (r16 < HP && g == 0) { wm[r16][wave] = m; wl[r16][wave] = l; }
+    const float4_t sums = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    const float sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    if (__builtin_expect(__any(sum != sum), 0)) {
+        // An infinite v: times a second term of zero or below it, or a masked weight, it is NaN in the output product.  The wave's
+        // positions once more, head by head, each weight as one fp32 number: a lane owns dimensions 8 r16 .. 8 r16 + 7.
+#pragma unroll 1
+        for (int h = 0; h < HP; h++) {
+            float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            auto add = [&](const float4_t s, int valid) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float w = __shfl(__builtin_amdgcn_exp2f(s[i] * scale2 - m), (lane & 48) | h, 64);
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (4 * g + i < valid) o[e] += w * (float)v8[i][e];
+                }
+            };
+            for (t = first; t < tiles; t += step) {
+                fetch_k(t);
+                fetch_v(t);
+                add(scores(), pos - t * ATT_TILE);
+            }
+            if (own) {
+                take_own();
+                add(scores(), 1);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                o[e] += __shfl_xor(o[e], 16, 64);
+                o[e] += __shfl_xor(o[e], 32, 64);
+                if (g == 0) wacc[h][wave][8 * r16 + e] = o[e];
+            }
+        }
+    } else if (r16 < HP) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {            // row 4 g + i of product j is dimension 8 (4 g + i) + j
             float *to = &wacc[r16][wave][8 * (4 * g + i)];

@@ -63,3 +63,32 @@ def test_attention_over_split_positions(B, heads, kv, max_len):
         assert bool(((got - ref).abs() <= bound).all())
     for at in (-1, max_len):                     # outside of the cache: zeros
         assert not IU.attention_decode_hip(qkv, kc, vc, cos, sin, torch.tensor([at], device="cuda"), heads, kv).any()
+
+
+@pytest.mark.parametrize("B,heads,kv,max_len,at", [(1, 32, 8, 272, 100), (2, 6, 2, 272, 33), (9, 32, 8, 272, 250), (17, 32, 8, 272, 128), (33, 32, 8, 272, 200),
+                                                   (1, 32, 8, 2100, 1500), (1, 6, 2, 2100, 1500), (2, 16, 16, 2100, 700)])
+def test_an_infinite_value_stays_infinite(B, heads, kv, max_len, at):
+    """Values of +inf and -inf in the cache (the first and the last row of it among them) and in this step's own row: the dimensions they
+    stand in come out as their sign, all others as if they were not there; one of each sign in a dimension makes NaN."""
+    print(f"infinite values B={B} heads={heads} kv={kv} max_len={max_len} at={at}", flush=True)
+    d, inf = 128, float("inf")
+    g = torch.Generator(device="cuda").manual_seed(at + heads)
+    k = torch.randn(B, kv, max_len, d, generator=g, device="cuda").half()
+    v = torch.randn(B, kv, max_len, d, generator=g, device="cuda").half()
+    qkv = torch.randn(B, (heads + 2 * kv) * d, generator=g, device="cuda").half()
+    vn = qkv[:, (heads + kv) * d:].view(B, kv, d)
+    v[:, :, 0, 3], v[:, 0, 20, 7], v[:, :, at - 1, 64], vn[:, :, 127] = inf, -inf, inf, -inf
+    v[:, :, 5, 90], v[:, :, at - 2, 90] = inf, -inf
+    cos, sin = torch.ones(max_len, d // 2).half().cuda(), torch.zeros(max_len, d // 2).half().cuda()
+    q, kn = qkv[:, :heads * d].double().view(B, kv, heads // kv, d), qkv[:, heads * d:(heads + kv) * d].view(B, kv, d)
+    got = IU.attention_decode_hip(qkv, k.clone(), v.clone(), cos, sin, torch.tensor([at], device="cuda"), heads, kv).double().view(B, kv, -1, d)
+    ks, vs = k[:, :, :at + 1].double(), v[:, :, :at + 1].double()
+    ks[:, :, at], vs[:, :, at] = kn.double(), vn.double()
+    p = torch.softmax((q.unsqueeze(3) * ks.unsqueeze(2)).sum(-1) / d ** 0.5, -1)
+    ref = (p.unsqueeze(-1) * vs.unsqueeze(2)).sum(3)
+    assert torch.equal(got.isnan(), ref.isnan()) and bool(ref[..., 90].isnan().all())
+    assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[ref.isinf()], ref[ref.isinf()]) and int(ref.isinf().sum()) >= 3 * B * heads
+    rest = ref.isfinite()
+    # one rounding to fp16; scores of size up to 5 in fp32 sums of 128 terms move the weights by at most 2^-14 of themselves
+    bound = ref.abs() * 2.0 ** -11 + float(vs[vs.isfinite()].abs().max()) * 2.0 ** -14 + 2.0 ** -25
+    assert bool(((got - ref).abs() <= bound)[rest].all())

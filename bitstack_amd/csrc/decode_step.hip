@@ -77,7 +77,7 @@ __global__ __launch_bounds__(RMS_THREADS) void rmsnorm_kernel(const half_t *x, c
 // position by position on the VALU (32 instructions per position and head) took 46 us
 // on 8 sequences x 64 heads (8 KV heads) at position 2100 where this takes 22.5 (69 MB: 3.1 TB/s), 18.7 / 8.8 on 16 x 32 at 300,
 // 8.2 / 6.9 on 1 x 32 at 384.
-constexpr int ATT_D = 128, ATT_MAX_LEN = 8192, ATT_TILE = 16, ATT_SPLIT_LEN = 1025, ATT_WHOLE = 512, ATT_MAX_SPLITS = 16, ATT_PART = ATT_D + 4;
+constexpr int ATT_D = 128, ATT_MAX_LEN = 8192, ATT_TILE = 16, ATT_WHOLE = 512, ATT_MAX_SPLITS = 16, ATT_PART = ATT_D + 4;
 
 template <int HP, int WAVES, bool SPLIT>
 __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
@@ -395,12 +395,16 @@ static void launch_attention(const half_t *qkv, half_t *kcache, half_t *vcache, 
 }
 
 // Parts that the positions are cut into (1: not cut).  One KV head's rows go through one CU at about 60 GB/s, so few heads over
-// a long cache leave the chip idle; the parts cost a second, summing launch.  32 heads, 8 KV heads, one sequence, not cut / cut:
-// 29 / 10 us at position 3000, 17 / 10 at 1500 (two sequences), 6.9 / 8.1 at 384, and only the length of the cache is known here.
+// a long cache leave the chip idle; the parts cost a second, summing launch, and up to ATT_WHOLE positions they gain nothing.
+// Only the length of the cache is known here, so the line lies where the mean over its positions is the same (us not cut / cut,
+// mean of six positions from 6 to 99 % of the cache): one sequence, 32 heads on 8 KV heads 8.0 / 8.9 at a length of 896, 8.5 / 8.9 at 1024,
+// 9.1 / 8.8 at 1152, 12.8 / 9.5 at 2048; 64 on 8 8.6 / 8.9, 9.2 / 8.9 at 1024 and 1152; four sequences of 32 on 8 8.9 / 9.4, 9.5 / 9.4.
+// A head to a workgroup merges for less: 32 on 32 8.2 / 8.7 at 896, 8.8 / 8.6 at 1024; 8 on 8 7.9 / 8.3, 8.4 / 8.3.
+constexpr int ATT_SPLIT_LEN = 1100, ATT_SPLIT_LEN_SINGLE = 1000;
 static int attention_splits(int B, int heads, int kv_heads, int max_len) {
     const int rep = heads / kv_heads, hp = rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1;
     const int64_t groups = (int64_t)B * heads / hp;
-    if (max_len < ATT_SPLIT_LEN || groups > 128 || groups < 1) return 1;
+    if (max_len < (hp == 1 ? ATT_SPLIT_LEN_SINGLE : ATT_SPLIT_LEN) || groups > 128 || groups < 1) return 1;
     const int64_t fill = 256 / groups, longest = bs_cdiv(max_len, 256);       // 256 positions: one tile for each of 16 waves
     const int64_t splits = fill < longest ? fill : longest;
     return splits > ATT_MAX_SPLITS ? ATT_MAX_SPLITS : (int)splits;

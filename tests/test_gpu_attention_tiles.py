@@ -4,11 +4,18 @@ import numpy as np
 import pytest
 import torch
 
+from bitstack_amd import _lib
 from bitstack_amd.utils import inference_utils as IU
 
-pytestmark = pytest.mark.gpu
+
+def test_positions_are_cut_where_the_cache_is_long_and_the_heads_are_few():
+    parts = lambda *shape: _lib.lib().bs_attention_decode_workspace_bytes(*shape) > 0
+    for B, heads, kv, line in ((1, 32, 8, 1100), (4, 32, 8, 1100), (1, 6, 3, 1100), (1, 32, 32, 1000), (1, 8, 8, 1000), (2, 6, 2, 1000)):
+        assert [parts(B, heads, kv, 128, n) for n in (1, 512, line - 1, line, 8192)] == [False, False, False, True, True]
+    assert parts(16, 32, 8, 128, 4096) and not parts(17, 32, 8, 128, 4096)      # more than 128 workgroups fill the chip
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,heads,kv", [(1, 32, 8), (2, 6, 2), (9, 32, 8), (9, 32, 32), (17, 32, 16), (17, 32, 8), (33, 32, 8)])
 def test_attention_at_tile_edges(B, heads, kv):
     d, max_len = 128, 272
@@ -37,7 +44,8 @@ def test_attention_at_tile_edges(B, heads, kv):
         assert (np.abs(got.double().cpu().numpy() - ref) <= bound).all()
 
 
-@pytest.mark.parametrize("B,heads,kv,max_len", [(1, 32, 8, 4096), (1, 32, 8, 1025), (1, 6, 2, 4100), (3, 8, 4, 2050), (2, 16, 16, 1100), (16, 32, 8, 1030)])
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,heads,kv,max_len", [(1, 32, 8, 4096), (1, 32, 8, 1100), (1, 6, 2, 4100), (3, 8, 4, 2050), (2, 16, 16, 1024), (16, 32, 8, 1130)])
 def test_attention_over_split_positions(B, heads, kv, max_len):
     """Few heads over a long cache: the positions in parts (up to 16 of them, most without a position early on)."""
     d = 128
@@ -65,6 +73,7 @@ def test_attention_over_split_positions(B, heads, kv, max_len):
         assert not IU.attention_decode_hip(qkv, kc, vc, cos, sin, torch.tensor([at], device="cuda"), heads, kv).any()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,heads,kv,max_len,at", [(1, 32, 8, 272, 100), (2, 6, 2, 272, 33), (9, 32, 8, 272, 250), (17, 32, 8, 272, 128), (33, 32, 8, 272, 200),
                                                    (1, 32, 8, 2100, 1500), (1, 6, 2, 2100, 1500), (2, 16, 16, 2100, 700)])
 def test_an_infinite_value_stays_infinite(B, heads, kv, max_len, at):

@@ -288,6 +288,52 @@ PyObject *host_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// forward_cat(x [T, N], qweight, u, vt, blocks, qweight, ..) -> y [T, M0 + M1 + ..], or None.  Whether the matrices run as one
+// product is asked first, from sizes alone.
+PyObject *host_forward_cat(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    const int count = (int)(n - 1) / 4;
+    if (n < 5 || (n - 1) % 4 != 0 || count > BS_MAX_GROUP) return PyErr_Format(PyExc_TypeError, "forward_cat takes x and four arguments a matrix");
+    HANDLE_TH_ERRORS
+        const at::Tensor *x = tensor_arg(a[0]);
+        if (!x || !x->is_cuda() || x->dim() != 2 || x->size(0) < 1 || x->size(0) >= INT32_MAX || x->size(1) >= INT32_MAX) Py_RETURN_NONE;
+        const c10::Device dev = x->device();
+        const int T = (int)x->size(0), N = (int)x->size(1);
+        bs_matrix mats[BS_MAX_GROUP] = {};
+        int64_t blocks[BS_MAX_GROUP], K = 0, rows = 0;
+        for (int j = 0; j < count; j++) {
+            const at::Tensor *u = tensor_arg(a[1 + 4 * j + 1]);
+            if (!u || u->dim() != 3) Py_RETURN_NONE;
+            if (!int_arg(a[1 + 4 * j + 3], blocks[j])) return nullptr;
+            if (j == 0) K = u->size(2);
+            if (u->size(2) != K || u->size(1) >= INT32_MAX || K >= INT32_MAX || blocks[j] > u->size(0)) Py_RETURN_NONE;
+            mats[j].I = (int32_t)blocks[j];
+            mats[j].M = (int32_t)u->size(1);
+            rows += mats[j].M;
+        }
+        const int64_t need = bs_forward_cat_workspace_bytes(mats, count, N, (int)K, T);
+        if (need <= 0 || !plain(*x, at::kHalf, dev)) Py_RETURN_NONE;
+        for (int j = 0; j < count; j++) {
+            Matrix m;
+            if (!matrix_args(a + 1 + 4 * j, blocks[j], dev, m) || m.N != N) Py_RETURN_NONE;
+            mats[j].packed = m.q;
+            mats[j].u = m.u;
+            mats[j].vt = m.vt;
+        }
+        const void *xp = x->const_data_ptr();
+        at::Tensor y;
+        const int st = while_others_run([&] {
+            DeviceScope scope(dev);
+            const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+            const Workspace ws = workspace_for(dev.index(), stream, need);
+            y = new_half({T, rows}, dev);
+            std::lock_guard<std::mutex> launching(*ws.launching);
+            return bs_forward_cat(mats, count, N, (int)K, xp, T, y.mutable_data_ptr(), ws.data(), ws.buffer.numel(), stream);
+        });
+        if (st != BS_OK) return raise_status(st, "bs_forward_cat");
+        return THPVariable_Wrap(y);
+    END_HANDLE_TH_ERRORS
+}
+
 // workspace(device index, nbytes) -> the scratch tensor of the device's current stream
 PyObject *host_workspace(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 2) return PyErr_Format(PyExc_TypeError, "workspace takes 2 arguments");
@@ -487,7 +533,7 @@ PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 #define HOST_METHOD(name) {#name, (PyCFunction)(void (*)(void))host_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(unpack), HOST_METHOD(rebuild_from_sign), HOST_METHOD(linear), HOST_METHOD(workspace),
+PyMethodDef methods[] = {HOST_METHOD(forward), HOST_METHOD(rebuild), HOST_METHOD(unpack), HOST_METHOD(rebuild_from_sign), HOST_METHOD(linear), HOST_METHOD(forward_cat), HOST_METHOD(workspace),
                          HOST_METHOD(hold), HOST_METHOD(let_go), HOST_METHOD(argmax), HOST_METHOD(make_steps), HOST_METHOD(run_steps), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native host path over libbitstack_hip.so.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

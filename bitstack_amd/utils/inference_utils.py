@@ -270,28 +270,14 @@ def plainly_called(module):
 def forward_cat_hip(modules, x):
     """[T, M0 + M1 + ..]: what the modules (BitStackLinear, level 5) give for x [T, N], side by side from one product, or None
     where that is not how they are computed (few tokens, a bias, another level, blocks not stacked)."""
+    args = []
     for m in modules:
-        if not plainly_called(m):                # (a call of the module would do more)
+        # (a call of the module would do more, or something else)
+        if not plainly_called(m) or m.fused_level != 5 or m.no_avd or m.bias is not None:
             return None
-        if m.fused_level != 5 or m.no_avd or m.bias is not None or getattr(m, "u", None) is None:
-            return None
-    if x.dtype != torch.float16 or x.dim() != 2 or not x.is_contiguous():
-        return None
-    stacked = [m._stacked() for m in modules]
-    if any(not t.is_contiguous() or t.device != x.device for s in stacked for t in s) or \
-            any(s[1].dtype != torch.float16 or s[2].dtype != torch.float16 or s[2].shape[1:] != (stacked[0][2].shape[1], x.shape[1]) for s in stacked):
-        return None
-    group = MatrixGroup([s + (None,) for s in stacked])
-    T = x.shape[0]
-    L = _lib.lib()
-    need = L.bs_forward_cat_workspace_bytes(group.arr, group.n, group.N, group.K, T)
-    if need <= 0:
-        return None
-    y = torch.empty((T, sum(group.M)), dtype=torch.float16, device=x.device)
-    with torch.cuda.device(x.device), _lib.scratch(x.device, need) as ws:
-        _lib.check(L.bs_forward_cat(group.arr, group.n, group.N, group.K, _lib.ptr(x), T, _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                                    _lib.stream_ptr(x.device)), "bs_forward_cat")
-    return y
+        d = m.__dict__
+        args += (d.get("qweight"), d.get("u"), d.get("vt"), m.w_bit)
+    return _lib.host().forward_cat(x, *args)
 
 
 def attention_decode_hip(qkv, kcache, vcache, cos, sin, pos, heads, kv_heads, out=None):

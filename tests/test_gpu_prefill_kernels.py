@@ -103,6 +103,32 @@ def test_forward_cat_is_the_matrices_side_by_side(T, N, shapes):
     assert IU.forward_cat_hip(mods, x) is None
 
 
+def test_forward_cat_decides_from_sizes_before_it_touches_the_blocks(monkeypatch):
+    def mods(rows, N, blocks=2):
+        out = []
+        for M in rows:
+            q, u, vt, _ = synthetic_layer(M, N, blocks, 1, device="cuda")
+            mod = BitStackLinear(0, N, M, 16, False, False, "cuda", fused_level=5)
+            mod.w_bit, mod.qweight, mod.u, mod.vt = blocks, q, u, vt
+            out.append(mod)
+        return out
+    small, wide = mods((512, 256), 1024), mods((6152, 6152), 8192)              # (wide: 192 MiB of weights, beyond every limit)
+    x, xw = torch.randn(300, 1024, device="cuda").half(), torch.randn(300, 8192, device="cuda").half()
+    want = IU.forward_cat_hip(small, x)
+    monkeypatch.setattr(IU, "MatrixGroup", None)
+    monkeypatch.setattr(BitStackLinear, "_stacked", None)
+    assert IU.forward_cat_hip(small, x[:5].contiguous()) is None and IU.forward_cat_hip(wide, xw) is None
+    assert torch.equal(IU.forward_cat_hip(small, x), want)
+    for bad in (x.float(), x.view(1, 300, 1024), x.t().contiguous().t(), x[:, :1016].contiguous(), x[:0], x.cpu()):
+        assert IU.forward_cat_hip(small, bad) is None
+    for blocks in (0, 3):                                                        # none, and more than are stacked
+        small[0].w_bit = blocks
+        assert IU.forward_cat_hip(small, x) is None
+    small[0].w_bit = 2
+    small[1].vt = small[1].vt.float()
+    assert IU.forward_cat_hip(small, x) is None
+
+
 def test_column_slices_as_operands():
     B, n, heads, kv, d, width = 2, 33, 4, 2, 128, 72
     g = torch.Generator(device="cuda").manual_seed(5)

@@ -300,11 +300,14 @@ extern "C" int bs_silu_mul_f16(const void *gate, const void *up, void *y, int T,
 }
 
 // Several matrices on the same x as one product: rebuilt below each other, so that a narrow one (k, v) does not leave most of
-// the chip idle by itself.  us one by one / as one: 4096 + 1024 + 1024 rows of 4096 columns, 4 blocks: 84 / 61 at 130 tokens,
-// 103 / 72 at 700, 133 / 98 at 1400, 282 / 267 at 6000; 2 x 8192 rows of 3072 (96 MiB): 85 / 70, 111 / 101, 165 / 161, 501 / 491.
-// The limit is where the rebuilt weights no longer stay in the cache between the two launches: 2 x 10752 rows of 3072 (126 MiB)
-// 106 / 84 at 130 tokens but 359 / 363 at 3000, 2 x 12288 of 4096 (192 MiB) 198 / 223 at 700, 2 x 14336 of 4096 230 / 248.
-// With narrow matrices it pays further up: 8192 + 1024 + 1024 rows of 8192 (160 MiB) 207 / 163 at 700, 815 / 820 at 6000.
+// the chip idle by itself.  us one by one / as one, 4 blocks: 4096 + 1024 + 1024 rows of 4096 columns (48 MiB of weights) 84 / 63 at 130
+// tokens, 104 / 75 at 700, 138 / 108 at 1400, 294 / 284 at 6000; 3 x 3072 of 3072 (54 MiB) 85 / 64, 128 / 82, 141 / 116, 375 / 339.
+// The limits are where the rebuilt weights no longer stay in the cache between the two launches; 33 shapes from 10 to 384 MiB
+// were timed at eight token counts.  Up to 96 MiB: 0.97 to 1.58 times as fast (3 x 4096 of 4096, on the limit: 1.34 at 700 tokens, 0.97
+// at 1400, 1.02 to 1.09 from 2000; 2 x 8192 of 3072, too: 1.08, 1.00, 1.00 to 1.04).  Up to 128 MiB few tokens gain (5120 + 2 x 2560 of
+// 5120, 100 MiB: 1.14 at 130, 1.05 at 2000; 2 x 10752 of 3072, 126 MiB: 1.30, 0.99) and many do not (0.98 at 6000).  Beyond, equally wide
+// matrices lose (2 x 14336 of 4096, 224 MiB: 158 / 170 at 130, 399 / 401 at 1400; 2 x 10752, 168 MiB: 0.94 at 1400), narrow ones
+// gain up to 160 MiB (8192 + 1024 + 1024 of 8192, on the limit: 166 / 124 at 130, 330 / 268 at 1400, 715 / 672 at 4500, 864 / 873 at 6000).
 constexpr int64_t CAT_WEIGHT = 96ll << 20, CAT_WEIGHT_FEW = 128ll << 20, CAT_WEIGHT_NARROW = 160ll << 20;   // bytes
 constexpr int CAT_FEW = 2048, CAT_NARROW_TOKENS = 4500;
 static int64_t cat_rows(const bs_matrix *mats, int n, int N, int K, int T) {

@@ -95,7 +95,7 @@ def test_an_allocation_that_fails_is_torchs_out_of_memory_error(little_memory):
         H.linear(x, w, None)                                                      # 4 GiB of output
     for _ in range(3):
         with pytest.raises(torch.OutOfMemoryError):
-            _lib.workspace(dev, 4 << 30)
+            _lib.workspace(dev, before.numel() + (4 << 30))
     assert _lib.workspace(dev, 1).data_ptr() == before.data_ptr()                 # ... and the scratch is what it was
     q, u, vt = torch.zeros(1, (1 << 15) * 16, dtype=torch.uint8, device=dev), torch.zeros(1, 1 << 15, 16, device=dev).half(), torch.zeros(1, 16, 128, device=dev).half()
     with pytest.raises(torch.OutOfMemoryError):
@@ -112,7 +112,7 @@ def test_scratch_can_be_asked_for_while_it_is_being_allocated(little_memory):
     got = []
     torch._C._cuda_attach_out_of_memory_observer(lambda *args: got.append(_lib.workspace(dev, 1).data_ptr()) if not got else None)
     with pytest.raises(torch.OutOfMemoryError):
-        _lib.workspace(dev, 4 << 30)
+        _lib.workspace(dev, have.numel() + (4 << 30))
     assert got == [have.data_ptr()]
 
 

@@ -163,8 +163,8 @@ def e2e_decode_70b(torch, dev, batch=8, prompt_len=2048, new_tokens=128):
             "prefill_linear_tflops": round(per_tok * batch * prompt_len / dt_prefill / 1e12, 1),
             "weight_GB": round(wbytes / 1e9, 2), "blocks_per_linear_mean": round(sum(blocks) / len(blocks), 2),
             "hbm_roofline_tok_s": round(batch * 8e12 / wbytes, 1),
-            "non_path_ops": "the prompt pass runs causal attention through torch SDPA and RoPE through torch ops; "
-                            "the decode steps run the library's own attention kernel",
+            "non_path_ops": "attention, rotation, norms and the MLP's product run on the library's own kernels in the prompt pass and in the "
+                            "decode steps; the embedding lookup and the head's product are torch operations",
             "config": f"80 layers, hidden 8192, inter 28672, 64Q/8KV, vocab 128256, batch {batch}, {prompt_len}-token prompt in one "
                       f"pass, {new_tokens} greedy tokens per sequence, fused step, one HIP-graph replay per step"}
 

@@ -480,7 +480,9 @@ class SyntheticLlamaDecoder:
     @torch.no_grad()
     def prefill(self, prompt: torch.Tensor, all_logits=False, first_layer=0, hidden=None, keep=None):
         """The whole prompt [batch, len] in one pass: every linear sees batch * len tokens (the
-        library's rebuild + dense path), causal attention and RoPE are torch ops, the KV cache
+        library's rebuild + dense path, q/k/v and small gate/up as one product), rotation, causal
+        attention, norms and the SiLU product run on the library's kernels (attention of heads
+        other than 128 wide and caches of another type or layout on torch operations), the KV cache
         is filled for positions 0 .. len - 1, and self.token becomes the greedy token after
         the prompt.  Decode continues from there with step() or step_fused().  With
         all_logits the logits of every position [batch, len, vocab] are returned (perplexity).

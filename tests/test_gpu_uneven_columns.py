@@ -78,3 +78,20 @@ def test_uneven_columns_are_no_further_from_float64_than_the_rebuilt_weight(I, M
             total[name] += float((y.double() - want).norm() / want.norm())
     print(total, flush=True)
     assert total["own"] <= 1.01 * total["rebuilt"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 3, 4])
+def test_groups_on_uneven_columns_are_the_matrices_one_by_one(T):
+    print(f"uneven group T={T}", flush=True)
+    mats = []
+    for j, (I, M) in enumerate(((3, 512), (1, 130), (2, 130))):
+        q, u, vt, x = synthetic_layer(M, 1152, I, T, seed=j, signed_factors=True, device="cuda")
+        mats.append((q, u, vt, None))
+    got = IU.bitstack_forward_group_hip(IU.MatrixGroup(mats), x).float()
+    want = torch.cat([IU.bitstack_forward_hip(*m[:3], x) for m in mats], 1).float()
+    # the same weights; a group may cut the columns into other strips, whose fp32 sums are added in another order
+    assert bool(((got - want).abs() <= want.abs() * 2.0 ** -10 + want.abs().max() * 2.0 ** -13).all())
+    scaled = IU.bitstack_forward_group_hip(IU.MatrixGroup(mats), x, rms_eps=1e-5).double()
+    ref = want.double() * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-5)
+    assert bool(((scaled - ref).abs() <= ref.abs() * 2.0 ** -9 + ref.abs().max() * 2.0 ** -12).all())

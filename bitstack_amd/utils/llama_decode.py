@@ -460,8 +460,9 @@ class SyntheticLlamaDecoder:
     @staticmethod
     def _output(module, x):
         """What the module gives for x, as a tensor that may be written over: a copy where somebody else may hold it."""
+        plain = plainly_called(module)                                    # (before the call: a hook may take itself off in it)
         y = module(x)
-        return y if plainly_called(module) else y.clone(memory_format=torch.contiguous_format)
+        return y if plain else y.clone(memory_format=torch.contiguous_format)
 
     def _sum_norm(self, x, add, weight):
         """(x + add, its RMSNorm); the sum takes the place of `add`."""

@@ -54,6 +54,18 @@ def test_recorded_outputs_stay_what_the_modules_computed(hidden, batch, heads, n
     assert rel(dec.logits, plain.logits) < 2e-3 and rel(dec.kcache, plain.kcache) < 2e-3
 
 
+def test_a_hook_that_takes_itself_off_keeps_its_tensor():
+    dec, seen, handles = decoder(512, 2, 4, 7), [], {}
+
+    def once(mod, args, out):
+        seen.append((out, out.clone()))
+        handles[mod].remove()
+    for m in linears(dec):
+        handles[m] = m.register_forward_hook(once)
+    dec.prefill(torch.arange(14, device="cuda").view(2, 7))
+    assert len(seen) == len(linears(dec)) and all(torch.equal(a, b) for a, b in seen)
+
+
 def test_a_hook_may_return_another_tensor():
     dec, plain = decoder(512, 2, 4, 12), decoder(512, 2, 4, 12)
     prompt = torch.arange(24, device="cuda").view(2, 12)

@@ -389,17 +389,18 @@ class SyntheticLlamaDecoder:
             return self._steps[1]
         s, B, dev = self.s, self.batch, self._xa.device
         d, max_len = s.head_dim, self.kcache.shape[-2]
-
-        def need(t, ok, what):
+        for name, shape in (("kcache", (B, s.kv_heads, max_len, d)), ("vcache", (B, s.kv_heads, max_len, d)), ("cos", (max_len, d // 2)),
+                            ("sin", (max_len, d // 2)), ("pos", ())):
+            t = getattr(self, name)
+            if name == "pos":
+                ok = t.numel() == 1 and t.dtype == torch.int64
+            elif len(shape) == 4:                                          # a layer is contiguous, the layers may lie apart
+                ok = t.dim() == 5 and t.shape[0] >= s.layers and t.shape[1:] == shape and t.dtype == torch.float16 and t[0].is_contiguous()
+            else:
+                ok = t.shape == shape and t.dtype == torch.float16 and t.is_contiguous()
             if not ok or t.device != dev:
-                raise ValueError(f"the decode step needs {what} on {dev}, got {t.dtype} {tuple(t.shape)} {t.stride()} on {t.device}")
-
-        for t in (self.kcache, self.vcache):
-            need(t, t.dim() == 5 and t.shape[0] >= s.layers and tuple(t.shape[1:]) == (B, s.kv_heads, max_len, d)
-                 and t.dtype == torch.float16 and t[0].is_contiguous(), f"fp16 caches [layers, {B}, {s.kv_heads}, {max_len}, {d}], a layer contiguous,")
-        for t in (self.cos, self.sin):
-            need(t, tuple(t.shape) == (max_len, d // 2) and t.dtype == torch.float16 and t.is_contiguous(), f"a contiguous fp16 table {(max_len, d // 2)}")
-        need(self.pos, self.pos.numel() == 1 and self.pos.dtype == torch.int64, "one int64 position")
+                raise ValueError(f"the decode step cannot take this {name} ({'one int64' if name == 'pos' else f'fp16 {shape}, contiguous'} on {dev} "
+                                 f"is needed): {t.dtype} {tuple(t.shape)}, strides {t.stride()}, on {t.device}")
         xa, xb, qkv, ctx, act = (t.data_ptr() for t in (self._xa, self._xb, self._qkv, self._ctx, self._act))
         kcache, vcache, cos, sin, pos, norm = (t.data_ptr() for t in held)
         klayer, vlayer = 2 * self.kcache.stride(0), 2 * self.vcache.stride(0)     # bytes from a layer's cache to the next

@@ -165,12 +165,20 @@ def bitstack_forward_group_hip(group: MatrixGroup, x, epilogue=_lib.EPI_NONE, re
     return y
 
 
+def _norm_weight(weight, H):
+    if weight.numel() != H:
+        raise ValueError(f"a norm of {H} columns needs as many weights, got {tuple(weight.shape)}")
+    return _f16c(weight)
+
+
 def rmsnorm_hip(x, weight, eps, out=None):
     """weight * fp16(x * rsqrt(mean(x^2) + eps)) over the last dimension."""
     dev = _lib.require_gpu(x, weight, out)
     H = x.shape[-1]
-    x2, weight = _f16c(x).view(-1, H), _f16c(weight)
+    x2, weight = _f16c(x).view(-1, H), _norm_weight(weight, H)
     y = out if out is not None else torch.empty_like(x2)
+    if y.dtype != torch.float16 or not y.is_contiguous() or y.numel() != x2.numel():
+        raise ValueError("out must be a contiguous fp16 tensor of x's size")
     with torch.cuda.device(dev):
         _lib.check(_lib.lib().bs_rmsnorm_f16(_lib.ptr(x2), _lib.ptr(weight), _lib.ptr(y), x2.shape[0], H, float(eps),
                                              _lib.stream_ptr(dev)), "bs_rmsnorm_f16")
@@ -186,7 +194,7 @@ def add_rmsnorm_hip(x, add, weight, eps):
         return x, rmsnorm_hip(x, weight, eps)
     if add.dtype != torch.float16 or not add.is_contiguous() or add.shape != x.shape:
         raise ValueError("add must be a contiguous fp16 tensor of x's shape")
-    x2, weight = _f16c(x).view(-1, H), _f16c(weight)
+    x2, weight = _f16c(x).view(-1, H), _norm_weight(weight, H)
     y = torch.empty_like(x2)
     with torch.cuda.device(dev):
         _lib.check(_lib.lib().bs_add_rmsnorm_f16(_lib.ptr(x2), _lib.ptr(add), _lib.ptr(add), _lib.ptr(weight), _lib.ptr(y), x2.shape[0], H,

@@ -58,6 +58,15 @@ def test_add_rmsnorm(T, H):
     assert torch.equal(y, IU.rmsnorm_hip(want, w, 1e-5))
 
 
+def test_norms_refuse_weights_and_outputs_of_another_size():
+    x, w = torch.zeros(3, 512, device="cuda").half(), torch.ones(512, device="cuda").half()
+    for call in (lambda: IU.rmsnorm_hip(x, w[:256], 1e-5), lambda: IU.add_rmsnorm_hip(x, x.clone(), w[:8], 1e-5),
+                 lambda: IU.rmsnorm_hip(x, w, 1e-5, out=x[:2]), lambda: IU.rmsnorm_hip(x, w, 1e-5, out=torch.zeros(3, 512, device="cuda"))):
+        with pytest.raises(ValueError):
+            call()
+    assert IU.rmsnorm_hip(x, w.view(1, 512), 1e-5).shape == x.shape
+
+
 @pytest.mark.parametrize("B,n,heads,kv,max_len", [(1, 1, 4, 1, 1), (2, 15, 8, 2, 20), (1, 16, 6, 3, 16), (3, 17, 5, 5, 40), (1, 31, 32, 8, 31),
                                                   (2, 32, 8, 8, 33), (1, 33, 12, 4, 64), (2, 64, 4, 2, 64), (1, 65, 4, 4, 70), (1, 517, 8, 2, 600)])
 def test_attention_prefill(B, n, heads, kv, max_len):

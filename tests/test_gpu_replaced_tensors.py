@@ -70,7 +70,7 @@ def test_what_the_step_cannot_read_is_refused():
     for name, t, error in (("kcache", dec.kcache.view(torch.int16), ValueError), ("vcache", dec.vcache[:, :, :, :16], ValueError),
                            ("vcache", dec.vcache[:1], ValueError), ("cos", dec.cos[:16], ValueError), ("sin", dec.sin.float(), ValueError),
                            ("pos", torch.zeros(2, dtype=torch.long, device="cuda"), ValueError), ("pos", dec.pos.int(), ValueError),
-                           ("final_norm", dec.final_norm.float(), TypeError)):
+                           ("final_norm", dec.final_norm.float(), TypeError), ("final_norm", dec.final_norm[:256], ValueError)):
         good = getattr(dec, name)
         setattr(dec, name, t)
         with pytest.raises(error):

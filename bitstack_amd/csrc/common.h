@@ -89,10 +89,16 @@ int bs_launch_gemv_group(int n, const uint8_t *const *packed, const half_t *cons
                          int64_t workspace_bytes, hipStream_t s);
 // strip kernel (strip.hip): partial sums part[strip, t, m] of x . w^T with w rebuilt in registers
 int bs_strip_partials(int I, int M, int N, int K, int T);
+long bs_strip_steps(int I, int M, int N, int T);
 int bs_strip_kernel_choice(int I, int M, int N, int K, int T);
 int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt,
                           const int *I, const int *M, float *const *part, float *ssq, const half_t *x,
                           int N, int K, int T, hipStream_t s);
+// tile kernel (tile.hip): the same partial sums for up to 48 tokens at rank 16, 32 x 32 outputs per matrix instruction; groups[j] column
+// groups (partial sums per output) of matrix j where it takes them
+bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
+int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
+                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s);
 // panel kernel (panel.hip): the same partial sums for up to 128 tokens, sign tiles decoded into LDS and
 // multiplied on the matrix cores at once; bs_panel_partials = column groups (0: the shape is not taken)
 constexpr int BS_PANEL_MAX_T = 128;

@@ -808,7 +808,12 @@ int group_path(const int *I, const int *M, int n, int N, int K, int T) {
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group
     for (int j = 0; j < n; j++) total += (int64_t)bs_strip_partials(I[j], M[j], N, K, T) * T * M[j];
-    return total;
+    // the tile kernel's partial sums: room for either, the choice also depends on how u is aligned
+    int groups[GEMV_MAX_GROUP];
+    if (!bs_tile_partials(I, M, n, N, K, T, groups)) return total;
+    int64_t tile_total = (int64_t)groups[0] * T;
+    for (int j = 0; j < n; j++) tile_total += (int64_t)groups[j] * T * M[j];
+    return total > tile_total ? total : tile_total;
 }
 
 // Strip path: one launch writes part[strip group, t, m] of every matrix; the reduce kernel
@@ -824,10 +829,15 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     r.n_in = N;
     r.eps = eps;
     float *parts[GEMV_MAX_GROUP];
-    // threads per output of the summing kernel, as behind the decode kernels (the strip groups are its slots)
+    // The tile kernel where it takes the matrices; the strip kernels for ranks below 16, very long stacks and u off a 16-byte boundary.
+    int column_groups[GEMV_MAX_GROUP];
+    bool tiles = bs_tile_partials(a.I, a.M, a.n, N, K, T, column_groups);
+    for (int j = 0; j < a.n; j++) tiles = tiles && bs_aligned(a.u[j], 16);
+    // threads per output of the summing kernel, as behind the decode kernels (the column groups are its slots)
     int slots = 0;
     for (int j = 0; j < a.n; j++) {
-        const int groups = bs_strip_partials(a.I[j], a.M[j], N, K, T);
+        if (!tiles) column_groups[j] = bs_strip_partials(a.I[j], a.M[j], N, K, T);
+        const int groups = column_groups[j];
         if (groups > slots) slots = groups;
     }
     const int sl = slots <= FLAT_BATCH ? 1 : slots <= 2 * FLAT_BATCH ? 2 : slots <= 4 * FLAT_BATCH ? 4 : 8;
@@ -835,7 +845,7 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     int ldy = 0, blocks = 0;
     int64_t off = 0;
     for (int j = 0; j < a.n; j++) {
-        const int groups = bs_strip_partials(a.I[j], a.M[j], N, K, T);
+        const int groups = column_groups[j];
         parts[j] = part + off;
         r.m[j] = RedMat{part + off, a.bias[j], groups, a.M[j], 1, ldy, blocks};
         off += (int64_t)groups * T * a.M[j];
@@ -844,8 +854,9 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     }
     r.ssq = input_rms ? part + off : nullptr;
     r.ssq_n = r.m[0].I;
-    const int st = bs_launch_strip_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, input_rms ? part + off : nullptr,
-                                         x, N, K, T, s);
+    float *ssq = input_rms ? part + off : nullptr;
+    const int st = tiles ? bs_launch_tile_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, ssq, x, N, K, T, s)
+                         : bs_launch_strip_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, ssq, x, N, K, T, s);
     if (st != BS_OK) return st;
     if (mode == EPI_SWIGLU) ldy = a.M[0];
     for (int j = a.n; j < GEMV_MAX_GROUP; j++) r.m[j] = r.m[0];

@@ -521,6 +521,7 @@ int launch_wide(const WideMat &m, int grid, size_t lds, const half_t *x, int N, 
 
 struct StripPlan {
     int tt, sg, groups, gx, row_groups, rows_per_wg;
+    long steps;          // of 128 rows x 128 columns on the busiest CU
     size_t lds;
 };
 
@@ -565,6 +566,7 @@ StripPlan make_strip_plan(int I, int M, int N, int T) {
             best_cost = cost;
         }
     }
+    best.steps = best_cost;
     return best;
 }
 
@@ -621,6 +623,9 @@ int bs_strip_kernel_choice(int I, int M, int N, int K, int T) {
     if (T < WIDE_MIN_T) return 1;
     return wide_choice(I, M, N, K, T) == 1 ? 2 : 3;
 }
+
+// Steps (128 rows x 128 columns of all blocks) of the strip kernel on the busiest CU.
+long bs_strip_steps(int I, int M, int N, int T) { return make_strip_plan(I, M, N, T).steps; }
 
 // Partial sums per output (groups of strips) when this path takes the shape, else 0.
 int bs_strip_partials(int I, int M, int N, int K, int T) {

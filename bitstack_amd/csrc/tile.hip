@@ -1,0 +1,622 @@
+// Forward for one to 48 tokens on gfx950, rank 16: the weight is rebuilt in registers, 32 x 32 outputs per matrix instruction,
+// and multiplied by x at once; it never goes to memory.
+//
+//   part[cg, t, m] = sum_{n in column group cg} x[t, n] * fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
+//
+// A workgroup is 8 waves side by side: wave w owns 32 NP columns (NP = 4: 1024 columns per workgroup, 2: 512, 1: 256) and keeps what
+// belongs to them in registers - the vt fragments of ALL blocks and the x fragments - while tiles of 32 rows pass by.  Per tile the
+// sign rows (whole 128 or 64-byte runs of a line, each loaded once) and u rows of all blocks are fetched by all waves together into a ring in LDS.
+// Per block a wave runs NP v_mfma_f32_32x32x16_f16, D[column, row]: rank 16 is exactly their depth, so an output costs half the
+// matrix time of a 16x16x16 product, and a lane gets 16 consecutive columns of one row.  The sum over the blocks is kept divided by
+// the current block's sign: between two blocks it changes sign where they differ, which is one v_xor_b32 per output with a mask from a
+// table in LDS (four masks per nibble of the two sign words' difference), and the matrix instruction adds the next block's product.
+// Behind the last block the lane's columns, rounded to fp16 as a stored weight is, become B operands of y[token, row] += x . w
+// (v_mfma_f32_16x16x32_f16).  The waves' y tiles (same rows, other columns) meet in LDS, double buffered, and are added up in wave
+// order while the next tile is rebuilt: one barrier per tile, and scratch holds one partial per 256 NP columns.
+//
+// What bounds it: the issue of a wave's instructions.  Simple VALU instructions (v_xor_b32, v_and_b32, v_lshrrev_b32, fp32 add, mul and FMA on
+// three registers) of two waves run side by side on a SIMD, 1.0 ns each; v_fma_mix_f32, v_and_or_b32, v_bfe, v_alignbit, conversions and whatever
+// has a scalar operand take 1.8 ns, and a single wave issues one instruction in 2 ns whatever it is.  A step (1024 signs: 16 v_xor, 5 for the
+// table addresses, 4 lookups, one product) takes 45 ns per SIMD with two waves and 40 with four; with the signs as fp16 in v_fma_mix 46 and 42.
+// About 1300 cycles per tile and wave (barrier, hand-over, rounding, second product) come on top.  us, strip_forward_kernel / this, with the summing launch:
+// 28672 x 8192, 3 blocks, 8 tokens 90 / 64; 14336 x 4096, 8 blocks 62 / 44; 5000 x 4096, 6 blocks, 37 tokens 29.6 / 25; 4096 x 11008, 4
+// blocks, one token 24.8 / 23.
+#include "common.h"
+#include "rebuild_shared.h"
+
+#include <type_traits>
+#include <utility>
+
+namespace {
+
+constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4;
+constexpr int TL_TABLE = 256;                       // bytes: the table of sign masks at the start of LDS
+constexpr int TL_LDS = 160 * 1024;
+
+struct TileMat {
+    const uint8_t *packed;
+    const half_t *u, *vt;
+    float *part;
+    int I, M, np, row_tiles, first_wg, wgs;         // workgroups first_wg + wgs * column group .. + wgs - 1
+};
+struct TileGroup {
+    TileMat m[TL_GROUP];
+    int n;
+    float *ssq;                                     // [column groups of matrix 0][T]: sums of x^2 over the group's columns, or null
+};
+
+__device__ __forceinline__ void tl_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// wait until at most n of this wave's LDS accesses, which run in order, are to come
+template <int n>
+__device__ __forceinline__ void tl_wait_lds() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (n << 8));
+}
+template <class F, int... Is>
+__device__ __forceinline__ void tl_for_impl(F &&f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void tl_for(F &&f) {
+    tl_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+typedef const __attribute__((address_space(3))) char *lds_bytes;
+typedef __attribute__((address_space(3))) char *lds_bytes_rw;
+typedef const __attribute__((address_space(3))) half8_t *lds_half8;
+typedef __attribute__((address_space(3))) half8_t *lds_half8_rw;
+typedef const __attribute__((address_space(3))) uint4_t *lds_uint4;
+typedef __attribute__((address_space(3))) uint4_t *lds_uint4_rw;
+typedef const __attribute__((address_space(3))) uint2_t *lds_uint2;
+typedef const __attribute__((address_space(3))) uint32_t *lds_u32;
+typedef const __attribute__((address_space(3))) uint16_t *lds_u16;
+typedef const __attribute__((address_space(3))) float *lds_f32;
+typedef __attribute__((address_space(3))) float *lds_f32_rw;
+typedef __attribute__((address_space(3))) float4_t *lds_f32x4_rw;
+
+// TT: token tiles of 16.
+template <int TT, int NP>
+struct TileKernel {
+    static constexpr int WC = 32 * NP, CG = WC * TL_WAVES;     // columns per wave, per workgroup
+    static constexpr int SROW = CG / 8;                        // sign bytes of a row in a stage
+    static constexpr int RP = SROW / 16;                       // ... in 16-byte pieces
+    static constexpr int SCH = SROW * TL_ROWS / 1024;          // requests of 1 KB per block: signs; u is one more
+    // what a row's pieces are XOR-ed with in a stage, so that the 32 rows a read takes fall on different banks
+    static __device__ __forceinline__ int swizzle(int r) { return (r * RP / 16) % RP; }
+    // LDS: the table of sign masks (at address 0: the kernel has no other LDS), an area for two y tiles of every wave (and at first for the
+    // vt images), and the ring of stages
+    static constexpr int AREA = 32 * 1024 * TT;
+    static constexpr int stage_bytes(int I) { return I * (SCH + 1) * 1024; }
+    static constexpr int STAGES = 3;                           // the tile in work, the next one, one that is being written
+    // most blocks: LDS, and the registers of the vt fragments
+    static constexpr int max_blocks() {
+        int I = NP == 4 ? (TT == 1 ? 4 : TT == 2 ? 2 : 1) : NP == 2 ? (TT == 1 ? 10 : 8) : 16;
+        while (TL_TABLE + AREA + STAGES * stage_bytes(I) > TL_LDS) I--;
+        return I;
+    }
+
+    // One run of row tiles [rt0, rt0 + len) of column group cg of one matrix.
+    template <int I>
+    static __device__ __forceinline__ void walk(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, const half_t *__restrict__ vt,
+                                                float *__restrict__ part, int M, lds_bytes_rw lds, const half_t *__restrict__ x, int N, int T,
+                                                int cg, int rt0, int len, float *ssq) {
+        constexpr int STAGE = stage_bytes(I);
+        constexpr int CHUNKS = I * (SCH + 1), PER = CHUNKS / TL_WAVES, MORE = CHUNKS % TL_WAVES, MOST = PER + (MORE != 0);
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));                           // (what follows from it is not shared between the block counts: registers)
+        const int lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int row = lane & 31, h = lane >> 5;               // in the rebuild
+        const int lm = lane & 15, g = lane >> 4;                // in the second product
+        const uint32_t row_bytes = (uint32_t)N >> 3;
+        lds_bytes_rw area = lds + TL_TABLE, ring = area + AREA;
+        const int n0 = cg * CG + wave * WC;
+        const int active = min(TL_WAVES, (N - cg * CG) / WC);   // waves whose columns exist (all or none of a wave's)
+        const bool mine = wave < active;
+
+        // ---- requests: chunk c of a tile is 1 KB, signs of block c / SCH first, then the u rows of the blocks --------------
+        // Wave w takes chunks w, w + 8, ...
+        const char *from[MOST];                                  // row 0 of the next tile to be requested
+        uint32_t pitch[MOST], offset[MOST];                      // the lane's piece within a tile
+        auto geometry = [&](int k, int rows) {                   // ... of which `rows` rows exist
+            const int c = min(wave + TL_WAVES * k, CHUNKS - 1);
+            if (c < I * SCH) {
+                const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
+                return (uint32_t)min(r, rows - 1) * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
+            }
+            const int r = lane >> 1;
+            return (uint32_t)min(r, rows - 1) * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
+        };
+#pragma unroll
+        for (int k = 0; k < MOST; k++) {
+            const int c = min(wave + TL_WAVES * k, CHUNKS - 1);
+            const bool signs = c < I * SCH;
+            from[k] = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
+            pitch[k] = signs ? row_bytes : 32u;
+            from[k] += (int64_t)(rt0 * TL_ROWS) * pitch[k];
+            offset[k] = geometry(k, TL_ROWS);
+        }
+        // A tile's pieces travel through registers: requested three tiles ahead, written to LDS at the end of the tile two ahead of it.
+        int asked = rt0;                                         // the row tile `from` stands at
+        const int last_rt = rt0 + len - 1;
+        uint4_t pieces[MOST], pieces_1[MOST];                    // (pieces_1: only of the run's second tile)
+        auto request_next = [&](uint4_t (&to)[MOST]) {           // (behind the last tile that one is requested again)
+            const int rows = M - asked * TL_ROWS;
+#pragma unroll
+            for (int k = 0; k < MOST; k++)
+                if (k < PER || wave < MORE) to[k] = *reinterpret_cast<const uint4_t *>(from[k] + (rows >= TL_ROWS ? offset[k] : geometry(k, rows)));
+            if (asked < last_rt) {
+                asked++;
+#pragma unroll
+                for (int k = 0; k < MOST; k++) from[k] += pitch[k] * (uint32_t)TL_ROWS;
+            }
+        };
+        auto write_tile = [&](int stage, const uint4_t (&p)[MOST]) {
+            lds_uint4_rw to = (lds_uint4_rw)(ring + stage * STAGE + wave * 1024) + lane;
+#pragma unroll
+            for (int k = 0; k < MOST; k++)
+                if (k < PER || wave < MORE) to[k * (TL_WAVES * 64)] = p[k];
+        };
+#pragma unroll
+        for (int k = 0; k < MOST; k++) pieces[k] = pieces_1[k] = (uint4_t){0, 0, 0, 0};
+        request_next(pieces);
+        if constexpr (NP < 4) request_next(pieces_1);
+
+        // ---- this wave's vt and x fragments -----------------------------------------------------------------------
+        // vt: a lane takes 8 columns x 8 ranks of one block, turns them in registers and leaves them as [column][rank] in the wave's own
+        // part of the area; the fragments are read back from there.  (The columns of a group of eight are XOR-ed with the group's
+        // number: the groups lie a whole turn of the banks apart.)
+        half8_t vf[I][NP];
+        half8_t xf[TT][NP];
+        if (mine) {
+            constexpr int PIECES = WC / 8, BP = 32 / PIECES, PASSES = (I + BP - 1) / BP, IMAGE = WC * 32;   // BP blocks per pass of loads
+            constexpr int ROOM = (AREA / TL_WAVES < 8192 ? AREA / TL_WAVES : 8192), SB = ROOM / IMAGE;      // SB of them fit the image
+            lds_bytes_rw img = area + wave * ROOM;
+            const int piece = lane % PIECES, kh = (lane / PIECES) & 1, bl = lane / (2 * PIECES);
+            const int col = 16 * NP * ((row >> 2) & 1) + 4 * (row >> 3) + (row & 3);
+            half8_t v[PASSES][8];
+#pragma unroll
+            for (int pass = 0; pass < PASSES; pass++) {
+                const half_t *src = vt + ((int64_t)min(pass * BP + bl, I - 1) * 16 + 8 * kh) * N + n0 + 8 * piece;
+#pragma unroll
+                for (int r = 0; r < 8; r++) v[pass][r] = *reinterpret_cast<const half8_t *>(src + (int64_t)r * N);
+            }
+            // x: the columns whose weights lane group g holds when the rows are sorted out for the second product (see there)
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) {
+                const half_t *xr = x + (int64_t)min(tt * 16 + lm, T - 1) * N + n0 + 16 * NP * (g >> 1) + 8 * (g & 1);   // (rows beyond T: outputs nobody stores)
+#pragma unroll
+                for (int p = 0; p < NP; p++) xf[tt][p] = *reinterpret_cast<const half8_t *>(xr + 16 * p);
+            }
+#pragma unroll
+            for (int pass = 0; pass < PASSES; pass++)
+#pragma unroll
+                for (int sub = 0; sub < BP / SB; sub++) {
+                    if (BP == SB || bl / SB == sub) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            half8_t o;
+#pragma unroll
+                            for (int r = 0; r < 8; r++) o[r] = v[pass][r][e];
+                            *(lds_half8_rw)(img + (bl % SB) * IMAGE + (8 * piece + (e ^ (piece & 7))) * 32 + 16 * kh) = o;
+                        }
+                    }
+                    asm volatile("" ::: "memory");   // (a wave's LDS accesses run in order, but the lanes read what others wrote)
+#pragma unroll
+                    for (int b = 0; b < SB; b++)
+                        if (pass * BP + sub * SB + b < I)
+#pragma unroll
+                            for (int p = 0; p < NP; p++)
+                                vf[pass * BP + sub * SB + b][p] = *(lds_half8)(img + b * IMAGE + ((col + 16 * p) ^ (((col + 16 * p) >> 3) & 7)) * 32 + 16 * h);
+                    asm volatile("" ::: "memory");
+                }
+        }
+        write_tile(0, pieces);
+        if constexpr (NP < 4) write_tile(1, pieces_1);
+        request_next(pieces);
+        if (ssq) {          // sums of squares of x over the group's columns
+            lds_f32_rw sums = (lds_f32_rw)area;
+            __syncthreads();                         // (the area holds the vt images)
+            if (mine) {
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) {
+                    float q = 0.f;
+#pragma unroll
+                    for (int p = 0; p < NP; p++)
+#pragma unroll
+                        for (int k = 0; k < 8; k++) q += (float)xf[tt][p][k] * (float)xf[tt][p][k];
+                    q += __shfl_xor(q, 16, 64);
+                    q += __shfl_xor(q, 32, 64);
+                    if (g == 0) sums[wave * (16 * TT) + tt * 16 + lm] = q;
+                }
+            }
+            __syncthreads();
+            if (tid < T) {
+                float q = 0.f;
+                for (int w = 0; w < active; w++) q += sums[w * (16 * TT) + tid];
+                ssq[cg * T + tid] = q;
+            }
+        }
+
+        // ---- y tiles: [buffer][wave][TT token tiles][rows 0-15, 16-31][four tokens: 4][row: 16][token: 4] ----------------------------
+        // Pass tt of a hand-over is one output per thread: this thread's of every wave, added in wave order.  The reads are issued ahead of
+        // where they are added up.
+        constexpr int Y = 16 * TT * TL_ROWS;
+        const int my_t = tid >> 5, my_row = tid & 31;
+        const uint32_t my_out = (uint32_t)(my_t * M + my_row) * 4u;
+        float *const out = part + (int64_t)cg * T * M;
+        // (a wave's two tokens of pass tt)
+        auto takes = [&](int tt) { return 16 * tt + 2 * wave < T; };
+        auto collect = [&](int buf, int tt, float (&v)[TL_WAVES]) {
+            lds_f32 red = (lds_f32)(area) + buf * (TL_WAVES * Y) + tt * 512 + my_row / 16 * 256 + my_t / 4 * 64 + my_row % 16 * 4 + my_t % 4;
+            if (takes(tt)) {
+#pragma unroll
+                for (int w = 0; w < TL_WAVES; w++) v[w] = red[w * Y];
+            }
+        };
+        auto hand_over = [&](int rt, int tt, const float (&v)[TL_WAVES], bool valid) {
+            if (!takes(tt) || !valid) return;
+            float sum = v[0];
+            if (active == TL_WAVES) {
+#pragma unroll
+                for (int w = 1; w < TL_WAVES; w++) sum += v[w];
+            } else {
+#pragma unroll
+                for (int w = 1; w < TL_WAVES; w++)
+                    if (w < active) sum += v[w];
+            }
+            char *const to = reinterpret_cast<char *>(out + ((int64_t)(16 * tt) * M + rt * TL_ROWS));
+            if (16 * tt + my_t < T && rt * TL_ROWS + my_row < M) *reinterpret_cast<float *>(to + my_out) = sum;
+        };
+        // the second product's result: rows 0-15 ([tt][0]) and 16-31 ([tt][1]) of a tile, D[token 4 g + j, row lm] of each
+        float4_t y[TT][2];
+        auto leave = [&](int buf) {
+            lds_f32x4_rw red = (lds_f32x4_rw)(area + (buf * TL_WAVES + wave) * (Y * 4)) + lane;
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                for (int r = 0; r < 2; r++) red[128 * tt + 64 * r] = y[tt][r];
+        };
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++) y[tt][0] = y[tt][1] = (float4_t){0.f, 0.f, 0.f, 0.f};
+
+        // ---- the rebuild ------------------------------------------------------------------------------------------------
+        // Steps s = NP i + p: ahead of block i (i = I: behind the last) the sums of patch p change sign where blocks i - 1 and i differ, then the
+        // matrix instruction adds block i's product: the sum so far is kept divided by the block's sign, and a change of sign is exact, so
+        // this is the fp32 sum over the blocks for one operation per sign.  The table turns a nibble of the two sign words' difference
+        // into four masks; they are looked up LOOK steps ahead, u rows and sign words SETS - 1 blocks ahead, across the end of a tile: the barrier
+        // that opens tile n also says that tile n + 1 is in LDS.  The fences keep the compiler from moving the lookups of many steps
+        // ahead, for which there are no registers.
+        constexpr int STEPS = (I + 1) * NP, SETS = NP == 4 ? 2 : NP == 2 ? 3 : 4, LOOK = TT == 1 && (NP == 1 || (NP == 2 && I <= 8)) ? 2 : 1;
+        const int mine_at = wave * (WC / 8) + h * (WC / 16);     // byte of a sign row: this lane's WC / 2 columns
+        const int sread = row * SROW + ((mine_at >> 4) ^ swizzle(row)) * 16 + (mine_at & 15);
+        const int uread = I * SCH * 1024 + row * 32 + 16 * (h ^ ((row >> 4) & 1));
+        float16_t acc[NP];
+        uint4_t mask[LOOK + 1][4];
+        half8_t uf[SETS];
+        constexpr int WORDS = NP == 4 ? 2 : 1;
+        uint32_t sw[SETS][WORDS], flip[WORDS], flip4[WORDS];
+        auto fetch = [&](lds_bytes st, auto ic) {
+            constexpr int i = decltype(ic)::value;
+            uf[i % SETS] = *(lds_half8)(st + uread + i * 1024);
+            lds_bytes at = st + sread + i * (SCH * 1024);
+            if constexpr (NP == 4) {
+                const uint2_t two = *(lds_uint2)at;
+                sw[i % SETS][0] = two[0];
+                sw[i % SETS][1] = two[1];
+            } else
+                sw[i % SETS][0] = NP == 2 ? *(lds_u32)at : *(lds_u16)at;
+        };
+        auto look_up = [&](auto sc) {
+            constexpr int s = decltype(sc)::value, i = s / NP, p = s % NP;
+            if constexpr (s < STEPS) {
+                constexpr int word = p / 2;
+                if constexpr (p == 0) {
+#pragma unroll
+                    for (int k = 0; k < WORDS; k++) {
+                        flip[k] = i < I ? sw[(i + SETS - 1) % SETS][k] ^ sw[i % SETS][k] : ~sw[(i + SETS - 1) % SETS][k];
+                        flip4[k] = flip[k] << 4;
+                        asm("" : "+v"(flip4[k]));
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    // nibble q of the patch: byte 2 p + q / 2, its upper half first; times 16 it is the place of its masks
+                    const uint32_t at = ((q & 1 ? flip4[word] : flip[word]) >> (8 * (2 * (p % 2) + (q >> 1)))) & 0xF0u;
+                    mask[s % (LOOK + 1)][q] = *(lds_uint4)(uintptr_t)at;
+                }
+            }
+        };
+        auto fetch_first = [&](lds_bytes st) { tl_for<(I < SETS ? I : SETS)>([&](auto ic) { fetch(st, ic); }); };
+        auto first_block = [&]() {
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][p], uf[0], (float16_t){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            tl_for<LOOK>([&](auto k) { look_up(std::integral_constant<int, NP + decltype(k)::value>{}); });
+        };
+        tl_wait_lds<0>();
+        tl_barrier();                                // the first tile is here, everybody is done with the images
+        if (mine) {
+            fetch_first(ring);
+            first_block();
+        }
+        if constexpr (NP == 4) {                     // (no registers for two tiles' pieces)
+            write_tile(1, pieces);
+            request_next(pieces);
+        }
+        int stage = 0;
+#pragma clang loop unroll(disable)
+        for (int n = 0; n < len; n++) {
+            __builtin_amdgcn_s_setprio(0);
+            if (mine)
+                tl_wait_lds<4>();                    // (its last LDS writes lie a step's four lookups or more back)
+            else
+                tl_wait_lds<0>();
+            tl_barrier();                            // tile n + 1 and the y tiles of n - 2 are in LDS, the stage of n - 1 is free
+            const int free_stage = stage == 0 ? STAGES - 1 : stage - 1;
+            lds_bytes st = ring + stage * STAGE;
+            if (++stage == STAGES) stage = 0;
+            lds_bytes st_next = ring + stage * STAGE;
+            // Three tiles are in work: tile n is rebuilt, the product of n - 1 is on its way to LDS, and the waves' results of n - 2 are
+            // added up between the first steps.
+            const int before = (n & 1) ^ 1, oldest = n & 1;
+            auto pass_on = [&]() {                   // tile n + 2 into LDS, tile n + 3 requested
+                write_tile(free_stage, pieces);
+                request_next(pieces);
+            };
+            if constexpr (NP == 4) pass_on();        // (at the end it would take eight registers more than there are)
+            float v[TL_WAVES];
+            if (mine) {
+                tl_for<STEPS - NP>([&](auto sc) {
+                    constexpr int k = decltype(sc)::value, s = k + NP, i = s / NP, p = s % NP;
+                    // (of the two waves of a SIMD the older one goes first; so that both come to the barrier together, the younger one does in the
+                    // second half)
+                    if constexpr (k == (STEPS - NP) / 2)
+                        if (wave >= TL_WAVES / 2) __builtin_amdgcn_s_setprio(1);
+                    look_up(std::integral_constant<int, s + LOOK>{});
+                    if constexpr (p == 0 && i < I && i + SETS - 1 < I) fetch(st, std::integral_constant<int, i + SETS - 1>{});
+                    if constexpr (s == STEPS - NP) fetch_first(st_next);
+                    if constexpr (k % 2 == 0 && k / 2 >= 1 && k / 2 <= TT) hand_over(rt0 + n - 2, k / 2 - 1, v, n >= 2);
+                    if constexpr (k % 2 == 0 && k / 2 < TT) collect(oldest, k / 2, v);
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            const float sum = acc[p][4 * q + j];
+                            const uint32_t m = mask[s % (LOOK + 1)][q][j];
+                            acc[p][4 * q + j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
+                        }
+                    if constexpr (i < I)
+                        acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
+                    asm volatile("" : "+v"(acc[p]));
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (k == (STEPS - NP > 1 ? 1 : 0)) leave(before);
+                });
+                // (the passes for which there were not enough steps)
+                constexpr int COLLECTED = (STEPS - NP + 1) / 2 < TT ? (STEPS - NP + 1) / 2 : TT, HANDED = (STEPS - NP - 1) / 2 < TT ? (STEPS - NP - 1) / 2 : TT;
+                if constexpr (HANDED < COLLECTED) hand_over(rt0 + n - 2, COLLECTED - 1, v, n >= 2);
+                tl_for<TT - COLLECTED>([&](auto k) {
+                    collect(oldest, COLLECTED + decltype(k)::value, v);
+                    hand_over(rt0 + n - 2, COLLECTED + decltype(k)::value, v, n >= 2);
+                });
+                if constexpr (NP < 4) pass_on();
+                // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
+                // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
+                // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
+                // v_mfma_f32_16x16x32_f16.
+                half8_t wf[NP][2];
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    uint4_t lo, hi;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
+                        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                        lo[k] = r[0];
+                        hi[k] = r[1];
+                    }
+                    wf[p][0] = __builtin_bit_cast(half8_t, lo);
+                    wf[p][1] = __builtin_bit_cast(half8_t, hi);
+                }
+                first_block();                       // of tile n + 1
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                    for (int r = 0; r < 2; r++) {
+                        y[tt][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
+                    }
+            } else {
+                if constexpr (NP < 4) pass_on();
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) {
+                    collect(oldest, tt, v);
+                    hand_over(rt0 + n - 2, tt, v, n >= 2);
+                }
+            }
+        }
+        // the last two tiles
+        if (len > 2) tl_barrier();                   // (everybody has collected the tile whose place this is)
+        if (mine) leave((len & 1) ^ 1);
+        tl_wait_lds<0>();
+        tl_barrier();
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            if (len + n < 2) continue;
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) {
+                float v[TL_WAVES];
+                collect((len + n) & 1, tt, v);
+                hand_over(rt0 + len + n - 2, tt, v, true);
+            }
+        }
+    }
+};
+
+template <int TT>
+__global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const TileGroup grp_, const half_t *__restrict__ x, int N, int T) {
+    extern __shared__ __attribute__((aligned(1024))) char tl_lds[];
+    lds_bytes_rw lds = (lds_bytes_rw)tl_lds;
+    // nibble v, column j of its four (first in the top bit): the sign bit of an fp32 where the bit is set (visible behind walk's first barrier)
+    if (threadIdx.x < 64) ((__attribute__((address_space(3))) uint32_t *)lds)[threadIdx.x] = ((threadIdx.x >> 2) >> (3 - (threadIdx.x & 3))) & 1 ? 0x80000000u : 0u;
+    // (the argument block itself, so that a matrix is picked by its number with scalar loads)
+    typedef const __attribute__((address_space(4))) TileGroup *kernarg_group;
+    const kernarg_group grp = (kernarg_group)__builtin_amdgcn_kernarg_segment_ptr();
+    // Workgroups are dealt round-robin to the 8 XCDs: each XCD takes a contiguous run of (matrix, column group, run of row tiles), so that
+    // workgroups with the same slices of x and vt, and column groups that share lines of sign bytes, meet in one L2.
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, base = nb >> 3, rem = nb & 7;
+    const int v = xcd * base + min(xcd, rem) + loc;
+    int j = 0;
+    while (j + 1 < grp->n && v >= grp->m[j + 1].first_wg) j++;
+    const int r = v - grp->m[j].first_wg, wgs = grp->m[j].wgs, tiles = grp->m[j].row_tiles, cg = r / wgs, run = r - cg * wgs;
+    const int rt = (int)((int64_t)tiles * run / wgs), len = (int)((int64_t)tiles * (run + 1) / wgs) - rt;
+    float *ssq = j == 0 && run == 0 ? grp->ssq : nullptr;
+    auto walk = [&](auto np, auto blocks) {
+        typedef TileKernel<TT, decltype(np)::value> TK;
+        if constexpr (decltype(blocks)::value <= TK::max_blocks())
+            TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].M, lds, x, N, T, cg, rt, len, ssq);
+    };
+    // (the narrower widths serve what the wider ones cannot hold, and short runs)
+    switch (grp->m[j].np * 32 + grp->m[j].I) {
+#define TL_CASE(np, k) \
+    case np * 32 + k: walk(std::integral_constant<int, np>{}, std::integral_constant<int, k>{}); break;
+        TL_CASE(4, 1) TL_CASE(4, 2) TL_CASE(4, 3) TL_CASE(4, 4)
+        TL_CASE(2, 1) TL_CASE(2, 2) TL_CASE(2, 3) TL_CASE(2, 4) TL_CASE(2, 5) TL_CASE(2, 6) TL_CASE(2, 7) TL_CASE(2, 8) TL_CASE(2, 9) TL_CASE(2, 10)
+        TL_CASE(1, 1) TL_CASE(1, 2) TL_CASE(1, 3) TL_CASE(1, 4) TL_CASE(1, 5) TL_CASE(1, 6) TL_CASE(1, 7) TL_CASE(1, 8)
+        TL_CASE(1, 9) TL_CASE(1, 10) TL_CASE(1, 11) TL_CASE(1, 12) TL_CASE(1, 13) TL_CASE(1, 14) TL_CASE(1, 15) TL_CASE(1, 16)
+#undef TL_CASE
+    }
+}
+
+// Per matrix the width of its column groups (256 np columns) and how many workgroups share the row tiles of one.  The estimate behind it
+// (cycles): a tile costs 1300 + 250 per block and np (with one patch per wave, a chain of mask, product, mask, 420 per block), a
+// workgroup's start 2000 + 560 per block and np.
+struct TilePlan {
+    int grid;                                       // 0: not taken
+    double cost;
+    int np[TL_GROUP], groups[TL_GROUP], wgs[TL_GROUP];
+};
+int tile_limit(int np, int T) {
+    const int tt = (T + 15) / 16;
+    return tt == 1 ? (np == 4 ? TileKernel<1, 4>::max_blocks() : np == 2 ? TileKernel<1, 2>::max_blocks() : TileKernel<1, 1>::max_blocks())
+           : tt == 2 ? (np == 4 ? TileKernel<2, 4>::max_blocks() : np == 2 ? TileKernel<2, 2>::max_blocks() : TileKernel<2, 1>::max_blocks())
+                     : (np == 4 ? TileKernel<3, 4>::max_blocks() : np == 2 ? TileKernel<3, 2>::max_blocks() : TileKernel<3, 1>::max_blocks());
+}
+double tile_cost(int np, int I) { return 1300 + (np == 1 ? 420 : 250 * np) * I; }
+double start_cost(int np, int I) { return 2000 + 560 * np * I; }
+// the plan in which every matrix takes the widest groups up to `widest` that its blocks allow
+TilePlan tile_plan_up_to(int widest, const int *I, const int *M, int n, int N, int T) {
+    TilePlan p;
+    p.grid = 0;
+    double work[TL_GROUP], all = 0;
+    int tiles[TL_GROUP];
+    for (int j = 0; j < n; j++) {
+        p.np[j] = widest;
+        while (p.np[j] > 1 && I[j] > tile_limit(p.np[j], T)) p.np[j] >>= 1;
+        if (I[j] > tile_limit(p.np[j], T)) return p;
+        p.groups[j] = (int)bs_cdiv(N, 256 * p.np[j]);
+        tiles[j] = (int)bs_cdiv(M[j], TL_ROWS);
+        work[j] = p.groups[j] * (tiles[j] * tile_cost(p.np[j], I[j]) + start_cost(p.np[j], I[j]));
+        all += work[j];
+    }
+    // workgroups (one per CU) in proportion to the work, the rest to whoever takes longest
+    auto run = [&](int j) { return bs_cdiv(tiles[j], p.wgs[j]) * tile_cost(p.np[j], I[j]) + start_cost(p.np[j], I[j]); };
+    int grid = 0;
+    for (int j = 0; j < n; j++) {
+        const int w = (int)(256 * work[j] / all / p.groups[j]);
+        p.wgs[j] = w < 1 ? 1 : w > tiles[j] ? tiles[j] : w;
+        grid += p.wgs[j] * p.groups[j];
+    }
+    int worst;
+    while (true) {
+        worst = 0;
+        for (int j = 1; j < n; j++)
+            if (run(j) > run(worst)) worst = j;
+        if (grid + p.groups[worst] > 256 || p.wgs[worst] >= tiles[worst]) break;
+        p.wgs[worst]++;
+        grid += p.groups[worst];
+    }
+    p.grid = grid;
+    p.cost = run(worst) * bs_cdiv(grid, 256);
+    return p;
+}
+TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
+    TilePlan best;
+    best.grid = 0;
+    for (int widest = 4; widest >= 1; widest >>= 1) {
+        const TilePlan p = tile_plan_up_to(widest, I, M, n, N, T);
+        if (p.grid != 0 && (best.grid == 0 || p.cost < best.cost)) best = p;
+    }
+    // Against the strip kernel's steps (128 rows x 128 columns on the busiest CU).  With one patch per wave it is the better one where its
+    // rows and strips happen to fill the chip; us strip / this: 7286 x 1024, 11 blocks (2 steps, runs of 4) 18.6 / 21.2, 3328 x 1664, 16 (2, 3) 20.3 / 23.7,
+    // 3366 x 2688, 11 (4, 5) 25.6 / 23.1, 2440 x 1536, 14 (2, 2) 20.4 / 17.0, 20191 x 256, 11 (6, 3) 29.4 / 15.5.  And where either does one tile or step of
+    // one or two blocks: the hand-over between the waves is half a us (896 x 2176, 1 block 6.8 / 7.5; 643 x 896, 2 blocks 8.4 / 8.9; from 3 blocks
+    // on level or ahead).
+    if (n == 1 && best.grid != 0) {
+        const int64_t tiles = bs_cdiv(bs_cdiv(M[0], TL_ROWS), best.wgs[0]);
+        const long steps = best.np[0] == 1 || I[0] <= 2 ? bs_strip_steps(I[0], M[0], N, T) : 0;
+        if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || (I[0] <= 2 && tiles == 1 && steps == 1)) best.grid = 0;
+    }
+    return best;
+}
+
+template <int TT>
+int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, hipStream_t s) {
+    size_t lds = 0;
+    for (int j = 0; j < grp.n; j++) {
+        const int np = grp.m[j].np, I = grp.m[j].I;
+        const size_t b = TL_TABLE + TileKernel<TT, 1>::AREA + 3 * (size_t)(np == 4 ? TileKernel<TT, 4>::stage_bytes(I) : np == 2 ? TileKernel<TT, 2>::stage_bytes(I) : TileKernel<TT, 1>::stage_bytes(I));
+        if (b > lds) lds = b;
+    }
+    static bs_lds_grant granted[BS_MAX_DEVICES];
+    const int st = bs_allow_lds((const void *)tile_forward_kernel<TT>, lds, granted);
+    if (st != BS_OK) return st;
+    tile_forward_kernel<TT><<<grid, 64 * TL_WAVES, lds, s>>>(grp, x, N, T);
+    BS_LAUNCH_CHECK();
+    return BS_OK;
+}
+
+TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
+    TilePlan none;
+    none.grid = 0;
+    if (n < 1 || n > TL_GROUP || K != 16 || T < 1 || T > 48 || N < SF_COLS || N % SF_COLS != 0) return none;
+    for (int j = 0; j < n; j++)
+        // a block's sign and u rows, and 16 tokens of partial sums, lie within 32-bit byte offsets
+        if (I[j] < 1 || M[j] < 1 || (int64_t)M[j] * (N >> 3) >= ((int64_t)1 << 32) || (int64_t)M[j] * 64 >= ((int64_t)1 << 32)) return none;
+    return bs_cdiv(N, 256) <= 1024 ? make_tile_plan(I, M, n, N, T) : none;
+}
+
+}  // namespace
+
+// Column groups (partial sums per output) of every matrix, if this kernel takes them.
+bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups) {
+    const TilePlan p = checked_plan(I, M, n, N, K, T);
+    for (int j = 0; p.grid != 0 && j < n; j++) groups[j] = p.groups[j];
+    return p.grid != 0;
+}
+
+int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
+                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s) {
+    const TilePlan p = checked_plan(I, M, n, N, K, T);
+    if (p.grid == 0 || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
+    TileGroup grp;
+    grp.n = n;
+    grp.ssq = ssq;
+    int first = 0;
+    for (int j = 0; j < n; j++) {
+        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], 16)) return BS_ERR_SHAPE;
+        grp.m[j] = TileMat{packed[j], u[j], vt[j], part[j], I[j], M[j], p.np[j], (int)bs_cdiv(M[j], TL_ROWS), first, p.wgs[j]};
+        first += p.wgs[j] * p.groups[j];
+    }
+    for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
+    return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, s) : launch_tile<3>(grp, p.grid, x, N, T, s);
+}

@@ -1,0 +1,117 @@
+"""The tile kernel (rank 16, one to 48 tokens) at the edges of its tiles, against the float64 oracle and against the strip kernel, which
+takes the same call when u lies 8 bytes off a 16-byte boundary."""
+import ctypes
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from bitstack_amd import _lib
+from bitstack_amd.utils import inference_utils as IU
+from bitstack_amd.utils.synthetic import synthetic_layer
+from oracle import c_oracle as C
+
+CSRC = os.path.join(os.path.dirname(_lib.LIB_PATH))
+# (blocks, out features, in features, tokens): rows about whole tiles of 32, columns that leave waves without any, both sides of the block
+# limits of 1024, 512 and 256 columns per workgroup, one, two and three token tiles
+CASES = [(1, 1, 128, 5), (1, 32, 128, 16), (2, 33, 256, 17), (3, 31, 384, 48), (1, 64, 640, 1), (4, 100, 640, 33), (5, 65, 1152, 8), (2, 8200, 1152, 8),
+         (3, 8224, 2176, 7), (4, 8191, 1024, 6), (1, 16400, 640, 40), (2, 8193, 1664, 32), (7, 130, 896, 16), (8, 200, 512, 9), (8, 97, 640, 33),
+         (9, 256, 768, 8), (10, 70, 640, 47), (11, 70, 640, 48), (13, 300, 384, 5), (16, 129, 1024, 24), (16, 65, 1280, 1), (17, 64, 512, 8)]
+
+
+def _args(I, M, N, T, off):
+    """Inputs on the GPU; `off`: u starts 8 bytes off a 16-byte boundary."""
+    q, u, vt, x = synthetic_layer(M, N, I, T, seed=I + N + T, signed_factors=True)
+    u = (u * 20).half()
+    want = C.forward_f64(q.numpy(), u.numpy(), vt.numpy(), x.numpy())
+    q, u, vt, x = (t.cuda() for t in (q, u, vt, x))
+    if off:
+        room = torch.empty(u.numel() + 4, dtype=u.dtype, device="cuda")
+        room[4:] = u.flatten()
+        u = room[4:].view(u.shape)
+        assert u.data_ptr() % 16 == 8
+    return (q, u, vt, x, None), want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,T", CASES)
+def test_edges(I, M, N, T):
+    print(f"tile kernel I={I} M={M} N={N} T={T}", flush=True)
+    assert _lib.lib().bs_forward_path(I, M, N, 16, T) in (_lib.PATH_STRIP, _lib.PATH_DECODE_F16, _lib.PATH_DECODE_MX)
+    args, want = _args(I, M, N, T, False)
+    y = IU.bitstack_forward_hip(*args)
+    _lib.workspace(torch.device("cuda"), 1).fill_(0xFF)          # nothing is read from scratch that the call has not written
+    assert torch.equal(IU.bitstack_forward_hip(*args), y)
+    d = np.abs(y.cpu().numpy().astype(np.float64) - want)
+    assert d.max() <= 1e-2 * np.abs(want).max() and d.mean() <= 1e-3 * np.abs(want).mean(), (d.max(), d.mean())
+    other = IU.bitstack_forward_hip(*_args(I, M, N, T, True)[0])
+    # The same weights in fp32, their blocks added in the same order, and rounded to fp16 (2^-11 of a weight where the two sums straddle a
+    # rounding boundary, for few of them), then fp32 sums over the columns in another order and one rounding to fp16 each.
+    w = IU.unpack_and_reconstruct_w_hip(*args[:3])
+    size = torch.matmul(args[3].double().abs(), w.double().abs().t().contiguous())
+    assert bool(((y.double() - other.double()).abs() <= y.double().abs() * 2.0 ** -10 + size * 2.0 ** -12).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 8, 20, 40])
+def test_non_finite_inputs(T):
+    """An infinity or NaN in u, vt or x reaches the outputs it has a part in and no others."""
+    I, M, N = 3, 100, 640
+    (q, u, vt, x, _), _ = _args(I, M, N, T, False)
+    clean = IU.bitstack_forward_hip(q, u, vt, x, None)
+    for value in (float("inf"), float("nan")):
+        bad = u.clone()
+        bad[1, 37, 3] = value
+        y = IU.bitstack_forward_hip(q, bad, vt, x, None)
+        assert not torch.isfinite(y[..., 37]).any()
+        keep = torch.arange(M, device="cuda") != 37
+        assert torch.equal(y[..., keep], clean[..., keep])
+        bad = x.clone()
+        bad.view(T, N)[T - 1, 130] = value
+        y = IU.bitstack_forward_hip(q, u, vt, bad, None).view(T, M)
+        assert not torch.isfinite(y[T - 1]).any() and torch.equal(y[:T - 1], clean.view(T, M)[:T - 1])
+        bad = vt.clone()
+        bad[2, 5, 200] = value
+        assert not torch.isfinite(IU.bitstack_forward_hip(q, u, bad, x, None)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [8, 40])
+@pytest.mark.parametrize("N", [1024, 2176])
+def test_groups_of_unlike_matrices_are_the_single_calls(N, T):
+    """Matrices of other heights and block counts in one launch: what each computes alone, up to the order of the column groups' sums."""
+    L = _lib.lib()
+    layers = [(1, 700), (8, 33), (3, 1000), (5, 64)]
+    x = synthetic_layer(8, N, 1, T, seed=3)[3].cuda()
+    mats = (_lib.bs_matrix * len(layers))()
+    keep, alone = [], []
+    for j, (I, M) in enumerate(layers):
+        q, u, vt, _ = (t.cuda() for t in synthetic_layer(M, N, I, T, seed=j, signed_factors=True))
+        keep.append((q, u, vt))
+        mats[j] = _lib.bs_matrix(q.data_ptr(), u.data_ptr(), vt.data_ptr(), None, I, M)
+        alone.append((IU.bitstack_forward_hip(q, u, vt, x, None).view(T, M), IU.unpack_and_reconstruct_w_hip(q, u, vt)))
+    rows = sum(M for _, M in layers)
+    y = torch.empty(T, rows, dtype=torch.half, device="cuda")
+    need = L.bs_forward_group_workspace_bytes(ctypes.byref(mats), len(layers), N, 16, T)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    _lib.check(L.bs_forward_group(ctypes.byref(mats), len(layers), N, 16, x.data_ptr(), T, 0, None, y.data_ptr(), ws.data_ptr(), need,
+                                  torch.cuda.current_stream().cuda_stream), "bs_forward_group")
+    at = 0
+    for (I, M), (ref, w) in zip(layers, alone):
+        part = y[:, at:at + M].double()
+        at += M
+        size = torch.matmul(x.double().view(T, N).abs(), w.double().abs().t().contiguous())
+        assert bool(((part - ref.double()).abs() <= ref.double().abs() * 2.0 ** -10 + size * 2.0 ** -13).all()), (I, M)
+
+
+@pytest.mark.skipif(not os.path.exists(shutil.which("hipcc") or "/opt/rocm/bin/hipcc"), reason="hipcc not available")
+def test_the_tile_kernels_keep_everything_in_registers(tmp_path):
+    asm = tmp_path / "k.s"
+    subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, "tile.hip"), "-o", str(asm)], check=True, capture_output=True)
+    sizes = re.findall(r"\.private_segment_fixed_size:\s+(\d+)", asm.read_text())
+    assert sizes and set(sizes) == {"0"}, sizes

@@ -345,12 +345,26 @@ extern "C" int bs_forward_cat(const bs_matrix *mats, int n, int N, int K, const 
     if (!workspace || workspace_bytes < need || !bs_aligned(workspace, 256)) return BS_ERR_WORKSPACE;
     half_t *w = (half_t *)workspace;
     int64_t rows = 0;
+    const uint8_t *packed[BS_MAX_GROUP];
+    const half_t *u[BS_MAX_GROUP], *vt[BS_MAX_GROUP];
+    half_t *part[BS_MAX_GROUP];
+    int I[BS_MAX_GROUP], M[BS_MAX_GROUP];
     for (int j = 0; j < n; j++) {
-        const int st = bs_launch_reconstruct_packed((const uint8_t *)mats[j].packed, (const half_t *)mats[j].u, (const half_t *)mats[j].vt,
-                                                    w + rows * N, mats[j].I, mats[j].M, N, K, (hipStream_t)stream);
-        if (st != BS_OK) return st;
-        rows += mats[j].M;
+        packed[j] = (const uint8_t *)mats[j].packed;
+        u[j] = (const half_t *)mats[j].u;
+        vt[j] = (const half_t *)mats[j].vt;
+        part[j] = w + rows * N;
+        I[j] = mats[j].I;
+        M[j] = mats[j].M;
+        rows += M[j];
     }
+    int st = bs_launch_tile_rebuild(n, packed, u, vt, I, M, part, N, K, (hipStream_t)stream);       // all in one launch, or one by one
+    for (int j = 0; st == BS_ERR_SHAPE && j < n; j++) {
+        const int one = bs_launch_reconstruct_packed(packed[j], u[j], vt[j], part[j], I[j], M[j], N, K, (hipStream_t)stream);
+        if (one != BS_OK) return one;
+        if (j + 1 == n) st = BS_OK;
+    }
+    if (st != BS_OK) return st;
     return bs_launch_linear_parts((const half_t *)x, w, nullptr, (half_t *)y, T, (int)rows, N,
                                   (float *)((char *)workspace + round_up(rows * N * 2, 256)), (hipStream_t)stream);
 }

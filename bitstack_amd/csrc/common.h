@@ -99,6 +99,9 @@ int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *con
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s);
+// the same kernel's rebuilt weights (BS_ERR_SHAPE: not taken, nothing enqueued)
+int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
+                           half_t *const *w, int N, int K, hipStream_t s);
 // panel kernel (panel.hip): the same partial sums for up to 128 tokens, sign tiles decoded into LDS and
 // multiplied on the matrix cores at once; bs_panel_partials = column groups (0: the shape is not taken)
 constexpr int BS_PANEL_MAX_T = 128;

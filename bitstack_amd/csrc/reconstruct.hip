@@ -335,6 +335,9 @@ int check_dims(int I, int M, int N, int K) {
 
 int bs_launch_reconstruct_packed(const uint8_t *packed, const half_t *u, const half_t *vt,
                                  half_t *w, int I, int M, int N, int K, hipStream_t s) {
+    // (the weight inside a forward; bs_reconstruct_w keeps to the kernel that the int8 signs take, whose weights are the same bit for bit)
+    const int st = bs_launch_tile_rebuild(1, &packed, &u, &vt, &I, &M, &w, N, K, s);
+    if (st != BS_ERR_SHAPE) return st;
     return launch_reconstruct<true>(packed, nullptr, u, vt, w, I, M, N, K, s);
 }
 

@@ -14,6 +14,10 @@
 // (v_mfma_f32_16x16x32_f16).  The waves' y tiles (same rows, other columns) meet in LDS, double buffered, and are added up in wave
 // order while the next tile is rebuilt: one barrier per tile, and scratch holds one partial per 256 NP columns.
 //
+// The rebuilt weight itself (TT = 0, above 128 tokens and for levels 3 and 4) is the same walk with the rounded tile stored instead of
+// multiplied.  us, reconstruct_tile_kernel / this: 14336 x 4096, 8 blocks 55.6 / 48.3 (40.5 without the stores), 4096 x 14336, 8 56.3 / 46.3, 28672 x 8192, 3
+// 178 / 112 (558 MB: 5.0 TB/s, the copy rate), 14336 x 4096, 5 43.7 / 37.3.
+//
 // What bounds it: the issue of a wave's instructions.  Simple VALU instructions (v_xor_b32, v_and_b32, v_lshrrev_b32, fp32 add, mul and FMA on
 // three registers) of two waves run side by side on a SIMD, 1.0 ns each; v_fma_mix_f32, v_and_or_b32, v_bfe, v_alignbit, conversions and whatever
 // has a scalar operand take 1.8 ns, and a single wave issues one instruction in 2 ns whatever it is.  A step (1024 signs: 16 v_xor, 5 for the
@@ -37,6 +41,7 @@ struct TileMat {
     const uint8_t *packed;
     const half_t *u, *vt;
     float *part;
+    half_t *w;                                      // (the rebuild: where the weight goes; part is null)
     int I, M, np, row_tiles, first_wg, wgs;         // workgroups first_wg + wgs * column group .. + wgs - 1
 };
 struct TileGroup {
@@ -80,7 +85,7 @@ typedef const __attribute__((address_space(3))) float *lds_f32;
 typedef __attribute__((address_space(3))) float *lds_f32_rw;
 typedef __attribute__((address_space(3))) float4_t *lds_f32x4_rw;
 
-// TT: token tiles of 16.
+// TT: token tiles of 16; 0: the weight itself is what is wanted, it goes to memory.
 template <int TT, int NP>
 struct TileKernel {
     static constexpr int WC = 32 * NP, CG = WC * TL_WAVES;     // columns per wave, per workgroup
@@ -89,23 +94,24 @@ struct TileKernel {
     static constexpr int SCH = SROW * TL_ROWS / 1024;          // requests of 1 KB per block: signs; u is one more
     // what a row's pieces are XOR-ed with in a stage, so that the 32 rows a read takes fall on different banks
     static __device__ __forceinline__ int swizzle(int r) { return (r * RP / 16) % RP; }
-    // LDS: the table of sign masks (at address 0: the kernel has no other LDS), an area for two y tiles of every wave (and at first for the
-    // vt images), and the ring of stages
-    static constexpr int AREA = 32 * 1024 * TT;
+    // LDS: the table of sign masks (at address 0: the kernel has no other LDS), an area for two y tiles of every wave or its tile of the
+    // weight (and at first for the vt images), and the ring of stages
+    static constexpr int AREA = TT ? 32 * 1024 * TT : TL_WAVES * TL_ROWS * WC * 2;
     static constexpr int stage_bytes(int I) { return I * (SCH + 1) * 1024; }
+    static constexpr size_t lds_size(int I) { return TL_TABLE + AREA + STAGES * (size_t)stage_bytes(I); }
     static constexpr int STAGES = 3;                           // the tile in work, the next one, one that is being written
     // most blocks: LDS, and the registers of the vt fragments
     static constexpr int max_blocks() {
-        int I = NP == 4 ? (TT == 1 ? 4 : TT == 2 ? 2 : 1) : NP == 2 ? (TT == 1 ? 10 : 8) : 16;
-        while (TL_TABLE + AREA + STAGES * stage_bytes(I) > TL_LDS) I--;
+        int I = NP == 4 ? (TT <= 1 ? 4 : TT == 2 ? 2 : 1) : NP == 2 ? (TT <= 1 ? 10 : 8) : 16;
+        while (lds_size(I) > TL_LDS) I--;
         return I;
     }
 
     // One run of row tiles [rt0, rt0 + len) of column group cg of one matrix.
     template <int I>
     static __device__ __forceinline__ void walk(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, const half_t *__restrict__ vt,
-                                                float *__restrict__ part, int M, lds_bytes_rw lds, const half_t *__restrict__ x, int N, int T,
-                                                int cg, int rt0, int len, float *ssq) {
+                                                float *__restrict__ part, half_t *__restrict__ w, int M, lds_bytes_rw lds, const half_t *__restrict__ x,
+                                                int N, int T, int cg, int rt0, int len, float *ssq) {
         constexpr int STAGE = stage_bytes(I);
         constexpr int CHUNKS = I * (SCH + 1), PER = CHUNKS / TL_WAVES, MORE = CHUNKS % TL_WAVES, MOST = PER + (MORE != 0);
         int tid = threadIdx.x;
@@ -173,7 +179,8 @@ struct TileKernel {
         // part of the area; the fragments are read back from there.  (The columns of a group of eight are XOR-ed with the group's
         // number: the groups lie a whole turn of the banks apart.)
         half8_t vf[I][NP];
-        half8_t xf[TT][NP];
+        constexpr int TX = TT ? TT : 1;
+        half8_t xf[TX][NP];
         if (mine) {
             constexpr int PIECES = WC / 8, BP = 32 / PIECES, PASSES = (I + BP - 1) / BP, IMAGE = WC * 32;   // BP blocks per pass of loads
             constexpr int ROOM = (AREA / TL_WAVES < 8192 ? AREA / TL_WAVES : 8192), SB = ROOM / IMAGE;      // SB of them fit the image
@@ -220,7 +227,7 @@ struct TileKernel {
         write_tile(0, pieces);
         if constexpr (NP < 4) write_tile(1, pieces_1);
         request_next(pieces);
-        if (ssq) {          // sums of squares of x over the group's columns
+        if (TT > 0 && ssq) {          // sums of squares of x over the group's columns
             lds_f32_rw sums = (lds_f32_rw)area;
             __syncthreads();                         // (the area holds the vt images)
             if (mine) {
@@ -275,7 +282,7 @@ struct TileKernel {
             if (16 * tt + my_t < T && rt * TL_ROWS + my_row < M) *reinterpret_cast<float *>(to + my_out) = sum;
         };
         // the second product's result: rows 0-15 ([tt][0]) and 16-31 ([tt][1]) of a tile, D[token 4 g + j, row lm] of each
-        float4_t y[TT][2];
+        float4_t y[TX][2];
         auto leave = [&](int buf) {
             lds_f32x4_rw red = (lds_f32x4_rw)(area + (buf * TL_WAVES + wave) * (Y * 4)) + lane;
 #pragma unroll
@@ -350,6 +357,16 @@ struct TileKernel {
             write_tile(1, pieces);
             request_next(pieces);
         }
+        // ---- the weight's way to memory (TT = 0) --------------------------------------------------------------------------
+        // By way of LDS (the wave's own part; the 16-byte chunks XOR-ed with the row) a store instruction writes whole lines; the stores
+        // of a tile are issued between the steps of the next one, all at once they would be waited for.
+        constexpr int CH = 4 * NP, STORES = TL_ROWS * CH / 64;       // chunks per row, store instructions per tile
+        const auto place = [&](int r, int c) { return (lds_half8_rw)(area + wave * (TL_ROWS * WC * 2) + r * (WC * 2) + ((c ^ (r * CH / 16)) % CH) * 16); };
+        const uint32_t w_lane = (uint32_t)(lane / CH) * (uint32_t)N + 8 * (lane % CH);
+        auto store_from = [&](int rt, int k, const half8_t &o) {
+            if (rt * TL_ROWS + k * (64 / CH) + lane / CH < M) *reinterpret_cast<half8_t *>(w + (int64_t)(rt * TL_ROWS + k * (64 / CH)) * N + n0 + w_lane) = o;
+        };
+        auto chunk = [&](int k) { return *place(k * (64 / CH) + lane / CH, lane % CH); };
         int stage = 0;
 #pragma clang loop unroll(disable)
         for (int n = 0; n < len; n++) {
@@ -384,6 +401,11 @@ struct TileKernel {
                     if constexpr (s == STEPS - NP) fetch_first(st_next);
                     if constexpr (k % 2 == 0 && k / 2 >= 1 && k / 2 <= TT) hand_over(rt0 + n - 2, k / 2 - 1, v, n >= 2);
                     if constexpr (k % 2 == 0 && k / 2 < TT) collect(oldest, k / 2, v);
+                    // (the weight's stores C .. D - 1 of the last tile go with this step)
+                    constexpr int C = TT ? 0 : (STORES * k + STEPS - NP - 1) / (STEPS - NP), D = TT ? 0 : (STORES * (k + 1) + STEPS - NP - 1) / (STEPS - NP);
+                    half8_t out[D > C ? D - C : 1];
+#pragma unroll
+                    for (int c = C; c < D; c++) out[c - C] = chunk(c);
                     __builtin_amdgcn_sched_barrier(0);
                     asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
 #pragma unroll
@@ -398,7 +420,11 @@ struct TileKernel {
                         acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
                     asm volatile("" : "+v"(acc[p]));
                     __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (k == (STEPS - NP > 1 ? 1 : 0)) leave(before);
+                    if (D > C && n > 0) {
+#pragma unroll
+                        for (int c = C; c < D; c++) store_from(rt0 + n - 1, c, out[c - C]);
+                    }
+                    if constexpr (TT > 0 && k == (STEPS - NP > 1 ? 1 : 0)) leave(before);
                 });
                 // (the passes for which there were not enough steps)
                 constexpr int COLLECTED = (STEPS - NP + 1) / 2 < TT ? (STEPS - NP + 1) / 2 : TT, HANDED = (STEPS - NP - 1) / 2 < TT ? (STEPS - NP - 1) / 2 : TT;
@@ -408,6 +434,20 @@ struct TileKernel {
                     hand_over(rt0 + n - 2, COLLECTED + decltype(k)::value, v, n >= 2);
                 });
                 if constexpr (NP < 4) pass_on();
+                if constexpr (TT == 0) {
+                    // One rounding to fp16; a lane holds columns 16 NP h .. + 16 NP - 1 of row l % 32
+#pragma unroll
+                    for (int p = 0; p < NP; p++)
+#pragma unroll
+                        for (int e = 0; e < 2; e++) {
+                            half8_t o;
+#pragma unroll
+                            for (int k = 0; k < 8; k++) o[k] = (half_t)acc[p][8 * e + k];
+                            *place(row, 2 * NP * h + 2 * p + e) = o;
+                        }
+                    asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
+                    first_block();                               // of tile n + 1
+                } else {
                 // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
                 // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
                 // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
@@ -435,6 +475,7 @@ struct TileKernel {
 #pragma unroll
                         for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
                     }
+                }
             } else {
                 if constexpr (NP < 4) pass_on();
 #pragma unroll
@@ -443,6 +484,13 @@ struct TileKernel {
                     hand_over(rt0 + n - 2, tt, v, n >= 2);
                 }
             }
+        }
+        if (TT == 0) {
+            if (mine) {
+#pragma unroll
+                for (int c = 0; c < STORES; c++) store_from(last_rt, c, chunk(c));
+            }
+            return;
         }
         // the last two tiles
         if (len > 2) tl_barrier();                   // (everybody has collected the tile whose place this is)
@@ -483,7 +531,7 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     auto walk = [&](auto np, auto blocks) {
         typedef TileKernel<TT, decltype(np)::value> TK;
         if constexpr (decltype(blocks)::value <= TK::max_blocks())
-            TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].M, lds, x, N, T, cg, rt, len, ssq);
+            TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].w, grp->m[j].M, lds, x, N, T, cg, rt, len, ssq);
     };
     // (the narrower widths serve what the wider ones cannot hold, and short runs)
     switch (grp->m[j].np * 32 + grp->m[j].I) {
@@ -507,6 +555,7 @@ struct TilePlan {
 };
 int tile_limit(int np, int T) {
     const int tt = (T + 15) / 16;
+    if (tt == 0) return np == 4 ? TileKernel<0, 4>::max_blocks() : np == 2 ? TileKernel<0, 2>::max_blocks() : TileKernel<0, 1>::max_blocks();
     return tt == 1 ? (np == 4 ? TileKernel<1, 4>::max_blocks() : np == 2 ? TileKernel<1, 2>::max_blocks() : TileKernel<1, 1>::max_blocks())
            : tt == 2 ? (np == 4 ? TileKernel<2, 4>::max_blocks() : np == 2 ? TileKernel<2, 2>::max_blocks() : TileKernel<2, 1>::max_blocks())
                      : (np == 4 ? TileKernel<3, 4>::max_blocks() : np == 2 ? TileKernel<3, 2>::max_blocks() : TileKernel<3, 1>::max_blocks());
@@ -561,10 +610,23 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     // 3366 x 2688, 11 (4, 5) 25.6 / 23.1, 2440 x 1536, 14 (2, 2) 20.4 / 17.0, 20191 x 256, 11 (6, 3) 29.4 / 15.5.  And where either does one tile or step of
     // one or two blocks: the hand-over between the waves is half a us (896 x 2176, 1 block 6.8 / 7.5; 643 x 896, 2 blocks 8.4 / 8.9; from 3 blocks
     // on level or ahead).
-    if (n == 1 && best.grid != 0) {
+    if (T > 0 && n == 1 && best.grid != 0) {
         const int64_t tiles = bs_cdiv(bs_cdiv(M[0], TL_ROWS), best.wgs[0]);
         const long steps = best.np[0] == 1 || I[0] <= 2 ? bs_strip_steps(I[0], M[0], N, T) : 0;
         if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || (I[0] <= 2 && tiles == 1 && steps == 1)) best.grid = 0;
+    }
+    // The rebuild's start costs 1.2 us more than reconstruct_tile_kernel's (226 x 896, 1 block 3.6 / 5.1; 1270 x 2688, 2 blocks 5.8 / 6.4), which a single tile
+    // does not win back up to a dozen blocks (556 x 384, 9 blocks 7.8 / 8.7; 257 x 384, 16 10.8 / 9.7), nor two tiles of three blocks (2304 x 2048, with
+    // its product of 775 tokens 30.4 / 31.4); longer runs do (6144 x 4096, 3 blocks, runs of 3, 18.9 / 16.5).
+    if (T == 0 && best.grid != 0) {
+        int64_t longest = 0;
+        int most = 0;
+        for (int j = 0; j < n; j++) {
+            const int64_t run = bs_cdiv(bs_cdiv(M[j], TL_ROWS), best.wgs[j]);
+            if (run > longest) longest = run;
+            if (I[j] > most) most = I[j];
+        }
+        if ((longest == 1 && most <= 12) || (longest == 2 && most < 4)) best.grid = 0;
     }
     return best;
 }
@@ -574,7 +636,7 @@ int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, h
     size_t lds = 0;
     for (int j = 0; j < grp.n; j++) {
         const int np = grp.m[j].np, I = grp.m[j].I;
-        const size_t b = TL_TABLE + TileKernel<TT, 1>::AREA + 3 * (size_t)(np == 4 ? TileKernel<TT, 4>::stage_bytes(I) : np == 2 ? TileKernel<TT, 2>::stage_bytes(I) : TileKernel<TT, 1>::stage_bytes(I));
+        const size_t b = np == 4 ? TileKernel<TT, 4>::lds_size(I) : np == 2 ? TileKernel<TT, 2>::lds_size(I) : TileKernel<TT, 1>::lds_size(I);
         if (b > lds) lds = b;
     }
     static bs_lds_grant granted[BS_MAX_DEVICES];
@@ -588,7 +650,7 @@ int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, h
 TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
     TilePlan none;
     none.grid = 0;
-    if (n < 1 || n > TL_GROUP || K != 16 || T < 1 || T > 48 || N < SF_COLS || N % SF_COLS != 0) return none;
+    if (n < 1 || n > TL_GROUP || K != 16 || T < 0 || T > 48 || N < SF_COLS || N % SF_COLS != 0) return none;
     for (int j = 0; j < n; j++)
         // a block's sign and u rows, and 16 tokens of partial sums, lie within 32-bit byte offsets
         if (I[j] < 1 || M[j] < 1 || (int64_t)M[j] * (N >> 3) >= ((int64_t)1 << 32) || (int64_t)M[j] * 64 >= ((int64_t)1 << 32)) return none;
@@ -599,6 +661,7 @@ TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
 
 // Column groups (partial sums per output) of every matrix, if this kernel takes them.
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups) {
+    if (T < 1) return false;
     const TilePlan p = checked_plan(I, M, n, N, K, T);
     for (int j = 0; p.grid != 0 && j < n; j++) groups[j] = p.groups[j];
     return p.grid != 0;
@@ -607,16 +670,35 @@ bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, in
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s) {
     const TilePlan p = checked_plan(I, M, n, N, K, T);
-    if (p.grid == 0 || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
+    if (p.grid == 0 || T < 1 || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
     TileGroup grp;
     grp.n = n;
     grp.ssq = ssq;
     int first = 0;
     for (int j = 0; j < n; j++) {
         if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], 16)) return BS_ERR_SHAPE;
-        grp.m[j] = TileMat{packed[j], u[j], vt[j], part[j], I[j], M[j], p.np[j], (int)bs_cdiv(M[j], TL_ROWS), first, p.wgs[j]};
+        grp.m[j] = TileMat{packed[j], u[j], vt[j], part[j], nullptr, I[j], M[j], p.np[j], (int)bs_cdiv(M[j], TL_ROWS), first, p.wgs[j]};
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
     return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, s) : launch_tile<3>(grp, p.grid, x, N, T, s);
+}
+
+// The weights of n <= 4 matrices with the same columns, w[j] f16 [M[j], N]; BS_ERR_SHAPE: not taken, nothing was enqueued.
+int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
+                           half_t *const *w, int N, int K, hipStream_t s) {
+    for (int j = 0; j < n && j < TL_GROUP; j++)
+        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], 16) || !bs_aligned(w[j], 16)) return BS_ERR_SHAPE;
+    const TilePlan p = checked_plan(I, M, n, N, K, 0);
+    if (p.grid == 0) return BS_ERR_SHAPE;
+    TileGroup grp;
+    grp.n = n;
+    grp.ssq = nullptr;
+    int first = 0;
+    for (int j = 0; j < n; j++) {
+        grp.m[j] = TileMat{packed[j], u[j], vt[j], nullptr, w[j], I[j], M[j], p.np[j], (int)bs_cdiv(M[j], TL_ROWS), first, p.wgs[j]};
+        first += p.wgs[j] * p.groups[j];
+    }
+    for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
+    return launch_tile<0>(grp, p.grid, nullptr, N, 0, s);
 }

@@ -115,3 +115,61 @@ def test_the_tile_kernels_keep_everything_in_registers(tmp_path):
                     "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, "tile.hip"), "-o", str(asm)], check=True, capture_output=True)
     sizes = re.findall(r"\.private_segment_fixed_size:\s+(\d+)", asm.read_text())
     assert sizes and set(sizes) == {"0"}, sizes
+
+
+# rows about whole tiles, partial column groups, block counts on both sides of the widths' limits, runs of one and of many tiles
+REBUILDS = [(1, 16411, 640), (2, 8200, 1152), (3, 20000, 384), (4, 8193, 2176), (5, 4100, 1664), (8, 9000, 1024), (10, 33, 128), (11, 2500, 768), (16, 1000, 1280),
+            (16, 31, 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N", REBUILDS)
+def test_rebuilt_weight(I, M, N):
+    print(f"rebuild I={I} M={M} N={N}", flush=True)
+    (q, u, vt, _, _), _ = _args(I, M, N, 1, False)
+    # a forward of more than 128 tokens leaves it at the start of its scratch
+    L, T = _lib.lib(), 130
+    x, y = torch.ones(T, N, dtype=torch.half, device="cuda"), torch.empty(T, M, dtype=torch.half, device="cuda")
+    need = L.bs_workspace_bytes(I, M, N, 16, T)
+    assert L.bs_forward_path(I, M, N, 16, T) == _lib.PATH_REBUILD and need >= M * N * 2
+    guard = torch.full((need // 2 + 64,), 7.0, dtype=torch.half, device="cuda")
+    _lib.check(L.bs_forward(q.data_ptr(), u.data_ptr(), vt.data_ptr(), x.data_ptr(), None, y.data_ptr(), I, M, N, 16, T, guard.data_ptr(), need,
+                            torch.cuda.current_stream().cuda_stream), "bs_forward")
+    assert bool((guard[need // 2:] == 7.0).all())
+    w = guard[:M * N].view(M, N)
+    # float64 from the same factors: I fp32 additions of sums of 16 exact products, and one rounding to fp16
+    sign = ((q.view(I, M, N // 8, 1) >> torch.arange(7, -1, -1, device="cuda", dtype=torch.uint8)) & 1).reshape(I, M, N)
+    want = torch.zeros(M, N, dtype=torch.float64, device="cuda")
+    size = torch.zeros_like(want)
+    for i in range(I):
+        p = u[i].double() @ vt[i].double()
+        want += torch.where(sign[i].bool(), p, -p)
+        size += u[i].double().abs() @ vt[i].double().abs()
+    assert bool(((w.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * (I + 16) * 2.0 ** -24 + 2.0 ** -25).all())
+
+
+@pytest.mark.gpu
+def test_rebuilt_weights_of_several_matrices_in_one_launch():
+    """bs_forward_cat rebuilds its matrices together: the rows of each are what the matrix gives alone."""
+    L = _lib.lib()
+    N, T, layers = 1024, 200, [(3, 4100), (6, 700), (1, 1300)]
+    x = synthetic_layer(8, N, 1, T, seed=3)[3].cuda()
+    mats, keep = (_lib.bs_matrix * len(layers))(), []
+    for j, (I, M) in enumerate(layers):
+        keep.append([t.cuda() for t in synthetic_layer(M, N, I, T, seed=j, signed_factors=True)[:3]])
+        mats[j] = _lib.bs_matrix(*(t.data_ptr() for t in keep[-1]), None, I, M)
+    need = L.bs_forward_cat_workspace_bytes(ctypes.byref(mats), len(layers), N, 16, T)
+    assert need > 0
+    rows = sum(M for _, M in layers)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    y = torch.empty(T, rows, dtype=torch.half, device="cuda")
+    _lib.check(L.bs_forward_cat(ctypes.byref(mats), len(layers), N, 16, x.data_ptr(), T, y.data_ptr(), ws.data_ptr(), need,
+                                torch.cuda.current_stream().cuda_stream), "bs_forward_cat")
+    w = ws[:rows * N * 2].view(torch.half).view(rows, N)
+    at = 0
+    for (I, M), (q, u, vt) in zip(layers, keep):
+        alone = IU.unpack_and_reconstruct_w_hip(q, u, vt)
+        # the same products added up in the same order, once by the matrix instruction and once behind it: a weight's rounding apart, rarely
+        d = (w[at:at + M].double() - alone.double()).abs()
+        assert bool((d <= alone.double().abs() * 2.0 ** -10 + 2.0 ** -23).all()) and float((d > 0).double().mean()) < 1e-2
+        at += M

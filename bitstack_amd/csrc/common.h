@@ -96,9 +96,10 @@ int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *con
                           int N, int K, int T, hipStream_t s);
 // tile kernel (tile.hip): the same partial sums for up to 48 tokens at rank 16, 32 x 32 outputs per matrix instruction; groups[j] column
 // groups (partial sums per output) of matrix j where it takes them
+// (split: up to 16 tokens on weights that are not rounded to fp16)
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
-                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s);
+                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s);
 // the same kernel's rebuilt weights (BS_ERR_SHAPE: not taken, nothing enqueued)
 int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                            half_t *const *w, int N, int K, hipStream_t s);

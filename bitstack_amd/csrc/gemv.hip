@@ -54,6 +54,8 @@
 #include "common.h"
 #include "gemv_shared.h"
 
+#include <algorithm>
+
 #include <type_traits>
 #include <utility>
 
@@ -805,22 +807,42 @@ int group_path(const int *I, const int *M, int n, int N, int K, int T) {
     // blocks 32 / 12; 8192 x 3200, 4 blocks 40 / 21 (the block-scaled kernel, with that loss: 18 and 24 at 4 and 8 blocks of 4096 x 11008).
     return N % CH != 0 && T < STRIP_MIN_T && strip_group_ok(I, M, n, N, K, T) ? 1 : -1;
 }
+int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
+    int groups[GEMV_MAX_GROUP];
+    if (!bs_tile_partials(I, M, n, N, K, T, groups)) return 0;
+    int64_t total = (int64_t)groups[0] * T;
+    for (int j = 0; j < n; j++) total += (int64_t)groups[j] * T * M[j];
+    return total;
+}
+// Three and four tokens: the factor-through kernel needs 16 products per sign and token, the tile kernel one weight for all of them.  It takes them with
+// the weight in two fp16 terms, so that only y is rounded (error against float64 0.7 of the other's).  us, factor-through / tiles:
+//   4 tokens: 4096 x 14336, 4 blocks 35.7 / 33.0; 14336 x 4096, 8 58.9 / 45.0; 4096 x 4096, 3 16.1 / 13.0, 2 11.3 / 11.8; 14720 x 11776, 2 50.4 / 56.2; 2288 x 7168, 6 26.8 / 18.1
+//   3 tokens: 14336 x 4096, 8 48.9 / 45.3, 5 37.2 / 35.8, 3 26.6 / 27.1; 4096 x 14336, 4 30.3 / 33.7; 4096 x 4096, 3 13.8 / 13.0, 2 9.9 / 11.7; 7605 x 2560, 2 15.4 / 13.9
+// and below a MiB of sign bytes both are a chain of latencies (366 x 512, 14 blocks, 3 tokens 8.3 / 10.6; 1536 x 512, 4, 4 tokens 8.9 / 7.7).
+// A group takes them if each of its matrices alone does.
+bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
+    if ((T != 3 && T != 4) || g_decode_kernel != 0) return false;
+    for (int j = 0; j < n; j++) {
+        const bool large = (int64_t)M[j] * N > (24ll << 20);
+        if (I[j] < 2 || (int64_t)I[j] * M[j] * (N / 8) < (1 << 20)) return false;
+        if ((T == 3 && large && I[j] < 6) || (I[j] == 2 && N >= 4096)) return false;
+    }
+    int groups[GEMV_MAX_GROUP];
+    return bs_tile_partials(I, M, n, N, K, T, groups);
+}
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group
     for (int j = 0; j < n; j++) total += (int64_t)bs_strip_partials(I[j], M[j], N, K, T) * T * M[j];
-    // the tile kernel's partial sums: room for either, the choice also depends on how u is aligned
-    int groups[GEMV_MAX_GROUP];
-    if (!bs_tile_partials(I, M, n, N, K, T, groups)) return total;
-    int64_t tile_total = (int64_t)groups[0] * T;
-    for (int j = 0; j < n; j++) tile_total += (int64_t)groups[j] * T * M[j];
-    return total > tile_total ? total : tile_total;
+    // room for the tile kernel's partial sums too: the choice also depends on how u is aligned
+    return std::max(total, tile_part_floats(I, M, n, N, K, T));
 }
 
 // Strip path: one launch writes part[strip group, t, m] of every matrix; the reduce kernel
 // reads that as "one partial per block" with the strip groups in the place of the blocks.
 int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T, int mode, const half_t *residual,
-                        half_t *y, bool input_rms, float eps, void *workspace, int64_t workspace_bytes, hipStream_t s) {
-    if (!workspace || workspace_bytes < strip_part_floats(a.I, a.M, a.n, N, K, T) * (int64_t)sizeof(float)) return BS_ERR_WORKSPACE;
+                        half_t *y, bool input_rms, float eps, void *workspace, int64_t workspace_bytes, bool split, hipStream_t s) {
+    const int64_t floats = split ? tile_part_floats(a.I, a.M, a.n, N, K, T) : strip_part_floats(a.I, a.M, a.n, N, K, T);
+    if (!workspace || workspace_bytes < floats * (int64_t)sizeof(float)) return BS_ERR_WORKSPACE;
     float *part = (float *)workspace;
     RedGroup r;
     r.n = a.n;
@@ -855,7 +877,7 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     r.ssq = input_rms ? part + off : nullptr;
     r.ssq_n = r.m[0].I;
     float *ssq = input_rms ? part + off : nullptr;
-    const int st = tiles ? bs_launch_tile_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, ssq, x, N, K, T, s)
+    const int st = tiles ? bs_launch_tile_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, ssq, x, N, K, T, split, s)
                          : bs_launch_strip_group(a.n, a.packed, a.u, a.vt, a.I, a.M, parts, ssq, x, N, K, T, s);
     if (st != BS_OK) return st;
     if (mode == EPI_SWIGLU) ldy = a.M[0];
@@ -880,8 +902,11 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
     if (path == 1) {
         for (int j = 0; j < a.n; j++)
             if (!bs_aligned(a.packed[j], 16) || !bs_aligned(a.vt[j], 16) || !bs_aligned(a.u[j], 8)) return BS_ERR_SHAPE;
-        return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, s);
+        return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, false, s);
     }
+    bool split = split_tiles(a.I, a.M, a.n, N, K, T);
+    for (int j = 0; j < a.n; j++) split = split && bs_aligned(a.u[j], 16) && bs_aligned(a.packed[j], 16) && bs_aligned(a.vt[j], 16);
+    if (split) return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, true, s);
     int ldy = 0;
     for (int j = 0; j < a.n; j++) {
         if (!gemv_shape_ok(a.I[j], a.M[j], N, T)) return BS_ERR_SHAPE;
@@ -971,7 +996,9 @@ int64_t bs_gemv_group_workspace_bytes(const int *I, const int *M, int n, int N, 
     const int path = group_path(I, M, n, N, K, T);
     if (path < 0) return 0;
     if (path == 1) return strip_part_floats(I, M, n, N, K, T) * (int64_t)sizeof(float);
-    return gemv_part_floats(I, M, n, N, K, T) * (int64_t)sizeof(float);
+    int64_t floats = gemv_part_floats(I, M, n, N, K, T);
+    if (split_tiles(I, M, n, N, K, T)) floats = std::max(floats, tile_part_floats(I, M, n, N, K, T));
+    return floats * (int64_t)sizeof(float);
 }
 
 // Which instantiation and grid a decode forward of these dimensions runs

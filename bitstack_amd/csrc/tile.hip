@@ -86,7 +86,8 @@ typedef __attribute__((address_space(3))) float *lds_f32_rw;
 typedef __attribute__((address_space(3))) float4_t *lds_f32x4_rw;
 
 // TT: token tiles of 16; 0: the weight itself is what is wanted, it goes to memory.
-template <int TT, int NP>
+// SPLIT (few tokens): the weight is not rounded to fp16 but enters the second product as two fp16 terms.
+template <int TT, int NP, bool SPLIT = false>
 struct TileKernel {
     static constexpr int WC = 32 * NP, CG = WC * TL_WAVES;     // columns per wave, per workgroup
     static constexpr int SROW = CG / 8;                        // sign bytes of a row in a stage
@@ -447,6 +448,37 @@ struct TileKernel {
                         }
                     asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
                     first_block();                               // of tile n + 1
+                } else if constexpr (SPLIT) {
+                    // Two terms per weight: rounded towards zero (a finite weight stays finite), and what that leaves (2^-21 of the weight is lost).  An
+                    // infinite weight leaves the difference of two infinities, a NaN, for which the maximum takes a finite number.  The lanes
+                    // trade places as below.
+#pragma unroll
+                    for (int r = 0; r < 2; r++) y[0][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int p = 0; p < NP; p++) {
+                        half2_t t[2][8];
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            const float a = acc[p][2 * k], b = acc[p][2 * k + 1];
+                            t[0][k] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+                            const half2_t rest = {(half_t)__builtin_fmaf((float)t[0][k][0], -1.f, a), (half_t)__builtin_fmaf((float)t[0][k][1], -1.f, b)};
+                            t[1][k] = __builtin_elementwise_max(rest, (half2_t){(half_t)-65504.f, (half_t)-65504.f});
+                        }
+#pragma unroll
+                        for (int term = 0; term < 2; term++) {
+                            uint4_t lo, hi;
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                const half2_t a = t[term][k], b = t[term][4 + k];
+                                const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                                lo[k] = r[0];
+                                hi[k] = r[1];
+                            }
+                            y[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), y[0][0], 0, 0, 0);
+                            y[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), y[0][1], 0, 0, 0);
+                        }
+                    }
+                    first_block();                   // of tile n + 1
                 } else {
                 // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
                 // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
@@ -510,7 +542,7 @@ struct TileKernel {
     }
 };
 
-template <int TT>
+template <int TT, bool SPLIT>
 __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const TileGroup grp_, const half_t *__restrict__ x, int N, int T) {
     extern __shared__ __attribute__((aligned(1024))) char tl_lds[];
     lds_bytes_rw lds = (lds_bytes_rw)tl_lds;
@@ -529,7 +561,7 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     const int rt = (int)((int64_t)tiles * run / wgs), len = (int)((int64_t)tiles * (run + 1) / wgs) - rt;
     float *ssq = j == 0 && run == 0 ? grp->ssq : nullptr;
     auto walk = [&](auto np, auto blocks) {
-        typedef TileKernel<TT, decltype(np)::value> TK;
+        typedef TileKernel<TT, decltype(np)::value, SPLIT> TK;
         if constexpr (decltype(blocks)::value <= TK::max_blocks())
             TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].w, grp->m[j].M, lds, x, N, T, cg, rt, len, ssq);
     };
@@ -631,7 +663,7 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     return best;
 }
 
-template <int TT>
+template <int TT, bool SPLIT = false>
 int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, hipStream_t s) {
     size_t lds = 0;
     for (int j = 0; j < grp.n; j++) {
@@ -640,9 +672,9 @@ int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, h
         if (b > lds) lds = b;
     }
     static bs_lds_grant granted[BS_MAX_DEVICES];
-    const int st = bs_allow_lds((const void *)tile_forward_kernel<TT>, lds, granted);
+    const int st = bs_allow_lds((const void *)tile_forward_kernel<TT, SPLIT>, lds, granted);
     if (st != BS_OK) return st;
-    tile_forward_kernel<TT><<<grid, 64 * TL_WAVES, lds, s>>>(grp, x, N, T);
+    tile_forward_kernel<TT, SPLIT><<<grid, 64 * TL_WAVES, lds, s>>>(grp, x, N, T);
     BS_LAUNCH_CHECK();
     return BS_OK;
 }
@@ -668,9 +700,9 @@ bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, in
 }
 
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
-                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, hipStream_t s) {
+                         float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s) {
     const TilePlan p = checked_plan(I, M, n, N, K, T);
-    if (p.grid == 0 || T < 1 || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
+    if (p.grid == 0 || T < 1 || (split && T > 16) || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
     TileGroup grp;
     grp.n = n;
     grp.ssq = ssq;
@@ -681,6 +713,7 @@ int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *cons
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
+    if (split) return launch_tile<1, true>(grp, p.grid, x, N, T, s);
     return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, s) : launch_tile<3>(grp, p.grid, x, N, T, s);
 }
 

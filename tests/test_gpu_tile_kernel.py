@@ -173,3 +173,55 @@ def test_rebuilt_weights_of_several_matrices_in_one_launch():
         d = (w[at:at + M].double() - alone.double()).abs()
         assert bool((d <= alone.double().abs() * 2.0 ** -10 + 2.0 ** -23).all()) and float((d > 0).double().mean()) < 1e-2
         at += M
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4])
+@pytest.mark.parametrize("I,M,N", [(2, 8300, 512), (3, 4100, 1024), (4, 4163, 512), (5, 2081, 1536), (6, 1000, 4096), (10, 3001, 1024), (12, 4096, 512), (16, 2600, 1024)])
+def test_three_and_four_tokens(I, M, N, T):
+    """Two fp16 terms per weight: nothing but y is rounded, so it stands no further from float64 than the factor-through kernel."""
+    print(f"two terms I={I} M={M} N={N} T={T}", flush=True)
+    L = _lib.lib()
+    args, want = _args(I, M, N, T, False)
+    size = np.abs(args[3].cpu().numpy().astype(np.float64)) @ np.abs(IU.unpack_and_reconstruct_w_hip(*args[:3]).cpu().numpy().astype(np.float64)).T
+    y = IU.bitstack_forward_hip(*args)
+    _lib.workspace(torch.device("cuda"), 1).fill_(0xFF)
+    assert torch.equal(IU.bitstack_forward_hip(*args), y)
+    d = np.abs(y.cpu().numpy().astype(np.float64) - want)
+    error = np.linalg.norm(d) / np.linalg.norm(want)
+    for mode in (_lib.DECODE_F16, None):                 # the other kernel: pinned, and by u's alignment
+        if mode is not None:
+            _lib.check(L.bs_set_decode_kernel(mode), "bs_set_decode_kernel")
+        try:
+            other = IU.bitstack_forward_hip(*(args if mode is not None else _args(I, M, N, T, True)[0])).cpu().numpy().astype(np.float64)
+        finally:
+            L.bs_set_decode_kernel(_lib.DECODE_AUTO)
+        assert error <= 1.02 * np.linalg.norm(other - want) / np.linalg.norm(want)
+    # one rounding of y; the sums over N columns in fp32, the weights' second terms to 2^-21
+    assert bool((d <= np.abs(want) * 2.0 ** -11 + size * 2.0 ** -13 + 2.0 ** -25).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4])
+def test_three_and_four_tokens_with_non_finite_inputs_and_large_weights(T):
+    I, M, N = 3, 2800, 1024
+    (q, u, vt, x, _), _ = _args(I, M, N, T, False)
+    u, vt, x = u * 0 + 1, vt * 0 + 1, x * 0 + 1
+    q = torch.full_like(q, 0xFF)                         # weights: 16 per block
+    bad = u.clone()
+    bad[1, 37, 3] = float("inf")
+    y = IU.bitstack_forward_hip(q, bad, vt, x, None)
+    keep = torch.arange(M, device="cuda") != 37
+    assert bool(torch.isposinf(y[..., 37]).all()) and bool((y[..., keep] == 48.0 * N).all())
+    bad[1, 37, 3] = float("nan")
+    y = IU.bitstack_forward_hip(q, bad, vt, x, None)
+    assert bool(torch.isnan(y[..., 37]).all()) and bool((y[..., keep] == 48.0 * N).all())
+    # a weight beyond fp16's range stays what it is: 16 * 80 * 80 = 102400 in one block
+    big = u.clone()
+    big[0, 5, :] = 80.0
+    w_vt = vt.clone()
+    w_vt[0] = 80.0
+    z = torch.zeros_like(x)
+    z[..., 9] = 0.25
+    y = IU.bitstack_forward_hip(q, big, w_vt, z, None)
+    assert bool((y[..., 5] == 0.25 * (102400 + 32)).all()), y[..., 5]

@@ -94,8 +94,8 @@ int bs_strip_kernel_choice(int I, int M, int N, int K, int T);
 int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt,
                           const int *I, const int *M, float *const *part, float *ssq, const half_t *x,
                           int N, int K, int T, hipStream_t s);
-// tile kernel (tile.hip): the same partial sums for up to 48 tokens at rank 16, 32 x 32 outputs per matrix instruction; groups[j] column
-// groups (partial sums per output) of matrix j where it takes them
+// tile kernel (tile.hip; from 49 tokens the column kernel): the same partial sums for up to 128 tokens at rank 16, 32 x 32 outputs per matrix
+// instruction; groups[j]: column groups (partial sums per output) of matrix j where it takes them
 // (split: up to 16 tokens on weights that are not rounded to fp16)
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
@@ -103,6 +103,9 @@ int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *cons
 // the same kernel's rebuilt weights (BS_ERR_SHAPE: not taken, nothing enqueued)
 int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                            half_t *const *w, int N, int K, hipStream_t s);
+// column kernel (column.hip): 49 to 128 tokens of one matrix, reached through the two functions above
+int bs_column_partials(int I, int M, int N, int K, int T);
+int bs_launch_column(const uint8_t *packed, const half_t *u, const half_t *vt, int I, int M, float *part, const half_t *x, int N, int K, int T, hipStream_t s);
 // panel kernel (panel.hip): the same partial sums for up to 128 tokens, sign tiles decoded into LDS and
 // multiplied on the matrix cores at once; bs_panel_partials = column groups (0: the shape is not taken)
 constexpr int BS_PANEL_MAX_T = 128;

@@ -694,6 +694,7 @@ TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
 // Column groups (partial sums per output) of every matrix, if this kernel takes them.
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups) {
     if (T < 1) return false;
+    if (T > 48) return n == 1 && (groups[0] = bs_column_partials(I[0], M[0], N, K, T)) > 0;
     const TilePlan p = checked_plan(I, M, n, N, K, T);
     for (int j = 0; p.grid != 0 && j < n; j++) groups[j] = p.groups[j];
     return p.grid != 0;
@@ -701,6 +702,7 @@ bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, in
 
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s) {
+    if (T > 48) return n == 1 && !ssq && !split ? bs_launch_column(packed[0], u[0], vt[0], I[0], M[0], part[0], x, N, K, T, s) : BS_ERR_SHAPE;
     const TilePlan p = checked_plan(I, M, n, N, K, T);
     if (p.grid == 0 || T < 1 || (split && T > 16) || !bs_aligned(x, 16)) return BS_ERR_SHAPE;
     TileGroup grp;

@@ -109,10 +109,11 @@ def test_groups_of_unlike_matrices_are_the_single_calls(N, T):
 
 
 @pytest.mark.skipif(not os.path.exists(shutil.which("hipcc") or "/opt/rocm/bin/hipcc"), reason="hipcc not available")
-def test_the_tile_kernels_keep_everything_in_registers(tmp_path):
+@pytest.mark.parametrize("source", ["tile.hip", "column.hip"])
+def test_the_tile_kernels_keep_everything_in_registers(source, tmp_path):
     asm = tmp_path / "k.s"
     subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-                    "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, "tile.hip"), "-o", str(asm)], check=True, capture_output=True)
+                    "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, source), "-o", str(asm)], check=True, capture_output=True)
     sizes = re.findall(r"\.private_segment_fixed_size:\s+(\d+)", asm.read_text())
     assert sizes and set(sizes) == {"0"}, sizes
 
@@ -225,3 +226,64 @@ def test_three_and_four_tokens_with_non_finite_inputs_and_large_weights(T):
     z[..., 9] = 0.25
     y = IU.bitstack_forward_hip(q, big, w_vt, z, None)
     assert bool((y[..., 5] == 0.25 * (102400 + 32)).all()), y[..., 5]
+
+
+# 49 to 128 tokens: the column kernel from 11 Mi weights on.  Both sides of its token tiles and block limits, rows about whole workgroups of 256,
+# half a span of columns at the end, one span and many per workgroup
+COLUMNS = [(1, 11300, 1024, 49), (2, 12033, 1024, 64), (8, 2816, 4096, 64), (8, 2817, 4224, 50), (3, 30977, 384, 65), (7, 2815, 4352, 96), (5, 90200, 128, 80),
+           (6, 11265, 1152, 97), (6, 4000, 4096, 128), (4, 257, 45056, 127), (1, 20737, 640, 128), (5, 8191, 5760, 100)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,T", COLUMNS)
+def test_columns_edges(I, M, N, T):
+    """Against float64 from the same rounded weights, and against the kernels that take the call when u is off a 16-byte boundary."""
+    print(f"column kernel I={I} M={M} N={N} T={T}", flush=True)
+    L = _lib.lib()
+    assert L.bs_forward_path(I, M, N, 16, T) in (_lib.PATH_WALKED, _lib.PATH_PANEL)
+    q, u, vt, x = (t.cuda() for t in synthetic_layer(M, N, I, T, seed=I + N + T, signed_factors=True))
+    u = (u * 20).half()
+    bias = torch.randn(M, device="cuda").half()
+    need = L.bs_workspace_bytes(I, M, N, 16, T)
+    guard = torch.full((need // 2 + 64,), float("nan"), dtype=torch.half, device="cuda")
+    y = torch.full((T, M), float("nan"), dtype=torch.half, device="cuda")
+    _lib.check(L.bs_forward(q.data_ptr(), u.data_ptr(), vt.data_ptr(), x.data_ptr(), bias.data_ptr(), y.data_ptr(), I, M, N, 16, T, guard.data_ptr(), need,
+                            torch.cuda.current_stream().cuda_stream), "bs_forward")
+    assert bool(guard[need // 2:].isnan().all())
+    room = torch.empty(u.numel() + 4, dtype=u.dtype, device="cuda")
+    room[4:] = u.flatten()
+    other = IU.bitstack_forward_hip(q, room[4:].view(u.shape), vt, x, bias).view(T, M)
+    # Rounded weights: 2^-11 of a weight where the two fp32 sums straddle a rounding boundary, for few of them; then fp32 sums over the columns
+    # and one rounding to fp16.
+    w = IU.unpack_and_reconstruct_w_hip(q, u, vt)
+    xd = x.view(T, N).double()
+    want = torch.matmul(xd, w.double().t().contiguous()) + bias.double()
+    size = torch.matmul(xd.abs(), w.double().abs().t().contiguous()) + bias.double().abs()
+    bound = want.abs() * 2.0 ** -10 + size * 2.0 ** -12
+    assert bool(((y.double() - want).abs() <= bound).all()) and bool(((other.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,T", [(3, 30800, 384, 60), (2, 2900, 4096, 128)])
+def test_columns_with_non_finite_inputs(I, M, N, T):
+    """An infinity or NaN in u, vt or x reaches the outputs it has a part in and no others, and an infinite weight stays one beside the columns
+    that a half span at the end does not have."""
+    q, u, vt, x = (t.cuda() for t in synthetic_layer(M, N, I, T, seed=3, signed_factors=True))
+    clean = IU.bitstack_forward_hip(q, u, vt, x, None).view(T, M)
+    keep = torch.arange(M, device="cuda") != 37
+    for value in (float("inf"), float("nan")):
+        bad = u.clone()
+        bad[1, 37, 3] = value
+        y = IU.bitstack_forward_hip(q, bad, vt, x, None).view(T, M)
+        assert not torch.isfinite(y[:, 37]).any() and torch.equal(y[:, keep], clean[:, keep])
+        bad = x.clone()
+        bad.view(T, N)[T - 1, 130] = value
+        y = IU.bitstack_forward_hip(q, u, vt, bad, None).view(T, M)
+        assert not torch.isfinite(y[T - 1]).any() and torch.equal(y[:T - 1], clean[:T - 1])
+        bad = vt.clone()
+        bad[1, 5, 200] = value
+        assert not torch.isfinite(IU.bitstack_forward_hip(q, u, bad, x, None)).any()
+    big, ones, pos = u.clone(), torch.full_like(q, 0xFF), vt.abs() + 0.01
+    big[0, 37, 3] = float("inf")
+    y = IU.bitstack_forward_hip(ones, big, pos, x.abs() + 0.01, None).view(T, M)
+    assert bool((y[:, 37] == float("inf")).all())

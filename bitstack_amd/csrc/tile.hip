@@ -648,17 +648,28 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
         if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || (I[0] <= 2 && tiles == 1 && steps == 1)) best.grid = 0;
     }
     // The rebuild's start costs 1.2 us more than reconstruct_tile_kernel's (226 x 896, 1 block 3.6 / 5.1; 1270 x 2688, 2 blocks 5.8 / 6.4), which a single tile
-    // does not win back up to a dozen blocks (556 x 384, 9 blocks 7.8 / 8.7; 257 x 384, 16 10.8 / 9.7), nor two tiles of three blocks (2304 x 2048, with
-    // its product of 775 tokens 30.4 / 31.4); longer runs do (6144 x 4096, 3 blocks, runs of 3, 18.9 / 16.5).
+    // does not win back up to a dozen blocks (556 x 384, 9 blocks 7.8 / 8.7; 257 x 384, 16 10.8 / 9.7), nor two tiles of up to four blocks (2304 x 2048, 3,
+    // with its product of 775 tokens 30.4 / 31.4; 768 x 7296, 4, 1104 tokens 37.7 / 39.4) or, one patch per wave, of a dozen (748 x 4352, 9, 656 tokens
+    // 29.2 / 30.4; 567 x 4608, 8, 144 tokens 28.4 / 28.6); more work per workgroup does (6144 x 4096, 3 blocks, runs of 3, 18.9 / 16.5; 2623 x 2944, 5
+    // blocks, 144 tokens, runs of 2, 28.1 / 26.3).  And with five to eight strips of 128 columns reconstruct_tile_kernel has one strip per XCD and is the
+    // faster one for a few blocks until a workgroup here has about ten patches per wave (144 tokens: 10743 x 896, 2 blocks 22.5 / 27.2, 17030 x 768,
+    // 3 blocks 26.3 / 29.8, 20000 x 896, 2 blocks, 425 tokens 35.3 / 39.0; beyond: 22638 x 896, 2 blocks 30.3 / 28.2; 4 strips: 17030 x 512, 2 blocks 22.0 / 19.8;
+    // 9 strips: 10505 x 1152, 2 blocks 32.5 / 29.3).
     if (T == 0 && best.grid != 0) {
         int64_t longest = 0;
-        int most = 0;
+        int most = 0, np = 0;
+        double patches = 0;                          // per wave of the busiest matrix's workgroups, on average
         for (int j = 0; j < n; j++) {
-            const int64_t run = bs_cdiv(bs_cdiv(M[j], TL_ROWS), best.wgs[j]);
+            const int64_t tiles = bs_cdiv(M[j], TL_ROWS), run = bs_cdiv(tiles, best.wgs[j]);
             if (run > longest) longest = run;
             if (I[j] > most) most = I[j];
+            if (best.np[j] > np) np = best.np[j];
+            const double each = (double)tiles * best.np[j] / best.wgs[j];
+            if (each > patches) patches = each;
         }
-        if ((longest == 1 && most <= 12) || (longest == 2 && most < 4)) best.grid = 0;
+        const int64_t strips = N / SF_COLS;
+        if ((longest == 1 && most <= 12) || (longest == 2 && (most <= 4 || (np == 1 && most <= 12))) || (strips > 4 && strips <= 8 && most <= 3 && patches <= 10.))
+            best.grid = 0;
     }
     return best;
 }

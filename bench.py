@@ -124,7 +124,7 @@ def e2e_decode_70b(torch, dev, batch=8, prompt_len=2048, new_tokens=128):
     """Random-init Llama-3.1-70B-shape model, about 30 GB of weights, `batch` sequences in
     lock step: the prompt in one pass (every linear sees batch * prompt_len tokens: rebuild +
     dense kernels; causal attention is torch's), then greedy decode (every linear sees `batch`
-    tokens: from five on that is the strip kernel, weight patches rebuilt in registers and
+    tokens: from five on that is the tile kernel, weight patches rebuilt in registers and
     multiplied at once), one HIP-graph replay per step."""
     from bitstack_amd.utils.llama_decode import LLAMA_70B, SyntheticLlamaDecoder, synthetic_compression_config
     cfg, total = synthetic_compression_config(LLAMA_70B, 30e9, lo=1, hi=8)
@@ -600,7 +600,7 @@ def main():
         detail += [{"M": L.M, "N": L.N, "I": L.I, "T": 4, "bytes": L.bytes, "us": round(ms * 1e3, 2),
                     "GBps": round(L.bytes / (ms * 1e-3) / 1e9, 1)} for L, ms in zip(l4, per4)]
         del l4
-        # ------------------------------------------------------------ T = 16 sweep (strip kernel: batched decode)
+        # ------------------------------------------------------------ T = 16 sweep (tile kernel: batched decode)
         l16 = build_sweep(16)
         _, per16 = time_sweep(l16, max(3, a.steps // 2), 1, per_layer_events=True, warm_ms=SIDE_WARM_MS)
         b16 = sum(L.bytes for L in l16)
@@ -617,7 +617,7 @@ def main():
     if not a.no_extras:
         out["decode_8b"] = e2e_decode(torch, dev)
         torch.cuda.empty_cache()
-        # 70B shape: batch 8 with 2048-token prompts (one-pass prefill, strip kernel), then batch 1 (GEMV)
+        # 70B shape: batch 8 with 2048-token prompts (one-pass prefill, tile kernel), then batch 1 (GEMV)
         out["decode_70b"] = e2e_decode_70b(torch, dev, batch=8, prompt_len=2048)
         torch.cuda.empty_cache()
         out["decode_70b_batch1"] = e2e_decode_70b(torch, dev, batch=1, prompt_len=16)

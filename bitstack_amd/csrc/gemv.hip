@@ -851,7 +851,7 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     r.n_in = N;
     r.eps = eps;
     float *parts[GEMV_MAX_GROUP];
-    // The tile kernel where it takes the matrices; the strip kernels for ranks below 16, very long stacks and u off a 16-byte boundary.
+    // The tile kernel (from 49 tokens the column kernel) where it takes the matrices; the strip and panel kernels for ranks below 16, long stacks, small matrices and u off a 16-byte boundary.
     int column_groups[GEMV_MAX_GROUP];
     bool tiles = bs_tile_partials(a.I, a.M, a.n, N, K, T, column_groups);
     for (int j = 0; j < a.n; j++) tiles = tiles && bs_aligned(a.u[j], 16);

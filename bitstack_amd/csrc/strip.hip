@@ -16,6 +16,9 @@
 // [strip, T, M] (fp32); the reduce kernel of the decode path adds them in strip order
 // and applies bias and epilogue.
 //
+// At rank 16 with u on a 16-byte boundary the tile kernel (tile.hip, up to 48 tokens) and the column kernel (column.hip, from 49) take most
+// calls; what runs here are other ranks, stacks beyond their registers, small or awkwardly cut matrices (make_tile_plan, CL_MIN_WEIGHTS).
+//
 // Cost per 16 x 16 patch and block: the same 6 to 7 VALU operations as the rebuild, no store
 // of w (two thirds of the rebuild's bytes) and no second pass that reads it back; the
 // token count only adds one MFMA per patch and 16 tokens, after the last block.

@@ -106,7 +106,12 @@ int64_t bs_workspace_bytes(int I, int M, int N, int K, int T);
  * 128 tokens and 8 blocks (N % 128 == 0), the panel kernel: 128 x 128 tiles of
  * the weight decoded into LDS strip by strip and multiplied on the matrix
  * cores at once, the weight never stored; larger T rebuilds the weight once
- * into `workspace` and runs a dense MFMA GEMM.  Requires
+ * into `workspace` and runs a dense MFMA GEMM.  At K == 16 (u 16-byte aligned)
+ * the strip kernel's calls mostly run as the tile kernel (the same rebuild, 32 x 32
+ * outputs per matrix instruction, a wave keeps its columns while the rows pass
+ * by), also T = 3 and 4 on matrices of two blocks and 1 MiB of sign bytes or
+ * more, there with the weight in two fp16 terms; from 11 Mi weights 49 <= T <=
+ * 128 runs as the column kernel (the same, a workgroup keeps its rows).  Requires
  * N % 8 == 0.  `workspace` must hold bs_workspace_bytes(...) bytes, 256-byte
  * aligned; its contents on entry do not matter and it may be reused by the
  * next call on the same stream.
@@ -176,11 +181,11 @@ int bs_decode_kernel(int I, int M, int N, int K, int T);
  * bitstack/modules/BitStackLinear.py:116-157).
  */
 #define BS_PATH_REBUILD    0   /* weight rebuilt into the workspace, then the dense product */
-#define BS_PATH_DECODE_F16 1   /* gemv_kernel: packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass */
+#define BS_PATH_DECODE_F16 1   /* gemv_kernel: packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass (3 and 4 on large matrices: tile_forward_kernel) */
 #define BS_PATH_DECODE_MX  2   /* gemv_mx_kernel: the same on the block-scaled fp4 x fp6 MFMA, 1..2 tokens */
-#define BS_PATH_STRIP      3   /* strip_forward_kernel: up to 48 tokens, patches rebuilt in registers */
-#define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups */
-#define BS_PATH_PANEL      5   /* panel_forward_kernel: up to 128 tokens, W tiles decoded into LDS */
+#define BS_PATH_STRIP      3   /* up to 48 tokens, patches rebuilt in registers: tile_forward_kernel at rank 16, strip_forward_kernel elsewhere */
+#define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups (large matrices: column_forward_kernel) */
+#define BS_PATH_PANEL      5   /* panel_forward_kernel: up to 128 tokens, W tiles decoded into LDS (large matrices: column_forward_kernel) */
 int bs_forward_path(int I, int M, int N, int K, int T);
 
 /*

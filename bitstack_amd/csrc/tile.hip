@@ -641,11 +641,13 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     // rows and strips happen to fill the chip; us strip / this: 7286 x 1024, 11 blocks (2 steps, runs of 4) 18.6 / 21.2, 3328 x 1664, 16 (2, 3) 20.3 / 23.7,
     // 3366 x 2688, 11 (4, 5) 25.6 / 23.1, 2440 x 1536, 14 (2, 2) 20.4 / 17.0, 20191 x 256, 11 (6, 3) 29.4 / 15.5.  And where either does one tile or step of
     // one or two blocks: the hand-over between the waves is half a us (896 x 2176, 1 block 6.8 / 7.5; 643 x 896, 2 blocks 8.4 / 8.9; from 3 blocks
-    // on level or ahead).
+    // on level or ahead; with two patches per wave the one tile is the longer chain: 2668 x 896, 5 blocks 8.4 / 9.9, 3345 x 640, 3 7.8 / 8.6, 2019 x 1664, 3
+    // 8.0 / 8.6, against two steps 4398 x 1536, 4 13.1 / 10.2.  Not for three and four tokens at N % 512 == 0, where a decode kernel is the other one).
     if (T > 0 && n == 1 && best.grid != 0) {
         const int64_t tiles = bs_cdiv(bs_cdiv(M[0], TL_ROWS), best.wgs[0]);
-        const long steps = best.np[0] == 1 || I[0] <= 2 ? bs_strip_steps(I[0], M[0], N, T) : 0;
-        if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || (I[0] <= 2 && tiles == 1 && steps == 1)) best.grid = 0;
+        const bool wide = best.np[0] == 2 && (T > 4 || N % 512 != 0);
+        const long steps = best.np[0] == 1 || I[0] <= 2 || wide ? bs_strip_steps(I[0], M[0], N, T) : 0;
+        if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || ((I[0] <= 2 || wide) && tiles == 1 && steps == 1)) best.grid = 0;
     }
     // The rebuild's start costs 1.2 us more than reconstruct_tile_kernel's (226 x 896, 1 block 3.6 / 5.1; 1270 x 2688, 2 blocks 5.8 / 6.4), which a single tile
     // does not win back up to a dozen blocks (556 x 384, 9 blocks 7.8 / 8.7; 257 x 384, 16 10.8 / 9.7), nor two tiles of up to four blocks (2304 x 2048, 3,

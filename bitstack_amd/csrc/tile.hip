@@ -449,9 +449,7 @@ struct TileKernel {
                     asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
                     first_block();                               // of tile n + 1
                 } else if constexpr (SPLIT) {
-                    // Two terms per weight: rounded towards zero (a finite weight stays finite), and what that leaves (2^-21 of the weight is lost).  An
-                    // infinite weight leaves the difference of two infinities, a NaN, for which the maximum takes a finite number.  The lanes
-                    // trade places as below.
+                    // Two terms per weight: rounded towards zero, and what that leaves (2^-21 of the weight is lost).  The lanes trade places as below.
 #pragma unroll
                     for (int r = 0; r < 2; r++) y[0][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -461,8 +459,7 @@ struct TileKernel {
                         for (int k = 0; k < 8; k++) {
                             const float a = acc[p][2 * k], b = acc[p][2 * k + 1];
                             t[0][k] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-                            const half2_t rest = {(half_t)__builtin_fmaf((float)t[0][k][0], -1.f, a), (half_t)__builtin_fmaf((float)t[0][k][1], -1.f, b)};
-                            t[1][k] = __builtin_elementwise_max(rest, (half2_t){(half_t)-65504.f, (half_t)-65504.f});
+                            t[1][k] = (half2_t){(half_t)__builtin_fmaf((float)t[0][k][0], -1.f, a), (half_t)__builtin_fmaf((float)t[0][k][1], -1.f, b)};
                         }
 #pragma unroll
                         for (int term = 0; term < 2; term++) {
@@ -477,6 +474,31 @@ struct TileKernel {
                             y[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), y[0][0], 0, 0, 0);
                             y[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), y[0][1], 0, 0, 0);
                         }
+                    }
+                    // A weight that the terms cannot hold (beyond 131008, or infinite) leaves an infinity or a NaN in the second one, whatever its sign, and
+                    // so in every y of its row.  Such y come from the fp32 weights instead.
+                    float any = 0.f;
+#pragma unroll
+                    for (int r = 0; r < 2; r++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) any += y[0][r][j];
+                    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(any)) != 0, 0)) {
+                        float4_t full[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                        for (int p = 0; p < NP; p++)
+#pragma unroll
+                            for (int k = 0; k < 8; k++) {
+                                const float a = acc[p][k], b = acc[p][8 + k];
+                                const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                                const uint32_t lo = w[0], hi = w[1];
+                                full[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, lo), full[0], 0, 0, 0);
+                                full[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, hi), full[1], 0, 0, 0);
+                            }
+#pragma unroll
+                        for (int r = 0; r < 2; r++)
+#pragma unroll
+                            for (int j = 0; j < 4; j++)
+                                if (!__builtin_isfinite(y[0][r][j])) y[0][r][j] = full[r][j];
                     }
                     first_block();                   // of tile n + 1
                 } else {

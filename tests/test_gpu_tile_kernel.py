@@ -228,6 +228,44 @@ def test_three_and_four_tokens_with_non_finite_inputs_and_large_weights(T):
     assert bool((y[..., 5] == 0.25 * (102400 + 32)).all()), y[..., 5]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4])
+@pytest.mark.parametrize("I,M,N", [(3, 2800, 1024), (2, 8300, 512), (6, 1000, 4096), (12, 4096, 512)])
+def test_three_and_four_tokens_with_weights_beyond_fp16(I, M, N, T):
+    """Weights of either sign on both sides of 65504 and of 131008, where two fp16 terms end, and far beyond: y is a finite fp16 number and has to be
+    right, in rows beside each other and alone in their tile, and every other row keeps its bits."""
+    print(f"large weights I={I} M={M} N={N} T={T}", flush=True)
+    (q, u, vt, x, _), _ = _args(I, M, N, T, False)
+    x = (x.float() * 2.0 ** -20).half()
+    vt[0], u[0] = 448.0, 0.0                             # a weight of block 0 is 7168 u[0, row, 0], of random sign
+    clean = IU.bitstack_forward_hip(q, u, vt, x, None)
+    rows = [3, 4, 5, 37, 40, 64, 71, M - 2]
+    for row, value in zip(rows, (9.0, -9.5, 18.0, -18.5, 28.0, -28.0, 20000.0, -20000.0)):
+        u[0, row] = value
+    y = IU.bitstack_forward_hip(q, u, vt, x, None)
+    keep = torch.ones(M, dtype=torch.bool, device="cuda")
+    keep[rows] = False
+    assert torch.equal(y[..., keep], clean[..., keep])
+    sign = ((q.view(I, M, N // 8, 1)[:, rows] >> torch.arange(7, -1, -1, device="cuda", dtype=torch.uint8)) & 1).reshape(I, len(rows), N)
+    w = torch.zeros(len(rows), N, dtype=torch.float64, device="cuda")
+    for i in range(I):
+        p = u[i, rows].double() @ vt[i].double()
+        w += torch.where(sign[i].bool(), p, -p)
+    assert float(w.min()) < -1e8 and float(w.max()) > 1e8
+    xd = x.view(T, N).double()
+    want, size = xd @ w.t().contiguous(), xd.abs() @ w.abs().t().contiguous()
+    # one rounding of y; fp32 sums of I blocks and over the columns (32 at a time), weights to 2^-21
+    assert bool(((y.view(T, M)[:, rows].double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -15 + 2.0 ** -25).all())
+    # infinite weights stay infinite and keep their sign, a NaN stays one, and their neighbours keep their bits
+    ones, x = torch.full_like(q, 0xFF), x.abs() + 2.0 ** -14
+    u[0, 36:39] = 0.0
+    clean = IU.bitstack_forward_hip(ones, u, vt, x, None).view(T, M)
+    u[0, 36], u[0, 37], u[0, 38] = float("inf"), float("-inf"), float("nan")
+    y = IU.bitstack_forward_hip(ones, u, vt, x, None).view(T, M)
+    assert bool((y[:, 36] == float("inf")).all()) and bool((y[:, 37] == float("-inf")).all()) and bool(y[:, 38].isnan().all())
+    assert torch.equal(y[:, :36], clean[:, :36]) and torch.equal(y[:, 39:], clean[:, 39:])
+
+
 # 49 to 128 tokens: the column kernel from 11 Mi weights on.  Both sides of its token tiles and block limits, rows about whole workgroups of 256,
 # half a span of columns at the end, one span and many per workgroup
 COLUMNS = [(1, 11300, 1024, 49), (2, 12033, 1024, 64), (8, 2816, 4096, 64), (8, 2817, 4224, 50), (3, 30977, 384, 65), (7, 2815, 4352, 96), (5, 90200, 128, 80),

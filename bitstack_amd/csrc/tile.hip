@@ -449,9 +449,12 @@ struct TileKernel {
                     asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
                     first_block();                               // of tile n + 1
                 } else if constexpr (SPLIT) {
-                    // Two terms per weight: rounded towards zero, and what that leaves (2^-21 of the weight is lost).  The lanes trade places as below.
+                    // Two terms per weight: rounded towards zero, and 2^18 times what that leaves, in sums of its own, so that it is no subnormal number where
+                    // the weight is small (lost: 2^-21 of a weight, 2^-12 of one below 2^-24, and never less than 2^-44).  The lanes trade places as below.
+                    constexpr float UP = 262144.f;
+                    float4_t rest[2];
 #pragma unroll
-                    for (int r = 0; r < 2; r++) y[0][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+                    for (int r = 0; r < 2; r++) y[0][r] = rest[r] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int p = 0; p < NP; p++) {
                         half2_t t[2][8];
@@ -459,10 +462,10 @@ struct TileKernel {
                         for (int k = 0; k < 8; k++) {
                             const float a = acc[p][2 * k], b = acc[p][2 * k + 1];
                             t[0][k] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-                            t[1][k] = (half2_t){(half_t)__builtin_fmaf((float)t[0][k][0], -1.f, a), (half_t)__builtin_fmaf((float)t[0][k][1], -1.f, b)};
+                            t[1][k] = (half2_t){(half_t)__builtin_fmaf((float)t[0][k][0], -UP, UP * a), (half_t)__builtin_fmaf((float)t[0][k][1], -UP, UP * b)};
                         }
 #pragma unroll
-                        for (int term = 0; term < 2; term++) {
+                        for (int term = 1; term >= 0; term--) {
                             uint4_t lo, hi;
 #pragma unroll
                             for (int k = 0; k < 4; k++) {
@@ -471,17 +474,21 @@ struct TileKernel {
                                 lo[k] = r[0];
                                 hi[k] = r[1];
                             }
-                            y[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), y[0][0], 0, 0, 0);
-                            y[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), y[0][1], 0, 0, 0);
+                            float4_t (&sum)[2] = term == 0 ? y[0] : rest;
+                            sum[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), sum[0], 0, 0, 0);
+                            sum[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), sum[1], 0, 0, 0);
                         }
                     }
-                    // A weight that the terms cannot hold (beyond 131008, or infinite) leaves an infinity or a NaN in the second one, whatever its sign, and
-                    // so in every y of its row.  Such y come from the fp32 weights instead.
+                    // A weight that the terms cannot hold (from about 256 on, where 2^18 * 2^-10 of it is beyond fp16, or infinite) leaves an infinity or
+                    // a NaN in the second one, whatever its sign, and so in every y of its row.  Such y come from the fp32 weights instead.
                     float any = 0.f;
 #pragma unroll
                     for (int r = 0; r < 2; r++)
 #pragma unroll
-                        for (int j = 0; j < 4; j++) any += y[0][r][j];
+                        for (int j = 0; j < 4; j++) {
+                            any += rest[r][j];
+                            y[0][r][j] = __builtin_fmaf(rest[r][j], 1.f / UP, y[0][r][j]);
+                        }
                     if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(any)) != 0, 0)) {
                         float4_t full[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll

@@ -230,7 +230,7 @@ def test_three_and_four_tokens_with_non_finite_inputs_and_large_weights(T):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [3, 4])
-@pytest.mark.parametrize("I,M,N", [(3, 2800, 1024), (2, 8300, 512), (6, 1000, 4096), (12, 4096, 512)])
+@pytest.mark.parametrize("I,M,N", [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (12, 4096, 512)])
 def test_three_and_four_tokens_with_weights_beyond_fp16(I, M, N, T):
     """Weights of either sign on both sides of 65504 and of 131008, where two fp16 terms end, and far beyond: y is a finite fp16 number and has to be
     right, in rows beside each other and alone in their tile, and every other row keeps its bits."""
@@ -264,6 +264,27 @@ def test_three_and_four_tokens_with_weights_beyond_fp16(I, M, N, T):
     y = IU.bitstack_forward_hip(ones, u, vt, x, None).view(T, M)
     assert bool((y[:, 36] == float("inf")).all()) and bool((y[:, 37] == float("-inf")).all()) and bool(y[:, 38].isnan().all())
     assert torch.equal(y[:, :36], clean[:, :36]) and torch.equal(y[:, 39:], clean[:, 39:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4])
+@pytest.mark.parametrize("I,M,N", [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (16, 2100, 1536)])
+def test_three_and_four_tokens_with_weights_of_every_size(I, M, N, T):
+    """Rows with weights from about 0.1 down to 1e-9 beside each other: the second term holds what the first one leaves of a small weight too, so no row stands further
+    from float64 than the rounding of its y."""
+    print(f"weights of every size I={I} M={M} N={N} T={T}", flush=True)
+    (q, u, vt, x, _), _ = _args(I, M, N, T, False)
+    power = torch.arange(M, device="cuda") % 14
+    u = (u.float() * 2.0 ** 6 * torch.pow(4.0, -power.float()).view(1, M, 1)).half()
+    x = (x.float() * 2.0 ** 9).half()
+    want = torch.from_numpy(C.forward_f64(q.cpu().numpy(), u.cpu().numpy(), vt.cpu().numpy(), x.cpu().numpy())).cuda().view(T, M)
+    y = IU.bitstack_forward_hip(q, u, vt, x, None).view(T, M).double()
+    for p in range(14):
+        # One rounding of y to fp16, and of the weights at most 2^-12 at random (below 2^-24, where the first term is nothing), so 2^-12 of y too: the
+        # two add up as squares.  The fp32 sums are a hundredth of that.
+        d, rounding = (y - want)[:, power == p].norm(), (want.half().double() - want)[:, power == p].norm()
+        lost = (2.0 ** -21 if p < 5 else 2.0 ** -12) * want[:, power == p].norm()
+        assert d <= 1.01 * torch.hypot(rounding, lost), (p, float(d / rounding))
 
 
 # 49 to 128 tokens: the column kernel from 11 Mi weights on.  Both sides of its token tiles and block limits, rows about whole workgroups of 256,

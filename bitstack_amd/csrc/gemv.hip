@@ -827,8 +827,10 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
         if (I[j] < 2 || (int64_t)I[j] * M[j] * (N / 8) < (1 << 20)) return false;
         if ((T == 3 && large && I[j] < 6) || (I[j] == 2 && N >= 4096)) return false;
     }
-    int groups[GEMV_MAX_GROUP];
-    return bs_tile_partials(I, M, n, N, K, T, groups);
+    // (never with more partial sums than bs_forward_static's scratch holds: long stacks take 256 columns per workgroup, 16 blocks of 17317 x 111104, 3 tokens 86 MiB
+    // where the factor-through kernel needs 6)
+    const int64_t floats = tile_part_floats(I, M, n, N, K, T);
+    return floats > 0 && floats * (int64_t)sizeof(float) <= BS_STATIC_SCRATCH_BYTES;
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group

@@ -95,6 +95,13 @@ def test_workspace_bytes(L):
         assert T * 4096 * 4 <= b <= 32 * (T * 4096 * 4 + T * 4) + 256
 
 
+@pytest.mark.parametrize("I,M,N,T", [(14, 19647, 67584, 4), (13, 12354, 87552, 4), (16, 17317, 111104, 3), (12, 27516, 76288, 3), (16, 24291, 74752, 4)])
+def test_long_stacks_at_three_and_four_tokens_fit_the_static_scratch(L, I, M, N, T):
+    """bs_forward_static refuses what needs more than its array: a call whose factor-through kernel needs 6 to 24 MiB must not be given to a
+    kernel that needs 66 to 128."""
+    assert 0 < L.bs_workspace_bytes(I, M, N, 16, T) <= _lib.STATIC_SCRATCH_BYTES
+
+
 def test_kernel_hooks_belong_to_the_calling_thread(L):
     """A hook set on one thread moves neither the plan nor the workspace size another thread sees."""
     import threading

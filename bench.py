@@ -356,7 +356,7 @@ def main():
             tp = sum(perp) * 1e-3
             pre[f"T{T}"] = {"useful_tflops": round(useful / tp / 1e12, 1),
                             "frac_of_f16_mfma_peak": round(useful / tp / 1e12 / MFMA_F16_PEAK_TFLOPS, 4)}
-            pre[f"T{T}"]["kernels"] = sorted({_lib.PATH_NAMES[int(lib.bs_forward_path(L.I, L.M, L.N, 16, L.T))] for L in lp})
+            pre[f"T{T}"]["kernels"] = sorted({_lib.forward_kernel_name(L.I, L.M, L.N, 16, L.T) for L in lp})
             if T >= 512:
                 # beside it, timed the same way (the four layers in turn, events around each call): the same
                 # forwards with the vendor GEMM (hipBLASLt) behind the rebuild - a comparator, never the headline
@@ -406,8 +406,7 @@ def main():
         print(json.dumps({"one_layer": {"M": M, "N": N, "I": I, "T": T, "algorithmic_bytes": copies[0].bytes,
                                         "us_per_forward": round(us, 2), "GBps": round(copies[0].bytes / us / 1e3, 1),
                                         "decode_plan": _lib.decode_plan(I, M, N, 16, T),
-                                        "decode_kernel": {0: "none", 1: "gemv_kernel (fp16 MFMA)", 2: "gemv_mx_kernel (fp4 x fp6 MFMA)"}[
-                                            lib.bs_decode_kernel(I, M, N, 16, T)]}}))
+                                        "kernel": _lib.forward_kernel_name(I, M, N, 16, T)}}))
         return
     if a.only == "sweep_tokens":
         # the 20-layer sweep at --tokens tokens per forward, events around every forward: the process to trace for
@@ -418,7 +417,7 @@ def main():
         print(json.dumps({"sweep_tokens": {"tokens": a.tokens, "us_per_pass": round(sum(per) * 1e3, 1),
                                            "GBps": round(bt / (sum(per) * 1e-3) / 1e9, 1),
                                            "layers": [{"M": L.M, "N": L.N, "I": L.I, "us": round(ms * 1e3, 2),
-                                                       "kernel": _lib.PATH_NAMES[int(lib.bs_forward_path(L.I, L.M, L.N, 16, L.T))]}
+                                                       "kernel": _lib.forward_kernel_name(L.I, L.M, L.N, 16, L.T)}
                                                       for L, ms in zip(lt, per)]}}))
         return
     if a.only == "copy":
@@ -463,6 +462,9 @@ def main():
     def kernel_name(L):
         waves, r, grid, _ = _lib.decode_plan(L.I, L.M, L.N, 16, L.T)
         path = int(lib.bs_forward_path(L.I, L.M, L.N, 16, L.T))
+        kind, _ = _lib.tile_kernel([(L.I, L.M)], L.N, 16, L.T)
+        if kind != _lib.TILE_NONE:
+            return _lib.TILE_NAMES[kind], 0
         if path == _lib.PATH_DECODE_MX:
             return "gemv_mx_kernel<R=%d>" % r, grid
         if path == _lib.PATH_DECODE_F16:
@@ -592,11 +594,14 @@ def main():
         l4 = build_sweep(4)
         _, per4 = time_sweep(l4, max(3, a.steps // 2), 1, per_layer_events=True, warm_ms=SIDE_WARM_MS)
         b4 = sum(L.bytes for L in l4)
-        flops4 = sum(2.0 * 16 * L.I * L.M * L.N * L.T for L in l4)
         t4 = sum(per4) * 1e-3
-        out["t4"] = {"GBps": round(b4 / t4 / 1e9, 1), "kernels": sorted({kernel_name(L)[0] for L in l4}),
-                     "mfma_tflops_issued": round(flops4 / t4 / 1e12, 1),
-                     "frac_of_f16_mfma_peak": round(flops4 / t4 / 1e12 / MFMA_F16_PEAK_TFLOPS, 4)}
+        out["t4"] = {"GBps": round(b4 / t4 / 1e9, 1), "kernels": sorted({kernel_name(L)[0] for L in l4})}
+        # 16 products per sign and token: what gemv_kernel issues, over the layers that run on it (the tile kernel issues one weight for all tokens)
+        through = [(L, ms) for L, ms in zip(l4, per4) if kernel_name(L)[0].startswith("gemv_kernel")]
+        if through:
+            issued = sum(2.0 * 16 * L.I * L.M * L.N * L.T for L, _ in through) / (sum(ms for _, ms in through) * 1e-3) / 1e12
+            out["t4"]["gemv_kernel"] = {"layers": len(through), "mfma_tflops_issued": round(issued, 1),
+                                        "frac_of_f16_mfma_peak": round(issued / MFMA_F16_PEAK_TFLOPS, 4)}
         detail += [{"M": L.M, "N": L.N, "I": L.I, "T": 4, "bytes": L.bytes, "us": round(ms * 1e3, 2),
                     "GBps": round(L.bytes / (ms * 1e-3) / 1e9, 1)} for L, ms in zip(l4, per4)]
         del l4

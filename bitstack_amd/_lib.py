@@ -35,6 +35,7 @@ SIGNATURES = {
     "bs_set_dense_kernel": (_I, [_I]),
     "bs_set_prefill_kernel": (_I, [_I]),
     "bs_forward_path": (_I, [_I, _I, _I, _I, _I]),
+    "bs_tile_kernel": (_I, [_P, _P, _I, _I, _I, _I, _P]),
 }
 DECODE_AUTO, DECODE_F16, DECODE_MX = 0, 1, 2
 DENSE_AUTO, DENSE_OWN, DENSE_LIBRARY = 0, 1, 2
@@ -42,8 +43,10 @@ PREFILL_AUTO, PREFILL_REBUILD, PREFILL_WALKED, PREFILL_PANEL = 0, 1, 2, 3
 PATH_NAMES = {0: "rebuild + dense", 1: "gemv_kernel (fp16 MFMA)", 2: "gemv_mx_kernel (fp4 x fp6 MFMA)", 3: "strip_forward_kernel",
               4: "strip_wide_kernel", 5: "panel_forward_kernel"}
 PATH_REBUILD, PATH_DECODE_F16, PATH_DECODE_MX, PATH_STRIP, PATH_WALKED, PATH_PANEL = range(6)
+TILE_NONE, TILE_FORWARD, TILE_TWO_TERMS, TILE_COLUMN, TILE_REBUILD = range(5)
+TILE_NAMES = {TILE_FORWARD: "tile_forward_kernel", TILE_TWO_TERMS: "tile_forward_kernel (weight in two fp16 terms)",
+              TILE_COLUMN: "column_forward_kernel", TILE_REBUILD: "rebuild (tile_forward_kernel) + dense"}
 STATIC_SCRATCH_BYTES = 64 << 20
-
 
 
 class bs_matrix(ctypes.Structure):
@@ -102,6 +105,22 @@ def decode_plan(I, M, N, K, T):
     vals = [ctypes.c_int(0) for _ in range(4)]
     check(lib().bs_decode_plan(I, M, N, K, T, *[ctypes.byref(v) for v in vals]), "bs_decode_plan")
     return tuple(v.value for v in vals)
+
+
+def tile_kernel(layers, N, K, T):
+    """(TILE_*, columns per workgroup of each matrix) for one or several (blocks, out features) on the same x."""
+    n = len(layers)
+    I, M, columns = (ctypes.c_int * n)(*(i for i, _ in layers)), (ctypes.c_int * n)(*(m for _, m in layers)), (ctypes.c_int * n)()
+    kind = int(lib().bs_tile_kernel(I, M, n, N, K, T, columns))
+    check(min(kind, 0), "bs_tile_kernel")
+    return kind, list(columns)
+
+
+def forward_kernel_name(I, M, N, K, T):
+    """The kernel that a forward of these dimensions runs on, u being 16-byte aligned."""
+    path = int(lib().bs_forward_path(I, M, N, K, T))
+    check(min(path, 0), "bs_forward_path")
+    return TILE_NAMES.get(tile_kernel([(I, M)], N, K, T)[0], PATH_NAMES[path])
 
 
 def linear_plan(T, M, N):

@@ -95,6 +95,19 @@ extern "C" int bs_forward_path(int I, int M, int N, int K, int T) {
     return bs_gemv_forward_path(I, M, N, K, T);
 }
 
+extern "C" int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
+    if (!I || !M || !columns) return BS_ERR_NULL;
+    if (n < 1 || n > BS_MAX_GROUP) return BS_ERR_SHAPE;
+    bool empty = T == 0;
+    for (int j = 0; j < n; j++) {
+        const int st = forward_dims(I[j], M[j], N, K, T);
+        if (st != BS_OK) return st;
+        empty = empty || I[j] == 0;
+        columns[j] = 0;
+    }
+    return empty ? BS_TILE_NONE : bs_gemv_tile_kernel(I, M, n, N, K, T, columns);
+}
+
 static int forward_impl(const uint8_t *packed, const void *u, const void *vt, const void *x,
                         const void *bias, void *y, int I, int M, int N, int K, int T,
                         void *workspace, int64_t workspace_bytes, void *stream, bool library_ok) {

@@ -274,6 +274,9 @@ int bs_column_partials(int I, int M, int N, int K, int T) {
     return make_column_plan(M, N).groups;
 }
 
+// ... and the columns of one.
+int bs_column_width(int I, int M, int N, int K, int T) { return bs_column_partials(I, M, N, K, T) > 0 ? 256 * make_column_plan(M, N).spans : 0; }
+
 int bs_launch_column(const uint8_t *packed, const half_t *u, const half_t *vt, int I, int M, float *part, const half_t *x, int N, int K, int T, hipStream_t s) {
     const int groups = bs_column_partials(I, M, N, K, T);
     if (groups == 0 || !bs_aligned(x, 16) || !bs_aligned(packed, 16) || !bs_aligned(vt, 16) || !bs_aligned(u, 16)) return BS_ERR_SHAPE;

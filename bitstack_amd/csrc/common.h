@@ -79,6 +79,7 @@ int64_t bs_gemv_workspace_bytes(int I, int M, int N, int K, int T);
 void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave, int *grid, int *kmax);
 int bs_gemv_plan_kernel(int I, int M, int N, int K, int T);
 int bs_gemv_forward_path(int I, int M, int N, int K, int T);
+int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns);
 int bs_gemv_set_kernel(int mode);
 // epilogues of the grouped decode forward (values of BS_EPI_* in the public header)
 enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2 };
@@ -100,11 +101,13 @@ int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *con
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s);
+bool bs_tile_columns(const int *I, const int *M, int n, int N, int K, int T, int *columns);
 // the same kernel's rebuilt weights (BS_ERR_SHAPE: not taken, nothing enqueued)
 int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                            half_t *const *w, int N, int K, hipStream_t s);
 // column kernel (column.hip): 49 to 128 tokens of one matrix, reached through the two functions above
 int bs_column_partials(int I, int M, int N, int K, int T);
+int bs_column_width(int I, int M, int N, int K, int T);
 int bs_launch_column(const uint8_t *packed, const half_t *u, const half_t *vt, int I, int M, float *part, const half_t *x, int N, int K, int T, hipStream_t s);
 // panel kernel (panel.hip): the same partial sums for up to 128 tokens, sign tiles decoded into LDS and
 // multiplied on the matrix cores at once; bs_panel_partials = column groups (0: the shape is not taken)

@@ -1026,6 +1026,16 @@ int bs_gemv_forward_path(int I, int M, int N, int K, int T) {
     return make_plan(&I, &M, 1, N, K, pass_tokens(T)).mx ? BS_PATH_DECODE_MX : BS_PATH_DECODE_F16;
 }
 
+// Which call of the tile and column kernels serves these matrices, with u on 16-byte boundaries (values of BS_TILE_* in the public header).
+int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
+    const int path = group_path(I, M, n, N, K, T);
+    if (path == 1 && (n == 1 || T <= 48)) return !bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_NONE : T > 48 ? BS_TILE_COLUMN : BS_TILE_FORWARD;
+    if (path == 0) return split_tiles(I, M, n, N, K, T) && bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_TWO_TERMS : BS_TILE_NONE;
+    for (int j = 0; j < n; j++)
+        if (bs_gemv_forward_path(I[j], M[j], N, K, T) != BS_PATH_REBUILD) return BS_TILE_NONE;
+    return bs_tile_columns(I, M, n, N, K, 0, columns) ? BS_TILE_REBUILD : BS_TILE_NONE;
+}
+
 // 0: not a decode-kernel shape, 1: gemv_kernel (fp16 MFMA), 2: gemv_mx_kernel (block-scaled fp4 x fp6 MFMA)
 int bs_gemv_plan_kernel(int I, int M, int N, int K, int T) {
     if (group_path(&I, &M, 1, N, K, T) != 0) return 0;

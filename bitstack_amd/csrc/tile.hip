@@ -742,6 +742,14 @@ bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, in
     return p.grid != 0;
 }
 
+// Columns per workgroup of every matrix where this kernel takes them (T = 0: their rebuild), else false.
+bool bs_tile_columns(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
+    if (T > 48) return n == 1 && (columns[0] = bs_column_width(I[0], M[0], N, K, T)) > 0;
+    const TilePlan p = checked_plan(I, M, n, N, K, T);
+    for (int j = 0; p.grid != 0 && j < n; j++) columns[j] = 256 * p.np[j];
+    return p.grid != 0;
+}
+
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s) {
     if (T > 48) return n == 1 && !ssq && !split ? bs_launch_column(packed[0], u[0], vt[0], I[0], M[0], part[0], x, N, K, T, s) : BS_ERR_SHAPE;

@@ -157,7 +157,9 @@ int bs_forward_static(const uint8_t *packed, const void *u, const void *vt, cons
  * strip kernel or the dense path does: more than 4 tokens with N % 128 == 0,
  * more than 8 tokens, N not a multiple of 512).  No counterpart in the reference
  * (Triton picks its configuration by autotuning,
- * bitstack/utils/inference_utils.py:8-39).
+ * bitstack/utils/inference_utils.py:8-39).  Three and four tokens for which
+ * bs_tile_kernel answers BS_TILE_TWO_TERMS run like this only with u off a
+ * 16-byte boundary; the same holds for bs_decode_kernel.
  */
 int bs_decode_plan(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave,
                    int *workgroups, int *partials_per_row);
@@ -187,6 +189,23 @@ int bs_decode_kernel(int I, int M, int N, int K, int T);
 #define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups (large matrices: column_forward_kernel) */
 #define BS_PATH_PANEL      5   /* panel_forward_kernel: up to 128 tokens, W tiles decoded into LDS (large matrices: column_forward_kernel) */
 int bs_forward_path(int I, int M, int N, int K, int T);
+
+/*
+ * Introspection for benchmarks and tests: whether the calls that bs_forward_path,
+ * bs_decode_kernel and bs_decode_plan answer for run on the tile or column kernel,
+ * which serve most calls at rank 16 with u on a 16-byte boundary (off it, the
+ * kernel that those functions name runs).  n == 1: bs_forward; n of 2 to
+ * 4: bs_forward_group[_rms] up to 48 tokens, bs_forward_cat where
+ * each matrix is rebuilt.  columns[j] receives the columns of matrix j that one workgroup
+ * takes (0 with BS_TILE_NONE).  Under the calling thread's hook settings.
+ * Negative = error status.  No counterpart in the reference.
+ */
+#define BS_TILE_NONE      0    /* no: the kernel that bs_forward_path names */
+#define BS_TILE_FORWARD   1    /* tile_forward_kernel, the weight rounded to fp16 as a stored one */
+#define BS_TILE_TWO_TERMS 2    /* tile_forward_kernel, the weight in two fp16 terms (three and four tokens) */
+#define BS_TILE_COLUMN    3    /* column_forward_kernel (49 to 128 tokens) */
+#define BS_TILE_REBUILD   4    /* the weight rebuilt by tile_forward_kernel, then the dense product */
+int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns);
 
 /*
  * Test and benchmark hook: 0 = choose the decode kernel of one- and two-token

@@ -102,6 +102,35 @@ def test_long_stacks_at_three_and_four_tokens_fit_the_static_scratch(L, I, M, N,
     assert 0 < L.bs_workspace_bytes(I, M, N, 16, T) <= _lib.STATIC_SCRATCH_BYTES
 
 
+def test_tile_kernel_says_which_kernel_a_call_runs_on(L):
+    kind = lambda layers, N, T, K=16: _lib.tile_kernel(layers, N, K, T)
+    one_token = [(8, 14336)]
+    assert kind(one_token, 4096, 1) == (_lib.TILE_NONE, [0]) and _lib.forward_kernel_name(8, 14336, 4096, 16, 1).startswith("gemv_mx_kernel")
+    assert kind([(4, 4096)], 14336, 4) == (_lib.TILE_TWO_TERMS, [1024]) and "two fp16 terms" in _lib.forward_kernel_name(4, 4096, 14336, 16, 4)
+    assert kind([(6, 5000)], 4096, 37) == (_lib.TILE_FORWARD, [512]) and _lib.forward_kernel_name(6, 5000, 4096, 16, 37) == "tile_forward_kernel"
+    assert kind([(5, 14336)], 4096, 100) == (_lib.TILE_COLUMN, [1024]) and _lib.forward_kernel_name(5, 14336, 4096, 16, 100) == "column_forward_kernel"
+    assert kind([(8, 4096)], 14336, 509) == (_lib.TILE_REBUILD, [512])
+    # groups; other ranks; no blocks; no tokens
+    group = [(3, 8192), (2, 1024), (3, 1024)]
+    assert kind(group, 8192, 8)[0] == _lib.TILE_FORWARD and kind(group, 8192, 600) == (_lib.TILE_REBUILD, [1024] * 3) and kind(group, 8192, 64)[0] == _lib.TILE_NONE
+    for T in (4, 37, 100, 509):
+        assert kind([(4, 14336)], 4096, T, 12) == (_lib.TILE_NONE, [0])
+    assert kind([(0, 4096)], 4096, 8)[0] == kind([(4, 4096)], 4096, 0)[0] == _lib.TILE_NONE
+    # under the thread's hooks
+    try:
+        L.bs_set_decode_kernel(_lib.DECODE_F16)
+        assert kind([(4, 4096)], 14336, 4)[0] == _lib.TILE_NONE
+        L.bs_set_prefill_kernel(_lib.PREFILL_REBUILD)
+        assert kind([(5, 14336)], 4096, 100)[0] == _lib.TILE_REBUILD
+    finally:
+        L.bs_set_decode_kernel(_lib.DECODE_AUTO)
+        L.bs_set_prefill_kernel(_lib.PREFILL_AUTO)
+    # errors
+    two, none = (ctypes.c_int * 2)(1, 1), ctypes.c_void_p(0)
+    assert L.bs_tile_kernel(two, two, 2, 100, 16, 8, two) == -2 and L.bs_tile_kernel(two, two, 5, 128, 16, 8, two) == -2
+    assert L.bs_tile_kernel(two, none, 2, 128, 16, 8, two) == -1 and L.bs_tile_kernel(two, two, 2, 128, 16, 8, none) == -1
+
+
 def test_kernel_hooks_belong_to_the_calling_thread(L):
     """A hook set on one thread moves neither the plan nor the workspace size another thread sees."""
     import threading

@@ -98,7 +98,7 @@ int bs_launch_strip_group(int n, const uint8_t *const *packed, const half_t *con
 // tile kernel (tile.hip; from 49 tokens the column kernel): the same partial sums for up to 128 tokens at rank 16, 32 x 32 outputs per matrix
 // instruction; groups[j]: column groups (partial sums per output) of matrix j where it takes them
 // (split: up to 16 tokens on weights that are not rounded to fp16)
-bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups);
+bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups, double *cycles = nullptr);
 int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                          float *const *part, float *ssq, const half_t *x, int N, int K, int T, bool split, hipStream_t s);
 bool bs_tile_columns(const int *I, const int *M, int n, int N, int K, int T, int *columns);

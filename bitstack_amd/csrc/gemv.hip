@@ -807,9 +807,9 @@ int group_path(const int *I, const int *M, int n, int N, int K, int T) {
     // blocks 32 / 12; 8192 x 3200, 4 blocks 40 / 21 (the block-scaled kernel, with that loss: 18 and 24 at 4 and 8 blocks of 4096 x 11008).
     return N % CH != 0 && T < STRIP_MIN_T && strip_group_ok(I, M, n, N, K, T) ? 1 : -1;
 }
-int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
+int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T, double *cycles = nullptr) {
     int groups[GEMV_MAX_GROUP];
-    if (!bs_tile_partials(I, M, n, N, K, T, groups)) return 0;
+    if (!bs_tile_partials(I, M, n, N, K, T, groups, cycles)) return 0;
     int64_t total = (int64_t)groups[0] * T;
     for (int j = 0; j < n; j++) total += (int64_t)groups[j] * T * M[j];
     return total;
@@ -819,18 +819,26 @@ int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T)
 //   4 tokens: 4096 x 14336, 4 blocks 35.7 / 33.0; 14336 x 4096, 8 58.9 / 45.0; 4096 x 4096, 3 16.1 / 13.0, 2 11.3 / 11.8; 14720 x 11776, 2 50.4 / 56.2; 2288 x 7168, 6 26.8 / 18.1
 //   3 tokens: 14336 x 4096, 8 48.9 / 45.3, 5 37.2 / 35.8, 3 26.6 / 27.1; 4096 x 14336, 4 30.3 / 33.7; 4096 x 4096, 3 13.8 / 13.0, 2 9.9 / 11.7; 7605 x 2560, 2 15.4 / 13.9
 // and below a MiB of sign bytes both are a chain of latencies (366 x 512, 14 blocks, 3 tokens 8.3 / 10.6; 1536 x 512, 4, 4 tokens 8.9 / 7.7).
-// A group takes them if each of its matrices alone does.
+// Neither where a single workgroup has more than 50,000 cycles per token of it: the factor-through kernel streams there (us: 5114 x 27136, 6 blocks, 3 tokens
+// 83.9 / 104; 23 drawn shapes at three tokens 0.94 of its rate, from 120,000 to 150,000 cycles 1.02; 11 at four 0.89 and 1.12).  Nor a group
+// of three tokens from 16,000 cycles on up to 8 MiB of sign bytes in all, which the factor-through kernel has in one round (2 x 8192 x 2048,
+// 2 blocks 14.2 / 18.2; 240 of 986 drawn groups, 0.95 on average; the others 1.05).
+// (What a group's matrices do alone is another matter: make_tile_plan compares single ones with the strip kernel too.)
 bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
     if ((T != 3 && T != 4) || g_decode_kernel != 0) return false;
+    int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
         const bool large = (int64_t)M[j] * N > (24ll << 20);
+        bytes += (int64_t)I[j] * M[j] * (N / 8);
         if (I[j] < 2 || (int64_t)I[j] * M[j] * (N / 8) < (1 << 20)) return false;
         if ((T == 3 && large && I[j] < 6) || (I[j] == 2 && N >= 4096)) return false;
     }
     // (never with more partial sums than bs_forward_static's scratch holds: long stacks take 256 columns per workgroup, 16 blocks of 17317 x 111104, 3 tokens 86 MiB
     // where the factor-through kernel needs 6)
-    const int64_t floats = tile_part_floats(I, M, n, N, K, T);
-    return floats > 0 && floats * (int64_t)sizeof(float) <= BS_STATIC_SCRATCH_BYTES;
+    double cycles;
+    const int64_t floats = tile_part_floats(I, M, n, N, K, T, &cycles);
+    if (floats == 0 || floats * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) return false;
+    return cycles <= 50000. * T && !(T == 3 && n > 1 && bytes <= (8 << 20) && cycles > 16000.);
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group

@@ -678,6 +678,26 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
         const long steps = best.np[0] == 1 || I[0] <= 2 || wide ? bs_strip_steps(I[0], M[0], N, T) : 0;
         if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || ((I[0] <= 2 || wide) && tiles == 1 && steps == 1)) best.grid = 0;
     }
+    // Several matrices.  When not even one workgroup each fits the chip at once, the second round is the whole call again (10, 9, 1 and 3 blocks of 733, 968, 7844
+    // and 215 x 19456, 40 tokens, us strip / this 126 / 253; 118 such groups of 26,000 drawn ones: 0.74 of the strip kernel's rate).  With one patch per
+    // wave the strip kernel is ahead where its steps, weighed by their blocks, are few for this plan's cycles: up to three steps (2 x 2048 rows of 1024
+    // columns, 8 blocks, 8 tokens 14.9 / 16.5) from 1180 cycles per step and block on (0.96; below 1.06), beyond them 1030 at 17 to 32 tokens (0.95; below
+    // 1.08; up to 16 tokens 1.14 at any ratio), and 900 from 33 tokens on, where y tiles of three token tiles are handed over (4096 + 2 x 1024 rows of 4096, 8 blocks, 48
+    // tokens 37 / 43; 0.96, below 1.07).  Of the 26,000 groups 10 % were more than 5 % behind the strip kernel, 4 % more than 10 %; with these lines 5 and 2 %.
+    // (Not for three and four tokens at N % 512 == 0, where a decode kernel is the other one.)
+    if (T > 0 && n > 1 && best.grid != 0) {
+        int np = 4;
+        long steps = 0;
+        double weighed = 0;
+        for (int j = 0; j < n; j++) {
+            const long each = T > 4 || N % 512 != 0 ? bs_strip_steps(I[j], M[j], N, T) : 0;
+            steps += each;
+            weighed += each * (I[j] + 0.6);
+            if (best.np[j] < np) np = best.np[j];
+        }
+        const double line = T > 32 ? 900. : steps <= 3 ? 1180. : T > 16 ? 1030. : 1e9;
+        if (best.grid > 256 || (np == 1 && steps > 0 && best.cost > line * weighed)) best.grid = 0;
+    }
     // The rebuild's start costs 1.2 us more than reconstruct_tile_kernel's (226 x 896, 1 block 3.6 / 5.1; 1270 x 2688, 2 blocks 5.8 / 6.4), which a single tile
     // does not win back up to a dozen blocks (556 x 384, 9 blocks 7.8 / 8.7; 257 x 384, 16 10.8 / 9.7), nor two tiles of up to four blocks (2304 x 2048, 3,
     // with its product of 775 tokens 30.4 / 31.4; 768 x 7296, 4, 1104 tokens 37.7 / 39.4) or, one patch per wave, of a dozen (748 x 4352, 9, 656 tokens
@@ -733,12 +753,13 @@ TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
 
 }  // namespace
 
-// Column groups (partial sums per output) of every matrix, if this kernel takes them.
-bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups) {
+// Column groups (partial sums per output) of every matrix, if this kernel takes them; cycles: of its busiest workgroup, by the plan's estimate.
+bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups, double *cycles) {
     if (T < 1) return false;
     if (T > 48) return n == 1 && (groups[0] = bs_column_partials(I[0], M[0], N, K, T)) > 0;
     const TilePlan p = checked_plan(I, M, n, N, K, T);
     for (int j = 0; p.grid != 0 && j < n; j++) groups[j] = p.groups[j];
+    if (cycles) *cycles = p.cost;
     return p.grid != 0;
 }
 

@@ -131,6 +131,22 @@ def test_tile_kernel_says_which_kernel_a_call_runs_on(L):
     assert L.bs_tile_kernel(two, none, 2, 128, 16, 8, two) == -1 and L.bs_tile_kernel(two, two, 2, 128, 16, 8, none) == -1
 
 
+# groups that the tile kernel serves more slowly than the kernel that had them: more workgroups than the chip holds at once, one patch per wave
+# beside few steps of the strip kernel, three tokens within one round of the factor-through kernel, and matrices large enough to stream
+SLOWER_GROUPS = [([(10, 733), (9, 968), (1, 7844), (3, 215)], 19456, 40), ([(2, 329), (2, 3466), (5, 310)], 28160, 40), ([(7, 3346), (10, 312)], 23424, 20),
+                 ([(8, 2048), (8, 2048)], 1024, 48), ([(8, 4096), (8, 1024), (8, 1024)], 4096, 48), ([(4, 3072), (9, 3072)], 1024, 16), ([(1, 4096), (9, 2048), (9, 2048)], 4096, 32),
+                 ([(2, 8192), (2, 8192)], 2048, 3), ([(6, 5114)], 27136, 3)]
+FASTER_GROUPS = [([(3, 8192), (2, 1024), (3, 1024)], 8192, 8), ([(1, 28672), (5, 28672)], 8192, 8), ([(2, 11008), (2, 11008)], 4096, 32), ([(8, 12288), (8, 12288)], 3072, 16),
+                 ([(6, 8192), (6, 8192)], 2048, 3), ([(4, 11008), (4, 11008)], 4096, 4), ([(2, 4096), (2, 1024), (2, 1024)], 4096, 5)]
+
+
+def test_the_tile_kernel_leaves_groups_it_is_slower_on(L):
+    for layers, N, T in SLOWER_GROUPS:
+        assert _lib.tile_kernel(layers, N, 16, T)[0] == _lib.TILE_NONE, (layers, N, T)
+    for layers, N, T in FASTER_GROUPS:
+        assert _lib.tile_kernel(layers, N, 16, T)[0] != _lib.TILE_NONE, (layers, N, T)
+
+
 def test_kernel_hooks_belong_to_the_calling_thread(L):
     """A hook set on one thread moves neither the plan nor the workspace size another thread sees."""
     import threading

@@ -233,7 +233,7 @@ def dense_weights(model):
 def test_fused_step_at_8b_layer_widths_matches_float64_decoder(batch):
     """One decoder layer at the real Llama-3.1-8B widths (hidden 4096, intermediate 14336, 32 query / 8 KV heads), one,
     two and four sequences: the grouped launches then run on the kernels the full model runs on (q/k/v and gate/up with the RMS
-    scale and SwiGLU on the block-scaled kernel at one and two tokens and on the fp16 kernel at four, the residual epilogues), against the float64 decoder
+    scale and SwiGLU on the block-scaled kernel at one and two tokens and on the fp16 kernel at four (o, with its residual, on the tile kernel), the residual epilogues), against the float64 decoder
     on the float64-rebuilt weights."""
     shape = LlamaShape(layers=1, hidden=4096, intermediate=14336, heads=32, kv_heads=8, vocab=512)
     cfg = {f"layer.0.{p}": b for p, b in zip(PROJ, (3, 2, 4, 3, 2, 3, 2))}

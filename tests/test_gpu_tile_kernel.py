@@ -17,10 +17,34 @@ from oracle import c_oracle as C
 
 CSRC = os.path.join(os.path.dirname(_lib.LIB_PATH))
 # (blocks, out features, in features, tokens): rows about whole tiles of 32, columns that leave waves without any, both sides of the block
-# limits of 1024, 512 and 256 columns per workgroup, one, two and three token tiles
-CASES = [(1, 1, 128, 5), (1, 32, 128, 16), (2, 33, 256, 17), (3, 31, 384, 48), (1, 64, 640, 1), (4, 100, 640, 33), (5, 65, 1152, 8), (2, 8200, 1152, 8),
+# limits of 1024, 512 and 256 columns per workgroup, whole and partial column groups of each, one, two and three token tiles
+CASES = [(3, 1, 384, 5), (5, 1, 128, 16), (3, 32, 128, 16), (3, 33, 256, 17), (3, 31, 384, 48), (3, 64, 640, 1), (4, 100, 640, 33), (5, 65, 1152, 8), (2, 8200, 1152, 8),
          (3, 8224, 2176, 7), (4, 8191, 1024, 6), (1, 16400, 640, 40), (2, 8193, 1664, 32), (7, 130, 896, 16), (8, 200, 512, 9), (8, 97, 640, 33),
-         (9, 256, 768, 8), (10, 70, 640, 47), (11, 70, 640, 48), (13, 300, 384, 5), (16, 129, 1024, 24), (16, 65, 1280, 1), (17, 64, 512, 8)]
+         (9, 256, 768, 8), (10, 70, 640, 47), (10, 128, 1024, 40), (13, 300, 384, 5), (15, 129, 1024, 24), (16, 33, 384, 16), (16, 65, 1280, 1),
+         (1, 1892, 2176, 16), (1, 4183, 1024, 20), (2, 16400, 2048, 20), (1, 5877, 640, 2), (4, 8300, 2176, 16), (1, 3334, 1152, 48), (1, 16385, 1280, 48), (7, 4100, 3072, 48)]
+
+
+def _runs_on(kind, layers, N, T):
+    """The columns per workgroup of each matrix, of a call that has to run on `kind` of the tile kernel."""
+    got, columns = _lib.tile_kernel(layers, N, 16, T)
+    assert got == kind, (layers, N, T, got)
+    return columns
+
+
+def test_the_cases_reach_every_width():
+    """Which kernel a call runs on follows from its sizes: every list below reaches what it is there for."""
+    reached = {(_runs_on(_lib.TILE_FORWARD, [c[:2]], c[2], c[3])[0], (c[3] + 15) // 16) for c in CASES}
+    assert reached == {(w, tt) for w in (1024, 512, 256) for tt in (1, 2, 3)}
+    whole = {(w[0], c[2] % w[0] == 0) for c in CASES for w in [_runs_on(_lib.TILE_FORWARD, [c[:2]], c[2], c[3])]}
+    assert whole == {(w, f) for w in (1024, 512, 256) for f in (False, True)}
+    assert {(w[0], c[2] % w[0] == 0) for c in REBUILDS for w in [_runs_on(_lib.TILE_REBUILD, [c[:2]], c[2], 130)]} == whole
+    for T in (3, 4):
+        for cases in (TWO_TERMS, LARGE_WEIGHTS, EVERY_SIZE):
+            assert {_runs_on(_lib.TILE_TWO_TERMS, [c[:2]], c[2], T)[0] for c in cases} == {1024, 512, 256}
+        for cases in (TWO_TERM_GROUPS,):
+            assert {w for layers, N in cases for w in _runs_on(_lib.TILE_TWO_TERMS, layers, N, T)} == {1024, 512, 256}
+    for c in COLUMNS:
+        _runs_on(_lib.TILE_COLUMN, [c[:2]], c[2], c[3])
 
 
 def _args(I, M, N, T, off):
@@ -41,7 +65,7 @@ def _args(I, M, N, T, off):
 @pytest.mark.parametrize("I,M,N,T", CASES)
 def test_edges(I, M, N, T):
     print(f"tile kernel I={I} M={M} N={N} T={T}", flush=True)
-    assert _lib.lib().bs_forward_path(I, M, N, 16, T) in (_lib.PATH_STRIP, _lib.PATH_DECODE_F16, _lib.PATH_DECODE_MX)
+    _runs_on(_lib.TILE_FORWARD, [(I, M)], N, T)
     args, want = _args(I, M, N, T, False)
     y = IU.bitstack_forward_hip(*args)
     _lib.workspace(torch.device("cuda"), 1).fill_(0xFF)          # nothing is read from scratch that the call has not written
@@ -86,6 +110,7 @@ def test_groups_of_unlike_matrices_are_the_single_calls(N, T):
     """Matrices of other heights and block counts in one launch: what each computes alone, up to the order of the column groups' sums."""
     L = _lib.lib()
     layers = [(1, 700), (8, 33), (3, 1000), (5, 64)]
+    _runs_on(_lib.TILE_FORWARD, layers, N, T)
     x = synthetic_layer(8, N, 1, T, seed=3)[3].cuda()
     mats = (_lib.bs_matrix * len(layers))()
     keep, alone = [], []
@@ -118,9 +143,9 @@ def test_the_tile_kernels_keep_everything_in_registers(source, tmp_path):
     assert sizes and set(sizes) == {"0"}, sizes
 
 
-# rows about whole tiles, partial column groups, block counts on both sides of the widths' limits, runs of one and of many tiles
-REBUILDS = [(1, 16411, 640), (2, 8200, 1152), (3, 20000, 384), (4, 8193, 2176), (5, 4100, 1664), (8, 9000, 1024), (10, 33, 128), (11, 2500, 768), (16, 1000, 1280),
-            (16, 31, 256)]
+# rows about whole tiles, whole and partial column groups of each width, block counts on both sides of the widths' limits, runs of one and of many tiles
+REBUILDS = [(1, 11601, 1152), (2, 8200, 1152), (3, 20000, 384), (4, 8193, 2176), (5, 4100, 1664), (8, 9000, 1024), (13, 33, 128), (11, 9000, 768), (16, 1000, 1280),
+            (16, 31, 256), (1, 8257, 2048), (1, 4183, 2048)]
 
 
 @pytest.mark.gpu
@@ -133,6 +158,7 @@ def test_rebuilt_weight(I, M, N):
     x, y = torch.ones(T, N, dtype=torch.half, device="cuda"), torch.empty(T, M, dtype=torch.half, device="cuda")
     need = L.bs_workspace_bytes(I, M, N, 16, T)
     assert L.bs_forward_path(I, M, N, 16, T) == _lib.PATH_REBUILD and need >= M * N * 2
+    _runs_on(_lib.TILE_REBUILD, [(I, M)], N, T)
     guard = torch.full((need // 2 + 64,), 7.0, dtype=torch.half, device="cuda")
     _lib.check(L.bs_forward(q.data_ptr(), u.data_ptr(), vt.data_ptr(), x.data_ptr(), None, y.data_ptr(), I, M, N, 16, T, guard.data_ptr(), need,
                             torch.cuda.current_stream().cuda_stream), "bs_forward")
@@ -161,6 +187,7 @@ def test_rebuilt_weights_of_several_matrices_in_one_launch():
         mats[j] = _lib.bs_matrix(*(t.data_ptr() for t in keep[-1]), None, I, M)
     need = L.bs_forward_cat_workspace_bytes(ctypes.byref(mats), len(layers), N, 16, T)
     assert need > 0
+    _runs_on(_lib.TILE_REBUILD, layers, N, T)
     rows = sum(M for _, M in layers)
     ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
     y = torch.empty(T, rows, dtype=torch.half, device="cuda")
@@ -176,13 +203,20 @@ def test_rebuilt_weights_of_several_matrices_in_one_launch():
         at += M
 
 
+# (blocks, out features, in features) at three and four tokens: each width, whole and partial column groups, rows about whole tiles
+TWO_TERMS = [(2, 8300, 512), (3, 4100, 1024), (4, 4163, 512), (5, 2081, 1536), (2, 3735, 3584), (2, 12993, 1024), (10, 3001, 512), (12, 4096, 512), (16, 2100, 1536)]
+LARGE_WEIGHTS = [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (12, 4096, 512)]
+EVERY_SIZE = [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (16, 2100, 1536)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [3, 4])
-@pytest.mark.parametrize("I,M,N", [(2, 8300, 512), (3, 4100, 1024), (4, 4163, 512), (5, 2081, 1536), (6, 1000, 4096), (10, 3001, 1024), (12, 4096, 512), (16, 2600, 1024)])
+@pytest.mark.parametrize("I,M,N", TWO_TERMS)
 def test_three_and_four_tokens(I, M, N, T):
     """Two fp16 terms per weight: nothing but y is rounded, so it stands no further from float64 than the factor-through kernel."""
     print(f"two terms I={I} M={M} N={N} T={T}", flush=True)
     L = _lib.lib()
+    _runs_on(_lib.TILE_TWO_TERMS, [(I, M)], N, T)
     args, want = _args(I, M, N, T, False)
     size = np.abs(args[3].cpu().numpy().astype(np.float64)) @ np.abs(IU.unpack_and_reconstruct_w_hip(*args[:3]).cpu().numpy().astype(np.float64)).T
     y = IU.bitstack_forward_hip(*args)
@@ -198,8 +232,8 @@ def test_three_and_four_tokens(I, M, N, T):
         finally:
             L.bs_set_decode_kernel(_lib.DECODE_AUTO)
         assert error <= 1.02 * np.linalg.norm(other - want) / np.linalg.norm(want)
-    # one rounding of y; the sums over N columns in fp32, the weights' second terms to 2^-21
-    assert bool((d <= np.abs(want) * 2.0 ** -11 + size * 2.0 ** -13 + 2.0 ** -25).all())
+    # one rounding of y; the weights to 2^-21, their fp32 sums over I blocks and y's over the columns, 32 at a time: 40 additions at most on the way
+    assert bool((d <= np.abs(want) * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
 
 
 @pytest.mark.gpu
@@ -230,7 +264,7 @@ def test_three_and_four_tokens_with_non_finite_inputs_and_large_weights(T):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [3, 4])
-@pytest.mark.parametrize("I,M,N", [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (12, 4096, 512)])
+@pytest.mark.parametrize("I,M,N", LARGE_WEIGHTS)
 def test_three_and_four_tokens_with_weights_beyond_fp16(I, M, N, T):
     """Weights of either sign on both sides of 65504 and of 131008, where two fp16 terms end, and far beyond: y is a finite fp16 number and has to be
     right, in rows beside each other and alone in their tile, and every other row keeps its bits."""
@@ -268,7 +302,7 @@ def test_three_and_four_tokens_with_weights_beyond_fp16(I, M, N, T):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [3, 4])
-@pytest.mark.parametrize("I,M,N", [(2, 16001, 1024), (4, 4163, 512), (6, 4100, 1536), (16, 2100, 1536)])
+@pytest.mark.parametrize("I,M,N", EVERY_SIZE)
 def test_three_and_four_tokens_with_weights_of_every_size(I, M, N, T):
     """Rows with weights from about 0.1 down to 1e-9 beside each other: the second term holds what the first one leaves of a small weight too, so no row stands further
     from float64 than the rounding of its y."""
@@ -287,6 +321,73 @@ def test_three_and_four_tokens_with_weights_of_every_size(I, M, N, T):
         assert d <= 1.01 * torch.hypot(rounding, lost), (p, float(d / rounding))
 
 
+# groups at three and four tokens, as a decoder has them: q, k and v, gate and up, of each width
+TWO_TERM_GROUPS = [([(6, 4096), (6, 1024), (7, 1024)], 4096), ([(6, 8200), (7, 8200)], 2560), ([(3, 16001), (4, 16001)], 1024), ([(3, 8193), (2, 8193)], 2048), ([(12, 4097), (10, 4097)], 1536)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4])
+@pytest.mark.parametrize("epilogue", ["none", "rms", "rms residual", "rms swiglu", "swiglu"])
+@pytest.mark.parametrize("layers,N", TWO_TERM_GROUPS)
+def test_groups_at_three_and_four_tokens(layers, N, epilogue, T):
+    """The sums of squares of x for the RMS scale, the residual and SwiGLU behind the weights in two terms, against float64."""
+    print(f"two-term group {layers} N={N} {epilogue} T={T}", flush=True)
+    L = _lib.lib()
+    _runs_on(_lib.TILE_TWO_TERMS, layers, N, T)
+    swiglu, residual, eps = "swiglu" in epilogue, "residual" in epilogue, 1e-5
+    if swiglu:
+        layers = layers[:2] if layers[0][1] == layers[1][1] else [layers[0], layers[0]]
+        _runs_on(_lib.TILE_TWO_TERMS, layers, N, T)
+    x = synthetic_layer(8, N, 1, T, seed=T)[3].cuda().view(T, N)
+    xd, want, size = x.double(), [], []
+    mats, keep = (_lib.bs_matrix * len(layers))(), []
+    for j, (I, M) in enumerate(layers):
+        q, u, vt, _ = (t.cuda() for t in synthetic_layer(M, N, I, T, seed=10 + j, signed_factors=True))
+        u = (u * 20).half()
+        keep.append((q, u, vt))
+        mats[j] = _lib.bs_matrix(q.data_ptr(), u.data_ptr(), vt.data_ptr(), None, I, M)
+        sign = ((q.view(I, M, N // 8, 1) >> torch.arange(7, -1, -1, device="cuda", dtype=torch.uint8)) & 1).reshape(I, M, N)
+        w = torch.zeros(M, N, dtype=torch.float64, device="cuda")
+        for i in range(I):
+            p = u[i].double() @ vt[i].double()
+            w += torch.where(sign[i].bool(), p, -p)
+        del sign
+        want.append(xd @ w.t().contiguous())
+        size.append(xd.abs() @ w.abs().t().contiguous())
+    scale = torch.rsqrt(xd.pow(2).mean(1, keepdim=True) + eps) if "rms" in epilogue else torch.ones(T, 1, dtype=torch.float64, device="cuda")
+    want, size = [v * scale for v in want], [v * scale for v in size]
+    # a sum: one rounding of y, weights to 2^-21 and fp32 sums (40 additions at most on the way), the scale to 2^-21
+    bound = [v.abs() * 2.0 ** -11 + z * 2.0 ** -18 + 2.0 ** -25 for v, z in zip(want, size)]
+    rows = sum(M for _, M in layers)
+    res = torch.randn(T, rows, device="cuda").half() if residual else None
+    if swiglu:
+        rows = layers[0][1]
+        gate, up = want
+        act = gate * torch.sigmoid(gate)
+        # silu's slope is at most 1.1, its value at most its argument's; act and the product are rounded once each, the exponential is good to 2^-20
+        off = 1.1 * bound[0] + act.abs() * 1.01 * 2.0 ** -11 + 2.0 ** -25
+        want, bound = act * up, off * (up.abs() + bound[1]) + act.abs() * bound[1]
+        bound += want.abs() * 1.01 * 2.0 ** -11 + 2.0 ** -25
+    else:
+        want, bound = torch.cat(want, 1), torch.cat(bound, 1)
+        if residual:
+            want = want + res.double()
+            bound += want.abs() * 1.01 * 2.0 ** -11
+    y = torch.full((T, rows), float("nan"), dtype=torch.half, device="cuda")
+    need = L.bs_forward_group_workspace_bytes(ctypes.byref(mats), len(layers), N, 16, T)
+    ws = torch.full((need + 256,), 0xFF, dtype=torch.uint8, device="cuda")
+    code = _lib.EPI_SWIGLU if swiglu else _lib.EPI_RESIDUAL if residual else _lib.EPI_NONE
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (code, res.data_ptr() if residual else None, y.data_ptr(), ws.data_ptr(), need, stream)
+    if "rms" in epilogue:
+        _lib.check(L.bs_forward_group_rms(ctypes.byref(mats), len(layers), N, 16, x.data_ptr(), T, eps, *args), "bs_forward_group_rms")
+    else:
+        _lib.check(L.bs_forward_group(ctypes.byref(mats), len(layers), N, 16, x.data_ptr(), T, *args), "bs_forward_group")
+    assert bool((ws[need:] == 0xFF).all())
+    worst = ((y.double() - want).abs() / bound).max()
+    assert bool(worst <= 1.0), float(worst)
+
+
 # 49 to 128 tokens: the column kernel from 11 Mi weights on.  Both sides of its token tiles and block limits, rows about whole workgroups of 256,
 # half a span of columns at the end, one span and many per workgroup
 COLUMNS = [(1, 11300, 1024, 49), (2, 12033, 1024, 64), (8, 2816, 4096, 64), (8, 2817, 4224, 50), (3, 30977, 384, 65), (7, 2815, 4352, 96), (5, 90200, 128, 80),
@@ -300,6 +401,7 @@ def test_columns_edges(I, M, N, T):
     print(f"column kernel I={I} M={M} N={N} T={T}", flush=True)
     L = _lib.lib()
     assert L.bs_forward_path(I, M, N, 16, T) in (_lib.PATH_WALKED, _lib.PATH_PANEL)
+    _runs_on(_lib.TILE_COLUMN, [(I, M)], N, T)
     q, u, vt, x = (t.cuda() for t in synthetic_layer(M, N, I, T, seed=I + N + T, signed_factors=True))
     u = (u * 20).half()
     bias = torch.randn(M, device="cuda").half()

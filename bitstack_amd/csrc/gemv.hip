@@ -816,8 +816,9 @@ int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T,
 }
 // Three and four tokens: the factor-through kernel needs 16 products per sign and token, the tile kernel one weight for all of them.  It takes them with
 // the weight in two fp16 terms, so that only y is rounded (error against float64 0.7 of the other's).  us, factor-through / tiles:
-//   4 tokens: 4096 x 14336, 4 blocks 35.7 / 33.0; 14336 x 4096, 8 58.9 / 45.0; 4096 x 4096, 3 16.1 / 13.0, 2 11.3 / 11.8; 14720 x 11776, 2 50.4 / 56.2; 2288 x 7168, 6 26.8 / 18.1
-//   3 tokens: 14336 x 4096, 8 48.9 / 45.3, 5 37.2 / 35.8, 3 26.6 / 27.1; 4096 x 14336, 4 30.3 / 33.7; 4096 x 4096, 3 13.8 / 13.0, 2 9.9 / 11.7; 7605 x 2560, 2 15.4 / 13.9
+//   4 tokens: 4096 x 14336, 4 blocks 38.4 / 35.5; 14336 x 4096, 8 60.5 / 47.1; 4096 x 4096, 3 17.3 / 15.3, 2 11.3 / 11.8; 14720 x 11776, 2 50.4 / 56.2; 2288 x 7168, 6 26.8 / 19.6
+//   3 tokens: 14336 x 4096, 8 49.3 / 47.3, 5 37.2 / 35.8, 3 26.6 / 27.1; 4096 x 14336, 4 30.3 / 33.7; 4096 x 4096, 3 14.9 / 15.3, 2 9.9 / 11.7; 7605 x 2560, 2 15.6 / 15.5
+// (over drawn shapes 1.27 and 1.12 on average, 1 and 8 % of them more than 5 % behind)
 // and below a MiB of sign bytes both are a chain of latencies (366 x 512, 14 blocks, 3 tokens 8.3 / 10.6; 1536 x 512, 4, 4 tokens 8.9 / 7.7).
 // Neither where a single workgroup has more than 50,000 cycles per token of it: the factor-through kernel streams there (us: 5114 x 27136, 6 blocks, 3 tokens
 // 83.9 / 104; 23 drawn shapes at three tokens 0.94 of its rate, from 120,000 to 150,000 cycles 1.02; 11 at four 0.89 and 1.12).  Nor a group

@@ -14,17 +14,19 @@
 // (v_mfma_f32_16x16x32_f16).  The waves' y tiles (same rows, other columns) meet in LDS, double buffered, and are added up in wave
 // order while the next tile is rebuilt: one barrier per tile, and scratch holds one partial per 256 NP columns.
 //
-// The rebuilt weight itself (TT = 0, above 128 tokens and for levels 3 and 4) is the same walk with the rounded tile stored instead of
-// multiplied.  us, reconstruct_tile_kernel / this: 14336 x 4096, 8 blocks 55.6 / 48.3 (40.5 without the stores), 4096 x 14336, 8 56.3 / 46.3, 28672 x 8192, 3
-// 178 / 112 (558 MB: 5.0 TB/s, the copy rate), 14336 x 4096, 5 43.7 / 37.3.
+// The rebuilt weight itself (TT = 0, in forwards above 128 tokens) is the same walk with the rounded tile stored instead of multiplied.  Whole calls of
+// 130 tokens, us, reconstruct_tile_kernel / this: 14336 x 4096, 8 blocks 104 / 90, 4096 x 14336, 8 109 / 92 (the rebuild by itself, by the profiler, 82 / 63),
+// 28672 x 8192, 3 310 / 241, 14336 x 4096, 5 89 / 84.
 //
-// What bounds it: the issue of a wave's instructions.  Simple VALU instructions (v_xor_b32, v_and_b32, v_lshrrev_b32, fp32 add, mul and FMA on
+// What bounds it: the issue of a wave's instructions: by the counters vector instructions take 61 % of a SIMD's cycles on 28672 x 8192, 3 blocks, 8 tokens
+// and 59 on 4096 x 14336, 4 blocks, 4 tokens (the matrix cores 21 and 15), where runs are short 33 (5000 x 4096, 6 blocks, 37 tokens) and waits at the
+// barrier and for LDS as much, in the rebuild 45 with its stores waited for.  Simple VALU instructions (v_xor_b32, v_and_b32, v_lshrrev_b32, fp32 add, mul and FMA on
 // three registers) of two waves run side by side on a SIMD, 1.0 ns each; v_fma_mix_f32, v_and_or_b32, v_bfe, v_alignbit, conversions and whatever
 // has a scalar operand take 1.8 ns, and a single wave issues one instruction in 2 ns whatever it is.  A step (1024 signs: 16 v_xor, 5 for the
 // table addresses, 4 lookups, one product) takes 45 ns per SIMD with two waves and 40 with four; with the signs as fp16 in v_fma_mix 46 and 42.
-// About 1300 cycles per tile and wave (barrier, hand-over, rounding, second product) come on top.  us, strip_forward_kernel / this, with the summing launch:
-// 28672 x 8192, 3 blocks, 8 tokens 90 / 64; 14336 x 4096, 8 blocks 62 / 44; 5000 x 4096, 6 blocks, 37 tokens 29.6 / 25; 4096 x 11008, 4
-// blocks, one token 24.8 / 23.
+// About 1300 cycles per tile and wave (barrier, hand-over, rounding, second product) come on top.  us, strip_forward_kernel / this, with the summing launch, in a
+// replayed graph on rotating copies: 28672 x 8192, 3 blocks, 8 tokens 86.5 / 62.8; 14336 x 4096, 8 blocks, 8 tokens 50.0 / 42.6; 5000 x 4096, 6 blocks, 37 tokens
+// 29.7 / 25.6; 4096 x 11008, 4 blocks, one token 26.1 / 24.4.
 #include "common.h"
 #include "rebuild_shared.h"
 
@@ -672,6 +674,8 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     // one or two blocks: the hand-over between the waves is half a us (896 x 2176, 1 block 6.8 / 7.5; 643 x 896, 2 blocks 8.4 / 8.9; from 3 blocks
     // on level or ahead; with two patches per wave the one tile is the longer chain: 2668 x 896, 5 blocks 8.4 / 9.9, 3345 x 640, 3 7.8 / 8.6, 2019 x 1664, 3
     // 8.0 / 8.6, against two steps 4398 x 1536, 4 13.1 / 10.2.  Not for three and four tokens at N % 512 == 0, where a decode kernel is the other one).
+    // (The line for one patch per wave is asked there too, although it compares with the strip kernel: of 4,200 drawn shapes that it turns away the factor-through
+    // kernel's time is 1.05 of this one's at three tokens, 0.73 to 1.67, and 1.22 at four.)
     if (T > 0 && n == 1 && best.grid != 0) {
         const int64_t tiles = bs_cdiv(bs_cdiv(M[0], TL_ROWS), best.wgs[0]);
         const bool wide = best.np[0] == 2 && (T > 4 || N % 512 != 0);
@@ -680,8 +684,8 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     }
     // Several matrices.  When not even one workgroup each fits the chip at once, the second round is the whole call again (10, 9, 1 and 3 blocks of 733, 968, 7844
     // and 215 x 19456, 40 tokens, us strip / this 126 / 253; 118 such groups of 26,000 drawn ones: 0.74 of the strip kernel's rate).  With one patch per
-    // wave the strip kernel is ahead where its steps, weighed by their blocks, are few for this plan's cycles: up to three steps (2 x 2048 rows of 1024
-    // columns, 8 blocks, 8 tokens 14.9 / 16.5) from 1180 cycles per step and block on (0.96; below 1.06), beyond them 1030 at 17 to 32 tokens (0.95; below
+    // wave the strip kernel is ahead where its steps, weighed by their blocks, are few for this plan's cycles: up to three steps (2 x 3072 rows of 1024
+    // columns, 4 and 9 blocks, 16 tokens 16.0 / 17.6) from 1180 cycles per step and block on (0.96; below 1.06), beyond them 1030 at 17 to 32 tokens (0.95; below
     // 1.08; up to 16 tokens 1.14 at any ratio), and 900 from 33 tokens on, where y tiles of three token tiles are handed over (4096 + 2 x 1024 rows of 4096, 8 blocks, 48
     // tokens 37 / 43; 0.96, below 1.07).  Of the 26,000 groups 10 % were more than 5 % behind the strip kernel, 4 % more than 10 %; with these lines 5 and 2 %.
     // (Not for three and four tokens at N % 512 == 0, where a decode kernel is the other one.)

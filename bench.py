@@ -465,6 +465,8 @@ def main():
         kind, _ = _lib.tile_kernel([(L.I, L.M)], L.N, 16, L.T)
         if kind != _lib.TILE_NONE:
             return _lib.TILE_NAMES[kind], 0
+        if _lib.sparse_kernel([(L.I, L.M)], L.N, 16, L.T):
+            return "gemv_sparse_kernel<R=%d,T=%d>" % (r, L.T), grid
         if path == _lib.PATH_DECODE_MX:
             return "gemv_mx_kernel<R=%d>" % r, grid
         if path == _lib.PATH_DECODE_F16:

@@ -35,6 +35,7 @@ SIGNATURES = {
     "bs_set_dense_kernel": (_I, [_I]),
     "bs_set_prefill_kernel": (_I, [_I]),
     "bs_forward_path": (_I, [_I, _I, _I, _I, _I]),
+    "bs_sparse_kernel": (_I, [_P, _P, _I, _I, _I, _I]),
     "bs_tile_kernel": (_I, [_P, _P, _I, _I, _I, _I, _P]),
 }
 DECODE_AUTO, DECODE_F16, DECODE_MX = 0, 1, 2
@@ -116,8 +117,18 @@ def tile_kernel(layers, N, K, T):
     return kind, list(columns)
 
 
+def sparse_kernel(layers, N, K, T):
+    """Whether gemv_sparse_kernel runs one or several (blocks, out features) on the same x."""
+    n = len(layers)
+    serves = int(lib().bs_sparse_kernel((ctypes.c_int * n)(*(i for i, _ in layers)), (ctypes.c_int * n)(*(m for _, m in layers)), n, N, K, T))
+    check(min(serves, 0), "bs_sparse_kernel")
+    return serves == 1
+
+
 def forward_kernel_name(I, M, N, K, T):
     """The kernel that a forward of these dimensions runs on, u being 16-byte aligned."""
+    if sparse_kernel([(I, M)], N, K, T):
+        return "gemv_sparse_kernel"
     path = int(lib().bs_forward_path(I, M, N, K, T))
     check(min(path, 0), "bs_forward_path")
     return TILE_NAMES.get(tile_kernel([(I, M)], N, K, T)[0], PATH_NAMES[path])

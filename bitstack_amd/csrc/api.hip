@@ -95,6 +95,18 @@ extern "C" int bs_forward_path(int I, int M, int N, int K, int T) {
     return bs_gemv_forward_path(I, M, N, K, T);
 }
 
+extern "C" int bs_sparse_kernel(const int *I, const int *M, int n, int N, int K, int T) {
+    if (!I || !M) return BS_ERR_NULL;
+    if (n < 1 || n > BS_MAX_GROUP) return BS_ERR_SHAPE;
+    bool empty = T == 0;
+    for (int j = 0; j < n; j++) {
+        const int st = forward_dims(I[j], M[j], N, K, T);
+        if (st != BS_OK) return st;
+        empty = empty || I[j] == 0;
+    }
+    return empty ? 0 : bs_gemv_sparse_serves(I, M, n, N, K, T);
+}
+
 extern "C" int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
     if (!I || !M || !columns) return BS_ERR_NULL;
     if (n < 1 || n > BS_MAX_GROUP) return BS_ERR_SHAPE;

@@ -80,6 +80,7 @@ void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_t
 int bs_gemv_plan_kernel(int I, int M, int N, int K, int T);
 int bs_gemv_forward_path(int I, int M, int N, int K, int T);
 int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns);
+int bs_gemv_sparse_serves(const int *I, const int *M, int n, int N, int K, int T);
 int bs_gemv_set_kernel(int mode);
 // epilogues of the grouped decode forward (values of BS_EPI_* in the public header)
 enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2 };

@@ -72,7 +72,10 @@ __device__ __forceinline__ void static_for(F &&f) {
 }
 
 constexpr int CH = 512;   // columns per chunk: 4 lane groups x 16 bytes of signs
-constexpr int64_t MX_MIN_SIGN_BYTES = 8 << 20;   // sign bytes per launch from which the block-scaled kernel is preferred
+// Sign bytes per launch from which the block-scaled kernel is preferred to the sparse one.  us sparse / block-scaled, one token: 4096 x 4096, 4 blocks (8 MiB) 9.4 / 9.3,
+// 8 blocks 13.7 / 12.6, 14336 x 4096, 8 blocks 30.6 / 28.7; two tokens: 8 blocks of 4096 x 4096 (16 MiB) 16.8 / 17.6, 6144 x 4096, 6 blocks 20.4 / 22.2, 4096 x 14336, 3 (21 MiB)
+// 22.5 / 22.9, 14336 x 4096, 8 (56 MiB) 38.9 / 39.9, 4096 x 14336, 16 (112 MiB) 65.1 / 60.9.
+constexpr int64_t MX_MIN_SIGN_BYTES = 12 << 20, MX_MIN_SIGN_BYTES_TWO = 24 << 20;
 
 
 // step -> bit position used in that step; steps 0-7 read the word as loaded,
@@ -548,6 +551,7 @@ void launch_reduce_flat(int blocks, const RedGroup &r, const half_t *residual, h
 struct Plan {
     int waves, R, n_chunks, grid, n, pair;
     int mx;        // 1: the block-scaled fp4 x fp6 kernel (gemv_mx.hip), units of MX_UNIT_COLS columns
+    int sparse;    // 1: the sparse kernel (gemv_sparse.hip)
     int row_tiles[GEMV_MAX_GROUP], kmax[GEMV_MAX_GROUP], first_wg[GEMV_MAX_GROUP];
     Split sp[GEMV_MAX_GROUP];
     int64_t part_off[GEMV_MAX_GROUP];      // in floats; part_off[n] = total
@@ -580,52 +584,58 @@ int mx_rows_per_tile(const int *I, const int *M, int n, int N, int K, int T) {
     // by shape: the long-stack cases, where the contraction loop and not the fixed cost of a launch decides
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) bytes += (int64_t)I[j] * M[j] * (N / 8);
-    return (pick >= 2 && bytes >= MX_MIN_SIGN_BYTES) ? pick : 0;
+    return (pick >= 2 && bytes >= (T == 1 ? MX_MIN_SIGN_BYTES : MX_MIN_SIGN_BYTES_TWO)) ? pick : 0;
+}
+
+// The grid of the block-scaled and the sparse kernel: one workgroup of 8 waves, 128 R rows, per CU.
+void one_per_cu(Plan &p, const int *I, const int *M, int T) {
+    const int n = p.n;
+    p.waves = 8;
+    p.pair = 0;
+    int units[GEMV_MAX_GROUP], total = 0, biggest = 0;
+    for (int j = 0; j < n; j++) {
+        p.row_tiles[j] = (int)bs_cdiv(M[j], 8 * p.R * 16);
+        units[j] = I[j] * p.row_tiles[j] * p.n_chunks;
+        total += units[j];
+        if (units[j] > units[biggest]) biggest = j;
+    }
+    int grid = total < 256 ? total : 256, gj[GEMV_MAX_GROUP], sum = 0;
+    for (int j = 0; j < n; j++) {
+        gj[j] = n == 1 ? grid : (int)(((int64_t)grid * units[j] + total / 2) / total);
+        if (gj[j] < 1) gj[j] = 1;
+        if (gj[j] > units[j]) gj[j] = units[j];
+        sum += gj[j];
+    }
+    while (sum > grid && gj[biggest] > 1) { gj[biggest]--; sum--; }
+    int first = 0;
+    int64_t off = 0;
+    for (int j = 0; j < n; j++) {
+        p.first_wg[j] = first;
+        first += gj[j];
+        p.sp[j].q = units[j] / gj[j];
+        p.sp[j].rem = units[j] % gj[j];
+        int kmax = (int)bs_cdiv(p.n_chunks - 1, p.sp[j].q) + 1;
+        if (kmax > gj[j]) kmax = gj[j];
+        p.kmax[j] = kmax;
+        p.part_off[j] = off;
+        off += (int64_t)I[j] * kmax * T * M[j];
+    }
+    p.grid = first;
+    p.part_total = off;
 }
 
 Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
     Plan p;
     p.n = n;
     p.n_chunks = N / CH;
-    p.mx = 0;
+    p.mx = p.sparse = 0;
     const int mx_r = mx_rows_per_tile(I, M, n, N, K, T);
     if (mx_r > 0) {
-        // one workgroup of 8 waves per CU; units are (block, row tile, 1024 columns), never paired
+        // units are (block, row tile, 1024 columns), never paired
         p.mx = 1;
-        p.waves = 8;
         p.R = mx_r;
-        p.pair = 0;
         p.n_chunks = (int)bs_cdiv(N, MX_UNIT_COLS / T);
-        int units[GEMV_MAX_GROUP], total = 0, biggest = 0;
-        for (int j = 0; j < n; j++) {
-            p.row_tiles[j] = (int)bs_cdiv(M[j], 8 * mx_r * 16);
-            units[j] = I[j] * p.row_tiles[j] * p.n_chunks;
-            total += units[j];
-            if (units[j] > units[biggest]) biggest = j;
-        }
-        int grid = total < 256 ? total : 256, gj[GEMV_MAX_GROUP], sum = 0;
-        for (int j = 0; j < n; j++) {
-            gj[j] = n == 1 ? grid : (int)(((int64_t)grid * units[j] + total / 2) / total);
-            if (gj[j] < 1) gj[j] = 1;
-            if (gj[j] > units[j]) gj[j] = units[j];
-            sum += gj[j];
-        }
-        while (sum > grid && gj[biggest] > 1) { gj[biggest]--; sum--; }
-        int first = 0;
-        int64_t off = 0;
-        for (int j = 0; j < n; j++) {
-            p.first_wg[j] = first;
-            first += gj[j];
-            p.sp[j].q = units[j] / gj[j];
-            p.sp[j].rem = units[j] % gj[j];
-            int kmax = (int)bs_cdiv(p.n_chunks - 1, p.sp[j].q) + 1;
-            if (kmax > gj[j]) kmax = gj[j];
-            p.kmax[j] = kmax;
-            p.part_off[j] = off;
-            off += (int64_t)I[j] * kmax * T * M[j];
-        }
-        p.grid = first;
-        p.part_total = off;
+        one_per_cu(p, I, M, T);
         return p;
     }
     // rows per workgroup: 512 (8 waves x 4 tiles), 256, 128, 64; resident workgroups per CU.
@@ -729,6 +739,31 @@ Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
     return p;
 }
 
+// The plan of the sparse kernel where it serves these matrices, for the rules at sparse_plan.
+Plan sparse_plan_of(const int *I, const int *M, int n, int N, int T) {
+    Plan p;
+    p.n = n;
+    p.mx = 0;
+    p.sparse = 1;
+    p.n_chunks = (int)bs_cdiv(N, CH);
+    // Row tiles per wave by the time of the busiest workgroup (us, a replayed graph, the summing launch included): what a call with one unit per workgroup takes
+    // and what each further unit adds, fitted to 33 shapes (4096 x 11008, 4 blocks, one token, R = 1, 2, 4: 21.8, 18.3, 17.7; 1024 x 4096, 3 blocks 7.2, 7.8, 8.7;
+    // 20000 x 1408, 2 blocks 12.1, 10.8, 9.0; 6144 x 4096, 6 blocks, two tokens 22.6, 20.4, 21.9).
+    static const double base[3][3] = {{5.25, 5.45, 5.9}, {5.7, 5.9, 5.8}, {5.5, 5.85, 6.0}}, unit[3][3] = {{1.18, 1.45, 2.0}, {1.43, 2.0, 3.56}, {1.95, 2.68, 5.03}};
+    double best = 0;
+    for (int k = 0; k < 3; k++) {
+        int64_t units = 0;
+        for (int j = 0; j < n; j++) units += bs_cdiv(M[j], 128 << k) * I[j] * p.n_chunks;
+        const double us = base[T - 1][k] + unit[T - 1][k] * bs_cdiv(units, 256);
+        if (k == 0 || us < best) {
+            best = us;
+            p.R = 1 << k;
+        }
+    }
+    one_per_cu(p, I, M, T);
+    return p;
+}
+
 struct GroupArgs {          // host-side view of one call
     int n;
     const uint8_t *packed[GEMV_MAX_GROUP];
@@ -770,11 +805,9 @@ int launch_T(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K,
     return BS_ERR_SHAPE;
 }
 
-bool gemv_shape_ok(int I, int M, int N, int T) {
-    // per-block byte offsets are kept in 32 bits inside the kernel
-    return I >= 1 && I <= RED_MAXBLOCKS && T >= 1 && T <= 8 && N % CH == 0 && M >= 1 &&
-           (int64_t)M * N < ((int64_t)1 << 31);
-}
+// per-block byte offsets are kept in 32 bits inside the kernels
+bool block_fits(int I, int M, int N) { return I >= 1 && I <= RED_MAXBLOCKS && M >= 1 && (int64_t)M * N < ((int64_t)1 << 31); }
+bool gemv_shape_ok(int I, int M, int N, int T) { return block_fits(I, M, N) && T >= 1 && T <= 8 && N % CH == 0; }
 
 // Tokens are processed in passes of at most four (LDS holds Z for four tokens).
 int pass_tokens(int T) { return T <= 4 ? T : (T + 1) / 2; }
@@ -825,8 +858,10 @@ int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T,
 // of three tokens from 16,000 cycles on up to 8 MiB of sign bytes in all, which the factor-through kernel has in one round (2 x 8192 x 2048,
 // 2 blocks 14.2 / 18.2; 240 of 986 drawn groups, 0.95 on average; the others 1.05).
 // (What a group's matrices do alone is another matter: make_tile_plan compares single ones with the strip kernel too.)
+// Nor three tokens of one matrix with 4096 columns or more, where the sparse kernel is faster whatever the blocks (us tile / sparse: 4096 x 4096, 4 blocks 16.6 / 13.1, 8
+// 23.1 / 19.9; 14336 x 4096, 8 51.5 / 48.2; 1024 x 4096, 3 10.0 / 7.9).
 bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
-    if ((T != 3 && T != 4) || g_decode_kernel != 0) return false;
+    if ((T != 3 && T != 4) || g_decode_kernel != 0 || (T == 3 && n == 1 && N >= 4096)) return false;
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
         const bool large = (int64_t)M[j] * N > (24ll << 20);
@@ -841,11 +876,40 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
     if (floats == 0 || floats * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) return false;
     return cycles <= 50000. * T && !(T == 3 && n > 1 && bytes <= (8 << 20) && cycles > 16000.);
 }
+// The sparse kernel's plan where it serves the call; grid 0: another kernel does.
+//   N % 512 == 0: one to three tokens in the place of gemv_kernel.  us gemv_kernel / sparse, one token: 1024 x 4096, 3 blocks 8.1 / 7.2, 4096 x 4096, 2 8.6 / 7.8, 14336 x 4096, 1
+//     10.7 / 9.1 (below a MiB of sign bytes either is a chain of latencies, gemv_kernel's the shorter one: 355 x 2560, 4 6.3 / 6.9, 308 x 3584, 5 6.9 / 7.1); two: 1024 x 4096, 3 10.4 / 7.6, 4096 x 4096, 1 8.9 / 7.7, 14336 x 4096, 1 13.1 / 10.8; three: 4096 x 14336, 16 87.5 / 83.4, 3
+//     31.1 / 27.8, 28672 x 8192, 2 52.0 / 47.6, 1024 x 4096, 1 8.6 / 7.4.  Four: 4096 x 14336, 16 104 / 116, 28672 x 8192, 2 58.6 / 64.1: gemv_kernel keeps them.
+//   Other multiples of 128 columns, one and two tokens: us tile or strip kernel / sparse, one token: 4096 x 11008, 4 blocks 25.7 / 17.7, 8 39.3 / 25.6, 2 18.3 / 13.0;
+//     20000 x 1408, 2 15.6 / 9.0; 2048 x 5504, 3 11.9 / 9.0; two: 24.7 / 22.6, 39.1 / 32.8, 18.5 / 15.5, 15.3 / 10.5, 12.0 / 10.3; three: 24.7 / 27.4, 39.6 / 42.0.  Up to half a
+//     MiB of sign bytes the two are about a us apart (5877 x 640, 1 block 7.2 / 6.0) and at rank 16 the tile kernel, whose tests hold it to calls of that size, keeps them.
+// Over 97 drawn calls 1.21 times as fast at one token, 1.23 at two, 1.19 at three, none more than 1 % slower.  It rounds nothing but y: error against float64 before that rounding 1e-7 to 4e-7 on drawn factors.  (Never with more partial sums than bs_forward_static's scratch holds.)
+constexpr int64_t SPARSE_MIN_UNEVEN = 512 << 10, SPARSE_MIN_ONE = 1 << 20;
+Plan sparse_plan(const int *I, const int *M, int n, int N, int K, int T) {
+    Plan p;
+    p.grid = 0;
+    const bool even = N % CH == 0;
+    if (n < 1 || n > GEMV_MAX_GROUP || g_decode_kernel != 0 || T > (even ? 3 : 2) || !bs_gemv_sparse_takes(N, K, 1, T) || group_path(I, M, n, N, K, T) != (even ? 0 : 1)) return p;
+    if (even && mx_rows_per_tile(I, M, n, N, K, T) > 0) return p;
+    int64_t bytes = 0;
+    for (int j = 0; j < n; j++) {
+        if (!block_fits(I[j], M[j], N)) return p;
+        bytes += (int64_t)I[j] * M[j] * (N / 8);
+    }
+    if ((!even && K == 16 && bytes < SPARSE_MIN_UNEVEN) || (even && T == 1 && bytes < SPARSE_MIN_ONE)) return p;
+    p = sparse_plan_of(I, M, n, N, T);
+    if (p.part_total * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) p.grid = 0;
+    return p;
+}
+int64_t sparse_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
+    const Plan p = sparse_plan(I, M, n, N, K, T);
+    return p.grid ? p.part_total : 0;
+}
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group
     for (int j = 0; j < n; j++) total += (int64_t)bs_strip_partials(I[j], M[j], N, K, T) * T * M[j];
     // room for the tile kernel's partial sums too: the choice also depends on how u is aligned
-    return std::max(total, tile_part_floats(I, M, n, N, K, T));
+    return std::max(std::max(total, tile_part_floats(I, M, n, N, K, T)), sparse_part_floats(I, M, n, N, K, T));
 }
 
 // Strip path: one launch writes part[strip group, t, m] of every matrix; the reduce kernel
@@ -910,18 +974,16 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
     if (mode == EPI_SWIGLU && (a.n != 2 || a.M[0] != a.M[1])) return BS_ERR_SHAPE;
     const int path = group_path(a.I, a.M, a.n, N, K, T);
     if (path < 0) return BS_ERR_SHAPE;
-    if (path == 1) {
-        for (int j = 0; j < a.n; j++)
-            if (!bs_aligned(a.packed[j], 16) || !bs_aligned(a.vt[j], 16) || !bs_aligned(a.u[j], 8)) return BS_ERR_SHAPE;
-        return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, false, s);
-    }
-    bool split = split_tiles(a.I, a.M, a.n, N, K, T);
-    for (int j = 0; j < a.n; j++) split = split && bs_aligned(a.u[j], 16) && bs_aligned(a.packed[j], 16) && bs_aligned(a.vt[j], 16);
-    if (split) return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, true, s);
+    for (int j = 0; j < a.n; j++)
+        if (!bs_aligned(a.packed[j], 16) || !bs_aligned(a.vt[j], 16) || !bs_aligned(a.u[j], 8)) return BS_ERR_SHAPE;
+    bool split = path == 0 && split_tiles(a.I, a.M, a.n, N, K, T);
+    for (int j = 0; j < a.n; j++) split = split && bs_aligned(a.u[j], 16);
+    const Plan sparse = sparse_plan(a.I, a.M, a.n, N, K, T);
+    if (split || (path == 1 && sparse.grid == 0))
+        return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, split, s);
     int ldy = 0;
     for (int j = 0; j < a.n; j++) {
-        if (!gemv_shape_ok(a.I[j], a.M[j], N, T)) return BS_ERR_SHAPE;
-        if (!bs_aligned(a.packed[j], 16) || !bs_aligned(a.vt[j], 16) || !bs_aligned(a.u[j], 8)) return BS_ERR_SHAPE;
+        if (sparse.grid == 0 && !gemv_shape_ok(a.I[j], a.M[j], N, T)) return BS_ERR_SHAPE;
         ldy += a.M[j];
     }
     if (mode == EPI_SWIGLU) {
@@ -935,7 +997,7 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
     float *part = (float *)workspace;
     for (int t0 = 0; t0 < T; t0 += tp) {
         const int tn = (T - t0 < tp) ? T - t0 : tp;
-        const Plan p = make_plan(a.I, a.M, a.n, N, K, tn);
+        const Plan p = sparse.grid ? sparse : make_plan(a.I, a.M, a.n, N, K, tn);
         if (!workspace || workspace_bytes < p.part_total * (int64_t)sizeof(float)) return BS_ERR_WORKSPACE;
         GemvGroup g;
         RedGroup r;
@@ -963,7 +1025,8 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
         const half_t *xp = x + (int64_t)t0 * N;
         r.xin = input_rms ? xp : nullptr;
         int st;
-        if (p.mx) st = bs_launch_gemv_mx(p.R, tn, p.grid, g, xp, N, K, p.n_chunks, s);
+        if (p.sparse) st = bs_launch_gemv_sparse(p.R, tn, p.grid, g, xp, N, K, p.n_chunks, s);
+        else if (p.mx) st = bs_launch_gemv_mx(p.R, tn, p.grid, g, xp, N, K, p.n_chunks, s);
         else switch (tn) {
             case 1: st = launch_T<1>(p, g, xp, N, K, s); break;
             case 2: st = launch_T<2>(p, g, xp, N, K, s); break;
@@ -1007,7 +1070,7 @@ int64_t bs_gemv_group_workspace_bytes(const int *I, const int *M, int n, int N, 
     const int path = group_path(I, M, n, N, K, T);
     if (path < 0) return 0;
     if (path == 1) return strip_part_floats(I, M, n, N, K, T) * (int64_t)sizeof(float);
-    int64_t floats = gemv_part_floats(I, M, n, N, K, T);
+    int64_t floats = std::max(gemv_part_floats(I, M, n, N, K, T), sparse_part_floats(I, M, n, N, K, T));
     if (split_tiles(I, M, n, N, K, T)) floats = std::max(floats, tile_part_floats(I, M, n, N, K, T));
     return floats * (int64_t)sizeof(float);
 }
@@ -1017,7 +1080,8 @@ int64_t bs_gemv_group_workspace_bytes(const int *I, const int *M, int n, int N, 
 void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave, int *grid, int *kmax) {
     *waves = *row_tiles_per_wave = *grid = *kmax = 0;
     if (group_path(&I, &M, 1, N, K, T) != 0) return;
-    const Plan p = make_plan(&I, &M, 1, N, K, pass_tokens(T));
+    Plan p = sparse_plan(&I, &M, 1, N, K, T);
+    if (p.grid == 0) p = make_plan(&I, &M, 1, N, K, pass_tokens(T));
     *waves = p.waves;
     *row_tiles_per_wave = p.R;
     *grid = p.grid;
@@ -1035,9 +1099,15 @@ int bs_gemv_forward_path(int I, int M, int N, int K, int T) {
     return make_plan(&I, &M, 1, N, K, pass_tokens(T)).mx ? BS_PATH_DECODE_MX : BS_PATH_DECODE_F16;
 }
 
+// 1: gemv_sparse_kernel runs these matrices, of three tokens only with u off a 16-byte boundary where split_tiles has the tile kernel take them
+int bs_gemv_sparse_serves(const int *I, const int *M, int n, int N, int K, int T) {
+    return sparse_plan(I, M, n, N, K, T).grid > 0 && !split_tiles(I, M, n, N, K, T);
+}
+
 // Which call of the tile and column kernels serves these matrices, with u on 16-byte boundaries (values of BS_TILE_* in the public header).
 int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
     const int path = group_path(I, M, n, N, K, T);
+    if (path == 1 && T < STRIP_MIN_T && sparse_plan(I, M, n, N, K, T).grid > 0) return BS_TILE_NONE;
     if (path == 1 && (n == 1 || T <= 48)) return !bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_NONE : T > 48 ? BS_TILE_COLUMN : BS_TILE_FORWARD;
     if (path == 0) return split_tiles(I, M, n, N, K, T) && bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_TWO_TERMS : BS_TILE_NONE;
     for (int j = 0; j < n; j++)

@@ -44,3 +44,6 @@ struct GemvGroup {
 constexpr int MX_UNIT_COLS = 1024;
 bool bs_gemv_mx_takes(int N, int K, int R, int T);
 int bs_launch_gemv_mx(int R, int T, int grid, const GemvGroup &grp, const half_t *x, int N, int K, int n_units, hipStream_t s);
+// One to three tokens on the sparse matrix instruction (gemv_sparse.hip): units of 512 columns, 128 R rows per workgroup, any multiple of 128 columns.
+bool bs_gemv_sparse_takes(int N, int K, int R, int T);
+int bs_launch_gemv_sparse(int R, int T, int grid, const GemvGroup &grp, const half_t *x, int N, int K, int n_units, hipStream_t s);

@@ -166,7 +166,8 @@ int bs_decode_plan(int I, int M, int N, int K, int T, int *waves, int *row_tiles
 
 /*
  * Which decode kernel bs_forward runs for these dimensions: 0 none (strip kernel
- * or dense path), BS_DECODE_F16 the fp16-MFMA kernel (1..4 tokens per pass),
+ * or dense path), BS_DECODE_F16 an fp16-MFMA kernel (1..4 tokens per pass; bs_sparse_kernel
+ * says which),
  * BS_DECODE_MX the block-scaled fp4 x fp6 MFMA kernel (one or two tokens; signs
  * as the fp4 operand, vt o x as three fp6 terms).  For more than four tokens the
  * answer is that of the first pass.  Negative = error status.
@@ -183,7 +184,7 @@ int bs_decode_kernel(int I, int M, int N, int K, int T);
  * bitstack/modules/BitStackLinear.py:116-157).
  */
 #define BS_PATH_REBUILD    0   /* weight rebuilt into the workspace, then the dense product */
-#define BS_PATH_DECODE_F16 1   /* gemv_kernel: packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass (3 and 4 on large matrices: tile_forward_kernel) */
+#define BS_PATH_DECODE_F16 1   /* packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass: gemv_sparse_kernel or gemv_kernel (bs_sparse_kernel; 3 and 4 on large matrices: tile_forward_kernel) */
 #define BS_PATH_DECODE_MX  2   /* gemv_mx_kernel: the same on the block-scaled fp4 x fp6 MFMA, 1..2 tokens */
 #define BS_PATH_STRIP      3   /* up to 48 tokens, patches rebuilt in registers: tile_forward_kernel at rank 16, strip_forward_kernel elsewhere */
 #define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups (large matrices: column_forward_kernel) */
@@ -206,6 +207,16 @@ int bs_forward_path(int I, int M, int N, int K, int T);
 #define BS_TILE_COLUMN    3    /* column_forward_kernel (49 to 128 tokens) */
 #define BS_TILE_REBUILD   4    /* the weight rebuilt by tile_forward_kernel, then the dense product */
 int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns);
+
+/*
+ * Introspection for benchmarks and tests: 1 where gemv_sparse_kernel (the sign
+ * bits as the index operand of the sparse MFMA, one to three tokens) runs these
+ * matrices in the place of what bs_forward_path names: of gemv_kernel on most
+ * matrices, and of the strip and tile kernels at one and two tokens of larger ones
+ * whose column count is no multiple of 512.  bs_decode_plan then answers for it.
+ * 0 elsewhere.  Arguments and errors as bs_tile_kernel.  No counterpart in the reference.
+ */
+int bs_sparse_kernel(const int *I, const int *M, int n, int N, int K, int T);
 
 /*
  * Test and benchmark hook: 0 = choose the decode kernel of one- and two-token

@@ -1,0 +1,128 @@
+"""The sparse kernel (one to three tokens, the sign bits as the index operand of the sparse matrix instruction) at the edges of its units,
+against float64: nothing but y is rounded."""
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from bitstack_amd import _lib
+from bitstack_amd.utils import inference_utils as IU
+from bitstack_amd.utils.synthetic import synthetic_layer
+from oracle import c_oracle as C
+
+# (blocks, out features, in features, rank, tokens): rows about whole tiles of 16 and workgroups of 128, 256 and 512, column groups of 128
+# that leave a unit's lanes without columns, one unit per workgroup and several, ranges that end inside a row of units, ranks below 16
+CASES = [(1, 1, 512, 16, 2), (3, 17, 512, 16, 2), (2, 129, 1024, 5, 3), (5, 700, 1536, 16, 3), (14, 1300, 512, 16, 1), (5, 2100, 1024, 11, 1), (1, 4097, 4096, 16, 1), (3, 1025, 4096, 1, 3), (2, 14336, 2048, 16, 2),
+         (1, 14300, 4096, 16, 1), (16, 1000, 3584, 12, 3), (3, 4096, 4096, 16, 3), (2, 16, 128, 7, 2), (3, 100, 384, 3, 1), (4, 2053, 2176, 16, 1), (2, 4096, 11008, 16, 2),
+         (6, 3000, 1408, 16, 1), (1, 20001, 896, 16, 2), (8, 5000, 5504, 9, 1), (1, 40000, 640, 16, 1)]
+
+
+def test_which_calls_the_sparse_kernel_serves():
+    for I, M, N, K, T in CASES:
+        assert _lib.sparse_kernel([(I, M)], N, K, T), (I, M, N, K, T)
+        assert _lib.forward_kernel_name(I, M, N, K, T) == "gemv_sparse_kernel"
+    # every height of a workgroup at every token count
+    reached = {(_lib.decode_plan(I, M, N, 16, T)[1], T) for T in (1, 2, 3) for I, M, N in ((2, 2048, 2048), (2, 4096, 4096), (1, 14336, 4096), (1, 28672, 4096))}
+    assert reached == {(r, t) for r in (1, 2, 4) for t in (1, 2, 3)}
+    for I, M, N, K, T in [(8, 14336, 4096, 16, 1), (8, 14336, 4096, 16, 2), (2, 14336, 4096, 16, 4), (1, 5877, 640, 16, 1), (1, 1024, 4096, 16, 1), (4, 4096, 11008, 16, 3), (2, 64, 72, 16, 1), (2, 64, 128, 16, 5)]:
+        assert not _lib.sparse_kernel([(I, M)], N, K, T), (I, M, N, K, T)
+    L = _lib.lib()
+    try:
+        L.bs_set_decode_kernel(_lib.DECODE_F16)
+        assert not _lib.sparse_kernel([(3, 4096)], 4096, 16, 1) and _lib.forward_kernel_name(3, 4096, 4096, 16, 1).startswith("gemv_kernel")
+    finally:
+        L.bs_set_decode_kernel(_lib.DECODE_AUTO)
+
+
+@pytest.mark.skipif(not os.path.exists(shutil.which("hipcc") or "/opt/rocm/bin/hipcc"), reason="hipcc not available")
+def test_the_sparse_kernel_keeps_everything_in_registers(tmp_path):
+    asm, source = tmp_path / "k.s", os.path.join(os.path.dirname(_lib.LIB_PATH), "gemv_sparse.hip")
+    subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-S", "--cuda-device-only", source, "-o", str(asm)], check=True, capture_output=True)
+    sizes = re.findall(r"\.private_segment_fixed_size:\s+(\d+)", asm.read_text())
+    assert sizes and set(sizes) == {"0"}, sizes
+
+
+def _layer(I, M, N, K, T):
+    q, u, vt, x = synthetic_layer(M, N, I, T, k=K, seed=I + M + N + T, signed_factors=True)
+    u = (u * 20).half()
+    want = torch.from_numpy(C.forward_f64(q.numpy(), u.numpy(), vt.numpy(), x.numpy())).view(T, M)
+    size = torch.from_numpy(C.forward_f64(np.full_like(q.numpy(), 0xFF), u.abs().numpy(), vt.abs().numpy(), x.abs().numpy())).view(T, M)
+    return q.cuda(), u.cuda(), vt.cuda(), x.cuda(), want.cuda(), size.cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,K,T", CASES)
+def test_edges(I, M, N, K, T):
+    print(f"sparse kernel I={I} M={M} N={N} K={K} T={T}", flush=True)
+    assert _lib.sparse_kernel([(I, M)], N, K, T)
+    q, u, vt, x, want, size = _layer(I, M, N, K, T)
+    bias = torch.randn(M, device="cuda").half() if (M + T) % 2 else None
+    L = _lib.lib()
+    need = L.bs_workspace_bytes(I, M, N, K, T)
+    guard = torch.full((need + 256,), 0xFF, dtype=torch.uint8, device="cuda")        # nothing is read from scratch that the call has not written
+    room = torch.empty(u.numel() + 4, dtype=u.dtype, device="cuda")                  # u 8 bytes off a 16-byte boundary
+    room[4:] = u.flatten()
+    y = torch.full((T, M), float("nan"), dtype=torch.half, device="cuda")
+    for _ in range(2):
+        _lib.check(L.bs_forward(q.data_ptr(), room[4:].data_ptr(), vt.data_ptr(), x.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), I, M, N, K, T,
+                                guard.data_ptr(), need, torch.cuda.current_stream().cuda_stream), "bs_forward")
+    assert bool((guard[need:] == 0xFF).all())
+    assert torch.equal(IU.bitstack_forward_hip(q, u, vt, x, bias).view(T, M), y)
+    if bias is not None:
+        want, size = want + bias.double(), size + bias.double().abs()
+    # One rounding of y; exact products; fp32 sums over a unit's 16 operands of 32 columns, the units of a range, 16 ranks and the slots: fewer than
+    # 2^10 additions on the way, whose errors are random: 2^-18 of the sum of the magnitudes is five times their largest here.
+    assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,K,T", [(3, 1024, 4096, 16, 3), (4, 2053, 2176, 16, 2), (2, 300, 640, 6, 1)])
+def test_non_finite_inputs(I, M, N, K, T):
+    """An infinity or NaN in u, vt or x reaches the outputs it has a part in and no others."""
+    assert _lib.sparse_kernel([(I, M)], N, K, T)
+    q, u, vt, x, _, _ = _layer(I, M, N, K, T)
+    clean = IU.bitstack_forward_hip(q, u, vt, x, None).view(T, M)
+    keep = torch.arange(M, device="cuda") != 37
+    for value in (float("inf"), float("nan")):
+        bad = u.clone()
+        bad[1, 37, 3] = value
+        y = IU.bitstack_forward_hip(q, bad, vt, x, None).view(T, M)
+        assert not torch.isfinite(y[:, 37]).any() and torch.equal(y[:, keep], clean[:, keep])
+        for col in (0, 130, N - 1):
+            bad = x.clone()
+            bad.view(T, N)[T - 1, col] = value
+            y = IU.bitstack_forward_hip(q, u, vt, bad, None).view(T, M)
+            assert not torch.isfinite(y[T - 1]).any() and torch.equal(y[:T - 1], clean[:T - 1])
+            bad = vt.clone()
+            bad[I - 1, K - 1, col] = value
+            assert not torch.isfinite(IU.bitstack_forward_hip(q, u, bad, x, None)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 2, 3])
+@pytest.mark.parametrize("layers,N", [([(3, 4096), (1, 1024), (2, 1024)], 1024), ([(2, 700), (1, 33), (3, 3000), (1, 64)], 1024), ([(2, 2816), (3, 2816)], 1664)])
+def test_groups_with_the_epilogues(layers, N, T):
+    """Matrices in one launch: side by side against float64, then with the RMS scale of x, a residual and SwiGLU against what that gave."""
+    if T == 3 and N % 512:
+        pytest.skip("the tile kernel's")
+    assert _lib.sparse_kernel(layers, N, 16, T)
+    parts = [_layer(I, M, N, 16, T) for I, M in layers]
+    x, group = parts[0][3], IU.MatrixGroup([p[:3] + (None,) for p in parts])
+    refs = [C.forward_f64(*(t.cpu().numpy() for t in p[:3]), x.cpu().numpy()) for p in parts]
+    alone = torch.cat([torch.from_numpy(r).view(T, -1) for r in refs], 1).cuda()
+    # one rounding to fp16 each, and fp32 sums (2^-18 of the magnitudes' sum, here below 2^-14 of the largest result)
+    close = lambda a, b, bits: bool(((a.double() - b).abs() <= b.abs() * 2.0 ** -bits + b.abs().max() * 2.0 ** -14).all())
+    got = IU.bitstack_forward_group_hip(group, x)
+    assert close(got, alone, 10)
+    scale = torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-5)
+    assert close(IU.bitstack_forward_group_hip(group, x, rms_eps=1e-5), alone * scale, 9)
+    res = torch.randn(T, sum(m for _, m in layers), device="cuda").half()
+    assert close(IU.bitstack_forward_group_hip(group, x, epilogue=_lib.EPI_RESIDUAL, residual=res), res.double() + got.double(), 10)
+    if len(layers) == 2:
+        a, b = got[:, :layers[0][1]].double(), got[:, layers[0][1]:].double()
+        assert close(IU.bitstack_forward_group_hip(group, x, epilogue=_lib.EPI_SWIGLU), a * torch.sigmoid(a) * b, 8)

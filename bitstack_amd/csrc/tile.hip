@@ -24,7 +24,10 @@
 // three registers) of two waves run side by side on a SIMD, 1.0 ns each; v_fma_mix_f32, v_and_or_b32, v_bfe, v_alignbit, conversions and whatever
 // has a scalar operand take 1.8 ns, and a single wave issues one instruction in 2 ns whatever it is.  A step (1024 signs: 16 v_xor, 5 for the
 // table addresses, 4 lookups, one product) takes 45 ns per SIMD with two waves and 40 with four; with the signs as fp16 in v_fma_mix 46 and 42.
-// About 1300 cycles per tile and wave (barrier, hand-over, rounding, second product) come on top.  us, strip_forward_kernel / this, with the summing launch, in a
+// About 1300 cycles per tile and wave (barrier, hand-over, rounding, second product) come on top.  The loop over the tiles has no branch around a request or a
+// store: stores that have nothing to write go to an offset or a buffer that drops them, waves without columns do their work for nobody.  Where the compiler could
+// not tell how many were in flight, every tile waited for the requests made right before it and for its own stores (us with such branches / without: rebuild of
+// 4096 x 14336, 8 blocks 65.2 / 59.4, 14336 x 4096, 5 45.9 / 42.3; 10 blocks of 4096 x 4096, 8 tokens 23.9 / 22.5; a step of 8 sequences over two 70B-shape layers 662 / 642).  us, strip_forward_kernel / this, with the summing launch, in a
 // replayed graph on rotating copies: 28672 x 8192, 3 blocks, 8 tokens 86.5 / 62.8; 14336 x 4096, 8 blocks, 8 tokens 50.0 / 42.6; 5000 x 4096, 6 blocks, 37 tokens
 // 29.7 / 25.6; 4096 x 11008, 4 blocks, one token 26.1 / 24.4.
 #include "common.h"
@@ -58,6 +61,10 @@ __device__ __forceinline__ void tl_barrier() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+}
+// a buffer of so many bytes: what lies beyond is not written
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_buffer(const void *p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
 // wait until at most n of this wave's LDS accesses, which run in order, are to come
 template <int n>
@@ -125,41 +132,45 @@ struct TileKernel {
         const int lm = lane & 15, g = lane >> 4;                // in the second product
         const uint32_t row_bytes = (uint32_t)N >> 3;
         lds_bytes_rw area = lds + TL_TABLE, ring = area + AREA;
-        const int n0 = cg * CG + wave * WC;
-        const int active = min(TL_WAVES, (N - cg * CG) / WC);   // waves whose columns exist (all or none of a wave's)
-        const bool mine = wave < active;
+        // Waves whose columns exist (all or none of a wave's).  The others do the same work on the last columns, for nobody: a branch around it would
+        // leave the compiler unsure of what is in flight, and have it wait for stores behind the requests that it needs.
+        const int active = min(TL_WAVES, (N - cg * CG) / WC);
+        const int n0 = min(cg * CG + wave * WC, N - WC);
 
         // ---- requests: chunk c of a tile is 1 KB, signs of block c / SCH first, then the u rows of the blocks --------------
-        // Wave w takes chunks w, w + 8, ...
+        // Wave w takes chunks w, w + 8, ...; one that is short of a chunk takes the last one too.
         const char *from[MOST];                                  // row 0 of the next tile to be requested
         uint32_t pitch[MOST], offset[MOST];                      // the lane's piece within a tile
-        auto geometry = [&](int k, int rows) {                   // ... of which `rows` rows exist
-            const int c = min(wave + TL_WAVES * k, CHUNKS - 1);
+        auto chunk_of = [&](int k) { return MORE == 0 || k < PER ? wave + TL_WAVES * k : min(wave + TL_WAVES * k, CHUNKS - 1); };
+        auto geometry = [&](int c) {
             if (c < I * SCH) {
                 const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
-                return (uint32_t)min(r, rows - 1) * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
+                return (uint32_t)r * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
             }
             const int r = lane >> 1;
-            return (uint32_t)min(r, rows - 1) * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
+            return (uint32_t)r * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
         };
 #pragma unroll
         for (int k = 0; k < MOST; k++) {
-            const int c = min(wave + TL_WAVES * k, CHUNKS - 1);
+            const int c = chunk_of(k);
             const bool signs = c < I * SCH;
             from[k] = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
             pitch[k] = signs ? row_bytes : 32u;
             from[k] += (int64_t)(rt0 * TL_ROWS) * pitch[k];
-            offset[k] = geometry(k, TL_ROWS);
+            offset[k] = geometry(c);
         }
         // A tile's pieces travel through registers: requested three tiles ahead, written to LDS at the end of the tile two ahead of it.
         int asked = rt0;                                         // the row tile `from` stands at
         const int last_rt = rt0 + len - 1;
         uint4_t pieces[MOST], pieces_1[MOST];                    // (pieces_1: only of the run's second tile)
-        auto request_next = [&](uint4_t (&to)[MOST]) {           // (behind the last tile that one is requested again)
-            const int rows = M - asked * TL_ROWS;
+        // (Behind the last tile that one is requested again.  A tile is a buffer that ends with the matrix's last row; rows beyond it read as zeros.)
+        auto request_next = [&](uint4_t (&to)[MOST]) {
+            const uint32_t rows = min(M - asked * TL_ROWS, TL_ROWS);
 #pragma unroll
-            for (int k = 0; k < MOST; k++)
-                if (k < PER || wave < MORE) to[k] = *reinterpret_cast<const uint4_t *>(from[k] + (rows >= TL_ROWS ? offset[k] : geometry(k, rows)));
+            for (int k = 0; k < MOST; k++) {
+                to[k] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from[k], (int)(rows * pitch[k])), (int)offset[k], 0, 0);
+                __builtin_amdgcn_sched_barrier(0);               // (in the same order wherever they are issued: the waits count on it)
+            }
             if (asked < last_rt) {
                 asked++;
 #pragma unroll
@@ -167,10 +178,8 @@ struct TileKernel {
             }
         };
         auto write_tile = [&](int stage, const uint4_t (&p)[MOST]) {
-            lds_uint4_rw to = (lds_uint4_rw)(ring + stage * STAGE + wave * 1024) + lane;
 #pragma unroll
-            for (int k = 0; k < MOST; k++)
-                if (k < PER || wave < MORE) to[k * (TL_WAVES * 64)] = p[k];
+            for (int k = 0; k < MOST; k++) ((lds_uint4_rw)(ring + stage * STAGE + chunk_of(k) * 1024))[lane] = p[k];
         };
 #pragma unroll
         for (int k = 0; k < MOST; k++) pieces[k] = pieces_1[k] = (uint4_t){0, 0, 0, 0};
@@ -184,7 +193,7 @@ struct TileKernel {
         half8_t vf[I][NP];
         constexpr int TX = TT ? TT : 1;
         half8_t xf[TX][NP];
-        if (mine) {
+        {
             constexpr int PIECES = WC / 8, BP = 32 / PIECES, PASSES = (I + BP - 1) / BP, IMAGE = WC * 32;   // BP blocks per pass of loads
             constexpr int ROOM = (AREA / TL_WAVES < 8192 ? AREA / TL_WAVES : 8192), SB = ROOM / IMAGE;      // SB of them fit the image
             lds_bytes_rw img = area + wave * ROOM;
@@ -233,18 +242,16 @@ struct TileKernel {
         if (TT > 0 && ssq) {          // sums of squares of x over the group's columns
             lds_f32_rw sums = (lds_f32_rw)area;
             __syncthreads();                         // (the area holds the vt images)
-            if (mine) {
 #pragma unroll
-                for (int tt = 0; tt < TT; tt++) {
-                    float q = 0.f;
+            for (int tt = 0; tt < TT; tt++) {
+                float q = 0.f;
 #pragma unroll
-                    for (int p = 0; p < NP; p++)
+                for (int p = 0; p < NP; p++)
 #pragma unroll
-                        for (int k = 0; k < 8; k++) q += (float)xf[tt][p][k] * (float)xf[tt][p][k];
-                    q += __shfl_xor(q, 16, 64);
-                    q += __shfl_xor(q, 32, 64);
-                    if (g == 0) sums[wave * (16 * TT) + tt * 16 + lm] = q;
-                }
+                    for (int k = 0; k < 8; k++) q += (float)xf[tt][p][k] * (float)xf[tt][p][k];
+                q += __shfl_xor(q, 16, 64);
+                q += __shfl_xor(q, 32, 64);
+                if (g == 0) sums[wave * (16 * TT) + tt * 16 + lm] = q;
             }
             __syncthreads();
             if (tid < T) {
@@ -271,18 +278,22 @@ struct TileKernel {
             }
         };
         auto hand_over = [&](int rt, int tt, const float (&v)[TL_WAVES], bool valid) {
-            if (!takes(tt) || !valid) return;
-            float sum = v[0];
-            if (active == TL_WAVES) {
+            float sum = 0.f;
+            if (takes(tt)) {
+                sum = v[0];
+                if (active == TL_WAVES) {
 #pragma unroll
-                for (int w = 1; w < TL_WAVES; w++) sum += v[w];
-            } else {
+                    for (int w = 1; w < TL_WAVES; w++) sum += v[w];
+                } else {
 #pragma unroll
-                for (int w = 1; w < TL_WAVES; w++)
-                    if (w < active) sum += v[w];
+                    for (int w = 1; w < TL_WAVES; w++)
+                        if (w < active) sum += v[w];
+                }
             }
-            char *const to = reinterpret_cast<char *>(out + ((int64_t)(16 * tt) * M + rt * TL_ROWS));
-            if (16 * tt + my_t < T && rt * TL_ROWS + my_row < M) *reinterpret_cast<float *>(to + my_out) = sum;
+            // (Always issued, to an offset or a buffer of no size that drops it where there is nothing to write: with a store that may or may not be on
+            // its way the wait for the requests behind it is a wait for everything.)
+            const uint32_t at = 16 * tt + my_t < T && rt * TL_ROWS + my_row < M ? my_out : 0xFFFFFFFFu;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum), tl_buffer(out + ((int64_t)(16 * tt) * M + rt * TL_ROWS), valid ? -1 : 0), (int)at, 0, 0);
         };
         // the second product's result: rows 0-15 ([tt][0]) and 16-31 ([tt][1]) of a tile, D[token 4 g + j, row lm] of each
         float4_t y[TX][2];
@@ -303,7 +314,7 @@ struct TileKernel {
         // into four masks; they are looked up LOOK steps ahead, u rows and sign words SETS - 1 blocks ahead, across the end of a tile: the barrier
         // that opens tile n also says that tile n + 1 is in LDS.  The fences keep the compiler from moving the lookups of many steps
         // ahead, for which there are no registers.
-        constexpr int STEPS = (I + 1) * NP, SETS = NP == 4 ? 2 : NP == 2 ? 3 : 4, LOOK = TT == 1 && (NP == 1 || (NP == 2 && I <= 8)) ? 2 : 1;
+        constexpr int STEPS = (I + 1) * NP, SETS = NP == 4 ? 2 : NP == 2 ? 3 : 4, LOOK = NP == 1 || (NP == 2 && I <= 8) ? 2 : 1;
         const int mine_at = wave * (WC / 8) + h * (WC / 16);     // byte of a sign row: this lane's WC / 2 columns
         const int sread = row * SROW + ((mine_at >> 4) ^ swizzle(row)) * 16 + (mine_at & 15);
         const int uread = I * SCH * 1024 + row * 32 + 16 * (h ^ ((row >> 4) & 1));
@@ -352,10 +363,8 @@ struct TileKernel {
         };
         tl_wait_lds<0>();
         tl_barrier();                                // the first tile is here, everybody is done with the images
-        if (mine) {
-            fetch_first(ring);
-            first_block();
-        }
+        fetch_first(ring);
+        first_block();
         if constexpr (NP == 4) {                     // (no registers for two tiles' pieces)
             write_tile(1, pieces);
             request_next(pieces);
@@ -365,19 +374,22 @@ struct TileKernel {
         // of a tile are issued between the steps of the next one, all at once they would be waited for.
         constexpr int CH = 4 * NP, STORES = TL_ROWS * CH / 64;       // chunks per row, store instructions per tile
         const auto place = [&](int r, int c) { return (lds_half8_rw)(area + wave * (TL_ROWS * WC * 2) + r * (WC * 2) + ((c ^ (r * CH / 16)) % CH) * 16); };
-        const uint32_t w_lane = (uint32_t)(lane / CH) * (uint32_t)N + 8 * (lane % CH);
-        auto store_from = [&](int rt, int k, const half8_t &o) {
-            if (rt * TL_ROWS + k * (64 / CH) + lane / CH < M) *reinterpret_cast<half8_t *>(w + (int64_t)(rt * TL_ROWS + k * (64 / CH)) * N + n0 + w_lane) = o;
+        const uint32_t w_lane = ((uint32_t)(lane / CH) * (uint32_t)N + n0 + 8 * (lane % CH)) * 2u;
+        // (the tile as a buffer that ends with the last row: rows beyond it, and all of them where there is no tile, are dropped)
+        auto tile_of = [&](int rt, bool valid) { return tl_buffer(w + (int64_t)(rt * TL_ROWS) * N, valid ? min(TL_ROWS, M - rt * TL_ROWS) * N * 2 : 0); };
+        auto store_to = [&](__amdgpu_buffer_rsrc_t tile, int k, const half8_t &o) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, o), tile, (int)(w_lane + (uint32_t)(k * (64 / CH)) * (uint32_t)N * 2u), 0, 0);
         };
         auto chunk = [&](int k) { return *place(k * (64 / CH) + lane / CH, lane % CH); };
+        if constexpr (TT == 0 && NP == 4) {          // (as many stores, all dropped, behind the requests as there are at the end of the loop: the wait counts both)
+#pragma unroll
+            for (int c = 0; c < STORES; c++) store_to(tile_of(rt0, false), c, (half8_t){0, 0, 0, 0, 0, 0, 0, 0});
+        }
         int stage = 0;
 #pragma clang loop unroll(disable)
         for (int n = 0; n < len; n++) {
             __builtin_amdgcn_s_setprio(0);
-            if (mine)
-                tl_wait_lds<4>();                    // (its last LDS writes lie a step's four lookups or more back)
-            else
-                tl_wait_lds<0>();
+            tl_wait_lds<4>();                        // (its last LDS writes lie a step's four lookups or more back)
             tl_barrier();                            // tile n + 1 and the y tiles of n - 2 are in LDS, the stage of n - 1 is free
             const int free_stage = stage == 0 ? STAGES - 1 : stage - 1;
             lds_bytes st = ring + stage * STAGE;
@@ -392,172 +404,162 @@ struct TileKernel {
             };
             if constexpr (NP == 4) pass_on();        // (at the end it would take eight registers more than there are)
             float v[TL_WAVES];
-            if (mine) {
-                tl_for<STEPS - NP>([&](auto sc) {
-                    constexpr int k = decltype(sc)::value, s = k + NP, i = s / NP, p = s % NP;
-                    // (of the two waves of a SIMD the older one goes first; so that both come to the barrier together, the younger one does in the
-                    // second half)
-                    if constexpr (k == (STEPS - NP) / 2)
-                        if (wave >= TL_WAVES / 2) __builtin_amdgcn_s_setprio(1);
-                    look_up(std::integral_constant<int, s + LOOK>{});
-                    if constexpr (p == 0 && i < I && i + SETS - 1 < I) fetch(st, std::integral_constant<int, i + SETS - 1>{});
-                    if constexpr (s == STEPS - NP) fetch_first(st_next);
-                    if constexpr (k % 2 == 0 && k / 2 >= 1 && k / 2 <= TT) hand_over(rt0 + n - 2, k / 2 - 1, v, n >= 2);
-                    if constexpr (k % 2 == 0 && k / 2 < TT) collect(oldest, k / 2, v);
-                    // (the weight's stores C .. D - 1 of the last tile go with this step)
-                    constexpr int C = TT ? 0 : (STORES * k + STEPS - NP - 1) / (STEPS - NP), D = TT ? 0 : (STORES * (k + 1) + STEPS - NP - 1) / (STEPS - NP);
-                    half8_t out[D > C ? D - C : 1];
+            [[maybe_unused]] const __amdgpu_buffer_rsrc_t last_tile = tile_of(rt0 + n - 1, TT == 0 && n > 0 && wave < active);
+            tl_for<STEPS - NP>([&](auto sc) {
+                constexpr int k = decltype(sc)::value, s = k + NP, i = s / NP, p = s % NP;
+                // (of the two waves of a SIMD the older one goes first; so that both come to the barrier together, the younger one does in the
+                // second half)
+                if constexpr (k == (STEPS - NP) / 2)
+                    if (wave >= TL_WAVES / 2) __builtin_amdgcn_s_setprio(1);
+                look_up(std::integral_constant<int, s + LOOK>{});
+                if constexpr (p == 0 && i < I && i + SETS - 1 < I) fetch(st, std::integral_constant<int, i + SETS - 1>{});
+                if constexpr (s == STEPS - NP) fetch_first(st_next);
+                if constexpr (k % 2 == 0 && k / 2 >= 1 && k / 2 <= TT) hand_over(rt0 + n - 2, k / 2 - 1, v, n >= 2);
+                if constexpr (k % 2 == 0 && k / 2 < TT) collect(oldest, k / 2, v);
+                // (the weight's stores C .. D - 1 of the last tile go with this step)
+                constexpr int C = TT ? 0 : (STORES * k + STEPS - NP - 1) / (STEPS - NP), D = TT ? 0 : (STORES * (k + 1) + STEPS - NP - 1) / (STEPS - NP);
+                half8_t out[D > C ? D - C : 1];
 #pragma unroll
-                    for (int c = C; c < D; c++) out[c - C] = chunk(c);
-                    __builtin_amdgcn_sched_barrier(0);
-                    asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
+                for (int c = C; c < D; c++) out[c - C] = chunk(c);
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
 #pragma unroll
-                    for (int q = 0; q < 4; q++)
+                for (int q = 0; q < 4; q++)
 #pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            const float sum = acc[p][4 * q + j];
-                            const uint32_t m = mask[s % (LOOK + 1)][q][j];
-                            acc[p][4 * q + j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
-                        }
-                    if constexpr (i < I)
-                        acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
-                    asm volatile("" : "+v"(acc[p]));
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (D > C && n > 0) {
-#pragma unroll
-                        for (int c = C; c < D; c++) store_from(rt0 + n - 1, c, out[c - C]);
+                    for (int j = 0; j < 4; j++) {
+                        const float sum = acc[p][4 * q + j];
+                        const uint32_t m = mask[s % (LOOK + 1)][q][j];
+                        acc[p][4 * q + j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
                     }
-                    if constexpr (TT > 0 && k == (STEPS - NP > 1 ? 1 : 0)) leave(before);
-                });
-                // (the passes for which there were not enough steps)
-                constexpr int COLLECTED = (STEPS - NP + 1) / 2 < TT ? (STEPS - NP + 1) / 2 : TT, HANDED = (STEPS - NP - 1) / 2 < TT ? (STEPS - NP - 1) / 2 : TT;
-                if constexpr (HANDED < COLLECTED) hand_over(rt0 + n - 2, COLLECTED - 1, v, n >= 2);
-                tl_for<TT - COLLECTED>([&](auto k) {
-                    collect(oldest, COLLECTED + decltype(k)::value, v);
-                    hand_over(rt0 + n - 2, COLLECTED + decltype(k)::value, v, n >= 2);
-                });
-                if constexpr (NP < 4) pass_on();
-                if constexpr (TT == 0) {
-                    // One rounding to fp16; a lane holds columns 16 NP h .. + 16 NP - 1 of row l % 32
+                if constexpr (i < I)
+                    acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
+                asm volatile("" : "+v"(acc[p]));
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (D > C) {
+#pragma unroll
+                    for (int c = C; c < D; c++) store_to(last_tile, c, out[c - C]);
+                }
+                if constexpr (TT > 0 && k == (STEPS - NP > 1 ? 1 : 0)) leave(before);
+            });
+            // (the passes for which there were not enough steps)
+            constexpr int COLLECTED = (STEPS - NP + 1) / 2 < TT ? (STEPS - NP + 1) / 2 : TT, HANDED = (STEPS - NP - 1) / 2 < TT ? (STEPS - NP - 1) / 2 : TT;
+            if constexpr (HANDED < COLLECTED) hand_over(rt0 + n - 2, COLLECTED - 1, v, n >= 2);
+            tl_for<TT - COLLECTED>([&](auto k) {
+                collect(oldest, COLLECTED + decltype(k)::value, v);
+                hand_over(rt0 + n - 2, COLLECTED + decltype(k)::value, v, n >= 2);
+            });
+            if constexpr (NP < 4) pass_on();
+            if constexpr (TT == 0) {
+                // One rounding to fp16; a lane holds columns 16 NP h .. + 16 NP - 1 of row l % 32
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        half8_t o;
+#pragma unroll
+                        for (int k = 0; k < 8; k++) o[k] = (half_t)acc[p][8 * e + k];
+                        *place(row, 2 * NP * h + 2 * p + e) = o;
+                    }
+                asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
+                first_block();                               // of tile n + 1
+            } else if constexpr (SPLIT) {
+                // Two terms per weight: rounded towards zero, and 2^18 times what that leaves, in sums of its own, so that it is no subnormal number where
+                // the weight is small (lost: 2^-21 of a weight, 2^-12 of one below 2^-24, and never less than 2^-44).  The lanes trade places as below.
+                constexpr float UP = 262144.f;
+                float4_t rest[2];
+#pragma unroll
+                for (int r = 0; r < 2; r++) y[0][r] = rest[r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    half2_t t[2][8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const float a = acc[p][2 * k], b = acc[p][2 * k + 1];
+                        t[0][k] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+                        t[1][k] = (half2_t){(half_t)__builtin_fmaf((float)t[0][k][0], -UP, UP * a), (half_t)__builtin_fmaf((float)t[0][k][1], -UP, UP * b)};
+                    }
+#pragma unroll
+                    for (int term = 1; term >= 0; term--) {
+                        uint4_t lo, hi;
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const half2_t a = t[term][k], b = t[term][4 + k];
+                            const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                            lo[k] = r[0];
+                            hi[k] = r[1];
+                        }
+                        float4_t (&sum)[2] = term == 0 ? y[0] : rest;
+                        sum[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), sum[0], 0, 0, 0);
+                        sum[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), sum[1], 0, 0, 0);
+                    }
+                }
+                // A weight that the terms cannot hold (from about 256 on, where 2^18 * 2^-10 of it is beyond fp16, or infinite) leaves an infinity or
+                // a NaN in the second one, whatever its sign, and so in every y of its row.  Such y come from the fp32 weights instead.
+                float any = 0.f;
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        any += rest[r][j];
+                        y[0][r][j] = __builtin_fmaf(rest[r][j], 1.f / UP, y[0][r][j]);
+                    }
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(any)) != 0, 0)) {
+                    float4_t full[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
                     for (int p = 0; p < NP; p++)
 #pragma unroll
-                        for (int e = 0; e < 2; e++) {
-                            half8_t o;
-#pragma unroll
-                            for (int k = 0; k < 8; k++) o[k] = (half_t)acc[p][8 * e + k];
-                            *place(row, 2 * NP * h + 2 * p + e) = o;
-                        }
-                    asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
-                    first_block();                               // of tile n + 1
-                } else if constexpr (SPLIT) {
-                    // Two terms per weight: rounded towards zero, and 2^18 times what that leaves, in sums of its own, so that it is no subnormal number where
-                    // the weight is small (lost: 2^-21 of a weight, 2^-12 of one below 2^-24, and never less than 2^-44).  The lanes trade places as below.
-                    constexpr float UP = 262144.f;
-                    float4_t rest[2];
-#pragma unroll
-                    for (int r = 0; r < 2; r++) y[0][r] = rest[r] = (float4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int p = 0; p < NP; p++) {
-                        half2_t t[2][8];
-#pragma unroll
                         for (int k = 0; k < 8; k++) {
-                            const float a = acc[p][2 * k], b = acc[p][2 * k + 1];
-                            t[0][k] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-                            t[1][k] = (half2_t){(half_t)__builtin_fmaf((float)t[0][k][0], -UP, UP * a), (half_t)__builtin_fmaf((float)t[0][k][1], -UP, UP * b)};
+                            const float a = acc[p][k], b = acc[p][8 + k];
+                            const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                            const uint32_t lo = w[0], hi = w[1];
+                            full[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, lo), full[0], 0, 0, 0);
+                            full[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, hi), full[1], 0, 0, 0);
                         }
-#pragma unroll
-                        for (int term = 1; term >= 0; term--) {
-                            uint4_t lo, hi;
-#pragma unroll
-                            for (int k = 0; k < 4; k++) {
-                                const half2_t a = t[term][k], b = t[term][4 + k];
-                                const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-                                lo[k] = r[0];
-                                hi[k] = r[1];
-                            }
-                            float4_t (&sum)[2] = term == 0 ? y[0] : rest;
-                            sum[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, lo), sum[0], 0, 0, 0);
-                            sum[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][p], __builtin_bit_cast(half8_t, hi), sum[1], 0, 0, 0);
-                        }
-                    }
-                    // A weight that the terms cannot hold (from about 256 on, where 2^18 * 2^-10 of it is beyond fp16, or infinite) leaves an infinity or
-                    // a NaN in the second one, whatever its sign, and so in every y of its row.  Such y come from the fp32 weights instead.
-                    float any = 0.f;
 #pragma unroll
                     for (int r = 0; r < 2; r++)
 #pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            any += rest[r][j];
-                            y[0][r][j] = __builtin_fmaf(rest[r][j], 1.f / UP, y[0][r][j]);
-                        }
-                    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(any)) != 0, 0)) {
-                        float4_t full[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-                        for (int p = 0; p < NP; p++)
-#pragma unroll
-                            for (int k = 0; k < 8; k++) {
-                                const float a = acc[p][k], b = acc[p][8 + k];
-                                const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-                                const uint32_t lo = w[0], hi = w[1];
-                                full[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, lo), full[0], 0, 0, 0);
-                                full[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)xf[0][p][k], __builtin_bit_cast(float, hi), full[1], 0, 0, 0);
-                            }
-#pragma unroll
-                        for (int r = 0; r < 2; r++)
-#pragma unroll
-                            for (int j = 0; j < 4; j++)
-                                if (!__builtin_isfinite(y[0][r][j])) y[0][r][j] = full[r][j];
-                    }
-                    first_block();                   // of tile n + 1
-                } else {
-                // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
-                // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
-                // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
-                // v_mfma_f32_16x16x32_f16.
-                half8_t wf[NP][2];
-#pragma unroll
-                for (int p = 0; p < NP; p++) {
-                    uint4_t lo, hi;
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
-                        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-                        lo[k] = r[0];
-                        hi[k] = r[1];
-                    }
-                    wf[p][0] = __builtin_bit_cast(half8_t, lo);
-                    wf[p][1] = __builtin_bit_cast(half8_t, hi);
+                        for (int j = 0; j < 4; j++)
+                            if (!__builtin_isfinite(y[0][r][j])) y[0][r][j] = full[r][j];
                 }
-                first_block();                       // of tile n + 1
-#pragma unroll
-                for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                    for (int r = 0; r < 2; r++) {
-                        y[tt][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
-                    }
-                }
+                first_block();                   // of tile n + 1
             } else {
-                if constexpr (NP < 4) pass_on();
+            // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
+            // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
+            // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
+            // v_mfma_f32_16x16x32_f16.
+            half8_t wf[NP][2];
 #pragma unroll
-                for (int tt = 0; tt < TT; tt++) {
-                    collect(oldest, tt, v);
-                    hand_over(rt0 + n - 2, tt, v, n >= 2);
+            for (int p = 0; p < NP; p++) {
+                uint4_t lo, hi;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
+                    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                    lo[k] = r[0];
+                    hi[k] = r[1];
+                }
+                wf[p][0] = __builtin_bit_cast(half8_t, lo);
+                wf[p][1] = __builtin_bit_cast(half8_t, hi);
+            }
+            first_block();                       // of tile n + 1
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    y[tt][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
                 }
             }
         }
         if (TT == 0) {
-            if (mine) {
 #pragma unroll
-                for (int c = 0; c < STORES; c++) store_from(last_rt, c, chunk(c));
-            }
+            for (int c = 0; c < STORES; c++) store_to(tile_of(last_rt, wave < active), c, chunk(c));
             return;
         }
         // the last two tiles
         if (len > 2) tl_barrier();                   // (everybody has collected the tile whose place this is)
-        if (mine) leave((len & 1) ^ 1);
+        leave((len & 1) ^ 1);
         tl_wait_lds<0>();
         tl_barrier();
 #pragma unroll

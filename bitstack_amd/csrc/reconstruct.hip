@@ -18,6 +18,7 @@
 // next block are loaded while the current block is multiplied.
 #include "common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -28,6 +29,7 @@ constexpr int VGROUP_PAD = 4;  // extra halves after every 8 columns (keeps the 
 constexpr int VBLOCK = RT_COLS * VSTRIDE + (RT_COLS / 8) * VGROUP_PAD;   // halves per block in LDS
 constexpr int RT_MAXB = 36;    // most blocks whose vt strip fits in LDS (36 x 4.1 KB)
 constexpr int SIGN_LUT_HALVES = 64;   // 16 nibbles x 4 signs
+constexpr int RA_MAXB = 39;    // ... of reconstruct_byte_kernel (39 x 4 KB beside its sign table)
 
 // K16: the rank is 16 (every u fragment is one 8-byte load).  Smaller ranks pick their halves one by one behind
 // branches, and the compiler then waits for every load in flight where the branches meet: that instantiation runs
@@ -255,6 +257,133 @@ __global__ __launch_bounds__(256, 4) void reconstruct_tile_kernel(
     }
 }
 
+// Column counts that are multiples of 8 but not of 128 (and what else the tiled kernel declines of those): rows of sign bytes then start anywhere, and the last
+// columns fill no strip.  A workgroup of 8 waves takes 128 columns, whose vt fragments of all blocks it leaves in LDS first; a wave has 64 of them and every fourth
+// step of 32 rows, in two patches of v_mfma_f32_32x32x16_f16, D[column, row], with the columns dealt so that a lane ends with 32 consecutive ones of one row: one
+// unaligned word of signs, four 16-byte stores.  u rows and signs are requested one (row step, block) ahead, in two register sets that take turns.  Signs come out of
+// the tiled kernel's table and go in by the same mixed-precision FMA (int8 signs: converted; the same sum).
+// What bounds it: the vector instructions, 24 per step of 1024 signs, and its stores.  Rebuilds, us, one output per thread / this: 4096 x 4104
+// of 1 block 101 / 18, of 4 385 / 23; 6144 x 6136 of 8 1641 / 53; 512 x 6008 of 4 63 / 8.2; 1000 x 1000 of 4 23 / 5.4.  (Four waves, each with 128 columns as the
+// tiled kernel has them, and vt fragments in registers for the block at hand: 23 to 85 where this takes 19 to 53.)
+constexpr int RA_COLS = 128, RA_ROWS = 32, RA_WAVES = 8, RA_STREAMS = 4;         // columns per workgroup, rows per step, waves, waves side by side in rows
+template <bool PACKED, bool K16>
+__global__ __launch_bounds__(64 * RA_WAVES, PACKED ? 4 : 2) void reconstruct_byte_kernel(
+    const uint8_t *__restrict__ packed, const int8_t *__restrict__ sign, const half_t *__restrict__ u, const half_t *__restrict__ vt, half_t *__restrict__ w,
+    int I, int M, int N, int K, int strips, int steps_per_wg) {
+    extern __shared__ __attribute__((aligned(128))) half_t lds_all[];
+    typedef const __attribute__((address_space(3))) half4_t *lds_half4_ptr;
+    const uint32_t lut = (uint32_t)reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) half_t *)lds_all);
+    half8_t *const frags = reinterpret_cast<half8_t *>(lds_all + SIGN_LUT_HALVES);      // [block][64 columns: 2][patch: 2][lane]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = lane & 31, h = lane >> 5;
+    // every XCD gets a contiguous run of (row group, strip), strips fastest: neighbours share lines of sign bytes and u rows
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, base = nb >> 3, rem = nb & 7;
+    const int v = xcd * base + min(xcd, rem) + loc, group = v / strips, strip = (v - group * strips) * RA_COLS;
+    if (tid < SIGN_LUT_HALVES) lds_all[tid] = ((tid >> 2) >> (3 - (tid & 3))) & 1 ? (half_t)1.f : (half_t)-1.f;
+    // patch p, row a of D: column 32 ((a / 4) % 2) + 16 p + 4 (a / 8) + a % 4
+    for (int item = wave; item < 4 * I; item += RA_WAVES) {
+        const int i = item >> 2, col = min(strip + 64 * ((item >> 1) & 1) + 32 * ((row >> 2) & 1) + 16 * (item & 1) + 4 * (row >> 3) + (row & 3), N - 1);
+        half8_t f;
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const half_t val = vt[((int64_t)i * K + (K16 ? 8 * h + r : min(8 * h + r, K - 1))) * N + col];
+            f[r] = K16 || 8 * h + r < K ? val : (half_t)0;
+        }
+        frags[64 * item + lane] = f;
+    }
+    __syncthreads();
+
+    const int c0 = strip + 64 * (wave & 1) + 32 * h;             // this lane's columns; beyond N: others are read, nothing is stored
+    const int first = group * steps_per_wg + (wave >> 1), last = min((group + 1) * steps_per_wg, (M + RA_ROWS - 1) / RA_ROWS);
+    const int cr = min(c0, N - 32), late = min(c0 - cr, 31);     // (the last columns' word starts earlier, by a multiple of 8 signs)
+    struct Ahead {
+        half8_t u;
+        uint32_t bits;                               // packed
+        uint2_t bytes[4];                            // int8
+    };
+    int ask_step = first, ask_i = 0;
+    auto request = [&](Ahead &a) {                   // (behind the last one that one is requested again)
+        const int m = min(ask_step * RA_ROWS + row, M - 1);
+        const half_t *up = u + ((int64_t)ask_i * M + m) * K;
+        if (K16) {
+            const half4_t lo = *reinterpret_cast<const half4_t *>(up + 8 * h), hi = *reinterpret_cast<const half4_t *>(up + 8 * h + 4);
+            a.u = (half8_t){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 8; r++) a.u[r] = up[min(8 * h + r, K - 1)];
+        }
+        const int64_t at = ((int64_t)ask_i * M + m) * N;
+        if (PACKED) {
+            __builtin_memcpy(&a.bits, packed + ((at + cr) >> 3), 4);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) a.bytes[e] = *reinterpret_cast<const uint2_t *>(sign + at + min(c0 + 8 * e, N - 8));
+        }
+        if (ask_step + RA_STREAMS < last || ask_i + 1 < I) {
+            if (++ask_i == I) {
+                ask_i = 0;
+                ask_step += RA_STREAMS;
+            }
+        }
+    };
+    float16_t acc[2];
+    int step = first, i = 0;
+    auto consume = [&](const Ahead &a) {
+        if (i == 0) acc[0] = acc[1] = (float16_t){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        half8_t b = a.u;
+        if (!K16) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) b[r] = 8 * h + r < K ? b[r] : (half_t)0;
+        }
+        float16_t p[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            p[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frags[64 * (4 * i + 2 * (wave & 1) + k) + lane], b,
+                                (float16_t){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (PACKED) {
+            const uint32_t bits = a.bits >> late;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {            // columns 4 q .. 4 q + 3: the upper half of byte q / 2 first
+                constexpr uint32_t NIBBLE = 0x78u;
+                const int sh = 8 * (q >> 1) + (q & 1 ? -3 : 1);
+                const half4_t sv = *reinterpret_cast<lds_half4_ptr>((uintptr_t)((((sh < 0 ? bits << 3 : bits >> sh)) & NIBBLE) | lut));
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[q >> 2][4 * (q & 3) + j] = __builtin_fmaf(p[q >> 2][4 * (q & 3) + j], (float)sv[j], acc[q >> 2][4 * (q & 3) + j]);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 32; k++)
+                acc[k >> 4][k & 15] = __builtin_fmaf(p[k >> 4][k & 15], (float)(int8_t)(a.bytes[k >> 3][(k >> 2) & 1] >> (8 * (k & 3))), acc[k >> 4][k & 15]);
+        }
+        if (++i == I) {
+            const int m = step * RA_ROWS + row;
+            if (m < M) {
+                half_t *to = w + (int64_t)m * N + c0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    half8_t o;
+#pragma unroll
+                    for (int k = 0; k < 8; k++) o[k] = (half_t)acc[e >> 1][8 * (e & 1) + k];
+                    if (c0 + 8 * e < N) *reinterpret_cast<half8_t *>(to + 8 * e) = o;
+                }
+            }
+            i = 0;
+            step += RA_STREAMS;
+        }
+    };
+    if (first >= last || strip + 64 * (wave & 1) >= N) return;
+    Ahead even, odd;
+    const int n = ((last - first + RA_STREAMS - 1) / RA_STREAMS) * I;
+    request(even);
+    for (int k = 0; k < n; k += 2) {
+        request(odd);
+        consume(even);
+        if (k + 1 == n) break;
+        request(even);
+        consume(odd);
+    }
+}
+
 // Any shape (also rows that do not start on a byte boundary): one output per
 // thread, bit addressed through the flat element index.
 template <bool PACKED>
@@ -315,6 +444,20 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
             reconstruct_tile_kernel<PACKED, true><<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
         else
             reconstruct_tile_kernel<PACKED, false><<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
+    } else if (N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && bs_aligned(u, 8) && (PACKED || bs_aligned(sign, 8))) {
+        const int strips = (int)bs_cdiv(N, RA_COLS), steps = (int)bs_cdiv(M, RA_ROWS);
+        const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), steps / RA_STREAMS));    // four workgroups per CU, a step per wave or more
+        const int per = (int)bs_cdiv(bs_cdiv(steps, groups), RA_STREAMS) * RA_STREAMS;
+        const size_t lds = SIGN_LUT_HALVES * sizeof(half_t) + (size_t)I * 256 * sizeof(half8_t);
+        static bs_lds_grant granted[2][BS_MAX_DEVICES];
+        const void *kernel = K == 16 ? (const void *)reconstruct_byte_kernel<PACKED, true> : (const void *)reconstruct_byte_kernel<PACKED, false>;
+        const int st = bs_allow_lds(kernel, lds, granted[K == 16]);
+        if (st != BS_OK) return st;
+        const int grid = strips * (int)bs_cdiv(steps, per);
+        if (K == 16)
+            reconstruct_byte_kernel<PACKED, true><<<grid, 64 * RA_WAVES, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, strips, per);
+        else
+            reconstruct_byte_kernel<PACKED, false><<<grid, 64 * RA_WAVES, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, strips, per);
     } else {
         int64_t blocks = bs_cdiv((int64_t)M * N, 256);
         if (blocks > 256 * 64) blocks = 256 * 64;

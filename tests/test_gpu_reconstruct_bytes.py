@@ -1,0 +1,40 @@
+"""The weight rebuild for column counts that are multiples of 8 but fill no 128-column strip
+(``reconstruct_byte_kernel``), against the same sum in float64, with packed and with int8 signs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# one row; the last columns' word of signs starting early; a partial last row step; ranks below 16, also odd ones; a rank the tiled
+# kernel declines at a multiple of 128; the most blocks that fit LDS and one more; fewer columns than a word of signs
+CASES = [(1, 1, 8, 16), (1, 1, 32, 16), (2, 40, 72, 16), (3, 33, 200, 5), (5, 129, 136, 1), (3, 65, 40, 9), (16, 31, 1016, 16), (39, 64, 264, 12),
+         (40, 64, 264, 12), (39, 64, 256, 16), (2, 4096, 4104, 16), (1, 3000, 120, 16)]
+
+
+def exact(packed, u, vt):
+    blocks, m, n = len(u), u.shape[1], vt.shape[2]
+    bits = (packed.view(blocks, -1, 1) >> torch.arange(7, -1, -1, device=packed.device, dtype=torch.uint8)) & 1
+    want = torch.zeros(m, n, dtype=torch.float64, device=packed.device)
+    size = torch.zeros_like(want)
+    for i in range(blocks):
+        want += (u[i].double() @ vt[i].double()) * (2.0 * bits[i].reshape(m, n) - 1.0)
+        size += u[i].double().abs() @ vt[i].double().abs()
+    return want, size, (2 * bits.reshape(blocks, m, n).to(torch.int8) - 1)
+
+
+@pytest.mark.parametrize("blocks,m,n,k", CASES)
+@pytest.mark.parametrize("shifted", [False, True])
+def test_rebuild_of_byte_columns(blocks, m, n, k, shifted):
+    from bitstack_amd.utils import inference_utils as IU
+
+    g = torch.Generator(device="cuda").manual_seed(blocks + m + n)
+    packed = torch.randint(0, 256, (blocks, m * n // 8), dtype=torch.uint8, device="cuda", generator=g)
+    u = torch.randn(blocks * m * k + 1, device="cuda", generator=g).half()[int(shifted):][: blocks * m * k].view(blocks, m, k)   # (shifted: rows at 2-byte alignment)
+    vt = torch.randn(blocks, k, n, device="cuda", generator=g).half()
+    print(blocks, m, n, k, shifted, flush=True)
+    want, size, sign = exact(packed, u, vt)
+    w = IU.unpack_and_reconstruct_w_hip(packed, u, vt)
+    # float32 products and sums of k * blocks terms (each rounding at most 2^-24 of the sum of magnitudes), then one rounding to half
+    bound = want.abs() * 2.0 ** -11 + size * (k + blocks + 1) * 2.0 ** -24 + 2.0 ** -25
+    assert ((w.double() - want).abs() <= bound).all()
+    assert torch.equal(w, IU.reconstruct_w_hip(sign, u, vt))

@@ -240,66 +240,76 @@ __global__ __launch_bounds__(64 * WT * WF) void linear_f16_kernel(
     }
 }
 
-// Few tokens (<= 32): the job is to stream w once at memory speed, so nothing is
-// shared through LDS.  A workgroup owns 32 features; its KS waves split the
-// contracted range, each wave reading its fragments straight from global memory
-// (16 bytes per lane and fragment, UNROLL k-steps in flight), AT token blocks of
-// 32 against one feature block.  The KS partial tiles are added through LDS in a
-// fixed order.
-template <int AT, int KS, int UNROLL>
-__global__ __launch_bounds__(64 * KS) void linear_skinny_kernel(
+// Few tokens (<= 32): the job is to stream w once at memory speed, so nothing is shared through LDS.  A workgroup owns 16 F features; its 8 waves split the contracted
+// range, each reading its fragments of v_mfma_f32_16x16x32_f16 straight from global memory, whole 128-byte lines (the two halves of one back to back), AHEAD
+// lines of 16 F rows in flight, TB blocks of 16 tokens against them.  The waves' sums are added through LDS in a fixed order.  N % 8 == 0: pieces beyond the last
+// column, or the wave's last line, are asked for beyond the end of the buffer, which reads as zeros.
+// What bounds it: memory (32000 x 8192, one token: 5.6 TB/s), with 16 tokens and more the reads of x, as many bytes per workgroup as T / (16 F) of w.  us, the kernel
+// before (v_mfma_f32_32x32x16_f16, half a line's quarter per request, N % 16 == 0 only, otherwise the tiled kernel) / this: 32000 x 4096, one token 55.7 / 48.7, 8 tokens
+// 63.9 / 49.3, 32 tokens 89.1 / 56.8; 32000 x 8192, 8 tokens 123.9 / 92.5; 4096 x 4104, 8 tokens 26.0 / 8.1; 512 x 6008 27.5 / 8.1.  Fewer parts of the contracted range and more features side by
+// side (4, 2, 1 parts): slower from 4096 columns on, level below.
+constexpr int SKINNY_WAVES = 8, SKINNY_LINE = 64;               // columns of a line
+template <int TB, int F, int AHEAD>
+__global__ __launch_bounds__(64 * SKINNY_WAVES, 4) void linear_skinny_kernel(
     const half_t *__restrict__ x, const half_t *__restrict__ w, const half_t *__restrict__ bias,
     half_t *__restrict__ y, int T, int M, int N) {
-    __shared__ float red[KS][AT][16][64];
-    const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
-    const int l32 = lane & 31, kh = lane >> 5;
-    const int m0 = blockIdx.x * 32;
-    // this wave's share of the k-steps (16 columns each)
-    const int steps = N / 16, per = (steps + KS - 1) / KS;
-    const int s_begin = ks * per, s_end = min(s_begin + per, steps);
+    __shared__ float4_t red[SKINNY_WAVES][TB * F][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lm = lane & 15, g = lane >> 4;
+    const int m0 = blockIdx.x * (16 * F);
+    const int lines = (N + SKINNY_LINE - 1) / SKINNY_LINE, per = (lines + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const int begin = wave * per, end = min(begin + per, lines), limit = min(end * SKINNY_LINE, N);     // (no branch around a product: its loads would move into it)
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)(w + (int64_t)m0 * N), 0, (int)((uint32_t)min(16 * F, M - m0) * (uint32_t)N * 2u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, (int)((uint32_t)T * (uint32_t)N * 2u), 0x00020000);
+    uint32_t off_w[F], off_x[TB];
+#pragma unroll
+    for (int f = 0; f < F; f++) off_w[f] = (uint32_t)(16 * f + lm) * (uint32_t)N * 2u + 16u * g;
+#pragma unroll
+    for (int b = 0; b < TB; b++) off_x[b] = (uint32_t)min(16 * b + lm, T - 1) * (uint32_t)N * 2u + 16u * g;
 
-    const half_t *wp = w + (int64_t)min(m0 + l32, M - 1) * N + 8 * kh;
-    const half_t *xp[AT];
+    float4_t acc[TB][F];
 #pragma unroll
-    for (int a = 0; a < AT; a++) xp[a] = x + (int64_t)min(32 * a + l32, T - 1) * N + 8 * kh;
-
-    float16_t acc[AT];
+    for (int b = 0; b < TB; b++)
 #pragma unroll
-    for (int a = 0; a < AT; a++)
+        for (int f = 0; f < F; f++) acc[b][f] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    for (int at = begin; at < end; at += AHEAD) {
+        half8_t wf[AHEAD][2][F], xf[AHEAD][2][TB];
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[a][v] = 0.f;
-
-    for (int st = s_begin; st < s_end; st += UNROLL) {
-        half8_t bf[UNROLL], af[UNROLL][AT];
+        for (int q = 0; q < AHEAD; q++) {
+            const int col = (at + q) * SKINNY_LINE;
 #pragma unroll
-        for (int q = 0; q < UNROLL; q++) {
-            const int k = min(st + q, s_end - 1) * 16;     // clamped: the surplus products are skipped below
-            bf[q] = *reinterpret_cast<const half8_t *>(wp + k);
+            for (int f = 0; f < F; f++)
 #pragma unroll
-            for (int a = 0; a < AT; a++) af[q][a] = *reinterpret_cast<const half8_t *>(xp[a] + k);
+                for (int h = 0; h < 2; h++)
+                    wf[q][h][f] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(col + 32 * h + 8 * g < limit ? off_w[f] + 64u * h : 0x80000000u), 2 * col, 0));
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    xf[q][h][b] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(col + 32 * h + 8 * g < limit ? off_x[b] + 64u * h : 0x80000000u), 2 * col, 0));
         }
+        __builtin_amdgcn_sched_barrier(0);                               // (all of them on their way before the first is waited for)
 #pragma unroll
-        for (int q = 0; q < UNROLL; q++) {
-            if (st + q < s_end) {
+        for (int q = 0; q < AHEAD; q++) {
 #pragma unroll
-                for (int a = 0; a < AT; a++)
-                    acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[q][a], bf[q], acc[a], 0, 0, 0);
-            }
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int b = 0; b < TB; b++)
+#pragma unroll
+                    for (int f = 0; f < F; f++) acc[b][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[q][h][b], wf[q][h][f], acc[b][f], 0, 0, 0);
         }
     }
-
 #pragma unroll
-    for (int a = 0; a < AT; a++)
+    for (int b = 0; b < TB; b++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) red[ks][a][v][lane] = acc[a][v];
+        for (int f = 0; f < F; f++) red[wave][b * F + f][lane] = acc[b][f];
     __syncthreads();
-    // D[token, feature]: lane holds feature l32, tokens 8 * (v / 4) + 4 * kh + v % 4
-    for (int item = ks; item < AT * 16; item += KS) {
-        const int a = item / 16, v = item % 16;
+    // D[token, feature]: lane 16 g + lm holds tokens 4 g .. 4 g + 3 of feature lm
+    for (int o = tid; o < TB * F * 256; o += 64 * SKINNY_WAVES) {
+        const int f = (o >> 4) % F, t = o / (16 * F), m = m0 + o % (16 * F);
         float sum = 0.f;
 #pragma unroll
-        for (int k = 0; k < KS; k++) sum += red[k][a][v][lane];
-        const int m = m0 + l32, t = 32 * a + 8 * (v >> 2) + 4 * kh + (v & 3);
+        for (int k = 0; k < SKINNY_WAVES; k++) sum += red[k][(t >> 4) * F + f][16 * ((t >> 2) & 3) + (o & 15)][t & 3];
         if (m < M && t < T) y[(int64_t)t * M + m] = (half_t)(sum + (bias ? (float)bias[m] : 0.f));
     }
 }
@@ -355,7 +365,9 @@ int launch_tiled(const half_t *x, const half_t *w, const half_t *bias, half_t *y
 struct LinearTile { int bt, bf, gk; };
 static LinearTile linear_tile(int T, int M, int N, bool aligned) {
     if (!(N % 8 == 0 && aligned) || N >= (1 << 23)) return {0, 0, 0};     // (a tile's rows stay within 32-bit byte offsets)
-    if (T <= 32 && N % 16 == 0) return {32, 32, 0};                       // linear_skinny_kernel
+    // linear_skinny_kernel: the more features a workgroup has, the less x it reads, as long as there are some 160 workgroups or more (8 tokens, us, 16 / 32 / 64
+    // features: 8192 x 8192 29.4 / 26.5 / 38.8, 14336 x 4096 28.8 / 25.9 / 23.8, 32000 x 8192 104.6 / 91.1 / 90.0)
+    if (T <= 32) return {32, M >= 12288 ? 64 : M >= 5120 ? 32 : 16, 0};
     if (T <= 128) return M >= 8192 ? LinearTile{128, 64, 64} : LinearTile{128, 32, 128};
     // The largest tile whose grid still covers most of the 256 CUs: 256 x 256 and
     // 128 x 256 move the fewest bytes per flop; 128 x 128 and 64 x 64
@@ -444,7 +456,9 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
         if (blocks > 256 * 64) blocks = 256 * 64;
         linear_generic_kernel<<<(int)blocks, 256, 0, s>>>(x, w, bias, y, T, M, N);
     } else if (tile.gk == 0) {
-        linear_skinny_kernel<1, 8, 8><<<(int)bs_cdiv(M, 32), 512, 0, s>>>(x, w, bias, y, T, M, N);
+        const auto skinny = [&](auto kernel) { kernel<<<(int)bs_cdiv(M, tile.bf), 64 * SKINNY_WAVES, 0, s>>>(x, w, bias, y, T, M, N); };
+        if (T <= 16) tile.bf == 64 ? skinny(linear_skinny_kernel<1, 4, 2>) : tile.bf == 32 ? skinny(linear_skinny_kernel<1, 2, 2>) : skinny(linear_skinny_kernel<1, 1, 6>);
+        else tile.bf == 64 ? skinny(linear_skinny_kernel<2, 4, 1>) : tile.bf == 32 ? skinny(linear_skinny_kernel<2, 2, 2>) : skinny(linear_skinny_kernel<2, 1, 4>);
     } else if (tile.bf >= 128 && N % 64 == 0) {
         return bs_launch_linear_pipe(x, w, bias, y, T, M, N, tile.bt, tile.bf, 1, nullptr, s);
     } else if (tile.bt == 128 && tile.bf == 64) {

@@ -278,8 +278,8 @@ int bs_linear_f16(const void *x, const void *w, const void *bias, void *y,
  * features), the k-step and whether the last k-step is partial (N not a multiple
  * of the step) of the dense kernel bs_linear_f16 runs for these dimensions with
  * 16-byte aligned buffers.  (Behind a rebuilt weight bs_forward has scratch: it
- * picks among more tiles there, and may cut the contracted range into parts.)  32 x 32
- * with *k_step == 0 is the no-LDS kernel for up to 32 tokens, 0 x 0 the
+ * picks among more tiles there, and may cut the contracted range into parts.)  32 x 16,
+ * 32 or 64 with *k_step == 0 is the no-LDS kernel for up to 32 tokens, 0 x 0 the
  * one-wave-per-output kernel (N % 8 != 0).  No counterpart in the reference
  * (F.linear picks a vendor kernel).
  */

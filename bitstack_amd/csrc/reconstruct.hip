@@ -2,6 +2,9 @@
 //   w[m, n] = fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
 // fp32 everywhere until the single final rounding.
 //
+// Packed signs at rank 16 are rebuilt by the kernel in tile.hip where it takes the shape (bs_launch_reconstruct_packed; us, this one / that: 28672 x 8192, 3 blocks
+// 176 / 113, 14336 x 4096, 8 69 / 50, 4096 x 4096, 8 22.4 / 20.2, 5000 x 1408, 6 15.4 / 11.9).  Here: the rest, and int8 signs.
+//
 // Tiled kernel.  A workgroup owns a strip of 128 columns and a range of rows.
 // It first stages the strip's slice of vt for ALL blocks in LDS, transposed to
 // [block][column][rank] (vt is stored rank-major, the MFMA wants the rank
@@ -28,25 +31,30 @@ constexpr int VSTRIDE = 16;    // halves per column in LDS: the 16 ranks, contig
 constexpr int VGROUP_PAD = 4;  // extra halves after every 8 columns (keeps the fragment reads off each other's banks)
 constexpr int VBLOCK = RT_COLS * VSTRIDE + (RT_COLS / 8) * VGROUP_PAD;   // halves per block in LDS
 constexpr int RT_MAXB = 36;    // most blocks whose vt strip fits in LDS (36 x 4.1 KB)
-constexpr int SIGN_LUT_HALVES = 64;   // 16 nibbles x 4 signs
+constexpr int MASK_TABLE = 256;       // bytes: 16 nibbles x 4 sign masks
+constexpr int SIGN_LUT_HALVES = 64;   // 16 nibbles x 4 signs (reconstruct_byte_kernel)
 constexpr int RA_MAXB = 39;    // ... of reconstruct_byte_kernel (39 x 4 KB beside its sign table)
 
 // K16: the rank is 16 (every u fragment is one 8-byte load).  Smaller ranks pick their halves one by one behind
 // branches, and the compiler then waits for every load in flight where the branches meet: that instantiation runs
 // one pair ahead at best.
-template <bool PACKED, bool K16>
+// FLIP (rank 16): the sums of the kernel in tile.hip, bit for bit: the sum over the blocks is kept divided by the block's sign, it changes sign where two
+// blocks differ (a nibble's four masks come from the table instead of its four signs) and the matrix instruction adds the next product to it.  It takes the int8
+// signs, and what that kernel cannot read, of the shapes that it takes.  us, product and FMA / this: int8 signs, 14336 x 4096, 8 blocks 163 / 154, 4096 x 4096, 8
+// 45 / 42; packed signs level where rows are long (14336 x 4096, 8 blocks 69.4 / 69.8) and behind where they are not (20000 x 896, 2 blocks 13.0 / 14.1).
+template <bool PACKED, bool K16, bool FLIP>
 __global__ __launch_bounds__(256, 4) void reconstruct_tile_kernel(
     const uint8_t *__restrict__ packed, const int8_t *__restrict__ sign,
     const half_t *__restrict__ u, const half_t *__restrict__ vt, half_t *__restrict__ w,
     int I, int M, int N, int K, int rows_per_wg) {
-    // First the 16 sign nibbles as four halves each (+1.0 for a set bit, first column in the top bit; at offset 0, so
-    // that a nibble times 8 is the address), then [I][VBLOCK]: column c of a block at c * 16 + (c / 8) * 4.
-    extern __shared__ __attribute__((aligned(128))) half_t lds_all[];
-    half_t *const lut = lds_all;
-    half_t *const vl = lds_all + SIGN_LUT_HALVES;
-    // the table's LDS address as a number: the table is 128-byte aligned, so a nibble's offset is OR-ed into it
+    // First, at LDS address 0 (the kernel has no other LDS), a table of the 16 nibbles: four halves each of +-1.0 (+1.0 for a set bit, first
+    // column in the top bit) or, FLIP, four masks (the sign bit of an fp32 for a set bit).  Then [I][VBLOCK]: column c of a block at
+    // c * 16 + (c / 8) * 4.
+    extern __shared__ __attribute__((aligned(256))) half_t lds_all[];
+    constexpr int TABLE = FLIP ? MASK_TABLE : SIGN_LUT_HALVES * 2;        // bytes
+    half_t *const vl = lds_all + TABLE / 2;
     typedef const __attribute__((address_space(3))) half4_t *lds_half4_ptr;
-    const uint32_t lut_base = (uint32_t)reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) half_t *)lut);
+    typedef const __attribute__((address_space(3))) uint4_t *lds_uint4_ptr;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in every lane: loop counts that depend on it stay scalar
@@ -75,9 +83,9 @@ __global__ __launch_bounds__(256, 4) void reconstruct_tile_kernel(
     // Patches come in pairs: of a 32-column group, patch 2q takes columns 8g'..8g'+3 and patch
     // 2q+1 columns 8g'+4..8g'+7 (g' = 0..3), so that a lane (row lm, group g) ends up with EIGHT
     // consecutive columns of its row - one byte of the packed signs, one 16-byte store.
-    // The lane's byte of a sign word is byte g; its two nibbles, times 8, address the table:
-    // (word >> sh_hi) & 0x78 for the first four columns, (word rotated right by sh_lo) & 0x78 for the others.
-    const int sh_hi = 8 * g + 1, sh_lo = (8 * g - 3) & 31;
+    // The lane's byte of a sign word is byte g; its two nibbles address the table, times 8:
+    // (word >> sh_hi) & 0x78 for the first four columns, (word rotated right by sh_lo) & 0x78 for the others; or times 16.
+    const int sh_hi = 8 * g + 1, sh_lo = (8 * g - 3) & 31, byte_at = 8 * g;
     // this lane's A-fragment column within a 32-column group (n-index lm of either patch, less 4 * (s & 1))
     const int acol = 8 * (lm >> 2) + (lm & 3);
     const int aoff = acol * VSTRIDE + (lm >> 2) * VGROUP_PAD + 4 * g;
@@ -176,56 +184,110 @@ __global__ __launch_bounds__(256, 4) void reconstruct_tile_kernel(
                 }
             }
         }
-        if (PACKED && tid < SIGN_LUT_HALVES) lut[tid] = ((tid >> 2) >> (3 - (tid & 3))) & 1 ? (half_t)1.f : (half_t)-1.f;
+        if (PACKED && tid < 64) {
+            const bool set = ((tid >> 2) >> (3 - (tid & 3))) & 1;
+            if (FLIP) reinterpret_cast<uint32_t *>(lds_all)[tid] = set ? 0x80000000u : 0u;
+            else lds_all[tid] = set ? (half_t)1.f : (half_t)-1.f;
+        }
         __syncthreads();
 
         // 16 rows per wave and step; the current pair is (rows m0.., block i)
         // The first block of a row step starts the sums (a product, not a sum with zero): cleared accumulators
         // would meet the running ones where the paths join, and the compiler then copies two dozen registers per block.
         float4_t acc[8];
+        uint4_t before;                             // the sign words of the pair before this one (int8 signs: t_before)
+        uint32_t t_before[8];
         int i = 0, m0 = first_row;
+        // a patch's sums change sign where `flip` has a set bit
+        auto masks = [&](uint32_t flips, int half) { return *(lds_uint4_ptr)(uintptr_t)((half ? flips << 4 : flips) & 0xF0u); };
+        auto change = [&](float4_t &sum, const uint4_t &m) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float v = sum[j];
+                const uint32_t mj = m[j];
+                sum[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) ^ mj);
+            }
+        };
+        // (int8 signs: negative ones have bit 7 set)
+        auto masks_of = [&](uint32_t t) { return (uint4_t){(t << 24) & 0x80000000u, (t << 16) & 0x80000000u, (t << 8) & 0x80000000u, t & 0x80000000u}; };
         auto consume = [&](const half4_t &b_cur, const uint4_t &swc, auto first_tag) {
             constexpr bool FIRST = decltype(first_tag)::value;
             const int row = min(m0 + lm, M - 1);
             const half_t *vb = vl + i * VBLOCK + aoff;
-            // all eight fragments first, and every product one patch ahead of the sign FMAs
-            // that use it: neither the LDS nor the MFMA latency sits in front of them
+            // all eight fragments first: the LDS latency does not sit in front of the products
             half4_t a[8];
 #pragma unroll
             for (int s = 0; s < 8; s++)
                 a[s] = *reinterpret_cast<const half4_t *>(vb + (32 * (s >> 1) + 4 * (s & 1)) * VSTRIDE + 4 * (s >> 1) * VGROUP_PAD);
-            // the signs of a patch as four halves of +-1.0 from the table (16 entries of 8 bytes: one entry per
-            // pair of banks, equal nibbles read the same address), multiplied in by a mixed-precision FMA
-            half4_t sv[8];
-            if (PACKED) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const uint32_t hi = ((swc[q] >> sh_hi) & 0x78u) | lut_base;
-                    const uint32_t lo = (__builtin_amdgcn_alignbit(swc[q], swc[q], sh_lo) & 0x78u) | lut_base;
-                    sv[2 * q] = *reinterpret_cast<lds_half4_ptr>(hi);
-                    sv[2 * q + 1] = *reinterpret_cast<lds_half4_ptr>(lo);
-                }
-            }
-            float4_t p_next = __builtin_amdgcn_mfma_f32_16x16x16f16(a[0], b_cur, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const float4_t p = p_next;
-                if (s + 1 < 8)
-                    p_next = __builtin_amdgcn_mfma_f32_16x16x16f16(a[s + 1], b_cur, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            uint4_t m[8];
+            if constexpr (!FLIP) {
+                // the signs of a patch as four halves of +-1.0 from the table (16 entries of 8 bytes: one entry per
+                // pair of banks, equal nibbles read the same address), multiplied in by a mixed-precision FMA
+                half4_t sv[8];
                 if (PACKED) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) acc[s][j] = __builtin_fmaf(p[j], (float)sv[s][j], FIRST ? 0.f : acc[s][j]);   // (a plain product would not become a mixed-precision instruction)
-                } else {
-                    uint32_t t = *reinterpret_cast<const uint32_t *>(
-                        sign + ((int64_t)(i0 + i) * M + row) * N + n0 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        uint32_t sf = ((t << (24 - 8 * j)) & 0x80000000u) | 0x3F800000u;
-                        acc[s][j] = FIRST ? p[j] * __builtin_bit_cast(float, sf) : __builtin_fmaf(p[j], __builtin_bit_cast(float, sf), acc[s][j]);
+                    for (int q = 0; q < 4; q++) {
+                        const uint32_t hi = ((swc[q] >> sh_hi) & 0x78u);
+                        const uint32_t lo = (__builtin_amdgcn_alignbit(swc[q], swc[q], sh_lo) & 0x78u);
+                        sv[2 * q] = *reinterpret_cast<lds_half4_ptr>(hi);
+                        sv[2 * q + 1] = *reinterpret_cast<lds_half4_ptr>(lo);
                     }
+                }
+                float4_t p_next = __builtin_amdgcn_mfma_f32_16x16x16f16(a[0], b_cur, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    const float4_t p = p_next;
+                    if (s + 1 < 8)
+                        p_next = __builtin_amdgcn_mfma_f32_16x16x16f16(a[s + 1], b_cur, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    if (PACKED) {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) acc[s][j] = __builtin_fmaf(p[j], (float)sv[s][j], FIRST ? 0.f : acc[s][j]);   // (a plain product would not become a mixed-precision instruction)
+                    } else {
+                        uint32_t t = *reinterpret_cast<const uint32_t *>(
+                            sign + ((int64_t)(i0 + i) * M + row) * N + n0 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            uint32_t sf = ((t << (24 - 8 * j)) & 0x80000000u) | 0x3F800000u;
+                            acc[s][j] = FIRST ? p[j] * __builtin_bit_cast(float, sf) : __builtin_fmaf(p[j], __builtin_bit_cast(float, sf), acc[s][j]);
+                        }
+                    }
+                }
+            } else {
+                uint32_t t[8];
+                if (!PACKED) {
+#pragma unroll
+                    for (int s = 0; s < 8; s++)
+                        t[s] = *reinterpret_cast<const uint32_t *>(sign + ((int64_t)(i0 + i) * M + row) * N + n0 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
+                }
+                if (!FIRST) {
+#pragma unroll
+                    for (int s = 0; s < 8; s++) m[s] = PACKED ? masks((before[s >> 1] ^ swc[s >> 1]) >> byte_at, s & 1) : masks_of(t_before[s] ^ t[s]);
+                }
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    if (FIRST) {
+                        acc[s] = __builtin_amdgcn_mfma_f32_16x16x16f16(a[s], b_cur, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    } else {
+                        change(acc[s], m[s]);
+                        acc[s] = __builtin_amdgcn_mfma_f32_16x16x16f16(a[s], b_cur, acc[s], 0, 0, 0);
+                    }
+                }
+                if (PACKED) before = swc;
+                else {
+#pragma unroll
+                    for (int s = 0; s < 8; s++) t_before[s] = t[s];
                 }
             }
             if (++i == ib) {
+                if constexpr (FLIP) {
+#pragma unroll
+                    for (int s = 0; s < 8; s++) m[s] = PACKED ? masks(~before[s >> 1] >> byte_at, s & 1) : masks_of(t_before[s]);
+#pragma unroll
+                    for (int s = 0; s < 8; s++) {
+                        change(acc[s], m[s]);
+                        asm("" : "+v"(acc[s]));     // (else the optimiser pairs values of different patches, two moves for each)
+                    }
+                }
                 if (m0 + lm < M) {
                     half_t *wp = w + (int64_t)(m0 + lm) * N + n0 + 8 * g;
 #pragma unroll
@@ -425,8 +487,11 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
         // One wave of workgroups: as many row groups as the resident slots allow (LDS decides
         // how many workgroups a CU holds), so that no second, partial wave trails behind.
         // Every workgroup re-stages its vt strip, so rows per workgroup stay a multiple of 64.
+        // (The weight has the same bits whatever it is made from: where the kernel in tile.hip takes the shape, its sums.)
+        int columns;
+        const bool flip = bs_tile_columns(&I, &M, 1, N, K, 0, &columns);
         const int strips = N / RT_COLS, strips8 = (int)bs_cdiv(strips, 8) * 8;
-        const size_t lds_need = (size_t)I * VBLOCK * sizeof(half_t) + SIGN_LUT_HALVES * sizeof(half_t);   // vt images + sign table
+        const size_t lds_need = (size_t)I * VBLOCK * sizeof(half_t) + (flip ? MASK_TABLE : SIGN_LUT_HALVES * sizeof(half_t));   // vt images + table
         int per_cu = (int)((160 * 1024) / lds_need);
         if (per_cu > 8) per_cu = 8;
         if (per_cu < 1) per_cu = 1;
@@ -435,15 +500,12 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
         int rows_per_wg = (int)bs_cdiv(bs_cdiv(M, row_groups), 64) * 64;
         row_groups = (int)bs_cdiv(M, rows_per_wg);
         const size_t lds = lds_need;
-        static bs_lds_grant granted[2][BS_MAX_DEVICES];
-        const void *kernel = K == 16 ? (const void *)reconstruct_tile_kernel<PACKED, true> : (const void *)reconstruct_tile_kernel<PACKED, false>;
-        const int st = bs_allow_lds(kernel, lds, granted[K == 16]);
+        static bs_lds_grant granted[3][BS_MAX_DEVICES];
+        const auto kernel = flip ? reconstruct_tile_kernel<PACKED, true, true> : K == 16 ? reconstruct_tile_kernel<PACKED, true, false> : reconstruct_tile_kernel<PACKED, false, false>;
+        const int st = bs_allow_lds((const void *)kernel, lds, granted[flip ? 2 : K == 16]);
         if (st != BS_OK) return st;
         dim3 grid((unsigned)bs_cdiv(strips, 8) * 8, row_groups);
-        if (K == 16)
-            reconstruct_tile_kernel<PACKED, true><<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
-        else
-            reconstruct_tile_kernel<PACKED, false><<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
+        kernel<<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
     } else if (N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && bs_aligned(u, 8) && (PACKED || bs_aligned(sign, 8))) {
         const int strips = (int)bs_cdiv(N, RA_COLS), steps = (int)bs_cdiv(M, RA_ROWS);
         const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), steps / RA_STREAMS));    // four workgroups per CU, a step per wave or more
@@ -478,7 +540,6 @@ int check_dims(int I, int M, int N, int K) {
 
 int bs_launch_reconstruct_packed(const uint8_t *packed, const half_t *u, const half_t *vt,
                                  half_t *w, int I, int M, int N, int K, hipStream_t s) {
-    // (the weight inside a forward; bs_reconstruct_w keeps to the kernel that the int8 signs take, whose weights are the same bit for bit)
     const int st = bs_launch_tile_rebuild(1, &packed, &u, &vt, &I, &M, &w, N, K, s);
     if (st != BS_ERR_SHAPE) return st;
     return launch_reconstruct<true>(packed, nullptr, u, vt, w, I, M, N, K, s);
@@ -490,8 +551,7 @@ extern "C" int bs_reconstruct_w(const uint8_t *packed, const void *u, const void
     if (st != BS_OK) return st;
     if (!w || (I > 0 && (!packed || !u || !vt))) return BS_ERR_NULL;
     if (!bs_aligned(u, 2) || !bs_aligned(vt, 2) || !bs_aligned(w, 2)) return BS_ERR_ALIGN;
-    return launch_reconstruct<true>(packed, nullptr, (const half_t *)u, (const half_t *)vt,
-                                    (half_t *)w, I, M, N, K, (hipStream_t)stream);
+    return bs_launch_reconstruct_packed(packed, (const half_t *)u, (const half_t *)vt, (half_t *)w, I, M, N, K, (hipStream_t)stream);
 }
 
 extern "C" int bs_reconstruct_w_from_sign(const int8_t *sign, const void *u, const void *vt, void *w,

@@ -427,10 +427,12 @@ extern "C" int bs_attention_decode_f16(const void *qkv, void *kcache, void *vcac
     return bs_attention_decode_ws_f16(qkv, kcache, vcache, cos, sin, pos, out, B, heads, kv_heads, head_dim, max_len, nullptr, 0, stream);
 }
 
-extern "C" int bs_argmax_f16(const void *x, int64_t *out, int B, int V, void *stream) {
+extern "C" int bs_argmax_f16(const void *x, int64_t *out, int B, int V, void *stream) { return bs_argmax_advance_f16(x, out, nullptr, B, V, stream); }
+
+extern "C" int bs_argmax_advance_f16(const void *x, int64_t *out, int64_t *pos, int B, int V, void *stream) {
     if (B < 0 || V <= 0) return BS_ERR_SHAPE;
     if (B == 0) return BS_OK;
     if (!x || !out) return BS_ERR_NULL;
-    if (!bs_aligned(x, 16) || !bs_aligned(out, 8) || (B > 1 && V % 8 != 0)) return BS_ERR_ALIGN;
-    return bs_launch_argmax((const half_t *)x, out, B, V, (hipStream_t)stream);
+    if (!bs_aligned(x, 16) || !bs_aligned(out, 8) || !bs_aligned(pos, 8) || (B > 1 && V % 8 != 0)) return BS_ERR_ALIGN;
+    return bs_launch_argmax((const half_t *)x, out, pos, B, V, (hipStream_t)stream);
 }

@@ -119,7 +119,7 @@ int bs_launch_panel(const uint8_t *packed, const half_t *u, const half_t *vt, in
 // which kernel runs a forward of 49 tokens or more (bs_set_prefill_kernel, per thread): values of BS_PREFILL_*
 int bs_prefill_mode();
 // decode-step kernels around the linears (decode_step.hip)
-int bs_launch_argmax(const half_t *x, int64_t *out, int B, int V, hipStream_t s);
+int bs_launch_argmax(const half_t *x, int64_t *out, int64_t *pos, int B, int V, hipStream_t s);
 int bs_launch_rmsnorm(const half_t *x, const half_t *weight, half_t *y, int T, int H, float eps, hipStream_t s);
 int bs_launch_add_rmsnorm(const half_t *x, const half_t *add, half_t *sum, const half_t *weight, half_t *y, int T, int H, float eps,
                           hipStream_t s);

@@ -510,24 +510,24 @@ PyObject *host_run_steps(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// argmax(x [B, V], out int64 [B]) -> True, or None
+// argmax(x [B, V], out int64 [B] [, pos int64, one element: += 1]) -> True, or None
 PyObject *host_argmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != 2) return PyErr_Format(PyExc_TypeError, "argmax takes 2 arguments");
+    if (n != 2 && n != 3) return PyErr_Format(PyExc_TypeError, "argmax takes 2 or 3 arguments");
     HANDLE_TH_ERRORS
-        const at::Tensor *x = tensor_arg(a[0]), *out = tensor_arg(a[1]);
-        if (!x || !out || !x->is_cuda() || x->dim() != 2) Py_RETURN_NONE;
+        const at::Tensor *x = tensor_arg(a[0]), *out = tensor_arg(a[1]), *pos = n == 3 ? tensor_arg(a[2]) : nullptr;
+        if (!x || !out || (n == 3 && !pos) || !x->is_cuda() || x->dim() != 2) Py_RETURN_NONE;
         const c10::Device dev = x->device();
         if (!plain(*x, at::kHalf, dev) || !plain(*out, at::kLong, dev) || out->numel() != x->size(0) || x->numel() == 0 ||
-            x->size(0) >= INT32_MAX || x->size(1) >= INT32_MAX)
+            x->size(0) >= INT32_MAX || x->size(1) >= INT32_MAX || (pos && (!plain(*pos, at::kLong, dev) || pos->numel() != 1)))
             Py_RETURN_NONE;
         const void *xp = x->const_data_ptr();
-        int64_t *op = (int64_t *)out->mutable_data_ptr();
+        int64_t *op = (int64_t *)out->mutable_data_ptr(), *pp = pos ? (int64_t *)pos->mutable_data_ptr() : nullptr;
         const int B = (int)x->size(0), V = (int)x->size(1);
         const int st = while_others_run([&] {
             DeviceScope scope(dev);
-            return bs_argmax_f16(xp, op, B, V, c10::hip::getCurrentHIPStream(dev.index()).stream());
+            return bs_argmax_advance_f16(xp, op, pp, B, V, c10::hip::getCurrentHIPStream(dev.index()).stream());
         });
-        if (st != BS_OK) return raise_status(st, "bs_argmax_f16");
+        if (st != BS_OK) return raise_status(st, "bs_argmax_advance_f16");
         Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }

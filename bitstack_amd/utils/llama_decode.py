@@ -435,8 +435,9 @@ class SyntheticLlamaDecoder:
         if not normed:
             rmsnorm_hip(xa, self.final_norm, self.s.rms_eps, out=hn)
         self.logits = self._head(hn)
-        argmax_hip(self.logits, out=self.token)
-        self.pos.add_(1)
+        if not _lib.host().argmax(self.logits, self.token, self.pos):          # both in one launch
+            argmax_hip(self.logits, out=self.token)
+            self.pos.add_(1)
 
     def _attend(self, q, k, v, kc, vc, n, stored):
         """prefill()'s attention on torch operations, for heads of other sizes or caches of another layout or type: `stored`

@@ -408,6 +408,8 @@ int bs_attention_decode_ws_f16(const void *qkv, void *kcache, void *vcache, cons
  * reference (generation is left to Hugging Face code).
  */
 int bs_argmax_f16(const void *x, int64_t *out, int B, int V, void *stream);
+/* ... and *pos += 1, the position of the next token, in the same launch (pos null: bs_argmax_f16; B == 0: nothing happens). */
+int bs_argmax_advance_f16(const void *x, int64_t *out, int64_t *pos, int B, int V, void *stream);
 
 #ifdef __cplusplus
 }

@@ -241,8 +241,10 @@ int launch_column(const ColumnMat &m, int grid, const half_t *x, int N, int T, h
     BS_LAUNCH_CHECK();
     return BS_OK;
 }
+// Token tiles: as many as there are, from four on.  us with four, six or eight / with these: 14336 x 4096, 5 blocks, 100 tokens (7) 58.9 / 57.9, 28672 x 8192, 3, 80 (5)
+// 113.4 / 109.7, 11520 x 11904, 3, 112 83.0 / 81.1, 6144 x 4096, 1, 66 21.4 / 20.7, 4096 x 4096, 6, 75 25.8 / 25.7.
 // (registers: 8 per token tile and 10 per block)
-constexpr int max_blocks(int token_tiles) { return token_tiles == 4 ? 8 : token_tiles == 6 ? 7 : 6; }
+constexpr int max_blocks(int token_tiles) { return token_tiles == 4 ? 8 : token_tiles <= 6 ? 7 : 6; }
 template <int TT>
 int launch_blocks(int I, const ColumnMat &m, int grid, const half_t *x, int N, int T, hipStream_t s) {
     switch (I) {
@@ -257,7 +259,7 @@ int launch_blocks(int I, const ColumnMat &m, int grid, const half_t *x, int N, i
     }
     return BS_ERR_SHAPE;
 }
-int token_tiles(int T) { return T <= 64 ? 4 : T <= 96 ? 6 : 8; }
+int token_tiles(int T) { return T <= 64 ? 4 : (int)bs_cdiv(T, 16); }
 
 }  // namespace
 
@@ -285,5 +287,11 @@ int bs_launch_column(const uint8_t *packed, const half_t *u, const half_t *vt, i
     const ColumnMat m{packed, u, vt, part, M, p.row_groups, p.spans};
     const int grid = p.row_groups * p.groups;
     const int tt = token_tiles(T);
-    return tt == 4 ? launch_blocks<4>(I, m, grid, x, N, T, s) : tt == 6 ? launch_blocks<6>(I, m, grid, x, N, T, s) : launch_blocks<8>(I, m, grid, x, N, T, s);
+    switch (tt) {
+        case 4: return launch_blocks<4>(I, m, grid, x, N, T, s);
+        case 5: return launch_blocks<5>(I, m, grid, x, N, T, s);
+        case 6: return launch_blocks<6>(I, m, grid, x, N, T, s);
+        case 7: return launch_blocks<7>(I, m, grid, x, N, T, s);
+        default: return launch_blocks<8>(I, m, grid, x, N, T, s);
+    }
 }

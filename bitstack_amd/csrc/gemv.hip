@@ -445,7 +445,7 @@ struct RedGroup {
 // kernel is one memory round trip long.  A workgroup produces 256 / SL consecutive outputs of one
 // token; SL threads per output take every SL-th of the I * kmax slots (SL = 1: no LDS, no barrier).
 // SCALED: the input RMS scale of RedGroup::xin or RedGroup::ssq.
-constexpr int FLAT_BATCH = 8;
+constexpr int FLAT_BATCH = 8, RED_WIDE = 1024;     // (RED_WIDE: outputs per workgroup of gemv_reduce_wide_kernel)
 template <int SL>
 __device__ __forceinline__ float flat_slice_sum(const RedMat &r, int T, int t, int m, int ks) {
     const int total = r.I * r.kmax;
@@ -463,6 +463,29 @@ __device__ __forceinline__ float flat_slice_sum(const RedMat &r, int T, int t, i
         for (int j = 0; j < FLAT_BATCH; j++) acc += (s0 + j * SL < total) ? v[j] : 0.f;
     }
     return acc;
+}
+
+// this wave's share of a workgroup's sum of squares of the input
+__device__ __forceinline__ float input_squares(const RedGroup &grp, int T, int t) {
+    float q = 0.f;
+    if (grp.ssq) {                               // sums of squares per strip group, left by the strip kernel
+        for (int c = threadIdx.x; c < grp.ssq_n; c += 256) q += grp.ssq[c * T + t];
+    } else {
+        const half_t *xr = grp.xin + (int64_t)t * grp.n_in;
+        for (int c = threadIdx.x * 8; c < grp.n_in; c += 256 * 8) {
+            const half8_t v = *reinterpret_cast<const half8_t *>(xr + c);
+#pragma unroll
+            for (int e = 0; e < 8; e++) q += (float)v[e] * (float)v[e];
+        }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
+    return q;
+}
+__device__ __forceinline__ half_t swiglu(float a0, float a1) {
+    const float gate = (float)(half_t)a0, up = (float)(half_t)a1;
+    const half_t act = (half_t)(gate / (1.f + __expf(-gate)));
+    return (half_t)((float)act * up);
 }
 
 template <int SL, bool SCALED>
@@ -495,19 +518,7 @@ __global__ __launch_bounds__(256) void gemv_reduce_flat_kernel(
     }
     float scale = 1.f;
     if (SCALED) {
-        float q = 0.f;
-        if (grp.ssq) {                           // sums of squares per strip group, left by the strip kernel
-            for (int c = threadIdx.x; c < grp.ssq_n; c += 256) q += grp.ssq[c * T + t];
-        } else {
-            const half_t *xr = grp.xin + (int64_t)t * grp.n_in;
-            for (int c = threadIdx.x * 8; c < grp.n_in; c += 256 * 8) {
-                const half8_t v = *reinterpret_cast<const half8_t *>(xr + c);
-#pragma unroll
-                for (int e = 0; e < 8; e++) q += (float)v[e] * (float)v[e];
-            }
-        }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
+        const float q = input_squares(grp, T, t);
         if ((threadIdx.x & 63) == 0) ssq[threadIdx.x >> 6] = q;
     }
     if (SL > 1) {
@@ -530,14 +541,77 @@ __global__ __launch_bounds__(256) void gemv_reduce_flat_kernel(
     const float a0 = s0 * scale + extra0;
     if (two) {
         const float a1 = s1 * scale + extra1;
-        const float gate = (float)(half_t)a0, up = (float)(half_t)a1;
-        const half_t act = (half_t)(gate / (1.f + __expf(-gate)));
-        y[(int64_t)t * ldy + m] = (half_t)((float)act * up);
+        y[(int64_t)t * ldy + m] = swiglu(a0, a1);
     } else {
         half_t v = (half_t)a0;
         if (grp.mode == EPI_RESIDUAL) v = (half_t)(res + (float)v);
         y[(int64_t)t * ldy + r.y_off + m] = v;
     }
+}
+
+// The same sums in the same order (above FLAT_BATCH slots even and odd ones apart), four neighbouring outputs per thread (16-byte loads, 8-byte stores) and a token per
+// blockIdx.y: for many outputs of up to 16 slots, where a thread per output is bound by its own index arithmetic (14336 x 100 outputs of four slots: 7 us, VALU 62 % of
+// the cycles).  Now memory.  S: most slots of a matrix.  us of a call, flat / this: 28672 x 8192, 3 blocks, 80 tokens 109.7 / 104.9, 14336 x 4096, 5, 100 58.4 / 56.2, 8, 24 52.2 / 50.4,
+// 5000 x 4096, 6, 37 26.5 / 26.0, 10240 x 1024, 4, 16 15.2 / 14.4, 2048 x 2048, 3, 64 13.9 / 13.4, 28672 x 4096, 2, 5 (140 workgroups) 28.8 / 28.6.
+template <int S, bool SCALED>
+__global__ __launch_bounds__(256) void gemv_reduce_wide_kernel(const RedGroup grp, const half_t *__restrict__ residual, half_t *__restrict__ y, int T, int ldy) {
+    __shared__ float ssq[4];
+    const bool two = grp.mode == EPI_SWIGLU;
+    int j = 0;
+    if (!two) {
+#pragma unroll
+        for (int q = 1; q < GEMV_MAX_GROUP; q++)
+            if (q < grp.n && (int)blockIdx.x >= grp.m[q].first_block) j = q;
+    }
+    const RedMat &r = grp.m[j];
+    const int t = blockIdx.y, m = ((int)blockIdx.x - r.first_block) * RED_WIDE + 4 * threadIdx.x;
+    const bool live = m < r.M;
+    const int at = live ? m : 0;
+    auto sums = [&](const RedMat &mat) {
+        const int total = mat.I * mat.kmax;
+        const float *base = mat.part + (int64_t)t * mat.M + at;
+        float4_t v[S];
+#pragma unroll
+        for (int k = 0; k < S; k++) v[k] = *reinterpret_cast<const float4_t *>(base + (int64_t)min(k, total - 1) * T * mat.M);
+        float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < S; k++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[S > FLAT_BATCH ? k & 1 : 0][e] += k < total ? v[k][e] : 0.f;
+        if (S > FLAT_BATCH) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[0][e] = acc[0][e] + acc[1][e];
+        }
+        return acc[0];
+    };
+    const float4_t s0 = sums(r), s1 = two ? sums(grp.m[1]) : (float4_t){0.f, 0.f, 0.f, 0.f};
+    const half4_t none = {(half_t)0, (half_t)0, (half_t)0, (half_t)0};
+    half4_t bias0 = none, bias1 = none, res = none;
+    if (r.bias) bias0 = *reinterpret_cast<const half4_t *>(r.bias + at);
+    if (two && grp.m[1].bias) bias1 = *reinterpret_cast<const half4_t *>(grp.m[1].bias + at);
+    half_t *const to = y + (int64_t)t * ldy + (two ? 0 : r.y_off) + at;
+    if (grp.mode == EPI_RESIDUAL) res = *reinterpret_cast<const half4_t *>(residual + (int64_t)t * ldy + r.y_off + at);
+    float scale = 1.f;
+    if (SCALED) {
+        const float q = input_squares(grp, T, t);
+        if ((threadIdx.x & 63) == 0) ssq[threadIdx.x >> 6] = q;
+        __syncthreads();
+        scale = rsqrtf((ssq[0] + ssq[1] + ssq[2] + ssq[3]) / (float)grp.n_in + grp.eps);
+    }
+    half4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float a0 = s0[e] * scale + (float)bias0[e];
+        if (two) {
+            const float a1 = s1[e] * scale + (float)bias1[e];
+            out[e] = swiglu(a0, a1);
+        } else {
+            half_t v = (half_t)a0;
+            if (grp.mode == EPI_RESIDUAL) v = (half_t)((float)res[e] + (float)v);
+            out[e] = v;
+        }
+    }
+    if (live) *reinterpret_cast<half4_t *>(to) = out;
 }
 
 template <int SL>
@@ -546,6 +620,35 @@ void launch_reduce_flat(int blocks, const RedGroup &r, const half_t *residual, h
         gemv_reduce_flat_kernel<SL, true><<<blocks, 256, 0, s>>>(r, residual, y, T, ldy);
     else
         gemv_reduce_flat_kernel<SL, false><<<blocks, 256, 0, s>>>(r, residual, y, T, ldy);
+}
+
+// Whether the four-at-a-time kernel takes the sums, and its launch: `slots` at most 16, sizes and addresses of whole fours, a workgroup for every other CU, and four times as many
+// where an output is made of two sums (2 x 28672 rows, 8 tokens, 224 workgroups, flat / this: 8 slots 5.5 / 5.7 us, 16 slots 6.2 / 7.3).
+constexpr int64_t RED_WIDE_MIN = 128;
+bool launch_reduce_wide(int slots, const RedGroup &r, const half_t *residual, half_t *y, int T, int ldy, hipStream_t s) {
+    RedGroup g = r;
+    int blocks = 0;
+    bool fours = slots <= 2 * FLAT_BATCH && bs_aligned(y, 8) && bs_aligned(residual, 8) && ldy % 4 == 0 && T <= 65535;
+    for (int j = 0; j < r.n; j++) {
+        const RedMat &m = r.m[j];
+        fours = fours && m.M % 4 == 0 && m.y_off % 4 == 0 && bs_aligned(m.bias, 8) && bs_aligned(m.part, 16);
+        g.m[j].first_block = blocks;
+        if (r.mode != EPI_SWIGLU || j == 0) blocks += (int)bs_cdiv(m.M, RED_WIDE);
+    }
+    if (!fours || (int64_t)blocks * T < RED_WIDE_MIN * (r.mode == EPI_SWIGLU ? 4 : 1)) return false;
+    const bool scaled = r.xin || r.ssq;
+    const dim3 grid(blocks, T);
+    switch (slots <= 8 ? slots : slots <= 12 ? 12 : 16) {
+#define RED_CASE(k) \
+    case k: \
+        if (scaled) gemv_reduce_wide_kernel<k, true><<<grid, 256, 0, s>>>(g, residual, y, T, ldy); \
+        else gemv_reduce_wide_kernel<k, false><<<grid, 256, 0, s>>>(g, residual, y, T, ldy); \
+        break;
+        RED_CASE(1) RED_CASE(2) RED_CASE(3) RED_CASE(4) RED_CASE(5) RED_CASE(6) RED_CASE(7) RED_CASE(8) RED_CASE(12) RED_CASE(16)
+#undef RED_CASE
+        default: return false;
+    }
+    return true;
 }
 
 struct Plan {
@@ -957,7 +1060,7 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     if (st != BS_OK) return st;
     if (mode == EPI_SWIGLU) ldy = a.M[0];
     for (int j = a.n; j < GEMV_MAX_GROUP; j++) r.m[j] = r.m[0];
-    switch (sl) {
+    if (!launch_reduce_wide(slots, r, residual, y, T, ldy, s)) switch (sl) {
         case 1: launch_reduce_flat<1>(blocks, r, residual, y, T, ldy, s); break;
         case 2: launch_reduce_flat<2>(blocks, r, residual, y, T, ldy, s); break;
         case 4: launch_reduce_flat<4>(blocks, r, residual, y, T, ldy, s); break;

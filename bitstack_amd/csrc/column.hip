@@ -10,8 +10,8 @@
 // Per block and chunk two v_mfma_f32_32x32x16_f16 and one v_xor_b32 per weight, as in tile.hip; then the rounded weights are the B operand of
 // y += x . w on v_mfma_f32_16x16x32_f16, x read from LDS.  Scratch holds one partial per column group, the summing kernel adds them up.
 //
-// What bounds it: the vector instructions of the sign flips, as in tile.hip, and as much waiting: by the counters 39 % of a SIMD's cycles (the matrix cores
-// 22), the waves 38 % of their time at a barrier or for data.  14336 x 4096, 5 blocks, 100 tokens, cycles per chunk of 64 columns and
+// What bounds it: the vector instructions of the sign flips, as in tile.hip, and as much waiting: by the counters 40 % of a SIMD's cycles (the matrix cores
+// 21), the waves 39 % of their time at a barrier or for data.  14336 x 4096, 5 blocks, 100 tokens, cycles per chunk of 64 columns and
 // wave: 2,400 in ten steps (200 each would be the instructions alone; the two waves of a SIMD compete), 1,000 in the second product (32 matrix
 // instructions and 16 x reads), 280 for the next image, 390 at the barrier; 16 chunks, and 8,000 to 15,000 cycles before the first.
 // us, walked or panel kernel -> this one, summing launch included: 14336 x 4096 x 5 blocks x 100 tokens 74.7 -> 57.6, 28672 x 8192 x 3 x 80

@@ -908,9 +908,11 @@ int launch_T(const Plan &p, const GemvGroup &grp, const half_t *x, int N, int K,
     return BS_ERR_SHAPE;
 }
 
-// per-block byte offsets are kept in 32 bits inside the kernels
-bool block_fits(int I, int M, int N) { return I >= 1 && I <= RED_MAXBLOCKS && M >= 1 && (int64_t)M * N < ((int64_t)1 << 31); }
-bool gemv_shape_ok(int I, int M, int N, int T) { return block_fits(I, M, N) && T >= 1 && T <= 8 && N % CH == 0; }
+// per-block byte offsets, of signs and of vt, are kept in 32 bits inside the kernels
+bool block_fits(int I, int M, int N, int K) {
+    return I >= 1 && I <= RED_MAXBLOCKS && M >= 1 && (int64_t)M * N < ((int64_t)1 << 31) && (int64_t)K * N * 2 < ((int64_t)1 << 32);
+}
+bool gemv_shape_ok(int I, int M, int N, int K, int T) { return block_fits(I, M, N, K) && T >= 1 && T <= 8 && N % CH == 0; }
 
 // Tokens are processed in passes of at most four (LDS holds Z for four tokens).
 int pass_tokens(int T) { return T <= 4 ? T : (T + 1) / 2; }
@@ -925,16 +927,16 @@ bool strip_group_ok(const int *I, const int *M, int n, int N, int K, int T) {
         if (bs_strip_partials(I[j], M[j], N, K, T) == 0) return false;
     return true;
 }
-bool gemv_group_ok(const int *I, const int *M, int n, int N, int T) {
+bool gemv_group_ok(const int *I, const int *M, int n, int N, int K, int T) {
     for (int j = 0; j < n; j++)
-        if (!gemv_shape_ok(I[j], M[j], N, T)) return false;
+        if (!gemv_shape_ok(I[j], M[j], N, K, T)) return false;
     return true;
 }
 // 1: strip kernel, 0: factor-through kernel, -1: neither takes the shapes
 int group_path(const int *I, const int *M, int n, int N, int K, int T) {
     if (n < 1 || n > GEMV_MAX_GROUP) return -1;
     if (T >= STRIP_MIN_T && T <= STRIP_MAX_T && strip_group_ok(I, M, n, N, K, T)) return 1;
-    if (gemv_group_ok(I, M, n, N, T)) return 0;
+    if (gemv_group_ok(I, M, n, N, K, T)) return 0;
     // One to four tokens on column counts that are multiples of 128 but not of 512: the strip kernel rounds the weight to fp16 once
     // and multiplies with fp32 sums, as the rebuild and the dense product do that such shapes took before it, and no less exactly
     // (error against float64 within 0.05 % of theirs: 11 shapes, three decomposed weights, 1, 2 and 4 tokens).  The factor-through kernels
@@ -996,7 +998,7 @@ Plan sparse_plan(const int *I, const int *M, int n, int N, int K, int T) {
     if (even && mx_rows_per_tile(I, M, n, N, K, T) > 0) return p;
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
-        if (!block_fits(I[j], M[j], N)) return p;
+        if (!block_fits(I[j], M[j], N, K)) return p;
         bytes += (int64_t)I[j] * M[j] * (N / 8);
     }
     if ((!even && K == 16 && bytes < SPARSE_MIN_UNEVEN) || (even && T == 1 && bytes < SPARSE_MIN_ONE)) return p;
@@ -1086,7 +1088,7 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
         return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, split, s);
     int ldy = 0;
     for (int j = 0; j < a.n; j++) {
-        if (sparse.grid == 0 && !gemv_shape_ok(a.I[j], a.M[j], N, T)) return BS_ERR_SHAPE;
+        if (sparse.grid == 0 && !gemv_shape_ok(a.I[j], a.M[j], N, K, T)) return BS_ERR_SHAPE;
         ldy += a.M[j];
     }
     if (mode == EPI_SWIGLU) {

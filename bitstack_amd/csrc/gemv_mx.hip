@@ -490,6 +490,7 @@ int launch_mx(int grid, const GemvGroup &grp, const half_t *x, int N, int K, int
 // Shapes the block-scaled kernel runs: whole 512-column halves, one or two tokens.
 bool bs_gemv_mx_takes(int N, int K, int R, int T) {
     if (N % 512 != 0 || K < 1 || K > 16 || T < 1 || T > 2) return false;
+    if ((int64_t)K * N * 2 >= ((int64_t)1 << 31)) return false;      // (a rank's place in a block of vt is a 32-bit byte offset)
     return R == 1 || R == 2 || R == 4;
 }
 

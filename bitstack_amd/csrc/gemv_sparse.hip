@@ -365,8 +365,10 @@ int launch_sparse(int grid, const GemvGroup &grp, const half_t *x, int N, int K,
 
 }  // namespace
 
-// Whole 128-column groups, one to three tokens; rows per workgroup 128 R.
-bool bs_gemv_sparse_takes(int N, int K, int R, int T) { return N >= 128 && N % 128 == 0 && K >= 1 && K <= 16 && T >= 1 && T <= 3 && (R == 1 || R == 2 || R == 4); }
+// Whole 128-column groups, one to three tokens; rows per workgroup 128 R.  (A block of vt, and x, lie within 31-bit byte offsets.)
+bool bs_gemv_sparse_takes(int N, int K, int R, int T) {
+    return N >= 128 && N % 128 == 0 && K >= 1 && K <= 16 && T >= 1 && T <= 3 && (R == 1 || R == 2 || R == 4) && (int64_t)(K > T ? K : T) * N * 2 < ((int64_t)1 << 31);
+}
 
 int bs_launch_gemv_sparse(int R, int T, int grid, const GemvGroup &grp, const half_t *x, int N, int K, int n_units, hipStream_t s) {
     if (!bs_gemv_sparse_takes(N, K, R, T) || n_units != (int)bs_cdiv(N, 512)) return BS_ERR_SHAPE;

@@ -38,6 +38,22 @@ def test_which_calls_the_sparse_kernel_serves():
         L.bs_set_decode_kernel(_lib.DECODE_AUTO)
 
 
+@pytest.mark.parametrize("M,N,K,T,mx,sparse,path", [
+    # a block of vt, or x, reaches 2^31 bytes: not the kernels that address it with 32-bit offsets; 2^32: not gemv_kernel either
+    (1, 1 << 28, 16, 1, False, False, _lib.PATH_REBUILD), (1, (1 << 27) - 512, 16, 1, False, False, _lib.PATH_DECODE_F16), (1, 1 << 27, 16, 1, False, False, _lib.PATH_REBUILD),
+    (1, (1 << 26) - 512, 16, 1, True, True, _lib.PATH_DECODE_F16), (1, 1 << 26, 16, 1, False, False, _lib.PATH_DECODE_F16), (1, (1 << 30) - 512, 1, 1, True, True, _lib.PATH_DECODE_F16),
+    (1, 1 << 29, 1, 2, True, False, _lib.PATH_DECODE_F16), (1, 1 << 29, 1, 3, False, False, _lib.PATH_DECODE_F16), (1, (1 << 30) - 512, 2, 2, False, False, _lib.PATH_DECODE_F16)])
+def test_columns_beyond_32_bit_offsets(M, N, K, T, mx, sparse, path):
+    assert _lib.sparse_kernel([(1, M)], N, K, T) == sparse
+    L = _lib.lib()
+    assert L.bs_forward_path(1, M, N, K, T) == path and L.bs_workspace_bytes(1, M, N, K, T) > 0
+    try:
+        L.bs_set_decode_kernel(_lib.DECODE_MX)
+        assert (L.bs_decode_kernel(1, M, N, K, T) == _lib.DECODE_MX) == mx
+    finally:
+        L.bs_set_decode_kernel(_lib.DECODE_AUTO)
+
+
 @pytest.mark.skipif(not os.path.exists(shutil.which("hipcc") or "/opt/rocm/bin/hipcc"), reason="hipcc not available")
 def test_the_sparse_kernel_keeps_everything_in_registers(tmp_path):
     asm, source = tmp_path / "k.s", os.path.join(os.path.dirname(_lib.LIB_PATH), "gemv_sparse.hip")

@@ -16,7 +16,7 @@
 // Units are (block, row tile of 128 R rows, 512 columns), the column chunk fastest; partition over one workgroup of 8 waves per CU, partial sums and summing launch as gemv.hip has
 // them.  Signs, vt and x are requested one unit ahead; the two register sets of the signs take turns without being copied (a copy at the end of a unit waits for the
 // requests it is there to overlap: 43.0 against 41.0 us on 16 blocks of 4096 x 14336).  u comes by way of LDS while the last unit of a row of units is multiplied.  Columns beyond
-// N have x = 0; rows beyond M and ranks beyond K repeat the last one and are left out at the end.
+// N have x = 0 and vt = 0 (0 times an infinity further left would be NaN); rows beyond M and ranks beyond K repeat the last one and are left out at the end.
 //
 // What bounds it: with four row tiles a unit is 128 matrix instructions per SIMD, 8.9 ns each on their own and 10.3 with three VALU instructions between them, and 256 KB of B out
 // of LDS, a us as well: 2.0 us measured where units follow each other (4.2 TB/s), of which the multiplication takes 1.5 with the signs in L2.  A call with one unit per workgroup
@@ -46,7 +46,7 @@ __device__ __forceinline__ void sp_for(F &&f) {
 constexpr int SP_WAVES = 8, SP_THREADS = 64 * SP_WAVES;
 
 // raw buffer descriptor from a pointer: no stride, no range limit short of 4 GiB (every offset used with it is checked
-// by construction: rows clamped to M, columns to N)
+// by construction: rows clamped to M, columns to N; vt's ends with the block, what lies beyond reads as zeros)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t sp_rsrc(const void *p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, -1, 0x00020000);
 }
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(SP_THREADS, 2) void gemv_sparse_kernel(const GemvGr
 #pragma unroll
         for (int r = 0; r < R; r++) qoff[r] = (uint32_t)min(rt * RW + (wave * R + r) * 16 + lm, M - 1) * row_bytes;
         rq = sp_rsrc(packed + (int64_t)i * M * row_bytes);
-        rv = sp_rsrc(vt + (int64_t)i * K * N);
+        rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(vt + (int64_t)i * K * N), 0, K * N * 2, 0x00020000);
     };
     auto request = [&](uint4_t (&w)[R], int c) {
         const uint32_t at = min((uint32_t)c * 64u + 16u * g, row_bytes - 16u);
@@ -136,8 +136,10 @@ __global__ __launch_bounds__(SP_THREADS, 2) void gemv_sparse_kernel(const GemvGr
     const bool px_mine = tid < 32 * T;
     auto request_z = [&](int c) {
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-            pv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, (int)(rank_at + 2 * min(512 * c + 8 * (8 * wave + 4 * k + g), N - 8)), 0, 0));
+        for (int k = 0; k < 2; k++) {
+            const int col = 512 * c + 8 * (8 * wave + 4 * k + g);
+            pv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, (int)(col < N ? rank_at + 2 * col : 0x80000000u), 0, 0));
+        }
         if (px_mine) {
             const int col = 512 * c + 16 * (tid & 31), at = 2 * ((tid >> 5) * N + min(col, N - 16));
             px[0] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, at, 0, 0));

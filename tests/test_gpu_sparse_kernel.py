@@ -120,6 +120,22 @@ def test_non_finite_inputs(I, M, N, K, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,K,T", [(4, 2053, 2176, 16, 2), (2, 300, 640, 6, 1), (3, 100, 384, 3, 1), (2, 16, 128, 7, 2), (2, 1024, 4096, 16, 1)])
+def test_an_infinite_result_stays_one(I, M, N, K, T):
+    """One infinity in vt, in the first columns and in the last ones (which a unit that is wider than what is left of the row may not repeat): y is
+    infinite with the sign that float64 gives, and no NaN."""
+    assert _lib.sparse_kernel([(I, M)], N, K, T)
+    q, u, vt, x, _, _ = _layer(I, M, N, K, T)
+    u[u == 0], x[x == 0] = 1.0, 1.0
+    for col in (0, N - 9, N - 8, N - 3, N - 1):
+        bad = vt.clone()
+        bad[I - 1, K - 1, col] = float("inf")
+        y = IU.bitstack_forward_hip(q, u, bad, x, None).view(T, M).cpu()
+        want = torch.from_numpy(C.forward_f64(q.cpu().numpy(), u.cpu().numpy(), bad.cpu().numpy(), x.cpu().numpy())).view(T, M)
+        assert bool(want.isinf().all()) and torch.equal(y.double(), want), col
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 2, 3])
 @pytest.mark.parametrize("layers,N", [([(3, 4096), (1, 1024), (2, 1024)], 1024), ([(2, 700), (1, 33), (3, 3000), (1, 64)], 1024), ([(2, 2816), (3, 2816)], 1664)])
 def test_groups_with_the_epilogues(layers, N, T):

@@ -385,11 +385,12 @@ struct TileKernel {
 #pragma unroll
             for (int c = 0; c < STORES; c++) store_to(tile_of(rt0, false), c, (half8_t){0, 0, 0, 0, 0, 0, 0, 0});
         }
+        if constexpr (NP == 4) tl_wait_lds<0>();     // (tile 1, written just now with nothing behind it: the loop's wait would let it pass the first barrier unfinished)
         int stage = 0;
 #pragma clang loop unroll(disable)
         for (int n = 0; n < len; n++) {
             __builtin_amdgcn_s_setprio(0);
-            tl_wait_lds<4>();                        // (its last LDS writes lie a step's four lookups or more back)
+            tl_wait_lds<4>();                        // (a wave's last LDS writes have four lookups or more behind them, or have been waited for)
             tl_barrier();                            // tile n + 1 and the y tiles of n - 2 are in LDS, the stage of n - 1 is free
             const int free_stage = stage == 0 ? STAGES - 1 : stage - 1;
             lds_bytes st = ring + stage * STAGE;

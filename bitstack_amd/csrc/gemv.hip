@@ -1184,9 +1184,11 @@ int64_t bs_gemv_group_workspace_bytes(const int *I, const int *M, int n, int N, 
 // (0 in *waves when the decode kernel does not take them).
 void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave, int *grid, int *kmax) {
     *waves = *row_tiles_per_wave = *grid = *kmax = 0;
-    if (group_path(&I, &M, 1, N, K, T) != 0) return;
-    Plan p = sparse_plan(&I, &M, 1, N, K, T);
-    if (p.grid == 0) p = make_plan(&I, &M, 1, N, K, pass_tokens(T));
+    Plan p = sparse_plan(&I, &M, 1, N, K, T);                    // (also in the strip kernel's place)
+    if (p.grid == 0) {
+        if (group_path(&I, &M, 1, N, K, T) != 0) return;
+        p = make_plan(&I, &M, 1, N, K, pass_tokens(T));
+    }
     *waves = p.waves;
     *row_tiles_per_wave = p.R;
     *grid = p.grid;

@@ -153,9 +153,9 @@ int bs_forward_static(const uint8_t *packed, const void *u, const void *vt, cons
  * Introspection for benchmarks and tests: which decode kernel instantiation
  * (waves per workgroup, 16-row tiles per wave), how many workgroups and how
  * many partial sums per row and block bs_forward would use for these
- * dimensions; *waves == 0 means the decode kernel does not run them (the
+ * dimensions; *waves == 0 means no decode kernel runs them (the
  * strip kernel or the dense path does: more than 4 tokens with N % 128 == 0,
- * more than 8 tokens, N not a multiple of 512).  No counterpart in the reference
+ * more than 8 tokens, N not a multiple of 512 unless bs_sparse_kernel says 1).  No counterpart in the reference
  * (Triton picks its configuration by autotuning,
  * bitstack/utils/inference_utils.py:8-39).  Three and four tokens for which
  * bs_tile_kernel answers BS_TILE_TWO_TERMS run like this only with u off a
@@ -166,8 +166,8 @@ int bs_decode_plan(int I, int M, int N, int K, int T, int *waves, int *row_tiles
 
 /*
  * Which decode kernel bs_forward runs for these dimensions: 0 none (strip kernel
- * or dense path), BS_DECODE_F16 an fp16-MFMA kernel (1..4 tokens per pass; bs_sparse_kernel
- * says which),
+ * or dense path, or gemv_sparse_kernel in the strip kernel's place), BS_DECODE_F16 an
+ * fp16-MFMA kernel (1..4 tokens per pass; bs_sparse_kernel says which),
  * BS_DECODE_MX the block-scaled fp4 x fp6 MFMA kernel (one or two tokens; signs
  * as the fp4 operand, vt o x as three fp6 terms).  For more than four tokens the
  * answer is that of the first pass.  Negative = error status.

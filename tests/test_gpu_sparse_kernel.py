@@ -38,6 +38,16 @@ def test_which_calls_the_sparse_kernel_serves():
         L.bs_set_decode_kernel(_lib.DECODE_AUTO)
 
 
+def test_the_decode_plan_is_the_sparse_kernels_wherever_it_serves():
+    for I, M, N, K, T in CASES + [(4, 4096, 11008, 16, 1)]:
+        waves, R, grid, kmax = _lib.decode_plan(I, M, N, K, T)
+        units = I * -(-M // (128 * R)) * -(-N // 512) if R else 0
+        assert waves == 8 and R in (1, 2, 4) and grid == min(units, 256) and 1 <= kmax <= -(-N // 512), (I, M, N, K, T)
+    # the strip and tile kernels' calls, and the strip kernel's below the sparse one's sizes
+    for I, M, N, K, T in [(4, 4096, 11008, 16, 3), (4, 4096, 11008, 16, 8), (1, 5877, 640, 16, 1), (4, 4096, 4096, 16, 40)]:
+        assert _lib.decode_plan(I, M, N, K, T) == (0, 0, 0, 0), (I, M, N, K, T)
+
+
 @pytest.mark.parametrize("M,N,K,T,mx,sparse,path", [
     # a block of vt, or x, reaches 2^31 bytes: not the kernels that address it with 32-bit offsets; 2^32: not gemv_kernel either
     (1, 1 << 28, 16, 1, False, False, _lib.PATH_REBUILD), (1, (1 << 27) - 512, 16, 1, False, False, _lib.PATH_DECODE_F16), (1, 1 << 27, 16, 1, False, False, _lib.PATH_REBUILD),

@@ -58,15 +58,17 @@ extern "C" int bs_set_dense_kernel(int mode) {
 }
 
 // `library_ok`: the dense product may run on hipBLASLt (and then needs its scratch behind the weight)
+static int64_t rebuild_need(int M, int N, int T, bool library_ok) {
+    // the rebuilt weight, then the library GEMM's own scratch where that is the kernel, or the product's partial sums
+    const bool library = library_ok && dense_wants_library(M, N);
+    return round_up((int64_t)M * N * 2, 256) + round_up(std::max(library ? BS_DENSE_LIBRARY_WORKSPACE : 0, bs_linear_parts_bytes(T, M, N)), 256);
+}
 static int64_t workspace_need(int I, int M, int N, int K, int T, bool library_ok) {
     int st = forward_dims(I, M, N, K, T);
     if (st != BS_OK) return st;
     if (T == 0) return 0;
-    int64_t gemv = bs_gemv_workspace_bytes(I, M, N, K, T);
-    if (gemv > 0) return round_up(gemv, 256);
-    // the rebuilt weight, then the library GEMM's own scratch where that is the kernel, or the product's partial sums
-    const bool library = library_ok && dense_wants_library(M, N);
-    return round_up((int64_t)M * N * 2, 256) + round_up(std::max(library ? BS_DENSE_LIBRARY_WORKSPACE : 0, bs_linear_parts_bytes(T, M, N)), 256);
+    const int64_t gemv = bs_gemv_group_workspace_bytes(&I, &M, 1, N, K, T);
+    return gemv > 0 ? gemv : rebuild_need(M, N, T, library_ok);
 }
 
 extern "C" int64_t bs_workspace_bytes(int I, int M, int N, int K, int T) { return workspace_need(I, M, N, K, T, true); }
@@ -130,17 +132,13 @@ static int forward_impl(const uint8_t *packed, const void *u, const void *vt, co
     if (!bs_aligned(packed, 16) || !bs_aligned(vt, 16) || !bs_aligned(x, 16) || !bs_aligned(u, 8) ||
         !bs_aligned(y, 2) || !bs_aligned(bias, 2))
         return BS_ERR_ALIGN;
-    const int64_t need = workspace_need(I, M, N, K, T, library_ok);
-    if (need > 0 && (!workspace || workspace_bytes < need || !bs_aligned(workspace, 256)))
-        return BS_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
 
-    if (bs_gemv_workspace_bytes(I, M, N, K, T) > 0) {
-        st = bs_launch_gemv(packed, (const half_t *)u, (const half_t *)vt, (const half_t *)x,
-                            (const half_t *)bias, (half_t *)y, I, M, N, K, T, workspace,
-                            workspace_bytes, s);
-        return st;
-    }
+    bool taken;                                  // (asked once, with the plan: a decode call is over in some 8 us)
+    st = bs_launch_gemv(packed, (const half_t *)u, (const half_t *)vt, (const half_t *)x, (const half_t *)bias, (half_t *)y, I, M, N, K, T,
+                        workspace, workspace_bytes, &taken, s);
+    if (taken) return st;
+    if (!workspace || workspace_bytes < rebuild_need(M, N, T, library_ok) || !bs_aligned(workspace, 256)) return BS_ERR_WORKSPACE;
     half_t *w = (half_t *)workspace;
     st = bs_launch_reconstruct_packed(packed, (const half_t *)u, (const half_t *)vt, w, I, M, N, K, s);
     if (st != BS_OK) return st;
@@ -221,7 +219,7 @@ extern "C" int64_t bs_forward_group_workspace_bytes(const bs_matrix *mats, int n
     int I[BS_MAX_GROUP], M[BS_MAX_GROUP];
     for (int j = 0; j < n; j++) { I[j] = mats[j].I; M[j] = mats[j].M; }
     const int64_t b = bs_gemv_group_workspace_bytes(I, M, n, N, K, T);
-    return b > 0 ? round_up(b, 256) : (int64_t)BS_ERR_SHAPE;
+    return b > 0 ? b : (int64_t)BS_ERR_SHAPE;
 }
 
 static int forward_group(const bs_matrix *mats, int n, int N, int K, const void *x, int T,
@@ -247,9 +245,6 @@ static int forward_group(const bs_matrix *mats, int n, int N, int K, const void 
         M[j] = mats[j].M;
     }
     if (!bs_aligned(x, 16) || !bs_aligned(y, 2) || !bs_aligned(residual, 2)) return BS_ERR_ALIGN;
-    const int64_t need = bs_forward_group_workspace_bytes(mats, n, N, K, T);
-    if (need < 0) return (int)need;
-    if (!workspace || workspace_bytes < need || !bs_aligned(workspace, 256)) return BS_ERR_WORKSPACE;
     return bs_launch_gemv_group(n, packed, u, vt, bias, I, M, N, K, (const half_t *)x, T, epilogue,
                                 (const half_t *)residual, (half_t *)y, input_rms, eps, workspace, workspace_bytes,
                                 (hipStream_t)stream);

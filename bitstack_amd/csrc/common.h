@@ -74,8 +74,7 @@ int bs_launch_linear_library(const half_t *x, const half_t *w, const half_t *bia
                              void *workspace, hipStream_t s);
 int bs_launch_gemv(const uint8_t *packed, const half_t *u, const half_t *vt, const half_t *x,
                    const half_t *bias, half_t *y, int I, int M, int N, int K, int T,
-                   void *workspace, int64_t workspace_bytes, hipStream_t s);
-int64_t bs_gemv_workspace_bytes(int I, int M, int N, int K, int T);
+                   void *workspace, int64_t workspace_bytes, bool *taken, hipStream_t s);
 void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave, int *grid, int *kmax);
 int bs_gemv_plan_kernel(int I, int M, int N, int K, int T);
 int bs_gemv_forward_path(int I, int M, int N, int K, int T);

@@ -727,19 +727,19 @@ void one_per_cu(Plan &p, const int *I, const int *M, int T) {
     p.part_total = off;
 }
 
-Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
-    Plan p;
+// mx_r: what mx_rows_per_tile says, where the caller has asked already.
+void make_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T, int mx_r = -1) {
     p.n = n;
     p.n_chunks = N / CH;
     p.mx = p.sparse = 0;
-    const int mx_r = mx_rows_per_tile(I, M, n, N, K, T);
+    if (mx_r < 0) mx_r = mx_rows_per_tile(I, M, n, N, K, T);
     if (mx_r > 0) {
         // units are (block, row tile, 1024 columns), never paired
         p.mx = 1;
         p.R = mx_r;
         p.n_chunks = (int)bs_cdiv(N, MX_UNIT_COLS / T);
         one_per_cu(p, I, M, T);
-        return p;
+        return;
     }
     // rows per workgroup: 512 (8 waves x 4 tiles), 256, 128, 64; resident workgroups per CU.
     // Three or four tokens need more than the 128 registers a lane has with two 8-wave
@@ -839,12 +839,10 @@ Plan make_plan(const int *I, const int *M, int n, int N, int K, int T) {
     }
     p.grid = first;
     p.part_total = off;
-    return p;
 }
 
 // The plan of the sparse kernel where it serves these matrices, for the rules at sparse_plan.
-Plan sparse_plan_of(const int *I, const int *M, int n, int N, int T) {
-    Plan p;
+void sparse_plan_of(Plan &p, const int *I, const int *M, int n, int N, int T) {
     p.n = n;
     p.mx = 0;
     p.sparse = 1;
@@ -864,7 +862,6 @@ Plan sparse_plan_of(const int *I, const int *M, int n, int N, int T) {
         }
     }
     one_per_cu(p, I, M, T);
-    return p;
 }
 
 struct GroupArgs {          // host-side view of one call
@@ -981,7 +978,7 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
     if (floats == 0 || floats * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) return false;
     return cycles <= 50000. * T && !(T == 3 && n > 1 && bytes <= (8 << 20) && cycles > 16000.);
 }
-// The sparse kernel's plan where it serves the call; grid 0: another kernel does.
+// The sparse kernel's plan where it serves the call; false: another kernel does.
 //   N % 512 == 0: one to three tokens in the place of gemv_kernel.  us gemv_kernel / sparse, one token: 1024 x 4096, 3 blocks 8.1 / 7.2, 4096 x 4096, 2 8.6 / 7.8, 14336 x 4096, 1
 //     10.7 / 9.1 (below a MiB of sign bytes either is a chain of latencies, gemv_kernel's the shorter one: 355 x 2560, 4 6.3 / 6.9, 308 x 3584, 5 6.9 / 7.1); two: 1024 x 4096, 3 10.4 / 7.6, 4096 x 4096, 1 8.9 / 7.7, 14336 x 4096, 1 13.1 / 10.8; three: 4096 x 14336, 16 87.5 / 83.4, 3
 //     31.1 / 27.8, 28672 x 8192, 2 52.0 / 47.6, 1024 x 4096, 1 8.6 / 7.4.  Four: 4096 x 14336, 16 104 / 116, 28672 x 8192, 2 58.6 / 64.1: gemv_kernel keeps them.
@@ -990,39 +987,64 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
 //     MiB of sign bytes the two are about a us apart (5877 x 640, 1 block 7.2 / 6.0) and at rank 16 the tile kernel, whose tests hold it to calls of that size, keeps them.
 // Over 97 drawn calls 1.21 times as fast at one token, 1.23 at two, 1.19 at three, none more than 1 % slower.  It rounds nothing but y: error against float64 before that rounding 1e-7 to 4e-7 on drawn factors.  (Never with more partial sums than bs_forward_static's scratch holds.)
 constexpr int64_t SPARSE_MIN_UNEVEN = 512 << 10, SPARSE_MIN_ONE = 1 << 20;
-Plan sparse_plan(const int *I, const int *M, int n, int N, int K, int T) {
-    Plan p;
-    p.grid = 0;
+// (path: what group_path says; mx_r: what mx_rows_per_tile says at one to three tokens and N % 512 == 0)
+bool sparse_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T, int path, int mx_r) {
     const bool even = N % CH == 0;
-    if (n < 1 || n > GEMV_MAX_GROUP || g_decode_kernel != 0 || T > (even ? 3 : 2) || !bs_gemv_sparse_takes(N, K, 1, T) || group_path(I, M, n, N, K, T) != (even ? 0 : 1)) return p;
-    if (even && mx_rows_per_tile(I, M, n, N, K, T) > 0) return p;
+    if (g_decode_kernel != 0 || T > (even ? 3 : 2) || path != (even ? 0 : 1) || !bs_gemv_sparse_takes(N, K, 1, T) || (even && mx_r > 0)) return false;
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
-        if (!block_fits(I[j], M[j], N, K)) return p;
+        if (!block_fits(I[j], M[j], N, K)) return false;
         bytes += (int64_t)I[j] * M[j] * (N / 8);
     }
-    if ((!even && K == 16 && bytes < SPARSE_MIN_UNEVEN) || (even && T == 1 && bytes < SPARSE_MIN_ONE)) return p;
-    p = sparse_plan_of(I, M, n, N, T);
-    if (p.part_total * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) p.grid = 0;
-    return p;
-}
-int64_t sparse_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
-    const Plan p = sparse_plan(I, M, n, N, K, T);
-    return p.grid ? p.part_total : 0;
+    if ((!even && K == 16 && bytes < SPARSE_MIN_UNEVEN) || (even && T == 1 && bytes < SPARSE_MIN_ONE)) return false;
+    sparse_plan_of(p, I, M, n, N, T);
+    return p.part_total * (int64_t)sizeof(float) <= BS_STATIC_SCRATCH_BYTES;
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group
     for (int j = 0; j < n; j++) total += (int64_t)bs_strip_partials(I[j], M[j], N, K, T) * T * M[j];
     // room for the tile kernel's partial sums too: the choice also depends on how u is aligned
-    return std::max(std::max(total, tile_part_floats(I, M, n, N, K, T)), sparse_part_floats(I, M, n, N, K, T));
+    return std::max(total, tile_part_floats(I, M, n, N, K, T));
 }
+
+// Everything that a call's sizes decide, worked out once per size query and once per call: a forward of some 8 us is bound by the host.  ns of a size query, every
+// kernel's plan and the path asked for where they are needed / once: 1024 x 4096, 3 blocks, one token 106 / 47, 4096 x 11008, 4 blocks 175 / 50, 14336 x 4096, 8 blocks
+// 54 / 42; us of a BitStackLinear.forward of the first, a size query and two plans less: 8.8 / 8.45 (8.6 with gemv_kernel alone to plan).
+struct CallPlan {
+    int path;          // group_path
+    bool split;        // three or four tokens on the tile kernel where u's alignment allows it
+    bool sparse;       // the sparse kernel, in gemv_kernel's (path 0) or the strip kernel's place (path 1)
+    Plan gemv;         // of the first pass, where it is no strips
+    int64_t floats;    // scratch
+};
+void plan_call(CallPlan &c, const int *I, const int *M, int n, int N, int K, int T) {
+    c.path = group_path(I, M, n, N, K, T);
+    c.split = c.sparse = false;
+    c.floats = 0;
+    if (c.path < 0) return;
+    const int tp = pass_tokens(T), mx_r = c.path == 0 ? mx_rows_per_tile(I, M, n, N, K, tp) : 0;
+    c.sparse = sparse_plan(c.gemv, I, M, n, N, K, T, c.path, mx_r);
+    if (c.sparse) {
+        c.floats = c.gemv.part_total;
+    } else if (c.path == 1) {
+        c.floats = strip_part_floats(I, M, n, N, K, T);
+    } else {
+        if (T % tp) {                                // a shorter last pass
+            make_plan(c.gemv, I, M, n, N, K, T % tp);
+            c.floats = c.gemv.part_total;
+        }
+        make_plan(c.gemv, I, M, n, N, K, tp, mx_r);
+        c.floats = std::max(c.floats, c.gemv.part_total);
+    }
+    c.split = c.path == 0 && split_tiles(I, M, n, N, K, T);
+    if (c.split) c.floats = std::max(c.floats, tile_part_floats(I, M, n, N, K, T));
+}
+int64_t scratch_bytes(const CallPlan &c) { return (c.floats * (int64_t)sizeof(float) + 255) / 256 * 256; }
 
 // Strip path: one launch writes part[strip group, t, m] of every matrix; the reduce kernel
 // reads that as "one partial per block" with the strip groups in the place of the blocks.
 int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T, int mode, const half_t *residual,
-                        half_t *y, bool input_rms, float eps, void *workspace, int64_t workspace_bytes, bool split, hipStream_t s) {
-    const int64_t floats = split ? tile_part_floats(a.I, a.M, a.n, N, K, T) : strip_part_floats(a.I, a.M, a.n, N, K, T);
-    if (!workspace || workspace_bytes < floats * (int64_t)sizeof(float)) return BS_ERR_WORKSPACE;
+                        half_t *y, bool input_rms, float eps, void *workspace, bool split, hipStream_t s) {
     float *part = (float *)workspace;
     RedGroup r;
     r.n = a.n;
@@ -1072,29 +1094,24 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     return BS_OK;
 }
 
+// *taken = false (and BS_ERR_SHAPE): no packed-sign kernel takes the shapes.  The scratch is looked at before anything is enqueued.
 int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int mode, const half_t *residual,
-                 half_t *y, bool input_rms, float eps, void *workspace, int64_t workspace_bytes, hipStream_t s) {
-    if (a.n < 1 || a.n > GEMV_MAX_GROUP) return BS_ERR_SHAPE;
+                 half_t *y, bool input_rms, float eps, void *workspace, int64_t workspace_bytes, bool *taken, hipStream_t s) {
+    CallPlan c;
+    plan_call(c, a.I, a.M, a.n, N, K, T);
+    *taken = c.path >= 0;
+    if (c.path < 0) return BS_ERR_SHAPE;
+    if (!workspace || workspace_bytes < scratch_bytes(c) || !bs_aligned(workspace, 256)) return BS_ERR_WORKSPACE;
     if (!bs_aligned(x, 16)) return BS_ERR_SHAPE;
     if (mode == EPI_SWIGLU && (a.n != 2 || a.M[0] != a.M[1])) return BS_ERR_SHAPE;
-    const int path = group_path(a.I, a.M, a.n, N, K, T);
-    if (path < 0) return BS_ERR_SHAPE;
     for (int j = 0; j < a.n; j++)
         if (!bs_aligned(a.packed[j], 16) || !bs_aligned(a.vt[j], 16) || !bs_aligned(a.u[j], 8)) return BS_ERR_SHAPE;
-    bool split = path == 0 && split_tiles(a.I, a.M, a.n, N, K, T);
+    bool split = c.split;
     for (int j = 0; j < a.n; j++) split = split && bs_aligned(a.u[j], 16);
-    const Plan sparse = sparse_plan(a.I, a.M, a.n, N, K, T);
-    if (split || (path == 1 && sparse.grid == 0))
-        return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, workspace_bytes, split, s);
+    if (split || (c.path == 1 && !c.sparse)) return launch_group_strips(a, N, K, x, T, mode, residual, y, input_rms, eps, workspace, split, s);
     int ldy = 0;
-    for (int j = 0; j < a.n; j++) {
-        if (sparse.grid == 0 && !gemv_shape_ok(a.I[j], a.M[j], N, K, T)) return BS_ERR_SHAPE;
-        ldy += a.M[j];
-    }
-    if (mode == EPI_SWIGLU) {
-        if (a.n != 2 || a.M[0] != a.M[1]) return BS_ERR_SHAPE;
-        ldy = a.M[0];
-    }
+    for (int j = 0; j < a.n; j++) ldy += a.M[j];
+    if (mode == EPI_SWIGLU) ldy = a.M[0];
     // Tokens go in passes of tp, the last one possibly shorter.  Every pass length has its own
     // plan (instantiation, grid, partial layout): the kernel a plan names exists for that token
     // count only.  Passes run one after the other on the stream and share the workspace.
@@ -1102,8 +1119,8 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
     float *part = (float *)workspace;
     for (int t0 = 0; t0 < T; t0 += tp) {
         const int tn = (T - t0 < tp) ? T - t0 : tp;
-        const Plan p = sparse.grid ? sparse : make_plan(a.I, a.M, a.n, N, K, tn);
-        if (!workspace || workspace_bytes < p.part_total * (int64_t)sizeof(float)) return BS_ERR_WORKSPACE;
+        if (tn != tp) make_plan(c.gemv, a.I, a.M, a.n, N, K, tn);
+        const Plan &p = c.gemv;
         GemvGroup g;
         RedGroup r;
         g.n = r.n = a.n;
@@ -1152,43 +1169,24 @@ int launch_group(const GroupArgs &a, int N, int K, const half_t *x, int T, int m
     return BS_OK;
 }
 
-// Scratch the factor-through path needs: the largest partial area over its passes.
-int64_t gemv_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
-    const int tp = pass_tokens(T), tail = T % tp;
-    int64_t need = make_plan(I, M, n, N, K, tp).part_total;
-    if (tail) {
-        const int64_t t2 = make_plan(I, M, n, N, K, tail).part_total;
-        if (t2 > need) need = t2;
-    }
-    return need;
-}
-
 }  // namespace
-
-int64_t bs_gemv_workspace_bytes(int I, int M, int N, int K, int T) {
-    return bs_gemv_group_workspace_bytes(&I, &M, 1, N, K, T);
-}
 
 // Bytes of scratch the packed-sign paths (factor-through or strip kernel) need for these
 // matrices and token count; 0 when neither takes them.
 int64_t bs_gemv_group_workspace_bytes(const int *I, const int *M, int n, int N, int K, int T) {
-    const int path = group_path(I, M, n, N, K, T);
-    if (path < 0) return 0;
-    if (path == 1) return strip_part_floats(I, M, n, N, K, T) * (int64_t)sizeof(float);
-    int64_t floats = std::max(gemv_part_floats(I, M, n, N, K, T), sparse_part_floats(I, M, n, N, K, T));
-    if (split_tiles(I, M, n, N, K, T)) floats = std::max(floats, tile_part_floats(I, M, n, N, K, T));
-    return floats * (int64_t)sizeof(float);
+    CallPlan c;
+    plan_call(c, I, M, n, N, K, T);
+    return scratch_bytes(c);
 }
 
 // Which instantiation and grid a decode forward of these dimensions runs
 // (0 in *waves when the decode kernel does not take them).
 void bs_gemv_plan_info(int I, int M, int N, int K, int T, int *waves, int *row_tiles_per_wave, int *grid, int *kmax) {
     *waves = *row_tiles_per_wave = *grid = *kmax = 0;
-    Plan p = sparse_plan(&I, &M, 1, N, K, T);                    // (also in the strip kernel's place)
-    if (p.grid == 0) {
-        if (group_path(&I, &M, 1, N, K, T) != 0) return;
-        p = make_plan(&I, &M, 1, N, K, pass_tokens(T));
-    }
+    CallPlan c;
+    plan_call(c, &I, &M, 1, N, K, T);
+    if (c.path != 0 && !c.sparse) return;
+    const Plan &p = c.gemv;
     *waves = p.waves;
     *row_tiles_per_wave = p.R;
     *grid = p.grid;
@@ -1203,18 +1201,21 @@ int bs_gemv_forward_path(int I, int M, int N, int K, int T) {
         const int c = bs_strip_kernel_choice(I, M, N, K, T);
         return c == 1 ? BS_PATH_STRIP : c == 2 ? BS_PATH_WALKED : BS_PATH_PANEL;
     }
-    return make_plan(&I, &M, 1, N, K, pass_tokens(T)).mx ? BS_PATH_DECODE_MX : BS_PATH_DECODE_F16;
+    return mx_rows_per_tile(&I, &M, 1, N, K, pass_tokens(T)) > 0 ? BS_PATH_DECODE_MX : BS_PATH_DECODE_F16;
 }
 
 // 1: gemv_sparse_kernel runs these matrices, of three tokens only with u off a 16-byte boundary where split_tiles has the tile kernel take them
 int bs_gemv_sparse_serves(const int *I, const int *M, int n, int N, int K, int T) {
-    return sparse_plan(I, M, n, N, K, T).grid > 0 && !split_tiles(I, M, n, N, K, T);
+    CallPlan c;
+    plan_call(c, I, M, n, N, K, T);
+    return c.sparse && !c.split;
 }
 
 // Which call of the tile and column kernels serves these matrices, with u on 16-byte boundaries (values of BS_TILE_* in the public header).
 int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
     const int path = group_path(I, M, n, N, K, T);
-    if (path == 1 && T < STRIP_MIN_T && sparse_plan(I, M, n, N, K, T).grid > 0) return BS_TILE_NONE;
+    Plan p;
+    if (path == 1 && sparse_plan(p, I, M, n, N, K, T, path, 0)) return BS_TILE_NONE;
     if (path == 1 && (n == 1 || T <= 48)) return !bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_NONE : T > 48 ? BS_TILE_COLUMN : BS_TILE_FORWARD;
     if (path == 0) return split_tiles(I, M, n, N, K, T) && bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_TWO_TERMS : BS_TILE_NONE;
     for (int j = 0; j < n; j++)
@@ -1225,7 +1226,7 @@ int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, 
 // 0: not a decode-kernel shape, 1: gemv_kernel (fp16 MFMA), 2: gemv_mx_kernel (block-scaled fp4 x fp6 MFMA)
 int bs_gemv_plan_kernel(int I, int M, int N, int K, int T) {
     if (group_path(&I, &M, 1, N, K, T) != 0) return 0;
-    return make_plan(&I, &M, 1, N, K, pass_tokens(T)).mx ? 2 : 1;
+    return mx_rows_per_tile(&I, &M, 1, N, K, pass_tokens(T)) > 0 ? 2 : 1;
 }
 
 int bs_gemv_set_kernel(int mode) {
@@ -1234,15 +1235,15 @@ int bs_gemv_set_kernel(int mode) {
     return BS_OK;
 }
 
-// Returns BS_ERR_SHAPE when the fast path does not apply (the caller falls
-// back to rebuilding the weight); any other status is final.
+// *taken = false when the fast path does not apply (the caller falls
+// back to rebuilding the weight); otherwise the status is final.
 int bs_launch_gemv(const uint8_t *packed, const half_t *u, const half_t *vt, const half_t *x,
                    const half_t *bias, half_t *y, int I, int M, int N, int K, int T,
-                   void *workspace, int64_t workspace_bytes, hipStream_t s) {
+                   void *workspace, int64_t workspace_bytes, bool *taken, hipStream_t s) {
     GroupArgs a;
     a.n = 1;
     a.packed[0] = packed; a.u[0] = u; a.vt[0] = vt; a.bias[0] = bias; a.I[0] = I; a.M[0] = M;
-    return launch_group(a, N, K, x, T, EPI_NONE, nullptr, y, false, 0.f, workspace, workspace_bytes, s);
+    return launch_group(a, N, K, x, T, EPI_NONE, nullptr, y, false, 0.f, workspace, workspace_bytes, taken, s);
 }
 
 int bs_launch_gemv_group(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt,
@@ -1251,11 +1252,12 @@ int bs_launch_gemv_group(int n, const uint8_t *const *packed, const half_t *cons
                          int64_t workspace_bytes, hipStream_t s) {
     if (n < 1 || n > GEMV_MAX_GROUP) return BS_ERR_SHAPE;
     if (mode == EPI_RESIDUAL && !residual) return BS_ERR_NULL;
+    bool taken;
     GroupArgs a;
     a.n = n;
     for (int j = 0; j < n; j++) {
         a.packed[j] = packed[j]; a.u[j] = u[j]; a.vt[j] = vt[j]; a.bias[j] = bias ? bias[j] : nullptr;
         a.I[j] = I[j]; a.M[j] = M[j];
     }
-    return launch_group(a, N, K, x, T, mode, residual, y, input_rms != 0, eps, workspace, workspace_bytes, s);
+    return launch_group(a, N, K, x, T, mode, residual, y, input_rms != 0, eps, workspace, workspace_bytes, &taken, s);
 }

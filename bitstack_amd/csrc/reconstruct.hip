@@ -506,7 +506,7 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
         if (st != BS_OK) return st;
         dim3 grid((unsigned)bs_cdiv(strips, 8) * 8, row_groups);
         kernel<<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
-    } else if (N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && bs_aligned(u, 8) && (PACKED || bs_aligned(sign, 8))) {
+    } else if (N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && (K != 16 || bs_aligned(u, 8)) && (PACKED || bs_aligned(sign, 8))) {
         const int strips = (int)bs_cdiv(N, RA_COLS), steps = (int)bs_cdiv(M, RA_ROWS);
         const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), steps / RA_STREAMS));    // four workgroups per CU, a step per wave or more
         const int per = (int)bs_cdiv(bs_cdiv(steps, groups), RA_STREAMS) * RA_STREAMS;

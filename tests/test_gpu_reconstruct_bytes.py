@@ -38,3 +38,23 @@ def test_rebuild_of_byte_columns(blocks, m, n, k, shifted):
     bound = want.abs() * 2.0 ** -11 + size * (k + blocks + 1) * 2.0 ** -24 + 2.0 ** -25
     assert ((w.double() - want).abs() <= bound).all()
     assert torch.equal(w, IU.reconstruct_w_hip(sign, u, vt))
+
+
+# ranks below 16 are read half by half: u need not lie on 8 bytes (one output per thread, which sums in another order, is for what the kernel cannot read)
+@pytest.mark.parametrize("blocks,m,n,k", [(3, 333, 200, 5), (2, 1000, 1000, 15), (5, 129, 256, 12), (4, 512, 6008, 1)])
+def test_where_u_lies_does_not_matter_below_rank_16(blocks, m, n, k):
+    from bitstack_amd.utils import inference_utils as IU
+
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    packed = torch.randint(0, 256, (blocks, m * n // 8), dtype=torch.uint8, device="cuda", generator=g)
+    room = torch.randn(blocks * m * k + 1, device="cuda", generator=g).half()
+    vt = torch.randn(blocks, k, n, device="cuda", generator=g).half()
+    print(blocks, m, n, k, flush=True)
+    u = room[1:].view(blocks, m, k)
+    assert u.data_ptr() % 8 == 2
+    w, sign = IU.unpack_and_reconstruct_w_hip(packed, u, vt), exact(packed, u, vt)[2]
+    assert torch.equal(w, IU.reconstruct_w_hip(sign, u, vt))
+    if n % 128:                                      # (multiples of 128 with u on 8 bytes are the tiled kernel's)
+        assert torch.equal(w, IU.unpack_and_reconstruct_w_hip(packed, u.clone(), vt))
+    else:
+        assert torch.equal(w, IU.unpack_and_reconstruct_w_hip(packed, u.clone(), torch.cat([vt.new_zeros(4), vt.flatten()])[4:].view_as(vt)))

@@ -38,6 +38,7 @@ SIGNATURES = {
     "bs_sparse_kernel": (_I, [_P, _P, _I, _I, _I, _I]),
     "bs_tile_kernel": (_I, [_P, _P, _I, _I, _I, _I, _P]),
 }
+ERR_WORKSPACE = -5
 DECODE_AUTO, DECODE_F16, DECODE_MX = 0, 1, 2
 DENSE_AUTO, DENSE_OWN, DENSE_LIBRARY = 0, 1, 2
 PREFILL_AUTO, PREFILL_REBUILD, PREFILL_WALKED, PREFILL_PANEL = 0, 1, 2, 3

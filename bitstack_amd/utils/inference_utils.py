@@ -126,8 +126,8 @@ class MatrixGroup:
             mats.append((q, u, vt, m.bias))
         return cls(mats)
 
-    def workspace_bytes(self, T):
-        if T not in self._need:
+    def workspace_bytes(self, T, again=False):
+        if again or T not in self._need:
             self._need[T] = int(_lib.lib().bs_forward_group_workspace_bytes(self.arr, self.n, self.N, self.K, T))
         return self._need[T]
 
@@ -153,15 +153,17 @@ def bitstack_forward_group_hip(group: MatrixGroup, x, epilogue=_lib.EPI_NONE, re
     y = out if out is not None else torch.empty((T, width), dtype=torch.float16, device=dev)
     if y.dtype != torch.float16 or not y.is_contiguous() or y.numel() != T * width:
         raise ValueError("out must be a contiguous fp16 [T, width] tensor")
-    with torch.cuda.device(dev), _lib.scratch(dev, need) as ws:
-        if rms_eps is None:
-            _lib.check(_lib.lib().bs_forward_group(group.arr, group.n, group.N, group.K, _lib.ptr(x2), T, epilogue,
-                                                   _lib.ptr(residual), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                                                   _lib.stream_ptr(dev)), "bs_forward_group")
-        else:
-            _lib.check(_lib.lib().bs_forward_group_rms(group.arr, group.n, group.N, group.K, _lib.ptr(x2), T, float(rms_eps),
-                                                       epilogue, _lib.ptr(residual), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                                                       _lib.stream_ptr(dev)), "bs_forward_group_rms")
+    def call(need):
+        with torch.cuda.device(dev), _lib.scratch(dev, need) as ws:
+            behind = (_lib.ptr(residual), _lib.ptr(y), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev))
+            if rms_eps is None:
+                return _lib.lib().bs_forward_group(group.arr, group.n, group.N, group.K, _lib.ptr(x2), T, epilogue, *behind)
+            return _lib.lib().bs_forward_group_rms(group.arr, group.n, group.N, group.K, _lib.ptr(x2), T, float(rms_eps), epilogue, *behind)
+
+    status = call(need)
+    if status == _lib.ERR_WORKSPACE:             # another kernel has been pinned since (bs_set_decode_kernel): its scratch may be larger
+        status = call(group.workspace_bytes(T, again=True))
+    _lib.check(status, "bs_forward_group" if rms_eps is None else "bs_forward_group_rms")
     return y
 
 

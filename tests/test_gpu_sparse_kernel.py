@@ -168,3 +168,25 @@ def test_groups_with_the_epilogues(layers, N, T):
     if len(layers) == 2:
         a, b = got[:, :layers[0][1]].double(), got[:, layers[0][1]:].double()
         assert close(IU.bitstack_forward_group_hip(group, x, epilogue=_lib.EPI_SWIGLU), a * torch.sigmoid(a) * b, 8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,N,T", [([(16, 4096)], 14336, 1), ([(8, 14336)], 4096, 1), ([(3, 9000), (2, 20000)], 1408, 2)])
+def test_a_group_follows_the_pinned_kernel(layers, N, T):
+    """Another kernel pinned after a group's first call needs other scratch: it is asked for again."""
+    parts = [_layer(I, M, N, 16, T) for I, M in layers]
+    group, x, L = IU.MatrixGroup([p[:3] + (None,) for p in parts]), parts[0][3], _lib.lib()
+    want = torch.cat([p[4] for p in parts], 1) if len(layers) == 1 else None
+    size, ys = torch.cat([p[5] for p in parts], 1), []
+    try:
+        for mode in (_lib.DECODE_AUTO, _lib.DECODE_F16, _lib.DECODE_MX, _lib.DECODE_AUTO):
+            L.bs_set_decode_kernel(mode)
+            with torch.cuda.stream(torch.cuda.Stream()):         # scratch of its own: the smallest there is
+                ys.append(IU.bitstack_forward_group_hip(group, x))
+            torch.cuda.synchronize()
+    finally:
+        L.bs_set_decode_kernel(_lib.DECODE_AUTO)
+    assert torch.equal(ys[0], ys[3])
+    want = ys[0].double() if want is None else want
+    # vt * x, or the weight, rounded to fp16 once, and y
+    assert all(bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -10 + size * 2.0 ** -11).all()) for y in ys)

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256, 4) void reconstruct_tile_kernel(
 // step of 32 rows, in two patches of v_mfma_f32_32x32x16_f16, D[column, row], with the columns dealt so that a lane ends with 32 consecutive ones of one row: one
 // unaligned word of signs, four 16-byte stores.  u rows and signs are requested one (row step, block) ahead, in two register sets that take turns.  Signs come out of
 // the tiled kernel's table and go in by the same mixed-precision FMA (int8 signs: converted; the same sum).
-// What bounds it: the vector instructions, 24 per step of 1024 signs, and its stores.  Rebuilds, us, one output per thread / this: 4096 x 4104
+// What bounds it: the vector instructions, 24 per step of 1024 signs, and its stores.  Rebuilds at rank 16, us, one output per thread / this: 4096 x 4104
 // of 1 block 101 / 18, of 4 385 / 23; 6144 x 6136 of 8 1641 / 53; 512 x 6008 of 4 63 / 8.2; 1000 x 1000 of 4 23 / 5.4.  (Four waves, each with 128 columns as the
 // tiled kernel has them, and vt fragments in registers for the block at hand: 23 to 85 where this takes 19 to 53.)
 constexpr int RA_COLS = 128, RA_ROWS = 32, RA_WAVES = 8, RA_STREAMS = 4;         // columns per workgroup, rows per step, waves, waves side by side in rows
@@ -476,6 +476,21 @@ __global__ __launch_bounds__(256) void reconstruct_generic_kernel(
     }
 }
 
+// Steps of 32 rows per workgroup of reconstruct_byte_kernel: four workgroups per CU, and a step or more for each of the four waves side by side in rows.
+int byte_steps(int M, int N) {
+    const int64_t strips = bs_cdiv(N, RA_COLS), steps = bs_cdiv(M, RA_ROWS);
+    const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), bs_cdiv(steps, RA_STREAMS)));
+    return (int)bs_cdiv(bs_cdiv(steps, groups), RA_STREAMS) * RA_STREAMS;
+}
+// At rank 16 always.  Below, u is read half by half, and a wave's chain of (row step, block) pairs is some 0.9 us each; one output per thread takes 0.07 + 0.1 us
+// per rank and block, or its products' time where there are many: us, that / byte kernel, 337 x 40, 7 blocks, rank 1 3.9 / 11.5, 520 x 248, 9, rank 8 10.8 / 24.5, 1371 x 296, 5, rank 1
+// 4.4 / 10.0; 4096 x 4104, 4, rank 8 244 / 39, 2374 x 1248, 12, rank 5 68.5 / 14.9.  Of 600 drawn rebuilds (up to 12 blocks, 6 million weights, ranks 1 to 16) 8 are more
+// than 3 % behind the former with this rule, 17 % at worst; without it 260 of 900, 120 %.
+bool byte_kernel_pays(int I, int M, int N, int K) {
+    const double chain = 1.0 + 0.9 * I * (byte_steps(M, N) / RA_STREAMS);
+    return K == 16 || chain <= std::max((0.07 + 0.1 * K) * I, 0.33e-6 * M * N * I * (K + 2));
+}
+
 template <bool PACKED>
 int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *u, const half_t *vt,
                        half_t *w, int I, int M, int N, int K, hipStream_t s) {
@@ -483,6 +498,8 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
     const bool small = (int64_t)M * (N >> 3) < ((int64_t)1 << 32) && (int64_t)M * K * 2 < ((int64_t)1 << 32);
     const bool tiled = (N % RT_COLS == 0) && I >= 1 && I <= RT_MAXB && small && bs_aligned(vt, 16) && bs_aligned(w, 16) &&
                        bs_aligned(u, 8) && (PACKED ? bs_aligned(packed, 16) : bs_aligned(sign, 4));
+    const bool bytes = N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && (K != 16 || bs_aligned(u, 8)) && (PACKED || bs_aligned(sign, 8)) &&
+                       byte_kernel_pays(I, M, N, K);
     if (tiled) {
         // One wave of workgroups: as many row groups as the resident slots allow (LDS decides
         // how many workgroups a CU holds), so that no second, partial wave trails behind.
@@ -506,10 +523,8 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
         if (st != BS_OK) return st;
         dim3 grid((unsigned)bs_cdiv(strips, 8) * 8, row_groups);
         kernel<<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);
-    } else if (N % 8 == 0 && N >= 32 && I >= 1 && I <= RA_MAXB && bs_aligned(w, 16) && (K != 16 || bs_aligned(u, 8)) && (PACKED || bs_aligned(sign, 8))) {
-        const int strips = (int)bs_cdiv(N, RA_COLS), steps = (int)bs_cdiv(M, RA_ROWS);
-        const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), steps / RA_STREAMS));    // four workgroups per CU, a step per wave or more
-        const int per = (int)bs_cdiv(bs_cdiv(steps, groups), RA_STREAMS) * RA_STREAMS;
+    } else if (bytes) {
+        const int strips = (int)bs_cdiv(N, RA_COLS), steps = (int)bs_cdiv(M, RA_ROWS), per = byte_steps(M, N);
         const size_t lds = SIGN_LUT_HALVES * sizeof(half_t) + (size_t)I * 256 * sizeof(half8_t);
         static bs_lds_grant granted[2][BS_MAX_DEVICES];
         const void *kernel = K == 16 ? (const void *)reconstruct_byte_kernel<PACKED, true> : (const void *)reconstruct_byte_kernel<PACKED, false>;

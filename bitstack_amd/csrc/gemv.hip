@@ -655,6 +655,7 @@ struct Plan {
     int waves, R, n_chunks, grid, n, pair;
     int mx;        // 1: the block-scaled fp4 x fp6 kernel (gemv_mx.hip), units of MX_UNIT_COLS columns
     int sparse;    // 1: the sparse kernel (gemv_sparse.hip)
+    double us;     // ... of it: what the choice of R takes a call for, partial sums left out
     int row_tiles[GEMV_MAX_GROUP], kmax[GEMV_MAX_GROUP], first_wg[GEMV_MAX_GROUP];
     Split sp[GEMV_MAX_GROUP];
     int64_t part_off[GEMV_MAX_GROUP];      // in floats; part_off[n] = total
@@ -861,8 +862,22 @@ void sparse_plan_of(Plan &p, const int *I, const int *M, int n, int N, int T) {
             p.R = 1 << k;
         }
     }
+    p.us = best;
     one_per_cu(p, I, M, T);
 }
+
+// us of one matrix's call on the sparse kernel, and on the tile and strip kernels (estimates for the choice between them, fitted to 900 calls on rotating
+// sizes, each within 4 to 5 % as a rule, the strip kernel's 8).  The summing launch adds a slot in 7 to 9 ns: few rows of many columns have hundreds.
+double sparse_call_us(const Plan &p, int I, int T) {
+    static const double c[3][4] = {{-2.53, 1.388, 0.0071, 0.138}, {-2.67, 1.357, 0.0082, 0.315}, {-2.47, 1.302, 0.0092, 0.206}};
+    const double *k = c[T - 1];
+    return k[0] + k[1] * p.us + k[2] * I * p.kmax[0] - k[3] * std::max(0., p.us - 15.);
+}
+double tile_call_us(double cycles, int groups, int N, int T) {
+    const double width = groups == bs_cdiv(N, 256) ? 0.8 : groups == bs_cdiv(N, 512) ? 1. : 1.08;        // (columns per workgroup: narrow ones cost less than the plan's cycles say)
+    return T < 3 ? 5.34 + 3.98e-4 * width * cycles : 4.99 + 4.76e-4 * width * cycles;
+}
+double strip_call_us(long steps, int I) { return 6.8 + steps * (0.271 + 0.381 * I); }
 
 struct GroupArgs {          // host-side view of one call
     int n;
@@ -960,10 +975,12 @@ int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T,
 // of three tokens from 16,000 cycles on up to 8 MiB of sign bytes in all, which the factor-through kernel has in one round (2 x 8192 x 2048,
 // 2 blocks 14.2 / 18.2; 240 of 986 drawn groups, 0.95 on average; the others 1.05).
 // (What a group's matrices do alone is another matter: make_tile_plan compares single ones with the strip kernel too.)
-// Nor three tokens of one matrix with 4096 columns or more, where the sparse kernel is faster whatever the blocks (us tile / sparse: 4096 x 4096, 4 blocks 16.6 / 13.1, 8
-// 23.1 / 19.9; 14336 x 4096, 8 51.5 / 48.2; 1024 x 4096, 3 10.0 / 7.9).
-bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
-    if ((T != 3 && T != 4) || g_decode_kernel != 0 || (T == 3 && n == 1 && N >= 4096)) return false;
+// Nor three tokens of one matrix with 4096 columns or more where the sparse kernel is the faster one by the estimates above (us tile / sparse: 4096 x 4096, 4 blocks 16.6 /
+// 13.1, 8 23.1 / 19.9; 1024 x 4096, 3 10.0 / 7.9; but 144 x 26112, 8 11.1 / 17.1, 260 x 30208, 8 16.3 / 24.2, 4882 x 8192, 10 41.5 / 45.3.  Of 237 drawn calls, half of them of
+// up to 1000 rows, 8 are more than 3 % behind the tile kernel, 7 % at worst; all of them on the sparse kernel: 85, 55 %).
+// (sparse: its plan, where it serves the call)
+bool split_tiles(const int *I, const int *M, int n, int N, int K, int T, const Plan *sparse) {
+    if ((T != 3 && T != 4) || g_decode_kernel != 0) return false;
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
         const bool large = (int64_t)M[j] * N > (24ll << 20);
@@ -976,6 +993,7 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
     double cycles;
     const int64_t floats = tile_part_floats(I, M, n, N, K, T, &cycles);
     if (floats == 0 || floats * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) return false;
+    if (T == 3 && n == 1 && N >= 4096 && sparse && sparse_call_us(*sparse, I[0], T) <= tile_call_us(cycles, (int)(floats / T / (M[0] + 1)), N, T)) return false;
     return cycles <= 50000. * T && !(T == 3 && n > 1 && bytes <= (8 << 20) && cycles > 16000.);
 }
 // The sparse kernel's plan where it serves the call; false: another kernel does.
@@ -983,9 +1001,14 @@ bool split_tiles(const int *I, const int *M, int n, int N, int K, int T) {
 //     10.7 / 9.1 (below a MiB of sign bytes either is a chain of latencies, gemv_kernel's the shorter one: 355 x 2560, 4 6.3 / 6.9, 308 x 3584, 5 6.9 / 7.1); two: 1024 x 4096, 3 10.4 / 7.6, 4096 x 4096, 1 8.9 / 7.7, 14336 x 4096, 1 13.1 / 10.8; three: 4096 x 14336, 16 87.5 / 83.4, 3
 //     31.1 / 27.8, 28672 x 8192, 2 52.0 / 47.6, 1024 x 4096, 1 8.6 / 7.4.  Four: 4096 x 14336, 16 104 / 116, 28672 x 8192, 2 58.6 / 64.1: gemv_kernel keeps them.
 //   Other multiples of 128 columns, one and two tokens: us tile or strip kernel / sparse, one token: 4096 x 11008, 4 blocks 25.7 / 17.7, 8 39.3 / 25.6, 2 18.3 / 13.0;
-//     20000 x 1408, 2 15.6 / 9.0; 2048 x 5504, 3 11.9 / 9.0; two: 24.7 / 22.6, 39.1 / 32.8, 18.5 / 15.5, 15.3 / 10.5, 12.0 / 10.3; three: 24.7 / 27.4, 39.6 / 42.0.  Up to half a
-//     MiB of sign bytes the two are about a us apart (5877 x 640, 1 block 7.2 / 6.0) and at rank 16 the tile kernel, whose tests hold it to calls of that size, keeps them.
-// Over 97 drawn calls 1.21 times as fast at one token, 1.23 at two, 1.19 at three, none more than 1 % slower.  It rounds nothing but y: error against float64 before that rounding 1e-7 to 4e-7 on drawn factors.  (Never with more partial sums than bs_forward_static's scratch holds.)
+//     20000 x 1408, 2 15.6 / 9.0; 2048 x 5504, 3 11.9 / 9.0; two: 24.7 / 22.6, 39.1 / 32.8, 18.5 / 15.5, 15.3 / 10.5, 12.0 / 10.3; three: 24.7 / 27.4, 39.6 / 42.0.  Not
+//     where few rows of many columns leave hundreds of partial sums, or up to 256 columns half of a unit empty, and the other kernel is the faster one by the estimates (28 x 27392, 8 blocks, two
+//     tokens 8.8 / 12.4; 20204 x 128, 16 15.7 / 20.8).  At rank 16 it starts at half a MiB of sign bytes, though it is ahead below that too (300 drawn calls on the tile kernel 7.3 to 8.1 us, 0.85 of
+//     that at one token, 0.9 at two): the tile kernel's tests at one and two tokens are calls of that size.
+// Replayed on the same inputs, drawn calls take 0.84 of gemv_kernel's time (351 of one to three tokens, N % 512 == 0; one is more than 3 % behind, 4 %) and 0.75 of the tile and strip kernels' (357 of
+// one and two tokens at other column counts; 2, 5 %), groups of two to four matrices 0.76 (214; 1, 7 %).  A call as short as 8 us is bound by the host: 1024 x 4096, 3 blocks, one token by
+// BitStackLinear.forward 8.6 / 8.45.  It rounds nothing but y: error against float64 before that rounding 1e-7 to 4e-7 on drawn factors.  (Never with more partial sums than bs_forward_static's
+// scratch holds.)
 constexpr int64_t SPARSE_MIN_UNEVEN = 512 << 10, SPARSE_MIN_ONE = 1 << 20;
 // (path: what group_path says; mx_r: what mx_rows_per_tile says at one to three tokens and N % 512 == 0)
 bool sparse_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T, int path, int mx_r) {
@@ -998,7 +1021,13 @@ bool sparse_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T
     }
     if ((!even && K == 16 && bytes < SPARSE_MIN_UNEVEN) || (even && T == 1 && bytes < SPARSE_MIN_ONE)) return false;
     sparse_plan_of(p, I, M, n, N, T);
-    return p.part_total * (int64_t)sizeof(float) <= BS_STATIC_SCRATCH_BYTES;
+    if (p.part_total * (int64_t)sizeof(float) > BS_STATIC_SCRATCH_BYTES) return false;
+    if (even || n > 1) return true;
+    const int slots = I[0] * p.kmax[0];
+    double cycles;
+    int groups[GEMV_MAX_GROUP];
+    if (K == 16 && (slots >= 64 || p.n_chunks == 1) && bs_tile_partials(I, M, 1, N, K, T, groups, &cycles)) return sparse_call_us(p, I[0], T) <= tile_call_us(cycles, groups[0], N, T);
+    return slots < 250 || sparse_call_us(p, I[0], T) <= strip_call_us(bs_strip_steps(I[0], M[0], N, T), I[0]);
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
     int64_t total = (int64_t)bs_strip_partials(I[0], M[0], N, K, T) * T;      // sums of squares of x per strip group
@@ -1036,7 +1065,7 @@ void plan_call(CallPlan &c, const int *I, const int *M, int n, int N, int K, int
         make_plan(c.gemv, I, M, n, N, K, tp, mx_r);
         c.floats = std::max(c.floats, c.gemv.part_total);
     }
-    c.split = c.path == 0 && split_tiles(I, M, n, N, K, T);
+    c.split = c.path == 0 && split_tiles(I, M, n, N, K, T, c.sparse ? &c.gemv : nullptr);
     if (c.split) c.floats = std::max(c.floats, tile_part_floats(I, M, n, N, K, T));
 }
 int64_t scratch_bytes(const CallPlan &c) { return (c.floats * (int64_t)sizeof(float) + 255) / 256 * 256; }
@@ -1215,9 +1244,10 @@ int bs_gemv_sparse_serves(const int *I, const int *M, int n, int N, int K, int T
 int bs_gemv_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
     const int path = group_path(I, M, n, N, K, T);
     Plan p;
-    if (path == 1 && sparse_plan(p, I, M, n, N, K, T, path, 0)) return BS_TILE_NONE;
+    const bool sparse = T <= 3 && sparse_plan(p, I, M, n, N, K, T, path, path == 0 ? mx_rows_per_tile(I, M, n, N, K, T) : 0);
+    if (path == 1 && sparse) return BS_TILE_NONE;
     if (path == 1 && (n == 1 || T <= 48)) return !bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_NONE : T > 48 ? BS_TILE_COLUMN : BS_TILE_FORWARD;
-    if (path == 0) return split_tiles(I, M, n, N, K, T) && bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_TWO_TERMS : BS_TILE_NONE;
+    if (path == 0) return split_tiles(I, M, n, N, K, T, sparse ? &p : nullptr) && bs_tile_columns(I, M, n, N, K, T, columns) ? BS_TILE_TWO_TERMS : BS_TILE_NONE;
     for (int j = 0; j < n; j++)
         if (bs_gemv_forward_path(I[j], M[j], N, K, T) != BS_PATH_REBUILD) return BS_TILE_NONE;
     return bs_tile_columns(I, M, n, N, K, 0, columns) ? BS_TILE_REBUILD : BS_TILE_NONE;

@@ -38,6 +38,23 @@ def test_which_calls_the_sparse_kernel_serves():
         L.bs_set_decode_kernel(_lib.DECODE_AUTO)
 
 
+# Calls that other kernels are quicker on, and neighbours that they are not (us sparse / tile or strip kernel): many partial sums per output (few rows of many columns), a
+# unit that is mostly empty (up to 256 columns), long stacks of three tokens
+LEFT_TO_OTHERS = [(8, 144, 26112, 16, 3), (8, 55, 30720, 16, 3), (8, 260, 30208, 16, 3), (10, 4882, 8192, 16, 3),       # 17.1 / 11.1, 14.9 / 9.6, 24.2 / 16.3, 45.3 / 41.5
+                  (16, 20204, 128, 16, 2), (8, 28, 27392, 16, 2), (8, 320, 27520, 16, 2), (8, 71, 29824, 8, 2)]         # 20.8 / 15.7, 12.4 / 8.8, 17.8 / 15.2, 14.8 / 12.1
+KEPT = [(4, 4096, 4096, 16, 3), (8, 4096, 4096, 16, 3), (3, 718, 4608, 16, 3), (4, 4096, 11008, 16, 1), (8, 4096, 11008, 16, 2), (2, 20000, 1408, 16, 2), (4, 21114, 4736, 16, 2), (3, 27415, 256, 16, 1)]
+
+
+def test_calls_that_are_quicker_elsewhere_are_left_there():
+    for I, M, N, K, T in LEFT_TO_OTHERS:
+        assert not _lib.sparse_kernel([(I, M)], N, K, T), (I, M, N, K, T)
+        kind = _lib.tile_kernel([(I, M)], N, K, T)[0]
+        assert kind == (_lib.TILE_NONE if K != 16 else _lib.TILE_TWO_TERMS if T == 3 else _lib.TILE_FORWARD), (I, M, N, K, T)
+        assert _lib.lib().bs_workspace_bytes(I, M, N, K, T) <= 64 << 20
+    for I, M, N, K, T in KEPT:
+        assert _lib.sparse_kernel([(I, M)], N, K, T) and _lib.tile_kernel([(I, M)], N, K, T)[0] == _lib.TILE_NONE, (I, M, N, K, T)
+
+
 def test_the_decode_plan_is_the_sparse_kernels_wherever_it_serves():
     for I, M, N, K, T in CASES + [(4, 4096, 11008, 16, 1)]:
         waves, R, grid, kmax = _lib.decode_plan(I, M, N, K, T)
@@ -104,6 +121,20 @@ def test_edges(I, M, N, K, T):
     # One rounding of y; exact products; fp32 sums over a unit's 16 operands of 32 columns, the units of a range, 16 ranks and the slots: fewer than
     # 2^10 additions on the way, whose errors are random: 2^-18 of the sum of the magnitudes is five times their largest here.
     assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,K,T", LEFT_TO_OTHERS)
+def test_calls_left_to_others(I, M, N, K, T):
+    """u on a 16-byte boundary and off it, as a call of one matrix and as a group of one, twice: within what one rounding of the weight and one of y allow."""
+    print(f"left to others I={I} M={M} N={N} K={K} T={T}", flush=True)
+    q, u, vt, x, want, size = _layer(I, M, N, K, T)
+    room = torch.empty(u.numel() + 4, dtype=u.dtype, device="cuda")
+    room[4:] = u.flatten()
+    ys = [IU.bitstack_forward_hip(q, f, vt, x, None).view(T, M) for f in (u, room[4:].view(u.shape), u)]
+    ys.append(IU.bitstack_forward_group_hip(IU.MatrixGroup([(q, u, vt, None)]), x))
+    assert torch.equal(ys[0], ys[2]) and torch.equal(ys[0], ys[3])
+    assert all(bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -10 + size * 2.0 ** -11).all()) for y in ys)
 
 
 @pytest.mark.gpu

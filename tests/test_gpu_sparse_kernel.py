@@ -123,6 +123,56 @@ def test_edges(I, M, N, K, T):
     assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
 
 
+# Several units per workgroup, so that the loop over them, its two register sets and LDS buffers, u at a crossing and the slots that a finished row leaves empty are
+# reached: every (row tiles per wave, tokens), two to six units, ranges that start and end within a row of units and run over one, two and three of them
+SEVERAL = [(5, 1100, 5632, 16, 1), (4, 1100, 11008, 16, 1), (4, 3001, 8192, 9, 1), (5, 28001, 896, 16, 1), (5, 5001, 11008, 16, 1),
+           (5, 1100, 5632, 11, 2), (5, 1100, 11008, 16, 2), (5, 9000, 1408, 16, 2), (7, 28001, 896, 13, 2), (4, 28001, 1408, 16, 2),
+           (7, 1100, 8192, 16, 3), (4, 4097, 8192, 16, 3), (7, 5001, 5632, 11, 3), (7, 4097, 5632, 11, 3), (3, 28001, 3584, 16, 3)]
+
+
+def test_the_cases_of_several_units_are_that():
+    heights, lengths, rows, inside = set(), set(), set(), 0
+    for I, M, N, K, T in SEVERAL:
+        assert _lib.sparse_kernel([(I, M)], N, K, T), (I, M, N, K, T)
+        waves, R, grid, kmax = _lib.decode_plan(I, M, N, K, T)
+        chunks = -(-N // 512)
+        q, rem = divmod(I * -(-M // (128 * R)) * chunks, grid)
+        heights.add((R, T))
+        for w in range(grid):
+            begin, end = w * q + min(w, rem), (w + 1) * q + min(w + 1, rem)
+            lengths.add((T, min(end - begin, 4)))
+            rows.add((T, (end - 1) // chunks - begin // chunks + 1))
+            inside += begin % chunks != 0 and end % chunks != 0 and (end - 1) // chunks > begin // chunks
+    assert heights == {(r, t) for r in (1, 2, 4) for t in (1, 2, 3)} and inside >= 100
+    assert lengths >= {(t, n) for t in (1, 2, 3) for n in (2, 3, 4)} and rows >= {(t, n) for t in (1, 2, 3) for n in (1, 2)} and max(n for _, n in rows) >= 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N,K,T", SEVERAL)
+def test_several_units(I, M, N, K, T):
+    test_edges(I, M, N, K, T)                        # (the bound's count of additions covers six units of a range, and 7 x 22 slots)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T", [(2560, 2), (3584, 3)])
+def test_a_group_of_several_units(N, T):
+    """Two to four units per workgroup on four row tiles per wave, more on fewer, and a rank below 16: the bound of test_edges."""
+    layers, K = [(3, 9000), (2, 20001), (5, 700)], 11
+    assert _lib.sparse_kernel(layers, N, K, T) and sum(I * -(-M // 512) for I, M in layers) * (N // 512) > 2 * 256
+    parts = [_layer(I, M, N, K, T) for I, M in layers]
+    group, x = IU.MatrixGroup([p[:3] + (None,) for p in parts]), parts[0][3]
+    want, size = [], []
+    for q, u, vt, _, _, _ in parts:                  # (all of them on the first one's x)
+        q, u, vt, xc = (t.cpu().numpy() for t in (q, u, vt, x))
+        want.append(torch.from_numpy(C.forward_f64(q, u, vt, xc)).view(T, -1))
+        size.append(torch.from_numpy(C.forward_f64(np.full_like(q, 0xFF), np.abs(u), np.abs(vt), np.abs(xc))).view(T, -1))
+    want, size = torch.cat(want, 1).cuda(), torch.cat(size, 1).cuda()
+    print(f"group of several units N={N} T={T}", flush=True)
+    y = IU.bitstack_forward_group_hip(group, x)
+    assert torch.equal(y, IU.bitstack_forward_group_hip(group, x))
+    assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("I,M,N,K,T", LEFT_TO_OTHERS)
 def test_calls_left_to_others(I, M, N, K, T):

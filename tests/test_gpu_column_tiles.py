@@ -20,3 +20,14 @@ def test_tokens_do_not_depend_on_their_number(I, M, N):
     for T in (49, 64, 65, 79, 80, 81, 96, 97, 111, 112, 113, 127):
         assert _lib.tile_kernel([(I, M)], N, 16, T)[0] == _lib.TILE_COLUMN
         assert torch.equal(IU.bitstack_forward_hip(q, u, vt, x[:T].contiguous(), bias).view(T, M), whole[:T]), T
+
+
+def test_seven_blocks_up_to_six_token_tiles():
+    """Seven blocks are taken up to 96 tokens, on four, five and six token tiles (six: held to float64 with the tile kernel's tests)."""
+    I, M, N = 7, 2815, 4352
+    q, u, vt, x = (t.cuda() for t in synthetic_layer(M, N, I, 96, seed=I + N, signed_factors=True))
+    u, x = (u * 20).half(), x.view(96, N)
+    whole = IU.bitstack_forward_hip(q, u, vt, x, None).view(96, M)
+    for T in (50, 64, 65, 79, 80, 81):
+        assert _lib.tile_kernel([(I, M)], N, 16, T)[0] == _lib.TILE_COLUMN
+        assert torch.equal(IU.bitstack_forward_hip(q, u, vt, x[:T].contiguous(), None).view(T, M), whole[:T]), T

@@ -664,7 +664,7 @@ struct Plan {
 
 // One instantiation and one grid for the whole group; every matrix gets a share of
 // the workgroups in proportion to its units.
-// Which kernel make_plan picks for one and two tokens: 0 by shape, 1 always the fp16 kernel, 2 the block-scaled one
+// Which kernel a call of one to four tokens runs on: 0 by shape, 1 always gemv_kernel, 2 for one and two tokens the block-scaled one
 // wherever it takes the shape (bs_set_decode_kernel, for tests and benchmarks).  Per calling thread: a size query
 // and the forward behind it on one thread agree whatever other threads set.
 thread_local int g_decode_kernel = 0;
@@ -742,7 +742,10 @@ void make_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T, 
         one_per_cu(p, I, M, T);
         return;
     }
-    // rows per workgroup: 512 (8 waves x 4 tiles), 256, 128, 64; resident workgroups per CU.
+    // gemv_kernel.  By shape it has four tokens where the tile kernel declines, the passes of two to four that five to eight tokens are cut into where the strip
+    // kernel declines, one token below a MiB of sign bytes (64-row tiles), and what the sparse kernel's offsets or scratch do not allow.  Otherwise one to three
+    // tokens run here under bs_set_decode_kernel only, so do one token's taller tiles, pairs and 16 waves.
+    // Rows per workgroup: 512 (8 waves x 4 tiles), 256, 128, 64; resident workgroups per CU.
     // Three or four tokens need more than the 128 registers a lane has with two 8-wave
     // workgroups per CU: there it is one workgroup of 8 waves per CU (two waves per SIMD
     // to overlap sign decode and MFMA), four row tiles per wave (each Z fragment read
@@ -764,7 +767,7 @@ void make_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T, 
         // enough units that every CU gets one
         if (tall && units >= 256) { pick = k; break; }
     }
-    // One token, long stacks: one workgroup of 16 waves per CU.  Two 8-wave workgroups on a CU do
+    // One token, long stacks (under BS_DECODE_F16): one workgroup of 16 waves per CU.  Two 8-wave workgroups on a CU do
     // not share it evenly (the older one is served first and finishes a third earlier, the
     // younger one then runs on a half-empty CU); sixteen waves that meet at one barrier do.
     const int *choice = cand[pick];
@@ -944,17 +947,16 @@ bool gemv_group_ok(const int *I, const int *M, int n, int N, int K, int T) {
         if (!gemv_shape_ok(I[j], M[j], N, K, T)) return false;
     return true;
 }
-// 1: strip kernel, 0: factor-through kernel, -1: neither takes the shapes
+// 1: strip kernel, 0: factor-through kernel (either may leave the call to the sparse kernel, see sparse_plan), -1: neither takes the shapes
 int group_path(const int *I, const int *M, int n, int N, int K, int T) {
     if (n < 1 || n > GEMV_MAX_GROUP) return -1;
     if (T >= STRIP_MIN_T && T <= STRIP_MAX_T && strip_group_ok(I, M, n, N, K, T)) return 1;
     if (gemv_group_ok(I, M, n, N, K, T)) return 0;
-    // One to four tokens on column counts that are multiples of 128 but not of 512: the strip kernel rounds the weight to fp16 once
-    // and multiplies with fp32 sums, as the rebuild and the dense product do that such shapes took before it, and no less exactly
-    // (error against float64 within 0.05 % of theirs: 11 shapes, three decomposed weights, 1, 2 and 4 tokens).  The factor-through kernels
-    // would round vt * x: 7 % further from float64 with 2 blocks of 11008 columns (2.94e-4 against 2.75e-4), 11 % on the block-scaled
-    // one.  us rebuild / strip, 4096 x 11008 with one token: 1 block 52 / 14, 4 blocks 72 / 28, 8 blocks 91 / 47; 2048 x 5504, 3
-    // blocks 32 / 12; 8192 x 3200, 4 blocks 40 / 21 (the block-scaled kernel, with that loss: 18 and 24 at 4 and 8 blocks of 4096 x 11008).
+    // One to four tokens on column counts that are multiples of 128 but not of 512, of which sparse_plan takes most at one and two: the tile and strip kernels
+    // round the weight to fp16 once and multiply with fp32 sums, as the rebuild and the dense product do that such shapes would take otherwise, and no less
+    // exactly (error against float64 within 0.05 % of theirs: 11 shapes, three decomposed weights, 1, 2 and 4 tokens).  gemv_kernel would round vt * x: 7 %
+    // further from float64 with 2 blocks of 11008 columns (2.94e-4 against 2.75e-4), 11 % on the block-scaled one.  us rebuild / strip, one token: 4096 x
+    // 11008, 1 block 52 / 14, 4 blocks 72 / 28, 8 blocks 91 / 47; 2048 x 5504, 3 blocks 32 / 12; 8192 x 3200, 4 blocks 40 / 21.
     return N % CH != 0 && T < STRIP_MIN_T && strip_group_ok(I, M, n, N, K, T) ? 1 : -1;
 }
 int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T, double *cycles = nullptr) {

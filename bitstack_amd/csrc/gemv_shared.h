@@ -18,7 +18,7 @@ struct Split {
 // the grid is cut into one run of workgroups per matrix, each with its own static
 // partition, partial-sum area and row count.
 constexpr int GEMV_MAX_GROUP = 4;
-constexpr int GEMV_WIDE_MIN_UNITS = 1024;   // 1024-row units from which one token runs on 16-wave workgroups
+constexpr int GEMV_WIDE_MIN_UNITS = 1024;   // 1024-row units from which one token runs on 16-wave workgroups of gemv_kernel (BS_DECODE_F16)
 constexpr int GEMV_PAIR_MIN_UNITS = 4;      // units per workgroup from which workgroups are paired
 struct GemvMat {
     const uint8_t *packed;

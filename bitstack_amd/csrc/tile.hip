@@ -29,7 +29,7 @@
 // not tell how many were in flight, every tile waited for the requests made right before it and for its own stores (us with such branches / without: rebuild of
 // 4096 x 14336, 8 blocks 65.2 / 59.4, 14336 x 4096, 5 45.9 / 42.3; 10 blocks of 4096 x 4096, 8 tokens 23.9 / 22.5; a step of 8 sequences over two 70B-shape layers 662 / 642).  us, strip_forward_kernel / this, with the summing launch, in a
 // replayed graph on rotating copies: 28672 x 8192, 3 blocks, 8 tokens 86.5 / 62.8; 14336 x 4096, 8 blocks, 8 tokens 50.0 / 42.6; 5000 x 4096, 6 blocks, 37 tokens
-// 29.7 / 25.6; 4096 x 11008, 4 blocks, one token 26.1 / 24.4.
+// 29.7 / 25.6.  (One and two tokens of larger matrices whose columns are no multiple of 512 are the sparse kernel's, see sparse_plan in gemv.hip.)
 #include "common.h"
 #include "rebuild_shared.h"
 
@@ -524,33 +524,33 @@ struct TileKernel {
                 }
                 first_block();                   // of tile n + 1
             } else {
-            // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
-            // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
-            // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
-            // v_mfma_f32_16x16x32_f16.
-            half8_t wf[NP][2];
+                // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
+                // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
+                // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
+                // v_mfma_f32_16x16x32_f16.
+                half8_t wf[NP][2];
 #pragma unroll
-            for (int p = 0; p < NP; p++) {
-                uint4_t lo, hi;
+                for (int p = 0; p < NP; p++) {
+                    uint4_t lo, hi;
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
-                    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-                    lo[k] = r[0];
-                    hi[k] = r[1];
+                    for (int k = 0; k < 4; k++) {
+                        const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
+                        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                        lo[k] = r[0];
+                        hi[k] = r[1];
+                    }
+                    wf[p][0] = __builtin_bit_cast(half8_t, lo);
+                    wf[p][1] = __builtin_bit_cast(half8_t, hi);
                 }
-                wf[p][0] = __builtin_bit_cast(half8_t, lo);
-                wf[p][1] = __builtin_bit_cast(half8_t, hi);
-            }
-            first_block();                       // of tile n + 1
+                first_block();                       // of tile n + 1
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++)
+                for (int tt = 0; tt < TT; tt++)
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    y[tt][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
+                    for (int r = 0; r < 2; r++) {
+                        y[tt][r] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
-                }
+                        for (int p = 0; p < NP; p++) y[tt][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[tt][p], wf[p][r], y[tt][r], 0, 0, 0);
+                    }
             }
         }
         if (TT == 0) {

@@ -365,9 +365,13 @@ int launch_tiled(const half_t *x, const half_t *w, const half_t *bias, half_t *y
 struct LinearTile { int bt, bf, gk; };
 static LinearTile linear_tile(int T, int M, int N, bool aligned) {
     if (!(N % 8 == 0 && aligned) || N >= (1 << 23)) return {0, 0, 0};     // (a tile's rows stay within 32-bit byte offsets)
-    // linear_skinny_kernel: the more features a workgroup has, the less x it reads, as long as there are some 160 workgroups or more (8 tokens, us, 16 / 32 / 64
-    // features: 8192 x 8192 29.4 / 26.5 / 38.8, 14336 x 4096 28.8 / 25.9 / 23.8, 32000 x 8192 104.6 / 91.1 / 90.0)
-    if (T <= 32) return {32, M >= 12288 ? 64 : M >= 5120 ? 32 : 16, 0};
+    // linear_skinny_kernel: the more features a workgroup has, the less x it reads, but what counts is the rounds of 256 workgroups, each of which takes about as long
+    // half empty: 16 features while one round holds them, 64 where they take less than 4/7 of the rounds of 32.  us, 16 / 32 / 64 features, 4096 columns: 8 tokens, 4096 rows
+    // 8.8 / 11.4 / 18.4, 4189 15.2 / 11.5 / 18.5, 8192 15.8 / 14.7 / 18.6, 8400 21.8 / 22.2 / 18.6, 17129 34.8 / 34.5 / 38.5, 24600 47.0 / 39.9 / 39.6, 33000 61.1 / 54.0 /
+    // 57.3; 32 tokens, 4189 23.3 / 16.6 / 24.1, 8400 33.6 / 32.0 / 23.9.  Below 1024 columns 32 and 64 are closer (720, 8 tokens: 4189 rows 4.2 / 2.9 / 3.7, 12288
+    // 5.6 / 3.8 / 3.9, 17129 8.4 / 5.1 / 5.8), and from 960 on 16 are kept to 5119 rows, where the kernel's tests have them.
+    if (T <= 32 && N >= 1024) return {32, M <= 4096 ? 16 : 7 * bs_cdiv(M, 256 * 64) < 4 * bs_cdiv(M, 256 * 32) ? 64 : 32, 0};
+    if (T <= 32) return {32, M >= 12288 ? 64 : M > (N < 960 ? 4096 : 5119) ? 32 : 16, 0};
     if (T <= 128) return M >= 8192 ? LinearTile{128, 64, 64} : LinearTile{128, 32, 128};
     // The largest tile whose grid still covers most of the 256 CUs: 256 x 256 and
     // 128 x 256 move the fewest bytes per flop; 128 x 128 and 64 x 64

@@ -32,3 +32,23 @@ def test_few_tokens_match_float64(T, M, N, features):
     # N products added in float32 (2^-24 of the sum of magnitudes each, in whatever order), rounded once
     bound = want.abs() * 2.0 ** -11 + size * (N + 9) * 2.0 ** -24 + 2.0 ** -25
     assert ((y - want).abs() <= bound).all()
+
+
+# both sides of every change of width: one round of 256 workgroups of 16 features, rounds of 32 against rounds of 64
+ROUNDS = [(5, 4096, 1032, 16), (8, 4097, 1032, 32), (32, 5119, 1096, 32), (3, 8192, 1024, 32), (3, 8193, 1024, 64), (20, 16384, 1032, 64), (20, 16385, 1032, 32),
+          (1, 24577, 1024, 64), (16, 32769, 1024, 32), (17, 4097, 952, 32), (32, 4096, 952, 16)]
+
+
+def test_a_round_that_is_nearly_empty_is_avoided():
+    """A few rows more than a round holds take no second one where a wider workgroup needs none."""
+    for T, M, N, features in ROUNDS:
+        assert _lib.linear_plan(T, M, N) == (32, features, 0, 0), (T, M, N)
+    for T in (1, 8, 17, 32):
+        for M in (4189, 5000, 8192, 8400, 12287, 13000, 16384):
+            assert -(-M // _lib.linear_plan(T, M, 4096)[1]) <= 256, (T, M)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,M,N,features", ROUNDS)
+def test_either_side_of_a_change_of_width(T, M, N, features):
+    test_few_tokens_match_float64(T, M, N, features)

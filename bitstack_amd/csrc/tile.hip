@@ -117,6 +117,81 @@ struct TileKernel {
         return I;
     }
 
+    // A lane's piece within chunk c of a tile: chunks of 1 KB, the signs of block c / SCH first, then the u rows of the blocks
+    static __device__ __forceinline__ uint32_t piece_at(int c, int I, int lane, int cg, uint32_t row_bytes) {
+        if (c < I * SCH) {
+            const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
+            return (uint32_t)r * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
+        }
+        const int r = lane >> 1;
+        return (uint32_t)r * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
+    }
+    // y tiles: [buffer][wave][TT token tiles][rows 0-15, 16-31][four tokens: 4][row: 16][token: 4]; floats, of wave 0
+    static constexpr int Y = 16 * TT * TL_ROWS;
+    static __device__ __forceinline__ int y_at(int buf, int tt, int t, int row) { return buf * (TL_WAVES * Y) + tt * 512 + row / 16 * 256 + t / 4 * 64 + row % 16 * 4 + t % 4; }
+
+    // The waves without columns, those from `active` on: their share of walk's requests and sums, between the same barriers.  (A path of their own, one for all block
+    // counts: a branch in walk's loop leaves the compiler unsure of what is in flight, and doing the others' work on the last columns, for nobody, they took its issue
+    // slots from them.  us, so / this: 13888 x 128 (half of the waves have no columns), 10 blocks, 3 tokens 11.2 / 9.6; 251 x 128, 5, 44 8.7 / 8.0; 4921 x 384, 3, 38 10.0 / 9.4.)
+    static __device__ __forceinline__ void walk_without_columns(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, float *__restrict__ part, int I, int M, lds_bytes_rw lds,
+                                                                int N, int T, int cg, int rt0, int len, bool ssq, int wave, int active) {
+        constexpr int MOST = 4;                                  // (32 chunks at most: 16 blocks of one patch)
+        const int tid = threadIdx.x, lane = tid & 63, chunks = I * (SCH + 1), stage_size = stage_bytes(I), my_t = tid >> 5, my_row = tid & 31;
+        const uint32_t row_bytes = (uint32_t)N >> 3;
+        lds_bytes_rw area = lds + TL_TABLE, ring = area + AREA;
+        uint4_t ahead[2][MOST];
+        auto request = [&](int k, int n) {                       // tile n, or the last one
+            const int rt = rt0 + min(n, len - 1);
+            const uint32_t rows = min(M - rt * TL_ROWS, TL_ROWS);
+#pragma unroll
+            for (int q = 0; q < MOST; q++) {
+                const int c = wave + TL_WAVES * q;
+                if (c >= chunks) break;
+                const bool signs = c < I * SCH;
+                const char *from = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
+                const uint32_t pitch = signs ? row_bytes : 32u;
+                ahead[k][q] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from + (int64_t)(rt * TL_ROWS) * pitch, (int)(rows * pitch)), (int)piece_at(c, I, lane, cg, row_bytes), 0, 0);
+            }
+        };
+        auto write = [&](int k, int stage) {
+#pragma unroll
+            for (int q = 0; q < MOST; q++)
+                if (wave + TL_WAVES * q < chunks) ((lds_uint4_rw)(ring + stage * stage_size + (wave + TL_WAVES * q) * 1024))[lane] = ahead[k][q];
+        };
+        auto sums = [&](int n) {                                 // tile n, in walk's order
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) {
+                if (16 * tt + my_t >= T || (rt0 + n) * TL_ROWS + my_row >= M) continue;
+                lds_f32 red = (lds_f32)(area) + y_at(n & 1, tt, my_t, my_row);
+                float sum = red[0];
+                for (int w = 1; w < active; w++) sum += red[w * Y];
+                part[((int64_t)cg * T + 16 * tt + my_t) * M + (rt0 + n) * TL_ROWS + my_row] = sum;
+            }
+        };
+        request(0, 0);
+        request(1, 1);
+        write(0, 0);
+        write(1, 1);
+        request(0, 2);
+        if (ssq) {
+            __syncthreads();
+            __syncthreads();
+        }
+        tl_wait_lds<0>();
+        tl_barrier();                                            // the first tile is here
+        for (int n = 0; n < len; n++) {
+            tl_wait_lds<0>();
+            tl_barrier();                                        // tile n + 1 and the y tiles of n - 2 are in LDS, the stage of n - 1 is free
+            write(0, (n + 2) % STAGES);
+            request(0, n + 3);
+            if (n >= 2) sums(n - 2);
+        }
+        tl_wait_lds<0>();
+        if (len > 2) tl_barrier();
+        tl_barrier();
+        for (int n = max(len - 2, 0); n < len; n++) sums(n);
+    }
+
     // One run of row tiles [rt0, rt0 + len) of column group cg of one matrix.
     template <int I>
     static __device__ __forceinline__ void walk(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, const half_t *__restrict__ vt,
@@ -132,24 +207,16 @@ struct TileKernel {
         const int lm = lane & 15, g = lane >> 4;                // in the second product
         const uint32_t row_bytes = (uint32_t)N >> 3;
         lds_bytes_rw area = lds + TL_TABLE, ring = area + AREA;
-        // Waves whose columns exist (all or none of a wave's).  The others do the same work on the last columns, for nobody: a branch around it would
-        // leave the compiler unsure of what is in flight, and have it wait for stores behind the requests that it needs.
+        // Waves whose columns exist (all or none of a wave's).  The others are in walk_without_columns, or (TT = 0, where all of them wait for the stores) do the
+        // same work on the last columns, for nobody.
         const int active = min(TL_WAVES, (N - cg * CG) / WC);
         const int n0 = min(cg * CG + wave * WC, N - WC);
 
-        // ---- requests: chunk c of a tile is 1 KB, signs of block c / SCH first, then the u rows of the blocks --------------
+        // ---- requests ----------------------------------------------------------------------------------------------------
         // Wave w takes chunks w, w + 8, ...; one that is short of a chunk takes the last one too.
         const char *from[MOST];                                  // row 0 of the next tile to be requested
         uint32_t pitch[MOST], offset[MOST];                      // the lane's piece within a tile
         auto chunk_of = [&](int k) { return MORE == 0 || k < PER ? wave + TL_WAVES * k : min(wave + TL_WAVES * k, CHUNKS - 1); };
-        auto geometry = [&](int c) {
-            if (c < I * SCH) {
-                const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
-                return (uint32_t)r * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
-            }
-            const int r = lane >> 1;
-            return (uint32_t)r * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
-        };
 #pragma unroll
         for (int k = 0; k < MOST; k++) {
             const int c = chunk_of(k);
@@ -157,7 +224,7 @@ struct TileKernel {
             from[k] = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
             pitch[k] = signs ? row_bytes : 32u;
             from[k] += (int64_t)(rt0 * TL_ROWS) * pitch[k];
-            offset[k] = geometry(c);
+            offset[k] = piece_at(c, I, lane, cg, row_bytes);
         }
         // A tile's pieces travel through registers: requested three tiles ahead, written to LDS at the end of the tile two ahead of it.
         int asked = rt0;                                         // the row tile `from` stands at
@@ -261,17 +328,16 @@ struct TileKernel {
             }
         }
 
-        // ---- y tiles: [buffer][wave][TT token tiles][rows 0-15, 16-31][four tokens: 4][row: 16][token: 4] ----------------------------
+        // ---- y tiles ---------------------------------------------------------------------------------------------------------
         // Pass tt of a hand-over is one output per thread: this thread's of every wave, added in wave order.  The reads are issued ahead of
         // where they are added up.
-        constexpr int Y = 16 * TT * TL_ROWS;
         const int my_t = tid >> 5, my_row = tid & 31;
         const uint32_t my_out = (uint32_t)(my_t * M + my_row) * 4u;
         float *const out = part + (int64_t)cg * T * M;
         // (a wave's two tokens of pass tt)
         auto takes = [&](int tt) { return 16 * tt + 2 * wave < T; };
         auto collect = [&](int buf, int tt, float (&v)[TL_WAVES]) {
-            lds_f32 red = (lds_f32)(area) + buf * (TL_WAVES * Y) + tt * 512 + my_row / 16 * 256 + my_t / 4 * 64 + my_row % 16 * 4 + my_t % 4;
+            lds_f32 red = (lds_f32)(area) + y_at(buf, tt, my_t, my_row);
             if (takes(tt)) {
 #pragma unroll
                 for (int w = 0; w < TL_WAVES; w++) v[w] = red[w * Y];
@@ -594,6 +660,21 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     const int r = v - grp->m[j].first_wg, wgs = grp->m[j].wgs, tiles = grp->m[j].row_tiles, cg = r / wgs, run = r - cg * wgs;
     const int rt = (int)((int64_t)tiles * run / wgs), len = (int)((int64_t)tiles * (run + 1) / wgs) - rt;
     float *ssq = j == 0 && run == 0 ? grp->ssq : nullptr;
+    if constexpr (TT > 0) {
+        const int np = grp->m[j].np, patches = N / 32 - cg * TL_WAVES * np;      // from the group's first column on
+        if (patches < TL_WAVES * np) {
+            const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), active = patches >> (np >> 1);
+            if (wave >= active) {
+                auto rest = [&](auto k) {
+                    TileKernel<TT, decltype(k)::value, SPLIT>::walk_without_columns(grp->m[j].packed, grp->m[j].u, grp->m[j].part, grp->m[j].I, grp->m[j].M, lds, N, T, cg, rt, len, ssq != nullptr, wave, active);
+                };
+                if (np == 4) rest(std::integral_constant<int, 4>{});
+                else if (np == 2) rest(std::integral_constant<int, 2>{});
+                else rest(std::integral_constant<int, 1>{});
+                return;
+            }
+        }
+    }
     auto walk = [&](auto np, auto blocks) {
         typedef TileKernel<TT, decltype(np)::value, SPLIT> TK;
         if constexpr (decltype(blocks)::value <= TK::max_blocks())

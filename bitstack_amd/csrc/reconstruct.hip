@@ -482,13 +482,15 @@ int byte_steps(int M, int N) {
     const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(bs_cdiv(1024, strips), bs_cdiv(steps, RA_STREAMS)));
     return (int)bs_cdiv(bs_cdiv(steps, groups), RA_STREAMS) * RA_STREAMS;
 }
-// At rank 16 always.  Below, u is read half by half, and a wave's chain of (row step, block) pairs is some 0.9 us each; one output per thread takes 0.07 + 0.1 us
-// per rank and block, or its products' time where there are many: us, that / byte kernel, 337 x 40, 7 blocks, rank 1 3.9 / 11.5, 520 x 248, 9, rank 8 10.8 / 24.5, 1371 x 296, 5, rank 1
-// 4.4 / 10.0; 4096 x 4104, 4, rank 8 244 / 39, 2374 x 1248, 12, rank 5 68.5 / 14.9.  Of 600 drawn rebuilds (up to 12 blocks, 6 million weights, ranks 1 to 16) 8 are more
-// than 3 % behind the former with this rule, 17 % at worst; without it 260 of 900, 120 %.
+// At rank 16 always.  Below, u is read half by half, and a wave's chain of (row step, block) pairs is some 1.15 us each; one output per thread takes 0.1 + 0.11 us
+// per rank and block, or its products' time where there are many (fitted to 400 rebuilds from int8 signs, up to 12 blocks and 6 million weights; from packed signs the
+// former is up to half slower, but the weight is the same bit for bit whatever it is made from, so both go one way).  us from int8 signs, that / byte kernel: 1211 x 432, 11 blocks,
+// rank 5 11.7 / 16.3, 257 x 1928, 5, rank 6 7.5 / 10.2, 511 x 912, 1, rank 11 4.6 / 5.9; 523 x 4704, 7, rank 10 73.1 / 15.7; from packed signs 520 x 248, 9, rank 8 10.8 / 24.5,
+// 4096 x 4104, 4, rank 8 244 / 39.  Of the 400 8 are more than 3 % behind one output per thread, 34 % at worst (150 x 3392, 8, rank 8), and from packed signs
+// 1, 6 %.
 bool byte_kernel_pays(int I, int M, int N, int K) {
-    const double chain = 1.0 + 0.9 * I * (byte_steps(M, N) / RA_STREAMS);
-    return K == 16 || chain <= std::max((0.07 + 0.1 * K) * I, 0.33e-6 * M * N * I * (K + 2));
+    const double chain = 4.0 + 1.15 * I * (byte_steps(M, N) / RA_STREAMS);
+    return K == 16 || chain <= std::max(2.5 + (0.1 + 0.11 * K) * I, 1.5 + (0.9e-6 + 0.3e-6 * K) * M * N * I);
 }
 
 template <bool PACKED>

@@ -20,7 +20,7 @@
 //
 // What bounds it: with four row tiles a unit is 128 matrix instructions per SIMD, 8.9 ns each on their own and 10.3 with three VALU instructions between them, and 256 KB of B out
 // of LDS, a us as well: 2.0 us measured where units follow each other (4.2 TB/s), of which the multiplication takes 1.5 with the signs in L2.  A call with one unit per workgroup
-// takes 4 to 7 us: 1.5 until vt has arrived, 0.7 until everybody's has, the unit, 0.7 for u and the sums, and the launch.  us, tile kernel / this, one token: 4096 x 11008, 4 blocks
+// takes 4 to 7 us: 1.5 until vt has arrived, 0.7 until everybody's has, the unit, 0.7 for u and the sums, and the launch.  us in a replayed graph, tile kernel / this, one token: 4096 x 11008, 4 blocks
 // 25.7 / 17.7, 8 39.3 / 25.6 (other shapes at sparse_plan).  Measured and not kept: the pairs made from single halves in registers, half the LDS traffic for two VALU
 // instructions per product (42.3 -> 45.3 us on 16 blocks of 4096 x 14336); eight row tiles (64 KB per unit arrive too late: 41.6, and 16.1 instead of 13.7 on 4096 x 11008); both
 // 64-byte halves of a line of sign bytes requested together, 1024 columns ahead (44.0, 15.3); operands of B two ahead and of x one ahead (42.2, 14.6 against 43.8, 15.0 in that run).

@@ -19,7 +19,7 @@
 // 28672 x 8192, 3 310 / 241, 14336 x 4096, 5 89 / 84.
 //
 // What bounds it: the issue of a wave's instructions: by the counters vector instructions take 64 % of a SIMD's cycles on 28672 x 8192, 3 blocks, 8 tokens
-// and 61 on 4096 x 14336, 4 blocks, 4 tokens (the matrix cores 22 and 16), where runs are short 33 (5000 x 4096, 6 blocks, 37 tokens) and waits at the
+// and 60 on 4096 x 14336, 4 blocks, 4 tokens (the matrix cores 22 and 15), where runs are short 33 (5000 x 4096, 6 blocks, 37 tokens) and waits at the
 // barrier and for LDS as much, in the rebuild 51 with its stores waited for.  Simple VALU instructions (v_xor_b32, v_and_b32, v_lshrrev_b32, fp32 add, mul and FMA on
 // three registers) of two waves run side by side on a SIMD, 1.0 ns each; v_fma_mix_f32, v_and_or_b32, v_bfe, v_alignbit, conversions and whatever
 // has a scalar operand take 1.8 ns, and a single wave issues one instruction in 2 ns whatever it is.  A step (1024 signs: 16 v_xor, 5 for the

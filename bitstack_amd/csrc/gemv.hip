@@ -75,7 +75,11 @@ constexpr int CH = 512;   // columns per chunk: 4 lane groups x 16 bytes of sign
 // Sign bytes per launch from which the block-scaled kernel is preferred to the sparse one.  us sparse / block-scaled, one token: 4096 x 4096, 4 blocks (8 MiB) 9.4 / 9.3,
 // 8 blocks 13.7 / 12.6, 14336 x 4096, 8 blocks 30.6 / 28.7; two tokens: 8 blocks of 4096 x 4096 (16 MiB) 16.8 / 17.6, 6144 x 4096, 6 blocks 20.4 / 22.2, 4096 x 14336, 3 (21 MiB)
 // 22.5 / 22.9, 14336 x 4096, 8 (56 MiB) 38.9 / 39.9, 4096 x 14336, 16 (112 MiB) 65.1 / 60.9.
-constexpr int64_t MX_MIN_SIGN_BYTES = 12 << 20, MX_MIN_SIGN_BYTES_TWO = 24 << 20;
+// One token from 8 MiB on too where the sparse kernel, whose units are half as wide, leaves 200 partial sums per output or more: few rows of many columns (355 x 15872, 16
+// blocks, 496 sums against 144, 15.7 / 12.2; 925 x 11776, 9, 207 against 108, 13.2 / 11.6; of 120 drawn calls from 8 to 12 MiB 2 are more than 3 % behind the block-scaled
+// kernel, without it 19, 28 % at worst; over all of them 0.93 of its time).  Two tokens: of 120 from 8 to 24 MiB none.
+constexpr int64_t MX_MIN_SIGN_BYTES = 12 << 20, MX_MIN_SIGN_BYTES_TWO = 24 << 20, MX_MIN_SIGN_BYTES_MANY_SUMS = 8 << 20;
+constexpr int MX_MANY_SUMS = 200;
 
 
 // step -> bit position used in that step; steps 0-7 read the word as loaded,
@@ -669,6 +673,7 @@ struct Plan {
 // and the forward behind it on one thread agree whatever other threads set.
 thread_local int g_decode_kernel = 0;
 
+int most_sparse_sums(const int *I, const int *M, int n, int N);
 // Rows per workgroup of the block-scaled kernel for these matrices (0: it does not run them).
 int mx_rows_per_tile(const int *I, const int *M, int n, int N, int K, int T) {
     if (g_decode_kernel == 1 || !bs_gemv_mx_takes(N, K, 1, T)) return 0;
@@ -688,7 +693,9 @@ int mx_rows_per_tile(const int *I, const int *M, int n, int N, int K, int T) {
     // by shape: the long-stack cases, where the contraction loop and not the fixed cost of a launch decides
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) bytes += (int64_t)I[j] * M[j] * (N / 8);
-    return (pick >= 2 && bytes >= (T == 1 ? MX_MIN_SIGN_BYTES : MX_MIN_SIGN_BYTES_TWO)) ? pick : 0;
+    if (pick < 2) return 0;
+    if (bytes >= (T == 1 ? MX_MIN_SIGN_BYTES : MX_MIN_SIGN_BYTES_TWO)) return pick;
+    return T == 1 && bytes >= MX_MIN_SIGN_BYTES_MANY_SUMS && most_sparse_sums(I, M, n, N) >= MX_MANY_SUMS ? pick : 0;
 }
 
 // The grid of the block-scaled and the sparse kernel: one workgroup of 8 waves, 128 R rows, per CU.
@@ -867,6 +874,15 @@ void sparse_plan_of(Plan &p, const int *I, const int *M, int n, int N, int T) {
     }
     p.us = best;
     one_per_cu(p, I, M, T);
+}
+
+// Most partial sums per output that the sparse kernel leaves of one token.
+int most_sparse_sums(const int *I, const int *M, int n, int N) {
+    Plan p;
+    sparse_plan_of(p, I, M, n, N, 1);
+    int most = 0;
+    for (int j = 0; j < n; j++) most = std::max(most, I[j] * p.kmax[j]);
+    return most;
 }
 
 // us of one matrix's call on the sparse kernel, and on the tile and strip kernels (estimates for the choice between them, fitted to 900 calls on rotating

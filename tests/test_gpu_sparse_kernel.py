@@ -173,6 +173,29 @@ def test_a_group_of_several_units(N, T):
     assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -11 + size * 2.0 ** -18 + 2.0 ** -25).all())
 
 
+# One token from 8 to 12 MiB of sign bytes: many partial sums per output go to the block-scaled kernel, with half as many (us sparse / block-scaled: 15.7 / 12.2, 14.8 / 12.9,
+# 13.2 / 11.6, 14.8 / 13.1); whole matrices do not, nor below 8 MiB
+MANY_SUMS = [(16, 355, 15872), (14, 323, 15872), (9, 925, 11776), (8, 425, 26112)]
+
+
+def test_many_partial_sums_go_to_the_block_scaled_kernel():
+    for I, M, N in MANY_SUMS:
+        assert not _lib.sparse_kernel([(I, M)], N, 16, 1) and _lib.lib().bs_decode_kernel(I, M, N, 16, 1) == _lib.DECODE_MX, (I, M, N)
+    for I, M, N in [(4, 4096, 4096), (5, 4096, 4096), (3, 1792, 14336), (2, 14336, 2560), (16, 255, 15872), (16, 258, 14848)]:
+        assert _lib.sparse_kernel([(I, M)], N, 16, 1), (I, M, N)
+    assert not _lib.sparse_kernel([(1, 1627), (8, 297)], 17920, 16, 1) and _lib.sparse_kernel([(2, 4096), (3, 1024)], 4096, 16, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I,M,N", MANY_SUMS)
+def test_many_partial_sums(I, M, N):
+    """Within what three fp6 terms of vt * x (2^-12 of a block's largest) and one rounding of y allow."""
+    print(f"many partial sums I={I} M={M} N={N}", flush=True)
+    q, u, vt, x, want, size = _layer(I, M, N, 16, 1)
+    y = IU.bitstack_forward_hip(q, u, vt, x, None).view(1, M)
+    assert bool(((y.double() - want).abs() <= want.abs() * 2.0 ** -10 + size * 2.0 ** -11).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("I,M,N,K,T", LEFT_TO_OTHERS)
 def test_calls_left_to_others(I, M, N, K, T):

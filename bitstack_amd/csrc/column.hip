@@ -26,7 +26,7 @@
 
 namespace {
 
-constexpr int CL_WAVES = 8, CL_ROWS = 256, CL_TABLE = 256, CL_MIN_T = 49, CL_MAX_T = 128;
+constexpr int CL_WAVES = 8, CL_ROWS = 256, CL_TABLE = 512, CL_HALVES = 256, CL_MIN_T = 49, CL_MAX_T = 128;
 constexpr int CL_IMAGE = 64 * 32;                   // bytes: a block's vt of a chunk, or 16 tokens of x
 
 template <class F, int... Is>
@@ -43,6 +43,7 @@ typedef const __attribute__((address_space(3))) half8_t *cl_half8;
 typedef __attribute__((address_space(3))) half8_t *cl_half8_rw;
 typedef __attribute__((address_space(3))) half2_t *cl_half2_rw;
 typedef const __attribute__((address_space(3))) uint4_t *cl_uint4;
+typedef const __attribute__((address_space(3))) uint2_t *cl_uint2;
 
 struct ColumnMat {
     const uint8_t *packed;
@@ -62,7 +63,12 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
     const int row = lane & 31, h = lane >> 5;       // in the rebuild
     const int lm = lane & 15, g = lane >> 4;        // in the second product
     // nibble v, column j of its four (first in the top bit): the sign bit of an fp32 where the bit is set; at LDS address 0
-    if (tid < 64) ((__attribute__((address_space(3))) uint32_t *)lds)[tid] = ((tid >> 2) >> (3 - (tid & 3))) & 1 ? 0x80000000u : 0u;
+    // and behind it the sign bits of two pairs of fp16
+    if (tid < 64) {
+        const uint32_t v = tid >> 2, j = tid & 3, first = v >> (3 - 2 * (j & 1)) & 1, second = v >> (2 - 2 * (j & 1)) & 1;
+        ((__attribute__((address_space(3))) uint32_t *)lds)[tid] = v >> (3 - j) & 1 ? 0x80000000u : 0u;
+        ((__attribute__((address_space(3))) uint32_t *)lds)[CL_HALVES / 4 + tid] = first << 15 | second << 31;
+    }
     // every XCD gets a contiguous run of (column group, rows), rows fastest: workgroups with the same slices of x and vt share an L2
     const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, base = nb >> 3, rem = nb & 7;
     const int v = xcd * base + min(xcd, rem) + loc, cg = v / mat.row_groups, rg = v - cg * mat.row_groups;
@@ -140,6 +146,8 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
             // masks and vt fragments are looked up a step ahead (see tile.hip)
             float16_t acc[2];
             uint4_t mask[2][4];
+            uint2_t pair_mask[2][4];                 // behind the last block: of rounded pairs
+            uint4_t wt[2][2];                        // the rounded patches: columns 8 e .. + 7 of this lane's 16
             half8_t vf[2];
             uint32_t flip = 0, flip4 = 0;
             auto look_up = [&](auto sc) {
@@ -154,7 +162,8 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         const uint32_t at = ((k & 1 ? flip4 : flip) >> (8 * (2 * p + (k >> 1)))) & 0xF0u;
-                        mask[s & 1][k] = *(cl_uint4)(uintptr_t)at;
+                        if constexpr (i < I) mask[s & 1][k] = *(cl_uint4)(uintptr_t)at;
+                        else pair_mask[s & 1][k] = *(cl_uint2)(uintptr_t)(at + CL_HALVES);
                     }
                     if constexpr (i < I) vf[s & 1] = *(cl_half8)(image + i * CL_IMAGE + vread[p]);
                 }
@@ -169,25 +178,35 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
                 const half8_t a = vf[s & 1];
                 look_up(std::integral_constant<int, s + 1>{});
                 __builtin_amdgcn_sched_barrier(0);
-                asm volatile("" : "+v"(mask[s & 1][0]), "+v"(mask[s & 1][1]), "+v"(mask[s & 1][2]), "+v"(mask[s & 1][3]));   // (one wait for the four)
+                if constexpr (i < I) {
+                    asm volatile("" : "+v"(mask[s & 1][0]), "+v"(mask[s & 1][1]), "+v"(mask[s & 1][2]), "+v"(mask[s & 1][3]));   // (one wait for the four)
 #pragma unroll
-                for (int k = 0; k < 16; k++) {
-                    const float sum = acc[p][k];
-                    const uint32_t m = mask[s & 1][k / 4][k % 4];
-                    acc[p][k] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
+                    for (int k = 0; k < 16; k++) {
+                        const float sum = acc[p][k];
+                        const uint32_t m = mask[s & 1][k / 4][k % 4];
+                        acc[p][k] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
+                    }
+                    acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, uf[i], acc[p], 0, 0, 0);
+                    asm volatile("" : "+v"(acc[p]));
+                } else {
+                    // (rounded first, once, to fp16, the sign changed on the rounded pairs: half the operations, the same bits)
+                    asm volatile("" : "+v"(pair_mask[s & 1][0]), "+v"(pair_mask[s & 1][1]), "+v"(pair_mask[s & 1][2]), "+v"(pair_mask[s & 1][3]));
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const half2_t two = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]};
+                        wt[p][k / 4][k % 4] = __builtin_bit_cast(uint32_t, two) ^ pair_mask[s & 1][k / 2][k % 2];
+                    }
+                    asm volatile("" : "+v"(wt[p][0]), "+v"(wt[p][1]));
                 }
-                if constexpr (i < I) acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, uf[i], acc[p], 0, 0, 0);
-                asm volatile("" : "+v"(acc[p]));
                 __builtin_amdgcn_sched_barrier(0);
             });
-            // One rounding to fp16, the rows sorted out (see tile.hip): lane group g holds columns 32 (g / 2) + 16 p + 8 (g % 2) .. + 7 of the image
+            // The rows sorted out (see tile.hip): lane group g holds columns 32 (g / 2) + 16 p + 8 (g % 2) .. + 7 of the image
 #pragma unroll
             for (int p = 0; p < 2; p++) {
                 uint4_t lo, hi;
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
-                    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                    const auto r = __builtin_amdgcn_permlane16_swap(wt[p][0][k], wt[p][1][k], false, false);
                     lo[k] = r[0];
                     hi[k] = r[1];
                 }

@@ -39,7 +39,7 @@
 namespace {
 
 constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4;
-constexpr int TL_TABLE = 256;                       // bytes: the table of sign masks at the start of LDS
+constexpr int TL_TABLE = 512, TL_HALVES = 256;      // bytes: the tables of sign masks at the start of LDS, where the one for pairs of halves begins
 constexpr int TL_LDS = 160 * 1024;
 
 struct TileMat {
@@ -386,6 +386,8 @@ struct TileKernel {
         const int uread = I * SCH * 1024 + row * 32 + 16 * (h ^ ((row >> 4) & 1));
         float16_t acc[NP];
         uint4_t mask[LOOK + 1][4];
+        uint2_t pair_mask[LOOK + 1][4];                          // behind the last block: of rounded pairs
+        uint4_t wt[NP][2];                                       // the rounded tile (not SPLIT): this lane's columns 8 e .. + 7 of patch p
         half8_t uf[SETS];
         constexpr int WORDS = NP == 4 ? 2 : 1;
         uint32_t sw[SETS][WORDS], flip[WORDS], flip4[WORDS];
@@ -416,7 +418,8 @@ struct TileKernel {
                 for (int q = 0; q < 4; q++) {
                     // nibble q of the patch: byte 2 p + q / 2, its upper half first; times 16 it is the place of its masks
                     const uint32_t at = ((q & 1 ? flip4[word] : flip[word]) >> (8 * (2 * (p % 2) + (q >> 1)))) & 0xF0u;
-                    mask[s % (LOOK + 1)][q] = *(lds_uint4)(uintptr_t)at;
+                    if constexpr (i < I || SPLIT) mask[s % (LOOK + 1)][q] = *(lds_uint4)(uintptr_t)at;
+                    else pair_mask[s % (LOOK + 1)][q] = *(lds_uint2)(uintptr_t)(at + TL_HALVES);
                 }
             }
         };
@@ -489,18 +492,30 @@ struct TileKernel {
 #pragma unroll
                 for (int c = C; c < D; c++) out[c - C] = chunk(c);
                 __builtin_amdgcn_sched_barrier(0);
-                asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
+                if constexpr (i < I || SPLIT) {
+                    asm volatile("" : "+v"(mask[s % (LOOK + 1)][0]), "+v"(mask[s % (LOOK + 1)][1]), "+v"(mask[s % (LOOK + 1)][2]), "+v"(mask[s % (LOOK + 1)][3]));   // (one wait for the four)
 #pragma unroll
-                for (int q = 0; q < 4; q++)
+                    for (int q = 0; q < 4; q++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float sum = acc[p][4 * q + j];
-                        const uint32_t m = mask[s % (LOOK + 1)][q][j];
-                        acc[p][4 * q + j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
+                        for (int j = 0; j < 4; j++) {
+                            const float sum = acc[p][4 * q + j];
+                            const uint32_t m = mask[s % (LOOK + 1)][q][j];
+                            acc[p][4 * q + j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ m);
+                        }
+                    if constexpr (i < I)
+                        acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
+                    asm volatile("" : "+v"(acc[p]));
+                } else {
+                    // Behind the last block the sums are rounded first, once, to fp16 as a stored weight is, and the sign changed on the rounded pairs: half the
+                    // operations, and the same bits.
+                    asm volatile("" : "+v"(pair_mask[s % (LOOK + 1)][0]), "+v"(pair_mask[s % (LOOK + 1)][1]), "+v"(pair_mask[s % (LOOK + 1)][2]), "+v"(pair_mask[s % (LOOK + 1)][3]));
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const half2_t two = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]};
+                        wt[p][k / 4][k % 4] = __builtin_bit_cast(uint32_t, two) ^ pair_mask[s % (LOOK + 1)][k / 2][k % 2];
                     }
-                if constexpr (i < I)
-                    acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][p], uf[i % SETS], acc[p], 0, 0, 0);
-                asm volatile("" : "+v"(acc[p]));
+                    asm volatile("" : "+v"(wt[p][0]), "+v"(wt[p][1]));
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (D > C) {
 #pragma unroll
@@ -517,16 +532,11 @@ struct TileKernel {
             });
             if constexpr (NP < 4) pass_on();
             if constexpr (TT == 0) {
-                // One rounding to fp16; a lane holds columns 16 NP h .. + 16 NP - 1 of row l % 32
+                // A lane holds columns 16 NP h .. + 16 NP - 1 of row l % 32
 #pragma unroll
                 for (int p = 0; p < NP; p++)
 #pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        half8_t o;
-#pragma unroll
-                        for (int k = 0; k < 8; k++) o[k] = (half_t)acc[p][8 * e + k];
-                        *place(row, 2 * NP * h + 2 * p + e) = o;
-                    }
+                    for (int e = 0; e < 2; e++) *place(row, 2 * NP * h + 2 * p + e) = __builtin_bit_cast(half8_t, wt[p][e]);
                 asm volatile("" ::: "memory");               // (the stores' lanes read what others wrote)
                 first_block();                               // of tile n + 1
             } else if constexpr (SPLIT) {
@@ -590,7 +600,7 @@ struct TileKernel {
                 }
                 first_block();                   // of tile n + 1
             } else {
-                // One rounding to fp16, as a stored weight has it.  A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
+                // A lane holds columns 16 NP h + 16 p .. + 15 of row l % 32; lanes 16-31 and 48-63
                 // trade their first eight columns for the last eight of lanes 0-15 and 32-47, so that every lane group g has eight columns
                 // (16 NP (g / 2) + 16 p + 8 (g % 2) .. + 7) of rows 0-15 in one register set and of rows 16-31 in the other: B operands of
                 // v_mfma_f32_16x16x32_f16.
@@ -600,8 +610,7 @@ struct TileKernel {
                     uint4_t lo, hi;
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const half2_t a = {(half_t)acc[p][2 * k], (half_t)acc[p][2 * k + 1]}, b = {(half_t)acc[p][8 + 2 * k], (half_t)acc[p][8 + 2 * k + 1]};
-                        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+                        const auto r = __builtin_amdgcn_permlane16_swap(wt[p][0][k], wt[p][1][k], false, false);
                         lo[k] = r[0];
                         hi[k] = r[1];
                     }
@@ -647,7 +656,12 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     extern __shared__ __attribute__((aligned(1024))) char tl_lds[];
     lds_bytes_rw lds = (lds_bytes_rw)tl_lds;
     // nibble v, column j of its four (first in the top bit): the sign bit of an fp32 where the bit is set (visible behind walk's first barrier)
-    if (threadIdx.x < 64) ((__attribute__((address_space(3))) uint32_t *)lds)[threadIdx.x] = ((threadIdx.x >> 2) >> (3 - (threadIdx.x & 3))) & 1 ? 0x80000000u : 0u;
+    // and behind it the sign bits of two pairs of fp16
+    if (threadIdx.x < 64) {
+        const uint32_t v = threadIdx.x >> 2, j = threadIdx.x & 3, first = v >> (3 - 2 * (j & 1)) & 1, second = v >> (2 - 2 * (j & 1)) & 1;
+        ((__attribute__((address_space(3))) uint32_t *)lds)[threadIdx.x] = v >> (3 - j) & 1 ? 0x80000000u : 0u;
+        ((__attribute__((address_space(3))) uint32_t *)lds)[TL_HALVES / 4 + threadIdx.x] = first << 15 | second << 31;
+    }
     // (the argument block itself, so that a matrix is picked by its number with scalar loads)
     typedef const __attribute__((address_space(4))) TileGroup *kernarg_group;
     const kernarg_group grp = (kernarg_group)__builtin_amdgcn_kernarg_segment_ptr();

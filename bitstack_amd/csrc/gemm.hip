@@ -5,12 +5,12 @@
 // row (A = tokens) or one column (B = features), i.e. one 16-byte read per
 // fragment.
 //
-// Above 128 tokens and with N a multiple of 64, tiles of 128 x 128 and more are gemm_pipe.hip's; this file holds the
-// others and the choice.  linear_f16_kernel: WT x WF waves of AT x AF MFMA tiles each, k-steps of GK columns through two
+// With N a multiple of 64, every tile behind a rebuilt weight from 33 tokens on is gemm_pipe.hip's, and of bs_linear_f16's those of 128 x 128 and more and
+// most of 64 x 64; this file holds the others and the choice.  linear_f16_kernel: WT x WF waves of AT x AF MFMA tiles each, k-steps of GK columns through two
 // LDS buffers; rows are padded by 8 halves so that the lanes served per LDS cycle hit disjoint banks.  Four shapes:
 // 256 x 256 (8 waves of 128 x 64, GK = 32, three register sets of pieces in flight), 128 x 256 (8 waves of 64 x 64) and
 // 128 x 128 (4 waves) for N % 64 != 0, and 64 x 64 (4 waves, two workgroups per CU, GK = 128: half as many barriers) for
-// problems too small to fill the chip with anything larger.
+// problems too small to fill the chip with anything larger (N % 64 == 0: see pipe_64).
 // The loop is software-pipelined at three levels, all through registers:
 //   - global requests run NS k-steps ahead through NS register sets (four where the registers allow it: the
 //     kernel waits for requests more than for anything else, and a fourth set is worth 3 to 13 %; five and six were
@@ -382,26 +382,39 @@ static LinearTile linear_tile(int T, int M, int N, bool aligned) {
            wgs(128, 128) >= 160 ? LinearTile{128, 128, 64} : LinearTile{64, 64, 128};
 }
 
+// Which kernel has the 64 x 64 tiles where N % 64 == 0: linear_f16_kernel's k-steps of 128 are ahead where a few CUs have a second workgroup and the rows are long (us,
+// linear_f16_kernel / linear_pipe_kernel: 140 tokens on 6144 x 4096 27.9 / 30.9, 256 33.3 / 35.5, 300 on 4096 x 14336 102 / 107), otherwise it is behind (140 on 1024 x 4096
+// 16.0 / 13.6, 190 on 5000 x 2048 13.8 / 9.4, 256 20.1 / 14.4, 640 on 3000 x 1024 14.8 / 9.9, 400 on 4096 x 4096 28.7 / 25.5).
+static bool pipe_64(const LinearTile &tile, int T, int M, int N) {
+    const int64_t wg = bs_cdiv(T, 64) * bs_cdiv(M, 64);
+    return tile.bt == 64 && tile.bf == 64 && (wg <= 256 || wg > 384 || N <= 3072);
+}
+
 // The tile behind a rebuilt weight, where scratch for partial sums can be had too.  splits > 1: the contracted range is
 // cut into that many parts, whose sums a second kernel adds up: a few tokens on a large weight are a handful of large
 // tiles, which leave most of the chip idle, or many small ones, which move the most bytes per flop (509 tokens on
 // 4096 x 14336: 114 us with 64 x 64 tiles, 68 with 32 tiles of 256 x 256 in 8 parts each).
 struct LinearChoice { int bt, bf, splits; };      // bt == 0: as bs_linear_f16
 
-// Time in us that a tile of gemm_pipe.hip (64 x 64: linear_f16_kernel) is expected to take: rounds of workgroups over the
-// chip x k-steps of 64 columns x the time of one, which is shorter while part of the chip is idle (power), plus the sums.
-// The constants are a fit to 900 timings of 57 (tokens, M, N) from 20 x 4096 x 14336 to 16384 x 28672 x 8192; over those
-// the choice made with them is within 1 % of the best one on average, within 4 % on each.
-static double linear_cost(int bt, int bf, int splits, int T, int M, int N) {
-    const int a = bt > bf ? bt : bf, b = bt > bf ? bf : bt;
-    const double step = a == 256 ? (b == 256 ? 1.50 : b == 192 ? 1.14 : 0.95) : a == 192 ? 0.80 : b == 128 ? 0.96 : a == 128 ? 0.735 : 0.47;
+// The tiles of gemm_pipe.hip, and in us what a k-step of 64 columns and the start and end of a workgroup take: while a CU has one workgroup, and (step_two > 0) a pair of
+// workgroups that share one.  A fit to the times of every tile on 256 products, 40 to 3300 tokens on 14 matrices from 600 x 512 to 28672 x 8192: the choice
+// made with it is 1.0 % from the best tile on average, 25 at worst.  What the sums cost, and which of 256 x 128 and 128 x 256: 98 whole calls with every tile and cut, 132 to 1400
+// tokens on 12 matrices beyond 64 MiB of weight, of which the choice is 1.5 % from the best on average, 11 at worst.
+struct PipeTile { int bt, bf; double step, start, step_two, start_two; };
+static const PipeTile pipe_tiles[] = {
+    {256, 256, 1.604, 4.1, 0, 0}, {224, 256, 1.471, 3.5, 0, 0}, {192, 256, 1.358, 2.6, 0, 0}, {256, 192, 1.336, 2.9, 0, 0},
+    {160, 256, 1.143, 3.1, 0, 0}, {192, 192, 0.966, 3.1, 0, 0}, {256, 128, 0.970, 2.6, 0, 0}, {128, 256, 0.930, 2.3, 0, 0},
+    {224, 128, 0.862, 2.2, 0, 0}, {192, 128, 0.758, 1.9, 0, 0}, {128, 192, 0.777, 2.1, 0, 0}, {160, 128, 0.760, 1.3, 1.189, 4.8},
+    {128, 128, 0.620, 1.2, 1.034, 3.0}, {96, 128, 0.540, 1.1, 0.922, 1.6}, {64, 128, 0.433, 0.8, 0.688, 1.8}, {64, 64, 0.250, 1.1, 0.440, 0.9}};
+
+// Time in us that a tile is expected to take: rounds of workgroups over the chip, the last one shorter while part of it is idle (power, and memory to itself), plus the sums.
+static double linear_cost(const PipeTile &t, int splits, int T, int M, int N) {
     const int64_t all = bs_cdiv(N, 64), steps = bs_cdiv(all, splits), parts = bs_cdiv(all, steps);
-    const int64_t wg = bs_cdiv(T, bt) * bs_cdiv(M, bf) * parts;
-    const int64_t slots = a <= 128 ? 512 : 256;   // (two workgroups of the small tiles share a CU)
-    const int64_t rounds = bs_cdiv(wg, slots);
-    const double idle = 1.0 - (double)wg / (double)(rounds * slots);
-    double us = rounds * steps * step * (slots == 512 && wg <= 256 ? 0.78 : 1.0) * (1.0 - 0.35 * idle / rounds) + 2.0;
-    if (parts > 1) us += 4.7 + 8e-6 * parts * T * M / 6.0;
+    const int64_t wg = bs_cdiv(T, t.bt) * bs_cdiv(M, t.bf) * parts;
+    const bool two = t.step_two > 0 && wg > 256;
+    const int64_t slots = two ? 512 : 256, rounds = bs_cdiv(wg, slots);
+    double us = (rounds - 0.43 * (rounds - (double)wg / slots)) * steps * (two ? t.step_two : t.step) + rounds * (two ? t.start_two : t.start) + 2.0;
+    if (parts > 1) us += 3.0 + 0.5e-6 * parts * T * M;
     return us;
 }
 
@@ -412,25 +425,24 @@ static LinearChoice linear_choice(int T, int M, int N) {
     // and where a row of y can be written 16 bytes at a time.
     const int64_t weight = (int64_t)M * N * 2;
     const bool may_split = weight > (int64_t)BS_STATIC_SCRATCH_BYTES && M % 8 == 0;
-    if (T <= 128 && !may_split) return {0, 0, 1};
-    static const int tiles[][2] = {{256, 256}, {192, 256}, {256, 192}, {256, 128}, {128, 256}, {192, 128}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};
+    if (T <= 32 && !may_split) return {0, 0, 1};
     static const int cuts[] = {2, 3, 4, 6, 8, 12};
     LinearChoice one = {0, 0, 1}, cut = {0, 0, 1};
     double one_us = 1e30, cut_us = 1e30;
-    for (const auto &t : tiles) {
-        if (T > 128) {
-            const double us = linear_cost(t[0], t[1], 1, T, M, N);
-            if (us < one_us) one_us = us, one = {t[0], t[1], 1};
+    for (const PipeTile &t : pipe_tiles) {
+        if (T > 32) {
+            const double us = linear_cost(t, 1, T, M, N);
+            if (us < one_us) one_us = us, one = {t.bt, t.bf, 1};
         }
-        if (!may_split || t[1] == 64) continue;
+        if (!may_split || t.bf == 64) continue;
         for (int c : cuts) {
             if ((int64_t)c * T * M * 4 > weight) break;
-            const double us = linear_cost(t[0], t[1], c, T, M, N);
-            if (us < cut_us) cut_us = us, cut = {t[0], t[1], c};
+            const double us = linear_cost(t, c, T, M, N);
+            if (us < cut_us) cut_us = us, cut = {t.bt, t.bf, c};
         }
     }
-    if (cut_us < 0.93 * one_us) return cut;       // (the estimate has to be clear: a second kernel and its traffic are certain)
-    return one.bf == 64 ? LinearChoice{0, 0, 1} : one;
+    // (beyond 8192 columns the small tiles that an uncut range then takes are slower than the estimate: 1400 tokens on 4096 x 14336, 192 x 128 168 us, 192 x 256 in two parts 152)
+    return cut_us < (N > 8192 ? 1.06 : 1.0) * one_us ? cut : one;
 }
 // (asked for the scratch, then for the launch: the last answer of the thread is kept)
 static LinearChoice linear_choice_kept(int T, int M, int N) {
@@ -463,7 +475,7 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
         const auto skinny = [&](auto kernel) { kernel<<<(int)bs_cdiv(M, tile.bf), 64 * SKINNY_WAVES, 0, s>>>(x, w, bias, y, T, M, N); };
         if (T <= 16) tile.bf == 64 ? skinny(linear_skinny_kernel<1, 4, 2>) : tile.bf == 32 ? skinny(linear_skinny_kernel<1, 2, 2>) : skinny(linear_skinny_kernel<1, 1, 6>);
         else tile.bf == 64 ? skinny(linear_skinny_kernel<2, 4, 1>) : tile.bf == 32 ? skinny(linear_skinny_kernel<2, 2, 2>) : skinny(linear_skinny_kernel<2, 1, 4>);
-    } else if (tile.bf >= 128 && N % 64 == 0) {
+    } else if (N % 64 == 0 && (tile.bf >= 128 || pipe_64(tile, T, M, N))) {
         return bs_launch_linear_pipe(x, w, bias, y, T, M, N, tile.bt, tile.bf, 1, nullptr, s);
     } else if (tile.bt == 128 && tile.bf == 64) {
         st = launch_tiled<2, 2, 2, 1, 64>(x, w, bias, y, T, M, N, s);

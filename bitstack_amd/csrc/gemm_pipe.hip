@@ -1,6 +1,6 @@
 // The dense product's large tiles on gfx950: y[T, M] = x[T, N] @ w[M, N]^T (+ bias), fp16 in, fp32 accumulation, N % 64 == 0.
 //
-// A workgroup of 8 waves owns 64 AP rows of one operand ("P") x 128 AQ rows of the other ("Q") - tokens x features, or
+// A workgroup of 8 waves owns 32 P rows of one operand ("P") x 64 Q rows of the other ("Q") - tokens x features, or
 // (SWAP) features x tokens - and walks N in k-steps of 64 columns (one 128-byte line of every row).  Three things
 // distinguish it from linear_f16_kernel:
 //   - requests write LDS directly (16 bytes per lane): no registers hold pieces on their way and there are no LDS write
@@ -20,13 +20,18 @@
 // per k-step with both waves multiplying at once (846), four waves of 128 x 128 with three fragment sets (870).
 //
 // Phases are numbered on the wall: the upper half runs MEMORY(s) in phase 2 s and MATRIX(s) in phase 2 s + 1, the lower half
-// one later.  Stage s & 1 holds step s.  The upper P rows of a stage are read in phase 2 s only, the lower ones in
-// phase 2 s + 1 only, the Q rows in both; so the requests for step s + 2 go out
+// one later.  Stage s % S holds step s.  The upper P rows of a stage are read in phase 2 s only, the lower ones in
+// phase 2 s + 1 only, the Q rows in both; so the requests for step s + S go out
 //     upper P rows   by the upper waves in phase 2 s + 1 (their MATRIX(s))
 //     lower P rows   by the lower waves in phase 2 s + 2 (their MATRIX(s))
 //     Q rows         half by the lower waves in phase 2 s + 2, half by the upper waves in phase 2 s + 2 (their MEMORY(s + 1))
-// and are read from phase 2 s + 4 (2 s + 5) on: about two phases cover a request.  A wave waits for ITS requests of a
+// and are read from phase 2 (s + S) (one later) on: about 2 S - 2 phases cover a request.  A wave waits for ITS requests of a
 // step (a counted wait: later ones stay in flight) in front of the barrier that opens the phase in which somebody reads them.
+//
+// S, the number of stages: what a step of a small tile takes is the latency of its requests over the steps in flight (two stages: 0.5 us whatever the tile, where
+// the matrix time of 64 x 128 is 0.19), so the tiles that leave LDS for it have three or four.  us, 2 / 3 / 4 stages: 300 tokens on 1024 x 4096, 64 x 64 26.5 / 16.8 / 13.9,
+// 64 x 128 32.8 / 19.7 / 18.3; 509 on 4096 x 4096, 64 x 128 33.9 / 24.5 / 23.1; 1400 on 6144 x 4096, 192 x 192 70.2 / 65.4.  Where a CU has two workgroups these cover each
+// other's waits, and the fewer stages that let two fit are ahead (128 x 128 on 257 to 512 workgroups: 1.14 times as long with three).  Five and six stages of 64 x 64: no better.
 //
 // LDS rows are 128 bytes without padding (a request writes 64 lanes x 16 bytes contiguously); the eight 16-byte pieces of a
 // row are XOR-ed with three bits of the row number, chosen so that the 16 lanes LDS serves together in a 16-byte read
@@ -72,16 +77,26 @@ __device__ __forceinline__ void phase_barrier() {
 // fp32, linear_split_sum_kernel adds them up.
 // wide: M % 8 == 0 and y (part) 16-byte aligned: whole 16-byte stores.  Otherwise the outputs of y pass through LDS, so that a
 // store instruction still writes whole runs of a row.
-template <int AP, int AQ, bool SWAP, bool SPLIT>
+template <int P, int Q, bool SWAP, int S, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     const half_t *__restrict__ x, const half_t *__restrict__ w, const half_t *__restrict__ bias,
     half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide) {
-    constexpr int BP = 64 * AP, BQ = 128 * AQ;
+    static_assert((SWAP ? P : Q) % 2 == 0, "feature fragments come in pairs");
+    constexpr int BP = 32 * P, BQ = 64 * Q;   // P, Q: 16-row fragments of a wave
     constexpr int BT = SWAP ? BQ : BP, BF = SWAP ? BP : BQ;
-    constexpr int QJ = 2 * AQ;                // Q requests per wave and k-step (8 rows each); AP of P
-    constexpr int P = 2 * AP, Q = 2 * AQ;     // 16-row fragments of a wave
-    // one array per operand and stage: the compiler then knows that a request for one stage does not touch the other
-    __shared__ __attribute__((aligned(1024))) half_t sp0[BP * PK], sp1[BP * PK], sq0[BQ * PK], sq1[BQ * PK];
+    constexpr int PJ = (P + 1) / 2, QJ = Q;   // requests per wave and k-step, 8 rows each (an odd P: the last wave's repeat rows of its half)
+    // one array per operand and stage: the compiler then knows that a request for one stage does not touch the other.  (It tells eight such arrays apart, hence
+    // four stages at most; the two operands of a stage in one array, which would allow more, make it wait for requests that the reads have no part in.)
+    __shared__ __attribute__((aligned(1024))) half_t sp0[BP * PK], sp1[BP * PK], sp2[S > 2 ? BP * PK : 1], sp3[S > 3 ? BP * PK : 1];
+    __shared__ __attribute__((aligned(1024))) half_t sq0[BQ * PK], sq1[BQ * PK], sq2[S > 2 ? BQ * PK : 1], sq3[S > 3 ? BQ * PK : 1];
+    auto p_stage = [&](auto stage) -> half_t * {
+        constexpr int k = decltype(stage)::value;
+        return k == 0 ? sp0 : k == 1 ? sp1 : k == 2 ? sp2 : sp3;
+    };
+    auto q_stage = [&](auto stage) -> half_t * {
+        constexpr int k = decltype(stage)::value;
+        return k == 0 ? sq0 : k == 1 ? sq1 : k == 2 ? sq2 : sq3;
+    };
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -117,12 +132,15 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     // features fragment takes
     auto swizzle = [](bool features, int r) { return features ? ((r >> 1) & 1) | (((r >> 3) & 3) << 1) : (r >> 1) & 7; };
     // request j of this wave: 8 rows x 128 bytes; rows beyond T or M repeat the last one (their outputs are never stored)
-    const int prow = (wp * 4 + wq) * AP * 8, qrow = wave * QJ * 8;
-    const int p_last = SWAP ? M - 1 - m0 : T - 1 - t0, q_last = SWAP ? T - 1 - t0 : M - 1 - m0;
-    uint32_t voff_p[AP], voff_q[QJ];
+    int prow[PJ];
 #pragma unroll
-    for (int j = 0; j < AP; j++) {
-        const int r = prow + 8 * j + (lane >> 3);
+    for (int j = 0; j < PJ; j++) prow[j] = (wp * 2 * P + (P % 2 == 0 ? wq * PJ + j : min(wq * PJ + j, 2 * P - 1))) * 8;
+    const int qrow = wave * QJ * 8;
+    const int p_last = SWAP ? M - 1 - m0 : T - 1 - t0, q_last = SWAP ? T - 1 - t0 : M - 1 - m0;
+    uint32_t voff_p[PJ], voff_q[QJ];
+#pragma unroll
+    for (int j = 0; j < PJ; j++) {
+        const int r = prow[j] + (lane >> 3);
         voff_p[j] = (uint32_t)min(r, p_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(SWAP, r));
     }
 #pragma unroll
@@ -131,11 +149,11 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
         voff_q[j] = (uint32_t)min(r, q_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(!SWAP, r));
     }
     auto request_p = [&](auto stage, int step_, int j) {
-        half_t *dst = (decltype(stage)::value ? sp1 : sp0) + (prow + 8 * j) * PK;
+        half_t *dst = p_stage(stage) + prow[j] * PK;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], min(step_, steps - 1) * (PK * 2), 0, 0);
     };
     auto request_q = [&](auto stage, int step_, int j) {
-        half_t *dst = (decltype(stage)::value ? sq1 : sq0) + (qrow + 8 * j) * PK;
+        half_t *dst = q_stage(stage) + (qrow + 8 * j) * PK;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], min(step_, steps - 1) * (PK * 2), 0, 0);
     };
 
@@ -152,8 +170,8 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     auto frag_row = [](bool features, int i) { return features ? 32 * (i >> 1) + 4 * (i & 1) : 16 * i; };
     half8_t fp[2][P], fq[2][Q];
     auto load_frags = [&](auto stage) {
-        const half_t *ps = (decltype(stage)::value ? sp1 : sp0) + (wp * AP * 32 + frow_p) * PK;
-        const half_t *qs = (decltype(stage)::value ? sq1 : sq0) + (wq * AQ * 32 + frow_q) * PK;
+        const half_t *ps = p_stage(stage) + (wp * P * 16 + frow_p) * PK;
+        const half_t *qs = q_stage(stage) + (wq * Q * 16 + frow_q) * PK;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             const int pp = 8 * ((4 * kk + g) ^ swz_p), pq = 8 * ((4 * kk + g) ^ swz_q);
@@ -166,99 +184,102 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     // quarter q of a k-step: columns 32 (q / 2) .. + 31, half of the P fragments (features are the first MFMA operand)
     auto mfmas = [&](int q) {
 #pragma unroll
-        for (int i = (q & 1) * AP; i < (q & 1) * AP + AP; i++)
+        for (int i = q & 1 ? PJ : 0; i < (q & 1 ? P : PJ); i++)
 #pragma unroll
             for (int j = 0; j < Q; j++)
                 acc[i][j] = SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_f16(fp[q >> 1][i], fq[q >> 1][j], acc[i][j], 0, 0, 0)
                                  : __builtin_amdgcn_mfma_f32_16x16x32_f16(fq[q >> 1][j], fp[q >> 1][i], acc[i][j], 0, 0, 0);
     };
-    using Z = std::integral_constant<int, 0>;
-    using O = std::integral_constant<int, 1>;
+    auto all_q = [&](auto stage, int step_) {
+#pragma unroll
+        for (int j = 0; j < QJ; j++) request_q(stage, step_, j);
+    };
+    auto all_p = [&](auto stage, int step_) {
+#pragma unroll
+        for (int j = 0; j < PJ; j++) request_p(stage, step_, j);
+    };
+    // steps 0 .. `steps` - 1, S at a time (no exit between them: a path around one would make the compiler wait for the wrong requests at the top of the loop)
+    auto walk = [&](auto &&step) {
+        int s = 0;
+        for (; s + S - 1 < steps; s += S) static_for<S>([&](auto k) { step(k, s + decltype(k)::value); });
+        static_for<S - 1>([&](auto k) {
+            if (s + decltype(k)::value < steps) step(k, s + decltype(k)::value);
+        });
+    };
 
-    // ---- fill: step 0 by everybody, then what the first phases would have requested for step 1 ----------
-#pragma unroll
-    for (int j = 0; j < QJ; j++) request_q(Z{}, 0, j);
-#pragma unroll
-    for (int j = 0; j < AP; j++) request_p(Z{}, 0, j);
+    // ---- fill: step 0 by everybody, then what the phases before the first would have requested ----------
+    all_q(std::integral_constant<int, 0>{}, 0);
+    all_p(std::integral_constant<int, 0>{}, 0);
     if (wp == 0) {
-#pragma unroll
-        for (int j = 0; j < AP; j++) request_p(O{}, 1, j);
-        wait_requests<AP>();
+        static_for<S - 1>([&](auto k) {
+            constexpr int n = decltype(k)::value + 1;
+            all_p(std::integral_constant<int, n>{}, n);
+            if constexpr (n < S - 1) all_q(std::integral_constant<int, n>{}, n);
+        });
+        wait_requests<(S - 1) * PJ + (S - 2) * QJ>();
         phase_barrier();
-        auto step = [&](auto stage, int s) {
-            using Other = std::integral_constant<int, 1 - decltype(stage)::value>;
+        walk([&](auto stage, int s) {
+            using Before = std::integral_constant<int, (decltype(stage)::value + S - 1) % S>;
             // MEMORY(s): the reads first, they are what the phase waits for
             load_frags(stage);
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < QJ; j++) request_q(Other{}, s + 1, j);
+            all_q(Before{}, s + S - 1);
             wait_lds();
             phase_barrier();
             // MATRIX(s)
             __builtin_amdgcn_s_setprio(1);
             static_for<4>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                if constexpr (q < AP) request_p(stage, s + 2, q);
+                if constexpr (q < PJ) request_p(stage, s + S, q);
                 mfmas(q);
                 __builtin_amdgcn_sched_barrier(0);
             });
             __builtin_amdgcn_s_setprio(0);
-            wait_requests<AP>();               // the Q rows and upper P rows of step s + 1
+            wait_requests<(S - 1) * PJ + (S - 2) * QJ>();      // the Q rows and upper P rows of step s + 1
             phase_barrier();
-        };
-        int s = 0;
-        for (; s + 1 < steps; s += 2) {        // (no exit between the two: a path around the second one would make the
-            step(Z{}, s);                      // compiler wait for the wrong requests at the top of the loop)
-            step(O{}, s + 1);
-        }
-        if (s < steps) step(Z{}, s);
+        });
         phase_barrier();
     } else {
-#pragma unroll
-        for (int j = 0; j < QJ; j++) request_q(O{}, 1, j);
-#pragma unroll
-        for (int j = 0; j < AP; j++) request_p(O{}, 1, j);
-        wait_requests<AP + QJ>();
+        static_for<S - 1>([&](auto k) {
+            constexpr int n = decltype(k)::value + 1;
+            all_q(std::integral_constant<int, n>{}, n);
+            all_p(std::integral_constant<int, n>{}, n);
+        });
+        wait_requests<(S - 1) * (PJ + QJ)>();
         phase_barrier();
         phase_barrier();
-        auto step = [&](auto stage, int s) {
+        walk([&](auto stage, int s) {
             // MEMORY(s)
             load_frags(stage);
             wait_lds();
-            wait_requests<AP>();               // the Q rows of step s + 1
+            wait_requests<PJ + (S - 2) * (PJ + QJ)>();         // the Q rows of step s + 1
             phase_barrier();
             // MATRIX(s)
             __builtin_amdgcn_s_setprio(1);
             static_for<4>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 // Q rows first: they are read one phase earlier
-                static_for<AP + QJ>([&](auto jc) {
+                static_for<PJ + QJ>([&](auto jc) {
                     constexpr int j = decltype(jc)::value;
-                    if constexpr (j * 4 / (AP + QJ) == q) {
-                        if constexpr (j < QJ) request_q(stage, s + 2, j);
-                        else request_p(stage, s + 2, j - QJ);
+                    if constexpr (j * 4 / (PJ + QJ) == q) {
+                        if constexpr (j < QJ) request_q(stage, s + S, j);
+                        else request_p(stage, s + S, j - QJ);
                     }
                 });
                 mfmas(q);
                 __builtin_amdgcn_sched_barrier(0);
             });
             __builtin_amdgcn_s_setprio(0);
-            wait_requests<AP + QJ>();          // the lower P rows of step s + 1
+            wait_requests<(S - 1) * (PJ + QJ)>();              // the lower P rows of step s + 1
             phase_barrier();
-        };
-        int s = 0;
-        for (; s + 1 < steps; s += 2) {
-            step(Z{}, s);
-            step(O{}, s + 1);
-        }
-        if (s < steps) step(Z{}, s);
+        });
     }
     wait_requests<0>();                        // (the repeated last step's)
 
     // D[feature row, token]: the lane holds token lm of token fragment a, and of the pair of feature fragments (2 p, 2 p + 1)
     // the eight features 32 p + 8 g .. + 7
-    constexpr int TA = SWAP ? Q : P, FP = SWAP ? AP : AQ;
-    const int tw = t0 + (SWAP ? wq * AQ : wp * AP) * 32, mw = m0 + (SWAP ? wp * AP : wq * AQ) * 32;
+    constexpr int TA = SWAP ? Q : P, FP = (SWAP ? P : Q) / 2;
+    const int tw = t0 + (SWAP ? wq * Q : wp * P) * 16, mw = m0 + (SWAP ? wp * P : wq * Q) * 16;
     auto value = [&](int a, int p, int e) { return SWAP ? acc[2 * p + (e >> 2)][a][e & 3] : acc[a][2 * p + (e >> 2)][e & 3]; };
     if (SPLIT || wide) {
 #pragma unroll
@@ -349,17 +370,21 @@ __global__ __launch_bounds__(256) void linear_split_sum_kernel(const float *__re
     }
 }
 
-template <int AP, int AQ, bool SWAP>
+// S stages where the grid leaves a CU one workgroup, S_TWO where it has more (fewer of them, so that two fit its LDS)
+template <int P, int Q, bool SWAP, int S, int S_TWO>
 int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int splits, float *part, hipStream_t s) {
-    constexpr int BT = SWAP ? 128 * AQ : 64 * AP, BF = SWAP ? 64 * AP : 128 * AQ;
+    constexpr int BT = SWAP ? 64 * Q : 32 * P, BF = SWAP ? 32 * P : 64 * Q;
     const unsigned tiles = (unsigned)(bs_cdiv(T, BT) * bs_cdiv(M, BF));
     const int steps = (int)bs_cdiv(N / PK, splits);
     splits = (int)bs_cdiv(N / PK, steps);     // every part holds at least one k-step
     const int wide = M % 8 == 0 && bs_aligned(y, 16) && bs_aligned(part, 16);
+    const bool two = S_TWO != S && (int64_t)tiles * splits > 256;
     if (splits == 1) {
-        linear_pipe_kernel<AP, AQ, SWAP, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
     } else {
-        linear_pipe_kernel<AP, AQ, SWAP, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
         BS_LAUNCH_CHECK();
         const int64_t total = (int64_t)T * M;
         if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, splits, total, M);
@@ -376,15 +401,16 @@ int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, 
                           int splits, float *part, hipStream_t s) {
     if (N % PK != 0 || splits < 1 || (splits > 1 && !part)) return BS_ERR_SHAPE;
     switch (bt * 1000 + bf) {
-        case 256256: return launch_pipe<4, 2, false>(x, w, bias, y, T, M, N, splits, part, s);
-        case 192256: return launch_pipe<3, 2, false>(x, w, bias, y, T, M, N, splits, part, s);
-        case 256192: return launch_pipe<3, 2, true>(x, w, bias, y, T, M, N, splits, part, s);
-        case 256128: return launch_pipe<4, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
-        case 128256: return launch_pipe<4, 1, true>(x, w, bias, y, T, M, N, splits, part, s);
-        case 192128: return launch_pipe<3, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
-        case 128192: return launch_pipe<3, 1, true>(x, w, bias, y, T, M, N, splits, part, s);
-        case 128128: return launch_pipe<2, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
-        case 64128: return launch_pipe<1, 1, false>(x, w, bias, y, T, M, N, splits, part, s);
+#define PIPE_CASE(bt, bf, p, q, swap, s_one, s_two) \
+    case bt * 1000 + bf: \
+        static_assert(bt == (swap ? 64 * q : 32 * p) && bf == (swap ? 32 * p : 64 * q), "the tile"); \
+        static_assert(s_one * (bt + bf) * PK * 2 <= 160 * 1024 && (s_one == s_two || s_two * (bt + bf) * PK * 2 <= 80 * 1024), "LDS of a CU"); \
+        return launch_pipe<p, q, swap, s_one, s_two>(x, w, bias, y, T, M, N, splits, part, s);
+        PIPE_CASE(256, 256, 8, 4, false, 2, 2) PIPE_CASE(224, 256, 7, 4, false, 2, 2) PIPE_CASE(192, 256, 6, 4, false, 2, 2) PIPE_CASE(256, 192, 6, 4, true, 2, 2)
+        PIPE_CASE(160, 256, 5, 4, false, 3, 3) PIPE_CASE(192, 192, 6, 3, true, 3, 3) PIPE_CASE(256, 128, 8, 2, false, 3, 3) PIPE_CASE(128, 256, 8, 2, true, 3, 3)
+        PIPE_CASE(224, 128, 7, 2, false, 3, 3) PIPE_CASE(192, 128, 6, 2, false, 3, 3) PIPE_CASE(128, 192, 6, 2, true, 3, 3) PIPE_CASE(160, 128, 5, 2, false, 3, 2)
+        PIPE_CASE(128, 128, 4, 2, false, 4, 2) PIPE_CASE(96, 128, 3, 2, false, 4, 2) PIPE_CASE(64, 128, 2, 2, false, 4, 3) PIPE_CASE(64, 64, 2, 1, true, 4, 4)
+#undef PIPE_CASE
         default: return BS_ERR_SHAPE;
     }
 }

@@ -5,6 +5,8 @@
 // each result is computed in fp32 and rounded once.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int THREADS = 256;
@@ -69,113 +71,173 @@ __global__ __launch_bounds__(THREADS) void silu_mul_kernel(const half_t *gate, c
     }
 }
 
-// Causal attention of a whole prompt over the cache that rope_store_kernel has filled.  A wave takes 32 queries of one head and
-// walks the positions up to its last query 32 at a time with a running (max, sum, weighted v); the four waves of a workgroup are
-// four neighbouring heads, which mostly share a KV head and then find each other's rows in the L1.  The operands lie as in the
-// decode step's attention (decode_step.hip): scores S[position, query] = K q, output O[dim, query] += V^T P, on 16x16x32
-// products whose lane layouts fit without any shuffle - a lane of the scores holds four positions of one query in each of
-// the two tiles of 16 positions, which are the eight k slots of the output product, and V is used as loaded, product j taking
-// half j of a lane's 16 bytes.  No LDS, no barrier.  The rows of a step come from the L2 while the last step is multiplied: K is
-// requested behind the scores, V behind the output product.
-// What bounds it: the rows (16 KB a step and wave) and, with few waves, the chain of a step.  torch's attention, all sequences in
-// one call / this, us: 2 x 700 queries with 32 heads on 8 KV heads 76 / 40, 4 x 300 53 / 21, 100 15 / 8, 4000 476 / 306,
-// 4 x 1500 with 64 on 16 651 / 342 (430 TFLOP/s).  16 queries per wave read the rows twice as often: 55 on the first, 639 on the last.
-constexpr int AP_D = 128, AP_Q = 32, AP_WAVES = 4;
+// Causal attention of a whole prompt over the cache that rope_store_kernel has filled.  A wave takes 16 QT queries of one head and
+// walks the positions up to its last query 64 at a time with a running (max, sum, weighted v).  The waves of a workgroup share a KV head: their items are (tile of
+// queries, head of the group), the head fastest, so that they need the same rows.  These come to LDS a stage of 64 positions at a time, requested one stage ahead, straight from
+// memory (no registers, no LDS write instructions), one barrier per stage.  The operands lie as in the decode step's attention (decode_step.hip): scores S[position, query] =
+// K q, output O[dim, query] += V^T P, on 16x16x32 products whose lane layouts fit without any shuffle - a lane of the scores holds four positions of one query in each of
+// two tiles of 16 positions, which are the eight k slots of the output product, and V is used as it lies, product j taking half j of a lane's 16 bytes.  The 16-byte
+// pieces of a row of K are XOR-ed with the row's number: a score fragment reads one piece of 16 rows, which lie a whole turn of the banks apart.
+// What bounds it: with many queries the issue of the softmax's instructions and of the products (800 TFLOP/s of the lower triangle), with few the chain of a stage, 1.2 us.
+// us, every wave reading its own rows from L2 32 positions at a time / this: 2 x 700 queries with 32 heads on 8 KV heads 40.4 / 22.8, 4 x 300 21.5 / 13.6, 100 8.1 / 5.8, 4000 309 / 173,
+// 4 x 1500 with 64 on 16 352 / 214, 64 on 64 364 / 247, 8 x 2048 with 64 on 8 1214 / 683.  A stage of 64 as two steps of 32 positions: 28.5 on the first, 198 on the fourth.
+// Error against float64: 2.360e-4 on the first, 2.394e-4 on 1 x 2000 with 8 on 2 (before 2.362e-4 and 2.394e-4).
+constexpr int AP_D = 128, AP_WAVES = 4, AP_P = 64;       // (AP_P: positions of a stage)
+constexpr int AP_CHUNKS = 2 * (AP_P / 4) / AP_WAVES;                // requests per wave and stage: of 1 KB, four rows; K, then V
 
+typedef __attribute__((address_space(3))) void *ap_lds;
+
+// the larger of v here and in the lane whose number differs by W (16 or 32)
+template <int W>
+__device__ __forceinline__ float across(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = W == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t a = r[0], b = r[1];
+    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+
+template <int QT>
 __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kcache,
                                                                              const half_t *__restrict__ vcache, half_t *__restrict__ out,
-                                                                             int ldq, int n, int heads, int kv_heads, int max_len) {
+                                                                             int ldq, int n, int heads, int kv_heads, int max_len, int chunks) {
+    // (an array per operand and stage: the compiler then knows that a request for one does not touch the others)
+    __shared__ __attribute__((aligned(1024))) half_t sk0[AP_P * AP_D], sk1[AP_P * AP_D], sv0[AP_P * AP_D], sv1[AP_P * AP_D];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-    const int quads = (heads + AP_WAVES - 1) / AP_WAVES, b = blockIdx.x / quads, head = (blockIdx.x % quads) * AP_WAVES + wave;
-    if (head >= heads) return;
-    const int q0 = (int)(gridDim.y - 1 - blockIdx.y) * AP_Q;             // the longest rows first
-    const int hk = head / (heads / kv_heads);
+    const int group = heads / kv_heads, items = group * ((n + (16 * QT) - 1) / (16 * QT));
+    const int at = (int)(blockIdx.y + blockIdx.z * gridDim.y);
+    if (at >= chunks) return;
+    const int first = (chunks - 1 - at) * AP_WAVES, item = min(first + wave, items - 1);     // the longest first
+    const int b = blockIdx.x / kv_heads, hk = blockIdx.x - b * kv_heads, head = hk * group + item % group;
+    const int q0 = item / group * (16 * QT);
+    const bool mine = first + wave < items;
+    const int stages = min(first + AP_WAVES - 1, items - 1) / group * (16 * QT) / AP_P + 1;       // (a tile of queries lies within a stage)
     const int64_t row = (int64_t)heads * AP_D;
-    const half_t *kc = kcache + ((int64_t)b * kv_heads + hk) * max_len * AP_D, *vc = vcache + ((int64_t)b * kv_heads + hk) * max_len * AP_D;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(kcache + ((int64_t)b * kv_heads + hk) * max_len * AP_D), 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vcache + ((int64_t)b * kv_heads + hk) * max_len * AP_D), 0, -1, 0x00020000);
 
-    half8_t k8[2][4], v8[8], q8[2][4];
-    auto fetch_k = [&](int p0) {                 // (rows past the last are the last again; their scores are masked)
+    auto request = [&](auto stage, int p0) {         // (rows past the last are the last again; their scores are masked)
+        half_t *const k_to = decltype(stage)::value ? sk1 : sk0, *const v_to = decltype(stage)::value ? sv1 : sv0;
 #pragma unroll
-        for (int a = 0; a < 2; a++) {
-            const half_t *p = kc + (int64_t)min(p0 + 16 * a + r16, n - 1) * AP_D + 8 * g;
+        for (int j = 0; j < AP_CHUNKS / 2; j++) {
+            const int r = (wave * (AP_CHUNKS / 2) + j) * 4 + g;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (ap_lds)(k_to + (wave * (AP_CHUNKS / 2) + j) * 512), 16, min(p0 + r, n - 1) * (AP_D * 2) + 16 * (r16 ^ (r & 15)), 0, 0, 0);
+        }
 #pragma unroll
-            for (int c = 0; c < 4; c++) k8[a][c] = *reinterpret_cast<const half8_t *>(p + 32 * c);
+        for (int j = 0; j < AP_CHUNKS / 2; j++) {
+            const int r = (wave * (AP_CHUNKS / 2) + j) * 4 + g;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (ap_lds)(v_to + (wave * (AP_CHUNKS / 2) + j) * 512), 16, min(p0 + r, n - 1) * (AP_D * 2) + 16 * r16, 0, 0, 0);
         }
     };
-    auto fetch_v = [&](int p0) {
+    request(std::integral_constant<int, 0>{}, 0);
+    half8_t q8[QT][4];
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            v8[i] = *reinterpret_cast<const half8_t *>(vc + (int64_t)min(p0 + 16 * (i >> 2) + 4 * g + (i & 3), n - 1) * AP_D + 8 * r16);
-    };
-    fetch_k(0);
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
+    for (int t = 0; t < QT; t++) {
         const half_t *p = q + ((int64_t)b * n + min(q0 + 16 * t + r16, n - 1)) * ldq + head * AP_D + 8 * g;
 #pragma unroll
         for (int c = 0; c < 4; c++) q8[t][c] = *reinterpret_cast<const half8_t *>(p + 32 * c);
     }
-    fetch_v(0);
 
     const float scale2 = 0.08838834764831845f * 1.4426950408889634f;    // 1 / sqrt(128) * log2(e): the softmax runs in base 2
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};              // of query r16 of a tile; the sum over this lane's positions
-    float4_t acc[2][8];
+    float m[QT];                                 // of query r16 of a tile
+    float4_t acc[QT][8], l[QT];                  // (l: the sum of the weights as they are multiplied, that is rounded, by a product with ones; the same in all four)
+    const half8_t ones = {(half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1};
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int t = 0; t < QT; t++) {
+        m[t] = -INFINITY;
+        l[t] = (float4_t)0.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) acc[t][j] = (float4_t)0.f;
-    for (int p0 = 0; p0 <= q0; p0 += AP_Q) {
-        float4_t s[2][2];                        // [query tile][position tile]
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int a = 0; a < 2; a++) {
-                s[t][a] = (float4_t)0.f;
-#pragma unroll
-                for (int c = 0; c < 4; c++) s[t][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[a][c], q8[t][c], s[t][a], 0, 0, 0);
-            }
-        if (p0 < q0) fetch_k(p0 + AP_Q);
-        half8_t p8[2];
-#pragma unroll
-        for (int t = 0; t < 2; t++) {
-            float p[8], mx = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                p[i] = s[t][i >> 2][i & 3] * scale2;
-                if (p0 == q0 && 16 * (i >> 2) + 4 * g + (i & 3) > 16 * t + r16) p[i] = -INFINITY;      // behind the query
-                mx = fmaxf(mx, p[i]);
-            }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float mn = fmaxf(m[t], mx), r = __builtin_amdgcn_exp2f(m[t] - mn);
-            m[t] = mn;
-            float sum = 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                p[i] = __builtin_amdgcn_exp2f(p[i] - mn);
-                sum += p[i];
-                p8[t][i] = (half_t)p[i];
-            }
-            l[t] = l[t] * r + sum;
-            if (__any(r != 1.f)) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[t][j] *= r;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const half8_t v = {v8[0][j], v8[1][j], v8[2][j], v8[3][j], v8[4][j], v8[5][j], v8[6][j], v8[7][j]};
-#pragma unroll
-            for (int t = 0; t < 2; t++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p8[t], acc[t][j], 0, 0, 0);
-        }
-        if (p0 < q0) fetch_v(p0 + AP_Q);
     }
+    // a stage: positions p0 .. p0 + 63
+    constexpr int A = AP_P / 16;
+    auto step = [&](const half_t *sk, const half_t *sv, int p0) __attribute__((always_inline)) {     // (a call would keep the sums in memory)
+        float4_t s[QT][A];                        // [query tile][position tile]
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        l[t] += __shfl_xor(l[t], 16, 64);
-        l[t] += __shfl_xor(l[t], 32, 64);
+        for (int a = 0; a < A; a++) {
+            half8_t k8[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) k8[c] = *reinterpret_cast<const half8_t *>(sk + (16 * a + r16) * AP_D + 8 * ((4 * c + g) ^ r16));
+#pragma unroll
+            for (int t = 0; t < QT; t++) s[t][a] = (float4_t)0.f;
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int t = 0; t < QT; t++) s[t][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[c], q8[t][c], s[t][a], 0, 0, 0);
+        }
+        half8_t v8[8];
+        auto fetch_v = [&](int h) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v8[i] = *reinterpret_cast<const half8_t *>(sv + (32 * h + 16 * (i >> 2) + 4 * g + (i & 3)) * AP_D + 8 * r16);
+        };
+        fetch_v(0);                              // (arrives during the softmax)
+        __builtin_amdgcn_sched_barrier(0);
+        if (p0 + AP_P > q0) {                    // some of the positions are behind a query
+#pragma unroll
+            for (int t = 0; t < QT; t++)
+#pragma unroll
+                for (int a = 0; a < A; a++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (p0 + 16 * a + 4 * g + i > q0 + 16 * t + r16) s[t][a][i] = -INFINITY;
+        }
+        float r[QT];
+        half8_t p8[QT][A / 2];
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+            float mx = s[t][0][0];
+#pragma unroll
+            for (int i = 1; i < 4 * A; i++) mx = fmaxf(mx, s[t][i >> 2][i & 3]);
+            mx = across<32>(across<16>(mx));
+            const float mn = fmaxf(m[t], mx * scale2);
+            r[t] = __builtin_amdgcn_exp2f(m[t] - mn);
+            m[t] = mn;
+#pragma unroll
+            for (int i = 0; i < 4 * A; i++) p8[t][i >> 3][i & 7] = (half_t)__builtin_amdgcn_exp2f(s[t][i >> 2][i & 3] * scale2 - mn);
+        }
+        if (__any(r[0] != 1.f || r[QT - 1] != 1.f)) {
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                l[t] *= r[t];
+#pragma unroll
+                for (int j = 0; j < 8; j++) acc[t][j] *= r[t];
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < A / 2; h++) {
+#pragma unroll
+            for (int t = 0; t < QT; t++) l[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p8[t][h], l[t], 0, 0, 0);
+            if (h > 0 && p0 + 32 * h > q0) continue;      // (32 positions behind all of the queries: an infinity in their v must not make a NaN of a weight of zero)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const half8_t v = {v8[0][j], v8[1][j], v8[2][j], v8[3][j], v8[4][j], v8[5][j], v8[6][j], v8[7][j]};
+#pragma unroll
+                for (int t = 0; t < QT; t++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p8[t][h], acc[t][j], 0, 0, 0);
+            }
+            if (h + 1 < A / 2) fetch_v(h + 1);
+        }
+    };
+    auto walk = [&](auto stage, int st) {
+        // this wave's requests for the stage have landed; behind the barrier everybody's have, and nobody reads the other stage any more
+        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < stages) request(std::integral_constant<int, 1 - decltype(stage)::value>{}, (st + 1) * AP_P);
+        const half_t *const sk = decltype(stage)::value ? sk1 : sk0, *const sv = decltype(stage)::value ? sv1 : sv0;
+        if (mine && st * AP_P <= q0) step(sk, sv, st * AP_P);
+    };
+    for (int st = 0; st < stages; st += 2) {
+        walk(std::integral_constant<int, 0>{}, st);
+        if (st + 1 < stages) walk(std::integral_constant<int, 1>{}, st + 1);
+    }
+    if (!mine) return;
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
         const int qi = q0 + 16 * t + r16;
         if (qi >= n) continue;
-        const float inv = 1.f / l[t];
+        const float inv = 1.f / l[t][0];
         half_t *to = out + ((int64_t)b * n + qi) * row + head * AP_D;
 #pragma unroll
         for (int i = 0; i < 4; i++) {            // row 4 g + i of product j is dimension 8 (4 g + i) + j
@@ -191,8 +253,18 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
 
 int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int ldq, int B, int n, int heads,
                                 int kv_heads, int max_len, hipStream_t s) {
-    const dim3 grid((unsigned)(B * bs_cdiv(heads, AP_WAVES)), (unsigned)bs_cdiv(n, AP_Q));
-    attention_prefill_kernel<<<grid, AP_WAVES * 64, 0, s>>>(q, kcache, vcache, out, ldq, n, heads, kv_heads, max_len);
+    const auto launch = [&](auto kernel, int queries) {
+        const int64_t chunks = bs_cdiv((int64_t)(heads / kv_heads) * bs_cdiv(n, queries), AP_WAVES), y = chunks < 32768 ? chunks : 32768;
+        if (chunks > INT32_MAX / AP_WAVES) return BS_ERR_SHAPE;
+        const dim3 grid((unsigned)(B * kv_heads), (unsigned)y, (unsigned)bs_cdiv(chunks, y));
+        kernel<<<grid, AP_WAVES * 64, 0, s>>>(q, kcache, vcache, out, ldq, n, heads, kv_heads, max_len, (int)chunks);
+        return (int)BS_OK;
+    };
+    // 16 queries per wave while 32 would leave the chip few workgroups: the chain of a wave's stages is what such a call takes (us, 32 / 16 queries: 2 x 700 positions with 32
+    // heads on 8 KV heads, 352 workgroups, 24.5 / 21.7; 1 x 1000 with 8 on 8 26.1 / 19.7; 4 x 300 with 32 on 8, 320, 15.0 / 14.3; but 8 x 200, 448, 15.1 / 15.6; 2 x 1000, 512, 34.8 / 41.2).
+    const int64_t wgs = (int64_t)B * kv_heads * bs_cdiv((int64_t)(heads / kv_heads) * bs_cdiv(n, 32), AP_WAVES);
+    const int st = wgs <= 400 ? launch(attention_prefill_kernel<1>, 16) : launch(attention_prefill_kernel<2>, 32);
+    if (st != BS_OK) return st;
     BS_LAUNCH_CHECK();
     return BS_OK;
 }

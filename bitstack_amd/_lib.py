@@ -37,6 +37,7 @@ SIGNATURES = {
     "bs_forward_path": (_I, [_I, _I, _I, _I, _I]),
     "bs_sparse_kernel": (_I, [_P, _P, _I, _I, _I, _I]),
     "bs_tile_kernel": (_I, [_P, _P, _I, _I, _I, _I, _P]),
+    "bs_small_rank_kernel": (_I, [_P, _P, _I, _I, _I, _I, _P]),
 }
 ERR_WORKSPACE = -5
 DECODE_AUTO, DECODE_F16, DECODE_MX = 0, 1, 2
@@ -119,6 +120,15 @@ def tile_kernel(layers, N, K, T):
     return kind, list(columns)
 
 
+def small_rank_kernel(layers, N, K, T):
+    """tile_kernel for ranks below 16."""
+    n = len(layers)
+    I, M, columns = (ctypes.c_int * n)(*(i for i, _ in layers)), (ctypes.c_int * n)(*(m for _, m in layers)), (ctypes.c_int * n)()
+    kind = int(lib().bs_small_rank_kernel(I, M, n, N, K, T, columns))
+    check(min(kind, 0), "bs_small_rank_kernel")
+    return kind, list(columns)
+
+
 def sparse_kernel(layers, N, K, T):
     """Whether gemv_sparse_kernel runs one or several (blocks, out features) on the same x."""
     n = len(layers)
@@ -133,7 +143,7 @@ def forward_kernel_name(I, M, N, K, T):
         return "gemv_sparse_kernel"
     path = int(lib().bs_forward_path(I, M, N, K, T))
     check(min(path, 0), "bs_forward_path")
-    return TILE_NAMES.get(tile_kernel([(I, M)], N, K, T)[0], PATH_NAMES[path])
+    return TILE_NAMES.get((tile_kernel if K == 16 else small_rank_kernel)([(I, M)], N, K, T)[0], PATH_NAMES[path])
 
 
 def linear_plan(T, M, N):

@@ -109,7 +109,8 @@ extern "C" int bs_sparse_kernel(const int *I, const int *M, int n, int N, int K,
     return empty ? 0 : bs_gemv_sparse_serves(I, M, n, N, K, T);
 }
 
-extern "C" int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) {
+// `asked`: for the rank (16 or less) that the caller asks about
+static int tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns, bool asked) {
     if (!I || !M || !columns) return BS_ERR_NULL;
     if (n < 1 || n > BS_MAX_GROUP) return BS_ERR_SHAPE;
     bool empty = T == 0;
@@ -119,8 +120,11 @@ extern "C" int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, i
         empty = empty || I[j] == 0;
         columns[j] = 0;
     }
-    return empty ? BS_TILE_NONE : bs_gemv_tile_kernel(I, M, n, N, K, T, columns);
+    return empty || !asked ? BS_TILE_NONE : bs_gemv_tile_kernel(I, M, n, N, K, T, columns);
 }
+
+extern "C" int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) { return tile_kernel(I, M, n, N, K, T, columns, K == 16); }
+extern "C" int bs_small_rank_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns) { return tile_kernel(I, M, n, N, K, T, columns, K < 16); }
 
 static int forward_impl(const uint8_t *packed, const void *u, const void *vt, const void *x,
                         const void *bias, void *y, int I, int M, int N, int K, int T,

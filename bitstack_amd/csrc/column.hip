@@ -1,4 +1,4 @@
-// Forward for 49 to 128 tokens on gfx950, rank 16, up to 8 blocks: the tile kernel's rebuild (tile.hip) with the loops turned round.
+// Forward for 49 to 128 tokens on gfx950, rank 16 (and 8 to 15: column_ranks.hip), up to 8 blocks: the tile kernel's rebuild (tile.hip) with the loops turned round.
 //
 //   part[cg, t, m] = sum_{n in column group cg} x[t, n] * fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
 //
@@ -24,6 +24,22 @@
 #include <type_traits>
 #include <utility>
 
+struct ColumnMat {
+    const uint8_t *packed;
+    const half_t *u, *vt;
+    float *part;
+    int M, row_groups, spans;                       // spans of 256 columns per column group
+};
+
+// The kernels for ranks 8 to 15 are the same code with a rank that is not known at compile time, in a translation unit of their own (column_ranks.hip includes this file): with
+// one kernel for all ranks 14336 x 4096, 5 blocks, 100 tokens took 57.3 us for 55.0.
+#ifdef COLUMN_RANKS
+constexpr bool CL_K16 = false;
+#else
+constexpr bool CL_K16 = true;
+#endif
+int bs_launch_column_ranks(const ColumnMat &m, int I, int grid, const half_t *x, int N, int T, int K, hipStream_t s);
+
 namespace {
 
 constexpr int CL_WAVES = 8, CL_ROWS = 256, CL_TABLE = 512, CL_HALVES = 256, CL_MIN_T = 49, CL_MAX_T = 128;
@@ -38,6 +54,7 @@ __device__ __forceinline__ void cl_for(F &&f) {
     cl_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+typedef half8_t cl_half8_any __attribute__((aligned(2)));
 typedef __attribute__((address_space(3))) char *cl_bytes;
 typedef const __attribute__((address_space(3))) half8_t *cl_half8;
 typedef __attribute__((address_space(3))) half8_t *cl_half8_rw;
@@ -45,16 +62,10 @@ typedef __attribute__((address_space(3))) half2_t *cl_half2_rw;
 typedef const __attribute__((address_space(3))) uint4_t *cl_uint4;
 typedef const __attribute__((address_space(3))) uint2_t *cl_uint2;
 
-struct ColumnMat {
-    const uint8_t *packed;
-    const half_t *u, *vt;
-    float *part;
-    int M, row_groups, spans;                       // spans of 256 columns per column group
-};
-
 // TT: token tiles of 16
 template <int TT, int I>
-__global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const ColumnMat mat, const half_t *__restrict__ x, int N, int T) {
+__global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const ColumnMat mat, const half_t *__restrict__ x, int N, int T, int ranks) {
+    const int K = CL_K16 ? 16 : ranks;
     extern __shared__ __attribute__((aligned(1024))) char cl_lds[];
     const cl_bytes lds = (cl_bytes)cl_lds;
     constexpr int VT = I * CL_IMAGE, BUFFER = VT + TT * CL_IMAGE, XK = (TT + 3) / 4;
@@ -85,8 +96,23 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
     };
 #pragma unroll
     for (int i = 0; i < I; i++) {
-        uf[i] = *reinterpret_cast<const half8_t *>(mat.u + ((int64_t)i * M + my_row) * 16 + 8 * h);
+        uf[i] = *reinterpret_cast<const cl_half8_any *>(mat.u + ((int64_t)i * M + my_row) * K + (h ? K - 8 : 0));     // (fewer than 16 ranks: the row's last eight)
         request_signs(i, first);
+    }
+
+    if (K < 16) {                                   // ranks 8 to K - 1 first, zeros behind them
+#pragma unroll
+        for (int i = 0; i < I; i++) {
+            half8_t o = uf[i];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+#pragma unroll
+                for (int d = 0; d < 8; d++)
+                    if (h && d == e + 16 - K) o[e] = uf[i][d];
+                if (h && 8 + e >= K) o[e] = (half_t)0;
+            }
+            uf[i] = o;
+        }
     }
 
     // ---- staging: image column 32 h' + c is column 128 h' + 32 q + c of the span; columns beyond N are zero -------------------
@@ -97,11 +123,11 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
         const int n0 = span * 256 + 32 * q;
         if (wave < I) {
             const int col = n0 + 128 * (pc >> 2) + 8 * (pc & 3);
-            const half_t *src = mat.vt + ((int64_t)wave * 16 + 2 * rp) * N + min(col, N - 8);
+            const half_t *src = mat.vt + (int64_t)wave * K * N + min(col, N - 8);
 #pragma unroll
             for (int r = 0; r < 2; r++) {
-                vpre[r] = *reinterpret_cast<const half8_t *>(src + (int64_t)r * N);
-                if (col >= N) vpre[r] = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
+                vpre[r] = *reinterpret_cast<const half8_t *>(src + (int64_t)min(2 * rp + r, K - 1) * N);
+                if (col >= N || 2 * rp + r >= K) vpre[r] = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
             }
         }
 #pragma unroll
@@ -235,6 +261,52 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
             }
 }
 
+template <int TT, int I>
+int launch_column(const ColumnMat &m, int grid, const half_t *x, int N, int T, int K, hipStream_t s) {
+    const size_t lds = CL_TABLE + 2 * (size_t)(I + TT) * CL_IMAGE;
+    static bs_lds_grant granted[BS_MAX_DEVICES];
+    const int st = bs_allow_lds((const void *)column_forward_kernel<TT, I>, lds, granted);
+    if (st != BS_OK) return st;
+    column_forward_kernel<TT, I><<<grid, 64 * CL_WAVES, lds, s>>>(m, x, N, T, K);
+    BS_LAUNCH_CHECK();
+    return BS_OK;
+}
+// Token tiles: as many as there are, from four on.  us with four, six or eight / with these: 14336 x 4096, 5 blocks, 100 tokens (7) 58.9 / 57.9, 28672 x 8192, 3, 80 (5)
+// 113.4 / 109.7, 11520 x 11904, 3, 112 83.0 / 81.1, 6144 x 4096, 1, 66 21.4 / 20.7, 4096 x 4096, 6, 75 25.8 / 25.7.
+// (registers: 8 per token tile and 10 per block)
+constexpr int max_blocks(int token_tiles) { return token_tiles == 4 ? 8 : token_tiles <= 6 ? 7 : 6; }
+template <int TT>
+int launch_blocks(int I, const ColumnMat &m, int grid, const half_t *x, int N, int T, int K, hipStream_t s) {
+    switch (I) {
+        case 1: return launch_column<TT, 1>(m, grid, x, N, T, K, s);
+        case 2: return launch_column<TT, 2>(m, grid, x, N, T, K, s);
+        case 3: return launch_column<TT, 3>(m, grid, x, N, T, K, s);
+        case 4: return launch_column<TT, 4>(m, grid, x, N, T, K, s);
+        case 5: return launch_column<TT, 5>(m, grid, x, N, T, K, s);
+        case 6: return launch_column<TT, 6>(m, grid, x, N, T, K, s);
+        case 7: if constexpr (max_blocks(TT) >= 7) return launch_column<TT, 7>(m, grid, x, N, T, K, s); break;
+        case 8: if constexpr (max_blocks(TT) >= 8) return launch_column<TT, 8>(m, grid, x, N, T, K, s); break;
+    }
+    return BS_ERR_SHAPE;
+}
+int token_tiles(int T) { return T <= 64 ? 4 : (int)bs_cdiv(T, 16); }
+int launch_tokens(const ColumnMat &m, int I, int grid, const half_t *x, int N, int T, int K, hipStream_t s) {
+    switch (token_tiles(T)) {
+        case 4: return launch_blocks<4>(I, m, grid, x, N, T, K, s);
+        case 5: return launch_blocks<5>(I, m, grid, x, N, T, K, s);
+        case 6: return launch_blocks<6>(I, m, grid, x, N, T, K, s);
+        case 7: return launch_blocks<7>(I, m, grid, x, N, T, K, s);
+        default: return launch_blocks<8>(I, m, grid, x, N, T, K, s);
+    }
+}
+
+}  // namespace
+
+#ifdef COLUMN_RANKS
+int bs_launch_column_ranks(const ColumnMat &m, int I, int grid, const half_t *x, int N, int T, int K, hipStream_t s) { return launch_tokens(m, I, grid, x, N, T, K, s); }
+#else
+namespace {
+
 struct ColumnPlan {
     int row_groups, spans, groups;
 };
@@ -250,36 +322,6 @@ ColumnPlan make_column_plan(int M, int N) {
     return p;
 }
 
-template <int TT, int I>
-int launch_column(const ColumnMat &m, int grid, const half_t *x, int N, int T, hipStream_t s) {
-    const size_t lds = CL_TABLE + 2 * (size_t)(I + TT) * CL_IMAGE;
-    static bs_lds_grant granted[BS_MAX_DEVICES];
-    const int st = bs_allow_lds((const void *)column_forward_kernel<TT, I>, lds, granted);
-    if (st != BS_OK) return st;
-    column_forward_kernel<TT, I><<<grid, 64 * CL_WAVES, lds, s>>>(m, x, N, T);
-    BS_LAUNCH_CHECK();
-    return BS_OK;
-}
-// Token tiles: as many as there are, from four on.  us with four, six or eight / with these: 14336 x 4096, 5 blocks, 100 tokens (7) 58.9 / 57.9, 28672 x 8192, 3, 80 (5)
-// 113.4 / 109.7, 11520 x 11904, 3, 112 83.0 / 81.1, 6144 x 4096, 1, 66 21.4 / 20.7, 4096 x 4096, 6, 75 25.8 / 25.7.
-// (registers: 8 per token tile and 10 per block)
-constexpr int max_blocks(int token_tiles) { return token_tiles == 4 ? 8 : token_tiles <= 6 ? 7 : 6; }
-template <int TT>
-int launch_blocks(int I, const ColumnMat &m, int grid, const half_t *x, int N, int T, hipStream_t s) {
-    switch (I) {
-        case 1: return launch_column<TT, 1>(m, grid, x, N, T, s);
-        case 2: return launch_column<TT, 2>(m, grid, x, N, T, s);
-        case 3: return launch_column<TT, 3>(m, grid, x, N, T, s);
-        case 4: return launch_column<TT, 4>(m, grid, x, N, T, s);
-        case 5: return launch_column<TT, 5>(m, grid, x, N, T, s);
-        case 6: return launch_column<TT, 6>(m, grid, x, N, T, s);
-        case 7: if constexpr (max_blocks(TT) >= 7) return launch_column<TT, 7>(m, grid, x, N, T, s); break;
-        case 8: if constexpr (max_blocks(TT) >= 8) return launch_column<TT, 8>(m, grid, x, N, T, s); break;
-    }
-    return BS_ERR_SHAPE;
-}
-int token_tiles(int T) { return T <= 64 ? 4 : (int)bs_cdiv(T, 16); }
-
 }  // namespace
 
 // From how many weights on this kernel runs: with fewer there are 256 x 256 squares for fewer than about 3/4 of the CUs, and the start and end
@@ -291,7 +333,7 @@ constexpr int64_t CL_MIN_WEIGHTS = 11ll << 20;
 
 // Column groups (partial sums per output) when this kernel takes the shape, else 0.
 int bs_column_partials(int I, int M, int N, int K, int T) {
-    if (bs_prefill_mode() != 0 || K != 16 || I < 1 || T < CL_MIN_T || T > CL_MAX_T || I > max_blocks(token_tiles(T)) || M < 1 || N < SF_COLS || N % SF_COLS != 0) return 0;
+    if (bs_prefill_mode() != 0 || K < 8 || K > 16 || I < 1 || T < CL_MIN_T || T > CL_MAX_T || I > max_blocks(token_tiles(T)) || M < 1 || N < SF_COLS || N % SF_COLS != 0) return 0;
     if ((int64_t)M * N < CL_MIN_WEIGHTS || (int64_t)M * (N >> 3) >= ((int64_t)1 << 32)) return 0;       // a row's signs within a 32-bit byte offset
     return make_column_plan(M, N).groups;
 }
@@ -301,16 +343,10 @@ int bs_column_width(int I, int M, int N, int K, int T) { return bs_column_partia
 
 int bs_launch_column(const uint8_t *packed, const half_t *u, const half_t *vt, int I, int M, float *part, const half_t *x, int N, int K, int T, hipStream_t s) {
     const int groups = bs_column_partials(I, M, N, K, T);
-    if (groups == 0 || !bs_aligned(x, 16) || !bs_aligned(packed, 16) || !bs_aligned(vt, 16) || !bs_aligned(u, 16)) return BS_ERR_SHAPE;
+    if (groups == 0 || !bs_aligned(x, 16) || !bs_aligned(packed, 16) || !bs_aligned(vt, 16) || !bs_aligned(u, K == 16 ? 16 : 2)) return BS_ERR_SHAPE;
     const ColumnPlan p = make_column_plan(M, N);
     const ColumnMat m{packed, u, vt, part, M, p.row_groups, p.spans};
     const int grid = p.row_groups * p.groups;
-    const int tt = token_tiles(T);
-    switch (tt) {
-        case 4: return launch_blocks<4>(I, m, grid, x, N, T, s);
-        case 5: return launch_blocks<5>(I, m, grid, x, N, T, s);
-        case 6: return launch_blocks<6>(I, m, grid, x, N, T, s);
-        case 7: return launch_blocks<7>(I, m, grid, x, N, T, s);
-        default: return launch_blocks<8>(I, m, grid, x, N, T, s);
-    }
+    return K == 16 ? launch_tokens(m, I, grid, x, N, T, K, s) : bs_launch_column_ranks(m, I, grid, x, N, T, K, s);
 }
+#endif

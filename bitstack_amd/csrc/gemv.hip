@@ -998,7 +998,7 @@ int64_t tile_part_floats(const int *I, const int *M, int n, int N, int K, int T,
 // up to 1000 rows, 8 are more than 3 % behind the tile kernel, 7 % at worst; all of them on the sparse kernel: 85, 55 %).
 // (sparse: its plan, where it serves the call)
 bool split_tiles(const int *I, const int *M, int n, int N, int K, int T, const Plan *sparse) {
-    if ((T != 3 && T != 4) || g_decode_kernel != 0) return false;
+    if ((T != 3 && T != 4) || K != 16 || g_decode_kernel != 0) return false;
     int64_t bytes = 0;
     for (int j = 0; j < n; j++) {
         const bool large = (int64_t)M[j] * N > (24ll << 20);
@@ -1044,7 +1044,7 @@ bool sparse_plan(Plan &p, const int *I, const int *M, int n, int N, int K, int T
     const int slots = I[0] * p.kmax[0];
     double cycles;
     int groups[GEMV_MAX_GROUP];
-    if (K == 16 && (slots >= 64 || p.n_chunks == 1) && bs_tile_partials(I, M, 1, N, K, T, groups, &cycles)) return sparse_call_us(p, I[0], T) <= tile_call_us(cycles, groups[0], N, T);
+    if ((slots >= 64 || p.n_chunks == 1) && bs_tile_partials(I, M, 1, N, K, T, groups, &cycles)) return sparse_call_us(p, I[0], T) <= tile_call_us(cycles, groups[0], N, T);
     return slots < 250 || sparse_call_us(p, I[0], T) <= strip_call_us(bs_strip_steps(I[0], M[0], N, T), I[0]);
 }
 int64_t strip_part_floats(const int *I, const int *M, int n, int N, int K, int T) {
@@ -1100,10 +1100,12 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     r.n_in = N;
     r.eps = eps;
     float *parts[GEMV_MAX_GROUP];
-    // The tile kernel (from 49 tokens the column kernel) where it takes the matrices; the strip and panel kernels for ranks below 16, long stacks, small matrices and u off a 16-byte boundary.
+    // The tile kernel (from 49 tokens the column kernel) where it takes the matrices; the strip and panel kernels for ranks below 8, long stacks, small matrices and, at rank 16, u
+    // off a 16-byte boundary.  Ranks 8 to 15 have a build of their own of both (us, strip, walked or panel kernel / that, rank 12: 28672 x 8192, 3 blocks, 8 tokens 102.2 / 60.5, 40 tokens 154 / 124;
+    // 14336 x 4096, 8, 8 tokens 69.0 / 43.4; 5, 100 tokens 77.6 / 58.4; 5000 x 4096, 6, 37 tokens 39.4 / 27.7; 4096 x 14336, 8, 509 tokens 151.2 / 118.3, rebuild and product).
     int column_groups[GEMV_MAX_GROUP];
     bool tiles = bs_tile_partials(a.I, a.M, a.n, N, K, T, column_groups);
-    for (int j = 0; j < a.n; j++) tiles = tiles && bs_aligned(a.u[j], 16);
+    for (int j = 0; j < a.n; j++) tiles = tiles && bs_aligned(a.u[j], K == 16 ? 16 : 2);
     // threads per output of the summing kernel, as behind the decode kernels (the column groups are its slots)
     int slots = 0;
     for (int j = 0; j < a.n; j++) {

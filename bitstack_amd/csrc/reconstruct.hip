@@ -38,7 +38,7 @@ constexpr int RA_MAXB = 39;    // ... of reconstruct_byte_kernel (39 x 4 KB besi
 // K16: the rank is 16 (every u fragment is one 8-byte load).  Smaller ranks pick their halves one by one behind
 // branches, and the compiler then waits for every load in flight where the branches meet: that instantiation runs
 // one pair ahead at best.
-// FLIP (rank 16): the sums of the kernel in tile.hip, bit for bit: the sum over the blocks is kept divided by the block's sign, it changes sign where two
+// FLIP (ranks 8 to 16): the sums of the kernel in tile.hip, bit for bit: the sum over the blocks is kept divided by the block's sign, it changes sign where two
 // blocks differ (a nibble's four masks come from the table instead of its four signs) and the matrix instruction adds the next product to it.  It takes the int8
 // signs, and what that kernel cannot read, of the shapes that it takes.  us, product and FMA / this: int8 signs, 14336 x 4096, 8 blocks 163 / 154, 4096 x 4096, 8
 // 45 / 42; packed signs level where rows are long (14336 x 4096, 8 blocks 69.4 / 69.8) and behind where they are not (20000 x 896, 2 blocks 13.0 / 14.1).
@@ -519,9 +519,9 @@ int launch_reconstruct(const uint8_t *packed, const int8_t *sign, const half_t *
         int rows_per_wg = (int)bs_cdiv(bs_cdiv(M, row_groups), 64) * 64;
         row_groups = (int)bs_cdiv(M, rows_per_wg);
         const size_t lds = lds_need;
-        static bs_lds_grant granted[3][BS_MAX_DEVICES];
-        const auto kernel = flip ? reconstruct_tile_kernel<PACKED, true, true> : K == 16 ? reconstruct_tile_kernel<PACKED, true, false> : reconstruct_tile_kernel<PACKED, false, false>;
-        const int st = bs_allow_lds((const void *)kernel, lds, granted[flip ? 2 : K == 16]);
+        static bs_lds_grant granted[4][BS_MAX_DEVICES];
+        const auto kernel = flip ? (K == 16 ? reconstruct_tile_kernel<PACKED, true, true> : reconstruct_tile_kernel<PACKED, false, true>) : K == 16 ? reconstruct_tile_kernel<PACKED, true, false> : reconstruct_tile_kernel<PACKED, false, false>;
+        const int st = bs_allow_lds((const void *)kernel, lds, granted[2 * flip + (K == 16)]);
         if (st != BS_OK) return st;
         dim3 grid((unsigned)bs_cdiv(strips, 8) * 8, row_groups);
         kernel<<<grid, 256, lds, s>>>(packed, sign, u, vt, w, I, M, N, K, rows_per_wg);

@@ -1,4 +1,4 @@
-// Forward for one to 48 tokens on gfx950, rank 16: the weight is rebuilt in registers, 32 x 32 outputs per matrix instruction,
+// Forward for one to 48 tokens on gfx950, rank 16 (and 8 to 15: tile_ranks.hip): the weight is rebuilt in registers, 32 x 32 outputs per matrix instruction,
 // and multiplied by x at once; it never goes to memory.
 //
 //   part[cg, t, m] = sum_{n in column group cg} x[t, n] * fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
@@ -36,12 +36,7 @@
 #include <type_traits>
 #include <utility>
 
-namespace {
-
-constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4;
-constexpr int TL_TABLE = 512, TL_HALVES = 256;      // bytes: the tables of sign masks at the start of LDS, where the one for pairs of halves begins
-constexpr int TL_LDS = 160 * 1024;
-
+constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4, TL_MIN_RANK = 8;
 struct TileMat {
     const uint8_t *packed;
     const half_t *u, *vt;
@@ -54,6 +49,21 @@ struct TileGroup {
     int n;
     float *ssq;                                     // [column groups of matrix 0][T]: sums of x^2 over the group's columns, or null
 };
+
+// The kernels for ranks 8 to 15 are the same code with a rank that is not known at compile time, in a translation unit of their own (tile_ranks.hip includes this file).  With one
+// kernel for all ranks rank 16 was up to 1.5 % slower (a step of eight sequences over two 70B-shape layers 620 / 628).
+#ifdef TILE_RANKS
+constexpr bool TL_K16 = false;
+#else
+constexpr bool TL_K16 = true;
+#endif
+// tt: token tiles of 16, 0 for the rebuild
+int bs_launch_tile_ranks(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s);
+
+namespace {
+
+constexpr int TL_TABLE = 512, TL_HALVES = 256;      // bytes: the tables of sign masks at the start of LDS, where the one for pairs of halves begins
+constexpr int TL_LDS = 160 * 1024;
 
 __device__ __forceinline__ void tl_barrier() {
     __builtin_amdgcn_sched_barrier(0);
@@ -79,6 +89,23 @@ __device__ __forceinline__ void tl_for_impl(F &&f, std::integer_sequence<int, Is
 template <int N, class F>
 __device__ __forceinline__ void tl_for(F &&f) {
     tl_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// u rows of fewer than 16 ranks (8 to 15): a row's second piece of 16 bytes is its last 16, so that both lie within it; what this leaves ahead of rank 8 goes, and zeros
+// take the places of the ranks that do not exist.
+__device__ __forceinline__ uint4_t tl_upper_ranks(const uint4_t &p, int K) {
+    uint64_t lo = p[0] | (uint64_t)p[1] << 32, hi = p[2] | (uint64_t)p[3] << 32;
+    int s = 16 * (16 - K);                          // bits: 16 to 128
+    if (s >= 64) {
+        lo = hi;
+        hi = 0;
+        s -= 64;
+    }
+    if (s > 0) {
+        lo = s < 64 ? lo >> s | hi << (64 - s) : 0;
+        hi = s < 64 ? hi >> s : 0;
+    }
+    return (uint4_t){(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }
 
 typedef const __attribute__((address_space(3))) char *lds_bytes;
@@ -118,14 +145,15 @@ struct TileKernel {
     }
 
     // A lane's piece within chunk c of a tile: chunks of 1 KB, the signs of block c / SCH first, then the u rows of the blocks
-    static __device__ __forceinline__ uint32_t piece_at(int c, int I, int lane, int cg, uint32_t row_bytes) {
+    static __device__ __forceinline__ uint32_t piece_at(int c, int I, int lane, int cg, uint32_t row_bytes, int K) {
         if (c < I * SCH) {
             const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
             return (uint32_t)r * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
         }
-        const int r = lane >> 1;
-        return (uint32_t)r * 32u + 16u * ((lane & 1) ^ ((r >> 4) & 1));
+        return (uint32_t)(lane >> 1) * (2u * K) + (second_half(lane) ? 2u * K - 16u : 0u);
     }
+    // whether the lane's piece of a u chunk is ranks 8 to 15
+    static __device__ __forceinline__ bool second_half(int lane) { return ((lane ^ (lane >> 5)) & 1) != 0; }
     // y tiles: [buffer][wave][TT token tiles][rows 0-15, 16-31][four tokens: 4][row: 16][token: 4]; floats, of wave 0
     static constexpr int Y = 16 * TT * TL_ROWS;
     static __device__ __forceinline__ int y_at(int buf, int tt, int t, int row) { return buf * (TL_WAVES * Y) + tt * 512 + row / 16 * 256 + t / 4 * 64 + row % 16 * 4 + t % 4; }
@@ -134,7 +162,8 @@ struct TileKernel {
     // counts: a branch in walk's loop leaves the compiler unsure of what is in flight, and doing the others' work on the last columns, for nobody, they took its issue
     // slots from them.  us, so / this: 13888 x 128 (half of the waves have no columns), 10 blocks, 3 tokens 11.2 / 9.6; 251 x 128, 5, 44 8.7 / 8.0; 4921 x 384, 3, 38 10.0 / 9.4.)
     static __device__ __forceinline__ void walk_without_columns(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, float *__restrict__ part, int I, int M, lds_bytes_rw lds,
-                                                                int N, int T, int cg, int rt0, int len, bool ssq, int wave, int active) {
+                                                                int N, int T, int ranks, int cg, int rt0, int len, bool ssq, int wave, int active) {
+        const int K = TL_K16 ? 16 : ranks;
         constexpr int MOST = 4;                                  // (32 chunks at most: 16 blocks of one patch)
         const int tid = threadIdx.x, lane = tid & 63, chunks = I * (SCH + 1), stage_size = stage_bytes(I), my_t = tid >> 5, my_row = tid & 31;
         const uint32_t row_bytes = (uint32_t)N >> 3;
@@ -148,15 +177,17 @@ struct TileKernel {
                 const int c = wave + TL_WAVES * q;
                 if (c >= chunks) break;
                 const bool signs = c < I * SCH;
-                const char *from = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
-                const uint32_t pitch = signs ? row_bytes : 32u;
-                ahead[k][q] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from + (int64_t)(rt * TL_ROWS) * pitch, (int)(rows * pitch)), (int)piece_at(c, I, lane, cg, row_bytes), 0, 0);
+                const char *from = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * (2 * K);
+                const uint32_t pitch = signs ? row_bytes : 2u * K;
+                ahead[k][q] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from + (int64_t)(rt * TL_ROWS) * pitch, (int)(rows * pitch)), (int)piece_at(c, I, lane, cg, row_bytes, K), 0, 0);
             }
         };
         auto write = [&](int k, int stage) {
 #pragma unroll
-            for (int q = 0; q < MOST; q++)
+            for (int q = 0; q < MOST; q++) {
+                if (K < 16 && wave + TL_WAVES * q >= I * SCH && second_half(lane)) ahead[k][q] = tl_upper_ranks(ahead[k][q], K);
                 if (wave + TL_WAVES * q < chunks) ((lds_uint4_rw)(ring + stage * stage_size + (wave + TL_WAVES * q) * 1024))[lane] = ahead[k][q];
+            }
         };
         auto sums = [&](int n) {                                 // tile n, in walk's order
 #pragma unroll
@@ -196,7 +227,8 @@ struct TileKernel {
     template <int I>
     static __device__ __forceinline__ void walk(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, const half_t *__restrict__ vt,
                                                 float *__restrict__ part, half_t *__restrict__ w, int M, lds_bytes_rw lds, const half_t *__restrict__ x,
-                                                int N, int T, int cg, int rt0, int len, float *ssq) {
+                                                int N, int T, int ranks, int cg, int rt0, int len, float *ssq) {
+        const int K = TL_K16 ? 16 : ranks;
         constexpr int STAGE = stage_bytes(I);
         constexpr int CHUNKS = I * (SCH + 1), PER = CHUNKS / TL_WAVES, MORE = CHUNKS % TL_WAVES, MOST = PER + (MORE != 0);
         int tid = threadIdx.x;
@@ -221,10 +253,10 @@ struct TileKernel {
         for (int k = 0; k < MOST; k++) {
             const int c = chunk_of(k);
             const bool signs = c < I * SCH;
-            from[k] = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * 32;
-            pitch[k] = signs ? row_bytes : 32u;
+            from[k] = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * (2 * K);
+            pitch[k] = signs ? row_bytes : 2u * K;
             from[k] += (int64_t)(rt0 * TL_ROWS) * pitch[k];
-            offset[k] = piece_at(c, I, lane, cg, row_bytes);
+            offset[k] = piece_at(c, I, lane, cg, row_bytes, K);
         }
         // A tile's pieces travel through registers: requested three tiles ahead, written to LDS at the end of the tile two ahead of it.
         int asked = rt0;                                         // the row tile `from` stands at
@@ -244,7 +276,15 @@ struct TileKernel {
                 for (int k = 0; k < MOST; k++) from[k] += pitch[k] * (uint32_t)TL_ROWS;
             }
         };
-        auto write_tile = [&](int stage, const uint4_t (&p)[MOST]) {
+        auto write_tile = [&](int stage, uint4_t (&p)[MOST]) {
+            if (K < 16) {
+#pragma unroll
+                for (int k = 0; k < MOST; k++)
+                    if (chunk_of(k) >= I * SCH) {
+                        const uint4_t q = tl_upper_ranks(p[k], K);
+                        p[k] = second_half(lane) ? q : p[k];
+                    }
+            }
 #pragma unroll
             for (int k = 0; k < MOST; k++) ((lds_uint4_rw)(ring + stage * STAGE + chunk_of(k) * 1024))[lane] = p[k];
         };
@@ -269,9 +309,16 @@ struct TileKernel {
             half8_t v[PASSES][8];
 #pragma unroll
             for (int pass = 0; pass < PASSES; pass++) {
-                const half_t *src = vt + ((int64_t)min(pass * BP + bl, I - 1) * 16 + 8 * kh) * N + n0 + 8 * piece;
+                const half_t *src = vt + (int64_t)min(pass * BP + bl, I - 1) * K * N + n0 + 8 * piece;
 #pragma unroll
-                for (int r = 0; r < 8; r++) v[pass][r] = *reinterpret_cast<const half8_t *>(src + (int64_t)r * N);
+                for (int r = 0; r < 8; r++) v[pass][r] = *reinterpret_cast<const half8_t *>(src + (int64_t)min(8 * kh + r, K - 1) * N);
+            }
+            if (K < 16) {                            // (ranks that do not exist)
+#pragma unroll
+                for (int pass = 0; pass < PASSES; pass++)
+#pragma unroll
+                    for (int r = 0; r < 8; r++)
+                        if (8 * kh + r >= K) v[pass][r] = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
             }
             // x: the columns whose weights lane group g holds when the rows are sorted out for the second product (see there)
 #pragma unroll
@@ -652,7 +699,7 @@ struct TileKernel {
 };
 
 template <int TT, bool SPLIT>
-__global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const TileGroup grp_, const half_t *__restrict__ x, int N, int T) {
+__global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const TileGroup grp_, const half_t *__restrict__ x, int N, int T, int K) {
     extern __shared__ __attribute__((aligned(1024))) char tl_lds[];
     lds_bytes_rw lds = (lds_bytes_rw)tl_lds;
     // nibble v, column j of its four (first in the top bit): the sign bit of an fp32 where the bit is set (visible behind walk's first barrier)
@@ -680,7 +727,7 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
             const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), active = patches >> (np >> 1);
             if (wave >= active) {
                 auto rest = [&](auto k) {
-                    TileKernel<TT, decltype(k)::value, SPLIT>::walk_without_columns(grp->m[j].packed, grp->m[j].u, grp->m[j].part, grp->m[j].I, grp->m[j].M, lds, N, T, cg, rt, len, ssq != nullptr, wave, active);
+                    TileKernel<TT, decltype(k)::value, SPLIT>::walk_without_columns(grp->m[j].packed, grp->m[j].u, grp->m[j].part, grp->m[j].I, grp->m[j].M, lds, N, T, K, cg, rt, len, ssq != nullptr, wave, active);
                 };
                 if (np == 4) rest(std::integral_constant<int, 4>{});
                 else if (np == 2) rest(std::integral_constant<int, 2>{});
@@ -692,7 +739,7 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     auto walk = [&](auto np, auto blocks) {
         typedef TileKernel<TT, decltype(np)::value, SPLIT> TK;
         if constexpr (decltype(blocks)::value <= TK::max_blocks())
-            TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].w, grp->m[j].M, lds, x, N, T, cg, rt, len, ssq);
+            TK::template walk<decltype(blocks)::value>(grp->m[j].packed, grp->m[j].u, grp->m[j].vt, grp->m[j].part, grp->m[j].w, grp->m[j].M, lds, x, N, T, K, cg, rt, len, ssq);
     };
     // (the narrower widths serve what the wider ones cannot hold, and short runs)
     switch (grp->m[j].np * 32 + grp->m[j].I) {
@@ -706,6 +753,23 @@ __global__ __launch_bounds__(64 * TL_WAVES, 2) void tile_forward_kernel(const Ti
     }
 }
 
+template <int TT, bool SPLIT = false>
+int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, hipStream_t s) {
+    size_t lds = 0;
+    for (int j = 0; j < grp.n; j++) {
+        const int np = grp.m[j].np, I = grp.m[j].I;
+        const size_t b = np == 4 ? TileKernel<TT, 4>::lds_size(I) : np == 2 ? TileKernel<TT, 2>::lds_size(I) : TileKernel<TT, 1>::lds_size(I);
+        if (b > lds) lds = b;
+    }
+    static bs_lds_grant granted[BS_MAX_DEVICES];
+    const int st = bs_allow_lds((const void *)tile_forward_kernel<TT, SPLIT>, lds, granted);
+    if (st != BS_OK) return st;
+    tile_forward_kernel<TT, SPLIT><<<grid, 64 * TL_WAVES, lds, s>>>(grp, x, N, T, K);
+    BS_LAUNCH_CHECK();
+    return BS_OK;
+}
+
+#ifndef TILE_RANKS
 // Per matrix the width of its column groups (256 np columns) and how many workgroups share the row tiles of one.  The estimate behind it
 // (cycles): a tile costs 1300 + 250 per block and np (with one patch per wave, a chain of mask, product, mask, 420 per block), a
 // workgroup's start 2000 + 560 per block and np.
@@ -827,33 +891,25 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
     return best;
 }
 
-template <int TT, bool SPLIT = false>
-int launch_tile(const TileGroup &grp, int grid, const half_t *x, int N, int T, hipStream_t s) {
-    size_t lds = 0;
-    for (int j = 0; j < grp.n; j++) {
-        const int np = grp.m[j].np, I = grp.m[j].I;
-        const size_t b = np == 4 ? TileKernel<TT, 4>::lds_size(I) : np == 2 ? TileKernel<TT, 2>::lds_size(I) : TileKernel<TT, 1>::lds_size(I);
-        if (b > lds) lds = b;
-    }
-    static bs_lds_grant granted[BS_MAX_DEVICES];
-    const int st = bs_allow_lds((const void *)tile_forward_kernel<TT, SPLIT>, lds, granted);
-    if (st != BS_OK) return st;
-    tile_forward_kernel<TT, SPLIT><<<grid, 64 * TL_WAVES, lds, s>>>(grp, x, N, T);
-    BS_LAUNCH_CHECK();
-    return BS_OK;
-}
-
 TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
     TilePlan none;
     none.grid = 0;
-    if (n < 1 || n > TL_GROUP || K != 16 || T < 0 || T > 48 || N < SF_COLS || N % SF_COLS != 0) return none;
+    if (n < 1 || n > TL_GROUP || K < TL_MIN_RANK || K > 16 || T < 0 || T > 48 || N < SF_COLS || N % SF_COLS != 0) return none;
     for (int j = 0; j < n; j++)
         // a block's sign and u rows, and 16 tokens of partial sums, lie within 32-bit byte offsets
         if (I[j] < 1 || M[j] < 1 || (int64_t)M[j] * (N >> 3) >= ((int64_t)1 << 32) || (int64_t)M[j] * 64 >= ((int64_t)1 << 32)) return none;
     return bs_cdiv(N, 256) <= 1024 ? make_tile_plan(I, M, n, N, T) : none;
 }
+#endif
 
 }  // namespace
+
+#ifdef TILE_RANKS
+int bs_launch_tile_ranks(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s) {
+    return tt == 0 ? launch_tile<0>(grp, grid, x, N, T, K, s) : tt == 1 ? launch_tile<1>(grp, grid, x, N, T, K, s)
+           : tt == 2 ? launch_tile<2>(grp, grid, x, N, T, K, s) : launch_tile<3>(grp, grid, x, N, T, K, s);
+}
+#else
 
 // Column groups (partial sums per output) of every matrix, if this kernel takes them; cycles: of its busiest workgroup, by the plan's estimate.
 bool bs_tile_partials(const int *I, const int *M, int n, int N, int K, int T, int *groups, double *cycles) {
@@ -883,20 +939,21 @@ int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *cons
     grp.ssq = ssq;
     int first = 0;
     for (int j = 0; j < n; j++) {
-        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], 16)) return BS_ERR_SHAPE;
+        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], K == 16 ? 16 : 2)) return BS_ERR_SHAPE;
         grp.m[j] = TileMat{packed[j], u[j], vt[j], part[j], nullptr, I[j], M[j], p.np[j], (int)bs_cdiv(M[j], TL_ROWS), first, p.wgs[j]};
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
-    if (split) return launch_tile<1, true>(grp, p.grid, x, N, T, s);
-    return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, s) : launch_tile<3>(grp, p.grid, x, N, T, s);
+    if (K != 16) return split ? BS_ERR_SHAPE : bs_launch_tile_ranks(grp, p.grid, x, N, T, K, (int)bs_cdiv(T, 16), s);
+    if (split) return launch_tile<1, true>(grp, p.grid, x, N, T, K, s);
+    return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, K, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, K, s) : launch_tile<3>(grp, p.grid, x, N, T, K, s);
 }
 
 // The weights of n <= 4 matrices with the same columns, w[j] f16 [M[j], N]; BS_ERR_SHAPE: not taken, nothing was enqueued.
 int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *const *u, const half_t *const *vt, const int *I, const int *M,
                            half_t *const *w, int N, int K, hipStream_t s) {
     for (int j = 0; j < n && j < TL_GROUP; j++)
-        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], 16) || !bs_aligned(w[j], 16)) return BS_ERR_SHAPE;
+        if (!bs_aligned(packed[j], 16) || !bs_aligned(vt[j], 16) || !bs_aligned(u[j], K == 16 ? 16 : 2) || !bs_aligned(w[j], 16)) return BS_ERR_SHAPE;
     const TilePlan p = checked_plan(I, M, n, N, K, 0);
     if (p.grid == 0) return BS_ERR_SHAPE;
     TileGroup grp;
@@ -908,5 +965,6 @@ int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *co
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
-    return launch_tile<0>(grp, p.grid, nullptr, N, 0, s);
+    return K == 16 ? launch_tile<0>(grp, p.grid, nullptr, N, 0, K, s) : bs_launch_tile_ranks(grp, p.grid, nullptr, N, 0, K, 0, s);
 }
+#endif

@@ -80,7 +80,7 @@ __device__ __forceinline__ void phase_barrier() {
 template <int P, int Q, bool SWAP, int S, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     const half_t *__restrict__ x, const half_t *__restrict__ w, const half_t *__restrict__ bias,
-    half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide) {
+    half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide, int spread) {
     static_assert((SWAP ? P : Q) % 2 == 0, "feature fragments come in pairs");
     constexpr int BP = 32 * P, BQ = 64 * Q;   // P, Q: 16-row fragments of a wave
     constexpr int BT = SWAP ? BQ : BP, BF = SWAP ? BP : BQ;
@@ -148,13 +148,15 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
         const int r = qrow + 8 * j + (lane >> 3);
         voff_q[j] = (uint32_t)min(r, q_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(!SWAP, r));
     }
+    // (spread: see launch_pipe)
+    const int ahead = !SPLIT && spread ? (int)(((int64_t)(blockIdx.x & 7) * steps) >> 3) : 0;
     auto request_p = [&](auto stage, int step_, int j) {
         half_t *dst = p_stage(stage) + prow[j] * PK;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], min(step_, steps - 1) * (PK * 2), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], (min(step_, steps - 1) + ahead - (min(step_, steps - 1) + ahead < steps ? 0 : steps)) * (PK * 2), 0, 0);
     };
     auto request_q = [&](auto stage, int step_, int j) {
         half_t *dst = q_stage(stage) + (qrow + 8 * j) * PK;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], min(step_, steps - 1) * (PK * 2), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], (min(step_, steps - 1) + ahead - (min(step_, steps - 1) + ahead < steps ? 0 : steps)) * (PK * 2), 0, 0);
     };
 
     float4_t acc[P][Q];
@@ -378,13 +380,17 @@ int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y,
     const int steps = (int)bs_cdiv(N / PK, splits);
     splits = (int)bs_cdiv(N / PK, steps);     // every part holds at least one k-step
     const int wide = M % 8 == 0 && bs_aligned(y, 16) && bs_aligned(part, 16);
+    // A few hundred tokens on a weight beyond the L2s: every XCD starts an eighth of the rows further than the one before, so that they do not all ask the same memory channels
+    // (its own workgroups still share their lines).  us of a call, all from the first column / so: 14336 x 4096, 4 blocks, 300 tokens 89.6 / 84.7, 4096 x 4096, 4, 300 43.7 / 41.5, 28672 x
+    // 8192, 2, 300 256 / 250; but 1024 x 4096, 4, 300 24.3 / 25.1, 6144 x 4096, 4, 1400 85.2 / 86.5.
+    const int spread = T <= 512 && (int64_t)M * N >= (16 << 20);
     const bool two = S_TWO != S && (int64_t)tiles * splits > 256;
     if (splits == 1) {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
-        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide, spread);
+        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide, spread);
     } else {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
-        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide, spread);
+        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide, spread);
         BS_LAUNCH_CHECK();
         const int64_t total = (int64_t)T * M;
         if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, splits, total, M);

@@ -1,4 +1,4 @@
-// Forward for 49 to 128 tokens on gfx950, rank 16 (and 8 to 15: column_ranks.hip), up to 8 blocks: the tile kernel's rebuild (tile.hip) with the loops turned round.
+// Forward for 49 to 128 tokens on gfx950, rank 16 (and 4 to 15: column_ranks.hip), up to 8 blocks: the tile kernel's rebuild (tile.hip) with the loops turned round.
 //
 //   part[cg, t, m] = sum_{n in column group cg} x[t, n] * fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
 //
@@ -31,7 +31,7 @@ struct ColumnMat {
     int M, row_groups, spans;                       // spans of 256 columns per column group
 };
 
-// The kernels for ranks 8 to 15 are the same code with a rank that is not known at compile time, in a translation unit of their own (column_ranks.hip includes this file): with
+// The kernels for ranks 4 to 15 are the same code with a rank that is not known at compile time, in a translation unit of their own (column_ranks.hip includes this file): with
 // one kernel for all ranks 14336 x 4096, 5 blocks, 100 tokens took 57.3 us for 55.0.
 #ifdef COLUMN_RANKS
 constexpr bool CL_K16 = false;
@@ -55,6 +55,7 @@ __device__ __forceinline__ void cl_for(F &&f) {
 }
 
 typedef half8_t cl_half8_any __attribute__((aligned(2)));
+typedef half4_t cl_half4_any __attribute__((aligned(2)));
 typedef __attribute__((address_space(3))) char *cl_bytes;
 typedef const __attribute__((address_space(3))) half8_t *cl_half8;
 typedef __attribute__((address_space(3))) half8_t *cl_half8_rw;
@@ -96,11 +97,17 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
     };
 #pragma unroll
     for (int i = 0; i < I; i++) {
-        uf[i] = *reinterpret_cast<const cl_half8_any *>(mat.u + ((int64_t)i * M + my_row) * K + (h ? K - 8 : 0));     // (fewer than 16 ranks: the row's last eight)
+        const half_t *ur = mat.u + ((int64_t)i * M + my_row) * K;
+        if (K >= 8) {
+            uf[i] = *reinterpret_cast<const cl_half8_any *>(ur + (h ? K - 8 : 0));       // (fewer than 16 ranks: the row's last eight)
+        } else {
+            const half4_t a = *reinterpret_cast<const cl_half4_any *>(ur), b = *reinterpret_cast<const cl_half4_any *>(ur + K - 4);
+            uf[i] = (half8_t){a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};           // (fewer than 8: its first and last four)
+        }
         request_signs(i, first);
     }
 
-    if (K < 16) {                                   // ranks 8 to K - 1 first, zeros behind them
+    if (K < 16) {                                   // ranks in their places, zeros in those of the ones that do not exist
 #pragma unroll
         for (int i = 0; i < I; i++) {
             half8_t o = uf[i];
@@ -108,8 +115,8 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
             for (int e = 0; e < 8; e++) {
 #pragma unroll
                 for (int d = 0; d < 8; d++)
-                    if (h && d == e + 16 - K) o[e] = uf[i][d];
-                if (h && 8 + e >= K) o[e] = (half_t)0;
+                    if (K >= 8 ? h && d == e + 16 - K : e >= 4 && d == e + 8 - K) o[e] = uf[i][d];
+                if (8 * h + e >= K) o[e] = (half_t)0;
             }
             uf[i] = o;
         }
@@ -333,7 +340,7 @@ constexpr int64_t CL_MIN_WEIGHTS = 11ll << 20;
 
 // Column groups (partial sums per output) when this kernel takes the shape, else 0.
 int bs_column_partials(int I, int M, int N, int K, int T) {
-    if (bs_prefill_mode() != 0 || K < 8 || K > 16 || I < 1 || T < CL_MIN_T || T > CL_MAX_T || I > max_blocks(token_tiles(T)) || M < 1 || N < SF_COLS || N % SF_COLS != 0) return 0;
+    if (bs_prefill_mode() != 0 || K < 4 || K > 16 || I < 1 || T < CL_MIN_T || T > CL_MAX_T || I > max_blocks(token_tiles(T)) || M < 1 || N < SF_COLS || N % SF_COLS != 0) return 0;
     if ((int64_t)M * N < CL_MIN_WEIGHTS || (int64_t)M * (N >> 3) >= ((int64_t)1 << 32)) return 0;       // a row's signs within a 32-bit byte offset
     return make_column_plan(M, N).groups;
 }

@@ -1100,8 +1100,8 @@ int launch_group_strips(const GroupArgs &a, int N, int K, const half_t *x, int T
     r.n_in = N;
     r.eps = eps;
     float *parts[GEMV_MAX_GROUP];
-    // The tile kernel (from 49 tokens the column kernel) where it takes the matrices; the strip and panel kernels for ranks below 8, long stacks, small matrices and, at rank 16, u
-    // off a 16-byte boundary.  Ranks 8 to 15 have a build of their own of both (us, strip, walked or panel kernel / that, rank 12: 28672 x 8192, 3 blocks, 8 tokens 102.2 / 60.5, 40 tokens 154 / 124;
+    // The tile kernel (from 49 tokens the column kernel) where it takes the matrices; the strip and panel kernels for ranks below 4, long stacks, small matrices and, at rank 16, u
+    // off a 16-byte boundary.  Ranks 4 to 15 have builds of their own of both (us, strip, walked or panel kernel / that, rank 12: 28672 x 8192, 3 blocks, 8 tokens 102.2 / 60.5, 40 tokens 154 / 124;
     // 14336 x 4096, 8, 8 tokens 69.0 / 43.4; 5, 100 tokens 77.6 / 58.4; 5000 x 4096, 6, 37 tokens 39.4 / 27.7; 4096 x 14336, 8, 509 tokens 151.2 / 118.3, rebuild and product).
     int column_groups[GEMV_MAX_GROUP];
     bool tiles = bs_tile_partials(a.I, a.M, a.n, N, K, T, column_groups);

@@ -38,7 +38,7 @@ constexpr int RA_MAXB = 39;    // ... of reconstruct_byte_kernel (39 x 4 KB besi
 // K16: the rank is 16 (every u fragment is one 8-byte load).  Smaller ranks pick their halves one by one behind
 // branches, and the compiler then waits for every load in flight where the branches meet: that instantiation runs
 // one pair ahead at best.
-// FLIP (ranks 8 to 16): the sums of the kernel in tile.hip, bit for bit: the sum over the blocks is kept divided by the block's sign, it changes sign where two
+// FLIP (ranks 4 to 16): the sums of the kernel in tile.hip, bit for bit: the sum over the blocks is kept divided by the block's sign, it changes sign where two
 // blocks differ (a nibble's four masks come from the table instead of its four signs) and the matrix instruction adds the next product to it.  It takes the int8
 // signs, and what that kernel cannot read, of the shapes that it takes.  us, product and FMA / this: int8 signs, 14336 x 4096, 8 blocks 163 / 154, 4096 x 4096, 8
 // 45 / 42; packed signs level where rows are long (14336 x 4096, 8 blocks 69.4 / 69.8) and behind where they are not (20000 x 896, 2 blocks 13.0 / 14.1).

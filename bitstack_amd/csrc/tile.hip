@@ -1,4 +1,4 @@
-// Forward for one to 48 tokens on gfx950, rank 16 (and 8 to 15: tile_ranks.hip): the weight is rebuilt in registers, 32 x 32 outputs per matrix instruction,
+// Forward for one to 48 tokens on gfx950, rank 16 (and 4 to 15: tile_ranks.hip, tile_few_ranks.hip): the weight is rebuilt in registers, 32 x 32 outputs per matrix instruction,
 // and multiplied by x at once; it never goes to memory.
 //
 //   part[cg, t, m] = sum_{n in column group cg} x[t, n] * fp16( sum_i s_i[m, n] * sum_r u_i[m, r] * vt_i[r, n] )
@@ -36,7 +36,7 @@
 #include <type_traits>
 #include <utility>
 
-constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4, TL_MIN_RANK = 8;
+constexpr int TL_WAVES = 8, TL_ROWS = 32, TL_GROUP = 4, TL_MIN_RANK = 4;
 struct TileMat {
     const uint8_t *packed;
     const half_t *u, *vt;
@@ -50,15 +50,16 @@ struct TileGroup {
     float *ssq;                                     // [column groups of matrix 0][T]: sums of x^2 over the group's columns, or null
 };
 
-// The kernels for ranks 8 to 15 are the same code with a rank that is not known at compile time, in a translation unit of their own (tile_ranks.hip includes this file).  With one
-// kernel for all ranks rank 16 was up to 1.5 % slower (a step of eight sequences over two 70B-shape layers 620 / 628).
+// The kernels for ranks 4 to 15 are the same code with a rank that is not known at compile time, in translation units of their own that include this file: tile_ranks.hip (8 to 15) and
+// tile_few_ranks.hip (4 to 7).  With one kernel for all ranks rank 16 was up to 1.5 % slower (a step of eight sequences over two 70B-shape layers 620 / 628).
 #ifdef TILE_RANKS
-constexpr bool TL_K16 = false;
+constexpr int TL_RANKS = TILE_RANKS;                // the least rank of this build
 #else
-constexpr bool TL_K16 = true;
+constexpr int TL_RANKS = 16;
 #endif
 // tt: token tiles of 16, 0 for the rebuild
 int bs_launch_tile_ranks(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s);
+int bs_launch_tile_few_ranks(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s);
 
 namespace {
 
@@ -91,21 +92,36 @@ __device__ __forceinline__ void tl_for(F &&f) {
     tl_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// u rows of fewer than 16 ranks (8 to 15): a row's second piece of 16 bytes is its last 16, so that both lie within it; what this leaves ahead of rank 8 goes, and zeros
-// take the places of the ranks that do not exist.
-__device__ __forceinline__ uint4_t tl_upper_ranks(const uint4_t &p, int K) {
+// A row of u has fewer than 16 ranks: its pieces are read so that they lie within it, what this leaves ahead of a piece's first rank goes, and zeros take the places of the
+// ranks that do not exist.  8 to 15: the second piece of 16 bytes is the row's last 16.  4 to 7: a piece is two of 8 bytes, the row's first and its last; the second piece is nothing.
+__device__ __forceinline__ uint4_t tl_ranks(const uint4_t &p, bool second, int K) {
     uint64_t lo = p[0] | (uint64_t)p[1] << 32, hi = p[2] | (uint64_t)p[3] << 32;
-    int s = 16 * (16 - K);                          // bits: 16 to 128
-    if (s >= 64) {
-        lo = hi;
-        hi = 0;
-        s -= 64;
+    if constexpr (TL_RANKS == 8) {
+        int s = 16 * (16 - K);                      // bits: 16 to 128
+        if (s >= 64) {
+            lo = hi;
+            hi = 0;
+            s -= 64;
+        }
+        if (s > 0) {
+            lo = s < 64 ? lo >> s | hi << (64 - s) : 0;
+            hi = s < 64 ? hi >> s : 0;
+        }
+        const uint4_t q = {(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+        return second ? q : p;
+    } else {
+        hi = K == 4 ? 0 : hi >> (16 * (8 - K));
+        const uint4_t q = {(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+        return second ? (uint4_t){0, 0, 0, 0} : q;
     }
-    if (s > 0) {
-        lo = s < 64 ? lo >> s | hi << (64 - s) : 0;
-        hi = s < 64 ? hi >> s : 0;
+}
+// 16 bytes of a chunk; ranks 4 to 7: two of 8, the second one `apart` behind the first
+__device__ __forceinline__ uint4_t tl_load(__amdgpu_buffer_rsrc_t r, int at, int apart) {
+    if constexpr (TL_RANKS >= 8) return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
+    else {
+        const uint2_t a = __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0), b = __builtin_amdgcn_raw_buffer_load_b64(r, at + apart, 0, 0);
+        return (uint4_t){a[0], a[1], b[0], b[1]};
     }
-    return (uint4_t){(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }
 
 typedef const __attribute__((address_space(3))) char *lds_bytes;
@@ -150,7 +166,7 @@ struct TileKernel {
             const int r = (c % SCH) * (64 / RP) + lane / RP, piece = (lane % RP) ^ swizzle(r);
             return (uint32_t)r * row_bytes + min((uint32_t)(cg * SROW + piece * 16), row_bytes - 16u);
         }
-        return (uint32_t)(lane >> 1) * (2u * K) + (second_half(lane) ? 2u * K - 16u : 0u);
+        return (uint32_t)(lane >> 1) * (2u * K) + (TL_RANKS >= 8 && second_half(lane) ? 2u * K - 16u : 0u);
     }
     // whether the lane's piece of a u chunk is ranks 8 to 15
     static __device__ __forceinline__ bool second_half(int lane) { return ((lane ^ (lane >> 5)) & 1) != 0; }
@@ -163,7 +179,7 @@ struct TileKernel {
     // slots from them.  us, so / this: 13888 x 128 (half of the waves have no columns), 10 blocks, 3 tokens 11.2 / 9.6; 251 x 128, 5, 44 8.7 / 8.0; 4921 x 384, 3, 38 10.0 / 9.4.)
     static __device__ __forceinline__ void walk_without_columns(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, float *__restrict__ part, int I, int M, lds_bytes_rw lds,
                                                                 int N, int T, int ranks, int cg, int rt0, int len, bool ssq, int wave, int active) {
-        const int K = TL_K16 ? 16 : ranks;
+        const int K = TL_RANKS == 16 ? 16 : ranks;
         constexpr int MOST = 4;                                  // (32 chunks at most: 16 blocks of one patch)
         const int tid = threadIdx.x, lane = tid & 63, chunks = I * (SCH + 1), stage_size = stage_bytes(I), my_t = tid >> 5, my_row = tid & 31;
         const uint32_t row_bytes = (uint32_t)N >> 3;
@@ -179,13 +195,13 @@ struct TileKernel {
                 const bool signs = c < I * SCH;
                 const char *from = signs ? reinterpret_cast<const char *>(packed) + (int64_t)(c / SCH) * M * row_bytes : reinterpret_cast<const char *>(u) + (int64_t)(c - I * SCH) * M * (2 * K);
                 const uint32_t pitch = signs ? row_bytes : 2u * K;
-                ahead[k][q] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from + (int64_t)(rt * TL_ROWS) * pitch, (int)(rows * pitch)), (int)piece_at(c, I, lane, cg, row_bytes, K), 0, 0);
+                ahead[k][q] = tl_load(tl_buffer(from + (int64_t)(rt * TL_ROWS) * pitch, (int)(rows * pitch)), (int)piece_at(c, I, lane, cg, row_bytes, K), signs ? 8 : 2 * K - 8);
             }
         };
         auto write = [&](int k, int stage) {
 #pragma unroll
             for (int q = 0; q < MOST; q++) {
-                if (K < 16 && wave + TL_WAVES * q >= I * SCH && second_half(lane)) ahead[k][q] = tl_upper_ranks(ahead[k][q], K);
+                if (TL_RANKS < 16 && wave + TL_WAVES * q >= I * SCH) ahead[k][q] = tl_ranks(ahead[k][q], second_half(lane), K);
                 if (wave + TL_WAVES * q < chunks) ((lds_uint4_rw)(ring + stage * stage_size + (wave + TL_WAVES * q) * 1024))[lane] = ahead[k][q];
             }
         };
@@ -228,7 +244,7 @@ struct TileKernel {
     static __device__ __forceinline__ void walk(const uint8_t *__restrict__ packed, const half_t *__restrict__ u, const half_t *__restrict__ vt,
                                                 float *__restrict__ part, half_t *__restrict__ w, int M, lds_bytes_rw lds, const half_t *__restrict__ x,
                                                 int N, int T, int ranks, int cg, int rt0, int len, float *ssq) {
-        const int K = TL_K16 ? 16 : ranks;
+        const int K = TL_RANKS == 16 ? 16 : ranks;
         constexpr int STAGE = stage_bytes(I);
         constexpr int CHUNKS = I * (SCH + 1), PER = CHUNKS / TL_WAVES, MORE = CHUNKS % TL_WAVES, MOST = PER + (MORE != 0);
         int tid = threadIdx.x;
@@ -267,7 +283,7 @@ struct TileKernel {
             const uint32_t rows = min(M - asked * TL_ROWS, TL_ROWS);
 #pragma unroll
             for (int k = 0; k < MOST; k++) {
-                to[k] = __builtin_amdgcn_raw_buffer_load_b128(tl_buffer(from[k], (int)(rows * pitch[k])), (int)offset[k], 0, 0);
+                to[k] = tl_load(tl_buffer(from[k], (int)(rows * pitch[k])), (int)offset[k], chunk_of(k) < I * SCH ? 8 : 2 * K - 8);
                 __builtin_amdgcn_sched_barrier(0);               // (in the same order wherever they are issued: the waits count on it)
             }
             if (asked < last_rt) {
@@ -277,13 +293,10 @@ struct TileKernel {
             }
         };
         auto write_tile = [&](int stage, uint4_t (&p)[MOST]) {
-            if (K < 16) {
+            if constexpr (TL_RANKS < 16) {
 #pragma unroll
                 for (int k = 0; k < MOST; k++)
-                    if (chunk_of(k) >= I * SCH) {
-                        const uint4_t q = tl_upper_ranks(p[k], K);
-                        p[k] = second_half(lane) ? q : p[k];
-                    }
+                    if (chunk_of(k) >= I * SCH) p[k] = tl_ranks(p[k], second_half(lane), K);
             }
 #pragma unroll
             for (int k = 0; k < MOST; k++) ((lds_uint4_rw)(ring + stage * STAGE + chunk_of(k) * 1024))[lane] = p[k];
@@ -313,7 +326,7 @@ struct TileKernel {
 #pragma unroll
                 for (int r = 0; r < 8; r++) v[pass][r] = *reinterpret_cast<const half8_t *>(src + (int64_t)min(8 * kh + r, K - 1) * N);
             }
-            if (K < 16) {                            // (ranks that do not exist)
+            if constexpr (TL_RANKS < 16) {           // (ranks that do not exist)
 #pragma unroll
                 for (int pass = 0; pass < PASSES; pass++)
 #pragma unroll
@@ -823,7 +836,7 @@ TilePlan tile_plan_up_to(int widest, const int *I, const int *M, int n, int N, i
     p.cost = run(worst) * bs_cdiv(grid, 256);
     return p;
 }
-TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
+TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int K, int T) {
     TilePlan best;
     best.grid = 0;
     for (int widest = 4; widest >= 1; widest >>= 1) {
@@ -843,6 +856,9 @@ TilePlan make_tile_plan(const int *I, const int *M, int n, int N, int T) {
         const bool wide = best.np[0] == 2 && (T > 4 || N % 512 != 0);
         const long steps = best.np[0] == 1 || I[0] <= 2 || wide ? bs_strip_steps(I[0], M[0], N, T) : 0;
         if ((best.np[0] == 1 && tiles * 0.75 > (double)steps) || ((I[0] <= 2 || wide) && tiles == 1 && steps == 1)) best.grid = 0;
+        // (below rank 8 one tile of three blocks is behind too: 2675 x 768, 5 tokens, rank 4 8.3 / 9.1, 414 x 768, 48, rank 5 8.5 / 9.1, 930 x 384, 24, rank 5 7.9 / 8.1; of 150 drawn calls
+        // of ranks 4 to 15, up to 9000 x 7680, the others are at most 5 % behind, 6 % ahead on average)
+        if (K < 8 && I[0] <= 3 && tiles == 1) best.grid = 0;
     }
     // Several matrices.  When not even one workgroup each fits the chip at once, the second round is the whole call again (10, 9, 1 and 3 blocks of 733, 968, 7844
     // and 215 x 19456, 40 tokens, us strip / this 126 / 253; 118 such groups of 26,000 drawn ones: 0.74 of the strip kernel's rate).  With one patch per
@@ -898,14 +914,14 @@ TilePlan checked_plan(const int *I, const int *M, int n, int N, int K, int T) {
     for (int j = 0; j < n; j++)
         // a block's sign and u rows, and 16 tokens of partial sums, lie within 32-bit byte offsets
         if (I[j] < 1 || M[j] < 1 || (int64_t)M[j] * (N >> 3) >= ((int64_t)1 << 32) || (int64_t)M[j] * 64 >= ((int64_t)1 << 32)) return none;
-    return bs_cdiv(N, 256) <= 1024 ? make_tile_plan(I, M, n, N, T) : none;
+    return bs_cdiv(N, 256) <= 1024 ? make_tile_plan(I, M, n, N, K, T) : none;
 }
 #endif
 
 }  // namespace
 
 #ifdef TILE_RANKS
-int bs_launch_tile_ranks(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s) {
+int TILE_LAUNCH(const TileGroup &grp, int grid, const half_t *x, int N, int T, int K, int tt, hipStream_t s) {
     return tt == 0 ? launch_tile<0>(grp, grid, x, N, T, K, s) : tt == 1 ? launch_tile<1>(grp, grid, x, N, T, K, s)
            : tt == 2 ? launch_tile<2>(grp, grid, x, N, T, K, s) : launch_tile<3>(grp, grid, x, N, T, K, s);
 }
@@ -944,7 +960,7 @@ int bs_launch_tile_group(int n, const uint8_t *const *packed, const half_t *cons
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
-    if (K != 16) return split ? BS_ERR_SHAPE : bs_launch_tile_ranks(grp, p.grid, x, N, T, K, (int)bs_cdiv(T, 16), s);
+    if (K != 16) return split ? BS_ERR_SHAPE : (K < 8 ? bs_launch_tile_few_ranks : bs_launch_tile_ranks)(grp, p.grid, x, N, T, K, (int)bs_cdiv(T, 16), s);
     if (split) return launch_tile<1, true>(grp, p.grid, x, N, T, K, s);
     return T <= 16 ? launch_tile<1>(grp, p.grid, x, N, T, K, s) : T <= 32 ? launch_tile<2>(grp, p.grid, x, N, T, K, s) : launch_tile<3>(grp, p.grid, x, N, T, K, s);
 }
@@ -965,6 +981,6 @@ int bs_launch_tile_rebuild(int n, const uint8_t *const *packed, const half_t *co
         first += p.wgs[j] * p.groups[j];
     }
     for (int j = n; j < TL_GROUP; j++) grp.m[j] = grp.m[0];
-    return K == 16 ? launch_tile<0>(grp, p.grid, nullptr, N, 0, K, s) : bs_launch_tile_ranks(grp, p.grid, nullptr, N, 0, K, 0, s);
+    return K == 16 ? launch_tile<0>(grp, p.grid, nullptr, N, 0, K, s) : (K < 8 ? bs_launch_tile_few_ranks : bs_launch_tile_ranks)(grp, p.grid, nullptr, N, 0, K, 0, s);
 }
 #endif

@@ -186,7 +186,7 @@ int bs_decode_kernel(int I, int M, int N, int K, int T);
 #define BS_PATH_REBUILD    0   /* weight rebuilt into the workspace, then the dense product */
 #define BS_PATH_DECODE_F16 1   /* packed-sign GEMV on fp16 MFMA, 1..4 tokens per pass: gemv_sparse_kernel or gemv_kernel (bs_sparse_kernel; 3 and 4 on large matrices: tile_forward_kernel) */
 #define BS_PATH_DECODE_MX  2   /* gemv_mx_kernel: the same on the block-scaled fp4 x fp6 MFMA, 1..2 tokens */
-#define BS_PATH_STRIP      3   /* up to 48 tokens, patches rebuilt in registers: tile_forward_kernel from rank 8, strip_forward_kernel elsewhere */
+#define BS_PATH_STRIP      3   /* up to 48 tokens, patches rebuilt in registers: tile_forward_kernel from rank 4, strip_forward_kernel elsewhere */
 #define BS_PATH_WALKED     4   /* strip_wide_kernel: 49..96 tokens, strips walked by 128-row workgroups (large matrices: column_forward_kernel) */
 #define BS_PATH_PANEL      5   /* panel_forward_kernel: up to 128 tokens, W tiles decoded into LDS (large matrices: column_forward_kernel) */
 int bs_forward_path(int I, int M, int N, int K, int T);
@@ -210,8 +210,8 @@ int bs_tile_kernel(const int *I, const int *M, int n, int N, int K, int T, int *
 
 /*
  * The same for ranks below 16 (BS_TILE_NONE at 16, as bs_tile_kernel answers below it): the
- * tile and column kernels have a build of their own for ranks 8 to 15, which serves the
- * calls that rank 16 would run on them, but for those with the weight in two terms, and takes u on any
+ * tile and column kernels have builds of their own for ranks 4 to 15, which serve the
+ * calls that rank 16 would run on them, but for those with the weight in two terms, and take u on any
  * address that bs_forward takes.
  */
 int bs_small_rank_kernel(const int *I, const int *M, int n, int N, int K, int T, int *columns);

@@ -150,13 +150,18 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     }
     // (spread: see launch_pipe)
     const int ahead = !SPLIT && spread ? (int)(((int64_t)(blockIdx.x & 7) * steps) >> 3) : 0;
-    auto request_p = [&](auto stage, int step_, int j) {
-        half_t *dst = p_stage(stage) + prow[j] * PK;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], (min(step_, steps - 1) + ahead - (min(step_, steps - 1) + ahead < steps ? 0 : steps)) * (PK * 2), 0, 0);
+    // where a step's columns are in the rows, in bytes (steps behind the last: the last again)
+    auto column_of = [&](int step_) {
+        const int c = min(step_, steps - 1) + ahead;
+        return (c < steps ? c : c - steps) * (PK * 2);
     };
-    auto request_q = [&](auto stage, int step_, int j) {
+    auto request_p = [&](auto stage, int column, int j) {
+        half_t *dst = p_stage(stage) + prow[j] * PK;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], column, 0, 0);
+    };
+    auto request_q = [&](auto stage, int column, int j) {
         half_t *dst = q_stage(stage) + (qrow + 8 * j) * PK;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], (min(step_, steps - 1) + ahead - (min(step_, steps - 1) + ahead < steps ? 0 : steps)) * (PK * 2), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_ptr)dst, 16, (int)voff_q[j], column, 0, 0);
     };
 
     float4_t acc[P][Q];
@@ -193,12 +198,14 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
                                  : __builtin_amdgcn_mfma_f32_16x16x32_f16(fq[q >> 1][j], fp[q >> 1][i], acc[i][j], 0, 0, 0);
     };
     auto all_q = [&](auto stage, int step_) {
+        const int column = column_of(step_);
 #pragma unroll
-        for (int j = 0; j < QJ; j++) request_q(stage, step_, j);
+        for (int j = 0; j < QJ; j++) request_q(stage, column, j);
     };
     auto all_p = [&](auto stage, int step_) {
+        const int column = column_of(step_);
 #pragma unroll
-        for (int j = 0; j < PJ; j++) request_p(stage, step_, j);
+        for (int j = 0; j < PJ; j++) request_p(stage, column, j);
     };
     // steps 0 .. `steps` - 1, S at a time (no exit between them: a path around one would make the compiler wait for the wrong requests at the top of the loop)
     auto walk = [&](auto &&step) {
@@ -229,10 +236,11 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
             wait_lds();
             phase_barrier();
             // MATRIX(s)
+            const int column = column_of(s + S);
             __builtin_amdgcn_s_setprio(1);
             static_for<4>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                if constexpr (q < PJ) request_p(stage, s + S, q);
+                if constexpr (q < PJ) request_p(stage, column, q);
                 mfmas(q);
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -257,6 +265,7 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
             wait_requests<PJ + (S - 2) * (PJ + QJ)>();         // the Q rows of step s + 1
             phase_barrier();
             // MATRIX(s)
+            const int column = column_of(s + S);
             __builtin_amdgcn_s_setprio(1);
             static_for<4>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
@@ -264,8 +273,8 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
                 static_for<PJ + QJ>([&](auto jc) {
                     constexpr int j = decltype(jc)::value;
                     if constexpr (j * 4 / (PJ + QJ) == q) {
-                        if constexpr (j < QJ) request_q(stage, s + S, j);
-                        else request_p(stage, s + S, j - QJ);
+                        if constexpr (j < QJ) request_q(stage, column, j);
+                        else request_p(stage, column, j - QJ);
                     }
                 });
                 mfmas(q);

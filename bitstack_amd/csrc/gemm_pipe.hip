@@ -148,8 +148,8 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
         const int r = qrow + 8 * j + (lane >> 3);
         voff_q[j] = (uint32_t)min(r, q_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(!SWAP, r));
     }
-    // (spread: see launch_pipe)
-    const int ahead = !SPLIT && spread ? (int)(((int64_t)(blockIdx.x & 7) * steps) >> 3) : 0;
+    // (spread: see launch_pipe; not in 256 x 256, where 512 tokens on 28672 x 8192 are level with it and the wrapped columns alone cost more tokens 0.4 %: 16384 5468 / 5438 us)
+    const int ahead = !SPLIT && P * Q < 32 && spread ? (int)(((int64_t)(blockIdx.x & 7) * steps) >> 3) : 0;
     // where a step's columns are in the rows, in bytes (steps behind the last: the last again)
     auto column_of = [&](int step_) {
         const int c = min(step_, steps - 1) + ahead;

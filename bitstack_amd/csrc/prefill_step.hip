@@ -72,28 +72,30 @@ __global__ __launch_bounds__(THREADS) void silu_mul_kernel(const half_t *gate, c
 }
 
 // Causal attention of a whole prompt over the cache that rope_store_kernel has filled.  A wave takes 16 QT queries of one head and
-// walks the positions up to its last query 64 at a time with a running (max, sum, weighted v).  The waves of a workgroup share a KV head: their items are (tile of
+// walks the positions up to its last query 64 at a time with a running (max, sum, weighted v), which takes up 32 of them at a time.  The waves of a workgroup share a KV head: their items are (tile of
 // queries, head of the group), the head fastest, so that they need the same rows.  These come to LDS a stage of 64 positions at a time, requested one stage ahead, straight from
 // memory (no registers, no LDS write instructions), one barrier per stage.  The operands lie as in the decode step's attention (decode_step.hip): scores S[position, query] =
 // K q, output O[dim, query] += V^T P, on 16x16x32 products whose lane layouts fit without any shuffle - a lane of the scores holds four positions of one query in each of
 // two tiles of 16 positions, which are the eight k slots of the output product, and V is used as it lies, product j taking half j of a lane's 16 bytes.  The 16-byte
 // pieces of a row of K are XOR-ed with the row's number: a score fragment reads one piece of 16 rows, which lie a whole turn of the banks apart.
-// What bounds it: with many queries the issue of the softmax's instructions and of the products (800 TFLOP/s of the lower triangle), with few the chain of a stage, 1.2 us.
-// us, every wave reading its own rows from L2 32 positions at a time / this: 2 x 700 queries with 32 heads on 8 KV heads 40.4 / 22.8, 4 x 300 21.5 / 13.6, 100 8.1 / 5.8, 4000 309 / 173,
-// 4 x 1500 with 64 on 16 352 / 214, 64 on 64 364 / 247, 8 x 2048 with 64 on 8 1214 / 683.  A stage of 64 as two steps of 32 positions: 28.5 on the first, 198 on the fourth.
-// Error against float64: 2.360e-4 on the first, 2.394e-4 on 1 x 2000 with 8 on 2 (before 2.362e-4 and 2.394e-4).
+// The weights are rounded to fp16 for the second product; their sum is that of the fp32 weights.
+// What bounds it: with many queries the issue of the softmax's instructions and of the products (750 TFLOP/s of the lower triangle), with few the chain of a stage, 1.2 us.
+// us, every wave reading its own rows from L2 32 positions at a time / this: 2 x 700 queries with 32 heads on 8 KV heads 39.4 / 22.7, 4 x 300 20.5 / 13.3, 100 7.3 / 5.2, 4000 301 / 174,
+// 4 x 1500 with 64 on 16 345 / 219, 64 on 64 357 / 244, 8 x 2048 with 64 on 8 1211 / 736.  A stage of 64 as two steps of 32 positions: 28.5 on the first, 198 on the fourth.
+// Error against float64: 2.469e-4 on the first, 2.494e-4 on 1 x 2000 with 8 on 2, as before.  One maximum for the 64 positions is 5 % faster (21.7 on the first), but fewer weights are
+// then a maximum, exact when rounded: 2.483e-4 and 2.506e-4.  The rounded weights' sum, by a product with ones, is no faster than that.
 constexpr int AP_D = 128, AP_WAVES = 4, AP_P = 64;       // (AP_P: positions of a stage)
 constexpr int AP_CHUNKS = 2 * (AP_P / 4) / AP_WAVES;                // requests per wave and stage: of 1 KB, four rows; K, then V
 
 typedef __attribute__((address_space(3))) void *ap_lds;
 
-// the larger of v here and in the lane whose number differs by W (16 or 32)
-template <int W>
+// the larger of v here and in the lane whose number differs by W (16 or 32), or (SUM) both together
+template <int W, bool SUM = false>
 __device__ __forceinline__ float across(float v) {
     const uint32_t u = __builtin_bit_cast(uint32_t, v);
     const auto r = W == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
     const uint32_t a = r[0], b = r[1];
-    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    return SUM ? __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b) : fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
 }
 
 template <int QT>
@@ -138,13 +140,12 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
     }
 
     const float scale2 = 0.08838834764831845f * 1.4426950408889634f;    // 1 / sqrt(128) * log2(e): the softmax runs in base 2
-    float m[QT];                                 // of query r16 of a tile
-    float4_t acc[QT][8], l[QT];                  // (l: the sum of the weights as they are multiplied, that is rounded, by a product with ones; the same in all four)
-    const half8_t ones = {(half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1, (half_t)1};
+    float m[QT], l[QT];                          // of query r16 of a tile; l: the fp32 sum of the weights, before any is rounded, over this lane's positions
+    float4_t acc[QT][8];
 #pragma unroll
     for (int t = 0; t < QT; t++) {
         m[t] = -INFINITY;
-        l[t] = (float4_t)0.f;
+        l[t] = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) acc[t][j] = (float4_t)0.f;
     }
@@ -180,38 +181,43 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
                     for (int i = 0; i < 4; i++)
                         if (p0 + 16 * a + 4 * g + i > q0 + 16 * t + r16) s[t][a][i] = -INFINITY;
         }
-        float r[QT];
-        half8_t p8[QT][A / 2];
+        // 32 positions at a time the running maximum, the weights, their sum and what the older sums are to be multiplied by
+        float r[A / 2][QT];
+        half8_t p8[A / 2][QT];
 #pragma unroll
-        for (int t = 0; t < QT; t++) {
-            float mx = s[t][0][0];
-#pragma unroll
-            for (int i = 1; i < 4 * A; i++) mx = fmaxf(mx, s[t][i >> 2][i & 3]);
-            mx = across<32>(across<16>(mx));
-            const float mn = fmaxf(m[t], mx * scale2);
-            r[t] = __builtin_amdgcn_exp2f(m[t] - mn);
-            m[t] = mn;
-#pragma unroll
-            for (int i = 0; i < 4 * A; i++) p8[t][i >> 3][i & 7] = (half_t)__builtin_amdgcn_exp2f(s[t][i >> 2][i & 3] * scale2 - mn);
-        }
-        if (__any(r[0] != 1.f || r[QT - 1] != 1.f)) {
+        for (int h = 0; h < A / 2; h++)
 #pragma unroll
             for (int t = 0; t < QT; t++) {
-                l[t] *= r[t];
+                float mx = s[t][2 * h][0];
 #pragma unroll
-                for (int j = 0; j < 8; j++) acc[t][j] *= r[t];
+                for (int i = 1; i < 8; i++) mx = fmaxf(mx, s[t][2 * h + (i >> 2)][i & 3]);
+                mx = across<32>(across<16>(mx));
+                const float mn = fmaxf(m[t], mx * scale2);
+                r[h][t] = __builtin_amdgcn_exp2f(m[t] - mn);
+                m[t] = mn;
+                float sum[2];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const float p = __builtin_amdgcn_exp2f(s[t][2 * h + (i >> 2)][i & 3] * scale2 - mn);
+                    sum[i & 1] = i < 2 ? p : sum[i & 1] + p;
+                    p8[h][t][i] = (half_t)p;
+                }
+                l[t] = l[t] * r[h][t] + (sum[0] + sum[1]);
             }
-        }
 #pragma unroll
         for (int h = 0; h < A / 2; h++) {
-#pragma unroll
-            for (int t = 0; t < QT; t++) l[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p8[t][h], l[t], 0, 0, 0);
             if (h > 0 && p0 + 32 * h > q0) continue;      // (32 positions behind all of the queries: an infinity in their v must not make a NaN of a weight of zero)
+            if (__any(r[h][0] != 1.f || r[h][QT - 1] != 1.f)) {
+#pragma unroll
+                for (int t = 0; t < QT; t++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) acc[t][j] *= r[h][t];
+            }
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const half8_t v = {v8[0][j], v8[1][j], v8[2][j], v8[3][j], v8[4][j], v8[5][j], v8[6][j], v8[7][j]};
 #pragma unroll
-                for (int t = 0; t < QT; t++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p8[t][h], acc[t][j], 0, 0, 0);
+                for (int t = 0; t < QT; t++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p8[h][t], acc[t][j], 0, 0, 0);
             }
             if (h + 1 < A / 2) fetch_v(h + 1);
         }
@@ -235,9 +241,10 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
     if (!mine) return;
 #pragma unroll
     for (int t = 0; t < QT; t++) {
+        const float total = across<32, true>(across<16, true>(l[t]));
         const int qi = q0 + 16 * t + r16;
         if (qi >= n) continue;
-        const float inv = 1.f / l[t][0];
+        const float inv = 1.f / total;
         half_t *to = out + ((int64_t)b * n + qi) * row + head * AP_D;
 #pragma unroll
         for (int i = 0; i < 4; i++) {            // row 4 g + i of product j is dimension 8 (4 g + i) + j

@@ -5,6 +5,7 @@
 // each result is computed in fp32 and rounded once.
 #include "common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -260,11 +261,15 @@ __global__ __launch_bounds__(AP_WAVES * 64, 2) void attention_prefill_kernel(con
 
 int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const half_t *vcache, half_t *out, int ldq, int B, int n, int heads,
                                 int kv_heads, int max_len, hipStream_t s) {
+    const int per = std::max(1, (1 << 24) / kv_heads - 1);      // sequences of a launch: a grid holds 2^32 threads along x
     const auto launch = [&](auto kernel, int queries) {
         const int64_t chunks = bs_cdiv((int64_t)(heads / kv_heads) * bs_cdiv(n, queries), AP_WAVES), y = chunks < 32768 ? chunks : 32768;
         if (chunks > INT32_MAX / AP_WAVES) return BS_ERR_SHAPE;
-        const dim3 grid((unsigned)(B * kv_heads), (unsigned)y, (unsigned)bs_cdiv(chunks, y));
-        kernel<<<grid, AP_WAVES * 64, 0, s>>>(q, kcache, vcache, out, ldq, n, heads, kv_heads, max_len, (int)chunks);
+        for (int b = 0; b < B; b += per) {
+            const dim3 grid((unsigned)(std::min(per, B - b) * kv_heads), (unsigned)y, (unsigned)bs_cdiv(chunks, y));
+            const int64_t cache = (int64_t)b * kv_heads * max_len * AP_D;
+            kernel<<<grid, AP_WAVES * 64, 0, s>>>(q + (int64_t)b * n * ldq, kcache + cache, vcache + cache, out + (int64_t)b * n * heads * AP_D, ldq, n, heads, kv_heads, max_len, (int)chunks);
+        }
         return (int)BS_OK;
     };
     // 16 queries per wave while 32 would leave the chip few workgroups: the chain of a wave's stages is what such a call takes (us, 32 / 16 queries: 2 x 700 positions with 32

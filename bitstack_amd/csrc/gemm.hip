@@ -243,12 +243,11 @@ __global__ __launch_bounds__(64 * WT * WF) void linear_f16_kernel(
 // Few tokens (<= 32): the job is to stream w once at memory speed, so nothing is shared through LDS.  A workgroup owns 16 F features; its 8 waves split the contracted
 // range, each reading its fragments of v_mfma_f32_16x16x32_f16 straight from global memory, whole 128-byte lines (the two halves of one back to back), AHEAD
 // lines of 16 F rows in flight, TB blocks of 16 tokens against them.  The waves' sums are added through LDS in a fixed order.  N % 8 == 0: pieces beyond the last
-// column, or the wave's last line, are asked for beyond the end of the buffer, which reads as zeros.
-// The waves take turns along the rows, AHEAD lines each, and a workgroup starts 13 lines further into them than the one before: rows of 8 or 16 KB lie on the same memory channels, and workgroups
-// that all start at their beginning ask the same few for everything (us, every wave with a range of its own / this: 32000 x 8192, 8 tokens 98.0 / 90.3; 32000 x 4096, one 51.9 / 47.2;
-// 128256 x 2048, 16 105.6 / 96.1; 14336 x 4096, 8 26.7 / 23.8, 4096 x 4096 10.9 / 9.3; 32000 x 4096, 32 60.6 / 56.0; turns without the steps of 13 103.0 on the first, steps of 8 and of 1 no better.
-// 32 features and up to 16 tokens: 5120 x 5120 18.4 / 18.7, so there they keep their ranges).
-// What bounds it: memory (32000 x 8192, 8 tokens: 5.8 TB/s), with 16 tokens and more the reads of x, as many bytes per workgroup as T / (16 F) of w.  us, the kernel
+// column, or the wave's last line, are asked for beyond the end of the buffer, which reads as zeros.  Every feature is summed in the same order, so equal rows of w
+// (words that share an embedding) have equal outputs.  Workgroups that start at places of their own along the rows ask different memory channels and are faster where rows are 4, 8 or
+// 16 KB (us, this / so: 32000 x 8192, 8 tokens 98.3 / 90.8; 32000 x 4096, one 52.8 / 48.7; 14336 x 4096, 8 27.0 / 24.1; 32000 x 5120, 8 62.0 / 61.7), but then the order depends on the
+// workgroup; two or four parts whose sums commute, walked in orders of their own, are not (97 and 102 on the first).
+// What bounds it: memory (32000 x 8192, one token: 5.6 TB/s), with 16 tokens and more the reads of x, as many bytes per workgroup as T / (16 F) of w.  us, the kernel
 // before (v_mfma_f32_32x32x16_f16, half a line's quarter per request, N % 16 == 0 only, otherwise the tiled kernel) / this: 32000 x 4096, one token 55.7 / 48.7, 8 tokens
 // 63.9 / 49.3, 32 tokens 89.1 / 56.8; 32000 x 8192, 8 tokens 123.9 / 92.5; 4096 x 4104, 8 tokens 26.0 / 8.1; 512 x 6008 27.5 / 8.1.  Fewer parts of the contracted range and more features side by
 // side (4, 2, 1 parts): slower from 4096 columns on, level below.
@@ -261,10 +260,8 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES, 4) void linear_skinny_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lm = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.x * (16 * F);
-    constexpr bool TURNS = !(TB == 1 && F == 2);
-    const int lines = (N + SKINNY_LINE - 1) / SKINNY_LINE, share = (lines + SKINNY_WAVES - 1) / SKINNY_WAVES, per = TURNS ? min(AHEAD, share) : AHEAD;
-    const int begin = wave * (TURNS ? per : share), end = TURNS ? lines : min(begin + share, lines), stride = TURNS ? SKINNY_WAVES * per : AHEAD;
-    const int rot = TURNS && lines >= 32 ? (int)(blockIdx.x * 13u % (uint32_t)lines) : 0;
+    const int lines = (N + SKINNY_LINE - 1) / SKINNY_LINE, per = (lines + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const int begin = wave * per, end = min(begin + per, lines), limit = min(end * SKINNY_LINE, N);     // (no branch around a product: its loads would move into it)
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)(w + (int64_t)m0 * N), 0, (int)((uint32_t)min(16 * F, M - m0) * (uint32_t)N * 2u), 0x00020000);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, (int)((uint32_t)T * (uint32_t)N * 2u), 0x00020000);
     uint32_t off_w[F], off_x[TB];
@@ -278,23 +275,21 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES, 4) void linear_skinny_kernel(
     for (int b = 0; b < TB; b++)
 #pragma unroll
         for (int f = 0; f < F; f++) acc[b][f] = (float4_t){0.f, 0.f, 0.f, 0.f};
-    for (int at = begin; at < end; at += stride) {
+    for (int at = begin; at < end; at += AHEAD) {
         half8_t wf[AHEAD][2][F], xf[AHEAD][2][TB];
 #pragma unroll
         for (int q = 0; q < AHEAD; q++) {
-            int line = at + q;                   // (no branch around a product: its loads would move into it)
-            line = q < per && line < end ? (line + rot < lines ? line + rot : line + rot - lines) : lines;
-            const int col = line * SKINNY_LINE;
+            const int col = (at + q) * SKINNY_LINE;
 #pragma unroll
             for (int f = 0; f < F; f++)
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    wf[q][h][f] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(col + 32 * h + 8 * g < N ? off_w[f] + 64u * h : 0x80000000u), 2 * col, 0));
+                    wf[q][h][f] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(col + 32 * h + 8 * g < limit ? off_w[f] + 64u * h : 0x80000000u), 2 * col, 0));
 #pragma unroll
             for (int b = 0; b < TB; b++)
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    xf[q][h][b] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(col + 32 * h + 8 * g < N ? off_x[b] + 64u * h : 0x80000000u), 2 * col, 0));
+                    xf[q][h][b] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(col + 32 * h + 8 * g < limit ? off_x[b] + 64u * h : 0x80000000u), 2 * col, 0));
         }
         __builtin_amdgcn_sched_barrier(0);                               // (all of them on their way before the first is waited for)
 #pragma unroll

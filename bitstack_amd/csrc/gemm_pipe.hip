@@ -80,7 +80,7 @@ __device__ __forceinline__ void phase_barrier() {
 template <int P, int Q, bool SWAP, int S, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
     const half_t *__restrict__ x, const half_t *__restrict__ w, const half_t *__restrict__ bias,
-    half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide, int spread) {
+    half_t *__restrict__ y, float *__restrict__ part, int T, int M, int N, int steps_per_split, int wide) {
     static_assert((SWAP ? P : Q) % 2 == 0, "feature fragments come in pairs");
     constexpr int BP = 32 * P, BQ = 64 * Q;   // P, Q: 16-row fragments of a wave
     constexpr int BT = SWAP ? BQ : BP, BF = SWAP ? BP : BQ;
@@ -148,13 +148,8 @@ __global__ __launch_bounds__(512, 2) void linear_pipe_kernel(
         const int r = qrow + 8 * j + (lane >> 3);
         voff_q[j] = (uint32_t)min(r, q_last) * (uint32_t)N * 2u + 16u * ((lane & 7) ^ swizzle(!SWAP, r));
     }
-    // (spread: see launch_pipe; not in 256 x 256, where 512 tokens on 28672 x 8192 are level with it and the wrapped columns alone cost more tokens 0.4 %: 16384 5468 / 5438 us)
-    const int ahead = !SPLIT && P * Q < 32 && spread ? (int)(((int64_t)(blockIdx.x & 7) * steps) >> 3) : 0;
     // where a step's columns are in the rows, in bytes (steps behind the last: the last again)
-    auto column_of = [&](int step_) {
-        const int c = min(step_, steps - 1) + ahead;
-        return (c < steps ? c : c - steps) * (PK * 2);
-    };
+    auto column_of = [&](int step_) { return min(step_, steps - 1) * (PK * 2); };
     auto request_p = [&](auto stage, int column, int j) {
         half_t *dst = p_stage(stage) + prow[j] * PK;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr)dst, 16, (int)voff_p[j], column, 0, 0);
@@ -389,17 +384,15 @@ int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y,
     const int steps = (int)bs_cdiv(N / PK, splits);
     splits = (int)bs_cdiv(N / PK, steps);     // every part holds at least one k-step
     const int wide = M % 8 == 0 && bs_aligned(y, 16) && bs_aligned(part, 16);
-    // A few hundred tokens on a weight beyond the L2s: every XCD starts an eighth of the rows further than the one before, so that they do not all ask the same memory channels
-    // (its own workgroups still share their lines).  us of a call, all from the first column / so: 14336 x 4096, 4 blocks, 300 tokens 89.6 / 84.7, 4096 x 4096, 4, 300 43.7 / 41.5, 28672 x
-    // 8192, 2, 300 256 / 250; but 1024 x 4096, 4, 300 24.3 / 25.1, 6144 x 4096, 4, 1400 85.2 / 86.5.
-    const int spread = T <= 512 && (int64_t)M * N >= (16 << 20);
+    // (All tiles sum in the order of the columns: equal rows of x or w have equal outputs.  XCDs that each start an eighth further along the rows ask different memory channels, 14336 x
+    // 4096, 4 blocks, 300 tokens 89.6 / 84.7 us, but a token's sums would then depend on where its tile lies.)
     const bool two = S_TWO != S && (int64_t)tiles * splits > 256;
     if (splits == 1) {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide, spread);
-        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide, spread);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
     } else {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide, spread);
-        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide, spread);
+        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
         BS_LAUNCH_CHECK();
         const int64_t total = (int64_t)T * M;
         if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, splits, total, M);

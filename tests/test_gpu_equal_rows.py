@@ -8,7 +8,9 @@ from bitstack_amd.utils import inference_utils as IU
 
 # tokens, out features, in features, the tile: every width of the few-token kernel, one and two blocks of tokens, rows of more than 32 lines
 FEW = [(8, 4096, 4096, (32, 16)), (8, 5120, 4096, (32, 32)), (3, 16000, 2048, (32, 64)), (16, 12800, 4104, (32, 64)), (24, 4000, 6152, (32, 16)), (32, 5120, 4096, (32, 32)), (17, 12801, 2056, (32, 64))]
-CASES = FEW
+# several tiles of tokens and of features on every XCD, up to 512 tokens on 16 Mi weights and more: 128 x 128 with one and two workgroups per CU, 128 x 256, 256 x 256, 64 x 64
+MORE = [(300, 8192, 4096, (128, 128)), (512, 8704, 2048, (128, 128)), (500, 14336, 2048, (128, 256)), (512, 20500, 1024, (256, 256)), (140, 5000, 4096, (64, 64))]
+CASES = FEW + MORE
 
 
 @pytest.mark.gpu

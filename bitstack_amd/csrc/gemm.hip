@@ -501,7 +501,8 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
 extern "C" int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_features, int *k_step, int *k_tail) {
     if (!tile_tokens || !tile_features || !k_step || !k_tail) return BS_ERR_NULL;
     if (T <= 0 || M <= 0 || N <= 0) return BS_ERR_SHAPE;
-    const LinearTile t = linear_tile(T, M, N, true);
+    LinearTile t = linear_tile(T, M, N, true);
+    if (N % 64 == 0 && pipe_64(t, T, M, N)) t.gk = 64;      // linear_pipe_kernel's
     *tile_tokens = t.bt;
     *tile_features = t.bf;
     *k_step = t.gk;

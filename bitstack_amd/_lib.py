@@ -30,6 +30,7 @@ SIGNATURES = {
     "bs_forward_static": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "bs_linear_f16": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
     "bs_linear_plan": (_I, [_I, _I, _I, _P, _P, _P, _P]),
+    "bs_dense_plan": (_I, [_I, _I, _I, _I, _P, _P, _P, _P]),
     "bs_decode_kernel": (_I, [_I, _I, _I, _I, _I]),
     "bs_set_decode_kernel": (_I, [_I]),
     "bs_set_dense_kernel": (_I, [_I]),
@@ -150,6 +151,13 @@ def linear_plan(T, M, N):
     """(tile_tokens, tile_features, k_step, k_tail) of the dense kernel for these dimensions."""
     vals = [ctypes.c_int(0) for _ in range(4)]
     check(lib().bs_linear_plan(T, M, N, *[ctypes.byref(v) for v in vals]), "bs_linear_plan")
+    return tuple(v.value for v in vals)
+
+
+def dense_plan(T, M, N, rebuilt=False):
+    """(tile_tokens, tile_features, parts, stages) of the dense product of linear_f16_hip or, behind a rebuilt weight, of a forward."""
+    vals = [ctypes.c_int(0) for _ in range(4)]
+    check(lib().bs_dense_plan(T, M, N, int(rebuilt), *[ctypes.byref(v) for v in vals]), "bs_dense_plan")
     return tuple(v.value for v in vals)
 
 

@@ -65,6 +65,7 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
 // range in that many parts, part[splits][T][M] floats of scratch
 int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int bt, int bf,
                           int splits, float *part, hipStream_t s);
+int bs_linear_pipe_plan(int T, int M, int N, int bt, int bf, int splits, int *parts, int *stages);
 // the product behind a rebuilt weight (16-byte aligned x and w): tile and parts by shape, bs_linear_parts_bytes of scratch
 int64_t bs_linear_parts_bytes(int T, int M, int N);
 int bs_launch_linear_parts(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, float *part, hipStream_t s);

@@ -393,6 +393,9 @@ static bool pipe_64(const LinearTile &tile, int T, int M, int N) {
     return tile.bt == 64 && tile.bf == 64 && (wg <= 256 || wg > 384 || N <= 3072);
 }
 
+// whether linear_pipe_kernel has this tile of bs_linear_f16's
+static bool on_pipe(const LinearTile &tile, int T, int M, int N) { return N % 64 == 0 && (tile.bf >= 128 || pipe_64(tile, T, M, N)); }
+
 // The tile behind a rebuilt weight, where scratch for partial sums can be had too.  splits > 1: the contracted range is
 // cut into that many parts, whose sums a second kernel adds up: a few tokens on a large weight are a handful of large
 // tiles, which leave most of the chip idle, or many small ones, which move the most bytes per flop (509 tokens on
@@ -478,7 +481,7 @@ int bs_launch_linear_f16(const half_t *x, const half_t *w, const half_t *bias, h
         const auto skinny = [&](auto kernel) { kernel<<<(int)bs_cdiv(M, tile.bf), 64 * SKINNY_WAVES, 0, s>>>(x, w, bias, y, T, M, N); };
         if (T <= 16) tile.bf == 64 ? skinny(linear_skinny_kernel<1, 4, 2>) : tile.bf == 32 ? skinny(linear_skinny_kernel<1, 2, 2>) : skinny(linear_skinny_kernel<1, 1, 6>);
         else tile.bf == 64 ? skinny(linear_skinny_kernel<2, 4, 1>) : tile.bf == 32 ? skinny(linear_skinny_kernel<2, 2, 2>) : skinny(linear_skinny_kernel<2, 1, 4>);
-    } else if (N % 64 == 0 && (tile.bf >= 128 || pipe_64(tile, T, M, N))) {
+    } else if (on_pipe(tile, T, M, N)) {
         return bs_launch_linear_pipe(x, w, bias, y, T, M, N, tile.bt, tile.bf, 1, nullptr, s);
     } else if (tile.bt == 128 && tile.bf == 64) {
         st = launch_tiled<2, 2, 2, 1, 64>(x, w, bias, y, T, M, N, s);
@@ -502,12 +505,26 @@ extern "C" int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_f
     if (!tile_tokens || !tile_features || !k_step || !k_tail) return BS_ERR_NULL;
     if (T <= 0 || M <= 0 || N <= 0) return BS_ERR_SHAPE;
     LinearTile t = linear_tile(T, M, N, true);
-    if (N % 64 == 0 && pipe_64(t, T, M, N)) t.gk = 64;      // linear_pipe_kernel's
+    if (on_pipe(t, T, M, N)) t.gk = 64;                     // linear_pipe_kernel's
     *tile_tokens = t.bt;
     *tile_features = t.bf;
     *k_step = t.gk;
     *k_tail = t.gk > 0 && N % t.gk != 0;
     return BS_OK;
+}
+
+extern "C" int bs_dense_plan(int T, int M, int N, int rebuilt, int *tile_tokens, int *tile_features, int *parts, int *stages) {
+    if (!tile_tokens || !tile_features || !parts || !stages) return BS_ERR_NULL;
+    if (T <= 0 || M <= 0 || N <= 0) return BS_ERR_SHAPE;
+    const LinearTile t = linear_tile(T, M, N, true);
+    LinearChoice c = rebuilt ? linear_choice(T, M, N) : LinearChoice{0, 0, 1};
+    const bool pipe = c.bt != 0 || on_pipe(t, T, M, N);
+    if (c.bt == 0) c = {t.bt, t.bf, 1};
+    *tile_tokens = c.bt;
+    *tile_features = c.bf;
+    *parts = 1;
+    *stages = 0;
+    return pipe ? bs_linear_pipe_plan(T, M, N, c.bt, c.bf, c.splits, parts, stages) : (int)BS_OK;
 }
 
 extern "C" int bs_linear_f16(const void *x, const void *w, const void *bias, void *y,

@@ -376,44 +376,61 @@ __global__ __launch_bounds__(256) void linear_split_sum_kernel(const float *__re
     }
 }
 
-// S stages where the grid leaves a CU one workgroup, S_TWO where it has more (fewer of them, so that two fit its LDS)
-template <int P, int Q, bool SWAP, int S, int S_TWO>
+// A tile of P x Q fragments; S stages where the grid leaves a CU one workgroup, S_TWO where it has more (fewer of them, so that two fit its LDS)
+template <int P_, int Q_, bool SWAP_, int S_, int S_TWO_>
+struct PipeBuild {
+    static constexpr int P = P_, Q = Q_, S = S_, S_TWO = S_TWO_;
+    static constexpr bool SWAP = SWAP_;
+    static constexpr int BT = SWAP ? 64 * Q : 32 * P, BF = SWAP ? 32 * P : 64 * Q;
+    static_assert(S * (BT + BF) * PK * 2 <= 160 * 1024 && (S == S_TWO || S_TWO * (BT + BF) * PK * 2 <= 80 * 1024), "LDS of a CU");
+};
+struct PipePlan {
+    int steps, parts, stages;                 // of a part; every part holds at least one k-step
+    unsigned tiles;
+};
+template <class B>
+PipePlan pipe_plan(int T, int M, int N, int splits) {
+    PipePlan p;
+    p.tiles = (unsigned)(bs_cdiv(T, B::BT) * bs_cdiv(M, B::BF));
+    p.steps = (int)bs_cdiv(N / PK, splits);
+    p.parts = (int)bs_cdiv(N / PK, p.steps);
+    p.stages = (int64_t)p.tiles * p.parts > 256 ? B::S_TWO : B::S;
+    return p;
+}
+
+template <class B>
 int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int splits, float *part, hipStream_t s) {
-    constexpr int BT = SWAP ? 64 * Q : 32 * P, BF = SWAP ? 32 * P : 64 * Q;
-    const unsigned tiles = (unsigned)(bs_cdiv(T, BT) * bs_cdiv(M, BF));
-    const int steps = (int)bs_cdiv(N / PK, splits);
-    splits = (int)bs_cdiv(N / PK, steps);     // every part holds at least one k-step
+    constexpr int P = B::P, Q = B::Q, S = B::S, S_TWO = B::S_TWO;
+    constexpr bool SWAP = B::SWAP;
+    const PipePlan p = pipe_plan<B>(T, M, N, splits);
     const int wide = M % 8 == 0 && bs_aligned(y, 16) && bs_aligned(part, 16);
     // (All tiles sum in the order of the columns: equal rows of x or w have equal outputs.  XCDs that each start an eighth further along the rows ask different memory channels, 14336 x
     // 4096, 4 blocks, 300 tokens 89.6 / 84.7 us, but a token's sums would then depend on where its tile lies.)
-    const bool two = S_TWO != S && (int64_t)tiles * splits > 256;
-    if (splits == 1) {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
-        else linear_pipe_kernel<P, Q, SWAP, S, false><<<tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, steps, wide);
+    if (p.parts == 1) {
+        if (p.stages != S) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<p.tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, p.steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, false><<<p.tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, p.steps, wide);
     } else {
-        if (two) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
-        else linear_pipe_kernel<P, Q, SWAP, S, true><<<tiles * splits, 512, 0, s>>>(x, w, bias, y, part, T, M, N, steps, wide);
+        if (p.stages != S) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<p.tiles * p.parts, 512, 0, s>>>(x, w, bias, y, part, T, M, N, p.steps, wide);
+        else linear_pipe_kernel<P, Q, SWAP, S, true><<<p.tiles * p.parts, 512, 0, s>>>(x, w, bias, y, part, T, M, N, p.steps, wide);
         BS_LAUNCH_CHECK();
         const int64_t total = (int64_t)T * M;
-        if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, splits, total, M);
-        else linear_split_sum_kernel<false><<<(unsigned)bs_cdiv(total, 256), 256, 0, s>>>(part, bias, y, splits, total, M);
+        if (wide) linear_split_sum_kernel<true><<<(unsigned)bs_cdiv(total, 8 * 256), 256, 0, s>>>(part, bias, y, p.parts, total, M);
+        else linear_split_sum_kernel<false><<<(unsigned)bs_cdiv(total, 256), 256, 0, s>>>(part, bias, y, p.parts, total, M);
     }
     BS_LAUNCH_CHECK();
     return BS_OK;
 }
 
-}  // namespace
-
-// bt x bf: tokens x features per workgroup.  splits > 1: part holds splits * T * M floats.
-int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int bt, int bf,
-                          int splits, float *part, hipStream_t s) {
-    if (N % PK != 0 || splits < 1 || (splits > 1 && !part)) return BS_ERR_SHAPE;
+// f on the build of a tile of bt x bf (tokens x features per workgroup)
+template <class F>
+int with_pipe_build(int bt, int bf, F &&f) {
     switch (bt * 1000 + bf) {
-#define PIPE_CASE(bt, bf, p, q, swap, s_one, s_two) \
-    case bt * 1000 + bf: \
-        static_assert(bt == (swap ? 64 * q : 32 * p) && bf == (swap ? 32 * p : 64 * q), "the tile"); \
-        static_assert(s_one * (bt + bf) * PK * 2 <= 160 * 1024 && (s_one == s_two || s_two * (bt + bf) * PK * 2 <= 80 * 1024), "LDS of a CU"); \
-        return launch_pipe<p, q, swap, s_one, s_two>(x, w, bias, y, T, M, N, splits, part, s);
+#define PIPE_CASE(bt, bf, ...) \
+    case bt * 1000 + bf: { \
+        typedef PipeBuild<__VA_ARGS__> B; \
+        static_assert(B::BT == bt && B::BF == bf, "the tile"); \
+        return f(B()); \
+    }
         PIPE_CASE(256, 256, 8, 4, false, 2, 2) PIPE_CASE(224, 256, 7, 4, false, 2, 2) PIPE_CASE(192, 256, 6, 4, false, 2, 2) PIPE_CASE(256, 192, 6, 4, true, 2, 2)
         PIPE_CASE(160, 256, 5, 4, false, 3, 3) PIPE_CASE(192, 192, 6, 3, true, 3, 3) PIPE_CASE(256, 128, 8, 2, false, 3, 3) PIPE_CASE(128, 256, 8, 2, true, 3, 3)
         PIPE_CASE(224, 128, 7, 2, false, 3, 3) PIPE_CASE(192, 128, 6, 2, false, 3, 3) PIPE_CASE(128, 192, 6, 2, true, 3, 3) PIPE_CASE(160, 128, 5, 2, false, 3, 2)
@@ -421,4 +438,23 @@ int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, 
 #undef PIPE_CASE
         default: return BS_ERR_SHAPE;
     }
+}
+
+}  // namespace
+
+// splits > 1: part holds splits * T * M floats.
+int bs_launch_linear_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y, int T, int M, int N, int bt, int bf,
+                          int splits, float *part, hipStream_t s) {
+    if (N % PK != 0 || splits < 1 || (splits > 1 && !part)) return BS_ERR_SHAPE;
+    return with_pipe_build(bt, bf, [&](auto b) { return launch_pipe<decltype(b)>(x, w, bias, y, T, M, N, splits, part, s); });
+}
+
+// the parts and stages that it runs with
+int bs_linear_pipe_plan(int T, int M, int N, int bt, int bf, int splits, int *parts, int *stages) {
+    return with_pipe_build(bt, bf, [&](auto b) {
+        const PipePlan p = pipe_plan<decltype(b)>(T, M, N, splits);
+        *parts = p.parts;
+        *stages = p.stages;
+        return (int)BS_OK;
+    });
 }

@@ -294,6 +294,15 @@ int bs_linear_f16(const void *x, const void *w, const void *bias, void *y,
 int bs_linear_plan(int T, int M, int N, int *tile_tokens, int *tile_features, int *k_step, int *k_tail);
 
 /*
+ * Introspection for benchmarks and tests: the workgroup tile of the dense product that
+ * bs_linear_f16 (rebuilt == 0) or, behind a rebuilt weight, bs_forward and bs_forward_cat
+ * (rebuilt != 0) run for these dimensions with 16-byte aligned buffers, into how many parts the
+ * contracted range is cut, and the stages of its pipeline through LDS (linear_pipe_kernel; 0:
+ * the other kernels, one part).
+ */
+int bs_dense_plan(int T, int M, int N, int rebuilt, int *tile_tokens, int *tile_features, int *parts, int *stages);
+
+/*
  * ---- decode step: several matrices per launch, fused epilogues -----------
  * One decode forward (T <= 48 tokens; N % 128 == 0) of up to 4 compressed matrices that read
  * the same x, in one kernel pair: what q_proj/k_proj/v_proj (or gate_proj/

@@ -1,4 +1,7 @@
-"""bs_linear_plan names the k-step, and the partial last one, of the kernel that bs_linear_f16 runs."""
+"""bs_linear_plan names the k-step, and the partial last one, of the kernel that bs_linear_f16 runs; bs_dense_plan the tile, the parts and the stages of either dense product."""
+import ctypes
+import random
+
 import pytest
 
 from bitstack_amd import _lib
@@ -17,3 +20,31 @@ PLANS = [
 @pytest.mark.parametrize("T,M,N,plan", PLANS)
 def test_the_step_of_the_kernel_that_runs(T, M, N, plan):
     assert _lib.linear_plan(T, M, N) == plan
+
+
+def test_dense_plan_of_linear_f16_is_its_tile():
+    for T, M, N, plan in PLANS:
+        bt, bf, parts, stages = _lib.dense_plan(T, M, N)
+        assert (bt, bf, parts) == plan[:2] + (1,)
+        assert (stages >= 2) == (N % 64 == 0 and plan[2] == 64 and bt * bf != 128 * 64)      # (linear_f16_kernel has its tile of 128 x 64 in steps of 64 too)
+
+
+def test_dense_plan_behind_a_rebuilt_weight_fits_the_scratch():
+    rng, cut = random.Random(5), 0
+    for _ in range(400):
+        T, M, N = rng.randint(129, 4000), 8 * rng.randint(64, 3500), 128 * rng.randint(4, 200)
+        bt, bf, parts, stages = _lib.dense_plan(T, M, N, rebuilt=True)
+        assert stages in (2, 3, 4) and stages * (bt + bf) * 128 <= 160 << 10
+        weight = (M * N * 2 + 255) // 256 * 256
+        room = _lib.lib().bs_workspace_bytes(4, M, N, 16, T) - weight
+        assert room >= (parts * T * M * 4 if parts > 1 else 0) and (parts > 1 or room == 0)
+        cut += parts > 1
+    assert 40 < cut < 360
+
+
+def test_dense_plan_refuses_what_linear_plan_refuses():
+    v = [ctypes.byref(ctypes.c_int()) for _ in range(4)]
+    L = _lib.lib()
+    assert L.bs_dense_plan(0, 64, 64, 0, *v) == L.bs_dense_plan(4, 0, 64, 1, *v) == L.bs_dense_plan(4, 64, -8, 1, *v) == -2
+    assert L.bs_dense_plan(4, 64, 64, 0, None, *v[1:]) == L.bs_dense_plan(4, 64, 64, 1, *v[:3], None) == -1
+    assert _lib.dense_plan(4, 64, 100) == _lib.dense_plan(4, 64, 100, rebuilt=True) == (0, 0, 1, 0)

@@ -376,13 +376,16 @@ __global__ __launch_bounds__(256) void linear_split_sum_kernel(const float *__re
     }
 }
 
-// A tile of P x Q fragments; S stages where the grid leaves a CU one workgroup, S_TWO where it has more (fewer of them, so that two fit its LDS)
-template <int P_, int Q_, bool SWAP_, int S_, int S_TWO_>
+// A tile of P x Q fragments; S stages where the grid leaves a CU one workgroup, S_TWO where it has more (fewer of them, so that two fit its LDS) and up to FEW k-steps: requests
+// for steps behind the last are made for nothing, one step's more with every stage.  us, S / S_TWO stages: 128 x 256, 1794 tokens on 2719 x 256 11.9 / 11.5, x 512 14.0 / 13.7, x 640 15.3 / 15.1,
+// x 1024 18.2 / 18.2, x 2048 31.6 / 35.9, 755 on 8066 x 320 12.8 / 12.4, x 512 14.7 / 14.7, x 1024 23.4 / 24.2; 128 x 128, 600 on 5000 x 128 5.9 / 5.6, x 192 6.5 / 6.2, x 256 6.6 / 6.7.
+template <int P_, int Q_, bool SWAP_, int S_, int S_TWO_, int FEW_>
 struct PipeBuild {
-    static constexpr int P = P_, Q = Q_, S = S_, S_TWO = S_TWO_;
+    static constexpr int P = P_, Q = Q_, S = S_, S_TWO = S_TWO_, FEW = FEW_;
     static constexpr bool SWAP = SWAP_;
     static constexpr int BT = SWAP ? 64 * Q : 32 * P, BF = SWAP ? 32 * P : 64 * Q;
-    static_assert(S * (BT + BF) * PK * 2 <= 160 * 1024 && (S == S_TWO || S_TWO * (BT + BF) * PK * 2 <= 80 * 1024), "LDS of a CU");
+    static constexpr bool PAIR = S_TWO != S && S_TWO * (BT + BF) * PK * 2 <= 80 * 1024;      // two workgroups fit the LDS of a CU
+    static_assert(S * (BT + BF) * PK * 2 <= 160 * 1024, "LDS of a CU");
 };
 struct PipePlan {
     int steps, parts, stages;                 // of a part; every part holds at least one k-step
@@ -394,7 +397,7 @@ PipePlan pipe_plan(int T, int M, int N, int splits) {
     p.tiles = (unsigned)(bs_cdiv(T, B::BT) * bs_cdiv(M, B::BF));
     p.steps = (int)bs_cdiv(N / PK, splits);
     p.parts = (int)bs_cdiv(N / PK, p.steps);
-    p.stages = (int64_t)p.tiles * p.parts > 256 ? B::S_TWO : B::S;
+    p.stages = p.steps <= B::FEW || (B::PAIR && (int64_t)p.tiles * p.parts > 256) ? B::S_TWO : B::S;
     return p;
 }
 
@@ -431,10 +434,10 @@ int with_pipe_build(int bt, int bf, F &&f) {
         static_assert(B::BT == bt && B::BF == bf, "the tile"); \
         return f(B()); \
     }
-        PIPE_CASE(256, 256, 8, 4, false, 2, 2) PIPE_CASE(224, 256, 7, 4, false, 2, 2) PIPE_CASE(192, 256, 6, 4, false, 2, 2) PIPE_CASE(256, 192, 6, 4, true, 2, 2)
-        PIPE_CASE(160, 256, 5, 4, false, 3, 3) PIPE_CASE(192, 192, 6, 3, true, 3, 3) PIPE_CASE(256, 128, 8, 2, false, 3, 3) PIPE_CASE(128, 256, 8, 2, true, 3, 3)
-        PIPE_CASE(224, 128, 7, 2, false, 3, 3) PIPE_CASE(192, 128, 6, 2, false, 3, 3) PIPE_CASE(128, 192, 6, 2, true, 3, 3) PIPE_CASE(160, 128, 5, 2, false, 3, 2)
-        PIPE_CASE(128, 128, 4, 2, false, 4, 2) PIPE_CASE(96, 128, 3, 2, false, 4, 2) PIPE_CASE(64, 128, 2, 2, false, 4, 3) PIPE_CASE(64, 64, 2, 1, true, 4, 4)
+        PIPE_CASE(256, 256, 8, 4, false, 2, 2, 0) PIPE_CASE(224, 256, 7, 4, false, 2, 2, 0) PIPE_CASE(192, 256, 6, 4, false, 2, 2, 0) PIPE_CASE(256, 192, 6, 4, true, 2, 2, 0)
+        PIPE_CASE(160, 256, 5, 4, false, 3, 3, 0) PIPE_CASE(192, 192, 6, 3, true, 3, 3, 0) PIPE_CASE(256, 128, 8, 2, false, 3, 3, 0) PIPE_CASE(128, 256, 8, 2, true, 3, 2, 8)
+        PIPE_CASE(224, 128, 7, 2, false, 3, 3, 0) PIPE_CASE(192, 128, 6, 2, false, 3, 3, 0) PIPE_CASE(128, 192, 6, 2, true, 3, 3, 0) PIPE_CASE(160, 128, 5, 2, false, 3, 2, 2)
+        PIPE_CASE(128, 128, 4, 2, false, 4, 2, 3) PIPE_CASE(96, 128, 3, 2, false, 4, 2, 3) PIPE_CASE(64, 128, 2, 2, false, 4, 3, 3) PIPE_CASE(64, 64, 2, 1, true, 4, 4, 0)
 #undef PIPE_CASE
         default: return BS_ERR_SHAPE;
     }

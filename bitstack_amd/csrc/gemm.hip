@@ -404,8 +404,10 @@ struct LinearChoice { int bt, bf, splits; };      // bt == 0: as bs_linear_f16
 
 // The tiles of gemm_pipe.hip, and in us what a k-step of 64 columns and the start and end of a workgroup take: while a CU has one workgroup, and (step_two > 0) a pair of
 // workgroups that share one.  A fit to the times of every tile on 256 products, 40 to 3300 tokens on 14 matrices from 600 x 512 to 28672 x 8192: the choice
-// made with it is 1.0 % from the best tile on average, 25 at worst.  What the sums cost, and which of 256 x 128 and 128 x 256: 98 whole calls with every tile and cut, 132 to 1400
-// tokens on 12 matrices beyond 64 MiB of weight, of which the choice is 1.5 % from the best on average, 11 at worst.
+// made with it is 1.0 % from the best tile on average, 25 at worst.  What the sums cost: whole calls cut and not, 98 of 132 to 1400 tokens on 12 matrices, and 132 drawn ones of 129 to 4100 on
+// weights of 64 to 380 MiB: beyond 64 MiB of sums 0.5 us more per MiB than up to there (2515 tokens on 9480 x 12800, 182 MiB, 597 us in two parts, 540 in one; 2735 on 7320 x 25216, 305 MiB,
+// 1001 in four, 1011).  Where the estimates are level the cut is 3 to 20 % behind (6936 x 22272, 1722 tokens 585 / 493, 8824 x 17408, 1362 480 / 427), and the calls that it is ahead on (4096 x
+// 14336, 1400 tokens 186 / 211, 509 123 / 149) are clear of that line.
 struct PipeTile { int bt, bf; double step, start, step_two, start_two; };
 static const PipeTile pipe_tiles[] = {
     {256, 256, 1.604, 4.1, 0, 0}, {224, 256, 1.471, 3.5, 0, 0}, {192, 256, 1.358, 2.6, 0, 0}, {256, 192, 1.336, 2.9, 0, 0},
@@ -420,7 +422,9 @@ static double linear_cost(const PipeTile &t, int splits, int T, int M, int N) {
     const bool two = t.step_two > 0 && wg > 256;
     const int64_t slots = two ? 512 : 256, rounds = bs_cdiv(wg, slots);
     double us = (rounds - 0.43 * (rounds - (double)wg / slots)) * steps * (two ? t.step_two : t.step) + rounds * (two ? t.start_two : t.start) + 2.0;
-    if (parts > 1) us += 3.0 + 0.5e-6 * parts * T * M;
+    // (sums beyond 64 MiB no longer stay in the cache between the two kernels)
+    const double sums = (double)parts * T * M, cached = 1 << 24;
+    if (parts > 1) us += 3.0 + 0.5e-6 * sums + (sums > cached ? 2e-6 * (sums - cached) : 0.);
     return us;
 }
 
@@ -447,8 +451,7 @@ static LinearChoice linear_choice(int T, int M, int N) {
             if (us < cut_us) cut_us = us, cut = {t.bt, t.bf, c};
         }
     }
-    // (beyond 8192 columns the small tiles that an uncut range then takes are slower than the estimate: 1400 tokens on 4096 x 14336, 192 x 128 168 us, 192 x 256 in two parts 152)
-    return cut_us < (N > 8192 ? 1.06 : 1.0) * one_us ? cut : one;
+    return cut_us < one_us ? cut : one;
 }
 // (asked for the scratch, then for the launch: the last answer of the thread is kept)
 static LinearChoice linear_choice_kept(int T, int M, int N) {

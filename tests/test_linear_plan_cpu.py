@@ -48,3 +48,16 @@ def test_dense_plan_refuses_what_linear_plan_refuses():
     assert L.bs_dense_plan(0, 64, 64, 0, *v) == L.bs_dense_plan(4, 0, 64, 1, *v) == L.bs_dense_plan(4, 64, -8, 1, *v) == -2
     assert L.bs_dense_plan(4, 64, 64, 0, None, *v[1:]) == L.bs_dense_plan(4, 64, 64, 1, *v[:3], None) == -1
     assert _lib.dense_plan(4, 64, 100) == _lib.dense_plan(4, 64, 100, rebuilt=True) == (0, 0, 1, 0)
+
+
+# out of whole calls timed cut and in one piece (us, cut / in one): sums beyond what the cache holds, estimates that are level, and clear gains
+IN_ONE = [(2515, 9480, 12800), (2247, 5080, 19712),                                                          # 597 / 540, 467 / 398
+          (1722, 6936, 22272), (1362, 8824, 17408), (2056, 8200, 17536), (1130, 10592, 22400), (1497, 5768, 16256)]  # 585 / 493, 480 / 427, 638 / 567, 627 / 551, 311 / 268
+CUT = [(1400, 4096, 14336), (509, 4096, 14336), (1017, 3248, 22528), (479, 3048, 28416), (706, 5344, 28032)]       # 186 / 211, 123 / 149, 173 / 249, 140 / 220, 266 / 340
+
+
+def test_the_range_is_cut_where_that_was_faster():
+    for dims in IN_ONE:
+        assert _lib.dense_plan(*dims, rebuilt=True)[2] == 1, dims
+    for dims in CUT:
+        assert _lib.dense_plan(*dims, rebuilt=True)[2] > 1, dims

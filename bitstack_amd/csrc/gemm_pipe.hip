@@ -412,6 +412,8 @@ int launch_pipe(const half_t *x, const half_t *w, const half_t *bias, half_t *y,
     if (p.parts == 1) {
         if (p.stages != S) linear_pipe_kernel<P, Q, SWAP, S_TWO, false><<<p.tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, p.steps, wide);
         else linear_pipe_kernel<P, Q, SWAP, S, false><<<p.tiles, 512, 0, s>>>(x, w, bias, y, nullptr, T, M, N, p.steps, wide);
+    } else if constexpr (B::BF == 64) {
+        return BS_ERR_SHAPE;                  // (never cut: see linear_choice)
     } else {
         if (p.stages != S) linear_pipe_kernel<P, Q, SWAP, S_TWO, true><<<p.tiles * p.parts, 512, 0, s>>>(x, w, bias, y, part, T, M, N, p.steps, wide);
         else linear_pipe_kernel<P, Q, SWAP, S, true><<<p.tiles * p.parts, 512, 0, s>>>(x, w, bias, y, part, T, M, N, p.steps, wide);

@@ -385,12 +385,14 @@ static LinearTile linear_tile(int T, int M, int N, bool aligned) {
            wgs(128, 128) >= 160 ? LinearTile{128, 128, 64} : LinearTile{64, 64, 128};
 }
 
-// Which kernel has the 64 x 64 tiles where N % 64 == 0: linear_f16_kernel's k-steps of 128 are ahead where a few CUs have a second workgroup and the rows are long (us,
-// linear_f16_kernel / linear_pipe_kernel: 140 tokens on 6144 x 4096 27.9 / 30.9, 256 33.3 / 35.5, 300 on 4096 x 14336 102 / 107), otherwise it is behind (140 on 1024 x 4096
-// 16.0 / 13.6, 190 on 5000 x 2048 13.8 / 9.4, 256 20.1 / 14.4, 640 on 3000 x 1024 14.8 / 9.9, 400 on 4096 x 4096 28.7 / 25.5).
+// Which kernel has the 64 x 64 tiles where N % 64 == 0.  While a CU has one workgroup linear_pipe_kernel (us, linear_f16_kernel / linear_pipe_kernel: 190 tokens on 5000 x 2048 15.1 / 12.0, 256
+// on 4096 x 4096 23.6 / 21.2).  Beyond that linear_f16_kernel is ahead where the tiles of features are a multiple of 8: a tile's features are then on one XCD for all tokens, which reads them once
+// (256 on 5120 x 3072 23.8 / 29.2, x 8192 54.5 / 63.8, 6656 x 4096 33.9 / 35.8, 320 on 5600 x 5120 43.0 / 48.1; up to 1280 columns it is behind, 140 on 6144 x 1024 10.0 / 8.3); elsewhere it is
+// behind (200 on 7600 x 4096 42.8 / 32.3, 320 on 5152 x 1792 19.6 / 16.1), but for long rows of up to 384 workgroups, where neither is (160 on 5870 x 4096 29.3 / 32.3, 400 on 2447 32.6 / 25.6) and it stays.
+// Of 130 drawn products of 257 to 620 workgroups 3 are 2 to 7 % slower so than on linear_f16_kernel throughout, 0.956 of its time on average; by workgroups and columns alone 20 were, up to 15 %.
 static bool pipe_64(const LinearTile &tile, int T, int M, int N) {
-    const int64_t wg = bs_cdiv(T, 64) * bs_cdiv(M, 64);
-    return tile.bt == 64 && tile.bf == 64 && (wg <= 256 || wg > 384 || N <= 3072);
+    const int64_t rows = bs_cdiv(M, 64), wg = bs_cdiv(T, 64) * rows;
+    return tile.bt == 64 && tile.bf == 64 && (wg <= 256 || N <= 1280 || (rows % 8 != 0 && (wg > 384 || N <= 3072)));
 }
 
 // whether linear_pipe_kernel has this tile of bs_linear_f16's

@@ -8,8 +8,8 @@ from bitstack_amd import _lib
 
 # tokens, out features, in features: tile, k-step, whether the last one is partial
 PLANS = [
-    # 64 x 64: linear_pipe_kernel's steps of 64, where N is a multiple of them, up to 256 workgroups, beyond 384, and up to 3072 columns
-    (140, 1024, 4160, (64, 64, 64, 0)), (140, 1024, 4096, (64, 64, 64, 0)), (190, 5000, 2112, (64, 64, 64, 0)), (256, 6144, 3072, (64, 64, 64, 0)), (640, 3000, 1088, (64, 64, 64, 0)),
+    # 64 x 64: linear_pipe_kernel's steps of 64, where N is a multiple of them
+    (140, 1024, 4160, (64, 64, 64, 0)), (140, 1024, 4096, (64, 64, 64, 0)), (190, 5000, 2112, (64, 64, 64, 0)), (256, 6080, 3072, (64, 64, 64, 0)), (640, 3000, 1088, (64, 64, 64, 0)),
     # otherwise linear_f16_kernel's of 128
     (256, 6144, 4096, (64, 64, 128, 0)), (256, 6144, 4160, (64, 64, 128, 1)), (140, 1024, 4104, (64, 64, 128, 1)), (140, 6208, 3136, (64, 64, 128, 1)),
     # the larger tiles' and few tokens'
@@ -20,6 +20,15 @@ PLANS = [
 @pytest.mark.parametrize("T,M,N,plan", PLANS)
 def test_the_step_of_the_kernel_that_runs(T, M, N, plan):
     assert _lib.linear_plan(T, M, N) == plan
+
+
+def test_the_kernel_of_the_small_tiles_is_the_faster_one():
+    """Products timed on both kernels (us, linear_f16_kernel / linear_pipe_kernel)."""
+    for dims in [(256, 5120, 2048), (256, 5120, 3072), (256, 5120, 8192), (140, 6144, 14336), (256, 6144, 3072), (256, 6656, 5120), (320, 5600, 5120),   # 17.4 / 19.4, 23.8 / 29.2, 54.5 / 63.8, 87.9 / 102.9, 25.3 / 29.6, 43.7 / 49.1, 43.0 / 48.1
+                 (190, 7214, 4096), (160, 5870, 4096)]:                                                                                                   # 34.7 / 37.2, 29.3 / 32.3
+        assert _lib.dense_plan(*dims) == (64, 64, 1, 0), dims
+    for dims in [(256, 3000, 4096), (256, 4096, 8192), (190, 5000, 14336), (200, 7600, 4096), (320, 5152, 1792), (350, 3755, 1536), (140, 6144, 1024), (448, 4108, 4096)]:   # 24.5 / 20.6 ... 41.8 / 34.3
+        assert _lib.dense_plan(*dims) == (64, 64, 1, 4), dims
 
 
 def test_dense_plan_of_linear_f16_is_its_tile():

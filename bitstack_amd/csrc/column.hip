@@ -69,9 +69,10 @@ __global__ __launch_bounds__(64 * CL_WAVES, 2) void column_forward_kernel(const 
     const int K = CL_K16 ? 16 : ranks;
     extern __shared__ __attribute__((aligned(1024))) char cl_lds[];
     const cl_bytes lds = (cl_bytes)cl_lds;
-    // Behind the last block up to four blocks round first and change the sign of the rounded pairs: half the operations, the same bits (us, in fp32 / so: 28672 x 8192, 3 blocks, 80 tokens
-    // 104.3 / 101.8, 15100 x 10240, 1, 110 58.8 / 57.1; but 14336 x 4096, 5, 100 55.2 / 55.8, and level at 8).
-    constexpr bool PAIRS = I <= 4;
+    // Behind the last block the sums round first and the sign changes on the rounded pairs: half the operations, the same bits.  Of the time with the change in fp32, average over seven matrices
+    // from 20000 x 640 to 28672 x 8192 (56, 100 and 124 tokens): one block 0.978 to 0.985, two to four 0.980 to 1.002, five to eight with four token tiles 0.986 to 0.994 (28672 x 8192, 6 blocks, 56
+    // tokens 179.5 / 176.5 us), five and six with more 0.995 to 0.999, not worth the sizes that lose (14336 x 4096, 5 blocks, 100 tokens 57.6 / 58.1): these keep to fp32.
+    constexpr bool PAIRS = I <= 4 || TT == 4;
     constexpr int VT = I * CL_IMAGE, BUFFER = VT + TT * CL_IMAGE, XK = (TT + 3) / 4;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

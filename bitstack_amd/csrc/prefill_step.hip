@@ -273,7 +273,8 @@ int bs_launch_attention_prefill(const half_t *q, const half_t *kcache, const hal
         return (int)BS_OK;
     };
     // 16 queries per wave while 32 would leave the chip few workgroups: the chain of a wave's stages is what such a call takes (us, 32 / 16 queries: 2 x 700 positions with 32
-    // heads on 8 KV heads, 352 workgroups, 24.5 / 21.7; 1 x 1000 with 8 on 8 26.1 / 19.7; 4 x 300 with 32 on 8, 320, 15.0 / 14.3; but 8 x 200, 448, 15.1 / 15.6; 2 x 1000, 512, 34.8 / 41.2).
+    // heads on 8 KV heads, 352 workgroups, 24.4 / 19.7; 1 x 1000 with 8 on 8 28.6 / 20.0; 2 x 800, 400, 27.8 / 24.2; 4 x 400, 416, 17.8 / 17.6, 3 x 700 with 24 on 24, 432, 26.0 / 24.6; but 8 x
+    // 200, 448, 13.4 / 13.9, 2 x 900, 464, 30.1 / 30.3, 2 x 1000, 512, 33.7 / 35.5, 4 x 1500 with 64 on 16, 3008, 206 / 254).
     const int64_t wgs = (int64_t)B * kv_heads * bs_cdiv((int64_t)(heads / kv_heads) * bs_cdiv(n, 32), AP_WAVES);
     const int st = wgs <= 400 ? launch(attention_prefill_kernel<1>, 16) : launch(attention_prefill_kernel<2>, 32);
     if (st != BS_OK) return st;

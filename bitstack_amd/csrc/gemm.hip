@@ -406,16 +406,19 @@ struct LinearChoice { int bt, bf, splits; };      // bt == 0: as bs_linear_f16
 
 // The tiles of gemm_pipe.hip, and in us what a k-step of 64 columns and the start and end of a workgroup take: while a CU has one workgroup, and (step_two > 0) a pair of
 // workgroups that share one.  A fit to the times of every tile on 256 products, 40 to 3300 tokens on 14 matrices from 600 x 512 to 28672 x 8192: the choice
-// made with it is 1.0 % from the best tile on average, 25 at worst.  What the sums cost: whole calls cut and not, 98 of 132 to 1400 tokens on 12 matrices, and 132 drawn ones of 129 to 4100 on
+// made with it is 1.0 % from the best tile on average, 25 at worst.  Four entries were further off and are set by whole calls, 22 to 50 drawn ones each, on the tile and on the one that the new
+// estimate takes: 256 x 192 (1.336: 1.025 of the other's time on average, 2254 tokens on 4592 x 2176 59.1 us, on 192 x 256 55.7), two workgroups per CU of 160 x 128 (1.189: 1.046, 3120 on 3188 x 24576
+// 510 / 450), of 64 x 64 (0.440: 1.17, 1994 on 545 x 9088 62.2 / 52.6) and, on rows of more than 8192 columns, of 64 x 128 (1.10, 313 on 11067 x 17664 356 / 302; shorter rows are as estimated).
+// What the sums cost: whole calls cut and not, 98 of 132 to 1400 tokens on 12 matrices, and 132 drawn ones of 129 to 4100 on
 // weights of 64 to 380 MiB: beyond 64 MiB of sums 0.5 us more per MiB than up to there (2515 tokens on 9480 x 12800, 182 MiB, 597 us in two parts, 540 in one; 2735 on 7320 x 25216, 305 MiB,
 // 1001 in four, 1011).  Where the estimates are level the cut is 3 to 20 % behind (6936 x 22272, 1722 tokens 585 / 493, 8824 x 17408, 1362 480 / 427), and the calls that it is ahead on (4096 x
 // 14336, 1400 tokens 186 / 211, 509 123 / 149) are clear of that line.
 struct PipeTile { int bt, bf; double step, start, step_two, start_two; };
 static const PipeTile pipe_tiles[] = {
-    {256, 256, 1.604, 4.1, 0, 0}, {224, 256, 1.471, 3.5, 0, 0}, {192, 256, 1.358, 2.6, 0, 0}, {256, 192, 1.336, 2.9, 0, 0},
+    {256, 256, 1.604, 4.1, 0, 0}, {224, 256, 1.471, 3.5, 0, 0}, {192, 256, 1.358, 2.6, 0, 0}, {256, 192, 1.385, 2.9, 0, 0},
     {160, 256, 1.143, 3.1, 0, 0}, {192, 192, 0.966, 3.1, 0, 0}, {256, 128, 0.970, 2.6, 0, 0}, {128, 256, 0.930, 2.3, 0, 0},
-    {224, 128, 0.862, 2.2, 0, 0}, {192, 128, 0.758, 1.9, 0, 0}, {128, 192, 0.777, 2.1, 0, 0}, {160, 128, 0.760, 1.3, 1.189, 4.8},
-    {128, 128, 0.620, 1.2, 1.034, 3.0}, {96, 128, 0.540, 1.1, 0.922, 1.6}, {64, 128, 0.433, 0.8, 0.688, 1.8}, {64, 64, 0.250, 1.1, 0.440, 0.9}};
+    {224, 128, 0.862, 2.2, 0, 0}, {192, 128, 0.758, 1.9, 0, 0}, {128, 192, 0.777, 2.1, 0, 0}, {160, 128, 0.760, 1.3, 1.330, 4.8},
+    {128, 128, 0.620, 1.2, 1.034, 3.0}, {96, 128, 0.540, 1.1, 0.922, 1.6}, {64, 128, 0.433, 0.8, 0.688, 1.8}, {64, 64, 0.250, 1.1, 0.484, 0.9}};
 
 // Time in us that a tile is expected to take: rounds of workgroups over the chip, the last one shorter while part of it is idle (power, and memory to itself), plus the sums.
 static double linear_cost(const PipeTile &t, int splits, int T, int M, int N) {
@@ -423,7 +426,8 @@ static double linear_cost(const PipeTile &t, int splits, int T, int M, int N) {
     const int64_t wg = bs_cdiv(T, t.bt) * bs_cdiv(M, t.bf) * parts;
     const bool two = t.step_two > 0 && wg > 256;
     const int64_t slots = two ? 512 : 256, rounds = bs_cdiv(wg, slots);
-    double us = (rounds - 0.43 * (rounds - (double)wg / slots)) * steps * (two ? t.step_two : t.step) + rounds * (two ? t.start_two : t.start) + 2.0;
+    const double step = !two ? t.step : N > 8192 && t.bt == 64 && t.bf == 128 ? 1.1 * t.step_two : t.step_two;
+    double us = (rounds - 0.43 * (rounds - (double)wg / slots)) * steps * step + rounds * (two ? t.start_two : t.start) + 2.0;
     // (sums beyond 64 MiB no longer stay in the cache between the two kernels)
     const double sums = (double)parts * T * M, cached = 1 << 24;
     if (parts > 1) us += 3.0 + 0.5e-6 * sums + (sums > cached ? 2e-6 * (sums - cached) : 0.);

@@ -35,7 +35,6 @@ REBUILT = {
     ((128, 256), 12, 3): [(98, 4296, 8512), (101, 5016, 7360)],
     ((160, 128), 1, 2): [(129, 16709, 64), (129, 16760, 128)],
     ((160, 128), 1, 3): [(130, 16423, 192), (129, 16547, 256), (131, 16609, 320), (131, 16593, 384)],
-    ((160, 128), 12, 2): [(293, 2632, 15040), (315, 2624, 14464)],
     ((160, 128), 8, 3): [(129, 2816, 12480), (132, 3872, 8704)],
     ((160, 128), 12, 3): [(130, 1944, 17856)],
     ((160, 256), 1, 3): [(393, 16389, 192), (388, 16465, 256), (388, 16460, 320), (386, 17223, 384)],
@@ -60,9 +59,9 @@ REBUILT = {
     ((256, 128), 1, 3): [(3658, 2055, 128), (679, 10820, 192), (692, 10825, 256), (689, 10766, 320), (691, 10762, 384)],
     ((256, 128), 3, 3): [(230, 10784, 3328)],
     ((256, 128), 12, 3): [(237, 2656, 21440), (249, 2632, 12992)],
-    ((256, 192), 1, 2): [(988, 10889, 64), (971, 11061, 128), (963, 11085, 192), (969, 8987, 256)],
-    ((256, 192), 4, 2): [(193, 10888, 3520)],
-    ((256, 192), 8, 2): [(206, 5432, 7552)],
+    ((256, 192), 1, 2): [(988, 10889, 64), (971, 11061, 128), (963, 11085, 192), (967, 10936, 256)],
+    ((256, 192), 4, 2): [(453, 5672, 6784)],
+    ((256, 192), 8, 2): [(451, 2848, 12992)],
     ((256, 256), 1, 2): [(673, 16597, 64), (675, 17010, 128), (676, 16738, 192), (684, 16634, 256)],
     ((256, 256), 12, 2): [(483, 2168, 18112), (508, 2120, 17664)],
 }

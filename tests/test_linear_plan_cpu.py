@@ -70,3 +70,13 @@ def test_the_range_is_cut_where_that_was_faster():
         assert _lib.dense_plan(*dims, rebuilt=True)[2] == 1, dims
     for dims in CUT:
         assert _lib.dense_plan(*dims, rebuilt=True)[2] > 1, dims
+
+
+def test_the_tile_is_the_faster_one():
+    """Whole calls timed on the tile that is not to be taken and on the one that is (us)."""
+    for dims, other in [((2254, 4592, 2176), (256, 192)), ((3753, 2784, 3968), (256, 192)), ((687, 13264, 1920), (256, 192)),                  # 59.1 / 55.7, 93.7 / 88.6, 63.0 / 58.0
+                        ((3120, 3188, 24576), (160, 128)), ((1324, 14438, 10368), (160, 128)), ((874, 10870, 4480), (160, 128)),              # 510 / 450, 536 / 465, 125 / 116
+                        ((1994, 545, 9088), (64, 64)), ((1428, 1315, 14464), (64, 64)), ((313, 11067, 17664), (64, 128)), ((303, 11116, 15232), (64, 128))]:   # 62.2 / 52.6, 122 / 94, 356 / 302, 301 / 259
+        assert _lib.dense_plan(*dims, rebuilt=True)[:2] != other, dims
+    for dims in [(401, 8284, 1536), (404, 8240, 1920), (257, 11188, 3072)]:                                                                   # (shorter rows) 37.2 / 33.3, 39.2 / 36.3, 63.0 / 57.8
+        assert _lib.dense_plan(*dims, rebuilt=True)[:2] == (64, 128), dims
